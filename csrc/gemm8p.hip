@@ -77,7 +77,8 @@ PS_DEV unsigned ps_g8_lds_off(const void* p) {
 // order them against the in-flight global_load_lds writes — draining the
 // pipeline each phase and reducing the schedule to 1-phase performance
 // (guide T3/T4 and common-mistake notes). Correct ordering is owned by the
-// phase barriers + the two counted vmcnt(4) waits.
+// phase barriers + the two counted vmcnt(2) waits; the registers are in
+// flight until the phase's lgkmcnt(0), which names every one of them.
 PS_DEV ps_g8bf16x8 ps_g8_ds_read_b128(unsigned addr) {
   ps_g8bf16x8 r;
   asm volatile("ds_read_b128 %0, %1" : "=v"(r) : "v"(addr));
@@ -101,9 +102,9 @@ __global__ __launch_bounds__(512, 2) void gemm8p_kernel(
   int wg = blockIdx.x;
   {
     const int q = nwg >> 3, r = nwg & 7, xcd = wg & 7, lin = wg >> 3;
+    if (lin >= q + (xcd < r ? 1 : 0)) return;  // grid rounded up to eights
     wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + lin;
   }
-  if (wg >= nwg) return;
   const int m0 = (wg % mt) * PS_G8_BM;
   const int n0 = (wg / mt) * PS_G8_BN;
 
@@ -186,7 +187,11 @@ __global__ __launch_bounds__(512, 2) void gemm8p_kernel(
   const unsigned a_lds0 = ps_g8_lds_off(&a_lds[0][0][0][0]);
   const unsigned b_lds0 = ps_g8_lds_off(&b_lds[0][0][0][0]);
 
-  auto phase = [&](int buf, int mh, int nh, int s_which, int s_kt) {
+  // `last`: the K-tile's last phase. Its stage refills the very A half that
+  // the waves of one M position read in this phase, so every wave's reads
+  // are drained ahead of the barrier and the stage follows it.
+  auto phase = [&](int buf, int mh, int nh, int s_which, int s_kt,
+                   bool last) {
     // A rows: half mh, rows mt*16 + rc (mt 0..3); B: wave's n-half
     const int bh = wn >> 1;  // B half this wave reads
     const int brow0 = (wn & 1) * 64 + nh * 32;
@@ -208,9 +213,23 @@ __global__ __launch_bounds__(512, 2) void gemm8p_kernel(
         bf[ks][ntl] = ps_g8_ds_read_b128(b_base + byte);
       }
     }
-    stage(s_which, s_kt);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (!last) {
+      stage(s_which, s_kt);
+      __builtin_amdgcn_s_barrier();
+    }
+    // one statement that waits and redefines the registers the reads above
+    // fill: no copy or use of them can move ahead of it
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(af[0][0]), "+v"(af[0][1]), "+v"(af[0][2]),
+                   "+v"(af[0][3]), "+v"(af[1][0]), "+v"(af[1][1]),
+                   "+v"(af[1][2]), "+v"(af[1][3]), "+v"(bf[0][0]),
+                   "+v"(bf[0][1]), "+v"(bf[1][0]), "+v"(bf[1][1])
+                 :
+                 : "memory");
+    if (last) {
+      __builtin_amdgcn_s_barrier();
+      stage(s_which, s_kt);
+    }
     __builtin_amdgcn_sched_barrier(0);  // guide rule #18: pin MFMAs after
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -234,24 +253,33 @@ __global__ __launch_bounds__(512, 2) void gemm8p_kernel(
     // LAST ds_read was in phase <= p-1 — the closing barrier of p-1
     // comes after every wave's lgkmcnt(0) drain, so no wave still has a
     // read of that slot in the LDS pipe when the staged write can land
-    // (global-load->LDS writes are NOT ordered against ds_reads).
+    // (global-load->LDS writes are NOT ordered against ds_reads). A(t)h0 is
+    // read up to p3 (A(t+1)h0 up to p7) by the waves of M position 0:
+    // those two phases drain their reads, meet, and stage after that.
     //   p0: B(t+1)h0  p1: B(t+1)h1  p2: A(t+1)h1  p3: A(t+2)h0
     //   p4: A(t+2)h1  p5: B(t+2)h0  p6: B(t+2)h1  p7: A(t+3)h0
     // Counted waits (guide T4): vmcnt(2) at the two half-iteration
     // starts; FIFO completion guarantees the 4 half-tiles the next 4
-    // phases read have landed while 1 half-tile stays in flight.
+    // phases read have landed while 1 half-tile stays in flight (the last
+    // iteration has none in flight and waits for all).
     asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    phase(b0, 0, 0, /*B(t+1)h0*/ 2, t + 1);
-    phase(b0, 0, 1, /*B(t+1)h1*/ 3, t + 1);
-    phase(b0, 1, 0, /*A(t+1)h1*/ 1, t + 1);
-    phase(b0, 1, 1, /*A(t+2)h0*/ 0, t + 2);
-    asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    phase(b0, 0, 0, /*B(t+1)h0*/ 2, t + 1, false);
+    phase(b0, 0, 1, /*B(t+1)h1*/ 3, t + 1, false);
+    phase(b0, 1, 0, /*A(t+1)h1*/ 1, t + 1, false);
+    phase(b0, 1, 1, /*A(t+2)h0*/ 0, t + 2, true);
+    // The last iteration stages nothing in p3 (t+2 lies past the range), so
+    // two outstanding loads would be p2's half of A(t+1), which the next
+    // phases read: everything has to have landed.
+    if (it + 1 < n_iter)
+      asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    phase(b1, 0, 0, /*A(t+2)h1*/ 1, t + 2);
-    phase(b1, 0, 1, /*B(t+2)h0*/ 2, t + 2);
-    phase(b1, 1, 0, /*B(t+2)h1*/ 3, t + 2);
-    phase(b1, 1, 1, /*A(t+3)h0*/ 0, t + 3);
+    phase(b1, 0, 0, /*A(t+2)h1*/ 1, t + 2, false);
+    phase(b1, 0, 1, /*B(t+2)h0*/ 2, t + 2, false);
+    phase(b1, 1, 0, /*B(t+2)h1*/ 3, t + 2, false);
+    phase(b1, 1, 1, /*A(t+3)h0*/ 0, t + 3, true);
   }
 
   // Drain every outstanding staged load before exit: an LDS write landing
@@ -313,7 +341,11 @@ int ps_gemm8p_splits(int M, int N, int K) {
   if (splits < 1) splits = 1;
   const int kpairs = K / 128;
   if (splits > kpairs) splits = kpairs;
-  return splits;
+  // the kernel hands out whole ranges of ceil(kpairs / splits) pairs: count
+  // the ranges that are not empty, since an empty one writes no partial and
+  // the combine pass would add what its workspace happened to hold
+  const int per_split = (kpairs + splits - 1) / splits;
+  return (kpairs + per_split - 1) / per_split;
 }
 
 int ps_gemm8p(void* out_bf16, void* ws, const void* x, const void* w, int M,

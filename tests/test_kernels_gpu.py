@@ -710,3 +710,26 @@ def test_fp8_linear_rowwise_matches_reference():
     got = ops.fp8_linear_rowwise(xq, sx, w_q, sw).float().cpu()
     want = (x.float() @ w.float().t()).cpu()
     _close(got, want, atol=0.4, rtol=0.1)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 2048, 8192),      # more ranges asked for than whole pairs fill
+    (192, 4096, 14336),   # 112 pairs in 23 ranges of 5, the last one of 2
+    (192, 6144, 4096),    # two pairs per range: one iteration is the last
+    (61, 256, 128),       # a single pair
+    (300, 512, 384),      # one range, remainder of a row tile
+])
+def test_gemm8p_split_ranges(m, n, k):
+    """Every output is the sum of all K ranges, none of them empty, and the
+    last iteration of a range waits for what it reads."""
+    x = torch.randn(m, k, dtype=torch.bfloat16, device="cuda")
+    w = torch.randn(n, k, dtype=torch.bfloat16, device="cuda")
+    # leave not-a-numbers in memory the workspace may be given
+    del_me = torch.full((48 * m * n,), float("nan"), device="cuda")
+    del del_me
+    want = x.double() @ w.double().t()
+    for _ in range(3):
+        got = ops.gemm8p(x, w).double()
+        # one bf16 rounding of an fp32 sum of k products
+        err = ((got - want).abs() / (want.abs() + k ** 0.5)).max().item()
+        assert err < 2 ** -7, err
