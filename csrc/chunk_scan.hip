@@ -1,0 +1,1425 @@
+// Chunk-parallel form of the recurrences with a decay per key channel: whole
+// chunks of 16 tokens go through matrix products instead of one token at a
+// time. Per head the state S is a D x DV fp32 matrix and every token does
+//
+//   general delta  w = exp(-scale sigmoid(zw + w0)), a = sigmoid(za + ab),
+//                  u = k / sqrt(sum k^2 + 1e-6)
+//                  S <- diag(w) S - (a u)(u^T S) + k v^T,   o = S^T r
+//   channel delta  w = exp(-exp(a_log) softplus(z + dt_bias)), k^, q^ unit
+//                  vectors (q^ times qscale), b = sigmoid(beta)
+//                  S <- diag(w) S;  S <- S + b k^ (v - S^T k^)^T, o = S^T q^
+//   gla            w = sigmoid(z + p0)^c0
+//                  S <- diag(w) S + k v^T,                  o = S^T (q qscale)
+//   ssd, mlstm     one decay a and write scale w per head and token
+//                  S <- a S + w k v^T,                      o = S^T (q qscale)
+//
+// Let W_t be the product of the decays of a chunk's tokens up to t, per key
+// channel, and Z_t = (what token t reads of the state before its own write).
+// Then for the chunk, S0 being the state before it,
+//
+//   general  (I - Bm) Z = U S0 + Km V,   Bm_ts = u_t W_{t-1}/W_s b_s  (s < t)
+//            with b = -a u, U_t = u_t W_{t-1}, Km likewise with k_s
+//            O = R S0 + Mb Z + Mk V,     R_t = r_t W_t, Mb_ts = r_t W_t/W_s b_s
+//            S = diag(W_C) S0 + B^T Z + K^T V,  B_s = b_s W_C/W_s, K_s likewise
+//   channel  (I + A) Y = V - U S0,       Y = V - Z, U_t = k_t W_t,
+//            A_ts = k_t W_t/W_s b_s k_s  (s < t);  O = R S0 + M Y,
+//            S = diag(W_C) S0 + K^T Y
+//   gla      O = R S0 + M V,  S = diag(W_C) S0 + K^T V
+//   scalar   O = diag(W) Q S0 + M V,  M_ts = q_t k_s W_t/W_s w_s (s <= t)
+//            S = W_C S0 + K^T diag(w W_C/W) V, Q and K as they are, shared by
+//            the heads of a group; every ratio is a product of its own
+//
+// Everything but the state is known ahead, so it is laid down by one fully
+// parallel kernel (one workgroup per chunk and head: the decays' products,
+// the 16 x 16 matrices, the triangular solve), and a second kernel walks the
+// chunks with the state in registers: a wave owns 16 columns of S as D / 16
+// accumulator tiles of v_mfma_f32_16x16x4_f32. The tiles' register layout (row
+// 4 g + i of a tile in lane group g, register i) is at once the layout of the
+// right operand of the products that read S when the left operand's columns
+// are taken in the order 4 g + i, so the state never leaves its registers; Z
+// and Y pass from one product into the next the same way.
+//
+// Arithmetic is fp32 throughout (the matrix unit's fp32 products: fp32 inputs,
+// fp32 accumulation). Ratios W_t / W_s are formed from products counted from
+// the middle of the chunk, so both factors stay in range while either half's
+// product is above 1e-30; chunks beyond that (or with decays that are no
+// numbers) form every ratio on its own.
+//
+// One token at a time is a chain of two dot products and two lane reductions
+// per token on D x DV lanes; measured at 32 heads of 128 x 128, 8011 tokens in
+// two prompts: 12.3 ms, 1.5 us a token. Figures of this form stand at the
+// launcher.
+#include "scan_common.h"
+
+// Float4 slots of a chunk's operands. Left operands whose rows are tokens:
+// lane (g, m) of tile t reads channels 16 t + 4 g .. + 3 of token m. The
+// token index is twisted so that writing one token's channels spreads over
+// all LDS banks.
+PS_DEV int ck_row_slot(int t, int g, int m) {
+  return t * 64 + g * 16 + (m ^ ((t * 4 + g) & 15));
+}
+// Left operands whose rows are channels: lane (g, m) reads tokens 4 g .. + 3
+// of channel 16 t + m.
+PS_DEV int ck_col_slot(int t, int g, int m) { return t * 64 + g * 16 + m; }
+
+// Floats of one chunk's operands and where each lies.
+template <int MODE, int DP>
+struct CkItem {
+  static constexpr int ROW = 16 * DP;  // one 16 x DP operand
+  static constexpr int R = 0;
+  static constexpr int K = ROW;
+  static constexpr int U = 2 * ROW;                        // delta forms
+  static constexpr int B = 3 * ROW;                        // general delta
+  static constexpr int NROW = MODE == CK_GD ? 4 : (MODE == CK_CD ? 3 : 2);
+  static constexpr int M = NROW * ROW;                     // on V (Y)
+  static constexpr int C = M + 256;                        // solve on V
+  static constexpr int MB = C + 256;                       // on Z
+  static constexpr int NSQ = MODE == CK_GD ? 3 : (MODE == CK_CD ? 2 : 1);
+  static constexpr int GAM = M + NSQ * 256;                // [DP]
+  static constexpr int FLAG = GAM + DP;  // not 0: an input is no finite number
+  static constexpr int TOTAL = FLAG + 4;
+};
+
+// Chunks of a segment of n rows in this pass (chunks c0 .. c0 + nc of every
+// segment; segments shorter than 16 rows are not this kernel's).
+PS_DEV int ck_count(int n, int c0, int nc) {
+  if (n < 16) return 0;
+  return max(0, min(nc, (n + 15) / 16 - c0));
+}
+
+// Which chunk of which segment this pass's item is; false past the last one.
+// Every wave of a block finds the same.
+PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int c0, int nc,
+                    int lane, int* seg, int* chunk) {
+  int base = 0;
+  for (int s0 = 0; s0 < S_; s0 += 64) {
+    const int s = s0 + lane;
+    const int cnt = s < S_ ? ck_count(seq_rows[4 * s + 1], c0, nc) : 0;
+    int incl = cnt;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += up;
+    }
+    const int first = base + incl - cnt;
+    const unsigned long long hit =
+        __ballot(cnt > 0 && item >= first && item < first + cnt);
+    if (hit) {
+      const int l = __ffsll((long long)hit) - 1;
+      *seg = s0 + l;
+      *chunk = c0 + item - __builtin_amdgcn_readlane(first, l);
+      return true;
+    }
+    base += __builtin_amdgcn_readlane(incl, 63);
+  }
+  return false;
+}
+
+template <typename T, int MODE, int DP>
+__global__ __launch_bounds__(256, 3) void ck_prep_kernel(
+    float* __restrict__ items, CkIn in, const int* __restrict__ seq_rows,
+    int S_, int H, int G, int D, float scale, float c0f, int c0, int nc) {
+  typedef CkItem<MODE, DP> It;
+  constexpr int LD = DP + 4;
+  // operand rows in channel order; reused for the fragments once the 16 x 16
+  // products are done
+  __shared__ __align__(16) float stage[
+      It::TOTAL > 4 * 16 * LD ? It::TOTAL : 4 * 16 * LD];
+  __shared__ __align__(16) float su[MODE == CK_GLA ? 4 : 16 * LD];
+  __shared__ __align__(16) float sm[4][16][20];
+  __shared__ float red[2][16][2];
+  __shared__ float half_prod[2][128];
+  float* X0 = stage;              // rows that read the state for Z
+  float* X1 = X0 + 16 * LD;       // rows that read it for the output
+  float* Y0 = X1 + 16 * LD;       // columns written with Z
+  float* Y1 = Y0 + 16 * LD;       // columns written with V
+
+  // which chunk of which segment
+  const int item = blockIdx.x, hd = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int seg, chunk;
+  if (!ck_find(seq_rows, S_, item, c0, nc, lane, &seg, &chunk)) return;
+  const int n = seq_rows[4 * seg + 1];
+  const int row0 = seq_rows[4 * seg] + 16 * chunk;
+  const int nv = min(16, n - 16 * chunk);
+
+  const int half = threadIdx.x >> 7, d = threadIdx.x & 127;
+  const bool on = d < DP, real = d < D;
+  const int grp = hd / (H / G);
+  const int hk = MODE == CK_GD ? hd * D + d : grp * D + d;
+  const int hz = hd * D + d;
+
+  const T* qp = (const T*)in.q;
+  const T* kp = (const T*)in.k;
+  const T* zp = (const T*)in.dec;
+  const T* ap = (const T*)in.a;
+  float kv[8], rv[8], wv[8], av[8];
+  // all loads ahead of any use, from a row and a channel that exist
+  const int dc = real ? 0 : -d;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const size_t row = (size_t)(row0 + min(half * 8 + e, nv - 1));
+    kv[e] = MxElem<T>::ld(kp + row * in.ldk + hk + dc);
+    rv[e] = MxElem<T>::ld(qp + row * in.ldq + hk + dc);
+    wv[e] = MxElem<T>::ld(zp + row * in.lddec + hz + dc);
+    av[e] = 0.f;
+    if (MODE == CK_GD) av[e] = MxElem<T>::ld(ap + row * in.lda + hz + dc);
+    if (MODE == CK_CD) av[e] = MxElem<T>::ld(ap + row * in.lda + hd);
+  }
+  const float c0z = in.p0[hz + dc];
+  float c1 = 0.f;
+  if (MODE == CK_GD) c1 = in.p1[hz + dc];
+  if (MODE == CK_CD) c1 = expf(in.p1[hd]);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const bool live = real && half * 8 + e < nv;
+    float w;
+    if (MODE == CK_GD) {
+      w = ck_exp(-scale * ck_sigmoid(wv[e] + c0z));
+      av[e] = ck_sigmoid(av[e] + c1);
+    } else if (MODE == CK_CD) {
+      w = ck_exp(-c1 * ck_softplus(wv[e] + c0z));
+      av[e] = ck_sigmoid(av[e]);
+    } else {
+      w = ck_exp(ck_log_sigmoid(wv[e] + c0z) * c0f);
+    }
+    wv[e] = live ? w : 1.f;  // rows past the segment's end change nothing
+    if (!live) kv[e] = rv[e] = av[e] = 0.f;
+  }
+
+  // unit vectors
+  if (MODE != CK_GLA) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float k2 = mx_wave_sum(kv[e] * kv[e]);
+      const float r2 = MODE == CK_CD ? mx_wave_sum(rv[e] * rv[e]) : 0.f;
+      if (lane == 0) {
+        red[0][half * 8 + e][wave & 1] = k2;
+        red[1][half * 8 + e][wave & 1] = r2;
+      }
+    }
+  }
+  // products of the decays within the half
+  float pin[8];   // up to and with token e, from the half's first
+  float suf[8];   // of the tokens behind e, to the half's last
+  {
+    float p = 1.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      p *= wv[e];
+      pin[e] = p;
+    }
+    float s = 1.f;
+#pragma unroll
+    for (int e = 7; e >= 0; --e) {
+      suf[e] = s;
+      s *= wv[e];
+    }
+  }
+  half_prod[half][d] = pin[7];
+  float mag = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    mag += fabsf(kv[e]) + fabsf(rv[e]) + fabsf(wv[e]) + fabsf(av[e]);
+  const bool odd = __syncthreads_or(!(mag < INFINITY));
+  // out of range (or no number): ratios are formed one by one
+  const bool slow =
+      __syncthreads_or(on && !(pin[7] > 1e-30f && pin[7] < 1e30f));
+  const float other = half_prod[half ^ 1][d];
+
+  float uv[8], bv[8];  // u (GD) / k^ (CD); b
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int tt = half * 8 + e;
+    uv[e] = bv[e] = 0.f;
+    if (MODE == CK_GD) {
+      const float ik = ck_rsqrt(red[0][tt][0] + red[0][tt][1] + 1e-6f);
+      uv[e] = kv[e] * ik;
+      bv[e] = -av[e] * uv[e];
+    } else if (MODE == CK_CD) {
+      const float ik = ck_rsqrt(red[0][tt][0] + red[0][tt][1] + 1e-6f);
+      const float iq = scale * ck_rsqrt(red[1][tt][0] + red[1][tt][1] + 1e-6f);
+      uv[e] = kv[e] * ik;
+      kv[e] = av[e] * uv[e];
+      rv[e] *= iq;
+    } else {
+      rv[e] *= scale;
+    }
+  }
+
+  if (on) {
+    // W_t counted from the middle (W_7 = 1) and its inverse; general delta's
+    // reading rows take W_{t-1}
+    float inv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) inv[e] = ck_rcp(half == 0 ? suf[e] : pin[e]);
+    const float from = half == 0 ? 1.f : other;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int tt = half * 8 + e;
+      float wt = half == 0 ? inv[e] : pin[e];
+      float iw = half == 0 ? suf[e] : inv[e];
+      float wp = half == 0 ? (e > 0 ? inv[e > 0 ? e - 1 : 0] : 0.f)
+                           : (e > 0 ? pin[e > 0 ? e - 1 : 0] : 1.f);
+      if (slow) wt = iw = wp = 1.f;
+      if (MODE == CK_GD) X0[tt * LD + d] = uv[e] * wp;
+      if (MODE == CK_CD) X0[tt * LD + d] = uv[e] * wt;
+      X1[tt * LD + d] = rv[e] * wt;
+      if (MODE == CK_GD) Y0[tt * LD + d] = bv[e] * iw;
+      Y1[tt * LD + d] = kv[e] * iw;
+      // what reads the state before the chunk: products from its start
+      if (MODE == CK_GD)
+        su[tt * LD + d] =
+            uv[e] * (e > 0 ? from * pin[e > 0 ? e - 1 : 0] : from);
+      if (MODE == CK_CD) su[tt * LD + d] = uv[e] * (from * pin[e]);
+    }
+  }
+  __syncthreads();
+
+  // the 16 x 16 products, one per wave: C[t][s], t in rows
+  const int g = lane >> 4, m16 = lane & 15;
+  if (!slow) {
+    const float* xa = nullptr;
+    const float* yb = nullptr;
+    if (MODE == CK_GD) {
+      xa = wave < 2 ? X0 : X1;
+      yb = (wave & 1) ? Y1 : Y0;
+    } else if (MODE == CK_CD) {
+      if (wave < 2) {
+        xa = wave == 0 ? X0 : X1;
+        yb = Y1;
+      }
+    } else if (wave == 0) {
+      xa = X1;
+      yb = Y1;
+    }
+    if (xa != nullptr) {
+      ck_f32x4 c = {0.f, 0.f, 0.f, 0.f}, c2 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < DP / 16; ++t) {
+        const ck_f32x4 x = *(const ck_f32x4*)(xa + m16 * LD + t * 16 + g * 4);
+        const ck_f32x4 y = *(const ck_f32x4*)(yb + m16 * LD + t * 16 + g * 4);
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0], y[0], c, 0, 0, 0);
+        c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[1], y[1], c2, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[2], y[2], c, 0, 0, 0);
+        c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[3], y[3], c2, 0, 0, 0);
+      }
+      const bool strict = xa == X0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = 4 * g + i;
+        const bool seen = strict ? t > m16 : t >= m16;
+        sm[wave][t][m16] = seen ? c[i] + c2[i] : 0.f;
+      }
+    }
+    __syncthreads();
+  } else {
+    // every ratio on its own: thread (t, s) multiplies the decays between
+    // its two tokens, channel by channel
+    float* sw = &sm[0][0][0];  // 16 x 16 decays of one channel tile
+    const int t = threadIdx.x >> 4, s = threadIdx.x & 15;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int d0 = 0; d0 < DP; d0 += 16) {
+      __syncthreads();
+      if (on && d >= d0 && d < d0 + 16) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          sw[(half * 8 + e) * 17 + d - d0] = wv[e];
+      }
+      __syncthreads();
+      for (int i = 0; i < 16; ++i) {
+        float ez = 1.f;  // behind s, up to t - 1
+        for (int jj = s + 1; jj < t; ++jj) ez *= sw[jj * 17 + i];
+        const float er = t > s ? ez * sw[t * 17 + i] : 1.f;
+        const float y1 = Y1[s * LD + d0 + i];
+        if (MODE == CK_GD) {
+          const float y0 = Y0[s * LD + d0 + i], x0 = X0[t * LD + d0 + i];
+          acc[0] += x0 * ez * y0;
+          acc[1] += x0 * ez * y1;
+          acc[2] += X1[t * LD + d0 + i] * er * y0;
+          acc[3] += X1[t * LD + d0 + i] * er * y1;
+        } else {
+          if (MODE == CK_CD) acc[0] += X0[t * LD + d0 + i] * er * y1;
+          acc[MODE == CK_CD ? 1 : 0] += X1[t * LD + d0 + i] * er * y1;
+        }
+      }
+    }
+    __syncthreads();
+    constexpr int STRICT = MODE == CK_GD ? 2 : (MODE == CK_CD ? 1 : 0);
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      sm[w][t][s] = (w < STRICT ? t > s : t >= s) ? acc[w] : 0.f;
+    __syncthreads();
+  }
+
+  // fragments (over the operand rows, which nothing reads any more)
+  constexpr int LAST = MODE == CK_GD ? 3 : (MODE == CK_CD ? 1 : 0);
+  if (on) {
+    const int t = d >> 4, dg = (d & 15) >> 2, di = d & 3;
+    float kf[8], bf[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int tt = half * 8 + e;
+      const float from = half == 0 ? pin[e] : other * pin[e];
+      const float to = half == 0 ? suf[e] * other : suf[e];
+      stage[It::R + ck_row_slot(t, dg, tt) * 4 + di] = rv[e] * from;
+      kf[e] = kv[e] * to;
+      bf[e] = bv[e] * to;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = ck_col_slot(t, half * 2 + h, d & 15) * 4;
+      *(ck_f32x4*)(stage + It::K + at) =
+          ck_f32x4{kf[4 * h], kf[4 * h + 1], kf[4 * h + 2], kf[4 * h + 3]};
+      if (MODE == CK_GD)
+        *(ck_f32x4*)(stage + It::B + at) =
+            ck_f32x4{bf[4 * h], bf[4 * h + 1], bf[4 * h + 2], bf[4 * h + 3]};
+    }
+    if (half == 0) stage[It::GAM + d] = pin[7] * other;
+    if (threadIdx.x < 4) stage[It::FLAG + threadIdx.x] = odd ? 1.f : 0.f;
+  }
+  if (wave == 3)
+    *(ck_f32x4*)(stage + It::M + lane * 4) =
+        *(const ck_f32x4*)(&sm[LAST][m16][g * 4]);
+  if (MODE == CK_GD && wave == 2)
+    *(ck_f32x4*)(stage + It::MB + lane * 4) =
+        *(const ck_f32x4*)(&sm[2][m16][g * 4]);
+  if (MODE != CK_GLA) {
+    // forward substitution, one thread per column of [U | Km] (general) or
+    // [U | I] (channel)
+    const int col = threadIdx.x;
+    if (col < DP + 16) {
+      float x[16];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        float b;
+        if (col < DP)
+          b = su[t * LD + col];
+        else if (MODE == CK_GD)
+          b = sm[1][t][col - DP];
+        else
+          b = t == col - DP ? 1.f : 0.f;
+#pragma unroll
+        for (int s4 = 0; s4 < (t + 3) / 4; ++s4) {
+          const ck_f32x4 r4 = *(const ck_f32x4*)(&sm[0][t][s4 * 4]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int s = s4 * 4 + i;
+            if (s < t) b += (MODE == CK_GD ? r4[i] : -r4[i]) * x[s];
+          }
+        }
+        x[t] = b;
+      }
+      if (col < DP) {
+        const int t = col >> 4, dg = (col & 15) >> 2, di = col & 3;
+#pragma unroll
+        for (int tt = 0; tt < 16; ++tt)
+          stage[It::U + ck_row_slot(t, dg, tt) * 4 + di] = x[tt];
+      } else {
+        const int s = col - DP;
+#pragma unroll
+        for (int tt = 0; tt < 16; ++tt)
+          stage[It::C + ((s >> 2) * 16 + tt) * 4 + (s & 3)] = x[tt];
+      }
+    }
+  }
+  __syncthreads();
+  float* dst = items + ((size_t)item * H + hd) * It::TOTAL;
+  for (int i = threadIdx.x; i < It::TOTAL / 4; i += 256)
+    *(ck_f32x4*)(dst + i * 4) = *(const ck_f32x4*)(stage + i * 4);
+}
+
+PS_DEV bool ck_finite(ck_f32x4 a) {
+  // the sum of the magnitudes is a number below infinity only if all are
+  return fabsf(a[0]) + fabsf(a[1]) + fabsf(a[2]) + fabsf(a[3]) < INFINITY;
+}
+
+// acc + (16 x 16 matrix) x term by term, x in the accumulators' layout, `frag`
+// the matrix in fragment order. The matrix's zeros above its diagonal are left
+// out: an entry of x that is no finite number would turn them into NaN and
+// reach earlier tokens. tmp: 256 floats of this wave's.
+PS_DEV ck_f32x4 ck_square_terms(const float* frag, ck_f32x4 x, ck_f32x4 acc,
+                                int lane, float* tmp) {
+  const int g = lane >> 4, n = lane & 15;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) tmp[(4 * g + i) * 16 + n] = x[i];
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+  for (int s = 0; s < 16; ++s) {
+    const float xs = tmp[s * 16 + n];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float a = frag[((s >> 2) * 16 + 4 * g + i) * 4 + (s & 3)];
+      if (a != 0.f) acc[i] += a * xs;
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  return acc;
+}
+
+// Walks the chunks of one (segment, head) for 32 columns of its state: four
+// waves, two per 16 columns, each with half of the state's rows. raw [T, H *
+// DV]: S^T r before the read-out's norm.
+//
+// The chain from one chunk to the next is what bounds this kernel (a prompt
+// has a few hundred chunks and 2 x heads x DV / 16 waves are about one per
+// SIMD), so a chunk's products are split over as many waves as pay for the
+// exchange: the halves of Z and O meet in LDS once per chunk. Operands come
+// in two chunks ahead, through registers into one of two LDS buffers.
+// Workgroups of one head are S_ * H apart, so that they share an XCD's L2
+// where that is a multiple of 8.
+template <typename T, int MODE, int DP>
+__global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
+    float* __restrict__ raw, const float* __restrict__ items, int cap,
+    const T* __restrict__ v, int ldv, float* __restrict__ state,
+    const int* __restrict__ seq_rows, int S_, int H, int D, int DV, int c0,
+    int nc) {
+  typedef CkItem<MODE, DP> It;
+  constexpr int NT = DP / 32;  // row tiles of one wave
+  constexpr int N4 = It::TOTAL / 4;
+  constexpr int PF = (N4 + 255) / 256;
+  extern __shared__ __align__(16) float lds[];  // [2][BUF], exchange, tmp
+  constexpr int BUF = PF * 1024;  // TOTAL and what the last threads overhang
+  float* xch = lds + 2 * BUF;     // [4 waves][2][64][4]
+  float* tmp = xch + 2048 + (threadIdx.x >> 6) * 256;
+
+  const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H);
+  const int seg = sh / H, hd = sh % H;
+  const int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
+  const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  int count = ck_count(n, c0, nc);
+  if (count == 0) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // this segment's first chunk among all
+  int first = 0;
+  for (int s = lane; s < seg; s += 64)
+    first += ck_count(seq_rows[4 * s + 1], c0, nc);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
+  first = __builtin_amdgcn_readfirstlane(first);
+  count = __builtin_amdgcn_readfirstlane(min(count, cap - first));
+  if (count <= 0) return;
+
+  const int g = lane >> 4, m16 = lane & 15;
+  const int ct = wave >> 1, ds = wave & 1;  // column tile, row half
+  const int tb = ds * NT;                   // this wave's first row tile
+  const int j = cb * 32 + ct * 16 + m16;    // this lane's column
+  const bool col = j < DV;
+  const int hv = hd * DV + j;
+  float* Sg = state + ((size_t)slot * H + hd) * (size_t)D * DV;
+  ck_f32x4 S[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = 16 * (tb + t) + 4 * g + i;
+      S[t][i] = (col && d < D && (p0 != 0 || c0 != 0))
+                    ? Sg[(size_t)d * DV + j]
+                    : 0.f;
+    }
+
+  const char* src = (const char*)(items + ((size_t)first * H + hd) * It::TOTAL);
+  const size_t step = (size_t)H * It::TOTAL * sizeof(float);
+  // a uniform base and a 32-bit offset per lane: no address arithmetic
+  const unsigned at16 = threadIdx.x * 16;
+  const unsigned at16l =
+      min((unsigned)(PF - 1) * 256 + threadIdx.x, (unsigned)N4 - 1) * 16;
+  const T* vcol = v + (size_t)t0 * ldv + (col ? hv : 0);
+  const size_t rs = (size_t)H * DV;
+  // values stay as loaded until they are used: a conversion here would wait
+  // for them
+  struct Vals {
+    T x[4];
+  };
+  auto fetch = [&](int c, ck_f32x4(&pf)[PF], Vals& pv) {
+    c = min(c, count - 1);
+    const char* base = src + (size_t)c * step;
+#pragma unroll
+    for (int u = 0; u < PF - 1; ++u)
+      pf[u] = *(const ck_f32x4*)(base + u * 4096 + at16);
+    pf[PF - 1] = *(const ck_f32x4*)(base + at16l);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int tt = min(16 * (c0 + c) + 4 * g + i, n - 1);
+      pv.x[i] = vcol[(size_t)tt * ldv];
+    }
+  };
+  auto put = [&](float* dst, const ck_f32x4(&pf)[PF]) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      const int i = u * 256 + threadIdx.x;
+      if (i < N4) *(ck_f32x4*)(dst + i * 4) = pf[u];
+    }
+  };
+
+  // valid rows of this lane group in chunk c, and their values
+  auto rows_left = [&](int c) {
+    return col ? n - 16 * (c0 + c) - 4 * g : 0;
+  };
+  auto values = [&](int c, const Vals& pv) {
+    ck_f32x4 V;
+    const int left = rows_left(c);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float x = MxElem<T>::ld(&pv.x[i]);
+      V[i] = i < left ? x : 0.f;
+    }
+    return V;
+  };
+
+  // One chunk from `buf` with the values `pv`. On the way the operands of
+  // chunk c + 2 are asked for (into pf / pv) and those of chunk c + 1 (`nf`)
+  // are put into `nbuf`: both among matrix products, which run on while the
+  // wave issues them.
+  auto walk = [&](int c, const float* buf, ck_f32x4(&pf)[PF], Vals& pv,
+                  float* nbuf, const ck_f32x4(&nf)[PF]) {
+    const ck_f32x4 V = values(c, pv);
+    // all operands of a stage are read ahead of its products
+    ck_f32x4 r4[NT], u4[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int at = ck_row_slot(tb + t, g, m16) * 4;
+      r4[t] = *(const ck_f32x4*)(buf + It::R + at);
+      if constexpr (MODE != CK_GLA)
+        u4[t] = *(const ck_f32x4*)(buf + It::U + at);
+    }
+    // the products with V that the other half does not make: half 0 has the
+    // solve's, half 1 the output's (gla: half 0 the output's)
+    const int sq = MODE == CK_GLA || (MODE == CK_GD && ds == 1)
+                       ? It::M : It::C;
+    const ck_f32x4 q4 = *(const ck_f32x4*)(buf + sq + lane * 4);
+    const bool fin =
+        buf[It::FLAG] == 0.f && !__any(!ck_finite(V));
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(c + 2, pf, pv);
+    ck_f32x4 O = {0.f, 0.f, 0.f, 0.f}, Z = O, X = O;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (MODE != CK_GLA) {
+          Z = __builtin_amdgcn_mfma_f32_16x16x4f32(u4[t][i], S[t][i], Z, 0, 0,
+                                                   0);
+          O = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i], S[t][i], O, 0, 0,
+                                                   0);
+        } else if (i & 1) {
+          // two chains: a dependent product waits for the one before it
+          Z = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i], S[t][i], Z, 0, 0,
+                                                   0);
+        } else {
+          O = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i], S[t][i], O, 0, 0,
+                                                   0);
+        }
+      }
+      X = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[t & 3], V[t & 3], X, 0, 0,
+                                               0);
+      if (NT < 4 && t == NT - 1) {
+#pragma unroll
+        for (int i = NT; i < 4; ++i)
+          X = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[i], V[i], X, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PF + 4; ++u) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // products
+      __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // addresses
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // a load
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const ck_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    if (!fin) X = ck_square_terms(buf + sq, V, zero, lane, tmp);
+    if constexpr (MODE == CK_GLA) {
+      O += Z;
+      if (ds == 0) O += X;
+    } else if constexpr (MODE == CK_GD) {
+      if (ds == 0)
+        Z += X;
+      else
+        O += X;
+    } else {
+      Z = ds == 0 ? X - Z : -Z;
+    }
+    // the other half's share
+    float* mine = xch + wave * 512 + lane * 4;
+    const float* theirs = xch + (wave ^ 1) * 512 + lane * 4;
+    *(ck_f32x4*)mine = O;
+    if constexpr (MODE != CK_GLA) *(ck_f32x4*)(mine + 256) = Z;
+    ck_f32x4 k4[NT], b4[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int at = ck_col_slot(tb + t, g, m16) * 4;
+      k4[t] = *(const ck_f32x4*)(buf + It::K + at);
+      if constexpr (MODE == CK_GD) b4[t] = *(const ck_f32x4*)(buf + It::B + at);
+      S[t] *= *(const ck_f32x4*)(buf + It::GAM + (tb + t) * 16 + g * 4);
+    }
+    const int osq = MODE == CK_GD ? It::MB : It::M;
+    const ck_f32x4 o4 = *(const ck_f32x4*)(buf + osq + lane * 4);
+    __syncthreads();
+    O += *(const ck_f32x4*)theirs;
+    if constexpr (MODE != CK_GLA) Z += *(const ck_f32x4*)(theirs + 256);
+    // what is written with the k columns
+    const ck_f32x4 Y = MODE == CK_CD ? Z : V;
+    __builtin_amdgcn_sched_barrier(0);
+    put(nbuf, nf);
+    // tile by tile is a chain: step by step over the tiles is NT chains
+    ck_f32x4 P = zero;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (MODE == CK_GD) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(b4[t][i], Z[i], S[t],
+                                                      0, 0, 0);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[t][i], Y[i], S[t], 0,
+                                                    0, 0);
+      if constexpr (MODE != CK_GLA)
+        P = __builtin_amdgcn_mfma_f32_16x16x4f32(o4[i], Z[i], P, 0, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // products
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // an LDS write
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (ds == 0) {
+      if constexpr (MODE != CK_GLA) {
+        if (!fin) P = ck_square_terms(buf + osq, Z, zero, lane, tmp);
+        O += P;
+      }
+      const int left = rows_left(c);
+      float* dst = raw + (size_t)(t0 + 16 * (c0 + c) + 4 * g) * rs + hv;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i < left) dst[i * rs] = O[i];
+    }
+  };
+
+  float* buf0 = lds;
+  float* buf1 = lds + BUF;
+  ck_f32x4 fa[PF], fb[PF];
+  Vals va, vb;
+  fetch(0, fa, va);
+  fetch(1, fb, vb);
+  put(buf0, fa);
+  // all landed: the waits inside the loop then count its own loads only
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  // at the top: buf0 and va hold chunk c, fb and vb chunk c + 1
+  for (int c = 0; c < count; c += 2) {
+    walk(c, buf0, fa, va, buf1, fb);
+    if (c + 1 >= count) break;
+    __syncthreads();
+    walk(c + 1, buf1, fb, vb, buf0, fa);
+    if (c + 2 >= count) break;
+    __syncthreads();
+  }
+  if (col) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * (tb + t) + 4 * g + i;
+        if (d < D) Sg[(size_t)d * DV + j] = S[t][i];
+      }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// one decay per head and token
+// ---------------------------------------------------------------------------
+template <int DP>
+struct CkGroup {  // per chunk and group: fragments of Q and K
+  static constexpr int R = 0;
+  static constexpr int K = 16 * DP;
+  static constexpr int TOTAL = 32 * DP;
+};
+struct CkHead {  // per chunk and head
+  static constexpr int M = 0;     // 16 x 16 on V, fragment order
+  static constexpr int DR = 256;  // [16] decay from the chunk's start
+  static constexpr int DK = 272;  // [16] write scale and decay to its end
+  static constexpr int GAM = 288; // decay over the chunk
+  static constexpr int TOTAL = 292;
+};
+
+// Gates of the matrix LSTM: i = cap(wr + p0), f = logsigmoid(cap(dec + p1)),
+// m' = max(f + m, i); ga / gw / ge [T, H] = exp(f + m - m'), exp(i - m'),
+// exp(-m'). One wave per (segment, head); the running maximum over 64 tokens
+// is a scan over lanes of the maps m -> max(m + A, B).
+template <typename T>
+__global__ __launch_bounds__(64) void ck_gates_kernel(
+    float* __restrict__ ga, float* __restrict__ gw, float* __restrict__ ge,
+    const T* __restrict__ wr, int ldwr, const T* __restrict__ dec, int lddec,
+    const float* __restrict__ p0, const float* __restrict__ p1,
+    float* __restrict__ aux, const int* __restrict__ seq_rows, int H, int D,
+    float cap) {
+  const int seg = blockIdx.x / H, hd = blockIdx.x % H, lane = threadIdx.x;
+  const int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
+  const int pos0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  if (n < 16) return;
+  float* mp = aux + ((size_t)slot * H + hd) * (D + 1) + D;
+  float m = pos0 != 0 ? *mp : 0.f;
+  const float bi = p0[hd], bf = p1[hd];
+  for (int tb = 0; tb < n; tb += 64) {
+    const int tt = min(tb + lane, n - 1);
+    const size_t row = (size_t)(t0 + tt);
+    const float zi = MxElem<T>::ld(wr + row * ldwr + hd) + bi;
+    const float zf = MxElem<T>::ld(dec + row * lddec + hd) + bf;
+    const float ig = cap * tanhf(zi / cap);
+    const float fg = ck_log_sigmoid(cap * tanhf(zf / cap));
+    float A = fg, B = ig;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float a1 = __shfl_up(A, off, 64), b1 = __shfl_up(B, off, 64);
+      if (lane >= off) {
+        B = fmaxf(b1 + A, B);
+        A += a1;
+      }
+    }
+    const float mn = fmaxf(m + A, B);
+    float mo = __shfl_up(mn, 1, 64);
+    if (lane == 0) mo = m;
+    if (tb + lane < n) {
+      ga[row * H + hd] = expf(fg + mo - mn);
+      gw[row * H + hd] = expf(ig - mn);
+      ge[row * H + hd] = expf(-mn);
+    }
+    m = __shfl(mn, min(63, n - 1 - tb), 64);
+  }
+  if (lane == 0) *mp = m;
+}
+
+template <typename T, int MODE, int DP>
+__global__ __launch_bounds__(256) void ck_prep_scalar_kernel(
+    float* __restrict__ gitems, float* __restrict__ hitems, CkIn in,
+    const float* __restrict__ ga, const float* __restrict__ gw,
+    const int* __restrict__ seq_rows, int S_, int H, int G, int D,
+    float qscale, int c0, int nc) {
+  typedef CkGroup<DP> Gi;
+  constexpr int LD = DP + 4;
+  __shared__ __align__(16) float Q[16 * LD];
+  __shared__ __align__(16) float K[16 * LD];
+  __shared__ __align__(16) float qk[256];
+  __shared__ __align__(16) float sa[16][16];
+  __shared__ float sw[16][16];
+
+  const int item = blockIdx.x, grp = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int seg, chunk;
+  if (!ck_find(seq_rows, S_, item, c0, nc, lane, &seg, &chunk)) return;
+  const int n = seq_rows[4 * seg + 1];
+  const int row0 = seq_rows[4 * seg] + 16 * chunk;
+  const int nv = min(16, n - 16 * chunk);
+  const T* qp = (const T*)in.q + grp * D;
+  const T* kp = (const T*)in.k + grp * D;
+  for (int i = threadIdx.x; i < 16 * DP; i += 256) {
+    const int t = i / DP, d = i % DP;
+    const size_t row = (size_t)(row0 + min(t, nv - 1));
+    const int dc = min(d, D - 1);
+    const float q = MxElem<T>::ld(qp + row * in.ldq + dc);
+    const float k = MxElem<T>::ld(kp + row * in.ldk + dc);
+    const bool live = t < nv && d < D;
+    Q[t * LD + d] = live ? q * qscale : 0.f;
+    K[t * LD + d] = live ? k : 0.f;
+  }
+  __syncthreads();
+  const int g = lane >> 4, m16 = lane & 15;
+  if (wave == 0) {
+    ck_f32x4 c = {0.f, 0.f, 0.f, 0.f}, c2 = c;
+#pragma unroll
+    for (int t = 0; t < DP / 16; ++t) {
+      const ck_f32x4 x = *(const ck_f32x4*)(Q + m16 * LD + t * 16 + g * 4);
+      const ck_f32x4 y = *(const ck_f32x4*)(K + m16 * LD + t * 16 + g * 4);
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0], y[0], c, 0, 0, 0);
+      c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[1], y[1], c2, 0, 0, 0);
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[2], y[2], c, 0, 0, 0);
+      c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[3], y[3], c2, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      qk[((m16 >> 2) * 16 + 4 * g + i) * 4 + (m16 & 3)] = c[i] + c2[i];
+  }
+  if (blockIdx.z == 0) {
+    float* dst = gitems + ((size_t)item * G + grp) * Gi::TOTAL;
+    for (int f = threadIdx.x; f < DP * 4; f += 256) {  // float4 slots
+      const int t = f >> 6, fg = (f >> 4) & 3, fm = f & 15;
+      *(ck_f32x4*)(dst + Gi::R + ck_row_slot(t, fg, fm) * 4) =
+          *(const ck_f32x4*)(Q + fm * LD + t * 16 + fg * 4);
+      ck_f32x4 kk;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kk[i] = K[(4 * fg + i) * LD + t * 16 + fm];
+      *(ck_f32x4*)(dst + Gi::K + f * 4) = kk;
+    }
+  }
+  // this slice's heads, 16 at a time: their scalars, then the matrices
+  const int per = H / G;
+  const int slice = (per + gridDim.z - 1) / gridDim.z;
+  const int h1 = min(per, (int)(blockIdx.z + 1) * slice);
+  for (int hb = blockIdx.z * slice; hb < h1; hb += 16) {
+    __syncthreads();
+    {
+      const int hl = threadIdx.x & 15, t = threadIdx.x >> 4;
+      const int hd = grp * per + min(hb + hl, h1 - 1);
+      const size_t row = (size_t)(row0 + min(t, nv - 1));
+      float a, w;
+      if (MODE == CK_SSD) {
+        w = ck_softplus(
+            MxElem<T>::ld((const T*)in.dec + row * in.lddec + hd) +
+            in.p0[hd]);
+        a = expf(-expf(in.p1[hd]) * w);
+      } else {
+        a = ga[row * H + hd];
+        w = gw[row * H + hd];
+      }
+      sa[hl][t] = t < nv ? a : 1.f;
+      sw[hl][t] = t < nv ? w : 0.f;
+    }
+    __syncthreads();
+    // thread = entry of the matrix in fragment order
+    const int s = wave * 4 + (threadIdx.x & 3), t = (threadIdx.x >> 2) & 15;
+    const float dot = qk[threadIdx.x];
+    for (int hl = 0; hl < 16 && hb + hl < h1; ++hl) {
+      float e = 1.f;
+#pragma unroll
+      for (int j4 = 0; j4 < 4; ++j4) {
+        const ck_f32x4 a4 = *(const ck_f32x4*)(&sa[hl][j4 * 4]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = j4 * 4 + i;
+          e *= (j > s && j <= t) ? a4[i] : 1.f;
+        }
+      }
+      float* dst = hitems +
+                   ((size_t)item * H + grp * per + hb + hl) * CkHead::TOTAL;
+      dst[CkHead::M + threadIdx.x] = t >= s ? dot * e * sw[hl][s] : 0.f;
+      if (s == 0) dst[CkHead::DR + t] = e * sa[hl][0];
+      if (t == 15) dst[CkHead::DK + s] = e * sw[hl][s];
+      if (s == 0 && t == 15) dst[CkHead::GAM] = e * sa[hl][0];
+    }
+  }
+}
+
+// The walk of ck_sweep_kernel for one decay per head and token. out: the
+// finished fp32 rows of ssd, (o + skip v) silu(gate), or the raw read-outs
+// [T, H * (DV + 1)] of mlstm, whose column DV is the normaliser's (its values
+// are 1, its state lies in aux).
+template <typename T, int MODE, int DP>
+__global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
+    float* __restrict__ out, int ldo, const float* __restrict__ gitems,
+    const float* __restrict__ hitems, int cap, CkIn in,
+    const float* __restrict__ p2, float* __restrict__ state,
+    float* __restrict__ aux, const int* __restrict__ seq_rows, int S_, int H,
+    int G, int D, int DV, int c0, int nc) {
+  typedef CkGroup<DP> Gi;
+  constexpr int NT = DP / 32;
+  constexpr int PG = Gi::TOTAL / 1024;  // DP is a multiple of 32
+  constexpr int BUF = Gi::TOTAL + 512;  // fragments, then the head's
+  __shared__ __align__(16) float lds[2 * BUF];
+  __shared__ __align__(16) float xch[4 * 256];
+  __shared__ __align__(16) float tmps[4 * 256];
+  float* tmp = tmps + (threadIdx.x >> 6) * 256;
+
+  const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H);
+  const int seg = sh / H, hd = sh % H, grp = hd / (H / G);
+  const int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
+  const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  int count = ck_count(n, c0, nc);
+  if (count == 0) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int first = 0;
+  for (int s = lane; s < seg; s += 64)
+    first += ck_count(seq_rows[4 * s + 1], c0, nc);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
+  first = __builtin_amdgcn_readfirstlane(first);
+  count = __builtin_amdgcn_readfirstlane(min(count, cap - first));
+  if (count <= 0) return;
+
+  const int g = lane >> 4, m16 = lane & 15;
+  const int ct = wave >> 1, ds = wave & 1, tb = ds * NT;
+  const int j = cb * 32 + ct * 16 + m16;
+  const bool col = j < DV;
+  const bool ncol = MODE == CK_MLSTM && j == DV;
+  const int hv = hd * DV + (col ? j : 0);
+  float* Sg = state + ((size_t)slot * H + hd) * (size_t)D * DV + j;
+  float* Ng = MODE == CK_MLSTM ? aux + ((size_t)slot * H + hd) * (D + 1)
+                               : nullptr;
+  ck_f32x4 S[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = 16 * (tb + t) + 4 * g + i;
+      float x = 0.f;
+      if (d < D && (p0 != 0 || c0 != 0)) {
+        if (col) x = Sg[(size_t)d * DV];
+        if (ncol) x = Ng[d];
+      }
+      S[t][i] = x;
+    }
+
+  const char* gsrc =
+      (const char*)(gitems + ((size_t)first * G + grp) * Gi::TOTAL);
+  const char* hsrc =
+      (const char*)(hitems + ((size_t)first * H + hd) * CkHead::TOTAL);
+  const size_t gstep = (size_t)G * Gi::TOTAL * sizeof(float);
+  const size_t hstep = (size_t)H * CkHead::TOTAL * sizeof(float);
+  const unsigned at16 = threadIdx.x * 16;
+  const unsigned ath = min((int)threadIdx.x, CkHead::TOTAL / 4 - 1) * 16;
+  const T* vcol = (const T*)in.v + (size_t)t0 * in.ldv + hv;
+  const T* gcol = (const T*)in.gate + (size_t)t0 * in.ldg + hv;
+  const float skip = MODE == CK_SSD ? p2[hd] : 0.f;
+  struct Next {
+    ck_f32x4 f[PG], h;
+    T v[4], gt[4];
+  };
+  auto fetch = [&](int c, Next& x) {
+    c = min(c, count - 1);
+#pragma unroll
+    for (int u = 0; u < PG; ++u)
+      x.f[u] = *(const ck_f32x4*)(gsrc + c * gstep + u * 4096 + at16);
+    x.h = *(const ck_f32x4*)(hsrc + c * hstep + ath);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int tt = min(16 * (c0 + c) + 4 * g + i, n - 1);
+      x.v[i] = vcol[(size_t)tt * in.ldv];
+      if (MODE == CK_SSD) x.gt[i] = gcol[(size_t)tt * in.ldg];
+    }
+  };
+  auto put = [&](float* dst, const Next& x) {
+#pragma unroll
+    for (int u = 0; u < PG; ++u)
+      *(ck_f32x4*)(dst + u * 1024 + threadIdx.x * 4) = x.f[u];
+    if (threadIdx.x < 128)
+      *(ck_f32x4*)(dst + Gi::TOTAL + threadIdx.x * 4) = x.h;
+  };
+  auto walk = [&](int c, const float* buf, Next& x, float* nbuf,
+                  const Next& nx) {
+    const float* hb = buf + Gi::TOTAL;
+    const int left = n - 16 * (c0 + c) - 4 * g;
+    ck_f32x4 V, gt;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float y = MxElem<T>::ld(&x.v[i]);
+      if (MODE == CK_MLSTM) y = col ? y : (ncol ? 1.f : 0.f);
+      V[i] = i < left && (MODE == CK_MLSTM || col) ? y : 0.f;
+      gt[i] = MODE == CK_SSD ? MxElem<T>::ld(&x.gt[i]) : 0.f;
+    }
+    ck_f32x4 r4[NT], k4[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      r4[t] = *(const ck_f32x4*)(buf + Gi::R + ck_row_slot(tb + t, g, m16) * 4);
+      k4[t] = *(const ck_f32x4*)(buf + Gi::K + ck_col_slot(tb + t, g, m16) * 4);
+    }
+    const ck_f32x4 q4 = *(const ck_f32x4*)(hb + CkHead::M + lane * 4);
+    const ck_f32x4 dr = *(const ck_f32x4*)(hb + CkHead::DR + g * 4);
+    const ck_f32x4 dk = *(const ck_f32x4*)(hb + CkHead::DK + g * 4);
+    const float gam = hb[CkHead::GAM];
+    const bool fin = !__any(!ck_finite(V));
+    fetch(c + 2, x);
+    put(nbuf, nx);
+    const ck_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    ck_f32x4 O = zero, Z = zero, X = zero;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        O = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i], S[t][i], O, 0, 0,
+                                                 0);
+        Z = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i + 1], S[t][i + 1], Z,
+                                                 0, 0, 0);
+      }
+    const ck_f32x4 W = V * dk;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) S[t] *= gam;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[t][i], W[i], S[t], 0,
+                                                    0, 0);
+      X = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[i], V[i], X, 0, 0, 0);
+    }
+    O += Z;
+    if (ds == 1) *(ck_f32x4*)(xch + ct * 256 + lane * 4) = O;
+    if (!fin) X = ck_square_terms(hb + CkHead::M, V, zero, lane, tmp);
+    // also: this chunk's buffer is read, the next one's is filled
+    __syncthreads();
+    if (ds == 0 && (col || ncol)) {
+      O = (O + *(const ck_f32x4*)(xch + ct * 256 + lane * 4)) * dr + X;
+      const size_t row = (size_t)(t0 + 16 * (c0 + c) + 4 * g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i < left) {
+          if (MODE == CK_SSD)
+            out[(row + i) * ldo + hv] =
+                (O[i] + skip * V[i]) * gt[i] * ck_sigmoid(gt[i]);
+          else
+            out[(row + i) * ldo + hd * (DV + 1) + j] = O[i];
+        }
+      }
+    }
+  };
+  Next xa, xb;
+  fetch(0, xa);
+  fetch(1, xb);
+  put(lds, xa);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  for (int c = 0; c < count; c += 2) {
+    walk(c, lds, xa, lds + BUF, xb);
+    if (c + 1 >= count) break;
+    // the exchange of the chunk before is read by then
+    __syncthreads();
+    walk(c + 1, lds + BUF, xb, lds, xa);
+    if (c + 2 >= count) break;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = 16 * (tb + t) + 4 * g + i;
+      if (d < D) {
+        if (col) Sg[(size_t)d * DV] = S[t][i];
+        if (ncol) Ng[d] = S[t][i];
+      }
+    }
+}
+
+// Read-out norm and gate: o / rms_DV(o) * weight * gate for the rows of
+// segments that the sweep walked. A wave takes four heads of a row; a lane
+// holds VEC neighbouring columns of each, 64 * VEC >= DV.
+template <typename T, int MODE, int VEC>
+__global__ __launch_bounds__(256) void ck_readout_kernel(
+    T* __restrict__ out, int ldo, const float* __restrict__ raw,
+    const T* __restrict__ gate, int ldg, const float* __restrict__ normw,
+    const int* __restrict__ seq_rows, int S_, int H, int DV, float eps,
+    const float* __restrict__ ge) {
+  // the matrix LSTM's rows carry n.q behind a head's columns
+  constexpr int EXTRA = MODE == CK_MLSTM ? 1 : 0;
+  const int t = blockIdx.x, lane = threadIdx.x & 63;
+  const int h0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * 4;
+  // rows of short segments are not this kernel's
+  bool mine = false;
+  for (int s0 = 0; s0 < S_ && !mine; s0 += 64) {
+    const int s = s0 + lane;
+    bool hit = false;
+    if (s < S_) {
+      const int a = seq_rows[4 * s], n = seq_rows[4 * s + 1];
+      hit = n >= 16 && t >= a && t < a + n;
+    }
+    mine = __any(hit);
+  }
+  if (!mine) return;
+  const float* r = raw + (size_t)t * ((size_t)H * (DV + EXTRA));
+  const T* gp = gate + (size_t)t * ldg;
+  T* op = out + (size_t)t * ldo;
+  const int c0 = lane * VEC;
+  float o[4][VEC], gv[4][VEC], nw[4][VEC], den[4];
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const int hd = min(h0 + h, H - 1);
+#pragma unroll
+    for (int u = 0; u < VEC; ++u) {
+      const int c = min(c0 + u, DV - 1);
+      o[h][u] = r[hd * (DV + EXTRA) + c];
+      gv[h][u] = MxElem<T>::ld(gp + hd * DV + c);
+      nw[h][u] =
+          normw[(MODE == CK_GD || MODE == CK_MLSTM ? hd * DV : 0) + c];
+    }
+    if (MODE == CK_MLSTM)
+      den[h] = fmaxf(fabsf(r[hd * (DV + 1) + DV]), ge[(size_t)t * H + hd]) +
+               1e-6f;
+  }
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    float ss = 0.f;
+    if (MODE == CK_MLSTM) {
+#pragma unroll
+      for (int u = 0; u < VEC; ++u) o[h][u] /= den[h];
+    }
+#pragma unroll
+    for (int u = 0; u < VEC; ++u)
+      if (c0 + u < DV) ss += o[h][u] * o[h][u];
+    ss = mx_wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)DV + eps);
+#pragma unroll
+    for (int u = 0; u < VEC; ++u) {
+      const float g = gv[h][u];
+      float gt = ck_sigmoid(g);
+      if (MODE == CK_GLA) gt *= g;
+      if (h0 + h < H && c0 + u < DV)
+        MxElem<T>::st(op + (h0 + h) * DV + c0 + u,
+                      o[h][u] * inv * nw[h][u] * gt);
+    }
+  }
+}
+
+// Key width as the kernels pad it (0: not built).
+static int ck_pad(int D) {
+  const int pads[] = {32, 64, 96, 128};
+  for (int p : pads)
+    if (D <= p) return p;
+  return 0;
+}
+
+// Floats per chunk: of all heads' (and groups') operands.
+static long ck_chunk_floats(int mode, int dp, int H, int G) {
+  if (mode >= CK_SSD)
+    return (long)G * 32 * dp + (long)H * CkHead::TOTAL;
+  const int rows = mode == CK_GD ? 4 : (mode == CK_CD ? 3 : 2);
+  const int sq = mode == CK_GD ? 3 : (mode == CK_CD ? 2 : 1);
+  return H * ((long)rows * 16 * dp + sq * 256 + dp + 4);
+}
+
+// Measured (bf16, one MI355X, whole operation; token by token -> this form):
+//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 1.00 ms
+//     (operands 0.24, walk 0.73: 2.2 us a chunk, of which the products take
+//     1.0 and the issue of loads and LDS writes most of the rest; read-out
+//     0.08)
+//   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
+//                                                            5.42 -> 0.70 ms
+//   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.64 ms
+//   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.15 ms
+//   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.84 ms
+// From 16 rows on a segment goes this way: one chunk costs about 15 us in
+// three launches, 16 tokens one by one 24 us.
+//
+// Chunks laid down at once and the chunks of a segment per pass. A step's
+// segments of 16 rows and more have at most T / 16 + S chunks, and at most
+// T / 8; passes keep the scratch below CK_BYTES.
+#define CK_BYTES (1l << 30)
+static void ck_plan(int mode, int T_, int S_, int H, int G, int D, int* cap,
+                    int* nc, int* passes) {
+  const long per = ck_chunk_floats(mode, ck_pad(D), H, G) * 4;
+  long all = (long)T_ / 16 + S_;
+  if (all > T_ / 8 + 1) all = T_ / 8 + 1;
+  long fit = CK_BYTES / per;
+  if (fit < S_) fit = S_;
+  const int longest = (T_ - S_ + 1 + 15) / 16;  // chunks of one segment
+  if (all <= fit) {
+    *cap = (int)all;
+    *nc = longest > 0 ? longest : 1;
+    *passes = 1;
+    return;
+  }
+  *nc = (int)(fit / S_);
+  *cap = (int)((long)*nc * S_ < all ? (long)*nc * S_ : all);
+  *passes = (longest + *nc - 1) / *nc;
+}
+
+#define CK_ARGS                                                              \
+  void *out, int ldo, CkIn in, const void *normw, const void *p2,            \
+      void *state, void *aux,                                                \
+      const void *seq_rows, int S_, int T_, int H, int G, int D, int DV,     \
+      float eps, float scale, float c0f, float *scratch, hipStream_t stream
+
+#define CK_PASS                                                              \
+  out, ldo, in, normw, p2, state, aux, seq_rows, S_, T_, H, G, D, DV, eps,   \
+      scale, c0f, scratch, stream
+
+// Floats of scratch per row: raw read-outs, and the matrix LSTM's gates.
+static long ck_rows_floats(int mode, int T_, int H, int DV) {
+  if (mode == CK_SSD) return 0;
+  return (long)T_ * H * (mode == CK_MLSTM ? DV + 4 : DV);
+}
+
+template <typename T, int MODE>
+static void ck_read(CK_ARGS, const float* raw, const float* gx) {
+#define CK_READ(VEC)                                                         \
+  hipLaunchKernelGGL((ck_readout_kernel<T, MODE, VEC>),                      \
+                     dim3(T_, (H + 15) / 16), dim3(256), 0, stream, (T*)out, \
+                     ldo, raw, (const T*)in.gate, in.ldg,                    \
+                     (const float*)normw, (const int*)seq_rows, S_, H, DV,   \
+                     eps, gx)
+  if (DV <= 64)
+    CK_READ(1);
+  else if (DV <= 128)
+    CK_READ(2);
+  else
+    CK_READ(4);
+#undef CK_READ
+}
+
+template <typename T, int MODE, int DP>
+static int ck_launch(CK_ARGS) {
+  typedef CkItem<MODE, DP> It;
+  int cap, nc, passes;
+  ck_plan(MODE, T_, S_, H, G, D, &cap, &nc, &passes);
+  float* raw = scratch;
+  float* items = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
+  const int ncb = (DV + 31) / 32;
+  const size_t lds =
+      (2 * ((It::TOTAL + 1023) / 1024) * 1024 + 2048 + 1024) * sizeof(float);
+  if (lds > 65536 &&
+      hipFuncSetAttribute((const void*)ck_sweep_kernel<T, MODE, DP>,
+                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)lds) != hipSuccess)
+    return 1;
+  for (int p = 0; p < passes; ++p) {
+    hipLaunchKernelGGL((ck_prep_kernel<T, MODE, DP>), dim3(cap, H), dim3(256),
+                       0, stream, items, in, (const int*)seq_rows, S_, H, G,
+                       D, scale, c0f, p * nc, nc);
+    hipLaunchKernelGGL((ck_sweep_kernel<T, MODE, DP>), dim3(S_ * H * ncb),
+                       dim3(256), lds, stream, raw, items, cap,
+                       (const T*)in.v, in.ldv, (float*)state,
+                       (const int*)seq_rows, S_, H, D, DV, p * nc, nc);
+  }
+  ck_read<T, MODE>(CK_PASS, raw, nullptr);
+  return 0;
+}
+
+template <typename T, int MODE, int DP>
+static int ck_launch_scalar(CK_ARGS) {
+  int cap, nc, passes;
+  ck_plan(MODE, T_, S_, H, G, D, &cap, &nc, &passes);
+  const bool lstm = MODE == CK_MLSTM;
+  float* raw = scratch;
+  float* ga = raw + (lstm ? (size_t)T_ * H * (DV + 1) : 0);
+  float* gw = ga + (lstm ? (size_t)T_ * H : 0);
+  float* ge = gw + (lstm ? (size_t)T_ * H : 0);
+  float* gitems = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
+  float* hitems = gitems + (size_t)cap * G * CkGroup<DP>::TOTAL;
+  const int ncb = (DV + (lstm ? 1 : 0) + 31) / 32;
+  if (lstm)
+    hipLaunchKernelGGL((ck_gates_kernel<T>), dim3(S_ * H), dim3(64), 0,
+                       stream, ga, gw, ge, (const T*)in.a, in.lda,
+                       (const T*)in.dec, in.lddec, in.p0, in.p1, (float*)aux,
+                       (const int*)seq_rows, H, D, c0f);
+  // a group's heads over a few blocks where there are many
+  const int slices = (H / G + 31) / 32;
+  for (int p = 0; p < passes; ++p) {
+    hipLaunchKernelGGL((ck_prep_scalar_kernel<T, MODE, DP>),
+                       dim3(cap, G, slices), dim3(256), 0, stream, gitems,
+                       hitems, in, ga, gw, (const int*)seq_rows, S_, H, G, D,
+                       scale, p * nc, nc);
+    hipLaunchKernelGGL((ck_sweep_scalar_kernel<T, MODE, DP>),
+                       dim3(S_ * H * ncb), dim3(256), 0, stream,
+                       lstm ? raw : (float*)out,
+                       lstm ? H * (DV + 1) : ldo, gitems, hitems, cap, in,
+                       (const float*)p2, (float*)state, (float*)aux,
+                       (const int*)seq_rows, S_, H, G, D, DV, p * nc, nc);
+  }
+  if constexpr (MODE == CK_MLSTM) ck_read<T, MODE>(CK_PASS, raw, ge);
+  return 0;
+}
+
+template <typename T, int MODE>
+static int ck_dispatch(CK_ARGS) {
+  switch (ck_pad(D)) {
+#define CK_CASE(DP)                                                         \
+  case DP:                                                                  \
+    if constexpr (MODE >= CK_SSD)                                           \
+      return ck_launch_scalar<T, MODE, DP>(CK_PASS);                        \
+    else                                                                    \
+      return ck_launch<T, MODE, DP>(CK_PASS);
+    CK_CASE(32)
+    CK_CASE(64)
+    CK_CASE(96)
+    CK_CASE(128)
+  }
+  return 1;
+}
+
+// One unit per form (CK_ONLY), so they build in parallel; unit 0 also
+// carries the entry points.
+#define CK_UNIT(NAME) extern "C" int NAME(int dtype, CK_ARGS)
+CK_UNIT(ck_general);
+CK_UNIT(ck_channel);
+CK_UNIT(ck_gla);
+CK_UNIT(ck_ssd);
+CK_UNIT(ck_mlstm);
+#define CK_BODY(MODE)                                                       \
+  {                                                                         \
+    if (dtype == MX_BF16) return ck_dispatch<mx_bf16, MODE>(CK_PASS);       \
+    return ck_dispatch<float, MODE>(CK_PASS);                               \
+  }
+#if !defined(CK_ONLY) || CK_ONLY == 0
+CK_UNIT(ck_general) CK_BODY(CK_GD)
+#endif
+#if !defined(CK_ONLY) || CK_ONLY == 1
+CK_UNIT(ck_channel) CK_BODY(CK_CD)
+#endif
+#if !defined(CK_ONLY) || CK_ONLY == 2
+CK_UNIT(ck_gla) CK_BODY(CK_GLA)
+#endif
+#if !defined(CK_ONLY) || CK_ONLY == 3
+CK_UNIT(ck_ssd) CK_BODY(CK_SSD)
+#endif
+#if !defined(CK_ONLY) || CK_ONLY == 4
+CK_UNIT(ck_mlstm) CK_BODY(CK_MLSTM)
+#endif
+
+#if !defined(CK_ONLY) || CK_ONLY == 0
+// Floats of scratch that the chunk form needs for a step of T_ rows in S_
+// segments, 0 where it does not cover it (no segment of 16 rows can be among
+// them, or the head widths are not built).
+extern "C" long mx_chunk_scratch(int mode, int T_, int S_, int H, int G,
+                                 int D, int DV) {
+  if (S_ <= 0 || T_ - S_ + 1 < 16 || ck_pad(D) == 0 || DV > 256) return 0;
+  int cap, nc, passes;
+  ck_plan(mode, T_, S_, H, G, D, &cap, &nc, &passes);
+  return ((ck_rows_floats(mode, T_, H, DV) + 3) & ~3l) +
+         cap * ck_chunk_floats(mode, ck_pad(D), H, G);
+}
+
+extern "C" int mx_chunk_delta(void* out, int ldo, const void* r, int ldr,
+                              const void* k, int ldk, const void* v, int ldv,
+                              const void* zw, int ldzw, const void* za,
+                              int ldza, const void* g, int ldg,
+                              const void* w0, const void* ab,
+                              const void* normw, void* state,
+                              const void* seq_rows, int S_, int T_, int H,
+                              int D, float eps, float decay_scale,
+                              void* scratch, int dtype, void* stream) {
+  CkIn in = {r, k, v, zw, za, g, ldr, ldk, ldv, ldzw, ldza, ldg,
+             (const float*)w0, (const float*)ab};
+  return ck_general(dtype, out, ldo, in, normw, nullptr, state, nullptr,
+                    seq_rows, S_, T_, H, H, D, D, eps, decay_scale, 0.f,
+                    (float*)scratch, (hipStream_t)stream);
+}
+
+extern "C" int mx_chunk_gated(void* out, int ldo, const void* q, int ldq,
+                              const void* k, int ldk, const void* v, int ldv,
+                              const void* beta, int ldb, const void* zdec,
+                              int ldzd, const void* zgate, int ldzg,
+                              const void* a_log, const void* dt_bias,
+                              const void* normw, void* state,
+                              const void* seq_rows, int S_, int T_, int H,
+                              int G, int D, int DV, float eps, float qscale,
+                              void* scratch, int dtype, void* stream) {
+  CkIn in = {q, k, v, zdec, beta, zgate, ldq, ldk, ldv, ldzd, ldb, ldzg,
+             (const float*)dt_bias, (const float*)a_log};
+  return ck_channel(dtype, out, ldo, in, normw, nullptr, state, nullptr,
+                    seq_rows, S_, T_, H, G, D, DV, eps, qscale, 0.f,
+                    (float*)scratch, (hipStream_t)stream);
+}
+
+// mode: 0 gla, 1 ssd, 2 mlstm, arguments as mx_linear_scan's
+extern "C" int mx_chunk_scan(
+    int mode, void* out, int ldo, const void* q, int ldq, const void* k,
+    int ldk, const void* v, int ldv, const void* dec, int lddec,
+    const void* wr, int ldwr, const void* gate, int ldg, const void* p0,
+    const void* p1, const void* p2, const void* normw, void* state, void* aux,
+    const void* seq_rows, int S_, int T_, int H, int G, int D, int DV,
+    float eps, float qscale, float c0, void* scratch, int dtype,
+    void* stream) {
+  CkIn in = {q, k, v, dec, wr, gate, ldq, ldk, ldv, lddec, ldwr, ldg,
+             (const float*)p0, (const float*)p1};
+#define CK_SCAN                                                              \
+  (dtype, out, ldo, in, normw, p2, state, aux, seq_rows, S_, T_, H, G, D,    \
+   DV, eps, qscale, c0, (float*)scratch, (hipStream_t)stream)
+  switch (mode) {
+    case 0: return ck_gla CK_SCAN;
+    case 1: return ck_ssd CK_SCAN;
+    case 2: return ck_mlstm CK_SCAN;
+  }
+  return 1;
+}
+#endif

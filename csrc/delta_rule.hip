@@ -20,6 +20,10 @@
 // cooperatively into LDS (stored so that each lane's rows are contiguous),
 // then each thread walks the tile's tokens with broadcast LDS reads and no
 // barrier.
+//
+// Segments of nmax rows and more are left to the chunk-parallel kernels
+// (chunk_scan.hip); this form takes single tokens, portions shorter than a
+// chunk and key widths those are not built for.
 #include "mix_common.h"
 
 template <typename T, int DKP, int TILE, int P>
@@ -31,7 +35,7 @@ void delta_rule_kernel(
     const T* __restrict__ g, int ldg, const float* __restrict__ w0,
     const float* __restrict__ ab, const float* __restrict__ normw,
     float* __restrict__ state, const int* __restrict__ seq_rows, int H, int D,
-    float eps, float decay_scale) {
+    float eps, float decay_scale, int nmax) {
   extern __shared__ __align__(16) float lds[];
   constexpr int R = DKP / P;        // rows per lane
   // a lane's R rows are contiguous; the P segments of a token are RP words
@@ -49,6 +53,7 @@ void delta_rule_kernel(
   const int seg = blockIdx.x / H, hd = blockIdx.x % H;
   const int t0 = seq_rows[4 * seg + 0], n = seq_rows[4 * seg + 1];
   const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  if (n >= nmax) return;  // the chunk kernels' segments
   const int j = threadIdx.x / P, p = threadIdx.x % P;
   const bool col = j < D;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -213,7 +218,8 @@ static void launch_delta(void* out, int ldo, const void* r, int ldr,
                          const void* g, int ldg, const void* w0,
                          const void* ab, const void* normw, void* state,
                          const void* seq_rows, int S_, int H, int D,
-                         float eps, float decay_scale, hipStream_t stream) {
+                         float eps, float decay_scale, int nmax,
+                         hipStream_t stream) {
   constexpr int TILE = DKP <= 128 ? 16 : 8;
   constexpr int P = DKP >= 64 ? 4 : (DKP >= 32 ? 2 : 1);
   const int threads = ((D * P + 63) / 64) * 64;
@@ -226,14 +232,14 @@ static void launch_delta(void* out, int ldo, const void* r, int ldr,
                      ldzw, (const T*)za, ldza, (const T*)g, ldg,
                      (const float*)w0, (const float*)ab,
                      (const float*)normw, (float*)state,
-                     (const int*)seq_rows, H, D, eps, decay_scale);
+                     (const int*)seq_rows, H, D, eps, decay_scale, nmax);
 }
 
 #define DR_CASE(P)                                                          \
   if (D <= P) {                                                             \
     launch_delta<T, P>(out, ldo, r, ldr, k, ldk, v, ldv, zw, ldzw, za,      \
                        ldza, g, ldg, w0, ab, normw, state, seq_rows, S_, H, \
-                       D, eps, decay_scale, (hipStream_t)stream);           \
+                       D, eps, decay_scale, nmax, (hipStream_t)stream);     \
     return 0;                                                               \
   }
 
@@ -244,7 +250,8 @@ static int dispatch_delta(void* out, int ldo, const void* r, int ldr,
                           const void* g, int ldg, const void* w0,
                           const void* ab, const void* normw, void* state,
                           const void* seq_rows, int S_, int H, int D,
-                          float eps, float decay_scale, void* stream) {
+                          float eps, float decay_scale, int nmax,
+                          void* stream) {
   DR_CASE(16)
   DR_CASE(32)
   DR_CASE(48)
@@ -266,10 +273,10 @@ static int dispatch_delta(void* out, int ldo, const void* r, int ldr,
       const void *v, int ldv, const void *zw, int ldzw, const void *za,      \
       int ldza, const void *g, int ldg, const void *w0, const void *ab,      \
       const void *normw, void *state, const void *seq_rows, int S_, int H,   \
-      int D, float eps, float decay_scale, void *stream
+      int D, float eps, float decay_scale, int nmax, void *stream
 #define DR_PASS                                                              \
   out, ldo, r, ldr, k, ldk, v, ldv, zw, ldzw, za, ldza, g, ldg, w0, ab,      \
-      normw, state, seq_rows, S_, H, D, eps, decay_scale, stream
+      normw, state, seq_rows, S_, H, D, eps, decay_scale, nmax, stream
 
 extern "C" int mx_delta_rule_bf16(DR_ARGS);
 extern "C" int mx_delta_rule_f32(DR_ARGS);
@@ -291,15 +298,15 @@ extern "C" int mx_delta_rule(void* out, int ldo, const void* r, int ldr,
                              const void* w0, const void* ab,
                              const void* normw, void* state,
                              const void* seq_rows, int S_, int H, int D,
-                             float eps, float decay_scale, int dtype,
-                             void* stream) {
+                             float eps, float decay_scale, int nmax,
+                             int dtype, void* stream) {
   if (S_ <= 0) return 0;
   if (dtype == MX_BF16)
     return mx_delta_rule_bf16(out, ldo, r, ldr, k, ldk, v, ldv, zw, ldzw, za,
                               ldza, g, ldg, w0, ab, normw, state, seq_rows,
-                              S_, H, D, eps, decay_scale, stream);
+                              S_, H, D, eps, decay_scale, nmax, stream);
   return mx_delta_rule_f32(out, ldo, r, ldr, k, ldk, v, ldv, zw, ldzw, za,
                            ldza, g, ldg, w0, ab, normw, state, seq_rows, S_,
-                           H, D, eps, decay_scale, stream);
+                           H, D, eps, decay_scale, nmax, stream);
 }
 #endif

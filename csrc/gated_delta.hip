@@ -23,6 +23,10 @@
 // cooperatively into LDS (each lane's rows contiguous, segments padded
 // against bank conflicts), then each thread walks the tile's tokens with
 // broadcast LDS reads and no barrier.
+//
+// Segments of nmax rows and more are left to the chunk-parallel kernels
+// (chunk_scan.hip); this form takes single tokens, portions shorter than a
+// chunk and widths those are not built for.
 #include "mix_common.h"
 
 PS_DEV float mx_softplus(float z) {
@@ -37,7 +41,7 @@ __global__ __launch_bounds__(MAXT) void gated_delta_kernel(
     const T* __restrict__ zgate, int ldzg, const float* __restrict__ a_log,
     const float* __restrict__ dt_bias, const float* __restrict__ normw,
     float* __restrict__ state, const int* __restrict__ seq_rows, int H, int G,
-    int D, int DV, float eps, float qscale) {
+    int D, int DV, float eps, float qscale, int nmax) {
   extern __shared__ __align__(16) float lds[];
   constexpr int R = DKP / P;        // rows per lane
   constexpr int RP = P > 1 ? R + 4 : R;
@@ -52,6 +56,7 @@ __global__ __launch_bounds__(MAXT) void gated_delta_kernel(
   const int seg = blockIdx.x / H, hd = blockIdx.x % H;
   const int t0 = seq_rows[4 * seg + 0], n = seq_rows[4 * seg + 1];
   const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  if (n >= nmax) return;  // the chunk kernels' segments
   const int j = threadIdx.x / P, p = threadIdx.x % P;
   const bool col = j < DV;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -266,11 +271,11 @@ __global__ __launch_bounds__(MAXT) void gated_delta_kernel(
       int ldzd, const void *zgate, int ldzg, const void *a_log,              \
       const void *dt_bias, const void *normw, void *state,                   \
       const void *seq_rows, int S_, int H, int G, int D, int DV, float eps,  \
-      float qscale, void *stream
+      float qscale, int nmax, void *stream
 #define GD_PASS                                                              \
   out, ldo, q, ldq, k, ldk, v, ldv, beta, ldb, zdec, ldzd, zgate, ldzg,      \
       a_log, dt_bias, normw, state, seq_rows, S_, H, G, D, DV, eps, qscale,  \
-      stream
+      nmax, stream
 
 template <typename T, int DKP>
 static int launch_gated_delta(GD_ARGS) {
@@ -291,7 +296,7 @@ static int launch_gated_delta(GD_ARGS) {
                      ldzd, (const T*)zgate, ldzg, (const float*)a_log,       \
                      (const float*)dt_bias, (const float*)normw,             \
                      (float*)state, (const int*)seq_rows, H, G, D, DV, eps,  \
-                     qscale)
+                     qscale, nmax)
   // the launch bound follows the thread count, so small launches get the
   // registers for the prefetched tile and a lane's rows stay out of scratch
   if (threads <= 256) {
@@ -343,7 +348,7 @@ extern "C" int mx_gated_delta(
     int ldzd, const void* zgate, int ldzg, const void* a_log,
     const void* dt_bias, const void* normw, void* state,
     const void* seq_rows, int S_, int H, int G, int D, int DV, float eps,
-    float qscale, int dtype, void* stream) {
+    float qscale, int nmax, int dtype, void* stream) {
   if (S_ <= 0) return 0;
   if (dtype == MX_BF16) return mx_gated_delta_bf16(GD_PASS);
   return mx_gated_delta_f32(GD_PASS);

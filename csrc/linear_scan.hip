@@ -36,6 +36,10 @@
 // itself). The read-out norm, which spans the head, then runs as a second
 // kernel over an fp32 scratch, and the new normaliser and maximum wait in
 // scratch until then: a part that starts late must still find the old ones.
+//
+// Segments of nmax rows and more are left to the chunk-parallel kernels
+// (chunk_scan.hip); this form takes single tokens, portions shorter than a
+// chunk and widths those are not built for.
 #include "mix_common.h"
 
 #define LS_GLA 0
@@ -59,7 +63,7 @@ __global__ __launch_bounds__(MAXT) void linear_scan_kernel(
     const float* __restrict__ normw, float* __restrict__ state,
     float* __restrict__ aux, const int* __restrict__ seq_rows, int H, int G,
     int D, int DV, float eps, float qscale, float c0, int CS, int DVB,
-    float* __restrict__ raw, float* __restrict__ naux) {
+    float* __restrict__ raw, float* __restrict__ naux, int nmax) {
   extern __shared__ __align__(16) float lds[];
   constexpr int R = DKP / P;        // rows per lane
   constexpr int RP = P > 1 ? R + 4 : R;
@@ -80,6 +84,7 @@ __global__ __launch_bounds__(MAXT) void linear_scan_kernel(
   const int seg = sh / H, hd = sh % H;
   const int t0 = seq_rows[4 * seg + 0], n = seq_rows[4 * seg + 1];
   const int pos0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  if (n >= nmax) return;  // the chunk kernels' segments
   const int jl = threadIdx.x / P, p = threadIdx.x % P;
   const int nloc = min(DVB, DV - cb * DVB);           // columns of this block
   const int j = cb * DVB + jl;
@@ -298,18 +303,29 @@ __global__ __launch_bounds__(256) void scan_readout_kernel(
     const T* __restrict__ gate, int ldg, const float* __restrict__ normw,
     int T_, int H, int DV, float eps, const float* __restrict__ naux,
     float* __restrict__ aux, const int* __restrict__ seq_rows, int S_,
-    int D) {
+    int D, int nmax) {
   const int w = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  if (w >= T_ * H) return;
-  if (naux != nullptr && w < S_ * H) {
+  // rows are enumerated one by one, or, where the chunk kernels have the
+  // longer segments, as the at most nmax - 1 rows of every segment
+  const bool all = nmax > T_;
+  if (w >= (all ? T_ : S_ * (nmax - 1)) * H) return;
+  if (naux != nullptr && w < S_ * H &&
+      seq_rows[4 * (w / H) + 1] < nmax) {
     // the matrix LSTM's new normaliser and maximum move into their slot
     const int slot = seq_rows[4 * (w / H) + 3];
     const float* src = naux + (size_t)w * (D + 1);
     float* dst = aux + ((size_t)slot * H + w % H) * (D + 1);
     for (int c = lane; c <= D; c += 64) dst[c] = src[c];
   }
-  const int t = w / H, hd = w % H, hv = hd * DV;
+  int t = w / H;
+  const int hd = w % H, hv = hd * DV;
+  if (!all) {
+    const int seg = t / (nmax - 1), i = t % (nmax - 1);
+    const int n = seq_rows[4 * seg + 1];
+    if (n >= nmax || i >= n) return;
+    t = seq_rows[4 * seg] + i;
+  }
   const float* r = raw + (size_t)t * ((size_t)H * DV) + hv;
   float ss = 0.f;
   for (int c = lane; c < DV; c += 64) ss += r[c] * r[c];
@@ -330,11 +346,11 @@ __global__ __launch_bounds__(256) void scan_readout_kernel(
       int ldwr, const void *gate, int ldg, const void *p0, const void *p1,   \
       const void *p2, const void *normw, void *state, void *aux,             \
       const void *seq_rows, int S_, int H, int G, int D, int DV, float eps,  \
-      float qscale, float c0, int T_, void *raw, void *stream
+      float qscale, float c0, int T_, void *raw, int nmax, void *stream
 #define LS_PASS                                                              \
   out, ldo, q, ldq, k, ldk, v, ldv, dec, lddec, wr, ldwr, gate, ldg, p0, p1, \
       p2, normw, state, aux, seq_rows, S_, H, G, D, DV, eps, qscale, c0,     \
-      T_, raw, stream
+      T_, raw, nmax, stream
 
 // Key width as the kernels pad it (0: not built).
 static int ls_pad(int D) {
@@ -388,7 +404,7 @@ static int launch_linear_scan_p(LS_ARGS, int CS) {
       (const T*)dec, lddec, (const T*)wr, ldwr, (const T*)gate, ldg,         \
       (const float*)p0, (const float*)p1, (const float*)p2,                  \
       (const float*)normw, (float*)state, (float*)aux, (const int*)seq_rows, \
-      H, G, D, DV, eps, qscale, c0, CS, DVB, rawp, nauxp)
+      H, G, D, DV, eps, qscale, c0, CS, DVB, rawp, nauxp, nmax)
   // the launch bound follows the thread count, so small launches keep a
   // lane's rows and the tile's outputs out of scratch
   bool small = false;
@@ -401,13 +417,14 @@ static int launch_linear_scan_p(LS_ARGS, int CS) {
 #undef LS_LAUNCH
   if constexpr (MODE != LS_SSD) {
     if (rawp != nullptr) {
-      const long waves = (long)T_ * H;
+      const long waves =
+          (nmax > T_ ? (long)T_ : (long)S_ * (nmax - 1)) * H;
       hipLaunchKernelGGL((scan_readout_kernel<T, MODE>),
                          dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
                          (hipStream_t)stream, (T*)out, ldo, rawp,
                          (const T*)gate, ldg, (const float*)normw, T_, H, DV,
                          eps, nauxp, (float*)aux, (const int*)seq_rows, S_,
-                         D);
+                         D, nmax);
     }
   }
   return 0;
@@ -512,7 +529,8 @@ extern "C" int mx_linear_scan(
     const void* wr, int ldwr, const void* gate, int ldg, const void* p0,
     const void* p1, const void* p2, const void* normw, void* state, void* aux,
     const void* seq_rows, int S_, int H, int G, int D, int DV, float eps,
-    float qscale, float c0, int T_, void* raw, int dtype, void* stream) {
+    float qscale, float c0, int T_, void* raw, int nmax, int dtype,
+    void* stream) {
   if (S_ <= 0) return 0;
   if (G < 1 || H % G) return 2;
   const bool bf = dtype == MX_BF16;

@@ -1282,6 +1282,25 @@ def short_conv_silu(x: torch.Tensor, w: torch.Tensor, state: torch.Tensor,
     return out
 
 
+# segments of this many rows and more go through the chunk-parallel
+# recurrence kernels, shorter ones token by token
+CHUNK_ROWS = 16
+_ALL_ROWS = 0x7fffffff
+_CHUNK_MODES = {"general": 0, "channel": 1, "gla": 2, "ssd": 3, "mlstm": 4}
+
+
+def _chunk_scratch(mode: str, T: int, S: int, H: int, G: int, D: int,
+                   DV: int, device):
+    """fp32 scratch of the chunk-parallel form of a recurrence over T rows in
+    S segments, None where it does not cover the step."""
+    if T - S + 1 < CHUNK_ROWS:      # no segment can be that long
+        return None
+    need = _mx().mx_chunk_scratch(_CHUNK_MODES[mode], T, S, H, G, D, DV)
+    if need <= 0:
+        return None
+    return torch.empty(need, dtype=torch.float32, device=device)
+
+
 def gated_delta(q, k, v, beta, zdec, zgate, a_log, dt_bias, normw, state,
                 seq_rows, heads: int, kv_heads: int, eps: float,
                 out: torch.Tensor = None) -> torch.Tensor:
@@ -1315,12 +1334,34 @@ def gated_delta(q, k, v, beta, zdec, zgate, a_log, dt_bias, normw, state,
         return out
     _check_seq_rows(seq_rows)
     assert state.is_contiguous()
+    S = seq_rows.shape[0]
+    shortest = _ALL_ROWS
+    scratch = _chunk_scratch("channel", T, S, H, G, D, DV, q.device)
+    if scratch is not None:
+        rc = _mx().mx_chunk_gated(
+            _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k),
+            _rows(k, "k"), _p(v), _rows(v, "v"), _p(beta),
+            _rows(beta, "beta"), _p(zdec), _rows(zdec, "zdec"), _p(zgate),
+            _rows(zgate, "zgate"), _p(a_log), _p(dt_bias), _p(normw),
+            _p(state), _p(seq_rows), S, T, H, G, D, DV, _f(eps),
+            _f(D ** -0.5), _p(scratch), _mx_dtype(q.dtype), _stream())
+        if rc == 0:
+            shortest = CHUNK_ROWS
+    rc = _mx().mx_token_scan(
+        _CHUNK_MODES["channel"], _p(out), _rows(out, "out"), _p(q),
+        _rows(q, "q"), _p(k), _rows(k, "k"), _p(v), _rows(v, "v"), _p(zdec),
+        _rows(zdec, "zdec"), _p(beta), _rows(beta, "beta"), _p(zgate),
+        _rows(zgate, "zgate"), _p(dt_bias), _p(a_log), _p(None), _p(normw),
+        _p(state), _p(None), _p(seq_rows), S, H, G, D, DV, _f(eps),
+        _f(D ** -0.5), _f(0.0), shortest, _mx_dtype(q.dtype), _stream())
+    if rc == 0:
+        return out
     rc = _mx().mx_gated_delta(
         _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k),
         _rows(k, "k"), _p(v), _rows(v, "v"), _p(beta), _rows(beta, "beta"),
         _p(zdec), _rows(zdec, "zdec"), _p(zgate), _rows(zgate, "zgate"),
         _p(a_log), _p(dt_bias), _p(normw), _p(state), _p(seq_rows),
-        seq_rows.shape[0], H, G, D, DV, _f(eps), _f(D ** -0.5),
+        S, H, G, D, DV, _f(eps), _f(D ** -0.5), shortest,
         _mx_dtype(q.dtype), _stream())
     if rc != 0:
         raise RuntimeError(
@@ -1358,12 +1399,33 @@ def delta_rule(r, k, v, zw, za, g, w0, ab, normw, state, seq_rows,
         out.copy_(y.reshape(T, HD))
         return out
     assert state.is_contiguous() and seq_rows.is_contiguous()
+    S = seq_rows.shape[0]
+    shortest = _ALL_ROWS
+    scratch = _chunk_scratch("general", T, S, H, H, D, D, r.device)
+    if scratch is not None:
+        rc = _mx().mx_chunk_delta(
+            _p(out), _rows(out, "out"), _p(r), _rows(r, "r"), _p(k),
+            _rows(k, "k"), _p(v), _rows(v, "v"), _p(zw), _rows(zw, "zw"),
+            _p(za), _rows(za, "za"), _p(g), _rows(g, "g"), _p(w0), _p(ab),
+            _p(normw), _p(state), _p(seq_rows), S, T, H, D, _f(eps),
+            _f(decay_scale), _p(scratch), _mx_dtype(r.dtype), _stream())
+        if rc == 0:
+            shortest = CHUNK_ROWS
+    rc = _mx().mx_token_scan(
+        _CHUNK_MODES["general"], _p(out), _rows(out, "out"), _p(r),
+        _rows(r, "r"), _p(k), _rows(k, "k"), _p(v), _rows(v, "v"), _p(zw),
+        _rows(zw, "zw"), _p(za), _rows(za, "za"), _p(g), _rows(g, "g"),
+        _p(w0), _p(ab), _p(None), _p(normw), _p(state), _p(None),
+        _p(seq_rows), S, H, H, D, D, _f(eps), _f(decay_scale), _f(0.0),
+        shortest, _mx_dtype(r.dtype), _stream())
+    if rc == 0:
+        return out
     rc = _mx().mx_delta_rule(
         _p(out), _rows(out, "out"), _p(r), _rows(r, "r"), _p(k),
         _rows(k, "k"), _p(v), _rows(v, "v"), _p(zw), _rows(zw, "zw"),
         _p(za), _rows(za, "za"), _p(g), _rows(g, "g"), _p(w0), _p(ab),
         _p(normw), _p(state), _p(seq_rows), seq_rows.shape[0], H, D,
-        _f(eps), _f(decay_scale), _mx_dtype(r.dtype), _stream())
+        _f(eps), _f(decay_scale), shortest, _mx_dtype(r.dtype), _stream())
     if rc != 0:
         raise RuntimeError(f"delta_rule: head dim {D} above 256 is not built")
     return out
@@ -1479,6 +1541,29 @@ def linear_scan(mode: str, q, k, v, dec, gate, state, seq_rows, heads: int,
         return out
     _check_seq_rows(seq_rows)
     assert state.is_contiguous() and (aux is None or aux.is_contiguous())
+    S = seq_rows.shape[0]
+    shortest = _ALL_ROWS
+    scratch = _chunk_scratch(mode, T, S, H, G, D, DV, q.device)
+    if scratch is not None:
+        rc = _mx().mx_chunk_scan(
+            SCAN_MODES[mode], _p(out), _rows(out, "out"), _p(q),
+            _rows(q, "q"), _p(k), _rows(k, "k"), _p(v), _rows(v, "v"),
+            _p(dec), _rows(dec, "dec"), _p(wr),
+            _rows(wr, "wr") if wr is not None else 0, _p(gate),
+            _rows(gate, "gate"), _p(p0), _p(p1), _p(p2), _p(normw),
+            _p(state), _p(aux), _p(seq_rows), S, T, H, G, D, DV, _f(eps),
+            _f(qscale), _f(c0), _p(scratch), _mx_dtype(dt), _stream())
+        if rc == 0:
+            shortest = CHUNK_ROWS
+    rc = _mx().mx_token_scan(
+        _CHUNK_MODES[mode], _p(out), _rows(out, "out"), _p(q),
+        _rows(q, "q"), _p(k), _rows(k, "k"), _p(v), _rows(v, "v"), _p(dec),
+        _rows(dec, "dec"), _p(wr), _rows(wr, "wr") if wr is not None else 0,
+        _p(gate), _rows(gate, "gate"), _p(p0), _p(p1), _p(p2), _p(normw),
+        _p(state), _p(aux), _p(seq_rows), S, H, G, D, DV, _f(eps),
+        _f(qscale), _f(c0), shortest, _mx_dtype(dt), _stream())
+    if rc == 0:
+        return out
     # wide heads: a head's value columns are shared out over several
     # workgroups and the read-out norm runs as a second kernel over this
     # fp32 scratch
@@ -1494,7 +1579,8 @@ def linear_scan(mode: str, q, k, v, dec, gate, state, seq_rows, heads: int,
         _rows(dec, "dec"), _p(wr), _rows(wr, "wr") if wr is not None else 0,
         _p(gate), _rows(gate, "gate"), _p(p0), _p(p1), _p(p2), _p(normw),
         _p(state), _p(aux), _p(seq_rows), seq_rows.shape[0], H, G, D, DV,
-        _f(eps), _f(qscale), _f(c0), T, _p(raw), _mx_dtype(dt), _stream())
+        _f(eps), _f(qscale), _f(c0), T, _p(raw), shortest, _mx_dtype(dt),
+        _stream())
     if rc != 0:
         raise RuntimeError(
             f"linear_scan: state {D}x{DV} per head is not built (key dims "

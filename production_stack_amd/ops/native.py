@@ -15,6 +15,7 @@ Groups (one shared library each):
   delta   delta_rule                        -> _mixops_delta.so
   gdelta  gated_delta                       -> _mixops_gdelta.so
   scan    linear_scan                       -> _mixops_scan.so
+  chunk   chunk_scan, token_scan            -> _mixops_chunk.so
 """
 
 from __future__ import annotations
@@ -63,6 +64,9 @@ GROUPS = {
     ],
     # one unit per (decay law, element type)
     "scan": [("linear_scan.hip", [f"-DLS_ONLY={i}"]) for i in range(6)],
+    # one unit per recurrence
+    "chunk": ([("chunk_scan.hip", [f"-DCK_ONLY={i}"]) for i in range(5)]
+              + [("token_scan.hip", [])]),
 }
 
 LIB_PATHS = {
@@ -70,6 +74,7 @@ LIB_PATHS = {
     "delta": os.path.join(PKG, "_mixops_delta.so"),
     "gdelta": os.path.join(PKG, "_mixops_gdelta.so"),
     "scan": os.path.join(PKG, "_mixops_scan.so"),
+    "chunk": os.path.join(PKG, "_mixops_chunk.so"),
 }
 
 # entry points outside the core group
@@ -78,6 +83,11 @@ SYMBOL_GROUP = {
     "mx_gated_delta": "gdelta",
     "mx_linear_scan": "scan",
     "mx_linear_scan_splits": "scan",
+    "mx_chunk_scratch": "chunk",
+    "mx_chunk_delta": "chunk",
+    "mx_chunk_gated": "chunk",
+    "mx_chunk_scan": "chunk",
+    "mx_token_scan": "chunk",
 }
 
 # entry points that return a status (the others return nothing)
@@ -86,11 +96,12 @@ INT_RESULT = {
     "mx_short_conv_silu", "mx_mfma_attention", "mx_linear_scan",
     "mx_linear_scan_splits", "mx_norm_conv32", "mx_moe_route",
     "mx_add_layer_norm32", "mx_expert_plan", "mx_expand_attention",
-    "mx_latent_decode", "mx_keyval_attention",
+    "mx_latent_decode", "mx_keyval_attention", "mx_chunk_delta",
+    "mx_chunk_gated", "mx_chunk_scan", "mx_token_scan",
 }
 
 # entry points that return a 64-bit count
-LONG_RESULT = {"mx_mingru_scratch"}
+LONG_RESULT = {"mx_mingru_scratch", "mx_chunk_scratch"}
 
 
 def _hipcc() -> str:

@@ -187,3 +187,168 @@ def test_delta_rule(dtype, H, D):
     t = tol(dtype)
     torch.testing.assert_close(got.cpu().float().view(sh), want, **t)
     torch.testing.assert_close(sg.cpu(), sr, rtol=1e-4, atol=1e-4)
+
+
+def _recurrence(mode, H, D, DV, segs, dtype, seed=0):
+    """(inputs, state, aux, call): call(inputs, state, aux, rows) runs one of
+    the five recurrences on the tensors' device."""
+    g = torch.Generator().manual_seed(seed)
+    T = sum(n for _, n, _, _ in segs)
+    G = H if mode in ("general", "gla", "mlstm") else max(1, H // 2)
+    dim = {"q": G * D, "k": G * D, "v": H * DV, "gate": H * DV}
+    dim["dec"] = H * D if mode in ("general", "channel", "gla") else H
+    dim["a"] = H * D if mode == "general" else H
+    # one fused buffer, odd row stride: views as a projection leaves them
+    proj = torch.randn(T, sum(dim.values()) + 3, generator=g).to(dtype)
+    x, at = {}, 0
+    for k, n in dim.items():
+        x[k], at = proj[:, at:at + n], at + n
+    x["p0"] = torch.randn(dim["dec"], generator=g) * 0.5
+    x["p1"] = torch.randn(dim["a"], generator=g) * 0.5
+    x["p2"] = torch.randn(H, generator=g)
+    x["nw"] = torch.randn(
+        H * DV if mode in ("general", "mlstm") else DV, generator=g)
+    state = torch.randn(len(segs), H, D, DV, generator=g) * 0.3
+    aux = None
+    if mode == "mlstm":
+        aux = torch.randn(len(segs), H, D + 1, generator=g).abs()
+
+    def call(x, state, aux, rows):
+        if mode == "general":
+            return ops.delta_rule(x["q"], x["k"], x["v"], x["dec"], x["a"],
+                                  x["gate"], x["p0"], x["p1"], x["nw"],
+                                  state, rows, H, 1e-5, 0.6)
+        if mode == "channel":
+            return ops.gated_delta(x["q"], x["k"], x["v"], x["a"], x["dec"],
+                                   x["gate"], x["p1"], x["p0"], x["nw"],
+                                   state, rows, H, G, 1e-5)
+        return ops.linear_scan(
+            mode, x["q"], x["k"], x["v"], x["dec"], x["gate"], state, rows,
+            H, G, 1e-5, qscale=D ** -0.5, c0=5.0 if mode == "mlstm" else 0.1,
+            wr=x["a"] if mode == "mlstm" else None, p0=x["p0"], p1=x["p1"],
+            p2=x["p2"], normw=x["nw"], aux=aux)
+
+    return x, state, aux, call
+
+
+def _to_gpu(x):
+    # keep the views' strides
+    base = x["q"]._base.cuda()
+    return {k: (torch.as_strided(base, v.shape, v.stride(),
+                                 v.storage_offset())
+                if v._base is not None else v.cuda()) for k, v in x.items()}
+
+
+def _rel(a, b):
+    a, b = a.double().cpu(), b.double().cpu()
+    return ((a - b).norm() / b.norm()).item()
+
+
+def _segs(lens, starts):
+    rows, at = [], 0
+    for i, (n, p) in enumerate(zip(lens, starts)):
+        rows.append((at, n, p, len(lens) - 1 - i))
+        at += n
+    return rows
+
+
+RECURRENCES = ["general", "channel", "gla", "ssd", "mlstm"]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("mode", RECURRENCES)
+@pytest.mark.parametrize("H,D,DV", [
+    (2, 20, 20), (2, 32, 32), (4, 48, 33), (2, 64, 96), (2, 96, 64),
+    (2, 128, 128), (2, 100, 160), (2, 128, 256)])
+def test_recurrence_chunk_edges(mode, H, D, DV, dtype):
+    """Segments of 15, 16, 17 ... rows (below, at and past whole chunks),
+    single rows between them, fresh and continued, on permuted slots."""
+    if mode == "general":
+        DV = D
+    rows = _segs([17, 1, 16, 15, 32, 2, 49, 1, 33],
+                 [0, 7, 5, 3, 0, 0, 9, 0, 1])
+    x, state, aux, call = _recurrence(mode, H, D, DV, rows, dtype)
+    # descending order of the rows: nothing may depend on it
+    rows = torch.tensor(rows[::-1], dtype=torch.int32)
+    sg = state.cuda()
+    ag = aux.cuda() if aux is not None else None
+    got = call(_to_gpu(x), sg, ag, rows.cuda())
+    want = call(x, state, aux, rows)
+    # fp32 sums of up to 49 tokens x 128 channels, then one rounding
+    assert _rel(got, want) < (2e-5 if dtype == torch.float32 else 6e-3)
+    assert _rel(sg, state) < 2e-6
+    if aux is not None:
+        assert _rel(ag, aux) < 2e-6
+
+
+@pytest.mark.parametrize("mode", RECURRENCES)
+def test_recurrence_chunk_not_a_number(mode):
+    """A value, key or decay that is no number reaches no earlier row, not
+    even of its own chunk, and no other sequence."""
+    rows = _segs([40, 33], [0, 4])
+    x, state, aux, call = _recurrence(mode, 2, 32, 32, rows, torch.float32)
+    rows = torch.tensor(rows, dtype=torch.int32).cuda()
+    xg = _to_gpu(x)
+    clean = call(xg, state.cuda(), aux.cuda() if aux is not None else None,
+                 rows)
+    for name, bad in (("v", float("nan")), ("v", float("inf")),
+                      ("k", float("nan")), ("dec", float("nan"))):
+        y = _to_gpu(x)
+        y[name][21, min(3, y[name].shape[1] - 1)] = bad
+        got = call(y, state.cuda(), aux.cuda() if aux is not None else None,
+                   rows)
+        assert _rel(got[:21], clean[:21]) < 1e-6, name
+        assert _rel(got[40:], clean[40:]) < 1e-6, name
+        assert not torch.isfinite(got[21:40]).all(), name
+
+
+@pytest.mark.parametrize("mode", ["general", "channel", "gla"])
+def test_recurrence_chunk_fast_decay(mode):
+    """Decays whose product over half a chunk leaves fp32's range: ratios of
+    neighbouring tokens stay exact."""
+    rows = _segs([50, 16], [0, 4])
+    x, state, aux, call = _recurrence(mode, 2, 64, 64, rows, torch.float32)
+    if mode == "channel":
+        x["p1"] += 3.0                  # rates around 20
+    elif mode == "gla":
+        x["p0"] -= 150.0                # logs around -15
+    else:
+        orig = call
+
+        def call(x, state, aux, rows):
+            return ops.delta_rule(x["q"], x["k"], x["v"], x["dec"], x["a"],
+                                  x["gate"], x["p0"], x["p1"], x["nw"],
+                                  state, rows, 2, 1e-5, 40.0)
+
+        assert orig is not call
+    rows = torch.tensor(rows, dtype=torch.int32)
+    sg = state.cuda()
+    got = call(_to_gpu(x), sg, None, rows.cuda())
+    want = call(x, state, aux, rows)
+    assert _rel(got, want) < 2e-5
+    assert _rel(sg, state) < 2e-5
+
+
+def test_recurrence_chunk_passes():
+    """A step whose operands exceed the scratch limit runs in passes: the same
+    results as two calls, each of which fits."""
+    H, D, T = 160, 32, 9600
+    g = torch.Generator(device="cuda").manual_seed(3)
+    proj = torch.randn(T, 6 * H * D, generator=g, device="cuda",
+                       dtype=torch.bfloat16)
+    v = [proj[:, i * H * D:(i + 1) * H * D] for i in range(6)]
+    par = [torch.randn(H * D, generator=g, device="cuda") for _ in range(3)]
+
+    def run(parts):
+        state = torch.zeros(1, H, D, D, device="cuda")
+        outs = []
+        for a, b in parts:
+            rows = torch.tensor([[0, b - a, a, 0]], dtype=torch.int32,
+                                device="cuda")
+            outs.append(ops.delta_rule(*[t[a:b] for t in v], *par, state,
+                                       rows, H, 1e-5, 0.6))
+        return torch.cat(outs), state
+
+    one, s1 = run([(0, T)])
+    two, s2 = run([(0, T // 2), (T // 2, T)])
+    assert torch.equal(one, two) and torch.equal(s1, s2)
