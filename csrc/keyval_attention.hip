@@ -35,24 +35,7 @@
 // is lane-local plus exchanges between the lanes of one head, and the weights
 // pack straight into the operand of the second product as three bf16 terms
 // (exact split of the 24-bit mantissa, fp32 accumulation).
-#include "mix_common.h"
-
-typedef __attribute__((ext_vector_type(8))) __bf16 kv_bf16x8;
-typedef __attribute__((ext_vector_type(16))) float kv_f32x16;
-typedef __attribute__((ext_vector_type(4))) float kv_f32x4;
-typedef __attribute__((ext_vector_type(4))) short kv_s4;
-typedef __attribute__((ext_vector_type(4))) unsigned int kv_u4;
-typedef __attribute__((address_space(3))) kv_s4 kv_lds_s4;
-
-#define KV_LOG2E 1.44269504f
-#define KV_LOW (-3.0e38f)
-
-union KvPack {
-  kv_bf16x8 v;
-  kv_s4 h[2];
-  unsigned int w[4];
-  uint4 q;
-};
+#include "attn_common.h"
 
 struct KvArgs {
   unsigned short* out;
@@ -76,22 +59,6 @@ struct KvArgs {
   int hpb, hblocks;             // heads per workgroup, head blocks per KV head
 };
 
-// Two weights (the first one low) cut into three bf16 terms of 8 mantissa bits
-// each (truncation; both remainders are exact).
-PS_DEV void kv_split(float p0, float p1, unsigned int* a, unsigned int* b,
-                     unsigned int* c) {
-  const unsigned int x0 = __float_as_uint(p0) & 0xffff0000u;
-  const unsigned int x1 = __float_as_uint(p1) & 0xffff0000u;
-  const float r0 = p0 - __uint_as_float(x0), r1 = p1 - __uint_as_float(x1);
-  const unsigned int y0 = __float_as_uint(r0) & 0xffff0000u;
-  const unsigned int y1 = __float_as_uint(r1) & 0xffff0000u;
-  const unsigned int z0 = __float_as_uint(r0 - __uint_as_float(y0));
-  const unsigned int z1 = __float_as_uint(r1 - __uint_as_float(y1));
-  *a = __builtin_amdgcn_perm(x1, x0, 0x07060302u);
-  *b = __builtin_amdgcn_perm(y1, y0, 0x07060302u);
-  *c = __builtin_amdgcn_perm(z1, z0, 0x07060302u);
-}
-
 // Distance from which on no head of h0 .. h0 + n - 1 sees anything that counts
 // (see above); a large number where there is no such distance.
 PS_DEV int kv_reach(const KvArgs& a, int h0, int n) {
@@ -102,37 +69,6 @@ PS_DEV int kv_reach(const KvArgs& a, int h0, int n) {
   if (!(sl > 0.f)) return far;
   const float d = (2.0f * a.bound2 + 40.0f) / (sl * KV_LOG2E);
   return d < 1.0e9f ? (int)d + 2 : far;
-}
-
-// One online-softmax step of a lane's N scores v (relative to the running
-// maximum m, or absolute while m is KV_LOW): weights into v, their sum into l,
-// the new maximum into m; returns the factor for what was accumulated before.
-// mx: the largest v over all lanes of the row. The factor is 1 for every lane
-// (and *moved false) when no maximum of the wave moves.
-template <int N>
-PS_DEV float kv_softmax(float* v, float mx, float* m, float* l, bool* moved) {
-  const bool fresh = *m == KV_LOW;
-  *moved = __any(mx > 0.f || (fresh && mx > -INFINITY));
-  float alpha = 1.f;
-  if (*moved) {
-    const float d = fresh ? (mx > -INFINITY ? mx : 0.f) : fmaxf(mx, 0.f);
-    if (!fresh) {
-      alpha = __builtin_amdgcn_exp2f(-d);
-      *m += d;
-    } else if (mx > -INFINITY) {
-      *m = d;
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] -= d;
-  }
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    v[i] = __builtin_amdgcn_exp2f(v[i]);
-    s += v[i];
-  }
-  *l = *l * alpha + s;
-  return alpha;
 }
 
 // ---------------------------------------------------------------------------
@@ -395,13 +331,6 @@ __global__ __launch_bounds__(256, OCC) void keyval_prompt_kernel(KvArgs a) {
 // ---------------------------------------------------------------------------
 #define KV_TT 32      // rows per tile of a wave
 #define KV_HEAD 4     // leading entries of a partial record
-
-// LDS written by some lanes of a wave is read by others of the same wave: the
-// wave's LDS accesses complete in order, this keeps the compiler to it.
-PS_DEV void kv_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
 
 // DK: 32-entry steps of a row (D <= 32 DK).
 template <int DK>

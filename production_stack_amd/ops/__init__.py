@@ -653,7 +653,9 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     single tokens over rows that carry their values take a kernel of their
     own first (variant 3; 7 insists on it), and so do prompt portions and
     single tokens over scaled keys that are their own values, whole rows
-    (variants 0 and 3; 8 and 9 insist on the portion / token form).
+    (variants 0 and 3; 8 and 9 insist on the portion / token form). Prompt
+    portions with a head mix over 32 heads of width 64 or 128 have a
+    matrix-core kernel too (variant 0; 10 insists on it).
     Returns [T, H*DV]."""
     NB, G, BS, D = k_cache.shape
     VR = v_cache.shape[3]
@@ -783,6 +785,20 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if variant in (5, 6):
         raise RuntimeError(
             "talk_attention: shape or dtype outside the matrix-core kernel")
+    # a head mix over prompt portions on the matrix cores
+    if (variant in (0, 10) and q.dtype == torch.bfloat16 and talk is not None
+            and keep_first == 0 and pool is None):
+        rc = _mx().mx_talk_mfma(
+            _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
+            _p(v_cache), _p(block_tables), block_tables.shape[1],
+            _p(token_seq), _p(token_pos), _p(talk), T, H, G, D, DV, BS,
+            _f(scale), int(chunk), int(window), int(bool(sink)),
+            _f(softcap), _p(sink_vals), int(VR), _stream())
+        if rc == 0:
+            return out
+    if variant == 10:
+        raise RuntimeError(
+            "talk_attention: shape or dtype outside the head-mix kernel")
     rc = _mx().mx_talk_attention(
         _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
         _p(v_cache), _p(block_tables), block_tables.shape[1],

@@ -9,9 +9,9 @@ shape checks live in the Python wrappers
 (production_stack_amd/ops/__init__.py).
 
 Groups (one shared library each):
-  core    resid32, norm_conv, mixer_prep, talk_attention, mfma_attention,
-          expand_attention, latent_decode, keyval_attention, moe_route,
-          moe_group, mingru_scan            -> _mixops.so
+  core    resid32, norm_conv, mixer_prep, talk_attention, talk_mfma,
+          mfma_attention, expand_attention, latent_decode, keyval_attention,
+          moe_route, moe_group, mingru_scan -> _mixops.so
   delta   delta_rule                        -> _mixops_delta.so
   gdelta  gated_delta                       -> _mixops_gdelta.so
   scan    linear_scan                       -> _mixops_scan.so
@@ -45,6 +45,7 @@ GROUPS = {
         ("resid32.hip", []),
         ("norm_conv.hip", []),
         ("talk_attention.hip", []),
+        ("talk_mfma.hip", []),
         ("mixer_prep.hip", []),
         ("mfma_attention.hip", []),
         ("expand_attention.hip", []),
@@ -97,7 +98,7 @@ INT_RESULT = {
     "mx_linear_scan_splits", "mx_norm_conv32", "mx_moe_route",
     "mx_add_layer_norm32", "mx_expert_plan", "mx_expand_attention",
     "mx_latent_decode", "mx_keyval_attention", "mx_chunk_delta",
-    "mx_chunk_gated", "mx_chunk_scan", "mx_token_scan",
+    "mx_chunk_gated", "mx_chunk_scan", "mx_token_scan", "mx_talk_mfma",
 }
 
 # entry points that return a 64-bit count

@@ -352,3 +352,42 @@ def test_recurrence_chunk_passes():
     one, s1 = run([(0, T)])
     two, s2 = run([(0, T // 2), (T // 2, T)])
     assert torch.equal(one, two) and torch.equal(s1, s2)
+
+
+@pytest.mark.parametrize("G,D,DV,chunk,window,softcap,learned", [
+    (8, 128, 128, 64, 0, 0.0, False), (8, 64, 64, 0, 50, 0.0, True),
+    (2, 128, 64, 0, 0, 0.0, True), (4, 64, 128, 40, 0, 9.0, True),
+    (1, 64, 64, 33, 20, 0.0, False)])
+def test_talk_attention_matrix_cores(G, D, DV, chunk, window, softcap,
+                                     learned):
+    """The 16-row head-mix kernel: portions that cross its row groups, rows
+    of several sequences in one group, key counts around its 32-key tiles, a
+    remainder of rows."""
+    g = torch.Generator().manual_seed(14)
+    H, bs, L = 32, 16, 150
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.bfloat16, g, 3)
+    ts, tp = [], []
+    for s, a, b in ((0, 0, 35), (1, 60, 66), (2, 31, 34), (1, 95, 98),
+                    (0, 127, 130), (2, 149, 150), (2, 0, 1)):
+        ts += [s] * (b - a)
+        tp += list(range(a, b))
+    T = len(ts)
+    q = torch.randn(T, H * D + 8, generator=g).to(torch.bfloat16)
+    talk = torch.eye(H) + 0.3 * torch.randn(H, H, generator=g)
+    sinks = torch.randn(H, generator=g) if learned else None
+    ts = torch.tensor(ts, dtype=torch.int32)
+    tp = torch.tensor(tp, dtype=torch.int32)
+    want = reference.talk_attention(
+        q[:, :H * D].float().reshape(T, H, D), kc.float(), vc.float(),
+        tables, ts, tp, D ** -0.5, chunk, window, True, talk, 0, softcap,
+        sinks)
+    out = torch.full((T, H * DV + 4), 7.0, dtype=torch.bfloat16,
+                     device="cuda")
+    ops.talk_attention(
+        q.cuda()[:, :H * D], kc.cuda(), vc.cuda(), tables.cuda(), ts.cuda(),
+        tp.cuda(), D ** -0.5, H, chunk=chunk, window=window, sink=True,
+        talk=talk.cuda(), softcap=softcap, variant=10,
+        sink_vals=sinks.cuda() if learned else None, out=out[:, :H * DV])
+    # fp32 up to the bf16 rounding of the result
+    assert _rel(out[:, :H * DV].float().reshape(T, H, DV), want) < 3e-3
+    assert (out[:, H * DV:] == 7.0).all()
