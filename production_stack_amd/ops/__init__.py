@@ -655,7 +655,9 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     single tokens over scaled keys that are their own values, whole rows
     (variants 0 and 3; 8 and 9 insist on the portion / token form). Prompt
     portions with a head mix over 32 heads of width 64 or 128 have a
-    matrix-core kernel too (variant 0; 10 insists on it).
+    matrix-core kernel too (variant 0; 10 insists on it). Without a head mix,
+    rows of whole 16-byte vectors up to 128 wide take a portion and a token
+    kernel of their own (variants 0 and 3; 11 and 12 insist on them).
     Returns [T, H*DV]."""
     NB, G, BS, D = k_cache.shape
     VR = v_cache.shape[3]
@@ -757,6 +759,39 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if variant in (8, 9):
         raise RuntimeError(
             "talk_attention: shape or dtype outside the key-value kernels")
+    # keys and values of their own, prompt portions or single tokens (also a
+    # few rows: 64 rows of 32/8 heads behind 2048 keys 85 us against 257, 8 x 16
+    # rows alone 16 against 16)
+    if (variant in (0, 3, 11, 12) and q.dtype == torch.bfloat16
+            and talk is None and chunk == 0 and not extra and pool is None):
+        token = variant in (3, 12)
+        shares = 1
+        if token:
+            # Two workgroups a CU cannot all be had from shares: merging the
+            # records costs 4 us and a share below 1024 keys is mostly its
+            # start (32/8 heads of 128: 1 token x 4001 keys 39 us whole, 19 in
+            # 4 shares, 20 in 16; 2 x 30001 260 whole, 48 in 8 and in 12; 8
+            # x 1024 16 whole, 20 in 2; 16 x 4001 41 whole, 46 in 2)
+            groups = T * G * ((H // G + 15) // 16)
+            keys = block_tables.shape[1] * BS
+            if window > 0:
+                keys = min(keys, window + keep_first)
+            shares = splits if splits > 0 else max(
+                1, min(16, 128 // groups, keys // 1024))
+        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
+                            device=q.device) if shares > 1 else None)
+        rc = _mx().mx_window_attention(
+            _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
+            _p(v_cache), _p(block_tables), block_tables.shape[1],
+            _p(token_seq), _p(token_pos), T, H, G, D, DV, BS, _f(scale),
+            int(window), int(bool(sink)), int(keep_first), _f(softcap),
+            _p(sink_vals), int(VR), int(token), int(shares), _p(part),
+            _stream())
+        if rc == 0:
+            return out
+    if variant in (11, 12):
+        raise RuntimeError(
+            "talk_attention: shape or dtype outside the window kernels")
     if variant not in (3, 4, 5, 6):
         splits = 1
     elif splits <= 0:

@@ -391,3 +391,43 @@ def test_talk_attention_matrix_cores(G, D, DV, chunk, window, softcap,
     # fp32 up to the bf16 rounding of the result
     assert _rel(out[:, :H * DV].float().reshape(T, H, DV), want) < 3e-3
     assert (out[:, H * DV:] == 7.0).all()
+
+
+@pytest.mark.parametrize("H,G,D,DV,window,keep,softcap,sink", [
+    (8, 2, 128, 128, 0, 0, 0.0, None), (32, 4, 64, 64, 70, 3, 20.0, "zero"),
+    (6, 2, 96, 40, 33, 64, 0.0, "heads"), (24, 1, 40, 128, 64, 66, 9.0, None),
+    (200, 1, 8, 8, 100, 0, 0.0, "heads"), (5, 5, 128, 64, 1, 0, 0.0, None)])
+def test_window_attention_kernels(H, G, D, DV, window, keep, softcap, sink):
+    """Portions that cross the 128-row groups, rows of several sequences in
+    one group, key counts around the 64- and 32-key tiles, kept keys before
+    and inside the window, head counts that leave rows idle; as portions and
+    as single tokens with one and several shares."""
+    g = torch.Generator().manual_seed(15)
+    bs, L = 16, 300
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.bfloat16, g, 3)
+    ts, tp = [], []
+    for s, a, b in ((0, 0, 70), (1, 60, 66), (2, 31, 34), (1, 127, 130),
+                    (0, 250, 300), (2, 299, 300), (2, 0, 1)):
+        ts += [s] * (b - a)
+        tp += list(range(a, b))
+    T = len(ts)
+    q = torch.randn(T, H * D + 8, generator=g).to(torch.bfloat16)
+    sinks = torch.randn(H, generator=g) if sink == "heads" else None
+    ts = torch.tensor(ts, dtype=torch.int32)
+    tp = torch.tensor(tp, dtype=torch.int32)
+    want = reference.talk_attention(
+        q[:, :H * D].float().reshape(T, H, D), kc.float(), vc.float(),
+        tables, ts, tp, D ** -0.5, 0, window, sink is not None, None, keep,
+        softcap, sinks)
+    for variant, splits in ((11, 0), (12, 1), (12, 0), (12, 5)):
+        out = torch.full((T, H * DV + 4), 7.0, dtype=torch.bfloat16,
+                         device="cuda")
+        ops.talk_attention(
+            q.cuda()[:, :H * D], kc.cuda(), vc.cuda(), tables.cuda(),
+            ts.cuda(), tp.cuda(), D ** -0.5, H, window=window,
+            keep_first=keep, sink=sink is not None, softcap=softcap,
+            variant=variant, splits=splits, out=out[:, :H * DV],
+            sink_vals=None if sinks is None else sinks.cuda())
+        # fp32 up to the bf16 rounding of the result
+        assert _rel(out[:, :H * DV].float().reshape(T, H, DV), want) < 3e-3
+        assert (out[:, H * DV:] == 7.0).all()
