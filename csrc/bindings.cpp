@@ -34,7 +34,7 @@ int ps_paged_attn_decode(void* out, void* ws_acc, void* ws_ml, const void* q,
                          const void* block_tables, const void* seq_lens,
                          int num_seqs, int max_blocks, float scale, int KH,
                          int GQ, int head_dim, int block_size, int num_splits,
-                         long q_stride, int variant, int kv_fp8, int window,
+                         int fill, long q_stride, int kv_fp8, int window,
                          hipStream_t stream);
 int ps_prefill_mfma32_splits(int num_tiles, int KH, int GQ);
 int ps_paged_attn_prefill_mfma32(void* out, void* ws_o, void* ws_ml,
@@ -183,11 +183,21 @@ void paged_attn_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   TORCH_CHECK(QH % KH == 0, "GQA group mismatch");
   const int GQ = QH / KH;
   const int max_blocks = (int)block_tables.size(1);
+  (void)variant;  // one kernel serves every value
+  int64_t fill = num_splits;
   if (num_splits <= 0) {
-    // fill ~3 workgroups per CU, bounded by useful split granularity
-    const int target = 2048;
-    num_splits = std::min<int64_t>(
-        32, std::max<int64_t>(1, target / std::max(1, S * KH)));
+    // One workgroup per CU: each of its waves keeps 16 KB of loads in flight,
+    // and with two a CU nothing is gained (32/8 heads of 128, bf16: 1 sequence
+    // of 4000 keys 38 us whole, 11.6 in 8 splits, 8.6 in 32; 8 of them 39
+    // whole, 25 in 4, 31 in 32; 64 of them 179 whole, 186 in 2, 197 in 8).
+    // Sequences long enough take more of the grid (see the kernel); that it
+    // is there for them costs the others 1.5 us at 32 sequences.
+    const int64_t groups = std::max(1, S * KH);
+    fill = std::min<int64_t>(32, std::max<int64_t>(1, 256 / groups));
+    int64_t keys = (int64_t)max_blocks * BS;
+    if (window > 0) keys = std::min<int64_t>(keys, window);
+    num_splits = std::max<int64_t>(
+        fill, std::min<int64_t>({32, 2048 / groups, (keys + 4095) / 4096}));
   }
   at::Tensor ws_acc, ws_ml;
   void *acc_p = nullptr, *ml_p = nullptr;
@@ -201,8 +211,8 @@ void paged_attn_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   int rc = ps_paged_attn_decode(
       out.data_ptr(), acc_p, ml_p, q.data_ptr(), k_cache.data_ptr(),
       v_cache.data_ptr(), block_tables.data_ptr(), seq_lens.data_ptr(), S,
-      max_blocks, (float)scale, KH, GQ, HD, BS, (int)num_splits,
-      q_row_stride(q, HD), (int)variant, kv_fp8, (int)window,
+      max_blocks, (float)scale, KH, GQ, HD, BS, (int)num_splits, (int)fill,
+      q_row_stride(q, HD), kv_fp8, (int)window,
       current_stream());
   TORCH_CHECK(rc == 0, "unsupported decode config: head_dim=", HD,
               " block_size=", BS, " gqa=", GQ);
@@ -466,7 +476,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rotary_embedding", &rotary_embedding,
         "Neox-style rotary embedding (bf16, in-place)");
   m.def("paged_attn_decode", &paged_attn_decode,
-        "Paged attention, decode phase (bf16 KV, split-KV)",
+        "Paged attention, decode phase (bf16 or fp8 KV, split-KV)",
         pybind11::arg("out"), pybind11::arg("q"), pybind11::arg("k_cache"),
         pybind11::arg("v_cache"), pybind11::arg("block_tables"),
         pybind11::arg("seq_lens"), pybind11::arg("scale"),

@@ -124,10 +124,8 @@ def paged_attn_decode(
     if q.is_cuda:
         _require_ext()
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        # variant 1 = low-register packed-q kernel (3 waves/SIMD): measured
-        # +17-26% over variant 0 across batch/ctx (profiles/attn_bench).
         _C.paged_attn_decode(
-            out, q, k_cache, v_cache, block_tables, seq_lens, scale, 0, 1,
+            out, q, k_cache, v_cache, block_tables, seq_lens, scale, 0, 0,
             window
         )
         return out

@@ -33,6 +33,7 @@ ext = CUDAExtension(
         "csrc/bindings.cpp",
         "csrc/norm_act_rope.hip",
         "csrc/attention.hip",
+        "csrc/decode_attention.hip",
         "csrc/prefill_mfma.hip",
         "csrc/prefill_mfma32.hip",
         "csrc/skinny_gemm.hip",

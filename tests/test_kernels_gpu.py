@@ -733,3 +733,45 @@ def test_gemm8p_split_ranges(m, n, k):
         # one bf16 rounding of an fp32 sum of k products
         err = ((got - want).abs() / (want.abs() + k ** 0.5)).max().item()
         assert err < 2 ** -7, err
+
+
+@pytest.mark.parametrize("kh,gq,hd,fp8,window", [
+    (2, 4, 128, False, 0), (2, 4, 128, True, 0), (1, 1, 128, False, 70),
+    (3, 8, 128, True, 45), (2, 3, 128, True, 1), (2, 8, 64, False, 0),
+    (1, 1, 64, False, 130)])
+@pytest.mark.parametrize("splits", [0, 1, 3, 40])
+def test_paged_attn_decode_tiles(kh, gq, hd, fp8, window, splits):
+    """Key counts around the 32- and 64-key tiles and what four waves take at
+    a time, an empty sequence, one longer than a split's share."""
+    from production_stack_amd import _C
+
+    g = torch.Generator().manual_seed(31)
+    lens = [0, 1, 31, 33, 64, 65, 127, 129, 257, 4200]
+    S, qh = len(lens), kh * gq
+    per = (max(lens) + 15) // 16
+    nb = 400
+    k = torch.randn(nb, kh, 16, hd, generator=g).to(torch.bfloat16)
+    v = torch.randn(nb, kh, 16, hd, generator=g).to(torch.bfloat16)
+    if fp8:
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+    bt = torch.randint(0, nb, (S, per), generator=g, dtype=torch.int32)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    q = torch.randn(S, qh + 2, hd, generator=g).to(torch.bfloat16)
+    want = torch.zeros(S, qh, hd, dtype=torch.float64)
+    for i, n in enumerate(lens):
+        lo = max(0, n - window) if window else 0
+        if n == 0:
+            continue
+        pos = torch.arange(lo, n)
+        rows = bt[i, pos // 16].long()
+        ki = k.double()[rows, :, pos % 16].repeat_interleave(gq, 1)
+        vi = v.double()[rows, :, pos % 16].repeat_interleave(gq, 1)
+        sc = torch.einsum("hd,nhd->hn", q[i, :qh].double(), ki) * 0.11
+        want[i] = torch.einsum("hn,nhd->hd", sc.softmax(-1), vi)
+    out = torch.empty(S, qh, hd, dtype=torch.bfloat16, device="cuda")
+    _C.paged_attn_decode(out, q.cuda()[:, :qh], k.cuda(), v.cuda(), bt.cuda(),
+                         sl.cuda(), 0.11, splits, 0, window)
+    got = out.cpu().double()
+    assert (got[0] == 0).all()
+    # fp32 up to the bf16 rounding of the result
+    assert ((got - want).norm() / want.norm()) < 3e-3
