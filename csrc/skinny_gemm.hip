@@ -31,6 +31,76 @@ PS_DEV ps_gbf16x8 ps_as_gbf16(ps_bf16x8 u) {
   return v.bf;
 }
 
+// Up to 16 rows of x: a workgroup owns 16 rows of W and all of K, its NW waves
+// take every NW-th 128-byte piece of them, UC pieces in flight each, and add up
+// in LDS at the end: no second kernel and no partial sums in memory. W goes
+// from memory straight into left operands, x from the caches into right ones
+// (rows past the last read as zeros without an access).
+// Bound by the read of W, at few rows of W by its latency: 1 x 4096 x 4096 in
+// 10.3 us (17.4 with the split kernel, its merge included), 1 x 28672 x 4096 in
+// 46 (79; 5.1 TB/s), 1 x 2048 x 2048 in 5.0 (13.1). Reading x costs as many
+// load instructions as reading W: 16 rows of it make the wide one 68 us.
+template <int UC, int NW>
+__global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
+    unsigned short* __restrict__ out, const unsigned short* __restrict__ x,
+    const unsigned short* __restrict__ w, int M, int N, int K, int x_stride) {
+  constexpr int PN = 20;  // pitch of a row of sums
+  __shared__ __align__(16) float s_sum[NW][16 * PN];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int rc = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  const int nc = K / 64;  // pieces
+  const unsigned short* wp = w + (long)(n0 + rc) * K + g * 8;
+  const auto xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)x, 0, ((M - 1) * x_stride + K) * 2, 0x00020000);
+  const unsigned int xo =
+      rc < M ? (unsigned int)(rc * x_stride + g * 8) * 2 : 0x80000000u;
+  ps_gf32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  ps_gbf16x8 wf[UC][2], xf[UC][2];
+  // pieces past the end repeat the last one and are not multiplied
+  auto load = [&](int u, int c) {
+    const int k = min(c, nc - 1) * 64;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      wf[u][h] = *(const ps_gbf16x8*)(wp + k + 32 * h);
+      xf[u][h] = __builtin_bit_cast(
+          ps_gbf16x8,
+          __builtin_amdgcn_raw_buffer_load_b128(xr, xo, k * 2 + 64 * h, 0));
+    }
+  };
+  const int w0 = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+  for (int u = 0; u < UC; ++u) load(u, w0 + NW * u);
+  for (int c = w0; c < nc; c += NW * UC) {
+#pragma unroll
+    for (int u = 0; u < UC; ++u) {
+      if (c + NW * u < nc) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][h], xf[u][h],
+                                                        acc, 0, 0, 0);
+      }
+      load(u, c + NW * (UC + u));
+    }
+  }
+  // acc[r]: row rc of x, row n0 + 4 g + r of W
+  *(ps_gf32x4*)(&s_sum[wave][rc * PN + 4 * g]) = acc;
+  __syncthreads();
+  if (tid < 64) {
+    const int m = tid >> 2, n = (tid & 3) * 4;
+    ps_gf32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < NW; ++k)
+      v += *(const ps_gf32x4*)(&s_sum[k][m * PN + n]);
+    if (m < M)
+      *(uint2*)(out + (long)m * N + n0 + n) = make_uint2(
+          (unsigned int)ps_f32_to_bf16(v[0]) |
+              ((unsigned int)ps_f32_to_bf16(v[1]) << 16),
+          (unsigned int)ps_f32_to_bf16(v[2]) |
+              ((unsigned int)ps_f32_to_bf16(v[3]) << 16));
+  }
+}
+
 template <int M_TILES>
 __global__ __launch_bounds__(256, 4) void skinny_gemm_kernel(
     unsigned short* __restrict__ out_bf16,  // [M, N] (splits == 1)
@@ -129,11 +199,17 @@ __global__ __launch_bounds__(256) void skinny_combine_kernel(
 
 extern "C" {
 
+// Rows of x for the kernel without splits; its byte offsets are 31 bits.
+static bool ps_skinny_rows(int M, int K, long x_stride) {
+  return M <= 16 && x_stride >= 0 && (M - 1) * x_stride + K < (1L << 30);
+}
+
 // ws == nullptr forces splits = 1. ps_skinny_gemm_splits reports the
 // split depth the heuristic will pick for a shape so the caller can size
 // the fp32 workspace.
 int ps_skinny_gemm_splits(int M, int N, int K) {
   if (N % 64 != 0 || K % 64 != 0 || M > 256) return -1;
+  if (M <= 16) return 1;
   const int kchunks = K / 64;
   const int target_wgs = 1024;
   int splits = target_wgs / (N / 64);
@@ -146,6 +222,22 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
                    int M, int N, int K, long x_stride, hipStream_t stream) {
   int splits = ps_skinny_gemm_splits(M, N, K);
   if (splits < 0) return -1;
+  if (ps_skinny_rows(M, K, x_stride)) {
+#define PS_SR(UC, NW)                                                       \
+  skinny_rows_kernel<UC, NW><<<N / 16, NW * 64, 0, stream>>>(               \
+      (unsigned short*)out_bf16, (const unsigned short*)x,                  \
+      (const unsigned short*)w, M, N, K, (int)x_stride)
+    // long rows: four pieces in flight a wave, else a piece and more waves (us
+    // at one row, 16 waves of one piece against 8 of four: 2048 x 2048 5.0 /
+    // 6.3, 16384 x 2048 16.5 / 20.8, 28672 x 4096 46.2 / 51.6, 4096 x 14336
+    // 28.0 / 25.2)
+    if (K <= 4096)
+      PS_SR(1, 16);
+    else
+      PS_SR(4, 8);
+#undef PS_SR
+    return 0;
+  }
   if (ws == nullptr) splits = 1;
   dim3 grid(N / 64, splits);
   dim3 block(256);
@@ -153,8 +245,7 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
   skinny_gemm_kernel<MT><<<grid, block, 0, stream>>>(                       \
       (unsigned short*)out_bf16, (float*)ws, (const unsigned short*)x,      \
       (const unsigned short*)w, M, N, K, x_stride)
-  if (M <= 16) PS_SG(1);
-  else if (M <= 32) PS_SG(2);
+  if (M <= 32) PS_SG(2);
   else if (M <= 64) PS_SG(4);
   else if (M <= 128) PS_SG(8);
   else PS_SG(16);

@@ -74,12 +74,32 @@ def tune(weights, buckets, device) -> None:
     )
 
 
+def _few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Untuned shapes that take the in-house kernel: up to 3 rows and rows of
+    W of up to 4096 entries. us, in-house / library: 1 x 2048 x 2048 4.9 / 8.2,
+    1 x 28672 x 4096 46 / 64, 3 x 4096 x 4096 11.0 / 15.8, 3 x 6144 x 4096
+    15.8 / 15.8; past the line 4 x 6144 x 4096 16.2 / 15.7, 1 x 2048 x 8192
+    14.5 / 12.8."""
+    from production_stack_amd import ops
+
+    return (x.dim() == 2 and 0 < x.shape[0] <= 3 and w.shape[1] <= 4096
+            and _eligible(x.shape[0], *w.shape) and x.stride(1) == 1
+            and x.shape[1] == w.shape[1] and w.dtype == torch.bfloat16
+            and w.is_contiguous() and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and ops.HAVE_EXT
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad)))
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear with autotuned dispatch (no bias; Llama has none). The
     in-house kernels are bfloat16 only; other types take the library."""
-    if x.is_cuda and _POLICY and x.dtype == torch.bfloat16:
+    if x.is_cuda and x.dtype == torch.bfloat16:
         key = (x.shape[0], w.shape[0], w.shape[1])
-        impl = _POLICY.get(key, 0)
+        impl = _POLICY.get(key)
+        if impl is None:
+            impl = int(_few_rows(x, w))
         if impl:
             from production_stack_amd import ops
 

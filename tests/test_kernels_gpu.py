@@ -775,3 +775,26 @@ def test_paged_attn_decode_tiles(kh, gq, hd, fp8, window, splits):
     assert (got[0] == 0).all()
     # fp32 up to the bf16 rounding of the result
     assert ((got - want).norm() / want.norm()) < 3e-3
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 64), (2, 128, 1024), (3, 192, 1088), (3, 64, 4096),
+    (15, 64, 4160), (16, 128, 2048), (16, 64, 8192), (1, 64, 2176)])
+def test_skinny_gemm_few_rows(M, N, K):
+    """Rows of W from less than one piece a wave to several rounds with a
+    remainder, full and partial row tiles, x with a row stride, and what the
+    dispatch does with the same operands."""
+    from production_stack_amd.ops import gemm_policy
+
+    g = torch.Generator().manual_seed(M + K)
+    buf = torch.randn(M + 1, K + 8, generator=g).to(torch.bfloat16)
+    buf[M:] = float("nan")
+    w = torch.randn(N, K, generator=g).to(torch.bfloat16)
+    x = buf.cuda()[:M, :K]
+    got = ops.skinny_gemm(x, w.cuda()).cpu().double()
+    want = buf[:M, :K].double() @ w.double().t()
+    # fp32 up to the bf16 rounding of the result (2^-9 at most each)
+    assert ((got - want).abs() <= want.abs() / 256 + 1e-3).all()
+    gemm_policy.reset()
+    via = gemm_policy.linear(x, w.cuda()).cpu().double()
+    assert ((via - want).abs() <= want.abs() / 256 + 1e-3).all()
