@@ -468,12 +468,19 @@ PS_DEV ck_f32x4 ck_square_terms(const float* frag, ck_f32x4 x, ck_f32x4 acc,
 // in two chunks ahead, through registers into one of two LDS buffers.
 // Workgroups of one head are S_ * H apart, so that they share an XCD's L2
 // where that is a multiple of 8.
-template <typename T, int MODE, int DP>
+//
+// PART 1 and 2 (gla, whose state only decays between writes): a segment's
+// chunks in `parts` runs that are walked at once. The first launch walks all
+// runs but the last from an empty state and leaves what each adds to the state
+// and its decays' product in `part` ([S_, H, parts] records of D x DV and DP;
+// the last run's record takes the state before the segment). The second starts
+// each run from what the runs before it leave and writes the outputs.
+template <typename T, int MODE, int DP, int PART>
 __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
     float* __restrict__ raw, const float* __restrict__ items, int cap,
     const T* __restrict__ v, int ldv, float* __restrict__ state,
     const int* __restrict__ seq_rows, int S_, int H, int D, int DV, int c0,
-    int nc) {
+    int nc, float* __restrict__ part, int parts) {
   typedef CkItem<MODE, DP> It;
   constexpr int NT = DP / 32;  // row tiles of one wave
   constexpr int N4 = It::TOTAL / 4;
@@ -483,12 +490,15 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
   float* xch = lds + 2 * BUF;     // [4 waves][2][64][4]
   float* tmp = xch + 2048 + (threadIdx.x >> 6) * 256;
 
-  const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H);
+  const int ncb = (DV + 31) / 32;
+  const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H) % ncb;
+  const int run = PART ? blockIdx.x / (S_ * H) / ncb : 0;
   const int seg = sh / H, hd = sh % H;
   const int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
   const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
   int count = ck_count(n, c0, nc);
   if (count == 0) return;
+  const bool old = p0 != 0 || c0 != 0;  // there is a state to start from
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // this segment's first chunk among all
@@ -500,6 +510,16 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
   first = __builtin_amdgcn_readfirstlane(first);
   count = __builtin_amdgcn_readfirstlane(min(count, cap - first));
   if (count <= 0) return;
+  bool last = true;  // this run ends the segment's chunks of the pass
+  if constexpr (PART != 0) {
+    const int per = (count + parts - 1) / parts;
+    last = (run + 1) * per >= count;
+    // a first run is always there; the others may be empty
+    if (run * per >= count) return;
+    first += run * per;
+    c0 += run * per;
+    count = min(per, count - run * per);
+  }
 
   const int g = lane >> 4, m16 = lane & 15;
   const int ct = wave >> 1, ds = wave & 1;  // column tile, row half
@@ -509,15 +529,53 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
   const int hv = hd * DV + j;
   float* Sg = state + ((size_t)slot * H + hd) * (size_t)D * DV;
   ck_f32x4 S[NT];
+  const size_t rec = (size_t)D * DV + DP;  // of one run
+  float* pt = PART ? part + (size_t)sh * parts * rec : nullptr;
+  if constexpr (PART != 2) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = 16 * (tb + t) + 4 * g + i;
-      S[t][i] = (col && d < D && (p0 != 0 || c0 != 0))
-                    ? Sg[(size_t)d * DV + j]
-                    : 0.f;
-    }
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * (tb + t) + 4 * g + i;
+        S[t][i] = (col && d < D && old) ? Sg[(size_t)d * DV + j] : 0.f;
+      }
+  }
+  if constexpr (PART == 1) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * (tb + t) + 4 * g + i;
+        if (run == 0 && col && d < D)
+          pt[(parts - 1) * rec + (size_t)d * DV + j] = S[t][i];
+        S[t][i] = 0.f;
+      }
+  }
+  if constexpr (PART == 2) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * (tb + t) + 4 * g + i;
+        S[t][i] = col && d < D ? pt[(parts - 1) * rec + (size_t)d * DV + j]
+                               : 0.f;
+      }
+#pragma unroll 2
+    for (int q = 0; q < run; ++q)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int d = 16 * (tb + t) + 4 * g + i;
+          const float add =
+              col && d < D ? pt[q * rec + (size_t)d * DV + j] : 0.f;
+          S[t][i] = S[t][i] * pt[q * rec + (size_t)D * DV + d] + add;
+        }
+  }
+  // product of the decays over the run, this wave's rows
+  ck_f32x4 decay[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) decay[t] = {1.f, 1.f, 1.f, 1.f};
 
   const char* src = (const char*)(items + ((size_t)first * H + hd) * It::TOTAL);
   const size_t step = (size_t)H * It::TOTAL * sizeof(float);
@@ -651,7 +709,10 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
       const int at = ck_col_slot(tb + t, g, m16) * 4;
       k4[t] = *(const ck_f32x4*)(buf + It::K + at);
       if constexpr (MODE == CK_GD) b4[t] = *(const ck_f32x4*)(buf + It::B + at);
-      S[t] *= *(const ck_f32x4*)(buf + It::GAM + (tb + t) * 16 + g * 4);
+      const ck_f32x4 gam =
+          *(const ck_f32x4*)(buf + It::GAM + (tb + t) * 16 + g * 4);
+      S[t] *= gam;
+      if constexpr (PART == 1) decay[t] *= gam;
     }
     const int osq = MODE == CK_GD ? It::MB : It::M;
     const ck_f32x4 o4 = *(const ck_f32x4*)(buf + osq + lane * 4);
@@ -686,7 +747,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
       __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // an LDS write
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (ds == 0) {
+    if (PART != 1 && ds == 0) {
       if constexpr (MODE != CK_GLA) {
         if (!fin) P = ck_square_terms(buf + osq, Z, zero, lane, tmp);
         O += P;
@@ -718,13 +779,24 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
     if (c + 2 >= count) break;
     __syncthreads();
   }
-  if (col) {
+  float* Se = Sg;
+  if constexpr (PART == 1) {
+    Se = pt + run * rec;
+    if (cb == 0 && ct == 0 && m16 == 0) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          Se[(size_t)D * DV + 16 * (tb + t) + 4 * g + i] = decay[t][i];
+    }
+  }
+  if (col && (PART != 2 || last)) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int d = 16 * (tb + t) + 4 * g + i;
-        if (d < D) Sg[(size_t)d * DV + j] = S[t][i];
+        if (d < D) Se[(size_t)d * DV + j] = S[t][i];
       }
   }
 }
@@ -906,14 +978,16 @@ __global__ __launch_bounds__(256) void ck_prep_scalar_kernel(
 // The walk of ck_sweep_kernel for one decay per head and token. out: the
 // finished fp32 rows of ssd, (o + skip v) silu(gate), or the raw read-outs
 // [T, H * (DV + 1)] of mlstm, whose column DV is the normaliser's (its values
-// are 1, its state lies in aux).
-template <typename T, int MODE, int DP>
+// are 1, its state lies in aux). PART, part and parts as there; a record is the
+// D x (DV, with the normaliser DV + 1) state and one decay.
+template <typename T, int MODE, int DP, int PART>
 __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     float* __restrict__ out, int ldo, const float* __restrict__ gitems,
     const float* __restrict__ hitems, int cap, CkIn in,
     const float* __restrict__ p2, float* __restrict__ state,
     float* __restrict__ aux, const int* __restrict__ seq_rows, int S_, int H,
-    int G, int D, int DV, int c0, int nc) {
+    int G, int D, int DV, int c0, int nc, float* __restrict__ part,
+    int parts) {
   typedef CkGroup<DP> Gi;
   constexpr int NT = DP / 32;
   constexpr int PG = Gi::TOTAL / 1024;  // DP is a multiple of 32
@@ -923,12 +997,15 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
   __shared__ __align__(16) float tmps[4 * 256];
   float* tmp = tmps + (threadIdx.x >> 6) * 256;
 
-  const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H);
+  const int cols = DV + (MODE == CK_MLSTM ? 1 : 0), ncb = (cols + 31) / 32;
+  const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H) % ncb;
+  const int run = PART ? blockIdx.x / (S_ * H) / ncb : 0;
   const int seg = sh / H, hd = sh % H, grp = hd / (H / G);
   const int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
   const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
   int count = ck_count(n, c0, nc);
   if (count == 0) return;
+  const bool old = p0 != 0 || c0 != 0;  // there is a state to start from
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int first = 0;
@@ -939,6 +1016,15 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
   first = __builtin_amdgcn_readfirstlane(first);
   count = __builtin_amdgcn_readfirstlane(min(count, cap - first));
   if (count <= 0) return;
+  bool last = true;  // this run ends the segment's chunks of the pass
+  if constexpr (PART != 0) {
+    const int per = (count + parts - 1) / parts;
+    last = (run + 1) * per >= count;
+    if (run * per >= count) return;
+    first += run * per;
+    c0 += run * per;
+    count = min(per, count - run * per);
+  }
 
   const int g = lane >> 4, m16 = lane & 15;
   const int ct = wave >> 1, ds = wave & 1, tb = ds * NT;
@@ -949,6 +1035,8 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
   float* Sg = state + ((size_t)slot * H + hd) * (size_t)D * DV + j;
   float* Ng = MODE == CK_MLSTM ? aux + ((size_t)slot * H + hd) * (D + 1)
                                : nullptr;
+  const size_t rec = (size_t)D * cols + 4;  // of one run
+  float* pt = PART ? part + (size_t)sh * parts * rec : nullptr;
   ck_f32x4 S[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -956,12 +1044,38 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     for (int i = 0; i < 4; ++i) {
       const int d = 16 * (tb + t) + 4 * g + i;
       float x = 0.f;
-      if (d < D && (p0 != 0 || c0 != 0)) {
+      if (PART != 2 && d < D && old) {
         if (col) x = Sg[(size_t)d * DV];
         if (ncol) x = Ng[d];
       }
+      if constexpr (PART == 1) {
+        if (run == 0 && d < D && (col || ncol))
+          pt[(parts - 1) * rec + (size_t)d * cols + j] = x;
+        x = 0.f;
+      }
+      if constexpr (PART == 2) {
+        if (d < D && (col || ncol))
+          x = pt[(parts - 1) * rec + (size_t)d * cols + j];
+      }
       S[t][i] = x;
     }
+  if constexpr (PART == 2) {
+#pragma unroll 2
+    for (int q = 0; q < run; ++q) {
+      const float a = pt[q * rec + (size_t)D * cols];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int d = 16 * (tb + t) + 4 * g + i;
+          const float add = d < D && (col || ncol)
+                                ? pt[q * rec + (size_t)d * cols + j]
+                                : 0.f;
+          S[t][i] = S[t][i] * a + add;
+        }
+    }
+  }
+  float decay = 1.f;  // over the run
 
   const char* gsrc =
       (const char*)(gitems + ((size_t)first * G + grp) * Gi::TOTAL);
@@ -1034,6 +1148,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
         Z = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i + 1], S[t][i + 1], Z,
                                                  0, 0, 0);
       }
+    if constexpr (PART == 1) decay *= gam;
     const ck_f32x4 W = V * dk;
 #pragma unroll
     for (int t = 0; t < NT; ++t) S[t] *= gam;
@@ -1050,7 +1165,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     if (!fin) X = ck_square_terms(hb + CkHead::M, V, zero, lane, tmp);
     // also: this chunk's buffer is read, the next one's is filled
     __syncthreads();
-    if (ds == 0 && (col || ncol)) {
+    if (PART != 1 && ds == 0 && (col || ncol)) {
       O = (O + *(const ck_f32x4*)(xch + ct * 256 + lane * 4)) * dr + X;
       const size_t row = (size_t)(t0 + 16 * (c0 + c) + 4 * g);
 #pragma unroll
@@ -1080,14 +1195,21 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     if (c + 2 >= count) break;
     __syncthreads();
   }
+  if (PART == 1 && cb == 0 && threadIdx.x == 0)
+    pt[run * rec + (size_t)D * cols] = decay;
+  if (PART == 2 && !last) return;
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int d = 16 * (tb + t) + 4 * g + i;
       if (d < D) {
-        if (col) Sg[(size_t)d * DV] = S[t][i];
-        if (ncol) Ng[d] = S[t][i];
+        if (PART == 1) {
+          if (col || ncol) pt[run * rec + (size_t)d * cols + j] = S[t][i];
+        } else {
+          if (col) Sg[(size_t)d * DV] = S[t][i];
+          if (ncol) Ng[d] = S[t][i];
+        }
       }
     }
 }
@@ -1186,7 +1308,7 @@ static long ck_chunk_floats(int mode, int dp, int H, int G) {
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
 //                                                            5.42 -> 0.70 ms
 //   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.64 ms
-//   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.15 ms
+//   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.09 ms
 //   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.84 ms
 // From 16 rows on a segment goes this way: one chunk costs about 15 us in
 // three launches, 16 tokens one by one 24 us.
@@ -1212,6 +1334,34 @@ static void ck_plan(int mode, int T_, int S_, int H, int G, int D, int* cap,
   *nc = (int)(fit / S_);
   *cap = (int)((long)*nc * S_ < all ? (long)*nc * S_ : all);
   *passes = (longest + *nc - 1) / *nc;
+}
+
+// Runs that a segment's chunks are walked in (not the delta forms, whose state
+// is multiplied by more than a decay). Two walks of count / runs chunks and
+// their start take the place of one of count chunks, so it pays from four runs
+// and 32 chunks on, where the workgroups of one walk (a head's columns by 32)
+// leave most of the chip idle: us in one walk -> in runs, bf16, one prompt: gla
+// 8 heads of 128 x 256, 1501 rows 147 -> 86, 400 rows (25 chunks, 4 runs) 57 ->
+// 60; 16 heads, 3000 rows (4 runs) 300 -> 258; ssd 48 heads of 128 x 64, 3000
+// rows (5 runs) 297 -> 180, 500 rows 74 -> 71; mlstm 16 heads of 128 x 128, 3000
+// rows (6 runs) 326 -> 222.
+static int ck_parts(int mode, int T_, int S_, int H, int DV) {
+  if (mode == CK_GD || mode == CK_CD) return 1;
+  const int cols = DV + (mode == CK_MLSTM ? 1 : 0);
+  const long blocks = (long)S_ * H * ((cols + 31) / 32);
+  const int longest = (T_ - S_ + 1 + 15) / 16;
+  long parts = 512 / blocks;
+  if (parts > 16) parts = 16;
+  if (parts > longest / 6) parts = longest / 6;
+  return parts < 4 || longest < 32 ? 1 : (int)parts;
+}
+// Floats of the runs' records.
+static long ck_part_floats(int mode, int T_, int S_, int H, int D, int DV) {
+  const int parts = ck_parts(mode, T_, S_, H, DV);
+  if (parts == 1) return 0;
+  const long rec = mode == CK_GLA ? (long)D * DV + ck_pad(D)
+                                  : (long)D * (DV + 1) + 4;
+  return (long)S_ * H * parts * rec;
 }
 
 #define CK_ARGS                                                              \
@@ -1255,10 +1405,12 @@ static int ck_launch(CK_ARGS) {
   float* raw = scratch;
   float* items = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
   const int ncb = (DV + 31) / 32;
+  const int parts = ck_parts(MODE, T_, S_, H, DV);
+  float* part = items + (((size_t)cap * H * It::TOTAL + 3) & ~(size_t)3);
   const size_t lds =
       (2 * ((It::TOTAL + 1023) / 1024) * 1024 + 2048 + 1024) * sizeof(float);
   if (lds > 65536 &&
-      hipFuncSetAttribute((const void*)ck_sweep_kernel<T, MODE, DP>,
+      hipFuncSetAttribute((const void*)ck_sweep_kernel<T, MODE, DP, 0>,
                           hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)lds) != hipSuccess)
     return 1;
@@ -1266,10 +1418,21 @@ static int ck_launch(CK_ARGS) {
     hipLaunchKernelGGL((ck_prep_kernel<T, MODE, DP>), dim3(cap, H), dim3(256),
                        0, stream, items, in, (const int*)seq_rows, S_, H, G,
                        D, scale, c0f, p * nc, nc);
-    hipLaunchKernelGGL((ck_sweep_kernel<T, MODE, DP>), dim3(S_ * H * ncb),
-                       dim3(256), lds, stream, raw, items, cap,
-                       (const T*)in.v, in.ldv, (float*)state,
-                       (const int*)seq_rows, S_, H, D, DV, p * nc, nc);
+#define CK_SWEEP(PART, RUNS)                                                 \
+  hipLaunchKernelGGL((ck_sweep_kernel<T, MODE, DP, PART>),                   \
+                     dim3(S_ * H * ncb * (RUNS)), dim3(256), lds, stream,    \
+                     raw, items, cap, (const T*)in.v, in.ldv, (float*)state, \
+                     (const int*)seq_rows, S_, H, D, DV, p * nc, nc, part,   \
+                     parts)
+    if constexpr (MODE == CK_GLA) {
+      if (parts > 1) {
+        CK_SWEEP(1, parts - 1);
+        CK_SWEEP(2, parts);
+        continue;
+      }
+    }
+    CK_SWEEP(0, 1);
+#undef CK_SWEEP
   }
   ck_read<T, MODE>(CK_PASS, raw, nullptr);
   return 0;
@@ -1287,6 +1450,8 @@ static int ck_launch_scalar(CK_ARGS) {
   float* gitems = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
   float* hitems = gitems + (size_t)cap * G * CkGroup<DP>::TOTAL;
   const int ncb = (DV + (lstm ? 1 : 0) + 31) / 32;
+  const int parts = ck_parts(MODE, T_, S_, H, DV);
+  float* part = hitems + (((size_t)cap * H * CkHead::TOTAL + 3) & ~(size_t)3);
   if (lstm)
     hipLaunchKernelGGL((ck_gates_kernel<T>), dim3(S_ * H), dim3(64), 0,
                        stream, ga, gw, ge, (const T*)in.a, in.lda,
@@ -1299,12 +1464,20 @@ static int ck_launch_scalar(CK_ARGS) {
                        dim3(cap, G, slices), dim3(256), 0, stream, gitems,
                        hitems, in, ga, gw, (const int*)seq_rows, S_, H, G, D,
                        scale, p * nc, nc);
-    hipLaunchKernelGGL((ck_sweep_scalar_kernel<T, MODE, DP>),
-                       dim3(S_ * H * ncb), dim3(256), 0, stream,
-                       lstm ? raw : (float*)out,
-                       lstm ? H * (DV + 1) : ldo, gitems, hitems, cap, in,
-                       (const float*)p2, (float*)state, (float*)aux,
-                       (const int*)seq_rows, S_, H, G, D, DV, p * nc, nc);
+#define CK_SWEEP(PART, RUNS)                                                 \
+  hipLaunchKernelGGL((ck_sweep_scalar_kernel<T, MODE, DP, PART>),            \
+                     dim3(S_ * H * ncb * (RUNS)), dim3(256), 0, stream,      \
+                     lstm ? raw : (float*)out, lstm ? H * (DV + 1) : ldo,    \
+                     gitems, hitems, cap, in, (const float*)p2,              \
+                     (float*)state, (float*)aux, (const int*)seq_rows, S_,   \
+                     H, G, D, DV, p * nc, nc, part, parts)
+    if (parts > 1) {
+      CK_SWEEP(1, parts - 1);
+      CK_SWEEP(2, parts);
+    } else {
+      CK_SWEEP(0, 1);
+    }
+#undef CK_SWEEP
   }
   if constexpr (MODE == CK_MLSTM) ck_read<T, MODE>(CK_PASS, raw, ge);
   return 0;
@@ -1366,7 +1539,8 @@ extern "C" long mx_chunk_scratch(int mode, int T_, int S_, int H, int G,
   int cap, nc, passes;
   ck_plan(mode, T_, S_, H, G, D, &cap, &nc, &passes);
   return ((ck_rows_floats(mode, T_, H, DV) + 3) & ~3l) +
-         cap * ck_chunk_floats(mode, ck_pad(D), H, G);
+         ((cap * ck_chunk_floats(mode, ck_pad(D), H, G) + 3) & ~3l) +
+         ck_part_floats(mode, T_, S_, H, D, DV);
 }
 
 extern "C" int mx_chunk_delta(void* out, int ldo, const void* r, int ldr,

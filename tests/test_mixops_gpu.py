@@ -431,3 +431,33 @@ def test_window_attention_kernels(H, G, D, DV, window, keep, softcap, sink):
         # fp32 up to the bf16 rounding of the result
         assert _rel(out[:, :H * DV].float().reshape(T, H, DV), want) < 3e-3
         assert (out[:, H * DV:] == 7.0).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("mode,H,D,DV", [
+    ("gla", 2, 40, 72), ("gla", 1, 128, 33), ("ssd", 4, 64, 32),
+    ("ssd", 2, 30, 40), ("mlstm", 2, 32, 31), ("mlstm", 1, 128, 64)])
+def test_recurrence_chunk_runs(mode, H, D, DV, dtype):
+    """Few heads and long segments: their chunks are walked in several runs
+    at once. Runs with a remainder, runs that stay empty in shorter segments,
+    fresh and continued states; a value that is no number reaches every later
+    run of its segment and nothing else."""
+    rows = _segs([700, 16, 401, 5, 90], [0, 3, 9, 0, 0])
+    x, state, aux, call = _recurrence(mode, H, D, DV, rows, dtype)
+    rows = torch.tensor(rows, dtype=torch.int32)
+    sg = state.cuda()
+    ag = aux.cuda() if aux is not None else None
+    bad = _to_gpu(x)
+    bad["v"][100] = float("nan")
+    lost = call(bad, sg.clone(), None if ag is None else ag.clone(),
+                rows.cuda())
+    got = call(_to_gpu(x), sg, ag, rows.cuda())
+    want = call(x, state, aux, rows)
+    # 2^-24 a token over up to 700 of them, both sides; outputs rounded once
+    assert _rel(got, want) < (2e-5 if dtype == torch.float32 else 6e-3)
+    assert _rel(sg, state) < 5e-6
+    if aux is not None:
+        assert _rel(ag, aux) < 5e-6
+    assert torch.equal(lost[:100], got[:100])
+    assert torch.equal(lost[700:], got[700:])
+    assert not torch.isfinite(lost[100:700]).all(1).any()
