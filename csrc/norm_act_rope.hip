@@ -11,111 +11,73 @@
 
 // ---------------------------------------------------------------------------
 // RMSNorm:  out[t, :] = x[t, :] * rsqrt(mean(x^2) + eps) * w
-// One workgroup per token row; row kept in registers between the two passes.
+// with ADD (the per-layer hot path)
+//   residual[t,:] += x[t,:];  x[t,:] = rmsnorm(residual[t,:]) * w
+// One workgroup per token row, the row and the weights in registers: 2 reads
+// and 2 writes per element. A decode batch is bound by the latency of the
+// chain, so the weights are asked for with the row and the waves' sums cross
+// one barrier (before: the weights after the second of two).
 // ---------------------------------------------------------------------------
-template <int BLOCK, int MAX_VPT>  // MAX_VPT = max ushort8 vectors per thread
+template <int BLOCK, int VPT, bool ADD>  // VPT ushort8 vectors per thread
 __global__ __launch_bounds__(BLOCK) void rms_norm_kernel(
-    unsigned short* __restrict__ out,      // [T, D]
+    unsigned short* __restrict__ out,      // [T, D]; with ADD in and out
     const unsigned short* __restrict__ x,  // [T, D]
+    unsigned short* __restrict__ residual, // [T, D], with ADD
     const unsigned short* __restrict__ w,  // [D]
     float eps, int D) {
-  const long t = blockIdx.x;
-  const unsigned short* xr = x + t * (long)D;
-  unsigned short* orow = out + t * (long)D;
+  const long row = blockIdx.x * (long)D;
+  unsigned short* orow = out + row;
+  const unsigned short* xr = ADD ? orow : x + row;
+  unsigned short* rr = ADD ? residual + row : nullptr;
 
-  float vals[MAX_VPT][8];
-  int nvec = 0;
-  float ss = 0.f;
-  for (int i = threadIdx.x * 8; i < D; i += BLOCK * 8) {
-    ps_bf16x8 xv = *(const ps_bf16x8*)(xr + i);
+  ps_bf16x8 xv[VPT], rv[VPT], wv[VPT];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      float f = ps_bf16_to_f32(xv[j]);
-      vals[nvec][j] = f;
-      ss += f * f;
+  for (int u = 0; u < VPT; u++) {
+    const int i = (u * BLOCK + (int)threadIdx.x) * 8;
+    if (i < D) {
+      xv[u] = *(const ps_bf16x8*)(xr + i);
+      if constexpr (ADD) rv[u] = *(const ps_bf16x8*)(rr + i);
+      wv[u] = *(const ps_bf16x8*)(w + i);
     }
-    nvec++;
+  }
+  float vals[VPT][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < VPT; u++) {
+    const int i = (u * BLOCK + (int)threadIdx.x) * 8;
+    if (i < D) {
+      ps_bf16x8 sv;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        float f = ps_bf16_to_f32(xv[u][j]);
+        if constexpr (ADD) f += ps_bf16_to_f32(rv[u][j]);
+        vals[u][j] = f;
+        ss += f * f;
+        sv[j] = ps_f32_to_bf16(f);
+      }
+      if constexpr (ADD) *(ps_bf16x8*)(rr + i) = sv;
+    }
   }
   // reduce ss across the block
   __shared__ float red[BLOCK / 64];
   ss = ps_group_sum<64>(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float tot = 0.f;
+  float tot = 0.f;
 #pragma unroll
-    for (int wv = 0; wv < BLOCK / 64; wv++) tot += red[wv];
-    red[0] = rsqrtf(tot / (float)D + eps);
-  }
-  __syncthreads();
-  const float inv = red[0];
+  for (int k = 0; k < BLOCK / 64; k++) tot += red[k];
+  const float inv = rsqrtf(tot / (float)D + eps);
 
-  nvec = 0;
-  for (int i = threadIdx.x * 8; i < D; i += BLOCK * 8) {
-    ps_bf16x8 wv = *(const ps_bf16x8*)(w + i);
-    ps_bf16x8 ov;
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      ov[j] = ps_f32_to_bf16(vals[nvec][j] * inv * ps_bf16_to_f32(wv[j]));
-    *(ps_bf16x8*)(orow + i) = ov;
-    nvec++;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Fused residual-add + RMSNorm (the per-layer hot path):
-//   residual[t,:] += x[t,:];  x[t,:] = rmsnorm(residual[t,:]) * w
-// Keeps the summed row in registers: 2 reads + 2 writes per element.
-// ---------------------------------------------------------------------------
-template <int BLOCK, int MAX_VPT>
-__global__ __launch_bounds__(BLOCK) void fused_add_rms_norm_kernel(
-    unsigned short* __restrict__ x,         // [T, D] in: delta, out: normed
-    unsigned short* __restrict__ residual,  // [T, D] in/out: accumulated
-    const unsigned short* __restrict__ w,   // [D]
-    float eps, int D) {
-  const long t = blockIdx.x;
-  unsigned short* xr = x + t * (long)D;
-  unsigned short* rr = residual + t * (long)D;
-
-  float vals[MAX_VPT][8];
-  int nvec = 0;
-  float ss = 0.f;
-  for (int i = threadIdx.x * 8; i < D; i += BLOCK * 8) {
-    ps_bf16x8 xv = *(const ps_bf16x8*)(xr + i);
-    ps_bf16x8 rv = *(const ps_bf16x8*)(rr + i);
-    ps_bf16x8 sv;
+  for (int u = 0; u < VPT; u++) {
+    const int i = (u * BLOCK + (int)threadIdx.x) * 8;
+    if (i < D) {
+      ps_bf16x8 ov;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      float f = ps_bf16_to_f32(xv[j]) + ps_bf16_to_f32(rv[j]);
-      vals[nvec][j] = f;
-      ss += f * f;
-      sv[j] = ps_f32_to_bf16(f);
+      for (int j = 0; j < 8; j++)
+        ov[j] = ps_f32_to_bf16(vals[u][j] * inv * ps_bf16_to_f32(wv[u][j]));
+      *(ps_bf16x8*)(orow + i) = ov;
     }
-    *(ps_bf16x8*)(rr + i) = sv;
-    nvec++;
-  }
-  __shared__ float red[BLOCK / 64];
-  ss = ps_group_sum<64>(ss);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float tot = 0.f;
-#pragma unroll
-    for (int wv = 0; wv < BLOCK / 64; wv++) tot += red[wv];
-    red[0] = rsqrtf(tot / (float)D + eps);
-  }
-  __syncthreads();
-  const float inv = red[0];
-
-  nvec = 0;
-  for (int i = threadIdx.x * 8; i < D; i += BLOCK * 8) {
-    ps_bf16x8 wv = *(const ps_bf16x8*)(w + i);
-    ps_bf16x8 ov;
-#pragma unroll
-    for (int j = 0; j < 8; j++)
-      ov[j] = ps_f32_to_bf16(vals[nvec][j] * inv * ps_bf16_to_f32(wv[j]));
-    *(ps_bf16x8*)(xr + i) = ov;
-    nvec++;
   }
 }
 
@@ -178,41 +140,35 @@ __global__ void rope_kernel(const int* __restrict__ positions,  // [T]
 // ---------------------------------------------------------------------------
 extern "C" {
 
+#define PS_NORM(VPT, ADD)                                                    \
+  rms_norm_kernel<256, VPT, ADD><<<dim3((unsigned)T), 256, 0, stream>>>(     \
+      (unsigned short*)out, (const unsigned short*)x,                        \
+      (unsigned short*)residual, (const unsigned short*)w, eps, D)
+#define PS_NORM_WIDTH(ADD)                                                   \
+  do {                                                                       \
+    if (D <= 2048)                                                           \
+      PS_NORM(1, ADD);                                                       \
+    else if (D <= 4096)                                                      \
+      PS_NORM(2, ADD);                                                       \
+    else if (D <= 8192)                                                      \
+      PS_NORM(4, ADD);                                                       \
+    else                                                                     \
+      PS_NORM(16, ADD);                                                      \
+  } while (0)
+
 void ps_rms_norm(void* out, const void* x, const void* w, float eps, long T,
                  int D, hipStream_t stream) {
-  constexpr int BLOCK = 256;
-  dim3 grid((unsigned)T);
-  if (D <= BLOCK * 8 * 2)
-    rms_norm_kernel<BLOCK, 2><<<grid, BLOCK, 0, stream>>>(
-        (unsigned short*)out, (const unsigned short*)x,
-        (const unsigned short*)w, eps, D);
-  else if (D <= BLOCK * 8 * 4)
-    rms_norm_kernel<BLOCK, 4><<<grid, BLOCK, 0, stream>>>(
-        (unsigned short*)out, (const unsigned short*)x,
-        (const unsigned short*)w, eps, D);
-  else
-    rms_norm_kernel<BLOCK, 16><<<grid, BLOCK, 0, stream>>>(
-        (unsigned short*)out, (const unsigned short*)x,
-        (const unsigned short*)w, eps, D);
+  void* residual = nullptr;
+  PS_NORM_WIDTH(false);
 }
 
-void ps_fused_add_rms_norm(void* x, void* residual, const void* w, float eps,
-                           long T, int D, hipStream_t stream) {
-  constexpr int BLOCK = 256;
-  dim3 grid((unsigned)T);
-  if (D <= BLOCK * 8 * 2)
-    fused_add_rms_norm_kernel<BLOCK, 2><<<grid, BLOCK, 0, stream>>>(
-        (unsigned short*)x, (unsigned short*)residual,
-        (const unsigned short*)w, eps, D);
-  else if (D <= BLOCK * 8 * 4)
-    fused_add_rms_norm_kernel<BLOCK, 4><<<grid, BLOCK, 0, stream>>>(
-        (unsigned short*)x, (unsigned short*)residual,
-        (const unsigned short*)w, eps, D);
-  else
-    fused_add_rms_norm_kernel<BLOCK, 16><<<grid, BLOCK, 0, stream>>>(
-        (unsigned short*)x, (unsigned short*)residual,
-        (const unsigned short*)w, eps, D);
+void ps_fused_add_rms_norm(void* out, void* residual, const void* w,
+                           float eps, long T, int D, hipStream_t stream) {
+  const void* x = nullptr;  // in place
+  PS_NORM_WIDTH(true);
 }
+#undef PS_NORM_WIDTH
+#undef PS_NORM
 
 void ps_silu_and_mul(void* out, const void* x, long T, int D,
                      hipStream_t stream) {
@@ -289,12 +245,97 @@ __global__ void fused_rope_cache_kernel(
   }
 }
 
+// The same where half a rotary width and what is left of a head are whole
+// 16-byte vectors: a thread rotates a pair of vectors or copies one, straight
+// from the packed row to where it belongs, with nothing read back and no
+// barrier. A token's vectors are shared by gridDim.y workgroups.
+template <typename KVT>
+__global__ __launch_bounds__(256) void fused_rope_cache_vec_kernel(
+    unsigned short* __restrict__ qkv, const int* __restrict__ positions,
+    const float* __restrict__ cos_sin, const long* __restrict__ slot_mapping,
+    KVT* __restrict__ k_cache, KVT* __restrict__ v_cache, int QH, int KH,
+    int HD, int ROT, long qkv_stride, int BS) {
+  using KVTr = ps_kv_traits<KVT>;
+  using kvec8 = typename KVTr::vec8;
+  const long t = blockIdx.x;
+  unsigned short* base = qkv + t * qkv_stride;
+  const float* cs = cos_sin + (long)positions[t] * ROT;
+  const long slot = slot_mapping[t];
+  const int half = ROT / 2, nr = half / 8, np = (HD - ROT) / 8, nv = HD / 8;
+  const int rot = (QH + KH) * nr;       // pairs of vectors to rotate
+  const int rest = rot + KH * np;       // then what of a key is not rotated
+  const int total = rest + KH * nv;     // then the values
+  // a cache row of a key or value head
+  auto row = [&](int h) {
+    return ((slot / BS * KH + h) * BS + slot % BS) * HD;
+  };
+  auto put = [&](KVT* cache, long at, ps_bf16x8 v) {
+    kvec8 o;
+#pragma unroll
+    for (int j = 0; j < 8; j++) o[j] = KVTr::from_f32(ps_bf16_to_f32(v[j]));
+    *(kvec8*)(cache + at) = o;
+  };
+  for (int i = blockIdx.y * 256 + threadIdx.x; i < total;
+       i += gridDim.y * 256) {
+    if (i < rot) {
+      const int h = i / nr, r = i % nr * 8;
+      unsigned short* hp = base + (long)h * HD + r;  // q heads then k heads
+      const ps_bf16x8 a = *(const ps_bf16x8*)hp;
+      const ps_bf16x8 b = *(const ps_bf16x8*)(hp + half);
+      float c[8], s[8];
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) {
+        *(float4*)(c + j) = *(const float4*)(cs + r + j);
+        *(float4*)(s + j) = *(const float4*)(cs + half + r + j);
+      }
+      ps_bf16x8 x, y;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float x1 = ps_bf16_to_f32(a[j]), x2 = ps_bf16_to_f32(b[j]);
+        x[j] = ps_f32_to_bf16(x1 * c[j] - x2 * s[j]);
+        y[j] = ps_f32_to_bf16(x2 * c[j] + x1 * s[j]);
+      }
+      *(ps_bf16x8*)hp = x;
+      *(ps_bf16x8*)(hp + half) = y;
+      if (h >= QH && slot >= 0) {
+        put(k_cache, row(h - QH) + r, x);
+        put(k_cache, row(h - QH) + r + half, y);
+      }
+    } else if (slot >= 0) {
+      const bool isv = i >= rest;
+      const int k = isv ? i - rest : i - rot, n = isv ? nv : np;
+      const int h = k / n, d = k % n * 8 + (isv ? 0 : ROT);
+      const ps_bf16x8 v = *(const ps_bf16x8*)(
+          base + (long)(QH + (isv ? KH : 0) + h) * HD + d);
+      put(isv ? v_cache : k_cache, row(h) + d, v);
+    }
+  }
+}
+
 extern "C" void ps_fused_rope_cache(void* qkv, const void* positions,
                                     const void* cos_sin,
                                     const void* slot_mapping, void* k_cache,
                                     void* v_cache, long T, int QH, int KH,
                                     int HD, int ROT, long qkv_stride, int BS,
                                     int kv_fp8, hipStream_t stream) {
+  if (ROT % 16 == 0 && HD % 8 == 0 && ROT <= HD && qkv_stride % 8 == 0 &&
+      (((size_t)qkv | (size_t)cos_sin | (size_t)k_cache | (size_t)v_cache) &
+       15) == 0) {
+    // few tokens: a vector a thread, many: a workgroup a token
+    const int work = (QH + KH) * (ROT / 16) + KH * (2 * HD - ROT) / 8;
+    const dim3 grid((unsigned)T, T < 512 ? (work + 255) / 256 : 1);
+#define PS_ROPE(KVT)                                                         \
+  fused_rope_cache_vec_kernel<KVT><<<grid, 256, 0, stream>>>(                \
+      (unsigned short*)qkv, (const int*)positions, (const float*)cos_sin,    \
+      (const long*)slot_mapping, (KVT*)k_cache, (KVT*)v_cache, QH, KH, HD,   \
+      ROT, qkv_stride, BS)
+    if (kv_fp8)
+      PS_ROPE(unsigned char);
+    else
+      PS_ROPE(unsigned short);
+#undef PS_ROPE
+    return;
+  }
   if (kv_fp8)
     fused_rope_cache_kernel<unsigned char>
         <<<dim3((unsigned)T), 256, 0, stream>>>(

@@ -798,3 +798,58 @@ def test_skinny_gemm_few_rows(M, N, K):
     gemm_policy.reset()
     via = gemm_policy.linear(x, w.cuda()).cpu().double()
     assert ((via - want).abs() <= want.abs() / 256 + 1e-3).all()
+
+
+@pytest.mark.parametrize("T,qh,kh,hd,rot,fp8", [
+    (1, 32, 8, 64, 64, False), (3, 7, 1, 128, 128, True),
+    (5, 4, 2, 96, 32, False), (511, 4, 4, 64, 48, True),
+    (513, 8, 2, 128, 128, False), (2, 4, 2, 64, 24, False)])
+def test_fused_rope_cache_vectors(T, qh, kh, hd, rot, fp8):
+    """Partly rotated heads, token counts around the line between several
+    workgroups a token and one, a rotary width of no whole vectors, tokens
+    without a slot."""
+    from production_stack_amd import _C
+
+    g = torch.Generator().manual_seed(T + hd)
+    bs, nb = 16, T // 16 + 2
+    qkv = torch.randn(T, (qh + 2 * kh) * hd, generator=g).to(torch.bfloat16)
+    cs = torch.randn(300, rot, generator=g)
+    pos = torch.randint(0, 300, (T,), generator=g, dtype=torch.int32)
+    slots = torch.randperm(nb * bs, generator=g)[:T]
+    slots[T // 2] = -1
+    qs, kvs = qh * hd, kh * hd
+    q, k = reference.rotary_embedding(
+        pos, qkv[:, :qs].clone(), qkv[:, qs:qs + kvs].clone(), cs, hd)
+    v = qkv[:, qs + kvs:].clone()
+    caches = [torch.zeros(nb, kh, bs, hd) for _ in range(2)]
+    for i in range(T):
+        if slots[i] >= 0:
+            for c, x in zip(caches, (k, v)):
+                c[slots[i] // bs, :, slots[i] % bs] = x[i].view(kh, hd).float()
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    got = [torch.zeros(nb, kh, bs, hd, dtype=dt, device="cuda")
+           for _ in range(2)]
+    gq = qkv.cuda()
+    _C.fused_rope_cache(gq, pos.cuda(), cs.cuda(), slots.cuda(), *got, qh, hd)
+    _close(gq[:, :qs], q)
+    _close(gq[:, qs:qs + kvs], k)
+    assert torch.equal(gq[:, qs + kvs:].cpu(), v)
+    # e4m3 keeps 4 bits: half a step is 2^-4, bf16's rounding may move one
+    tol = 2 ** -3 if fp8 else 2e-2
+    _close(got[0], caches[0], atol=2e-2, rtol=tol)
+    _close(got[1], caches[1].to(dt).float(), atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("D", [8, 2048, 2056, 4104, 8200, 16384])
+def test_rms_norm_widths(D):
+    """Widths around the vectors per thread, with and without the sum."""
+    g = torch.Generator().manual_seed(D)
+    x, r = (torch.randn(3, D, generator=g).to(torch.bfloat16)
+            for _ in range(2))
+    w = torch.randn(D, generator=g).to(torch.bfloat16)
+    _close(ops.rms_norm(x.cuda(), w.cuda(), 1e-5),
+           reference.rms_norm(x, w, 1e-5))
+    wn, wr = reference.fused_add_rms_norm(x.clone(), r.clone(), w, 1e-5)
+    gn, gr = ops.fused_add_rms_norm(x.cuda(), r.cuda(), w.cuda(), 1e-5)
+    _close(gr, wr)
+    _close(gn, wn)
