@@ -72,6 +72,8 @@ void ps_kv_dequant(void* out, const void* in, const void* scales, long rows,
 int ps_skinny_gemm_splits(int M, int N, int K);
 int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
                    int M, int N, int K, long x_stride, hipStream_t stream);
+int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
+                    int K, long x_stride, hipStream_t stream);
 int ps_gemm8p_splits(int M, int N, int K);
 int ps_gemm8p(void* out_bf16, void* ws, const void* x, const void* w, int M,
               int N, int K, long x_stride, hipStream_t stream);
@@ -361,6 +363,21 @@ void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w) {
   TORCH_CHECK(rc == 0, "skinny gemm launch failed");
 }
 
+void skinny_gated(at::Tensor out, at::Tensor x, at::Tensor w) {
+  CHECK_GPU_BF16(out);
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16,
+              "x must be bf16");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "x must be 2D row-major");
+  CHECK_GPU_BF16(w);
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  TORCH_CHECK(w.size(1) == K, "K mismatch");
+  TORCH_CHECK(out.numel() == (long)M * (N / 2), "out size mismatch");
+  const int rc = ps_skinny_gated(out.data_ptr(), x.data_ptr(), w.data_ptr(),
+                                 M, N, K, x.stride(0), current_stream());
+  TORCH_CHECK(rc == 0, "unsupported gated skinny gemm M=", M, " N=", N,
+              " K=", K);
+}
+
 void rms_norm_fp8(at::Tensor out_q, at::Tensor scales, at::Tensor x,
                   at::Tensor residual, at::Tensor w, double eps,
                   int64_t fused) {
@@ -510,5 +527,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "8-phase deep-pipelined bf16 GEMM (out = x @ w.T)");
   m.def("skinny_gemm", &skinny_gemm,
         "Split-K MFMA GEMM for decode-shaped (M<=128) projections");
+  m.def("skinny_gated", &skinny_gated,
+        "silu(x @ wg.T) * (x @ wu.T) of up to 16 rows, w = [wg; wu]");
   m.def("kv_dequant", &kv_dequant, "Row-wise int8 KV dequantization");
 }

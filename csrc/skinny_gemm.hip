@@ -40,7 +40,9 @@ PS_DEV ps_gbf16x8 ps_as_gbf16(ps_bf16x8 u) {
 // 10.3 us (17.4 with the split kernel, its merge included), 1 x 28672 x 4096 in
 // 46 (79; 5.1 TB/s), 1 x 2048 x 2048 in 5.0 (13.1). Reading x costs as many
 // load instructions as reading W: 16 rows of it make the wide one 68 us.
-template <int UC, int NW>
+// GATED: W holds N / 2 gate rows, then as many up rows; a workgroup takes eight
+// of each and writes silu(gate) up, both rounded to bf16 first: [M, N / 2].
+template <int UC, int NW, bool GATED>
 __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
     unsigned short* __restrict__ out, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w, int M, int N, int K, int x_stride) {
@@ -48,9 +50,10 @@ __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
   __shared__ __align__(16) float s_sum[NW][16 * PN];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int rc = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16;
+  const int n0 = blockIdx.x * (GATED ? 8 : 16);
   const int nc = K / 64;  // pieces
-  const unsigned short* wp = w + (long)(n0 + rc) * K + g * 8;
+  const int wrow = GATED && rc >= 8 ? N / 2 + n0 + rc - 8 : n0 + rc;
+  const unsigned short* wp = w + (long)wrow * K + g * 8;
   const auto xr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)x, 0, ((M - 1) * x_stride + K) * 2, 0x00020000);
   const unsigned int xo =
@@ -92,8 +95,18 @@ __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
 #pragma unroll
     for (int k = 0; k < NW; ++k)
       v += *(const ps_gf32x4*)(&s_sum[k][m * PN + n]);
-    if (m < M)
-      *(uint2*)(out + (long)m * N + n0 + n) = make_uint2(
+    if constexpr (GATED) {
+      // the quad of up columns is two lanes on
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float gv = ps_bf16_to_f32(ps_f32_to_bf16(v[r]));
+        const float uv = ps_bf16_to_f32(
+            ps_f32_to_bf16(__shfl_down(v[r], 2, 64)));
+        v[r] = gv / (1.f + __expf(-gv)) * uv;
+      }
+    }
+    if (m < M && (!GATED || n < 8))
+      *(uint2*)(out + (long)m * (GATED ? N / 2 : N) + n0 + n) = make_uint2(
           (unsigned int)ps_f32_to_bf16(v[0]) |
               ((unsigned int)ps_f32_to_bf16(v[1]) << 16),
           (unsigned int)ps_f32_to_bf16(v[2]) |
@@ -197,11 +210,40 @@ __global__ __launch_bounds__(256) void skinny_combine_kernel(
 
 
 
-extern "C" {
-
 // Rows of x for the kernel without splits; its byte offsets are 31 bits.
 static bool ps_skinny_rows(int M, int K, long x_stride) {
   return M <= 16 && x_stride >= 0 && (M - 1) * x_stride + K < (1L << 30);
+}
+
+template <bool GATED>
+static void ps_skinny_rows_go(void* out, const void* x, const void* w, int M,
+                              int N, int K, long x_stride,
+                              hipStream_t stream) {
+#define PS_SR(UC, NW)                                                       \
+  skinny_rows_kernel<UC, NW, GATED><<<N / 16, NW * 64, 0, stream>>>(        \
+      (unsigned short*)out, (const unsigned short*)x,                       \
+      (const unsigned short*)w, M, N, K, (int)x_stride)
+  // long rows: four pieces in flight a wave, else a piece and more waves (us
+  // at one row, 16 waves of one piece against 8 of four: 2048 x 2048 5.0 /
+  // 6.3, 16384 x 2048 16.5 / 20.8, 28672 x 4096 46.2 / 51.6, 4096 x 14336
+  // 28.0 / 25.2)
+  if (K <= 4096)
+    PS_SR(1, 16);
+  else
+    PS_SR(4, 8);
+#undef PS_SR
+}
+
+extern "C" {
+
+
+// out [M, N / 2] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu]; -1: not built
+int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
+                    int K, long x_stride, hipStream_t stream) {
+  if (M < 1 || N % 64 != 0 || K % 64 != 0 || !ps_skinny_rows(M, K, x_stride))
+    return -1;
+  ps_skinny_rows_go<true>(out, x, w, M, N, K, x_stride, stream);
+  return 0;
 }
 
 // ws == nullptr forces splits = 1. ps_skinny_gemm_splits reports the
@@ -223,19 +265,7 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
   int splits = ps_skinny_gemm_splits(M, N, K);
   if (splits < 0) return -1;
   if (ps_skinny_rows(M, K, x_stride)) {
-#define PS_SR(UC, NW)                                                       \
-  skinny_rows_kernel<UC, NW><<<N / 16, NW * 64, 0, stream>>>(               \
-      (unsigned short*)out_bf16, (const unsigned short*)x,                  \
-      (const unsigned short*)w, M, N, K, (int)x_stride)
-    // long rows: four pieces in flight a wave, else a piece and more waves (us
-    // at one row, 16 waves of one piece against 8 of four: 2048 x 2048 5.0 /
-    // 6.3, 16384 x 2048 16.5 / 20.8, 28672 x 4096 46.2 / 51.6, 4096 x 14336
-    // 28.0 / 25.2)
-    if (K <= 4096)
-      PS_SR(1, 16);
-    else
-      PS_SR(4, 8);
-#undef PS_SR
+    ps_skinny_rows_go<false>(out_bf16, x, w, M, N, K, x_stride, stream);
     return 0;
   }
   if (ws == nullptr) splits = 1;

@@ -324,8 +324,11 @@ class LlamaLayer(nn.Module):
             )
             if fp8 is not None:
                 gate_up = ops.fp8_linear(hidden, *fp8["gate_up"])
-            else:
+            elif meta.lora_groups or (slots is not None
+                                      and meta.lora_idx is not None):
                 gate_up = gemm_policy.linear(hidden, self.gate_up_proj)
+            else:
+                gate_up = None  # no adapter reads the two halves
         if slots is not None and meta.lora_idx is not None:
             slots.apply("gate", self.layer_idx, gate_up, hidden,
                         meta.lora_idx)
@@ -345,7 +348,8 @@ class LlamaLayer(nn.Module):
             act = gate_up[:, : self.inter]  # only LoRA reads act; unused
             mlp_out = ops.fp8_linear_rowwise(aq, sa, *fp8["down"])
         else:
-            act = ops.silu_and_mul(gate_up)
+            act = (gemm_policy.silu_mul(hidden, self.gate_up_proj)
+                   if gate_up is None else ops.silu_and_mul(gate_up))
             if fp8 is not None:
                 mlp_out = ops.fp8_linear(act, *fp8["down"])
             else:

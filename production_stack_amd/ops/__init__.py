@@ -256,6 +256,18 @@ def skinny_gemm(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def skinny_gated(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x @ wg.T) * (x @ wu.T) with w = [wg; wu], up to 16 rows: the
+    activation in the GEMM's last step, same roundings as skinny_gemm and
+    silu_and_mul one after the other. GPU only."""
+    _require_ext()
+    out = torch.empty(
+        (x.shape[0], w.shape[0] // 2), dtype=torch.bfloat16, device=x.device
+    )
+    _C.skinny_gated(out, x, w)
+    return out
+
+
 def cachegen_encode(q: torch.Tensor) -> torch.Tensor:
     """Entropy-encode int8 KV (CPU adaptive range coder, per-channel
     contexts). Falls back to a pure-Python reference when the extension

@@ -92,19 +92,34 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
                      and (x.requires_grad or w.requires_grad)))
 
 
+def _choose(x: torch.Tensor, w: torch.Tensor) -> int:
+    """0: the library, 1: skinny, 2: 8-phase."""
+    if not x.is_cuda or x.dtype != torch.bfloat16:
+        return 0
+    impl = _POLICY.get((x.shape[0], w.shape[0], w.shape[1]))
+    return int(_few_rows(x, w)) if impl is None else impl
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear with autotuned dispatch (no bias; Llama has none). The
     in-house kernels are bfloat16 only; other types take the library."""
-    if x.is_cuda and x.dtype == torch.bfloat16:
-        key = (x.shape[0], w.shape[0], w.shape[1])
-        impl = _POLICY.get(key)
-        if impl is None:
-            impl = int(_few_rows(x, w))
-        if impl:
-            from production_stack_amd import ops
+    impl = _choose(x, w)
+    if impl:
+        from production_stack_amd import ops
 
-            return (ops.skinny_gemm if impl == 1 else ops.gemm8p)(x, w)
+        return (ops.skinny_gemm if impl == 1 else ops.gemm8p)(x, w)
     return F.linear(x, w)
+
+
+def silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu_and_mul(linear(x, w)). Up to 16 rows that take the skinny kernel
+    have the activation in its last step (a launch of its own costs a decode
+    step 4.5 us a layer)."""
+    from production_stack_amd import ops
+
+    if x.shape[0] <= 16 and _choose(x, w) == 1:
+        return ops.skinny_gated(x, w)
+    return ops.silu_and_mul(linear(x, w))
 
 
 def reset() -> None:

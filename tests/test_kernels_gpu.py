@@ -853,3 +853,15 @@ def test_rms_norm_widths(D):
     gn, gr = ops.fused_add_rms_norm(x.cuda(), r.cuda(), w.cuda(), 1e-5)
     _close(gr, wr)
     _close(gn, wn)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 64), (3, 192, 2048), (16, 128, 4160), (5, 64, 1088)])
+def test_skinny_gated(M, N, K):
+    """The activation in the GEMM's last step: bit for bit what the two
+    kernels give one after the other."""
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(N, K, generator=g) / 16).to(torch.bfloat16).cuda()
+    want = ops.silu_and_mul(ops.skinny_gemm(x, w))
+    assert torch.equal(ops.skinny_gated(x, w), want)
