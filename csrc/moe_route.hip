@@ -13,9 +13,11 @@
 // which the all-experts path of small batches consumes directly.
 //
 // One workgroup per token: its waves share out the router outputs' dot
-// products (16-byte loads where the rows allow it), then the first wave
-// shares the outputs among its lanes for the softmax and the `top` rounds of
-// arg-max.
+// products (16-byte loads where the rows allow it),
+// then the first wave shares the outputs among its lanes for the softmax and
+// the `top` rounds of arg-max. A decode batch is bound by the latency of that
+// chain, so there a wave has one output where 16 waves suffice and eight loads of
+// a row in flight.
 #include "mix_common.h"
 
 #define MR_MAX_OUT 1024
@@ -26,11 +28,14 @@ PS_DEV float mr_wave_max(float v) {
   return v;
 }
 
-// Partial dot product of two rows over this lane's share of W entries.
+// Partial dot product of two rows over this lane's share of W entries, U loads
+// of each in flight.
+template <int U>
 PS_DEV float mr_dot(const float* a, const float* b, int W, int lane,
                     bool vec) {
   float acc = 0.f;
   if (vec) {
+#pragma unroll U
     for (int c = lane * 4; c < W; c += 256) {
       const float4 u = *(const float4*)(a + c), w = *(const float4*)(b + c);
       acc += u.x * w.x + u.y * w.y + u.z * w.z + u.w * w.w;
@@ -41,10 +46,12 @@ PS_DEV float mr_dot(const float* a, const float* b, int W, int lane,
   return acc;
 }
 
+template <int U>
 PS_DEV float mr_dot(const mx_bf16* a, const mx_bf16* b, int W, int lane,
                     bool vec) {
   float acc = 0.f;
   if (vec) {
+#pragma unroll U
     for (int c = lane * 8; c < W; c += 512) {
       const uint4 u = *(const uint4*)(a + c), w = *(const uint4*)(b + c);
       const unsigned int uu[4] = {u.x, u.y, u.z, u.w};
@@ -63,8 +70,8 @@ PS_DEV float mr_dot(const mx_bf16* a, const mx_bf16* b, int W, int lane,
   return acc;
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void moe_route_kernel(
+template <typename T, int U, int THREADS>
+__global__ __launch_bounds__(THREADS) void moe_route_kernel(
     int64_t* __restrict__ sel, float* __restrict__ wts,
     float* __restrict__ dense, const T* __restrict__ x, int ldx,
     const T* __restrict__ rw, const float* __restrict__ corr,
@@ -80,7 +87,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
   const T* xr = x + (size_t)t * ldx;
   for (int e = wave; e < n_out; e += nw) {
     const float acc =
-        mx_wave_sum(mr_dot(xr, rw + (size_t)e * W, W, lane, vec != 0));
+        mx_wave_sum(mr_dot<U>(xr, rw + (size_t)e * W, W, lane, vec != 0));
     if (lane == 0) score[e] = bias != nullptr ? acc + bias[e] : acc;
   }
   __syncthreads();
@@ -209,12 +216,24 @@ extern "C" int mx_moe_route(void* sel, void* wts, void* dense, const void* x,
                    (((size_t)x | (size_t)rw) & 15) == 0)
                       ? 1
                       : 0;
+  // Up to two workgroups a CU: a wave per output and deep loads (us, before ->
+  // with them: 128 rows of 2048, 16 outputs 7.9 -> 5.7; 128 of 4096, 64 outputs
+  // 31.6 -> 15.9; 512 of 4096, 8 outputs 7.4 -> 6.8). More rows hide the latency
+  // themselves (513 of 4096, 8 outputs 7.3 -> 8.1; 8192 of 2048 24.6 -> 25.7).
+#define MR_GO(U, THREADS, WAVES)                                             \
+  hipLaunchKernelGGL((moe_route_kernel<T, U, THREADS>), dim3(T_),            \
+                     dim3(64 * (WAVES)), lds, (hipStream_t)stream,           \
+                     (int64_t*)sel, (float*)wts, (float*)dense, (const T*)x, \
+                     ldx, (const T*)rw, (const float*)corr,                  \
+                     (const float*)bias, T_, W, n_out, top, sigmoid_scores,  \
+                     renorm, renorm_eps, scale, vec)
+  const int waves = n_out < 4 ? 4 : (n_out < 16 ? n_out : 16);
   MX_DISPATCH_DTYPE(dtype, {
-    hipLaunchKernelGGL((moe_route_kernel<T>), dim3(T_), dim3(256), lds,
-                       (hipStream_t)stream, (int64_t*)sel, (float*)wts,
-                       (float*)dense, (const T*)x, ldx, (const T*)rw,
-                       (const float*)corr, (const float*)bias, T_, W, n_out,
-                       top, sigmoid_scores, renorm, renorm_eps, scale, vec);
+    if (T_ <= 512)
+      MR_GO(8, 1024, waves);
+    else
+      MR_GO(1, 256, 4);
   })
+#undef MR_GO
   return 0;
 }

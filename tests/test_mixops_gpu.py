@@ -461,3 +461,23 @@ def test_recurrence_chunk_runs(mode, H, D, DV, dtype):
     assert torch.equal(lost[:100], got[:100])
     assert torch.equal(lost[700:], got[700:])
     assert not torch.isfinite(lost[100:700]).all(1).any()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("W,n_out,top", [
+    (64, 1, 1), (520, 3, 2), (4104, 5, 5), (2044, 17, 4), (4096, 70, 8)])
+def test_moe_route_waves(W, n_out, top, dtype):
+    """Both launch forms (up to 512 rows, more): the sums are made in the same
+    order, so the same rows give the same bits; weights as the reference's."""
+    g = torch.Generator().manual_seed(W)
+    x = torch.randn(513, W, generator=g).to(dtype)
+    rw = (torch.randn(n_out, W, generator=g) / W ** 0.5).to(dtype)
+    many = ops.moe_route(x.cuda(), rw.cuda(), top)
+    few = ops.moe_route(x[:512].cuda(), rw.cuda(), top)
+    for a, b in zip(many, few):
+        assert torch.equal(a[:512], b)
+    want, sel, _ = reference.moe_route(x, rw, top, "softmax", True, None, 1.0,
+                                       0.0)
+    # logits are fp32 sums of W products; equal ones may change places
+    assert (many[0].cpu() - want).abs().max() < 1e-4
+    assert (many[1].cpu() == sel).float().mean() > 0.999
