@@ -21,8 +21,10 @@
 // overlap. The form before (mfma_attention.hip; it remains for pooled blocks,
 // wider values and odd widths) staged 32 keys between two barriers with nothing
 // in flight and read values as single 16-bit words. 32/8 heads of 128, two
-// prompts of 2048: 161 us, 182 with a window of 1024 and a cap (598 and 408
-// before); 256 rows behind 2048 keys 92 (302).
+// prompts of 2048: 159 us, 159 with a window of 1024 and a cap (598 and 408
+// before; 182 with the cap's subtraction of the running maximum on its own); 256
+// rows behind 2048 keys 91 (302). Raised wave priority during the products made
+// it 5 % slower.
 // The token form is bound by the keys and values it reads, at few tokens by the
 // latency of its tiles: 64 tokens x 4001 keys 177 us, 5.9 TB/s (424 before);
 // window 1024 42 us (119); 8 tokens of it 16 us (32).
@@ -50,13 +52,13 @@ struct WaArgs {
   int hpb, hblocks;  // heads per workgroup, head blocks per KV head
 };
 
-// A raw product as a score in powers of two. With a cap: cap tanh(s / cap) =
-// cap (1 - 2 / (exp(2 s / cap) + 1)).
+// A raw product as a score in powers of two, less `base`. With a cap: cap
+// tanh(s / cap) = cap (1 - 2 / (exp(2 s / cap) + 1)); top = cap - base.
 template <bool CAP>
-PS_DEV float wa_score(const WaArgs& a, float st) {
-  if constexpr (!CAP) return st * a.scale2;
+PS_DEV float wa_score(const WaArgs& a, float st, float base, float top) {
+  if constexpr (!CAP) return st * a.scale2 - base;
   const float e = __builtin_amdgcn_exp2f(st * a.icap2);
-  return a.cap2 - 2.f * a.cap2 * __builtin_amdgcn_rcpf(e + 1.f);
+  return top - 2.f * a.cap2 * __builtin_amdgcn_rcpf(e + 1.f);
 }
 
 #define WA_KT 64
@@ -228,7 +230,7 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          w[16 * h + r] = wa_score<CAP>(a, st[h][r]) - base;
+          w[16 * h + r] = wa_score<CAP>(a, st[h][r], base, a.cap2 - base);
       const int dist = pos - j0 - 8 * hi;  // of this lane's first key
       if (kept) {
         const int left = mine ? k0 - j0 - 8 * hi : 0;
@@ -435,7 +437,7 @@ __global__ __launch_bounds__(256, 2) void window_token_kernel(WaArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int i = 4 * x + r;
-        p[i] = wa_score<CAP>(a, st[x][r]) - base;
+        p[i] = wa_score<CAP>(a, st[x][r], base, a.cap2 - base);
         if (i >= left) p[i] = -INFINITY;
         mx = fmaxf(mx, p[i]);
       }
