@@ -13,8 +13,8 @@
 //   x (tiny) is staged per 64-wide K-chunk in XOR-swizzled LDS and consumed
 //   as A-frags for ceil(M/16) m-tiles; per-k-chunk MFMA count scales with
 //   m-tiles while W traffic stays fixed.
-//   Split-K partials combine via fp32 atomicAdd into the pre-zeroed output
-//   (device-scope; SPLITS atomics per element).
+//   Split-K partials go to an fp32 workspace that a second kernel adds up.
+// That is the form for 17 to 256 rows; fewer have one of their own, below.
 // mfma_f32_16x16x32_bf16; operand k-pattern as verified in
 // csrc/tools/mfma_probe.hip.
 #include "ps_common.h"
