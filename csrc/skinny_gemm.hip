@@ -257,7 +257,12 @@ int ps_skinny_gemm_splits(int M, int N, int K) {
   int splits = target_wgs / (N / 64);
   if (splits < 1) splits = 1;
   if (splits > kchunks) splits = kchunks;
-  return splits;
+  if (splits < 1) return -1;  // K = 0
+  // the kernel hands out whole ranges of ceil(kchunks / splits) chunks: count
+  // the ranges that are not empty, since an empty one writes no partial and
+  // the combine pass would add what its workspace happened to hold
+  const int per_split = (kchunks + splits - 1) / splits;
+  return (kchunks + per_split - 1) / per_split;
 }
 
 int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,

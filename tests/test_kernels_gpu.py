@@ -865,3 +865,25 @@ def test_skinny_gated(M, N, K):
     w = (torch.randn(N, K, generator=g) / 16).to(torch.bfloat16).cuda()
     want = ops.silu_and_mul(ops.skinny_gemm(x, w))
     assert torch.equal(ops.skinny_gated(x, w), want)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (17, 3072, 2048),     # 21 ranges asked for, 32 pieces fill 16 of two
+    (64, 6144, 2048),     # 10 asked for, 8 filled
+    (200, 3072, 8192),    # 21 asked for, 19 filled
+    (32, 5120, 4096),     # 12 asked for, 11 filled
+    (256, 64, 128),       # a piece per range
+])
+def test_skinny_gemm_split_ranges(m, n, k):
+    """Every output is the sum of all K ranges, none of them empty."""
+    x = torch.randn(m, k, dtype=torch.bfloat16, device="cuda")
+    w = torch.randn(n, k, dtype=torch.bfloat16, device="cuda")
+    # leave not-a-numbers in memory the workspace may be given
+    del_me = torch.full((24 * m * n,), float("nan"), device="cuda")
+    del del_me
+    want = x.double() @ w.double().t()
+    for _ in range(3):
+        got = ops.skinny_gemm(x, w).double()
+        # one bf16 rounding of an fp32 sum of k products
+        err = ((got - want).abs() / (want.abs() + k ** 0.5)).max().item()
+        assert err < 2 ** -7, err
