@@ -240,7 +240,8 @@ extern "C" {
 // out [M, N / 2] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu]; -1: not built
 int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
                     int K, long x_stride, hipStream_t stream) {
-  if (M < 1 || N % 64 != 0 || K % 64 != 0 || !ps_skinny_rows(M, K, x_stride))
+  if (M < 1 || N < 64 || K < 64 || N % 64 != 0 || K % 64 != 0 ||
+      !ps_skinny_rows(M, K, x_stride))
     return -1;
   ps_skinny_rows_go<true>(out, x, w, M, N, K, x_stride, stream);
   return 0;
@@ -250,14 +251,13 @@ int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
 // split depth the heuristic will pick for a shape so the caller can size
 // the fp32 workspace.
 int ps_skinny_gemm_splits(int M, int N, int K) {
-  if (N % 64 != 0 || K % 64 != 0 || M > 256) return -1;
+  if (N < 64 || K < 64 || N % 64 != 0 || K % 64 != 0 || M > 256) return -1;
   if (M <= 16) return 1;
   const int kchunks = K / 64;
   const int target_wgs = 1024;
   int splits = target_wgs / (N / 64);
   if (splits < 1) splits = 1;
   if (splits > kchunks) splits = kchunks;
-  if (splits < 1) return -1;  // K = 0
   // the kernel hands out whole ranges of ceil(kchunks / splits) chunks: count
   // the ranges that are not empty, since an empty one writes no partial and
   // the combine pass would add what its workspace happened to hold
@@ -269,6 +269,7 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
                    int M, int N, int K, long x_stride, hipStream_t stream) {
   int splits = ps_skinny_gemm_splits(M, N, K);
   if (splits < 0) return -1;
+  if (M < 1) return 0;  // no rows: their size in bytes would wrap below
   if (ps_skinny_rows(M, K, x_stride)) {
     ps_skinny_rows_go<false>(out_bf16, x, w, M, N, K, x_stride, stream);
     return 0;

@@ -887,3 +887,17 @@ def test_skinny_gemm_split_ranges(m, n, k):
         # one bf16 rounding of an fp32 sum of k products
         err = ((got - want).abs() / (want.abs() + k ** 0.5)).max().item()
         assert err < 2 ** -7, err
+
+
+def test_skinny_gemm_nothing_to_do():
+    """No columns of K are refused for any number of rows, no rows give no
+    rows, also where they are a view of a wider matrix."""
+    w = torch.randn(64, 64, device="cuda").to(torch.bfloat16)
+    for m in (1, 16, 17):
+        x = torch.empty(m, 0, dtype=torch.bfloat16, device="cuda")
+        with pytest.raises(RuntimeError, match="unsupported"):
+            ops.skinny_gemm(x, w[:, :0].contiguous())
+        with pytest.raises(RuntimeError, match="unsupported"):
+            ops.skinny_gated(x, w[:, :0].contiguous())
+    wide = torch.randn(4, 256, device="cuda").to(torch.bfloat16)
+    assert ops.skinny_gemm(wide[:0, :64], w).shape == (0, 64)
