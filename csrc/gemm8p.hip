@@ -332,9 +332,9 @@ __global__ void gemm8p_combine_kernel(unsigned short* __restrict__ out,
 extern "C" {
 
 // Returns split count the heuristic picks (for ws sizing), or -1 if the
-// shape is unsupported (N % 256, K % 128).
+// shape is unsupported (N % 256, K % 128, nothing to do).
 int ps_gemm8p_splits(int M, int N, int K) {
-  if (N % 256 != 0 || K % 128 != 0) return -1;
+  if (M < 1 || N < 256 || K < 128 || N % 256 != 0 || K % 128 != 0) return -1;
   const int mt = (M + 255) / 256;
   const int nwg = mt * (N / 256);
   int splits = 384 / nwg;

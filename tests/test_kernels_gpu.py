@@ -901,3 +901,12 @@ def test_skinny_gemm_nothing_to_do():
             ops.skinny_gated(x, w[:, :0].contiguous())
     wide = torch.randn(4, 256, device="cuda").to(torch.bfloat16)
     assert ops.skinny_gemm(wide[:0, :64], w).shape == (0, 64)
+
+
+def test_gemm8p_nothing_to_do():
+    """No rows, no columns of W or of K are refused with an error."""
+    for m, n, k in ((4, 256, 0), (4, 0, 128), (0, 256, 128)):
+        x = torch.empty(m, k, dtype=torch.bfloat16, device="cuda")
+        w = torch.empty(n, k, dtype=torch.bfloat16, device="cuda")
+        with pytest.raises(RuntimeError, match="unsupported"):
+            ops.gemm8p(x, w)
