@@ -69,6 +69,22 @@ PS_DEV float kv_softmax(float* v, float mx, float* m, float* l, bool* moved) {
   return alpha;
 }
 
+// A sink (natural log units) joins a finished row of maximum m and denominator
+// l; returns the factor for the row's sums. It comes last: scores relative to
+// a sink far below them would lose their digits, and to one of minus infinity
+// be no numbers.
+PS_DEV float kv_sink(float sink, float* m, float* l) {
+  const float d = fmaf(sink, KV_LOG2E, -*m);
+  if (!(d > 0.f)) {
+    *l += __builtin_amdgcn_exp2f(d);
+    return 1.f;
+  }
+  const float f = __builtin_amdgcn_exp2f(-d);
+  *l = *l * f + 1.f;
+  *m = fminf(*m + d, -KV_LOW);  // the product may be past the largest float
+  return f;
+}
+
 // LDS written by some lanes of a wave is read by others of the same wave: the
 // wave's LDS accesses complete in order, this keeps the compiler to it.
 PS_DEV void kv_wave_sync() {

@@ -481,3 +481,35 @@ def test_moe_route_waves(W, n_out, top, dtype):
     # logits are fp32 sums of W products; equal ones may change places
     assert (many[0].cpu() - want).abs().max() < 1e-4
     assert (many[1].cpu() == sel).float().mean() > 0.999
+
+
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+@pytest.mark.parametrize("low", [-math.inf, -3.4e38, -1e9, -1e4, 1e9, 3e38])
+def test_window_attention_far_sinks(low, softcap):
+    """Sinks far from every score, beside ordinary ones: a low one takes
+    nothing, a high one everything, and neither costs the scores their
+    digits."""
+    g = torch.Generator().manual_seed(16)
+    H, G, D, DV, bs, L = 8, 2, 64, 64, 16, 200
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.bfloat16, g, 2)
+    ts = torch.tensor([0] * 70 + [1] * 3, dtype=torch.int32)
+    tp = torch.tensor(list(range(130, 200)) + [0, 1, 150], dtype=torch.int32)
+    T = len(ts)
+    q = torch.randn(T, H * D, generator=g).to(torch.bfloat16)
+    sinks = torch.randn(H, generator=g)
+    sinks[1::2] = low
+    want = reference.talk_attention(
+        q.float().reshape(T, H, D), kc.float(), vc.float(), tables, ts, tp,
+        D ** -0.5, 0, 90, True, None, 3, softcap, sinks)
+    for variant, splits in ((11, 0), (12, 1), (12, 3)):
+        out = ops.talk_attention(
+            q.cuda(), kc.cuda(), vc.cuda(), tables.cuda(), ts.cuda(),
+            tp.cuda(), D ** -0.5, H, window=90, keep_first=3, sink=True,
+            softcap=softcap, variant=variant, splits=splits,
+            sink_vals=sinks.cuda()).float().cpu().reshape(T, H, DV)
+        # fp32 up to the bf16 rounding of the result, head by head
+        assert _rel(out[:, ::2], want[:, ::2]) < 3e-3
+        if low > 0:
+            assert (out[:, 1::2] == 0).all()
+        else:
+            assert _rel(out[:, 1::2], want[:, 1::2]) < 3e-3
