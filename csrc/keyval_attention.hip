@@ -129,10 +129,6 @@ __global__ __launch_bounds__(256, OCC) void keyval_prompt_kernel(KvArgs a) {
     }
   }
   float m = KV_LOW, l = 0.f;
-  if (a.sink) {
-    m = (a.sink_vals != nullptr ? a.sink_vals[head] : 0.f) * KV_LOG2E;
-    l = hi == 0 ? 1.f : 0.f;  // a row's two lanes are added at the end
-  }
   kv_f32x16 acc[CB];
 #pragma unroll
   for (int c = 0; c < CB; ++c)
@@ -301,7 +297,10 @@ __global__ __launch_bounds__(256, OCC) void keyval_prompt_kernel(KvArgs a) {
 
   l += __shfl_xor(l, 32, 64);  // a lane summed its own keys
   if (!valid) return;
-  const float f = 1.0f / l;
+  float own = 1.f;
+  if (a.sink)
+    own = kv_sink(a.sink_vals != nullptr ? a.sink_vals[head] : 0.f, &m, &l);
+  const float f = own / l;
   unsigned short* o = a.out + (size_t)tok * a.ldout + (size_t)head * D;
   const bool vec = ((D | a.ldout) & 3) == 0 && ((size_t)a.out & 7) == 0;
   // acc[c][4 q + i] = O[row][32 c + 8 q + 4 hi + i]
@@ -375,12 +374,7 @@ __global__ __launch_bounds__(256, DK < 4 ? 4 : DK == 4 ? 3 : 1) void keyval_toke
       qr[s] = u.v;
     }
   }
-  // the sink belongs to the first wave of share 0
   float m = KV_LOW, l = 0.f;
-  if (a.sink && ks == 0 && wave == 0) {
-    m = (a.sink_vals != nullptr ? a.sink_vals[head] : 0.f) * KV_LOG2E;
-    l = kq == 0 ? 1.f : 0.f;  // a head's four lanes are added at the end
-  }
   kv_f32x4 acc[NB];
 #pragma unroll
   for (int c = 0; c < NB; ++c) acc[c] = {0.f, 0.f, 0.f, 0.f};
@@ -502,8 +496,8 @@ __global__ __launch_bounds__(256, DK < 4 ? 4 : DK == 4 ? 3 : 1) void keyval_toke
   const bool vec = (a.ldout & 3) == 0 && ((size_t)a.out & 7) == 0;
   for (int idx = tid; idx < nh * vpr; idx += 256) {
     const int h = idx / vpr, c = (idx - h * vpr) * 4;
-    const float mh = fmaxf(fmaxf(s_m[0][h], s_m[1][h]),
-                           fmaxf(s_m[2][h], s_m[3][h]));
+    float mh = fmaxf(fmaxf(s_m[0][h], s_m[1][h]),
+                     fmaxf(s_m[2][h], s_m[3][h]));
     float lt = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
@@ -514,6 +508,12 @@ __global__ __launch_bounds__(256, DK < 4 ? 4 : DK == 4 ? 3 : 1) void keyval_toke
       o[1] += v.y * f;
       o[2] += v.z * f;
       o[3] += v.w * f;
+    }
+    if (a.sink && ks == 0) {  // the sink is share 0's
+      const float own = kv_sink(
+          a.sink_vals != nullptr ? a.sink_vals[h0 + h] : 0.f, &mh, &lt);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] *= own;
     }
     if (a.KS == 1) {
       const float f = 1.0f / lt;

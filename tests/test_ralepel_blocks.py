@@ -3,6 +3,8 @@ through scattered and previously used pages) against the float64 oracle in
 tests/oracle_ralepel.py, and, marked gpu, the HIP kernels against the
 reference ops."""
 
+import math
+
 import pytest
 import torch
 
@@ -648,3 +650,33 @@ def test_vector_kernels_take_factors_and_slopes(variant, shape):
             variant=variant, splits=splits, key_scale=fac.cuda(),
             slopes=slopes.cuda())
         assert relerr(got, want) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("low", [-math.inf, -3.4e38, -1e9, -1e4, 1e9, 3e38])
+def test_keyval_far_sinks(low):
+    """Sinks far from every score beside ordinary ones: a low one takes
+    nothing, a high one everything, and neither costs the scores their
+    digits; portions, and single tokens in one and several shares."""
+    H, G, D, win, BS = 8, 2, 64, 70, 16
+    lens = [150, 33, 1]
+    tables, rows, fac = page_setup(lens, G, D, BS, 3)
+    pos = torch.cat([torch.arange(90, 150), torch.tensor([32, 0])]).int()
+    seq = torch.tensor([0] * 60 + [1, 2]).int()
+    T = len(pos)
+    q = rnd((T, H * D), 2, 1.0, torch.bfloat16)
+    sv = rnd((H,), 5)
+    sv[1::2] = low
+    want = R.talk_attention(
+        q.reshape(T, H, D), rows, rows, tables, seq, pos, D ** -0.5, 0, win,
+        True, None, 0, 0.0, sv, D, None, fac, None).float()
+    cc = rows.cuda()
+    for variant, splits in ((8, 0), (9, 1), (9, 3)):
+        got = ops.talk_attention(
+            q.cuda(), cc, cc, tables.cuda(), seq.cuda(), pos.cuda(),
+            D ** -0.5, H, variant=variant, splits=splits, window=win,
+            sink=True, vdim=D, sink_vals=sv.cuda(), key_scale=fac.cuda()
+        ).float().cpu().view(T, H, D)
+        err = (got - want).norm(dim=-1)
+        assert float((err[:, ::2] / want[:, ::2].norm(dim=-1)).max()) < 1e-2
+        assert float((err / want.norm(dim=-1).clamp_min(1e-30)).max()) < 1e-2
