@@ -105,7 +105,10 @@ __global__ __launch_bounds__(256, 2) void expand_attn_kernel(XaArgs a) {
 
   float m = -3.0e38f, l = 0.f;
   if (a.sink) {
+    // within the finite numbers: a tile that hides all its keys from a row
+    // leaves it at this maximum
     m = (a.sink_vals != nullptr ? a.sink_vals[head] : 0.f) * 1.44269504f;
+    m = fminf(fmaxf(m, -3.0e38f), 3.0e38f);
     l = hi == 0 ? 1.f : 0.f;  // a row's two lanes are added at the end
   }
   xa_f32x16 acc[CB];

@@ -93,9 +93,10 @@ __global__ __launch_bounds__(512, 2) void latent_decode_kernel(LdArgs a) {
   const int orow = lane & 31, hi = lane >> 5;
   const int col0 = wave * 32 * CW;
   const bool cols = col0 < DV;
-  auto sink2 = [&](int r) -> float {
-    return (a.sink_vals != nullptr ? a.sink_vals[min(hb + r, a.H - 1)] : 0.f) *
-           1.44269504f;
+  auto sink2 = [&](int r) -> float {  // within the finite numbers
+    const float s =
+        a.sink_vals != nullptr ? a.sink_vals[min(hb + r, a.H - 1)] : 0.f;
+    return fminf(fmaxf(s * 1.44269504f, -3.0e38f), 3.0e38f);
   };
   const bool own_sink = a.sink && ks == 0;
   float m_s = own_sink ? sink2(srow) : -3.0e38f;   // of head row srow

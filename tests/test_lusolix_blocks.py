@@ -597,3 +597,44 @@ def test_experts_sum_kernel(dtype, W_):
         got = ops.experts_sum(c(ys), c(pos), top, c(weights), 0.25, c(s), E,
                               c(x), c(a), c(b))
         assert got.dtype == torch.float32 and relerr(got, want) < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("low", [float("-inf"), -3.4e38, -1e9, 3e38])
+def test_latent_far_sinks(low):
+    """Sinks far from every score beside ordinary ones, in the expanded form
+    (a first tile that hides all its keys from some rows) and for single
+    tokens."""
+    H, D, DV, win, n = 4, 64, 64, 40, 200
+    bf = torch.bfloat16
+    sv = rnd((H,), 5)
+    sv[1::2] = low
+    k, vt = rnd((256, H * D), 2, 1.0, bf), rnd((H * DV, 256), 3, 1.0, bf)
+    k[n:] = 0
+    vt[:, n:] = 0
+    q = rnd((n, H * D), 1, 1.0, bf)
+    tiles = torch.tensor([(0, 128, 0, 0), (128, n - 128, 0, 128)]).int()
+    want = R.expanded_attention(q, k, vt, tiles, 0.2, H, win, True, sv, None)
+    got = ops.expanded_attention(
+        q.cuda(), k.cuda(), vt.cuda(), tiles.cuda(), 0.2, H, window=win,
+        sink=True, sink_vals=sv.cuda()).cpu()
+    pairs = [(got, want)]
+    cache = rnd((8, 1, 16, D), 4, 1.0, bf)
+    table = torch.randperm(8, generator=torch.Generator().manual_seed(1))
+    table = table.int()[None].repeat(3, 1)
+    pos = torch.tensor([0, 63, 120], dtype=torch.int32)
+    seq = torch.arange(3, dtype=torch.int32)
+    want = R.talk_attention(q[:3].reshape(3, H, D), cache, cache, table, seq,
+                            pos, 0.2, 0, 0, True, None, 0, 0.0, sv, D)
+    cc = cache.cuda()
+    for splits in (1, 2):
+        got = ops.talk_attention(
+            q[:3].cuda(), cc, cc, table.cuda(), seq.cuda(), pos.cuda(), 0.2,
+            H, variant=7, splits=splits, sink=True, vdim=D,
+            sink_vals=sv.cuda()).cpu()
+        pairs.append((got, want.reshape(3, H * D)))
+    for got, want in pairs:
+        got = got.float().view(len(got), H, -1)
+        want = want.float().view(len(want), H, -1)
+        err, size = (got - want).norm(dim=-1), want.norm(dim=-1)
+        assert float((err / size.clamp_min(1e-30)).max()) < 1e-2
