@@ -28,9 +28,10 @@
 // remains for fp32 and other shapes): 13 TF/s, every product of the mix and of
 // both contractions an fp32 multiply-add. Here a tile takes about 4600 cycles
 // of a SIMD's matrix unit, 1024 of them the scores, 2048 the mix, 1536 the
-// output, and 14500 in all: with one workgroup a CU (its LDS) the four barriers
+// output, and 14200 in all: with one workgroup a CU (its LDS) the four barriers
 // between those stages leave the matrix unit waiting. 32/8 heads of 128, 4099
-// rows in two prompts, chunks of 2048: 0.67 ms (11.7 before).
+// rows in two prompts, chunks of 2048: 0.63 ms (11.7 before; 0.65 with a branch
+// around every exponential).
 #include "attn_common.h"
 #include "scan_common.h"
 
@@ -38,6 +39,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 tm_bf16x8;
 typedef __attribute__((ext_vector_type(4))) short tm_s4;
 typedef __attribute__((address_space(3))) tm_s4 tm_lds_s4;
 typedef __attribute__((ext_vector_type(4))) unsigned int tm_u4;
+typedef __attribute__((ext_vector_type(2))) unsigned short tm_us2;
 
 union TmPack {
   tm_bf16x8 v;
@@ -68,6 +70,9 @@ struct TmArgs {
   const float* sink_vals;
 };
 
+// A bf16 entry that is an infinity or no number.
+PS_DEV bool tm_odd(unsigned int e) { return (e & 0x7f80u) == 0x7f80u; }
+
 // ND = D / 32, NV = DV / 16; CAP: with a score cap
 template <int ND, int NV, bool CAP>
 __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
@@ -82,6 +87,8 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   float* sAL = sPM + 8 * 256;                      // [16][16]
   unsigned short* sV = (unsigned short*)(sAL + 256);  // [4][32][PV]
   __shared__ int s_seq[16], s_pos[16];
+  // first and last tile of a run whose values (of two waves) are not all finite
+  __shared__ int s_odd[4][2];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, n = lane & 15;
@@ -122,7 +129,9 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   float m[4], l[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    m[i] = a.sink ? (a.sink_vals != nullptr ? a.sink_vals[h0 + i] : 0.f)
+    m[i] = a.sink ? (a.sink_vals != nullptr
+                         ? fmaxf(a.sink_vals[h0 + i], PS_NEG_INF)
+                         : 0.f)
                   : PS_NEG_INF;
     l[i] = a.sink && wave == 0 ? 1.f : 0.f;
   }
@@ -197,6 +206,10 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
                 a.vr +
             (lane % PR) * 8);
       __syncthreads();
+      if (t == 0 && threadIdx.x < 4) {  // read by all for the run before
+        s_odd[threadIdx.x][0] = nt;
+        s_odd[threadIdx.x][1] = -1;
+      }
 
       // mixed scores x[e][i]: key 4 wave + e, head h0 + i, row n
       ck_f32x4 x[4];
@@ -223,7 +236,8 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
         const int j = j0 + 4 * wave + e;
         const bool vis = j >= my_lo && j <= my_hi;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[e][i] = vis ? x[e][i] : PS_NEG_INF;
+        for (int i = 0; i < 4; ++i)  // no number counts as hidden
+          x[e][i] = vis ? fmaxf(x[e][i], PS_NEG_INF) : PS_NEG_INF;
       }
       float* pm = sPM + 4 * g * 16 + n;
 #pragma unroll
@@ -238,19 +252,44 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) mn = fmaxf(mn, pm[k * 256 + i * 16]);
         // nothing visible yet: weights of 0 below, whatever is subtracted
+        // (ck_exp of minus infinity; no branches around it)
         const float ms = mn > PS_NEG_INF ? mn : 0.f;
-        const float al = m[i] > PS_NEG_INF ? ck_exp(m[i] - ms) : 0.f;
+        const float al = ck_exp(m[i] - ms);
         m[i] = mn;
         if (wave == 0) sAL[(4 * g + i) * 16 + n] = al;
         float sum = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          x[e][i] = x[e][i] > PS_NEG_INF ? ck_exp(x[e][i] - ms) : 0.f;
+          x[e][i] = ck_exp(x[e][i] - ms);
           sum += x[e][i];
         }
         l[i] = l[i] * al + sum;
         *(ck_f32x4*)(sS + ((4 * g + i) * 16 + n) * TM_PS + 4 * wave) =
             ck_f32x4{x[0][i], x[1][i], x[2][i], x[3][i]};
+      }
+      // Values that are not finite stay out of the products, where a hidden
+      // key's weight of zero would carry them to rows that do not see it (rows
+      // of other sequences among them); they join behind the walk.
+      tm_us2 top = {0, 0};
+#pragma unroll
+      for (int u = 0; u < NL; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          top = __builtin_elementwise_max(
+              top, __builtin_bit_cast(tm_us2, vr[u][i] & 0x7fff7fffu));
+      if (__any(tm_odd(top[0]) || tm_odd(top[1]))) {
+#pragma unroll
+        for (int u = 0; u < NL; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const unsigned int e = vr[u][i];
+            vr[u][i] = (tm_odd(e) ? 0u : e & 0xffffu) |
+                       (tm_odd(e >> 16) ? 0u : e & 0xffff0000u);
+          }
+        if (lane == 0) {
+          atomicMin(&s_odd[wave >> 1][0], t);
+          atomicMax(&s_odd[wave >> 1][1], t);
+        }
       }
 #pragma unroll
       for (int u = 0; u < NL; ++u)
@@ -298,6 +337,28 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
       // not before: beside the value operands they would spill
       fetch_k(ridx);
       __syncthreads();  // the weights are read
+    }
+    // values that are not finite, to the rows that see their keys: whatever
+    // the weight, which is above zero, they decide the sum
+    const int odd0 = s_odd[wave >> 1][0], odd1 = s_odd[wave >> 1][1];
+#pragma unroll 1
+    for (int j = kmin + odd0 * TM_KT;
+         j < min(kmin + (odd1 + 1) * TM_KT, kmax + 1); ++j) {
+      if (j < my_lo || j > my_hi) continue;
+      const unsigned short* p =
+          a.vc + ((int64_t)(table[j / a.BS] * a.G + vgrp) * a.BS + j % a.BS) *
+                     a.vr + 4 * g;
+#pragma unroll
+      for (int c = 0; c < NV; ++c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const unsigned int e = p[16 * c + i];
+          const float x = tm_odd(e) ? __uint_as_float(e << 16) : 0.f;
+          acc[0][c][i] += x;
+          acc[1][c][i] += x;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     rs = re;
   }

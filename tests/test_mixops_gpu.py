@@ -513,3 +513,41 @@ def test_window_attention_far_sinks(low, softcap):
             assert (out[:, 1::2] == 0).all()
         else:
             assert _rel(out[:, 1::2], want[:, 1::2]) < 3e-3
+
+
+@pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
+@pytest.mark.parametrize("G,D,DV", [(8, 128, 128), (2, 64, 64)])
+def test_talk_attention_value_no_number(G, D, DV, bad):
+    """A cached value that is no finite number reaches the rows that see its
+    key and no other: neither earlier rows of its sequence nor another
+    sequence's in the same 16, to the last bit."""
+    g = torch.Generator().manual_seed(17)
+    H, bs, L = 32, 16, 120
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.bfloat16, g, 2)
+    # rows 0-5 sequence 0, 6-15 sequence 1, 16-20 sequence 0 again
+    ts = torch.tensor([0] * 6 + [1] * 10 + [0] * 5, dtype=torch.int32)
+    tp = torch.tensor(list(range(60, 66)) + list(range(90, 100))
+                      + list(range(66, 71)), dtype=torch.int32)
+    T = len(ts)
+    q = torch.randn(T, H * D, generator=g).to(torch.bfloat16).cuda()
+    talk = (torch.eye(H) + 0.3 * torch.randn(H, H, generator=g)).cuda()
+
+    def run(v, variant):
+        return ops.talk_attention(
+            q, kc.cuda(), v.cuda(), tables.cuda(), ts.cuda(), tp.cuda(),
+            D ** -0.5, H, window=40, sink=True, talk=talk,
+            variant=variant).cpu().reshape(T, H, DV)
+
+    clean = run(vc, 10)
+    j, col = 94, 5                      # key 94 of sequence 1: rows 10-15
+    broken = vc.clone()
+    broken[tables[1, j // bs], 0, j % bs, col] = bad
+    got = run(broken, 10)
+    old = run(broken, 1)                # the general kernel
+    sees = torch.zeros(T, H, DV, dtype=torch.bool)
+    sees[10:16, :H // G, col] = True
+    assert torch.equal(got[~sees], clean[~sees])
+    for want in (math.inf, -math.inf):
+        assert torch.equal(got == want, old == want)
+    assert torch.equal(got.isnan(), old.isnan())
+    assert not torch.isfinite(got[sees]).any()
