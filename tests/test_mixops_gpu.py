@@ -551,3 +551,28 @@ def test_talk_attention_value_no_number(G, D, DV, bad):
         assert torch.equal(got == want, old == want)
     assert torch.equal(got.isnan(), old.isnan())
     assert not torch.isfinite(got[sees]).any()
+
+
+@pytest.mark.parametrize("mode", ["general", "channel"])
+def test_recurrence_chunk_long_keys(mode):
+    """Keys whose squared norm leaves fp32's range: their unit vectors are
+    zero in whole chunks as they are token by token."""
+    segs = [(0, 20, 3, 0)]
+    x, state, aux, call = _recurrence(mode, 2, 32, 32, segs, torch.float32)
+    xg = _to_gpu(x)
+    xg["k"][7] *= 1e20
+    if mode == "channel":
+        xg["q"][9] *= 1e20
+    sg, st = state.cuda(), state.cuda()
+    whole = call(xg, sg, None,
+                 torch.tensor(segs, dtype=torch.int32).cuda())
+    # the same rows in portions too short for a chunk
+    parts = []
+    for a in (0, 10):
+        y = {k: v[a:a + 10] if v.shape[0] == 20 and v.dim() == 2 else v
+             for k, v in xg.items()}
+        parts.append(call(y, st, None, torch.tensor(
+            [(0, 10, 3 + a, 0)], dtype=torch.int32).cuda()))
+    assert torch.isfinite(whole).all()
+    assert _rel(whole, torch.cat(parts)) < 2e-5
+    assert _rel(sg, st) < 2e-5
