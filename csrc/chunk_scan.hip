@@ -1324,10 +1324,10 @@ static void ck_plan(int mode, int T_, int S_, int H, int G, int D, int* cap,
   if (all > T_ / 8 + 1) all = T_ / 8 + 1;
   long fit = CK_BYTES / per;
   if (fit < S_) fit = S_;
-  const int longest = (T_ - S_ + 1 + 15) / 16;  // chunks of one segment
+  const int longest = (T_ + 15) / 16;  // chunks of one segment, others empty
   if (all <= fit) {
     *cap = (int)all;
-    *nc = longest > 0 ? longest : 1;
+    *nc = longest;
     *passes = 1;
     return;
   }

@@ -576,3 +576,21 @@ def test_recurrence_chunk_long_keys(mode):
     assert torch.isfinite(whole).all()
     assert _rel(whole, torch.cat(parts)) < 2e-5
     assert _rel(sg, st) < 2e-5
+
+
+@pytest.mark.parametrize("mode", RECURRENCES)
+def test_recurrence_empty_segments(mode):
+    """Segments without rows beside a long one: all of its rows are walked."""
+    lens = [0, 60, 0, 0, 1] + [0] * 30
+    rows = _segs(lens, [2] * len(lens))
+    x, state, aux, call = _recurrence(mode, 2, 32, 32, rows, torch.float32)
+    rows = torch.tensor(rows, dtype=torch.int32)
+    sg = state.cuda()
+    ag = aux.cuda() if aux is not None else None
+    got = call(_to_gpu(x), sg, ag, rows.cuda())
+    want = call(x, state, aux, rows)
+    # fp32 sums of up to 60 tokens x 32 channels
+    assert _rel(got, want) < 2e-5
+    assert _rel(sg, state) < 2e-6
+    if aux is not None:
+        assert _rel(ag, aux) < 2e-6
