@@ -21,6 +21,10 @@ Groups (one shared library each):
 from __future__ import annotations
 
 import ctypes
+import functools
+import glob
+import hashlib
+import mmap
 import os
 import shutil
 import subprocess
@@ -114,9 +118,49 @@ def _hipcc() -> str:
     return exe
 
 
+SRC_DIR = os.path.join(ROOT, "csrc")
+_KEY = b"mx_build_key="
+
+
+@functools.lru_cache(maxsize=None)
+def source_key(group: str) -> str:
+    """Names what a group's library is built from: its units and defines, the
+    shared headers, the flags. Empty where the sources are not there."""
+    units = GROUPS[group]
+    names = sorted({src for src, _ in units})
+    names += sorted(os.path.basename(h)
+                    for h in glob.glob(os.path.join(SRC_DIR, "*.h")))
+    digest = hashlib.sha256(repr((HIPCC_FLAGS, units, names)).encode())
+    for name in names:
+        try:
+            with open(os.path.join(SRC_DIR, name), "rb") as f:
+                digest.update(hashlib.sha256(f.read()).digest())
+        except OSError:
+            return ""
+    return digest.hexdigest()[:16]
+
+
+def built_key(path: str) -> str:
+    """The key in a built library, empty where it has none."""
+    with open(path, "rb") as f, mmap.mmap(
+            f.fileno(), 0, access=mmap.ACCESS_READ) as m:
+        at = m.find(_KEY)
+        return m[at + len(_KEY):at + len(_KEY) + 16].decode() if at >= 0 else ""
+
+
+def current(group: str) -> bool:
+    """A library is there and built from the sources that are. The entry
+    points are called without types: one of other sources may take other
+    arguments and would read them as its own."""
+    path = LIB_PATHS[group]
+    return os.path.exists(path) and source_key(group) in (
+        "", built_key(path))
+
+
 def _build_group(group: str) -> str:
     hipcc = _hipcc()
-    src_dir = os.path.join(ROOT, "csrc")
+    src_dir = SRC_DIR
+    key = source_key(group)
     units = GROUPS[group]
     tmp = tempfile.mkdtemp(prefix=f"mixops-{group}-", dir=PKG)
     try:
@@ -134,10 +178,14 @@ def _build_group(group: str) -> str:
 
         with ThreadPoolExecutor(max_workers=len(units)) as ex:
             objs = list(ex.map(compile_one, enumerate(units)))
+        mark = os.path.join(tmp, "key.c")
+        with open(mark, "w") as f:
+            f.write('__attribute__((used)) const char mx_build_key[] = "%s";\n'
+                    % (_KEY.decode() + key))
         out = os.path.join(tmp, "lib.so")
         r = subprocess.run(
             [hipcc, "-shared", "-fPIC", "--offload-arch=gfx950", *objs,
-             "-o", out],
+             "-x", "c", mark, "-o", out],
             stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stdout[-4000:]}")
@@ -149,9 +197,11 @@ def _build_group(group: str) -> str:
 
 def build(force: bool = False, groups=None) -> str:
     """Compile the libraries in-tree (atomic replace), all groups unless
-    `groups` names some. Returns the core library's path."""
-    todo = [g for g in (groups or GROUPS)
-            if force or not os.path.exists(LIB_PATHS[g])]
+    `groups` names some; those that are current only with `force`. Returns
+    the core library's path."""
+    if force:
+        source_key.cache_clear()
+    todo = [g for g in (groups or GROUPS) if force or not current(g)]
     with ThreadPoolExecutor(max_workers=max(len(todo), 1)) as ex:
         list(ex.map(_build_group, todo))
     return LIB_PATH
@@ -159,7 +209,8 @@ def build(force: bool = False, groups=None) -> str:
 
 class _Libs:
     """Attribute access resolves an entry point in its group's library,
-    which is loaded (and built, when nothing is built) on first use."""
+    which is loaded (and built, when it is not there or was built from other
+    sources) on first use."""
 
     def __init__(self) -> None:
         self._handles = {}
@@ -167,7 +218,7 @@ class _Libs:
     def _handle(self, group: str):
         h = self._handles.get(group)
         if h is None:
-            if not os.path.exists(LIB_PATHS[group]):
+            if not current(group):
                 _build_group(group)
             h = ctypes.CDLL(LIB_PATHS[group])
             self._handles[group] = h
