@@ -361,6 +361,10 @@ __global__ __launch_bounds__(256, 2) void window_token_kernel(WaArgs a) {
     }
   }
   float m = KV_LOW, l = 0.f;
+  // Values the compiler cannot see through where there is a sink: knowing the
+  // first tile's state, it lays the walk out such that every tile waits longer
+  // (32/8 heads of 64, 8000 keys among 16 x 1000: 54 -> 59 us).
+  if (a.sink && ks == 0 && wave == 0) asm volatile("" : "+v"(m), "+v"(l));
   kv_f32x4 acc[NB];
 #pragma unroll
   for (int c = 0; c < NB; ++c) acc[c] = {0.f, 0.f, 0.f, 0.f};
