@@ -50,6 +50,7 @@ struct WaArgs {
   int KS;
   float* part;
   int hpb, hblocks;  // heads per workgroup, head blocks per KV head
+  int tpt;           // tokens per workgroup (prompt form)
 };
 
 // A raw product as a score in powers of two, less `base`. With a cap: cap
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int row = lane & 31, hi = lane >> 5;
   const int D = a.D, DV = a.DV, rep = a.H / a.G, HPB = a.hpb;
-  const int TPT = 128 / HPB;
+  const int TPT = a.tpt;
   const int NT = (a.T + TPT - 1) / TPT;
   // rows that see the most keys first
   const int GH = a.G * a.hblocks;
@@ -125,13 +126,23 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
                   4 * (i16 & 3);
   const unsigned vis = a.window > 0 ? a.window : 0x7fffffff;
 
+  // rows that do not continue the sequence of the row before them
+  auto starts = [&](int i) {
+    return i < ntok && (i == 0 || s_seq[i] != s_seq[i - 1] ||
+                        s_pos[i] != s_pos[i - 1] + 1);
+  };
+  const unsigned long long start0 = __ballot(starts(lane)),
+                           start1 = __ballot(starts(64 + lane));
+  auto next_start = [&](int i) {  // behind row i
+    unsigned long long m = i < 63 ? start0 & (~1ull << i) : 0;
+    if (m) return __ffsll(m) - 1;
+    m = i < 64 ? start1 : i < 127 ? start1 & (~1ull << (i - 64)) : 0;
+    return m ? __ffsll(m) + 63 : ntok;
+  };
   int rs = 0;
   while (rs < ntok) {
     // batch rows rs .. re - 1 continue one sequence
-    int re = rs + 1;
-    while (re < ntok && s_seq[re] == s_seq[rs] &&
-           s_pos[re] == s_pos[re - 1] + 1)
-      ++re;
+    const int re = next_start(rs);
     const bool mine = valid && my_i >= rs && my_i < re;
     const bool all_mine = __all(mine);
     const int* table = a.block_tables + (size_t)s_seq[rs] * a.max_blocks;
@@ -566,14 +577,25 @@ int mx_window_attention(void* out, int ldout, const void* q, int ldq,
               BS, scale * KV_LOG2E, softcap * KV_LOG2E,
               cap ? 2.f * scale * KV_LOG2E / softcap : 0.f, window,
               keep_first > 0 && window > 0 ? keep_first : 0, sink,
-              (const float*)sink_vals, 1, nullptr, 0, 0};
+              (const float*)sink_vals, 1, nullptr, 0, 0, 0};
   dim3 grid;
   if (!token) {
     a.hpb = rep < 128 ? rep : 128;
     a.hblocks = (rep + a.hpb - 1) / a.hpb;
-    const int tpt = 128 / a.hpb;
-    grid = dim3((unsigned)((T_ + tpt - 1) / tpt) *
-                (unsigned)(G * a.hblocks));
+    const unsigned gh = G * a.hblocks;
+    // 128 rows a workgroup, fewer (to one wave's 32) where those leave CUs idle:
+    // a portion of one sequence loses nothing, and short portions of several
+    // no longer wait for each other in one workgroup. us, 128 rows -> this (the
+    // kernel before): 16 heads of 128 on their own, 8 portions of 16 behind 4000
+    // keys 1314 -> 344 (876), 32 of 20 behind 100 70 -> 40 (58); 32/8 heads, 64 of
+    // 5 behind 1000 356 -> 185 (366), 64 rows behind 2000 87 -> 81 (226). Down to
+    // 16 rows, half a wave's: 344 -> 177, but 81 -> 97; up to 512 workgroups: 2
+    // prompts of 2048, 8 heads of 40 60 -> 67.
+    a.tpt = 128 / a.hpb;
+    while (a.tpt > 1 && a.tpt * a.hpb > 32 &&
+           (unsigned)((T_ + a.tpt / 2 - 1) / (a.tpt / 2)) * gh <= 256)
+      a.tpt /= 2;
+    grid = dim3((unsigned)((T_ + a.tpt - 1) / a.tpt) * gh);
   } else {
     a.KS = splits > 1 && scratch != nullptr ? splits : 1;
     if (a.KS > 16) return 1;

@@ -594,3 +594,28 @@ def test_recurrence_empty_segments(mode):
     assert _rel(sg, state) < 2e-6
     if aux is not None:
         assert _rel(ag, aux) < 2e-6
+
+
+@pytest.mark.parametrize("H,G,D,S,n", [
+    (8, 8, 40, 70, 31),      # 128 rows a workgroup, of five sequences
+    (8, 8, 64, 36, 31),      # 64 rows
+    (16, 4, 64, 40, 13),     # 32 rows, of eight tokens
+    (8, 8, 64, 2, 1100)])    # portions of many workgroups
+def test_window_attention_row_groups(H, G, D, S, n):
+    """Workgroups of 128, 64 and 32 rows that hold several sequences, one run
+    from row 0 to 127, runs of single rows, runs that end on a group's last
+    row."""
+    g = torch.Generator().manual_seed(18)
+    past = [5 * i % 40 for i in range(S)]
+    kc, vc, tables = _paged(n + 40, G, D, D, 16, torch.bfloat16, g, S)
+    ts = torch.cat([torch.full((n,), i) for i in range(S)]).int()
+    tp = torch.cat([p + torch.arange(n) for p in past]).int()
+    tp[130:137] = torch.tensor([9, 7, 5, 3, 1, 0, 2])  # rows on their own
+    q = torch.randn(S * n, H * D, generator=g).to(torch.bfloat16).cuda()
+    got, want = (ops.talk_attention(
+        q, kc.cuda(), vc.cuda(), tables.cuda(), ts.cuda(), tp.cuda(),
+        D ** -0.5, H, window=50, keep_first=2, sink=True, softcap=9.0,
+        variant=v).float().reshape(-1, H, D) for v in (11, 1))
+    # two roundings to bf16, row by row
+    err = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert err.max().item() < 1e-2
