@@ -42,19 +42,25 @@ PS_DEV void kv_split(float p0, float p1, unsigned int* a, unsigned int* b,
 // maximum m, or absolute while m is KV_LOW): weights into v, their sum into l,
 // the new maximum into m; returns the factor for what was accumulated before.
 // mx: the largest v over all lanes of the row. The factor is 1 for every lane
-// (and *moved false) when no maximum of the wave moves.
+// (and *moved false) when no maximum of the wave moves. sink2: a sink in powers
+// of two that joins with the row's first maximum, of which this lane has
+// `share` (the alternative to kv_sink where what lives past the walk costs).
 template <int N>
-PS_DEV float kv_softmax(float* v, float mx, float* m, float* l, bool* moved) {
+PS_DEV float kv_softmax(float* v, float mx, float* m, float* l, bool* moved,
+                        float sink2 = -INFINITY, float share = 0.f) {
   const bool fresh = *m == KV_LOW;
   *moved = __any(mx > 0.f || (fresh && mx > -INFINITY));
   float alpha = 1.f;
   if (*moved) {
-    const float d = fresh ? (mx > -INFINITY ? mx : 0.f) : fmaxf(mx, 0.f);
+    const float top = share != 0.f ? fmaxf(mx, sink2) : mx;
+    const float d =
+        fresh ? (mx > -INFINITY ? top : 0.f) : fmaxf(mx, 0.f);
     if (!fresh) {
       alpha = __builtin_amdgcn_exp2f(-d);
       *m += d;
     } else if (mx > -INFINITY) {
       *m = d;
+      if (share != 0.f) *l = share * __builtin_amdgcn_exp2f(sink2 - d);
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) v[i] -= d;
