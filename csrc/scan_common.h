@@ -38,10 +38,12 @@ PS_DEV float ck_rcp(float y) {
   return fmaf(fmaf(-y, r, 1.f), r, r);
 }
 
-// 1 / sqrt(y) likewise; 0 for an infinite y, where the step has no number
+// 1 / sqrt(y) likewise; 0 for an infinite y, where the step's correction (far
+// below 1 otherwise) is no number and the minimum takes the other argument. A
+// choice between the two results cost the operands' kernel 6 %.
 PS_DEV float ck_rsqrt(float y) {
   const float r = __builtin_amdgcn_rsqf(y);
-  return y > 3.4e38f ? r : fmaf(fmaf(-y * r, r, 1.f), 0.5f * r, r);
+  return fmaf(fminf(fmaf(-y * r, r, 1.f), 1.f), 0.5f * r, r);
 }
 
 PS_DEV float ck_sigmoid(float x) {
