@@ -80,21 +80,19 @@ struct CkItem {
   static constexpr int TOTAL = FLAG + 4;
 };
 
-// Chunks of a segment of n rows in this pass (chunks c0 .. c0 + nc of every
-// segment; segments shorter than 16 rows are not this kernel's).
-PS_DEV int ck_count(int n, int c0, int nc) {
-  if (n < 16) return 0;
-  return max(0, min(nc, (n + 15) / 16 - c0));
-}
+// Chunks of a segment of n rows (segments shorter than 16 rows are not this
+// kernel's). The chunks of all segments, one segment after the other, are the
+// items; a pass takes `cap` of them from `base` on.
+PS_DEV int ck_count(int n) { return n < 16 ? 0 : (n + 15) / 16; }
 
-// Which chunk of which segment this pass's item is; false past the last one.
-// Every wave of a block finds the same.
-PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int c0, int nc,
-                    int lane, int* seg, int* chunk) {
+// Which chunk of which segment an item is; false past the last one. Every wave
+// of a block finds the same.
+PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int lane, int* seg,
+                    int* chunk) {
   int base = 0;
   for (int s0 = 0; s0 < S_; s0 += 64) {
     const int s = s0 + lane;
-    const int cnt = s < S_ ? ck_count(seq_rows[4 * s + 1], c0, nc) : 0;
+    const int cnt = s < S_ ? ck_count(seq_rows[4 * s + 1]) : 0;
     int incl = cnt;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -107,7 +105,7 @@ PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int c0, int nc,
     if (hit) {
       const int l = __ffsll((long long)hit) - 1;
       *seg = s0 + l;
-      *chunk = c0 + item - __builtin_amdgcn_readlane(first, l);
+      *chunk = item - __builtin_amdgcn_readlane(first, l);
       return true;
     }
     base += __builtin_amdgcn_readlane(incl, 63);
@@ -118,7 +116,7 @@ PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int c0, int nc,
 template <typename T, int MODE, int DP>
 __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
     float* __restrict__ items, CkIn in, const int* __restrict__ seq_rows,
-    int S_, int H, int G, int D, float scale, float c0f, int c0, int nc) {
+    int S_, int H, int G, int D, float scale, float c0f, int base) {
   typedef CkItem<MODE, DP> It;
   constexpr int LD = DP + 4;
   // operand rows in channel order; reused for the fragments once the 16 x 16
@@ -138,7 +136,7 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
   const int item = blockIdx.x, hd = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int seg, chunk;
-  if (!ck_find(seq_rows, S_, item, c0, nc, lane, &seg, &chunk)) return;
+  if (!ck_find(seq_rows, S_, base + item, lane, &seg, &chunk)) return;
   const int n = seq_rows[4 * seg + 1];
   const int row0 = seq_rows[4 * seg] + 16 * chunk;
   const int nv = min(16, n - 16 * chunk);
@@ -479,8 +477,8 @@ template <typename T, int MODE, int DP, int PART>
 __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
     float* __restrict__ raw, const float* __restrict__ items, int cap,
     const T* __restrict__ v, int ldv, float* __restrict__ state,
-    const int* __restrict__ seq_rows, int S_, int H, int D, int DV, int c0,
-    int nc, float* __restrict__ part, int parts) {
+    const int* __restrict__ seq_rows, int S_, int H, int D, int DV, int base,
+    float* __restrict__ part, int parts) {
   typedef CkItem<MODE, DP> It;
   constexpr int NT = DP / 32;  // row tiles of one wave
   constexpr int N4 = It::TOTAL / 4;
@@ -494,22 +492,25 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
   const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H) % ncb;
   const int run = PART ? blockIdx.x / (S_ * H) / ncb : 0;
   const int seg = sh / H, hd = sh % H;
-  const int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
+  int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
   const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
-  int count = ck_count(n, c0, nc);
-  if (count == 0) return;
-  const bool old = p0 != 0 || c0 != 0;  // there is a state to start from
+  const int all = ck_count(n);
+  if (all == 0) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // this segment's first chunk among all
   int first = 0;
   for (int s = lane; s < seg; s += 64)
-    first += ck_count(seq_rows[4 * s + 1], c0, nc);
+    first += ck_count(seq_rows[4 * s + 1]);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
-  first = __builtin_amdgcn_readfirstlane(first);
-  count = __builtin_amdgcn_readfirstlane(min(count, cap - first));
+  first = __builtin_amdgcn_readfirstlane(first) - base;  // of this pass
+  int c0 = max(0, -first);
+  int count =
+      __builtin_amdgcn_readfirstlane(min(all, cap - first) - c0);
   if (count <= 0) return;
+  first += c0;
+  const bool old = p0 != 0 || c0 != 0;  // there is a state to start from
   bool last = true;  // this run ends the segment's chunks of the pass
   if constexpr (PART != 0) {
     const int per = (count + parts - 1) / parts;
@@ -520,6 +521,9 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
     c0 += run * per;
     count = min(per, count - run * per);
   }
+  // the rows from the first chunk on
+  t0 += 16 * c0;
+  n -= 16 * c0;
 
   const int g = lane >> 4, m16 = lane & 15;
   const int ct = wave >> 1, ds = wave & 1;  // column tile, row half
@@ -599,7 +603,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
     pf[PF - 1] = *(const ck_f32x4*)(base + at16l);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int tt = min(16 * (c0 + c) + 4 * g + i, n - 1);
+      const int tt = min(16 * c + 4 * g + i, n - 1);
       pv.x[i] = vcol[(size_t)tt * ldv];
     }
   };
@@ -613,7 +617,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
 
   // valid rows of this lane group in chunk c, and their values
   auto rows_left = [&](int c) {
-    return col ? n - 16 * (c0 + c) - 4 * g : 0;
+    return col ? n - 16 * c - 4 * g : 0;
   };
   auto values = [&](int c, const Vals& pv) {
     ck_f32x4 V;
@@ -753,7 +757,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
         O += P;
       }
       const int left = rows_left(c);
-      float* dst = raw + (size_t)(t0 + 16 * (c0 + c) + 4 * g) * rs + hv;
+      float* dst = raw + (size_t)(t0 + 16 * c + 4 * g) * rs + hv;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (i < left) dst[i * rs] = O[i];
@@ -870,7 +874,7 @@ __global__ __launch_bounds__(256) void ck_prep_scalar_kernel(
     float* __restrict__ gitems, float* __restrict__ hitems, CkIn in,
     const float* __restrict__ ga, const float* __restrict__ gw,
     const int* __restrict__ seq_rows, int S_, int H, int G, int D,
-    float qscale, int c0, int nc) {
+    float qscale, int base) {
   typedef CkGroup<DP> Gi;
   constexpr int LD = DP + 4;
   __shared__ __align__(16) float Q[16 * LD];
@@ -882,7 +886,7 @@ __global__ __launch_bounds__(256) void ck_prep_scalar_kernel(
   const int item = blockIdx.x, grp = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int seg, chunk;
-  if (!ck_find(seq_rows, S_, item, c0, nc, lane, &seg, &chunk)) return;
+  if (!ck_find(seq_rows, S_, base + item, lane, &seg, &chunk)) return;
   const int n = seq_rows[4 * seg + 1];
   const int row0 = seq_rows[4 * seg] + 16 * chunk;
   const int nv = min(16, n - 16 * chunk);
@@ -986,7 +990,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     const float* __restrict__ hitems, int cap, CkIn in,
     const float* __restrict__ p2, float* __restrict__ state,
     float* __restrict__ aux, const int* __restrict__ seq_rows, int S_, int H,
-    int G, int D, int DV, int c0, int nc, float* __restrict__ part,
+    int G, int D, int DV, int base, float* __restrict__ part,
     int parts) {
   typedef CkGroup<DP> Gi;
   constexpr int NT = DP / 32;
@@ -1001,21 +1005,24 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
   const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H) % ncb;
   const int run = PART ? blockIdx.x / (S_ * H) / ncb : 0;
   const int seg = sh / H, hd = sh % H, grp = hd / (H / G);
-  const int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
+  int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
   const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
-  int count = ck_count(n, c0, nc);
-  if (count == 0) return;
-  const bool old = p0 != 0 || c0 != 0;  // there is a state to start from
+  const int all = ck_count(n);
+  if (all == 0) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int first = 0;
   for (int s = lane; s < seg; s += 64)
-    first += ck_count(seq_rows[4 * s + 1], c0, nc);
+    first += ck_count(seq_rows[4 * s + 1]);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
-  first = __builtin_amdgcn_readfirstlane(first);
-  count = __builtin_amdgcn_readfirstlane(min(count, cap - first));
+  first = __builtin_amdgcn_readfirstlane(first) - base;  // of this pass
+  int c0 = max(0, -first);
+  int count =
+      __builtin_amdgcn_readfirstlane(min(all, cap - first) - c0);
   if (count <= 0) return;
+  first += c0;
+  const bool old = p0 != 0 || c0 != 0;  // there is a state to start from
   bool last = true;  // this run ends the segment's chunks of the pass
   if constexpr (PART != 0) {
     const int per = (count + parts - 1) / parts;
@@ -1025,6 +1032,9 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     c0 += run * per;
     count = min(per, count - run * per);
   }
+  // the rows from the first chunk on
+  t0 += 16 * c0;
+  n -= 16 * c0;
 
   const int g = lane >> 4, m16 = lane & 15;
   const int ct = wave >> 1, ds = wave & 1, tb = ds * NT;
@@ -1100,7 +1110,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     x.h = *(const ck_f32x4*)(hsrc + c * hstep + ath);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int tt = min(16 * (c0 + c) + 4 * g + i, n - 1);
+      const int tt = min(16 * c + 4 * g + i, n - 1);
       x.v[i] = vcol[(size_t)tt * in.ldv];
       if (MODE == CK_SSD) x.gt[i] = gcol[(size_t)tt * in.ldg];
     }
@@ -1115,7 +1125,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
   auto walk = [&](int c, const float* buf, Next& x, float* nbuf,
                   const Next& nx) {
     const float* hb = buf + Gi::TOTAL;
-    const int left = n - 16 * (c0 + c) - 4 * g;
+    const int left = n - 16 * c - 4 * g;
     ck_f32x4 V, gt;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1167,7 +1177,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     __syncthreads();
     if (PART != 1 && ds == 0 && (col || ncol)) {
       O = (O + *(const ck_f32x4*)(xch + ct * 256 + lane * 4)) * dr + X;
-      const size_t row = (size_t)(t0 + 16 * (c0 + c) + 4 * g);
+      const size_t row = (size_t)(t0 + 16 * c + 4 * g);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         if (i < left) {
@@ -1313,27 +1323,22 @@ static long ck_chunk_floats(int mode, int dp, int H, int G) {
 // From 16 rows on a segment goes this way: one chunk costs about 15 us in
 // three launches, 16 tokens one by one 24 us.
 //
-// Chunks laid down at once and the chunks of a segment per pass. A step's
-// segments of 16 rows and more have at most T / 16 + S chunks, and at most
-// T / 8; passes keep the scratch below CK_BYTES.
+// Chunks laid down at once, and the passes over all of them. A step's segments
+// of 16 rows and more have at most T / 16 + S chunks, and at most T / 8; passes
+// keep the scratch below CK_BYTES. They follow the chunks of one segment after
+// the other: by chunk number within every segment, 256 segments of 48 rows took
+// 250 passes for the one segment that could be (general delta, 32 heads of
+// 128 x 128: 27 ms, 2.1 with two passes, 3.7 token by token).
 #define CK_BYTES (1l << 30)
 static void ck_plan(int mode, int T_, int S_, int H, int G, int D, int* cap,
-                    int* nc, int* passes) {
+                    int* passes) {
   const long per = ck_chunk_floats(mode, ck_pad(D), H, G) * 4;
   long all = (long)T_ / 16 + S_;
   if (all > T_ / 8 + 1) all = T_ / 8 + 1;
   long fit = CK_BYTES / per;
-  if (fit < S_) fit = S_;
-  const int longest = (T_ + 15) / 16;  // chunks of one segment, others empty
-  if (all <= fit) {
-    *cap = (int)all;
-    *nc = longest;
-    *passes = 1;
-    return;
-  }
-  *nc = (int)(fit / S_);
-  *cap = (int)((long)*nc * S_ < all ? (long)*nc * S_ : all);
-  *passes = (longest + *nc - 1) / *nc;
+  if (fit < 1) fit = 1;
+  *cap = (int)(all < fit ? all : fit);
+  *passes = (int)((all + *cap - 1) / *cap);
 }
 
 // Runs that a segment's chunks are walked in (not the delta forms, whose state
@@ -1400,8 +1405,8 @@ static void ck_read(CK_ARGS, const float* raw, const float* gx) {
 template <typename T, int MODE, int DP>
 static int ck_launch(CK_ARGS) {
   typedef CkItem<MODE, DP> It;
-  int cap, nc, passes;
-  ck_plan(MODE, T_, S_, H, G, D, &cap, &nc, &passes);
+  int cap, passes;
+  ck_plan(MODE, T_, S_, H, G, D, &cap, &passes);
   float* raw = scratch;
   float* items = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
   const int ncb = (DV + 31) / 32;
@@ -1417,12 +1422,12 @@ static int ck_launch(CK_ARGS) {
   for (int p = 0; p < passes; ++p) {
     hipLaunchKernelGGL((ck_prep_kernel<T, MODE, DP>), dim3(cap, H), dim3(256),
                        0, stream, items, in, (const int*)seq_rows, S_, H, G,
-                       D, scale, c0f, p * nc, nc);
+                       D, scale, c0f, p * cap);
 #define CK_SWEEP(PART, RUNS)                                                 \
   hipLaunchKernelGGL((ck_sweep_kernel<T, MODE, DP, PART>),                   \
                      dim3(S_ * H * ncb * (RUNS)), dim3(256), lds, stream,    \
                      raw, items, cap, (const T*)in.v, in.ldv, (float*)state, \
-                     (const int*)seq_rows, S_, H, D, DV, p * nc, nc, part,   \
+                     (const int*)seq_rows, S_, H, D, DV, p * cap, part,   \
                      parts)
     if constexpr (MODE == CK_GLA) {
       if (parts > 1) {
@@ -1440,8 +1445,8 @@ static int ck_launch(CK_ARGS) {
 
 template <typename T, int MODE, int DP>
 static int ck_launch_scalar(CK_ARGS) {
-  int cap, nc, passes;
-  ck_plan(MODE, T_, S_, H, G, D, &cap, &nc, &passes);
+  int cap, passes;
+  ck_plan(MODE, T_, S_, H, G, D, &cap, &passes);
   const bool lstm = MODE == CK_MLSTM;
   float* raw = scratch;
   float* ga = raw + (lstm ? (size_t)T_ * H * (DV + 1) : 0);
@@ -1463,14 +1468,14 @@ static int ck_launch_scalar(CK_ARGS) {
     hipLaunchKernelGGL((ck_prep_scalar_kernel<T, MODE, DP>),
                        dim3(cap, G, slices), dim3(256), 0, stream, gitems,
                        hitems, in, ga, gw, (const int*)seq_rows, S_, H, G, D,
-                       scale, p * nc, nc);
+                       scale, p * cap);
 #define CK_SWEEP(PART, RUNS)                                                 \
   hipLaunchKernelGGL((ck_sweep_scalar_kernel<T, MODE, DP, PART>),            \
                      dim3(S_ * H * ncb * (RUNS)), dim3(256), 0, stream,      \
                      lstm ? raw : (float*)out, lstm ? H * (DV + 1) : ldo,    \
                      gitems, hitems, cap, in, (const float*)p2,              \
                      (float*)state, (float*)aux, (const int*)seq_rows, S_,   \
-                     H, G, D, DV, p * nc, nc, part, parts)
+                     H, G, D, DV, p * cap, part, parts)
     if (parts > 1) {
       CK_SWEEP(1, parts - 1);
       CK_SWEEP(2, parts);
@@ -1536,8 +1541,8 @@ CK_UNIT(ck_mlstm) CK_BODY(CK_MLSTM)
 extern "C" long mx_chunk_scratch(int mode, int T_, int S_, int H, int G,
                                  int D, int DV) {
   if (S_ <= 0 || T_ - S_ + 1 < 16 || ck_pad(D) == 0 || DV > 256) return 0;
-  int cap, nc, passes;
-  ck_plan(mode, T_, S_, H, G, D, &cap, &nc, &passes);
+  int cap, passes;
+  ck_plan(mode, T_, S_, H, G, D, &cap, &passes);
   return ((ck_rows_floats(mode, T_, H, DV) + 3) & ~3l) +
          ((cap * ck_chunk_floats(mode, ck_pad(D), H, G) + 3) & ~3l) +
          ck_part_floats(mode, T_, S_, H, D, DV);

@@ -619,3 +619,73 @@ def test_window_attention_row_groups(H, G, D, S, n):
     # two roundings to bf16, row by row
     err = (got - want).norm(dim=-1) / want.norm(dim=-1)
     assert err.max().item() < 1e-2
+
+
+@pytest.mark.parametrize("mode,T", [("general", 9700), ("mlstm", 20600)])
+def test_recurrence_chunk_passes_of_segments(mode, T):
+    """Passes that end inside a segment, between two and past the last: every
+    segment as in a call of its own, bit for bit, and no more passes than the
+    chunks need."""
+    H, D = 160, 32
+    g = torch.Generator(device="cuda").manual_seed(4)
+    lens = [17, 3000, 1, 40, T - 3098, 16, 24]
+    proj = torch.randn(T, 5 * H * D + 2 * H, generator=g, device="cuda",
+                       dtype=torch.bfloat16)
+    par = [torch.randn(H * D, generator=g, device="cuda") for _ in range(3)]
+    first = torch.randn(len(lens), H, D, D, generator=g, device="cuda")
+    norm = torch.rand(len(lens), H, D + 1, generator=g, device="cuda")
+    q, k, v, zw, gate = (proj[:, i * H * D:(i + 1) * H * D]
+                         for i in range(5))
+    i, f = proj[:, 5 * H * D:5 * H * D + H], proj[:, 5 * H * D + H:]
+
+    def run(rows, state, aux, a, b):
+        rows = torch.tensor(rows, dtype=torch.int32, device="cuda")
+        if mode == "general":
+            return ops.delta_rule(q[a:b], k[a:b], v[a:b], zw[a:b], q[a:b],
+                                  gate[a:b], *par, state, rows, H, 1e-5, 0.6)
+        return ops.linear_scan(
+            "mlstm", q[a:b], k[a:b], v[a:b], f[a:b], gate[a:b], state, rows,
+            H, H, 1e-5, qscale=D ** -0.5, c0=5.0, wr=i[a:b], p0=par[0][:H],
+            p1=par[1][:H], normw=par[2], aux=aux)
+
+    starts = [sum(lens[:n]) for n in range(len(lens))]
+    state, aux = first.clone(), norm.clone()
+    got = run([(a, n, s % 2, s) for s, (a, n) in enumerate(zip(starts, lens))],
+              state, aux, 0, T)
+    one, aux1 = first.clone(), norm.clone()
+    for s, (a, n) in enumerate(zip(starts, lens)):
+        want = run([(0, n, s % 2, s)], one, aux1, a, a + n)
+        assert torch.equal(got[a:a + n], want), s
+    assert torch.equal(state, one) and torch.equal(aux, aux1)
+
+
+def test_recurrence_chunk_many_segments():
+    """Many segments whose operands exceed the scratch limit: a few passes, in
+    less time than twice the rows of half as many take."""
+    H, D, S, n = 32, 128, 256, 48
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(S * n, 6 * H * D, generator=g, device="cuda",
+                    dtype=torch.bfloat16)
+    v = [x[:, i * H * D:(i + 1) * H * D] for i in range(6)]
+    par = [torch.randn(H * D, generator=g, device="cuda") for _ in range(3)]
+    state = torch.zeros(S, H, D, D, device="cuda")
+
+    def run(s):
+        rows = torch.tensor([(i * n, n, 0, i) for i in range(s)],
+                            dtype=torch.int32, device="cuda")
+        part = [t[:s * n] for t in v]
+        times = []
+        for _ in range(4):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            out = ops.delta_rule(*part, *par, state, rows, H, 1e-5, 0.6)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return out, min(times)
+
+    few, t_few = run(64)
+    many, t_many = run(S)
+    assert torch.equal(many[:64 * n], few)
+    # four times the work; the passes by chunk number took 50 times as long
+    assert t_many < 8 * t_few
