@@ -76,6 +76,9 @@ class BatchMeta:
         self.token_seq = token_seq
         self.seq_rows = seq_rows
         self.seq_rows_host = seq_rows_host
+        # what the recurrences ask about their lengths (see ops.segment_spans)
+        self.seq_spans = (ops.segment_spans(seq_rows_host)
+                          if seq_rows_host else None)
 
 
 def build_cos_sin_cache(

@@ -579,7 +579,8 @@ class GeneralDelta(nn.Module):
         zw = gemm_policy.linear(torch.tanh(proj[:, 5 * HD:]), self.w2)
         return ops.delta_rule(
             r, k, v, zw, za, g, self.w0, self.a_bias, self.out_norm, cache,
-            meta.seq_rows, self.H, self.eps, DELTA_DECAY_SCALE, out=out)
+            meta.seq_rows, self.H, self.eps, DELTA_DECAY_SCALE, out=out,
+            spans=getattr(meta, "seq_spans", None))
 
 
 class ChannelDelta(nn.Module):
@@ -645,7 +646,8 @@ class ChannelDelta(nn.Module):
         return ops.gated_delta(
             qkv[:, :G * D], qkv[:, G * D:2 * G * D], qkv[:, 2 * G * D:],
             beta, zdec, zgate, self.a_log, self.dt_bias, self.out_norm,
-            state, meta.seq_rows, H, G, self.eps, out=out)
+            state, meta.seq_rows, H, G, self.eps, out=out,
+            spans=getattr(meta, "seq_spans", None))
 
 
 class _ScanMixer(nn.Module):
@@ -706,7 +708,8 @@ class GatedLinearAttention(_ScanMixer):
             "gla", proj[:, :a], proj[:, a:b], proj[:, b:c], z,
             proj[:, c:c + H * DV], cache, meta.seq_rows, H, H, self.eps,
             qscale=D ** -0.5, c0=1.0 / self.spec.tau, p0=self.a_bias,
-            normw=self.out_norm, out=out)
+            normw=self.out_norm, out=out,
+            spans=getattr(meta, "seq_spans", None))
 
 
 class MatrixLSTM(_ScanMixer):
@@ -750,7 +753,8 @@ class MatrixLSTM(_ScanMixer):
             proj[:, e + H:e + 2 * H], proj[:, c:e], state, meta.seq_rows,
             H, H, self.eps, qscale=D ** -0.5, c0=self.spec.gate_cap,
             wr=proj[:, e:e + H], p0=self.i_bias, p1=self.f_bias,
-            normw=self.out_norm, aux=aux, out=out)
+            normw=self.out_norm, aux=aux, out=out,
+            spans=getattr(meta, "seq_spans", None))
 
 
 class StateSpaceDuality(_ScanMixer):
@@ -806,7 +810,8 @@ class StateSpaceDuality(_ScanMixer):
             "ssd", xbc[:, inner + G * N:], xbc[:, inner:inner + G * N],
             xbc[:, :inner], proj[:, inner + C:inner + C + H],
             proj[:, :inner], state, meta.seq_rows, H, G, self.eps,
-            p0=self.dt_bias, p1=self.a_log, p2=self.d_skip)
+            p0=self.dt_bias, p1=self.a_log, p2=self.d_skip,
+            spans=getattr(meta, "seq_spans", None))
         y = ops.add_rms_norm32(y32, [], self.out_norm, self.eps, proj.dtype,
                                max(self.spec.norm_groups, 1))
         if out is not None:

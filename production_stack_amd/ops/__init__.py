@@ -1350,12 +1350,44 @@ _ALL_ROWS = 0x7fffffff
 _CHUNK_MODES = {"general": 0, "channel": 1, "gla": 2, "ssd": 3, "mlstm": 4}
 
 
+def segment_spans(seq_rows) -> tuple:
+    """What the recurrences' `spans` is, of a host copy of seq_rows: the rows
+    of the longest segment, and of the longest one shorter than a chunk (-1:
+    there is none)."""
+    rows = [r[1] for r in seq_rows]
+    return (max(rows, default=0),
+            max((n for n in rows if n < CHUNK_ROWS), default=-1))
+
+
+def _segment_forms(T: int, S: int, cells: int, spans) -> tuple:
+    """(chunk, short, token): whether segments of a chunk and more may be
+    there, whether shorter ones may, and whether those go token by token with
+    the state's rows in registers (token_scan) or through the sequential
+    kernels, which prepare 16 tokens at once. `cells`: entries of one
+    segment's state.
+
+    Short segments in a few workgroups are a chain of tokens: us, token_scan
+    / sequential, one segment of 15 rows: gla 8 heads of 128 x 256 49 / 29,
+    general delta 32 heads of 128 x 128 44 / 38; of 8 rows 28 / 22 and 26 / 27;
+    of 4 rows 17 / 19 and 15 / 21. With 10M entries of state a step is bound by
+    the state's bytes: 64 x 15 rows of that general delta 136 / 310, 64 x 8 of
+    64 heads ssd of 128 x 64 72 / 129. Without `spans` the mean stands for the rows where
+    no segment can fill a chunk; launches that find nothing cost 9 us (chunks)
+    and 4 us (short segments): 8 x 8 rows of channel delta, 32 heads of
+    128 x 128, 38 without and 30 with it."""
+    if spans is None:
+        chunk, short = T - S + 1 >= CHUNK_ROWS, True
+        rows = 1 if chunk else T / max(S, 1)
+    else:
+        longest, rows = spans
+        chunk, short = longest >= CHUNK_ROWS, rows >= 0
+    return chunk, short, rows <= 6 or S * cells >= 10 << 20
+
+
 def _chunk_scratch(mode: str, T: int, S: int, H: int, G: int, D: int,
                    DV: int, device):
     """fp32 scratch of the chunk-parallel form of a recurrence over T rows in
     S segments, None where it does not cover the step."""
-    if T - S + 1 < CHUNK_ROWS:      # no segment can be that long
-        return None
     need = _mx().mx_chunk_scratch(_CHUNK_MODES[mode], T, S, H, G, D, DV)
     if need <= 0:
         return None
@@ -1364,12 +1396,13 @@ def _chunk_scratch(mode: str, T: int, S: int, H: int, G: int, D: int,
 
 def gated_delta(q, k, v, beta, zdec, zgate, a_log, dt_bias, normw, state,
                 seq_rows, heads: int, kv_heads: int, eps: float,
-                out: torch.Tensor = None) -> torch.Tensor:
+                out: torch.Tensor = None, spans=None) -> torch.Tensor:
     """Gated delta rule with per-(head, key channel) decay over a ragged
     batch (see reference.gated_delta). q/k [T, G*D], v [T, H*DV], beta
     [T, H], zdec [T, H*D], zgate [T, H*DV]: row-strided views of one
     dtype; a_log fp32 [H], dt_bias fp32 [H*D], normw fp32 [DV]; state fp32
-    [slots, H, D, DV], updated in place. Returns [T, H*DV]."""
+    [slots, H, D, DV], updated in place; spans: segment_spans of a host copy
+    of seq_rows, where there is one. Returns [T, H*DV]."""
     T = q.shape[0]
     H, G = heads, kv_heads
     D = q.shape[1] // G
@@ -1397,7 +1430,9 @@ def gated_delta(q, k, v, beta, zdec, zgate, a_log, dt_bias, normw, state,
     assert state.is_contiguous()
     S = seq_rows.shape[0]
     shortest = _ALL_ROWS
-    scratch = _chunk_scratch("channel", T, S, H, G, D, DV, q.device)
+    chunk, short, token = _segment_forms(T, S, H * D * DV, spans)
+    scratch = (_chunk_scratch("channel", T, S, H, G, D, DV, q.device)
+               if chunk else None)
     if scratch is not None:
         rc = _mx().mx_chunk_gated(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k),
@@ -1408,7 +1443,9 @@ def gated_delta(q, k, v, beta, zdec, zgate, a_log, dt_bias, normw, state,
             _f(D ** -0.5), _p(scratch), _mx_dtype(q.dtype), _stream())
         if rc == 0:
             shortest = CHUNK_ROWS
-    rc = _mx().mx_token_scan(
+            if not short:
+                return out
+    rc = 1 if not token else _mx().mx_token_scan(
         _CHUNK_MODES["channel"], _p(out), _rows(out, "out"), _p(q),
         _rows(q, "q"), _p(k), _rows(k, "k"), _p(v), _rows(v, "v"), _p(zdec),
         _rows(zdec, "zdec"), _p(beta), _rows(beta, "beta"), _p(zgate),
@@ -1433,12 +1470,13 @@ def gated_delta(q, k, v, beta, zdec, zgate, a_log, dt_bias, normw, state,
 
 def delta_rule(r, k, v, zw, za, g, w0, ab, normw, state, seq_rows,
                heads: int, eps: float, decay_scale: float,
-               out: torch.Tensor = None) -> torch.Tensor:
+               out: torch.Tensor = None, spans=None) -> torch.Tensor:
     """Gated delta-rule recurrence over a ragged batch (see
     reference.delta_rule). r/k/v/zw/za/g: [T, H*D] row-strided views of one
     dtype; w0/ab/normw fp32 [H*D]; state fp32 [slots, H, D, D], updated in
     place; seq_rows int32 [S, 4] = (first row, rows, first position, state
-    slot) per segment. Returns [T, H*D] (written into `out` when given)."""
+    slot) per segment; spans as in gated_delta. Returns [T, H*D] (written
+    into `out` when given)."""
     T, HD = r.shape
     H = heads
     D = HD // H
@@ -1462,7 +1500,9 @@ def delta_rule(r, k, v, zw, za, g, w0, ab, normw, state, seq_rows,
     assert state.is_contiguous() and seq_rows.is_contiguous()
     S = seq_rows.shape[0]
     shortest = _ALL_ROWS
-    scratch = _chunk_scratch("general", T, S, H, H, D, D, r.device)
+    chunk, short, token = _segment_forms(T, S, H * D * D, spans)
+    scratch = (_chunk_scratch("general", T, S, H, H, D, D, r.device)
+               if chunk else None)
     if scratch is not None:
         rc = _mx().mx_chunk_delta(
             _p(out), _rows(out, "out"), _p(r), _rows(r, "r"), _p(k),
@@ -1472,7 +1512,9 @@ def delta_rule(r, k, v, zw, za, g, w0, ab, normw, state, seq_rows,
             _f(decay_scale), _p(scratch), _mx_dtype(r.dtype), _stream())
         if rc == 0:
             shortest = CHUNK_ROWS
-    rc = _mx().mx_token_scan(
+            if not short:
+                return out
+    rc = 1 if not token else _mx().mx_token_scan(
         _CHUNK_MODES["general"], _p(out), _rows(out, "out"), _p(r),
         _rows(r, "r"), _p(k), _rows(k, "k"), _p(v), _rows(v, "v"), _p(zw),
         _rows(zw, "zw"), _p(za), _rows(za, "za"), _p(g), _rows(g, "g"),
@@ -1550,7 +1592,7 @@ SCAN_MODES = {"gla": 0, "ssd": 1, "mlstm": 2}
 def linear_scan(mode: str, q, k, v, dec, gate, state, seq_rows, heads: int,
                 groups: int, eps: float, qscale: float = 1.0,
                 c0: float = 1.0, wr=None, p0=None, p1=None, p2=None,
-                normw=None, aux=None, out=None) -> torch.Tensor:
+                normw=None, aux=None, out=None, spans=None) -> torch.Tensor:
     """Gated linear recurrences S <- diag(a) S + w k v^T, o = S^T q over a
     ragged batch (see reference.linear_scan for the three decay laws and
     read-outs: "gla" one decay per key channel, "ssd" one per head with a
@@ -1558,8 +1600,9 @@ def linear_scan(mode: str, q, k, v, dec, gate, state, seq_rows, heads: int,
     maximum and a normaliser). q/k [T, G*D], v/gate [T, H*DV], dec
     [T, H*D] (gla) or [T, H], wr [T, H] (mlstm): row-strided views of one
     dtype; p0/p1/p2/normw fp32; state fp32 [slots, H, D, DV] and aux fp32
-    [slots, H, D+1] (mlstm) are updated in place. Returns [T, H*DV], fp32
-    for "ssd" (a grouped norm follows), else the inputs' dtype."""
+    [slots, H, D+1] (mlstm) are updated in place; spans as in gated_delta.
+    Returns [T, H*DV], fp32 for "ssd" (a grouped norm follows), else the
+    inputs' dtype."""
     T = q.shape[0]
     H, G = heads, groups
     D = q.shape[1] // G
@@ -1604,7 +1647,9 @@ def linear_scan(mode: str, q, k, v, dec, gate, state, seq_rows, heads: int,
     assert state.is_contiguous() and (aux is None or aux.is_contiguous())
     S = seq_rows.shape[0]
     shortest = _ALL_ROWS
-    scratch = _chunk_scratch(mode, T, S, H, G, D, DV, q.device)
+    chunk, short, token = _segment_forms(T, S, H * D * DV, spans)
+    scratch = (_chunk_scratch(mode, T, S, H, G, D, DV, q.device)
+               if chunk else None)
     if scratch is not None:
         rc = _mx().mx_chunk_scan(
             SCAN_MODES[mode], _p(out), _rows(out, "out"), _p(q),
@@ -1616,7 +1661,9 @@ def linear_scan(mode: str, q, k, v, dec, gate, state, seq_rows, heads: int,
             _f(qscale), _f(c0), _p(scratch), _mx_dtype(dt), _stream())
         if rc == 0:
             shortest = CHUNK_ROWS
-    rc = _mx().mx_token_scan(
+            if not short:
+                return out
+    rc = 1 if not token else _mx().mx_token_scan(
         _CHUNK_MODES[mode], _p(out), _rows(out, "out"), _p(q),
         _rows(q, "q"), _p(k), _rows(k, "k"), _p(v), _rows(v, "v"), _p(dec),
         _rows(dec, "dec"), _p(wr), _rows(wr, "wr") if wr is not None else 0,

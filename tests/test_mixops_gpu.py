@@ -689,3 +689,47 @@ def test_recurrence_chunk_many_segments():
     assert torch.equal(many[:64 * n], few)
     # four times the work; the passes by chunk number took 50 times as long
     assert t_many < 8 * t_few
+
+
+@pytest.mark.parametrize("mode", RECURRENCES)
+@pytest.mark.parametrize("lens", [
+    (7,), (15, 1), (1, 1, 1), (40,), (17, 33), (40, 1, 2), (30, 9, 1, 16),
+    (0, 5, 0), (0, 20)])
+def test_recurrence_spans(mode, lens):
+    """With the lengths known ahead: chunks alone, short segments alone token
+    by token and through the sequential kernels, both, and empty segments."""
+    rows = _segs(lens, [2 * i for i in range(len(lens))])
+    x, state, aux, call = _recurrence(mode, 2, 32, 32, rows, torch.float32)
+    spans = ops.segment_spans(rows)
+    names = {"general": "delta_rule", "channel": "gated_delta"}
+    op = getattr(ops, names.get(mode, "linear_scan"))
+    rows = torch.tensor(rows, dtype=torch.int32)
+    sg = state.cuda()
+    ag = aux.cuda() if aux is not None else None
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(ops, op.__name__, lambda *a, **k: op(*a, **k, spans=spans))
+        got = call(_to_gpu(x), sg, ag, rows.cuda())
+    want = call(x, state, aux, rows)
+    # fp32 sums of up to 40 tokens x 32 channels
+    assert _rel(got, want) < 2e-5
+    assert _rel(sg, state) < 2e-6
+    if aux is not None:
+        assert _rel(ag, aux) < 2e-6
+
+
+def test_recurrence_spans_launches():
+    """No launch for segments that are not there: what a batch of a few rows
+    per sequence takes with and without its lengths."""
+    S, n, H, D = 8, 8, 32, 128
+    rows = [(i * n, n, 5, i) for i in range(S)]
+    assert ops.segment_spans(rows) == (8, 8)
+    assert ops.segment_spans([(0, 30, 0, 0), (30, 1, 4, 1)]) == (30, 1)
+    assert ops.segment_spans([(0, 30, 0, 0), (30, 16, 4, 1)]) == (30, -1)
+    forms = ops._segment_forms
+    cells = H * D * D
+    assert forms(64, S, cells, (8, 8)) == (False, True, False)
+    assert forms(64, S, cells, None) == (True, True, True)
+    assert forms(64, 64, cells, None) == (False, True, True)
+    assert forms(15, 1, cells, None) == (False, True, False)
+    assert forms(512, 64, cells, (8, 8)) == (False, True, True)
+    assert forms(46, 2, cells, (30, -1)) == (True, False, True)
