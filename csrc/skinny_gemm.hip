@@ -210,9 +210,14 @@ __global__ __launch_bounds__(256) void skinny_combine_kernel(
 
 
 
-// Rows of x for the kernel without splits; its byte offsets are 31 bits.
-static bool ps_skinny_rows(int M, int K, long x_stride) {
-  return M <= 16 && x_stride >= 0 && (M - 1) * x_stride + K < (1L << 30);
+// Whether the kernel without splits takes it; its byte offsets are 31 bits.
+// More than 8 rows reread x too often where the other form needs no splits
+// (N > 32768; us, this / split, distinct weights: 16 x 128256 x 4096 283 / 213,
+// 16 x 128256 x 2048 151 / 126, 16 x 51200 x 2560 82 / 79; 8 x 128256 x 4096 222 /
+// 236; with splits 16 x 28672 x 4096 68 / 71).
+static bool ps_skinny_rows(int M, int N, int K, long x_stride) {
+  return (M <= 8 || (M <= 16 && N <= 32768)) && x_stride >= 0 &&
+         (M - 1) * x_stride + K < (1L << 30);
 }
 
 template <bool GATED>
@@ -226,11 +231,17 @@ static void ps_skinny_rows_go(void* out, const void* x, const void* w, int M,
   // long rows: four pieces in flight a wave, else a piece and more waves (us
   // at one row, 16 waves of one piece against 8 of four: 2048 x 2048 5.0 /
   // 6.3, 16384 x 2048 16.5 / 20.8, 28672 x 4096 46.2 / 51.6, 4096 x 14336
-  // 28.0 / 25.2)
-  if (K <= 4096)
-    PS_SR(1, 16);
-  else
+  // 28.0 / 25.2). Enough workgroups to fill the chip on short rows want smaller
+  // ones, the more so where 16 waves do not share out the pieces evenly (16 / 8
+  // waves of one piece: 50304 x 768 22.4 / 18.3, 65536 x 1024 33.8 / 27.3, 51200 x
+  // 2560 53.3 / 50.4, 16384 x 2048 17.1 / 16.8; 28672 x 4096 47.0 / 48.8, 18944 x
+  // 3584 29.8 / 31.2, 8192 x 1024 5.7 / 6.2)
+  if (K > 4096)
     PS_SR(4, 8);
+  else if (N >= 12288 && K <= 3072)
+    PS_SR(1, 8);
+  else
+    PS_SR(1, 16);
 #undef PS_SR
 }
 
@@ -241,7 +252,7 @@ extern "C" {
 int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
                     int K, long x_stride, hipStream_t stream) {
   if (M < 1 || N < 64 || K < 64 || N % 64 != 0 || K % 64 != 0 ||
-      !ps_skinny_rows(M, K, x_stride))
+      !ps_skinny_rows(M, N, K, x_stride))
     return -1;
   ps_skinny_rows_go<true>(out, x, w, M, N, K, x_stride, stream);
   return 0;
@@ -270,7 +281,7 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
   int splits = ps_skinny_gemm_splits(M, N, K);
   if (splits < 0) return -1;
   if (M < 1) return 0;  // no rows: their size in bytes would wrap below
-  if (ps_skinny_rows(M, K, x_stride)) {
+  if (ps_skinny_rows(M, N, K, x_stride)) {
     ps_skinny_rows_go<false>(out_bf16, x, w, M, N, K, x_stride, stream);
     return 0;
   }
@@ -281,7 +292,8 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
   skinny_gemm_kernel<MT><<<grid, block, 0, stream>>>(                       \
       (unsigned short*)out_bf16, (float*)ws, (const unsigned short*)x,      \
       (const unsigned short*)w, M, N, K, x_stride)
-  if (M <= 32) PS_SG(2);
+  if (M <= 16) PS_SG(1);
+  else if (M <= 32) PS_SG(2);
   else if (M <= 64) PS_SG(4);
   else if (M <= 128) PS_SG(8);
   else PS_SG(16);

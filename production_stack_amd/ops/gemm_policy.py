@@ -79,11 +79,14 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     W of up to 4096 entries. us, in-house / library: 1 x 2048 x 2048 4.9 / 8.2,
     1 x 28672 x 4096 46 / 64, 3 x 4096 x 4096 11.0 / 15.8, 3 x 6144 x 4096
     15.8 / 15.8; past the line 4 x 6144 x 4096 16.2 / 15.7, 1 x 2048 x 8192
-    14.5 / 12.8."""
+    14.5 / 12.8. Short rows of a wide W are the library's: 3 x 65536 x 1024
+    29.1 / 27.7, 3 x 50304 x 768 19.5 / 18.8 (3 x 51200 x 2560 53 / 52, 1 row 50 /
+    52)."""
     from production_stack_amd import ops
 
     return (x.dim() == 2 and 0 < x.shape[0] <= 3 and w.shape[1] <= 4096
             and _eligible(x.shape[0], *w.shape) and x.stride(1) == 1
+            and (w.shape[1] > 1024 or w.shape[0] < 32768)
             and x.shape[1] == w.shape[1] and w.dtype == torch.bfloat16
             and w.is_contiguous() and x.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
@@ -112,12 +115,13 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """silu_and_mul(linear(x, w)). Up to 16 rows that take the skinny kernel
-    have the activation in its last step (a launch of its own costs a decode
-    step 4.5 us a layer)."""
+    """silu_and_mul(linear(x, w)). Up to 16 rows (8 of a W of more than 32768)
+    that take the skinny kernel without splits have the activation in its last
+    step (a launch of its own costs a decode step 4.5 us a layer)."""
     from production_stack_amd import ops
 
-    if x.shape[0] <= 16 and _choose(x, w) == 1:
+    rows = 8 if w.shape[0] > 32768 else 16
+    if x.shape[0] <= rows and _choose(x, w) == 1:
         return ops.skinny_gated(x, w)
     return ops.silu_and_mul(linear(x, w))
 

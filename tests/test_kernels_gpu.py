@@ -910,3 +910,29 @@ def test_gemm8p_nothing_to_do():
         w = torch.empty(n, k, dtype=torch.bfloat16, device="cuda")
         with pytest.raises(RuntimeError, match="unsupported"):
             ops.gemm8p(x, w)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 12288, 64), (3, 12288, 768), (16, 12288, 2560), (2, 12288, 3136),
+    (8, 32832, 128), (9, 32832, 128), (16, 32832, 1088), (9, 32768, 128)])
+def test_skinny_gemm_wide(M, N, K):
+    """Workgroups of eight waves on wide short rows, fewer pieces than waves
+    and uneven shares; up to 8 rows and more on either side of the width from
+    which the form with splits has one; the dispatch's own choice and the
+    activation behind it."""
+    from production_stack_amd.ops import gemm_policy
+
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") / 16).to(
+        torch.bfloat16)
+    want = x.double() @ w.double().t()
+    gemm_policy.reset()
+    for got in (ops.skinny_gemm(x, w), gemm_policy.linear(x, w)):
+        # fp32 up to the bf16 rounding of the result (2^-9 at most each)
+        assert ((got.double() - want).abs() <= want.abs() / 256 + 1e-3).all()
+    for impl in (0, 1):
+        gemm_policy._POLICY[(M, N, K)] = impl
+        got = gemm_policy.silu_mul(x, w)
+        assert torch.equal(got, ops.silu_and_mul(gemm_policy.linear(x, w)))
+    gemm_policy.reset()
