@@ -275,8 +275,8 @@ __global__ __launch_bounds__(256) void fused_rope_cache_vec_kernel(
     for (int j = 0; j < 8; j++) o[j] = KVTr::from_f32(ps_bf16_to_f32(v[j]));
     *(kvec8*)(cache + at) = o;
   };
-  for (int i = blockIdx.y * 256 + threadIdx.x; i < total;
-       i += gridDim.y * 256) {
+  for (int i = blockIdx.y * blockDim.x + threadIdx.x; i < total;
+       i += gridDim.y * blockDim.x) {
     if (i < rot) {
       const int h = i / nr, r = i % nr * 8;
       unsigned short* hp = base + (long)h * HD + r;  // q heads then k heads
@@ -324,8 +324,11 @@ extern "C" void ps_fused_rope_cache(void* qkv, const void* positions,
     // few tokens: a vector a thread, many: a workgroup a token
     const int work = (QH + KH) * (ROT / 16) + KH * (2 * HD - ROT) / 8;
     const dim3 grid((unsigned)T, T < 512 ? (work + 255) / 256 : 1);
+    // no more waves than vectors: 4096 tokens of 8/1 heads of 64 5.9 us, 6.5 with
+    // four waves
+    const int block = work < 256 ? (work + 63) / 64 * 64 : 256;
 #define PS_ROPE(KVT)                                                         \
-  fused_rope_cache_vec_kernel<KVT><<<grid, 256, 0, stream>>>(                \
+  fused_rope_cache_vec_kernel<KVT><<<grid, block, 0, stream>>>(              \
       (unsigned short*)qkv, (const int*)positions, (const float*)cos_sin,    \
       (const long*)slot_mapping, (KVT*)k_cache, (KVT*)v_cache, QH, KH, HD,   \
       ROT, qkv_stride, BS)
