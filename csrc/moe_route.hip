@@ -227,9 +227,10 @@ extern "C" int mx_moe_route(void* sel, void* wts, void* dense, const void* x,
                      ldx, (const T*)rw, (const float*)corr,                  \
                      (const float*)bias, T_, W, n_out, top, sigmoid_scores,  \
                      renorm, renorm_eps, scale, vec)
-  const int waves = n_out < 4 ? 4 : (n_out < 16 ? n_out : 16);
+  // Fewer outputs than four waves gain nothing (64 of 4096, 1 output 5.1 -> 5.4).
+  const int waves = n_out < 16 ? n_out : 16;
   MX_DISPATCH_DTYPE(dtype, {
-    if (T_ <= 512)
+    if (T_ <= 512 && n_out >= 4)
       MR_GO(8, 1024, waves);
     else
       MR_GO(1, 256, 4);
