@@ -3,8 +3,9 @@
 //
 // A workgroup has one (sequence, KV head, split of the keys): the query heads
 // of a KV head share every byte read. Each of its four waves walks tiles of
-// its own (32 keys, 64 of fp8) in private LDS, no barrier before the merge; the
-// next tile's 16 KB (8 of heads of 64) are on their way during a tile.
+// its own (32 keys) in private LDS, no barrier before the merge; the next tile's
+// 16 KB (8 of fp8 or heads of 64) are on their way during a tile. Sequences of a
+// few tiles of many heads have a wave per head instead.
 // Keys go from memory straight into left operands of K Q^T (16 x 16 x 32, the
 // query heads padded to 16), so a lane holds runs of 8 consecutive keys of one
 // head: the softmax is lane-local plus two exchanges, and the weights pack into
@@ -15,10 +16,10 @@
 // Bound by the cache read; 32/8 heads of 128 (before: a lane per 8 entries of a
 // key on the vector pipe, whose conversions and dot products stood in the way,
 // most of all with fp8):
-//   64 x 4000 keys   bf16 175 us, 6.0 TB/s (203-235)   fp8  95 us (222)
+//   64 x 4000 keys   bf16 175 us, 6.0 TB/s (203-235)   fp8  93 us (222)
 //   256 x 2000 keys  bf16 346 us (375)                 fp8 183 us (390)
 //   32 x 2000 keys   bf16  40 us (58)                  fp8  25 us (65)
-//   1 x 4000 keys    bf16 8.7 us (22)                  fp8 9.8 us (22)
+//   1 x 4000 keys    bf16 8.7 us (22)                  fp8 8.2 us (22)
 // At few keys per CU it is bound by the latency of one tile after another.
 #include "attn_common.h"
 
@@ -37,6 +38,7 @@ struct DaArgs {
   int seqs;
   int splits;              // of the grid and the workspaces
   int fill;                // splits that a sequence gets at any length
+  int packed;              // a wave per head up to this many tiles
 };
 
 // Keys of one split at most, where the grid has splits left: a workgroup alone
@@ -66,8 +68,8 @@ PS_DEV kv_bf16x8 da_bf16(unsigned int lo, unsigned int hi) {
   return u.v;
 }
 
-template <int D, int TT, bool FP8>
-__global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(DaArgs a) {
+template <int D, int TT, bool FP8, int WPE>
+__global__ __launch_bounds__(256, WPE) void paged_attn_decode_kernel(DaArgs a) {
   constexpr int EB = FP8 ? 1 : 2;      // bytes per entry
   constexpr int RB = D * EB;           // per cache row
   constexpr int CR = RB / 16;          // 16-byte pieces of a row
@@ -82,7 +84,8 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(DaArgs a) {
   static_assert(16 * PA * 4 <= TT * PV * 2, "merge fits the value tile");
   __shared__ __align__(16) unsigned short sV[4][TT * PV];
   __shared__ float s_m[4][16], s_l[4][16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int KH = a.KH, GQ = a.GQ;
   // Workgroups go round the XCDs and their shader engines in turn. Heads are
   // counted first, so that a long sequence is on all of them; splits last, so
@@ -91,7 +94,8 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(DaArgs a) {
   // here); and each split starts one sequence on, which moves a sequence's
   // splits apart where there are few heads (32 sequences, one of 30000 keys:
   // 176 us with its splits on one XCD).
-  const int kvh = blockIdx.x % KH, r = blockIdx.x / KH;
+  int kvh = blockIdx.x % KH;
+  const int r = blockIdx.x / KH;
   const int split = r / a.seqs;
   const int seq = (r - split * a.seqs + split) % a.seqs;
   const int ctx = a.seq_lens[seq];
@@ -99,6 +103,15 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(DaArgs a) {
   const int nt = (ctx - lo + TT - 1) / TT;
   const int nsplit = da_splits<TT>(ctx - lo, a.splits, a.fill);
   if (split >= nsplit) return;
+  // Few tiles of many heads: one workgroup of four has a wave for each of four
+  // heads, the other three end here. Which one goes with the sequence such
+  // that all XCDs, and all of an XCD's engines, get the same share (512 x 40
+  // keys of 16/8 heads 42 us with kvh + seq, 20 so).
+  const bool packed = a.packed > 0 && nt <= a.packed;
+  if (packed) {
+    if (((kvh + seq + (seq >> 2)) & 3) != 0) return;
+    kvh = (kvh & ~3) + wave;
+  }
   const int* table = a.block_tables + (long)seq * a.max_blocks;
   const int hr = lane & 15, kq = lane >> 4;   // head row, key group
   const unsigned char* kc = (const unsigned char*)a.kc;
@@ -147,14 +160,14 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(DaArgs a) {
       pre[u] = *(const kv_u4*)(vc + vr * RB + idx % CR * 16);
     }
   };
-  // Loads of tiles past the last repeat it (nothing reads them): without a
-  // branch around them no wait is longer than its use asks for. The page
-  // number is loaded two tiles ahead.
-  const int step = 4 * nsplit;
-  int n = split * 4 + wave, page = 0;
+  // Loads of tiles past the last are all of the last key (nothing reads them):
+  // without a branch around them no wait is longer than its use asks for. The
+  // page number is loaded two tiles ahead.
+  const int step = packed ? 1 : 4 * nsplit;
+  int n = packed ? 0 : split * 4 + wave, page = 0;
   if (n < nt) {
     fetch(n, table[key_of(n) / BS]);
-    page = table[key_of(min(n + step, nt - 1)) / BS];
+    page = table[key_of(n + step) / BS];
   }
   const unsigned short* va = sw + (8 * kq + (hr >> 2)) * PV + 4 * (hr & 3);
   for (; n < nt; n += step) {
@@ -189,8 +202,8 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(DaArgs a) {
       }
     }
     kv_wave_sync();
-    fetch(min(n + step, nt - 1), page);
-    page = table[key_of(min(n + 2 * step, nt - 1)) / BS];
+    fetch(n + step, page);
+    page = table[key_of(n + 2 * step) / BS];
 
     const int left = ctx - (lo + n * TT) - 8 * kq;
     const float base = m == KV_LOW ? 0.f : m;
@@ -252,6 +265,21 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(DaArgs a) {
   for (int c = 0; c < NB; ++c)
     *(float4*)(sa + 16 * c) =
         make_float4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
+  if (packed) {
+    kv_wave_sync();
+    for (int idx = lane; idx < GQ * (D / 4); idx += 64) {
+      const int h = idx / (D / 4), c = idx % (D / 4) * 4;
+      const float lt = s_l[wave][h];
+      const float f = lt > 0.f ? 1.0f / lt : 0.f;
+      const float4 v = *(const float4*)((const float*)sw + h * PA + c);
+      *(uint2*)(a.out + (((long)seq * KH + kvh) * GQ + h) * D + c) =
+          make_uint2((unsigned int)ps_f32_to_bf16(v.x * f) |
+                         ((unsigned int)ps_f32_to_bf16(v.y * f) << 16),
+                     (unsigned int)ps_f32_to_bf16(v.z * f) |
+                         ((unsigned int)ps_f32_to_bf16(v.w * f) << 16));
+    }
+    return;
+  }
   __syncthreads();
   for (int idx = tid; idx < GQ * (D / 4); idx += 256) {
     const int h = idx / (D / 4), c = idx % (D / 4) * 4;
@@ -346,6 +374,16 @@ extern "C" int ps_paged_attn_decode(
   if (head_dim != 128 &&
       (head_dim != 64 || kv_fp8 || GQ == 3 || GQ == 6 || GQ == 7))
     return -1;
+  // A wave per head where four waves would not have a tile each and every CU has
+  // eight workgroups to go through: their chain of loads and the merge take
+  // longer than the few keys (us, four waves a head -> one, in brackets the
+  // vector kernel that was here before; 32 heads of their own, 128: bf16 512 x 40
+  // keys 93 -> 67 (73), 256 x 60 50 -> 43 (43); fp8 512 x 40 72 -> 41 (41), 256 x
+  // 100 46 -> 36 (37), 64 x 100 15.8 -> 15.7 (13.7)). Of bf16 up to two tiles (64
+  // x 100 keys 20.8 -> 23.0 with three), of heads of 64 twice the workgroups (64 x
+  // 40 8.0 -> 8.6, 128 x 30 14.0 -> 11.4).
+  const bool many = (long)num_seqs * KH >= (head_dim == 64 ? 4096 : 2048);
+  const int packed = KH % 4 == 0 && many ? (kv_fp8 ? 4 : 2) : 0;
   const DaArgs a = {(unsigned short*)out,
                     (float*)ws_acc,
                     (float*)ws_ml,
@@ -362,26 +400,32 @@ extern "C" int ps_paged_attn_decode(
                     window,
                     num_seqs,
                     num_splits,
-                    fill};
+                    fill,
+                    packed};
   const dim3 grid((unsigned)num_seqs * KH * num_splits), block(256);
   const dim3 heads(num_seqs * KH * GQ);
-#define DA_GO(D, TT, FP8)                                                    \
+#define DA_GO(D, TT, FP8, WPE)                                               \
   do {                                                                       \
-    paged_attn_decode_kernel<D, TT, FP8><<<grid, block, 0, stream>>>(a);     \
+    paged_attn_decode_kernel<D, TT, FP8, WPE><<<grid, block, 0, stream>>>(a); \
     if (num_splits > 1)                                                      \
       paged_attn_combine_kernel<D, TT><<<heads, block, 0, stream>>>(a);      \
   } while (0)
-  // heads of 64 in tiles of 32 keys too, though their rows are half as long:
-  // short contexts then share out among the waves, and four workgroups fit a CU
-  // (us, 64 keys -> 32; before in brackets: 64 x 300 keys, 32 heads of their own
-  // 30.7 -> 26.3 (27.1), 256 x 200 86.5 -> 77.5 (80.6), 32/8 heads 256 x 200 23.4 ->
-  // 19.5, 64 x 4000 95.4 -> 94.9)
+  // Tiles of 32 keys everywhere: short contexts share out among the waves (us, 64
+  // keys -> 32, before in brackets: heads of 64, 64 x 300 keys, 32 heads of their
+  // own 30.7 -> 26.3 (27.1), 32/8 heads 256 x 200 23.4 -> 19.5; fp8, 32 heads of
+  // their own, 64 x 300 36.6 -> 28.9 (28.3), 256 x 300 137 -> 111 (119), 64 x 4000
+  // 348 -> 347 (409), 32 x 2000 94 -> 99 (111); 32/8 256 x 300 37.0 -> 28.9).
+  // bf16 of 128: a third workgroup a CU where there is one (32 heads of their own,
+  // 256 x 100 keys 90 -> 78 (84), 64 x 100 23.4 -> 20.9 (20.3)); for two a CU its
+  // registers cost 3 % (8 x 1000 keys of 8 heads 10.0 -> 10.3).
   if (head_dim == 64)
-    DA_GO(64, 32, false);
+    DA_GO(64, 32, false, 2);
   else if (kv_fp8)
-    DA_GO(128, 64, true);
+    DA_GO(128, 32, true, 2);
+  else if ((long)num_seqs * KH * fill > 512)
+    DA_GO(128, 32, false, 3);
   else
-    DA_GO(128, 32, false);
+    DA_GO(128, 32, false, 2);
 #undef DA_GO
   return 0;
 }

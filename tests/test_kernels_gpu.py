@@ -117,6 +117,41 @@ def test_paged_attn_decode(qh, kh, hd):
     _close(got, want)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("S,qh,kh,hd,window", [
+    (66, 32, 32, 128, 0),     # a wave per head up to two tiles (four of fp8)
+    (130, 32, 16, 128, 50),   # two query heads, trailing window
+    (129, 32, 32, 64, 0),
+    (70, 30, 30, 128, 0),     # no whole fours of heads: four waves a head
+    (20, 32, 32, 128, 0)])    # more than two workgroups a CU, fewer than eight
+def test_paged_attn_decode_many_heads(S, qh, kh, hd, window, fp8):
+    """Short contexts of many heads, at the edges of the tiles and of the rule
+    that gives a head one wave; an empty context gives zeros."""
+    if fp8 and hd != 128:
+        pytest.skip("fp8 caches have heads of 128")
+    torch.manual_seed(5)
+    bs, max_blocks = 16, 20
+    edges = [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128,
+             129, 160, 300]
+    lens = torch.tensor([edges[i % len(edges)] for i in range(S)],
+                        dtype=torch.int32)
+    k_cache, v_cache = _make_cache(S * max_blocks + 1, kh, bs, hd)
+    if fp8:
+        k_cache, v_cache = (c.to(torch.float8_e4m3fn)
+                            for c in (k_cache, v_cache))
+    tables = torch.randperm(S * max_blocks).int().view(S, max_blocks) + 1
+    q = torch.randn((S, qh, hd), dtype=torch.bfloat16, device="cuda")
+    got = ops.paged_attn_decode(q, k_cache, v_cache, tables.cuda(),
+                                lens.cuda(), hd ** -0.5, window=window)
+    some = lens > 0
+    want = reference.paged_attn_decode(
+        q.cpu()[some], k_cache.cpu().to(torch.bfloat16),
+        v_cache.cpu().to(torch.bfloat16), tables[some], lens[some],
+        hd ** -0.5, window=window)
+    assert not got.cpu()[~some].any()
+    _close(got.cpu()[some], want)
+
+
 @pytest.mark.parametrize("num_splits", [1, 2, 4, 8, 32])
 def test_paged_attn_decode_split_kv(num_splits):
     """All split factors must agree with the reference (incl. splits that
