@@ -185,7 +185,7 @@ void paged_attn_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   TORCH_CHECK(QH % KH == 0, "GQA group mismatch");
   const int GQ = QH / KH;
   const int max_blocks = (int)block_tables.size(1);
-  (void)variant;  // one kernel serves every value
+  (void)variant;  // callers may pass it: one kernel serves every value
   int64_t fill = num_splits;
   if (num_splits <= 0) {
     // One workgroup per CU: each of its waves keeps 16 KB of loads in flight,
@@ -526,7 +526,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm8p", &gemm8p,
         "8-phase deep-pipelined bf16 GEMM (out = x @ w.T)");
   m.def("skinny_gemm", &skinny_gemm,
-        "Split-K MFMA GEMM for decode-shaped (M<=128) projections");
+        "MFMA GEMM for decode-shaped (M<=256) projections");
   m.def("skinny_gated", &skinny_gated,
         "silu(x @ wg.T) * (x @ wu.T) of up to 16 rows, w = [wg; wu]");
   m.def("kv_dequant", &kv_dequant, "Row-wise int8 KV dequantization");

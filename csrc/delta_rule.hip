@@ -1,5 +1,5 @@
-// Gated delta-rule recurrence (prefill portions and single decode tokens in
-// one launch).
+// Gated delta-rule recurrence, token by token (portions and single tokens of a
+// ragged batch in one launch).
 //
 // Per head the state S is a D x D fp32 matrix (rows = key channels, columns
 // = value channels). For every token
@@ -22,8 +22,10 @@
 // barrier.
 //
 // Segments of nmax rows and more are left to the chunk-parallel kernels
-// (chunk_scan.hip); this form takes single tokens, portions shorter than a
-// chunk and key widths those are not built for.
+// (chunk_scan.hip), single tokens, segments of a few rows and steps with much
+// state to the kernel that keeps the state's rows in registers (token_scan.hip).
+// This form takes what is left: some 7 to 15 rows with little state, and widths
+// that neither is built for (keys above 128, values above 256).
 #include "mix_common.h"
 
 template <typename T, int DKP, int TILE, int P>

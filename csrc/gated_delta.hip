@@ -25,8 +25,10 @@
 // broadcast LDS reads and no barrier.
 //
 // Segments of nmax rows and more are left to the chunk-parallel kernels
-// (chunk_scan.hip); this form takes single tokens, portions shorter than a
-// chunk and widths those are not built for.
+// (chunk_scan.hip), single tokens, segments of a few rows and steps with much
+// state to the kernel that keeps the state's rows in registers (token_scan.hip).
+// This form takes what is left: some 7 to 15 rows with little state, and widths
+// that neither is built for (keys above 128, values above 256).
 #include "mix_common.h"
 
 PS_DEV float mx_softplus(float z) {

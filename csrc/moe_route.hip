@@ -13,11 +13,11 @@
 // which the all-experts path of small batches consumes directly.
 //
 // One workgroup per token: its waves share out the router outputs' dot
-// products (16-byte loads where the rows allow it),
-// then the first wave shares the outputs among its lanes for the softmax and
-// the `top` rounds of arg-max. A decode batch is bound by the latency of that
-// chain, so there a wave has one output where 16 waves suffice and eight loads of
-// a row in flight.
+// products (16-byte loads where the rows allow it), then the first wave shares
+// the outputs among its lanes for the softmax and the `top` rounds of arg-max.
+// A decode batch is bound by the latency of that chain, so there (from four
+// outputs on) a wave has one output where 16 waves suffice and eight loads of a
+// row in flight.
 #include "mix_common.h"
 
 #define MR_MAX_OUT 1024

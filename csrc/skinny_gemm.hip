@@ -14,7 +14,8 @@
 //   as A-frags for ceil(M/16) m-tiles; per-k-chunk MFMA count scales with
 //   m-tiles while W traffic stays fixed.
 //   Split-K partials go to an fp32 workspace that a second kernel adds up.
-// That is the form for 17 to 256 rows; fewer have one of their own, below.
+// That is the form for 17 to 256 rows, and for 9 to 16 where W has more than
+// 32768; fewer have one of their own, below.
 // mfma_f32_16x16x32_bf16; operand k-pattern as verified in
 // csrc/tools/mfma_probe.hip.
 #include "ps_common.h"
@@ -31,11 +32,11 @@ PS_DEV ps_gbf16x8 ps_as_gbf16(ps_bf16x8 u) {
   return v.bf;
 }
 
-// Up to 16 rows of x: a workgroup owns 16 rows of W and all of K, its NW waves
-// take every NW-th 128-byte piece of them, UC pieces in flight each, and add up
-// in LDS at the end: no second kernel and no partial sums in memory. W goes
-// from memory straight into left operands, x from the caches into right ones
-// (rows past the last read as zeros without an access).
+// Up to 16 rows of x (8 of a W of more than 32768): a workgroup owns 16 rows of W
+// and all of K, its NW waves take every NW-th 128-byte piece of them, UC pieces
+// in flight each, and add up in LDS at the end: no second kernel and no partial
+// sums in memory. W goes from memory straight into left operands, x from the
+// caches into right ones (rows past the last read as zeros without an access).
 // Bound by the read of W, at few rows of W by its latency: 1 x 4096 x 4096 in
 // 10.3 us (17.4 with the split kernel, its merge included), 1 x 28672 x 4096 in
 // 46 (79; 5.1 TB/s), 1 x 2048 x 2048 in 5.0 (13.1). Reading x costs as many
