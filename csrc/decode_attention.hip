@@ -415,14 +415,16 @@ extern "C" int ps_paged_attn_decode(
   // own 30.7 -> 26.3 (27.1), 32/8 heads 256 x 200 23.4 -> 19.5; fp8, 32 heads of
   // their own, 64 x 300 36.6 -> 28.9 (28.3), 256 x 300 137 -> 111 (119), 64 x 4000
   // 348 -> 347 (409), 32 x 2000 94 -> 99 (111); 32/8 256 x 300 37.0 -> 28.9).
-  // bf16 of 128: a third workgroup a CU where there is one (32 heads of their own,
-  // 256 x 100 keys 90 -> 78 (84), 64 x 100 23.4 -> 20.9 (20.3)); for two a CU its
-  // registers cost 3 % (8 x 1000 keys of 8 heads 10.0 -> 10.3).
+  // bf16 of 128: a third workgroup a CU where there is one and heads have keys of
+  // their own (32 heads, 256 x 100 keys 90 -> 78 (84), 64 x 100 23.4 -> 20.9 (20.3)).
+  // Heads that share them are 5 % faster or slower with it as the lengths differ
+  // (32/8, 100 sequences of 500 to 3000 keys 156 -> 151, 150 of 40 to 2000 127 ->
+  // 132); two a CU cost its registers 3 % (8 x 1000 keys of 8 heads 10.0 -> 10.3).
   if (head_dim == 64)
     DA_GO(64, 32, false, 2);
   else if (kv_fp8)
     DA_GO(128, 32, true, 2);
-  else if ((long)num_seqs * KH * fill > 512)
+  else if (GQ == 1 && (long)num_seqs * KH * fill > 512)
     DA_GO(128, 32, false, 3);
   else
     DA_GO(128, 32, false, 2);
