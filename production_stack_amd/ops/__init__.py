@@ -1359,29 +1359,42 @@ def segment_spans(seq_rows) -> tuple:
             max((n for n in rows if n < CHUNK_ROWS), default=-1))
 
 
-def _segment_forms(T: int, S: int, cells: int, spans) -> tuple:
+def _segment_forms(T: int, S: int, cells: int, spans, mode: str = "general",
+                   heads: int = 0, columns: int = 0) -> tuple:
     """(chunk, short, token): whether segments of a chunk and more may be
     there, whether shorter ones may, and whether those go token by token with
     the state's rows in registers (token_scan) or through the sequential
     kernels, which prepare 16 tokens at once. `cells`: entries of one
     segment's state.
 
-    Short segments in a few workgroups are a chain of tokens: us, token_scan
-    / sequential, one segment of 15 rows: gla 8 heads of 128 x 256 49 / 29,
-    general delta 32 heads of 128 x 128 44 / 38; of 8 rows 28 / 22 and 26 / 27;
-    of 4 rows 17 / 19 and 15 / 21. With 10M entries of state a step is bound by
-    the state's bytes: 64 x 15 rows of that general delta 136 / 310, 64 x 8 of
-    64 heads ssd of 128 x 64 72 / 129. Without `spans` the mean stands for the rows where
-    no segment can fill a chunk; launches that find nothing cost 9 us (chunks)
-    and 4 us (short segments): 8 x 8 rows of channel delta, 32 heads of
-    128 x 128, 38 without and 30 with it."""
+    Short segments in a few workgroups are a chain of tokens, whose link is
+    longer in token_scan (about 2 us, 2.4 of wide heads) than in the sequential
+    kernels, which in turn take 5 us or more to start: us, token_scan /
+    sequential, one segment of 8 rows: gla 16 heads of 64 x 64 16 / 20, channel
+    delta 64 of 128 x 64 25 / 33, gla 8 of 128 x 256 28 / 22, ssd 16 of 128 x 256
+    25 / 17; 8 segments of 15 rows: gla 8 heads of 128 x 256 45 / 30, channel
+    delta 32 of 128 x 128 51 / 41.
+    With millions of entries of state a step is bound by their bytes: 8 x 10
+    rows of channel delta, 64 heads of 128 x 64 (4M, two workgroups a CU) 35 / 77,
+    128 x 10 rows of mlstm, 16 heads of 64 x 64 (8M) 63 / 121. The matrix LSTM's sequential kernel
+    shares heads of many value columns out over workgroups and starts in 100 us
+    (8 heads of 128 x 256, 15 rows 52 / 163). Without `spans` the mean stands for
+    the rows where no segment can fill a chunk; launches that find nothing cost
+    9 us (chunks) and 4 us (short segments): 8 x 8 rows of channel delta, 32
+    heads of 128 x 128, 38 without and 30 with it."""
     if spans is None:
         chunk, short = T - S + 1 >= CHUNK_ROWS, True
         rows = 1 if chunk else T / max(S, 1)
     else:
         longest, rows = spans
         chunk, short = longest >= CHUNK_ROWS, rows >= 0
-    return chunk, short, rows <= 6 or S * cells >= 10 << 20
+    wide = columns > 128
+    few = 6 if mode == "ssd" or (mode == "gla" and wide) else 8
+    # workgroups of the sequential channel delta fill a CU each
+    rounds = mode == "channel" and S * heads > 256
+    return chunk, short, (rows <= few
+                          or S * cells >= (1 if rounds else 6) << 20
+                          or (mode == "mlstm" and wide))
 
 
 def _chunk_scratch(mode: str, T: int, S: int, H: int, G: int, D: int,
@@ -1430,7 +1443,8 @@ def gated_delta(q, k, v, beta, zdec, zgate, a_log, dt_bias, normw, state,
     assert state.is_contiguous()
     S = seq_rows.shape[0]
     shortest = _ALL_ROWS
-    chunk, short, token = _segment_forms(T, S, H * D * DV, spans)
+    chunk, short, token = _segment_forms(T, S, H * D * DV, spans,
+                                         "channel", H, DV)
     scratch = (_chunk_scratch("channel", T, S, H, G, D, DV, q.device)
                if chunk else None)
     if scratch is not None:
@@ -1647,7 +1661,8 @@ def linear_scan(mode: str, q, k, v, dec, gate, state, seq_rows, heads: int,
     assert state.is_contiguous() and (aux is None or aux.is_contiguous())
     S = seq_rows.shape[0]
     shortest = _ALL_ROWS
-    chunk, short, token = _segment_forms(T, S, H * D * DV, spans)
+    chunk, short, token = _segment_forms(T, S, H * D * DV, spans, mode,
+                                         H, DV)
     scratch = (_chunk_scratch(mode, T, S, H, G, D, DV, q.device)
                if chunk else None)
     if scratch is not None:

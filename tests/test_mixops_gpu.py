@@ -717,14 +717,23 @@ def test_recurrence_spans(mode, lens):
 def test_recurrence_spans_launches():
     """No launch for segments that are not there: what a batch of a few rows
     per sequence takes with and without its lengths."""
-    S, n, H, D = 8, 8, 32, 128
+    S, n, H, D = 8, 12, 32, 128
     rows = [(i * n, n, 5, i) for i in range(S)]
-    assert ops.segment_spans(rows) == (8, 8)
+    assert ops.segment_spans(rows) == (12, 12)
     assert ops.segment_spans([(0, 30, 0, 0), (30, 1, 4, 1)]) == (30, 1)
     assert ops.segment_spans([(0, 30, 0, 0), (30, 16, 4, 1)]) == (30, -1)
     forms = ops._segment_forms
     cells = H * D * D
-    assert forms(64, S, cells, (8, 8)) == (False, True, False)
+    assert forms(96, S, cells, (12, 12)) == (False, True, False)
+    assert forms(96, S, cells, (12, 12), "channel", H, D) == (
+        False, True, False)
+    assert forms(96, S, cells, (12, 12), "channel", 2 * H, 64) == (
+        False, True, True)
+    assert forms(8, 1, cells, (8, 8)) == (False, True, True)
+    assert forms(8, 1, cells, (8, 8), "ssd", H, D) == (False, True, False)
+    assert forms(8, 1, cells, (8, 8), "gla", 8, 256) == (False, True, False)
+    assert forms(15, 1, cells, (15, 15), "mlstm", 8, 256) == (
+        False, True, True)
     assert forms(64, S, cells, None) == (True, True, True)
     assert forms(64, 64, cells, None) == (False, True, True)
     assert forms(15, 1, cells, None) == (False, True, False)
