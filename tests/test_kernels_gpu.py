@@ -117,18 +117,19 @@ def test_paged_attn_decode(qh, kh, hd):
     _close(got, want)
 
 
-@pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("S,qh,kh,hd,window", [
-    (66, 32, 32, 128, 0),     # a wave per head up to two tiles (four of fp8)
-    (130, 32, 16, 128, 50),   # two query heads, trailing window
-    (129, 32, 32, 64, 0),
-    (70, 30, 30, 128, 0),     # no whole fours of heads: four waves a head
-    (20, 32, 32, 128, 0)])    # more than two workgroups a CU, fewer than eight
+@pytest.mark.parametrize("S,qh,kh,hd,window,fp8", [
+    (66, 32, 32, 128, 0, False),    # a wave per head up to two tiles
+    (66, 32, 32, 128, 0, True),     # (four of fp8)
+    (130, 32, 16, 128, 50, False),  # two query heads, trailing window
+    (130, 32, 16, 128, 50, True),
+    (129, 32, 32, 64, 0, False),
+    (70, 30, 30, 128, 0, False),    # no whole fours of heads: four waves a head
+    (70, 30, 30, 128, 0, True),
+    (20, 32, 32, 128, 0, False),    # more than two workgroups a CU, under eight
+    (20, 32, 32, 128, 0, True)])
 def test_paged_attn_decode_many_heads(S, qh, kh, hd, window, fp8):
     """Short contexts of many heads, at the edges of the tiles and of the rule
     that gives a head one wave; an empty context gives zeros."""
-    if fp8 and hd != 128:
-        pytest.skip("fp8 caches have heads of 128")
     torch.manual_seed(5)
     bs, max_blocks = 16, 20
     edges = [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128,
