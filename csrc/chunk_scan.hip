@@ -33,7 +33,7 @@
 // parallel kernel (one workgroup per chunk and head: the decays' products,
 // the 16 x 16 matrices, the triangular solve), and a second kernel walks the
 // chunks with the state in registers: a wave owns 16 columns of S as D / 16
-// accumulator tiles of v_mfma_f32_16x16x4_f32. The tiles' register layout (row
+// accumulator tiles of v_mfma_f32_16x16x4_f32 (or shares its rows with others). The tiles' register layout (row
 // 4 g + i of a tile in lane group g, register i) is at once the layout of the
 // right operand of the products that read S when the left operand's columns
 // are taken in the order 4 g + i, so the state never leaves its registers; Z
@@ -111,6 +111,25 @@ PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int lane, int* seg,
     base += __builtin_amdgcn_readlane(incl, 63);
   }
   return false;
+}
+
+// The segment that `rank` others are longer than (of equal ones the first),
+// -1 where it has no chunks. Workgroups start in the order of their numbers, so
+// the longest walks start first, and the CU of one takes a shorter one beside
+// it: general delta, 32 heads, prompts of 336 and 166 chunks, 0.60 -> 0.47 ms.
+// Past 64 segments, more than a step has of prompts, they go as they come.
+PS_DEV int ck_by_length(const int* seq_rows, int S_, int rank) {
+  if (S_ > 64 || S_ == 1) return rank;
+  const int lane = threadIdx.x & 63;
+  const int mine = lane < S_ ? seq_rows[4 * lane + 1] : 0;
+  if (rank >= __popcll(__ballot(ck_count(mine) > 0))) return -1;
+  int longer = 0;
+  for (int s = 0; s < S_; ++s) {
+    const int n = __builtin_amdgcn_readlane(mine, s);
+    longer += n > mine || (n == mine && s < lane);
+  }
+  return __ffsll((unsigned long long)__ballot(lane < S_ && longer == rank)) -
+         1;
 }
 
 template <typename T, int MODE, int DP>
@@ -455,17 +474,48 @@ PS_DEV ck_f32x4 ck_square_terms(const float* frag, ck_f32x4 x, ck_f32x4 acc,
   return acc;
 }
 
-// Walks the chunks of one (segment, head) for 32 columns of its state: four
-// waves, two per 16 columns, each with half of the state's rows. raw [T, H *
-// DV]: S^T r before the read-out's norm.
+// The same for one product's tokens 4 k + i (k: lane group): f the matrix's
+// entries as that product takes them, x the lane's value, sums in its order.
+PS_DEV ck_f32x4 ck_token_terms(float f, float x, ck_f32x4 acc, int lane,
+                               float* tmp) {
+  const int g = lane >> 4, n = lane & 15;
+  tmp[lane] = f;
+  tmp[64 + lane] = x;
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+  for (int k = 0; k < 4; ++k) {
+    const float xs = tmp[64 + k * 16 + n];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float a = tmp[k * 16 + 4 * g + i];
+      if (a != 0.f) acc[i] = fmaf(a, xs, acc[i]);
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  return acc;
+}
+
+// Walks the chunks of one (segment, head) for 16 columns of its state: a wave
+// per 32 rows of it, DP / 32 waves. raw [T, H * DV]: S^T r before the
+// read-out's norm.
 //
-// The chain from one chunk to the next is what bounds this kernel (a prompt
-// has a few hundred chunks and 2 x heads x DV / 16 waves are about one per
-// SIMD), so a chunk's products are split over as many waves as pay for the
-// exchange: the halves of Z and O meet in LDS once per chunk. Operands come
-// in two chunks ahead, through registers into one of two LDS buffers.
-// Workgroups of one head are S_ * H apart, so that they share an XCD's L2
-// where that is a multiple of 8.
+// The chain from one chunk to the next is what bounds this kernel: a prompt
+// has a few hundred chunks, and heads x DV / 16 workgroups are one or two a
+// CU, so that a SIMD issues for one or two waves and every instruction counts.
+// Rows are split over the waves: no two of them read the same operands, which
+// come from memory straight into registers about a chunk and a half ahead, and
+// only the waves' shares of Z and O pass through LDS. There are two sets of
+// both, so a chunk has one barrier: a set is written again behind the barrier
+// of the next chunk, which no wave reaches before it has read it. O's shares
+// are added one chunk later, behind that chunk's barrier. Products with the
+// 16 x 16 matrices are shared out by tokens, one of each group of four a wave.
+// Loads of values and stores of rows go through buffers that end with the
+// segment: no branches in a chunk, and what lies outside reads as zero.
+// Measured (general delta, 128 x 128, one prompt of 336 chunks): 2.13 us a
+// chunk with operands through LDS and 32 columns a workgroup, 1.05 now, of
+// which the products take 0.5.
+// Workgroups of one head are H apart, so that they share an XCD's L2 where
+// that is a multiple of 8.
 //
 // PART 1 and 2 (gla, whose state only decays between writes): a segment's
 // chunks in `parts` runs that are walked at once. The first launch walks all
@@ -474,24 +524,25 @@ PS_DEV ck_f32x4 ck_square_terms(const float* frag, ck_f32x4 x, ck_f32x4 acc,
 // the last run's record takes the state before the segment). The second starts
 // each run from what the runs before it leave and writes the outputs.
 template <typename T, int MODE, int DP, int PART>
-__global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
+__global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
     float* __restrict__ raw, const float* __restrict__ items, int cap,
     const T* __restrict__ v, int ldv, float* __restrict__ state,
     const int* __restrict__ seq_rows, int S_, int H, int D, int DV, int base,
     float* __restrict__ part, int parts) {
   typedef CkItem<MODE, DP> It;
-  constexpr int NT = DP / 32;  // row tiles of one wave
-  constexpr int N4 = It::TOTAL / 4;
-  constexpr int PF = (N4 + 255) / 256;
-  extern __shared__ __align__(16) float lds[];  // [2][BUF], exchange, tmp
-  constexpr int BUF = PF * 1024;  // TOTAL and what the last threads overhang
-  float* xch = lds + 2 * BUF;     // [4 waves][2][64][4]
-  float* tmp = xch + 2048 + (threadIdx.x >> 6) * 256;
+  constexpr int NW = DP / 32;          // waves
+  constexpr int NQ = (4 + NW - 1) / NW;  // tokens of four a wave takes
+  constexpr int SET = NW * 64;         // shares of one chunk, float4
+  __shared__ ck_f32x4 zx[2 * SET], ox[2 * SET];
+  __shared__ float tmps[NW * 128];
 
-  const int ncb = (DV + 31) / 32;
-  const int sh = blockIdx.x % (S_ * H), cb = blockIdx.x / (S_ * H) % ncb;
+  const int ncb = (DV + 15) / 16;
   const int run = PART ? blockIdx.x / (S_ * H) / ncb : 0;
-  const int seg = sh / H, hd = sh % H;
+  const int rest = blockIdx.x - run * S_ * H * ncb;
+  const int hd = rest % H, cb = rest / H % ncb;
+  const int seg = ck_by_length(seq_rows, S_, rest / (H * ncb));
+  if (seg < 0) return;
+  const int sh = seg * H + hd;
   int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
   const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
   const int all = ck_count(n);
@@ -522,286 +573,341 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_kernel(
     count = min(per, count - run * per);
   }
   // the rows from the first chunk on
-  t0 += 16 * c0;
-  n -= 16 * c0;
+  t0 = __builtin_amdgcn_readfirstlane(t0 + 16 * c0);
+  n = __builtin_amdgcn_readfirstlane(n - 16 * c0);
 
   const int g = lane >> 4, m16 = lane & 15;
-  const int ct = wave >> 1, ds = wave & 1;  // column tile, row half
-  const int tb = ds * NT;                   // this wave's first row tile
-  const int j = cb * 32 + ct * 16 + m16;    // this lane's column
+  const int j = cb * 16 + m16;  // this lane's column
   const bool col = j < DV;
-  const int hv = hd * DV + j;
+  // row i of row tile t of the state
+  auto row = [&](int t, int i) { return 32 * wave + 16 * t + 4 * g + i; };
   float* Sg = state + ((size_t)slot * H + hd) * (size_t)D * DV;
-  ck_f32x4 S[NT];
+  ck_f32x4 S[2];
   const size_t rec = (size_t)D * DV + DP;  // of one run
   float* pt = PART ? part + (size_t)sh * parts * rec : nullptr;
-  if constexpr (PART != 2) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 16 * (tb + t) + 4 * g + i;
-        S[t][i] = (col && d < D && old) ? Sg[(size_t)d * DV + j] : 0.f;
+    for (int i = 0; i < 4; ++i) {
+      const int d = row(t, i);
+      const bool in = col && d < D;
+      const size_t at = (size_t)d * DV + j;
+      float x = 0.f;
+      if (PART != 2 && in && old) x = Sg[at];
+      if constexpr (PART == 1) {
+        if (run == 0 && in) pt[(parts - 1) * rec + at] = x;
+        x = 0.f;
       }
-  }
-  if constexpr (PART == 1) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 16 * (tb + t) + 4 * g + i;
-        if (run == 0 && col && d < D)
-          pt[(parts - 1) * rec + (size_t)d * DV + j] = S[t][i];
-        S[t][i] = 0.f;
+      if constexpr (PART == 2) {
+        if (in) x = pt[(parts - 1) * rec + at];
       }
-  }
+      S[t][i] = x;
+    }
   if constexpr (PART == 2) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 16 * (tb + t) + 4 * g + i;
-        S[t][i] = col && d < D ? pt[(parts - 1) * rec + (size_t)d * DV + j]
-                               : 0.f;
-      }
 #pragma unroll 2
     for (int q = 0; q < run; ++q)
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int d = 16 * (tb + t) + 4 * g + i;
+          const int d = row(t, i);
           const float add =
               col && d < D ? pt[q * rec + (size_t)d * DV + j] : 0.f;
           S[t][i] = S[t][i] * pt[q * rec + (size_t)D * DV + d] + add;
         }
   }
   // product of the decays over the run, this wave's rows
-  ck_f32x4 decay[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) decay[t] = {1.f, 1.f, 1.f, 1.f};
+  ck_f32x4 decay[2] = {{1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}};
 
-  const char* src = (const char*)(items + ((size_t)first * H + hd) * It::TOTAL);
+  // Operands through buffers, too: a uniform base, a uniform offset and a
+  // 32-bit one per lane, so that a load is one instruction. `next` is the chunk
+  // to fetch (the last one again behind it).
+  const char* next = (const char*)(items + ((size_t)first * H + hd) * It::TOTAL);
   const size_t step = (size_t)H * It::TOTAL * sizeof(float);
-  // a uniform base and a 32-bit offset per lane: no address arithmetic
-  const unsigned at16 = threadIdx.x * 16;
-  const unsigned at16l =
-      min((unsigned)(PF - 1) * 256 + threadIdx.x, (unsigned)N4 - 1) * 16;
-  const T* vcol = v + (size_t)t0 * ldv + (col ? hv : 0);
-  const size_t rs = (size_t)H * DV;
-  // values stay as loaded until they are used: a conversion here would wait
-  // for them
-  struct Vals {
-    T x[4];
+  const unsigned at_row0 = ck_row_slot(2 * wave, g, m16) * 16;
+  const unsigned at_row1 = ck_row_slot(2 * wave + 1, g, m16) * 16;
+  const unsigned at_col = ck_col_slot(2 * wave, g, m16) * 16;
+  const unsigned at_gam = (32 * wave + 4 * g) * 4;
+  const unsigned at_sq = (lane * 4 + wave) * 4;
+  auto operands = [&] {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)next, 0, It::TOTAL * 4,
+                                             0x00020000);
   };
-  auto fetch = [&](int c, ck_f32x4(&pf)[PF], Vals& pv) {
-    c = min(c, count - 1);
-    const char* base = src + (size_t)c * step;
+  auto load4 = [&](__amdgpu_buffer_rsrc_t r, unsigned at, int op) {
+    return __builtin_bit_cast(
+        ck_f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, op * 4, 0));
+  };
+  auto load1 = [&](__amdgpu_buffer_rsrc_t r, unsigned at, int op) {
+    return __uint_as_float(
+        __builtin_amdgcn_raw_buffer_load_b32(r, at, op * 4, 0));
+  };
+  // columns past the last one: beyond any buffer
+  const unsigned off = 0x80000000u;
+  unsigned at_v[4];
 #pragma unroll
-    for (int u = 0; u < PF - 1; ++u)
-      pf[u] = *(const ck_f32x4*)(base + u * 4096 + at16);
-    pf[PF - 1] = *(const ck_f32x4*)(base + at16l);
+  for (int i = 0; i < 4; ++i)
+    at_v[i] = col ? ((4 * g + i) * (unsigned)ldv + j) * sizeof(T) : off;
+  const unsigned rs = H * DV;
+  const unsigned at_out = col ? (g * rs + j) * 4 : off;
+  const T* vseg = v + (size_t)t0 * ldv + hd * DV;
+  float* oseg = raw + (size_t)t0 * rs + hd * DV;
+  // chunk c's rows (and more, up to the segment's end) of `p`, rows of `ld`
+  // elements of `e` bytes
+  auto rows_from = [&](const void* p, int c, unsigned ld, unsigned e) {
+    const unsigned more = min(n - 16 * c - 1, 16);
+    return __builtin_amdgcn_make_buffer_rsrc(
+        (char*)p + (size_t)c * (16u * e) * ld, 0, (more * ld + DV) * e,
+        0x00020000);
+  };
+
+  // operands of a chunk: what meets the state before it, and what is written
+  struct Reads {
+    ck_f32x4 r[2], u[2];
+    float cx[NQ], mx[NQ];  // this wave's tokens of the matrices on V
+    T v[4];                // as loaded: a conversion here would wait for them
+    float flag;
+  };
+  struct Writes {
+    ck_f32x4 k[2], b[2], gam[2];
+    float zx[NQ];  // this wave's tokens of the matrix on Z (Y)
+  };
+  constexpr int LASTSQ = MODE == CK_GD ? It::MB : It::M;
+  auto fetch_reads = [&](int c, Reads& x) {
+    const auto p = operands();
+    if constexpr (MODE != CK_GLA) {
+      x.u[0] = load4(p, at_row0, It::U);
+      x.u[1] = load4(p, at_row1, It::U);
+    }
+    if constexpr (PART != 1) {
+      x.r[0] = load4(p, at_row0, It::R);
+      x.r[1] = load4(p, at_row1, It::R);
+      x.flag = ((const float*)next)[It::FLAG];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int at = wave + q * NW < 4 ? q * NW * 4 : 0;
+      if constexpr (MODE != CK_GLA) x.cx[q] = load1(p, at_sq + at, It::C);
+      if constexpr (MODE != CK_CD && PART != 1)
+        x.mx[q] = load1(p, at_sq + at, It::M);
+    }
+    const auto vr = rows_from(vseg, min(c, count - 1), ldv, sizeof(T));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int tt = min(16 * c + 4 * g + i, n - 1);
-      pv.x[i] = vcol[(size_t)tt * ldv];
+      if constexpr (sizeof(T) == 2)
+        x.v[i].x = __builtin_amdgcn_raw_buffer_load_b16(vr, at_v[i], 0, 0);
+      else
+        x.v[i] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(vr, at_v[i], 0, 0));
     }
   };
-  auto put = [&](float* dst, const ck_f32x4(&pf)[PF]) {
+  auto fetch_writes = [&](int c, Writes& x) {
+    const auto p = operands();
 #pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      const int i = u * 256 + threadIdx.x;
-      if (i < N4) *(ck_f32x4*)(dst + i * 4) = pf[u];
+    for (int t = 0; t < 2; ++t) {
+      x.gam[t] = load4(p, at_gam, It::GAM + t * 16);
+      x.k[t] = load4(p, at_col, It::K + t * 256);
+      if constexpr (MODE == CK_GD) x.b[t] = load4(p, at_col, It::B + t * 256);
+    }
+    if constexpr (MODE != CK_GLA) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        x.zx[q] = load1(p, at_sq + (wave + q * NW < 4 ? q * NW * 4 : 0),
+                        LASTSQ);
+    }
+    if (c + 1 < count) next += step;
+  };
+
+  // the waves' shares of chunk c's rows: every wave takes groups of four,
+  // reads them early and adds them later
+  struct Shares {
+    float o[NQ][NW];
+  };
+  auto shares_of = [&](int c, Shares& x) {
+    const ck_f32x4* from = ox + (c & 1) * SET;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int w = 0; w < NW; ++w)
+        x.o[q][w] = ((const float*)(from + w * 64 +
+                                    min(wave + q * NW, 3) * 16 + m16))[g];
+  };
+  auto emit = [&](int c, const Shares& x) {
+    const auto out = rows_from(oseg, max(c, 0), rs, 4);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int tg = wave + q * NW;
+      float o = x.o[q][0];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) o += x.o[q][w];
+      __builtin_amdgcn_raw_buffer_store_b32(
+          __float_as_uint(o), out, c < 0 || tg > 3 ? off : at_out,
+          16 * tg * rs, 0);
     }
   };
 
-  // valid rows of this lane group in chunk c, and their values
-  auto rows_left = [&](int c) {
-    return col ? n - 16 * c - 4 * g : 0;
-  };
-  auto values = [&](int c, const Vals& pv) {
-    ck_f32x4 V;
-    const int left = rows_left(c);
+  const ck_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  // Chunk c from `rd` and `wr`; those of chunk c + 2 take their places as
+  // soon as they are used.
+  auto walk = [&](int c, Reads& rd, Writes& wr) {
+    ck_f32x4 V, Z[2] = {zero, zero}, O[2] = {zero, zero};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float x = MxElem<T>::ld(&pv.x[i]);
-      V[i] = i < left ? x : 0.f;
-    }
-    return V;
-  };
-
-  // One chunk from `buf` with the values `pv`. On the way the operands of
-  // chunk c + 2 are asked for (into pf / pv) and those of chunk c + 1 (`nf`)
-  // are put into `nbuf`: both among matrix products, which run on while the
-  // wave issues them.
-  auto walk = [&](int c, const float* buf, ck_f32x4(&pf)[PF], Vals& pv,
-                  float* nbuf, const ck_f32x4(&nf)[PF]) {
-    const ck_f32x4 V = values(c, pv);
-    // all operands of a stage are read ahead of its products
-    ck_f32x4 r4[NT], u4[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int at = ck_row_slot(tb + t, g, m16) * 4;
-      r4[t] = *(const ck_f32x4*)(buf + It::R + at);
-      if constexpr (MODE != CK_GLA)
-        u4[t] = *(const ck_f32x4*)(buf + It::U + at);
-    }
-    // the products with V that the other half does not make: half 0 has the
-    // solve's, half 1 the output's (gla: half 0 the output's)
-    const int sq = MODE == CK_GLA || (MODE == CK_GD && ds == 1)
-                       ? It::M : It::C;
-    const ck_f32x4 q4 = *(const ck_f32x4*)(buf + sq + lane * 4);
+    for (int i = 0; i < 4; ++i) V[i] = MxElem<T>::ld(&rd.v[i]);
+    // the same in every wave: all have all of V
     const bool fin =
-        buf[It::FLAG] == 0.f && !__any(!ck_finite(V));
-    __builtin_amdgcn_sched_barrier(0);
-    fetch(c + 2, pf, pv);
-    ck_f32x4 O = {0.f, 0.f, 0.f, 0.f}, Z = O, X = O;
+        PART == 1 || __all(rd.flag == 0.f && ck_finite(V));
+    // this wave's token of each group of four
+    auto pick = [&](const ck_f32x4& x, int q) {
+      const int i = wave + q * NW;
+      float y = i == 1 ? x[1] : x[0];
+      y = i == 2 ? x[2] : y;
+      return i == 3 ? x[3] : y;
+    };
+    // a product with a 16 x 16 matrix; where a number is not finite its terms
+    // come from `terms` below instead
+    const unsigned mask = __builtin_amdgcn_readfirstlane(fin ? ~0u : 0u);
+    auto on_tokens = [&](const float (&f)[NQ], const ck_f32x4& x,
+                         ck_f32x4& acc) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
+      for (int q = 0; q < NQ; ++q)
+        if (4 % NW == 0 || wave + q * NW < 4)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              __uint_as_float(__float_as_uint(f[q]) & mask),
+              __uint_as_float(__float_as_uint(pick(x, q)) & mask), acc, 0, 0,
+              0);
+    };
+    // The same term by term, zeros above the diagonal left out: beside a value
+    // that is no finite number they would reach earlier tokens. No loads here:
+    // where ways meet, waits are for the latest load of either.
+    auto terms = [&](const float (&f)[NQ], const ck_f32x4& x, ck_f32x4& acc) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (MODE != CK_GLA) {
-          Z = __builtin_amdgcn_mfma_f32_16x16x4f32(u4[t][i], S[t][i], Z, 0, 0,
-                                                   0);
-          O = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i], S[t][i], O, 0, 0,
-                                                   0);
-        } else if (i & 1) {
-          // two chains: a dependent product waits for the one before it
-          Z = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i], S[t][i], Z, 0, 0,
-                                                   0);
-        } else {
-          O = __builtin_amdgcn_mfma_f32_16x16x4f32(r4[t][i], S[t][i], O, 0, 0,
-                                                   0);
-        }
-      }
-      X = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[t & 3], V[t & 3], X, 0, 0,
-                                               0);
-      if (NT < 4 && t == NT - 1) {
-#pragma unroll
-        for (int i = NT; i < 4; ++i)
-          X = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[i], V[i], X, 0, 0, 0);
-      }
+      for (int q = 0; q < NQ; ++q)
+        if (4 % NW == 0 || wave + q * NW < 4)
+          acc = ck_token_terms(f[q], pick(x, q), acc, lane,
+                               tmps + wave * 128);
+    };
+    if (!fin) {
+      if constexpr (MODE != CK_GLA) terms(rd.cx, V, Z[1]);
+      if constexpr (MODE != CK_CD && PART != 1) terms(rd.mx, V, O[1]);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (MODE != CK_GLA) {
+      on_tokens(rd.cx, V, Z[1]);
 #pragma unroll
-    for (int u = 0; u < PF + 4; ++u) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // products
-      __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // addresses
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          // channel: Y = C V - U S
+          Z[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              MODE == CK_CD ? -rd.u[t][i] : rd.u[t][i], S[t][i], Z[i & 1], 0,
+              0, 0);
+    }
+    if constexpr (PART != 1) {
+      if constexpr (MODE != CK_CD) on_tokens(rd.mx, V, O[1]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          O[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              rd.r[t][i], S[t][i], O[i & 1], 0, 0, 0);
+    }
+    ck_f32x4* zs = zx + (c & 1) * SET;
+    if constexpr (MODE != CK_GLA && NW > 1) zs[wave * 64 + lane] = Z[0] + Z[1];
+    fetch_reads(c + 2, rd);
+#pragma unroll
+    for (int u = 0; u < 18; ++u) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x004, 2, 0);
       __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // a load
     }
+    if constexpr (PART != 1) __syncthreads();
+    ck_f32x4 zr[NW];
+    Shares so;
+    if constexpr (MODE != CK_GLA && NW > 1) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) zr[w] = zs[w * 64 + lane];
+    }
+    if constexpr (PART != 1) shares_of(c - 1, so);
     __builtin_amdgcn_sched_barrier(0);
-    const ck_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    if (!fin) X = ck_square_terms(buf + sq, V, zero, lane, tmp);
-    if constexpr (MODE == CK_GLA) {
-      O += Z;
-      if (ds == 0) O += X;
-    } else if constexpr (MODE == CK_GD) {
-      if (ds == 0)
-        Z += X;
-      else
-        O += X;
-    } else {
-      Z = ds == 0 ? X - Z : -Z;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      S[t] *= wr.gam[t];
+      if constexpr (PART == 1) decay[t] *= wr.gam[t];
     }
-    // the other half's share
-    float* mine = xch + wave * 512 + lane * 4;
-    const float* theirs = xch + (wave ^ 1) * 512 + lane * 4;
-    *(ck_f32x4*)mine = O;
-    if constexpr (MODE != CK_GLA) *(ck_f32x4*)(mine + 256) = Z;
-    ck_f32x4 k4[NT], b4[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int at = ck_col_slot(tb + t, g, m16) * 4;
-      k4[t] = *(const ck_f32x4*)(buf + It::K + at);
-      if constexpr (MODE == CK_GD) b4[t] = *(const ck_f32x4*)(buf + It::B + at);
-      const ck_f32x4 gam =
-          *(const ck_f32x4*)(buf + It::GAM + (tb + t) * 16 + g * 4);
-      S[t] *= gam;
-      if constexpr (PART == 1) decay[t] *= gam;
-    }
-    const int osq = MODE == CK_GD ? It::MB : It::M;
-    const ck_f32x4 o4 = *(const ck_f32x4*)(buf + osq + lane * 4);
-    __syncthreads();
-    O += *(const ck_f32x4*)theirs;
-    if constexpr (MODE != CK_GLA) Z += *(const ck_f32x4*)(theirs + 256);
-    // what is written with the k columns
-    const ck_f32x4 Y = MODE == CK_CD ? Z : V;
-    __builtin_amdgcn_sched_barrier(0);
-    put(nbuf, nf);
-    // tile by tile is a chain: step by step over the tiles is NT chains
-    ck_f32x4 P = zero;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (MODE == CK_GD) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(b4[t][i], Z[i], S[t],
-                                                      0, 0, 0);
-      }
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[t][i], Y[i], S[t], 0,
-                                                    0, 0);
-      if constexpr (MODE != CK_GLA)
-        P = __builtin_amdgcn_mfma_f32_16x16x4f32(o4[i], Z[i], P, 0, 0, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // products
-      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // an LDS write
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (PART != 1 && ds == 0) {
-      if constexpr (MODE != CK_GLA) {
-        if (!fin) P = ck_square_terms(buf + osq, Z, zero, lane, tmp);
-        O += P;
-      }
-      const int left = rows_left(c);
-      float* dst = raw + (size_t)(t0 + 16 * c + 4 * g) * rs + hv;
+    if constexpr (MODE == CK_GD) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (i < left) dst[i * rs] = O[i];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr.k[t][i], V[i], S[t],
+                                                      0, 0, 0);
+    }
+    ck_f32x4 Y = V;
+    if constexpr (MODE != CK_GLA) {
+      Y = NW > 1 ? zr[0] : Z[0] + Z[1];
+      // in one order, so that every wave has the same sum
+#pragma unroll
+      for (int w = 1; w < NW; ++w) Y += zr[w];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            MODE == CK_GD ? wr.b[t][i] : wr.k[t][i], Y[i], S[t], 0, 0, 0);
+    if constexpr (MODE != CK_GLA) {
+      on_tokens(wr.zx, Y, O[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (!fin) terms(wr.zx, Y, O[0]);
+    }
+    fetch_writes(c + 2, wr);
+    if constexpr (PART != 1) {
+      emit(c - 1, so);
+      ox[(c & 1) * SET + wave * 64 + lane] = O[0] + O[1];
     }
   };
 
-  float* buf0 = lds;
-  float* buf1 = lds + BUF;
-  ck_f32x4 fa[PF], fb[PF];
-  Vals va, vb;
-  fetch(0, fa, va);
-  fetch(1, fb, vb);
-  put(buf0, fa);
-  // all landed: the waits inside the loop then count its own loads only
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  // at the top: buf0 and va hold chunk c, fb and vb chunk c + 1
-  for (int c = 0; c < count; c += 2) {
-    walk(c, buf0, fa, va, buf1, fb);
-    if (c + 1 >= count) break;
+  Reads ra, rb;
+  Writes wa, wb;
+  fetch_reads(0, ra);
+  __builtin_amdgcn_sched_barrier(0);  // landing in this order, as below
+  fetch_writes(0, wa);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_reads(1, rb);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_writes(1, wb);
+  __builtin_amdgcn_sched_barrier(0);
+  // one way out: where ways meet, waits are for the latest load of either
+  int c = 0;
+#pragma unroll 1
+  for (; c + 1 < count; c += 2) {
+    walk(c, ra, wa);
+    walk(c + 1, rb, wb);
+  }
+  if (c < count) walk(c, ra, wa);
+  if constexpr (PART != 1) {
     __syncthreads();
-    walk(c + 1, buf1, fb, vb, buf0, fa);
-    if (c + 2 >= count) break;
-    __syncthreads();
+    Shares so;
+    shares_of(count - 1, so);
+    emit(count - 1, so);
   }
   float* Se = Sg;
   if constexpr (PART == 1) {
     Se = pt + run * rec;
-    if (cb == 0 && ct == 0 && m16 == 0) {
+    if (cb == 0 && m16 == 0) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          Se[(size_t)D * DV + 16 * (tb + t) + 4 * g + i] = decay[t][i];
+          Se[(size_t)D * DV + row(t, i)] = decay[t][i];
     }
   }
   if (col && (PART != 2 || last)) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 16 * (tb + t) + 4 * g + i;
-        if (d < D) Se[(size_t)d * DV + j] = S[t][i];
-      }
+      for (int i = 0; i < 4; ++i)
+        if (row(t, i) < D) Se[(size_t)row(t, i) * DV + j] = S[t][i];
   }
 }
 
@@ -1311,14 +1417,12 @@ static long ck_chunk_floats(int mode, int dp, int H, int G) {
 }
 
 // Measured (bf16, one MI355X, whole operation; token by token -> this form):
-//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 1.00 ms
-//     (operands 0.24, walk 0.73: 2.2 us a chunk, of which the products take
-//     1.0 and the issue of loads and LDS writes most of the rest; read-out
-//     0.08)
+//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.74 ms
+//     (operands 0.24, walk 0.41, read-out 0.08)
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
-//                                                            5.42 -> 0.70 ms
+//                                                            5.42 -> 0.55 ms
 //   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.64 ms
-//   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.09 ms
+//   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.07 ms
 //   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.84 ms
 // From 16 rows on a segment goes this way: one chunk costs about 15 us in
 // three launches, 16 tokens one by one 24 us.
@@ -1346,7 +1450,7 @@ static void ck_plan(int mode, int T_, int S_, int H, int G, int D, int* cap,
 // their start take the place of one of count chunks, so it pays from four runs
 // and 32 chunks on, where the workgroups of one walk (a head's columns by 32)
 // leave most of the chip idle: us in one walk -> in runs, bf16, one prompt: gla
-// 8 heads of 128 x 256, 1501 rows 147 -> 86, 400 rows (25 chunks, 4 runs) 57 ->
+// 8 heads of 128 x 256, 1501 rows 147 -> 86 (70 now), 400 rows (25 chunks, 4 runs) 57 ->
 // 60; 16 heads, 3000 rows (4 runs) 300 -> 258; ssd 48 heads of 128 x 64, 3000
 // rows (5 runs) 297 -> 180, 500 rows 74 -> 71; mlstm 16 heads of 128 x 128, 3000
 // rows (6 runs) 326 -> 222.
@@ -1409,26 +1513,18 @@ static int ck_launch(CK_ARGS) {
   ck_plan(MODE, T_, S_, H, G, D, &cap, &passes);
   float* raw = scratch;
   float* items = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
-  const int ncb = (DV + 31) / 32;
   const int parts = ck_parts(MODE, T_, S_, H, DV);
   float* part = items + (((size_t)cap * H * It::TOTAL + 3) & ~(size_t)3);
-  const size_t lds =
-      (2 * ((It::TOTAL + 1023) / 1024) * 1024 + 2048 + 1024) * sizeof(float);
-  if (lds > 65536 &&
-      hipFuncSetAttribute((const void*)ck_sweep_kernel<T, MODE, DP, 0>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)lds) != hipSuccess)
-    return 1;
   for (int p = 0; p < passes; ++p) {
     hipLaunchKernelGGL((ck_prep_kernel<T, MODE, DP>), dim3(cap, H), dim3(256),
                        0, stream, items, in, (const int*)seq_rows, S_, H, G,
                        D, scale, c0f, p * cap);
 #define CK_SWEEP(PART, RUNS)                                                 \
   hipLaunchKernelGGL((ck_sweep_kernel<T, MODE, DP, PART>),                   \
-                     dim3(S_ * H * ncb * (RUNS)), dim3(256), lds, stream,    \
-                     raw, items, cap, (const T*)in.v, in.ldv, (float*)state, \
-                     (const int*)seq_rows, S_, H, D, DV, p * cap, part,   \
-                     parts)
+                     dim3(S_ * H * ((DV + 15) / 16) * (RUNS)), dim3(DP * 2), \
+                     0, stream, raw, items, cap, (const T*)in.v, in.ldv,     \
+                     (float*)state, (const int*)seq_rows, S_, H, D, DV,      \
+                     p * cap, part, parts)
     if constexpr (MODE == CK_GLA) {
       if (parts > 1) {
         CK_SWEEP(1, parts - 1);

@@ -593,6 +593,24 @@ def test_recurrence_empty_segments(mode):
         assert _rel(ag, aux) < 2e-6
 
 
+@pytest.mark.parametrize("mode", ["general", "channel", "gla"])
+@pytest.mark.parametrize("lens", [
+    [33, 16, 0, 33, 70, 1, 16], [17] * 64, [16 + i % 3 for i in range(65)]])
+def test_recurrence_chunk_order(mode, lens):
+    """Walks start by length, up to 64 segments: equal lengths, empty and
+    single rows among them, one segment more; values end with their segment,
+    columns of the last workgroup beyond the head's."""
+    rows = _segs(lens, [3 * (i % 2) for i in range(len(lens))])
+    x, state, aux, call = _recurrence(mode, 2, 40, 40, rows, torch.float32)
+    rows = torch.tensor(rows, dtype=torch.int32)
+    sg = state.cuda()
+    got = call(_to_gpu(x), sg, None, rows.cuda())
+    want = call(x, state, None, rows)
+    # fp32 sums of up to 70 tokens x 40 channels
+    assert _rel(got, want) < 2e-5
+    assert _rel(sg, state) < 2e-6
+
+
 @pytest.mark.parametrize("H,G,D,S,n", [
     (8, 8, 40, 70, 31),      # 128 rows a workgroup, of five sequences
     (8, 8, 64, 36, 31),      # 64 rows
