@@ -83,16 +83,20 @@ struct CkItem {
 // Chunks of a segment of n rows (segments shorter than 16 rows are not this
 // kernel's). The chunks of all segments, one segment after the other, are the
 // items; a pass takes `cap` of them from `base` on.
-PS_DEV int ck_count(int n) { return n < 16 ? 0 : (n + 15) / 16; }
+template <int L = 16>
+PS_DEV int ck_count(int n) {
+  return n < 16 ? 0 : (n + L - 1) / L;
+}
 
 // Which chunk of which segment an item is; false past the last one. Every wave
 // of a block finds the same.
+template <int L = 16>
 PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int lane, int* seg,
                     int* chunk) {
   int base = 0;
   for (int s0 = 0; s0 < S_; s0 += 64) {
     const int s = s0 + lane;
-    const int cnt = s < S_ ? ck_count(seq_rows[4 * s + 1]) : 0;
+    const int cnt = s < S_ ? ck_count<L>(seq_rows[4 * s + 1]) : 0;
     int incl = cnt;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -740,8 +744,8 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
 #pragma unroll
       for (int w = 1; w < NW; ++w) o += x.o[q][w];
       __builtin_amdgcn_raw_buffer_store_b32(
-          __float_as_uint(o), out, c < 0 || tg > 3 ? off : at_out,
-          16 * tg * rs, 0);
+          __float_as_uint(o), out,
+          (c < 0 || tg > 3 ? off : at_out) + 16 * tg * rs, 0, 0);
     }
   };
 
@@ -946,11 +950,20 @@ __global__ __launch_bounds__(64) void ck_gates_kernel(
   float* mp = aux + ((size_t)slot * H + hd) * (D + 1) + D;
   float m = pos0 != 0 ? *mp : 0.f;
   const float bi = p0[hd], bf = p1[hd];
+  // the next 64 tokens' inputs are asked for before these are used: a wave
+  // alone on its SIMD has nothing else to wait beside
+  auto fetch = [&](int tb, float* zi, float* zf) {
+    const size_t row = (size_t)(t0 + min(tb + lane, n - 1));
+    *zi = MxElem<T>::ld(wr + row * ldwr + hd);
+    *zf = MxElem<T>::ld(dec + row * lddec + hd);
+  };
+  float zi, zf, ni, nf;
+  fetch(0, &ni, &nf);
   for (int tb = 0; tb < n; tb += 64) {
-    const int tt = min(tb + lane, n - 1);
-    const size_t row = (size_t)(t0 + tt);
-    const float zi = MxElem<T>::ld(wr + row * ldwr + hd) + bi;
-    const float zf = MxElem<T>::ld(dec + row * lddec + hd) + bf;
+    const size_t row = (size_t)(t0 + min(tb + lane, n - 1));
+    zi = ni + bi;
+    zf = nf + bf;
+    fetch(tb + 64, &ni, &nf);
     const float ig = cap * tanhf(zi / cap);
     const float fg = ck_log_sigmoid(cap * tanhf(zf / cap));
     float A = fg, B = ig;
@@ -1330,6 +1343,617 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
     }
 }
 
+// ---------------------------------------------------------------------------
+// one decay per head and token, bf16 rows: chunks of 32 on the bf16 unit
+// ---------------------------------------------------------------------------
+// The order of a chunk's 32 tokens in the inner index of a product: a lane
+// group's eight are 4 g .. + 3 and 16 + 4 g .. + 3, which are also the rows it
+// has of two accumulator tiles.
+#define CK_WIDE 32
+
+template <int DP>
+struct CkWide {  // per chunk and group, bytes
+  static constexpr int Q = 0;               // [2 token tiles][DP / 32][64] x 16
+  static constexpr int K = 64 * DP;         // [DP / 16][64] x 16, transposed
+  static constexpr int QK = 128 * DP;       // [3 blocks][64] x 16: q_t k_s, fp32
+  static constexpr int TOTAL = QK + 3072;
+};
+struct CkWideHead {  // per chunk and head, floats
+  static constexpr int A = 0;     // [32] decay of a token
+  static constexpr int W = 32;    // [32] its write scale
+  static constexpr int DR = 64;   // [32] decay from the start, with it, scaled
+  static constexpr int DK = 96;   // [32] write scale and decay to the end
+  static constexpr int P = 128;   // [32] decay from the block of four's start
+  static constexpr int SUF = 160; // [16] first half: behind it to 15
+  static constexpr int PRE = 176; // [16] second half: from 16, with it
+  static constexpr int GAM = 192; // decay over the chunk
+  static constexpr int TOTAL = 196;
+};
+
+template <int MODE, int DP>
+__global__ __launch_bounds__(256) void ck_prep_wide_kernel(
+    char* __restrict__ gitems, float* __restrict__ hitems, CkIn in,
+    const float* __restrict__ ga, const float* __restrict__ gw,
+    const int* __restrict__ seq_rows, int S_, int H, int G, int D,
+    float qscale, int base) {
+  typedef CkWide<DP> Gi;
+  typedef CkWideHead Hd;
+  constexpr int LD = DP + 8;
+  __shared__ __align__(16) unsigned short Q[32 * LD], K[32 * LD];
+  __shared__ __align__(16) float sa[8][32];
+  __shared__ float sw[8][32];
+
+  const int item = blockIdx.x, grp = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int seg, chunk;
+  if (!ck_find<CK_WIDE>(seq_rows, S_, base + item, lane, &seg, &chunk)) return;
+  const int n = seq_rows[4 * seg + 1];
+  const int row0 = seq_rows[4 * seg] + 32 * chunk;
+  const int nv = min(32, n - 32 * chunk);
+  const int g = lane >> 4, m16 = lane & 15;
+  if (blockIdx.z == 0) {
+    const mx_bf16* qp = (const mx_bf16*)in.q + grp * D;
+    const mx_bf16* kp = (const mx_bf16*)in.k + grp * D;
+    for (int i = threadIdx.x; i < 32 * DP; i += 256) {
+      const int t = i / DP, d = i % DP;
+      const size_t row = (size_t)(row0 + min(t, nv - 1));
+      const int dc = min(d, D - 1);
+      const unsigned short q = qp[row * in.ldq + dc].x;
+      const unsigned short k = kp[row * in.ldk + dc].x;
+      const bool live = t < nv && d < D;
+      Q[t * LD + d] = live ? q : 0;
+      K[t * LD + d] = live ? k : 0;
+    }
+    __syncthreads();
+    char* dst = gitems + ((size_t)item * G + grp) * Gi::TOTAL;
+    auto rows8 = [&](const unsigned short* x, int tok, int ks) {
+      const unsigned short* p = x + tok * LD + 32 * ks + 4 * g;
+      return ck_join(*(const ck_u32x2*)p, *(const ck_u32x2*)(p + 16));
+    };
+    if (wave < 3) {
+      // blocks (tokens t, s): (0, 0), (1, 0), (1, 1), s in rows
+      ck_f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < DP / 32; ++ks)
+        c = ck_mfma(rows8(K, (wave == 2 ? 16 : 0) + m16, ks),
+                    rows8(Q, (wave == 0 ? 0 : 16) + m16, ks), c);
+      *(ck_f32x4*)(dst + Gi::QK + (wave * 64 + lane) * 16) = c * qscale;
+    }
+    for (int f = wave; f < DP / 16; f += 4) {
+      // f: token tile and 32 channels of Q, 16 channels of K
+      const int mt = f / (DP / 32), ks = f % (DP / 32);
+      *(ck_u32x4*)(dst + Gi::Q + (f * 64 + lane) * 16) =
+          rows8(Q, 16 * mt + m16, ks);
+      unsigned short x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        x[j] = K[((j >> 2) * 16 + 4 * g + (j & 3)) * LD + 16 * f + m16];
+      ck_u32x4 y;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = x[2 * j] | (unsigned)x[2 * j + 1] << 16;
+      *(ck_u32x4*)(dst + Gi::K + (f * 64 + lane) * 16) = y;
+    }
+  }
+  // this slice's heads, 8 at a time: a thread per token
+  const int per = H / G;
+  const int slice = (per + gridDim.z - 1) / gridDim.z;
+  const int h1 = min(per, (int)(blockIdx.z + 1) * slice);
+  const int hl = threadIdx.x >> 5, t = threadIdx.x & 31;
+  for (int hb = blockIdx.z * slice; hb < h1; hb += 8) {
+    const int hd = grp * per + min(hb + hl, h1 - 1);
+    const size_t row = (size_t)(row0 + min(t, nv - 1));
+    float a, w;
+    if (MODE == CK_SSD) {
+      w = ck_softplus(
+          MxElem<mx_bf16>::ld((const mx_bf16*)in.dec + row * in.lddec + hd) +
+          in.p0[hd]);
+      a = expf(-expf(in.p1[hd]) * w);
+    } else {
+      a = ga[row * H + hd];
+      w = gw[row * H + hd];
+    }
+    a = t < nv ? a : 1.f;
+    w = t < nv ? w : 0.f;
+    __syncthreads();
+    sa[hl][t] = a;
+    sw[hl][t] = w;
+    __syncthreads();
+    if (hb + hl < h1) {
+      // products up to t (of all, of its half, of its four) and behind t; a
+      // decay that is not in a product must not touch it: no quotients
+      float dr = 1.f, pre = 1.f, p4 = 1.f, to = 1.f, suf = 1.f;
+#pragma unroll
+      for (int j4 = 0; j4 < 8; ++j4) {
+        const ck_f32x4 a4 = *(const ck_f32x4*)(&sa[hl][j4 * 4]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = j4 * 4 + i;
+          const float up = j <= t ? a4[i] : 1.f;
+          dr *= up;
+          if (j >= 16) pre *= up;
+          p4 *= j >= (t & ~3) ? up : 1.f;
+          const float down = j > t ? a4[i] : 1.f;
+          to *= down;
+          if (j < 16) suf *= down;
+        }
+      }
+      float* dst = hitems +
+                   ((size_t)item * H + grp * per + hb + hl) * Hd::TOTAL;
+      dst[Hd::A + t] = a;
+      dst[Hd::W + t] = w;
+      dst[Hd::DR + t] = dr * qscale;
+      dst[Hd::DK + t] = to * w;
+      dst[Hd::P + t] = p4;
+      if (t < 16)
+        dst[Hd::SUF + t] = suf;
+      else
+        dst[Hd::PRE + t - 16] = pre;
+      if (t == 31) dst[Hd::GAM] = dr;
+    }
+  }
+}
+
+// Walks the chunks of one (segment, head): NW tiles of 16 columns of the state a
+// workgroup, each in two waves that have half of its rows (one wave where DP is
+// no multiple of 64). out, PART, part and parts as in ck_sweep_scalar_kernel,
+// whose products these are, for bf16 q, k and v.
+//
+// Q, K and V go into the products as they are and the state, the weights of the
+// chunk's own rows (M) and the scaled values (W) as three bf16 terms: no number
+// is rounded, and the matrix unit takes 3 / 16 of the fp32 products' time. What
+// bounds the walk is then the issue of instructions, above all cutting the
+// state into terms (176 for a tile's rows), once a chunk, which is why a chunk
+// has 32 tokens. M, the same for all columns of a head, is made by three waves
+// and passes through LDS, a chunk ahead; the two waves of a tile exchange their
+// shares of O there, each for the token tile that the other one writes. One
+// barrier a chunk does for both.
+// Measured (ssd, 128 heads of 128 x 64, 8192 rows in 2 prompts): 605 us by
+// fp32 products in chunks of 16, 330 with all rows of a tile in one wave (one
+// wave a SIMD: 800 instructions in 5300 cycles), 285 with two.
+template <int MODE, int DP, int PART, int NW>
+__global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_wide_kernel(
+    float* __restrict__ out, int ldo, const char* __restrict__ gitems,
+    const float* __restrict__ hitems, int cap, CkIn in,
+    const float* __restrict__ p2, float* __restrict__ state,
+    float* __restrict__ aux, const int* __restrict__ seq_rows, int S_, int H,
+    int G, int D, int DV, int base, float* __restrict__ part, int parts) {
+  typedef CkWide<DP> Gi;
+  typedef CkWideHead Hd;
+  constexpr int RH = DP % 64 == 0 ? 2 : 1;   // waves that share a column tile
+  constexpr int NT = DP / 16, NK = DP / 32;  // tiles of the state
+  constexpr int WT = NT / RH, WK = NK / RH;  // and of a wave
+  __shared__ ck_u32x4 mfrag[2][2][3][64];  // set, token tile, term
+  __shared__ float vtmp[NW * RH][512];
+  __shared__ ck_f32x4 share[2][RH == 2 ? NW * RH : 1][64];
+
+  const int cols = DV + (MODE == CK_MLSTM ? 1 : 0);
+  const int ncb = ((cols + 15) / 16 + NW - 1) / NW;
+  const int run = PART ? blockIdx.x / (S_ * H) / ncb : 0;
+  const int rest = blockIdx.x - run * S_ * H * ncb;
+  const int hd = rest % H, cb = rest / H % ncb;
+  const int seg = ck_by_length(seq_rows, S_, rest / (H * ncb));
+  if (seg < 0) return;
+  const int sh = seg * H + hd, grp = hd / (H / G);
+  int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
+  const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  const int all = ck_count<CK_WIDE>(n);
+  if (all == 0) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int first = 0;
+  for (int s = lane; s < seg; s += 64)
+    first += ck_count<CK_WIDE>(seq_rows[4 * s + 1]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
+  first = __builtin_amdgcn_readfirstlane(first) - base;  // of this pass
+  int c0 = max(0, -first);
+  int count =
+      __builtin_amdgcn_readfirstlane(min(all, cap - first) - c0);
+  if (count <= 0) return;
+  first += c0;
+  const bool old = p0 != 0 || c0 != 0;  // there is a state to start from
+  bool last = true;  // this run ends the segment's chunks of the pass
+  if constexpr (PART != 0) {
+    const int per = (count + parts - 1) / parts;
+    last = (run + 1) * per >= count;
+    if (run * per >= count) return;
+    first += run * per;
+    c0 += run * per;
+    count = min(per, count - run * per);
+  }
+  // the rows from the first chunk on
+  t0 = __builtin_amdgcn_readfirstlane(t0 + 32 * c0);
+  n = __builtin_amdgcn_readfirstlane(n - 32 * c0);
+
+  const int g = lane >> 4, m16 = lane & 15;
+  // which part of the rows; a wave's rows of the output are the token tile of
+  // that number where two share them
+  const int rh = RH == 2 ? wave & 1 : 0;
+  const int j = (cb * NW + wave / RH) * 16 + m16;
+  const bool col = j < DV;
+  const bool ncol = MODE == CK_MLSTM && j == DV;
+  float* Sg = state + ((size_t)slot * H + hd) * (size_t)D * DV + j;
+  float* Ng = MODE == CK_MLSTM ? aux + ((size_t)slot * H + hd) * (D + 1)
+                               : nullptr;
+  const size_t rec = (size_t)D * cols + 4;  // of one run
+  float* pt = PART ? part + (size_t)sh * parts * rec : nullptr;
+  ck_f32x4 S[WT];
+#pragma unroll
+  for (int t = 0; t < WT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = 16 * (WT * rh + t) + 4 * g + i;
+      float x = 0.f;
+      if (PART != 2 && d < D && old) {
+        if (col) x = Sg[(size_t)d * DV];
+        if (ncol) x = Ng[d];
+      }
+      if constexpr (PART == 1) {
+        if (run == 0 && d < D && (col || ncol))
+          pt[(parts - 1) * rec + (size_t)d * cols + j] = x;
+        x = 0.f;
+      }
+      if constexpr (PART == 2) {
+        if (d < D && (col || ncol))
+          x = pt[(parts - 1) * rec + (size_t)d * cols + j];
+      }
+      S[t][i] = x;
+    }
+  if constexpr (PART == 2) {
+#pragma unroll 2
+    for (int q = 0; q < run; ++q) {
+      const float a = pt[q * rec + (size_t)D * cols];
+#pragma unroll
+      for (int t = 0; t < WT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int d = 16 * (WT * rh + t) + 4 * g + i;
+          const float add = d < D && (col || ncol)
+                                ? pt[q * rec + (size_t)d * cols + j]
+                                : 0.f;
+          S[t][i] = S[t][i] * a + add;
+        }
+    }
+  }
+  float decay = 1.f;  // over the run
+
+  // Everything comes through buffers: a uniform base, a uniform offset and a
+  // 32-bit one per lane; rows behind the segment read as zero and are not
+  // written, nor are columns behind the last one (`off` is beyond any buffer).
+  const size_t gstep = (size_t)G * Gi::TOTAL;
+  const size_t hstep = (size_t)H * Hd::TOTAL * sizeof(float);
+  // of the chunk ahead by one, two (the last one again behind it)
+  const char* g1 = gitems + ((size_t)first * G + grp) * Gi::TOTAL;
+  const char* g2 = g1;
+  const char* h2 =
+      (const char*)(hitems + ((size_t)first * H + hd) * Hd::TOTAL);
+  const unsigned at16 = lane * 16, off = 0x80000000u;
+  const unsigned rsv = in.ldv * 2, rsg = in.ldg * 2, rso = ldo * 4;
+  const unsigned at_v = col ? 4 * g * rsv + j * 2 : off;
+  const unsigned at_g = col ? 4 * g * rsg + j * 2 : off;
+  const unsigned at_o = col || ncol ? 4 * g * rso + j * 4 : off;
+  const char* vseg =
+      (const char*)((const mx_bf16*)in.v + (size_t)t0 * in.ldv + hd * DV);
+  const char* gseg =
+      MODE == CK_SSD
+          ? (const char*)((const mx_bf16*)in.gate + (size_t)t0 * in.ldg +
+                          hd * DV)
+          : nullptr;
+  char* oseg = (char*)(out + (size_t)t0 * ldo +
+                       hd * (MODE == CK_SSD ? DV : DV + 1));
+  // chunk c's rows (and more, up to the segment's end) of `p`, `rb` bytes
+  // apart, `width` bytes of each
+  auto rows_from = [&](const char* p, int c, unsigned rb, unsigned width) {
+    const unsigned more = min(n - 32 * c - 1, 32);
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(p + (size_t)c * 32 * rb),
+                                             0, more * rb + width, 0x00020000);
+  };
+  const float skip = MODE == CK_SSD ? p2[hd] : 0.f;
+
+  struct Cells {  // of this lane's rows, as loaded
+    unsigned short v[8], gt[8 / RH];
+  };
+  struct Block {  // of M: scores, decays (or what lies behind), scales
+    ck_f32x4 qk, x, w;
+    float y, u1, u2;
+  };
+  struct Scales {
+    ck_f32x4 dr[2 / RH], dk[2];
+    float gam;
+  };
+  // of Q the wave's own token tile first
+  ck_u32x4 Q[PART == 1 ? 1 : 2 * WK], K[WT];
+  auto fetch_q = [&] {
+    const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)g1, 0, Gi::TOTAL,
+                                                     0x00020000);
+#pragma unroll
+    for (int f = 0; f < 2 * WK; ++f)
+      Q[f] = __builtin_bit_cast(
+          ck_u32x4,
+          __builtin_amdgcn_raw_buffer_load_b128(
+              r, at16,
+              Gi::Q + (((f / WK) ^ rh) * NK + WK * rh + f % WK) * 1024, 0));
+  };
+  auto fetch_k = [&] {
+    const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)g1, 0, Gi::TOTAL,
+                                                     0x00020000);
+#pragma unroll
+    for (int f = 0; f < WT; ++f)
+      K[f] = __builtin_bit_cast(
+          ck_u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                        r, at16, Gi::K + (WT * rh + f) * 1024, 0));
+  };
+  auto fetch_cells = [&](int c, Cells& x) {
+    c = min(c, count - 1);
+    const auto vr = rows_from(vseg, c, rsv, DV * 2);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      x.v[i] = __builtin_amdgcn_raw_buffer_load_b16(
+          vr, at_v + ((i >> 2) * 16 + (i & 3)) * rsv, 0, 0);
+    if constexpr (MODE == CK_SSD && PART != 1) {
+      const auto gr = rows_from(gseg, c, rsg, DV * 2);
+#pragma unroll
+      for (int i = 0; i < 8 / RH; ++i)
+        x.gt[i] = __builtin_amdgcn_raw_buffer_load_b16(
+            gr, at_g + ((i >> 2) * 16 + rh * 16 + (i & 3)) * rsg, 0, 0);
+    }
+  };
+  auto head_buffer = [&] {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)h2, 0, Hd::TOTAL * 4,
+                                             0x00020000);
+  };
+  auto load4 = [&](__amdgpu_buffer_rsrc_t r, unsigned at, int from) {
+    return __builtin_bit_cast(
+        ck_f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, from, 0));
+  };
+  auto fetch_block = [&](int h, Block& x) {
+    h = min(h, 2);
+    const auto r = head_buffer();
+    const int b = h == 2 ? 16 : 0;
+    x.qk = load4(__builtin_amdgcn_make_buffer_rsrc((void*)g2, 0, Gi::TOTAL,
+                                                   0x00020000),
+                 at16, Gi::QK + h * 1024);
+    x.x = load4(r, g * 16, (h == 1 ? Hd::SUF : Hd::A + b) * 4);
+    x.w = load4(r, g * 16, (Hd::W + b) * 4);
+    x.y = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+        r, m16 * 4, (h == 1 ? Hd::PRE : Hd::P + b) * 4, 0));
+    x.u1 = ((const float*)h2)[Hd::P + b + 7];
+    x.u2 = ((const float*)h2)[Hd::P + b + 11];
+  };
+  auto fetch_scales = [&](Scales& x) {
+    const auto r = head_buffer();
+    if constexpr (PART != 1) {
+#pragma unroll
+      for (int mt = 0; mt < 2 / RH; ++mt)
+        x.dr[mt] = load4(r, g * 16, (Hd::DR + 16 * (mt + rh)) * 4);
+    }
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+      x.dk[mt] = load4(r, g * 16, (Hd::DK + 16 * mt) * 4);
+    x.gam = ((const float*)h2)[Hd::GAM];
+  };
+  // a block of M: rows s = 4 g + i of its half, column t = m16 of its own;
+  // every decay between them by products of its own
+  auto make_block = [&](int h, const Block& x, ck_u32x4* to) {
+    h = min(h, 2);
+    // no branches: where ways meet, waits are for the latest load of either
+    const int b = h == 1 ? 4 : m16 >> 2;
+    float tail = b > g ? x.y : 1.f;
+    tail *= g < 1 && (b == 2 || b == 3) ? x.u1 : 1.f;
+    tail *= g < 2 && b == 3 ? x.u2 : 1.f;
+    ck_f32x4 e;
+    e[3] = h == 1 ? tail * x.x[3] : tail;
+#pragma unroll
+    for (int i = 2; i >= 0; --i)
+      e[i] = h == 1 ? tail * x.x[i]
+                    : e[i + 1] * (4 * g + i + 1 <= m16 ? x.x[i + 1] : 1.f);
+    ck_f32x4 m;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      m[i] = h == 1 || 4 * g + i <= m16 ? x.qk[i] * e[i] * x.w[i] : 0.f;
+    const CkTerms4 tm = ck_split(m);
+    // token tile, half of the lane's eight
+    ck_u32x2* dst = (ck_u32x2*)(to + (h == 0 ? 0 : 192) + lane) + (h == 2);
+    dst[0] = tm.h;
+    dst[128] = tm.m;
+    dst[256] = tm.l;
+  };
+
+  const ck_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  // Chunk c; what is used makes room for a later chunk's at once.
+  auto walk = [&](int c, Cells& cells, Scales& sc, Block& blk) {
+    // the next chunk's M
+    if constexpr (PART != 1) {
+      make_block(wave, blk, &mfrag[(c + 1) & 1][0][0][0]);
+      fetch_block(wave, blk);
+    }
+    ck_f32x4 V[2], W[2], O[2] = {zero, zero}, X[2] = {zero, zero};
+    float gt[8 / RH];
+    const int left = n - 32 * c - 4 * g;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float y = __uint_as_float((unsigned)cells.v[i] << 16);
+      if (MODE == CK_MLSTM && ncol)
+        y = (i >> 2) * 16 + (i & 3) < left ? 1.f : 0.f;
+      V[i >> 2][i & 3] = y;
+    }
+#pragma unroll
+    for (int i = 0; i < 8 / RH; ++i)
+      gt[i] = __uint_as_float((unsigned)cells.gt[i] << 16);
+    const Scales s0 = sc;
+    const bool fin =
+        PART == 1 || __all(ck_finite(V[0]) && ck_finite(V[1]));
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_cells(c + 2, cells);
+    fetch_scales(sc);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) W[mt] = V[mt] * s0.dk[mt];
+    if constexpr (PART != 1) {
+      // values that are no finite numbers are left out here: beside the zeros
+      // above M's diagonal they would reach earlier tokens
+      ck_f32x4 F[2] = {V[0], V[1]};
+      if (!fin) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (!(fabsf(V[i >> 2][i & 3]) < INFINITY)) F[i >> 2][i & 3] = 0.f;
+      }
+      const ck_u32x4 vb = {
+          ck_pack_high(F[0][0], F[0][1]), ck_pack_high(F[0][2], F[0][3]),
+          ck_pack_high(F[1][0], F[1][1]), ck_pack_high(F[1][2], F[1][3])};
+      const ck_u32x4(*mf)[3][64] = mfrag[c & 1];
+#pragma unroll
+      for (int q = 2; q >= 0; --q)
+#pragma unroll
+        for (int mt = 0; mt < 2 / RH; ++mt)
+          X[mt] = ck_mfma(mf[mt + rh][q][lane], vb, X[mt]);
+      if (!fin) {
+        // what the left out values add
+        float* tmp = vtmp[wave];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          tmp[((i >> 2) * 16 + 4 * g + (i & 3)) * 16 + m16] =
+              V[i >> 2][i & 3];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int s = 0; s < 32; ++s) {
+          const float xs = tmp[s * 16 + m16];
+          if (fabsf(xs) < INFINITY) continue;
+#pragma unroll
+          for (int i = 0; i < 8 / RH; ++i) {
+            // entry (t, s) of M in fragment order
+            const int at = ((s >> 2 & 3) * 16 + 4 * g + (i & 3)) * 8 +
+                           (s >> 4) * 4 + (s & 3);
+            float a = 0.f;
+#pragma unroll
+            for (int q = 2; q >= 0; --q)
+              a += ps_bf16_to_f32(
+                  ((const unsigned short*)mfrag[c & 1][(i >> 2) + rh][q])[at]);
+            if (a != 0.f) X[i >> 2][i & 3] += a * xs;
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < WK; ++ks) {
+      if constexpr (PART != 1) {
+        const CkTerms8 ts = ck_split(S[2 * ks], S[2 * ks + 1]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+          O[mt] = ck_mfma(Q[mt * WK + ks], ts.l, O[mt]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+          O[mt] = ck_mfma(Q[mt * WK + ks], ts.m, O[mt]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+          O[mt] = ck_mfma(Q[mt * WK + ks], ts.h, O[mt]);
+      }
+      S[2 * ks] *= s0.gam;
+      S[2 * ks + 1] *= s0.gam;
+    }
+    if constexpr (PART != 1) {
+      fetch_q();
+      if constexpr (RH == 2) share[c & 1][wave][lane] = O[1];
+    }
+    if constexpr (PART == 1) decay *= s0.gam;
+    const CkTerms8 tw = ck_split(W[0], W[1]);
+#pragma unroll
+    for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.l, S[t]);
+#pragma unroll
+    for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.m, S[t]);
+#pragma unroll
+    for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.h, S[t]);
+    fetch_k();
+    g1 = g2;
+    if (c + 3 < count) {
+      g2 += gstep;
+      h2 += hstep;
+    }
+    if constexpr (PART != 1) {
+      // also: the next chunk's M is there, this one's is read
+      __syncthreads();
+      if constexpr (RH == 2) O[0] += share[c & 1][wave ^ 1][lane];
+      const auto orow =
+          rows_from(oseg, c, rso, (MODE == CK_SSD ? DV : DV + 1) * 4);
+#pragma unroll
+      for (int i = 0; i < 8 / RH; ++i) {
+        const int mt = i >> 2, e = i & 3;
+        float o = fmaf(O[mt][e], s0.dr[mt][e], X[mt][e]);
+        if (MODE == CK_SSD)
+          o = fmaf(skip, rh ? V[1][e] : V[mt][e], o) * gt[i] *
+              ck_sigmoid(gt[i]);
+        __builtin_amdgcn_raw_buffer_store_b32(
+            __float_as_uint(o), orow, at_o + (mt * 16 + rh * 16 + e) * rso, 0,
+            0);
+      }
+    }
+  };
+
+  Cells ca, cb2;
+  Scales sa, sb;
+  Block blk;
+  const char *gn = g2, *hn = h2;  // chunk 1's
+  if (count > 1) {
+    gn += gstep;
+    hn += hstep;
+  }
+  if constexpr (PART != 1) {
+    const ck_u32x2 none = {0, 0};
+    for (int i = threadIdx.x; i < 384; i += 64 * NW * RH)  // tile 0, second half
+      ((ck_u32x2*)&mfrag[i / 192][0][i / 64 % 3][i % 64])[1] = none;
+    fetch_block(wave, blk);
+    make_block(wave, blk, &mfrag[0][0][0][0]);
+    __syncthreads();
+  }
+  // the order in which a chunk's loads are asked for below: the waits of the
+  // loop are for what is later in either
+  fetch_cells(0, ca);
+  fetch_scales(sa);
+  __builtin_amdgcn_sched_barrier(0);
+  g2 = gn;
+  h2 = hn;
+  if constexpr (PART != 1) fetch_block(wave, blk);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_cells(1, cb2);
+  fetch_scales(sb);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (PART != 1) fetch_q();
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_k();
+  __builtin_amdgcn_sched_barrier(0);
+  g1 = gn;
+  if (count > 2) {
+    g2 += gstep;
+    h2 += hstep;
+  }
+  int c = 0;
+#pragma unroll 1
+  for (; c + 1 < count; c += 2) {
+    walk(c, ca, sa, blk);
+    walk(c + 1, cb2, sb, blk);
+  }
+  if (c < count) walk(c, ca, sa, blk);
+  if (PART == 1 && cb == 0 && threadIdx.x == 0)
+    pt[run * rec + (size_t)D * cols] = decay;
+  if (PART == 2 && !last) return;
+#pragma unroll
+  for (int t = 0; t < WT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = 16 * (WT * rh + t) + 4 * g + i;
+      if (d < D) {
+        if (PART == 1) {
+          if (col || ncol) pt[run * rec + (size_t)d * cols + j] = S[t][i];
+        } else {
+          if (col) Sg[(size_t)d * DV] = S[t][i];
+          if (ncol) Ng[d] = S[t][i];
+        }
+      }
+    }
+}
+
 // Read-out norm and gate: o / rms_DV(o) * weight * gate for the rows of
 // segments that the sweep walked. A wave takes four heads of a row; a lane
 // holds VEC neighbouring columns of each, 64 * VEC >= DV.
@@ -1407,8 +2031,15 @@ static int ck_pad(int D) {
   return 0;
 }
 
-// Floats per chunk: of all heads' (and groups') operands.
-static long ck_chunk_floats(int mode, int dp, int H, int G) {
+// bf16 rows with one decay per head and token go in chunks of 32.
+template <typename T, int MODE>
+static constexpr bool ck_wide() {
+  return MODE >= CK_SSD && sizeof(T) == 2;
+}
+// Floats per chunk of L rows: of all heads' (and groups') operands.
+static long ck_chunk_floats(int mode, int dp, int H, int G, int L) {
+  if (L == CK_WIDE)
+    return (long)G * (32 * dp + 768) + (long)H * CkWideHead::TOTAL;
   if (mode >= CK_SSD)
     return (long)G * 32 * dp + (long)H * CkHead::TOTAL;
   const int rows = mode == CK_GD ? 4 : (mode == CK_CD ? 3 : 2);
@@ -1421,52 +2052,70 @@ static long ck_chunk_floats(int mode, int dp, int H, int G) {
 //     (operands 0.24, walk 0.41, read-out 0.08)
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
 //                                                            5.42 -> 0.55 ms
-//   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.64 ms
+//   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.31 ms
 //   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.07 ms
 //   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.84 ms
 // From 16 rows on a segment goes this way: one chunk costs about 15 us in
 // three launches, 16 tokens one by one 24 us.
 //
 // Chunks laid down at once, and the passes over all of them. A step's segments
-// of 16 rows and more have at most T / 16 + S chunks, and at most T / 8; passes
-// keep the scratch below CK_BYTES. They follow the chunks of one segment after
-// the other: by chunk number within every segment, 256 segments of 48 rows took
-// 250 passes for the one segment that could be (general delta, 32 heads of
-// 128 x 128: 27 ms, 2.1 with two passes, 3.7 token by token).
+// of 16 rows and more have at most T / L + S chunks of L rows, and at most
+// 2 T / L (T / 16 of 32); passes keep the scratch below CK_BYTES. They follow
+// the chunks of one segment after the other: by chunk number within every
+// segment, 256 segments of 48 rows took 250 passes for the one segment that
+// could be (general delta, 32 heads of 128 x 128: 27 ms, 2.1 with two passes,
+// 3.7 token by token).
 #define CK_BYTES (1l << 30)
-static void ck_plan(int mode, int T_, int S_, int H, int G, int D, int* cap,
-                    int* passes) {
-  const long per = ck_chunk_floats(mode, ck_pad(D), H, G) * 4;
-  long all = (long)T_ / 16 + S_;
-  if (all > T_ / 8 + 1) all = T_ / 8 + 1;
+static void ck_plan(int mode, int T_, int S_, int H, int G, int D, int L,
+                    int* cap, int* passes) {
+  const long per = ck_chunk_floats(mode, ck_pad(D), H, G, L) * 4;
+  long all = (long)T_ / L + S_;
+  if (all > T_ / (L / 2) + 1) all = T_ / (L / 2) + 1;
   long fit = CK_BYTES / per;
   if (fit < 1) fit = 1;
   *cap = (int)(all < fit ? all : fit);
   *passes = (int)((all + *cap - 1) / *cap);
 }
 
+// Column tiles that a workgroup of the wide walk has: three where four would
+// leave waves without columns.
+static int ck_wide_tiles(int tiles) {
+  return tiles % 3 == 0 && tiles % 4 != 0 ? 3 : 4;
+}
 // Runs that a segment's chunks are walked in (not the delta forms, whose state
 // is multiplied by more than a decay). Two walks of count / runs chunks and
-// their start take the place of one of count chunks, so it pays from four runs
-// and 32 chunks on, where the workgroups of one walk (a head's columns by 32)
-// leave most of the chip idle: us in one walk -> in runs, bf16, one prompt: gla
-// 8 heads of 128 x 256, 1501 rows 147 -> 86 (70 now), 400 rows (25 chunks, 4 runs) 57 ->
-// 60; 16 heads, 3000 rows (4 runs) 300 -> 258; ssd 48 heads of 128 x 64, 3000
-// rows (5 runs) 297 -> 180, 500 rows 74 -> 71; mlstm 16 heads of 128 x 128, 3000
-// rows (6 runs) 326 -> 222.
-static int ck_parts(int mode, int T_, int S_, int H, int DV) {
+// their start take the place of one of count chunks, so it pays while the
+// workgroups of all runs still find room: one a CU of the wide walk (eight
+// waves), two of gla's. us in one walk, two, four, eight runs, bf16:
+//   ssd    48 heads of 128 x 64, 1 prompt of  300   39   41   42   42
+//                                             600   49   48   41   48
+//                                            3000  182  133   83   91
+//         128 heads,             1 prompt of  600   54   52   58   76
+//                                            3000  186  140  149  168
+//   mlstm  16 heads of 128 x 128,            3000  218  185  140  146
+//   gla     8 heads of 128 x 256,             300   38   41   41   40
+//                                             600   48   46   44   47
+//                                            1501   88   75   68   71
+//          16 heads,                          600   51   54   56   64
+//                                            3000  172  160  159  173
+// The fp32 walk of ssd and mlstm as it was measured first: four and more.
+static int ck_parts(int mode, int T_, int S_, int H, int DV, int L) {
   if (mode == CK_GD || mode == CK_CD) return 1;
-  const int cols = DV + (mode == CK_MLSTM ? 1 : 0);
-  const long blocks = (long)S_ * H * ((cols + 31) / 32);
+  const int tiles = (DV + (mode == CK_MLSTM ? 1 : 0) + 15) / 16;
+  const bool narrow = mode != CK_GLA && L != CK_WIDE;
+  const int wg = mode == CK_GLA ? 1 : (narrow ? 2 : ck_wide_tiles(tiles));
+  const long blocks = (long)S_ * H * ((tiles + wg - 1) / wg);
   const int longest = (T_ - S_ + 1 + 15) / 16;
-  long parts = 512 / blocks;
+  long parts = (L == CK_WIDE ? 256 : 512) / blocks;
   if (parts > 16) parts = 16;
   if (parts > longest / 6) parts = longest / 6;
-  return parts < 4 || longest < 32 ? 1 : (int)parts;
+  const int fewest = narrow || longest < 64 ? 4 : 2;
+  return parts < fewest || longest < 32 ? 1 : (int)parts;
 }
 // Floats of the runs' records.
-static long ck_part_floats(int mode, int T_, int S_, int H, int D, int DV) {
-  const int parts = ck_parts(mode, T_, S_, H, DV);
+static long ck_part_floats(int mode, int T_, int S_, int H, int D, int DV,
+                           int L) {
+  const int parts = ck_parts(mode, T_, S_, H, DV, L);
   if (parts == 1) return 0;
   const long rec = mode == CK_GLA ? (long)D * DV + ck_pad(D)
                                   : (long)D * (DV + 1) + 4;
@@ -1510,10 +2159,10 @@ template <typename T, int MODE, int DP>
 static int ck_launch(CK_ARGS) {
   typedef CkItem<MODE, DP> It;
   int cap, passes;
-  ck_plan(MODE, T_, S_, H, G, D, &cap, &passes);
+  ck_plan(MODE, T_, S_, H, G, D, 16, &cap, &passes);
   float* raw = scratch;
   float* items = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
-  const int parts = ck_parts(MODE, T_, S_, H, DV);
+  const int parts = ck_parts(MODE, T_, S_, H, DV, 16);
   float* part = items + (((size_t)cap * H * It::TOTAL + 3) & ~(size_t)3);
   for (int p = 0; p < passes; ++p) {
     hipLaunchKernelGGL((ck_prep_kernel<T, MODE, DP>), dim3(cap, H), dim3(256),
@@ -1542,7 +2191,7 @@ static int ck_launch(CK_ARGS) {
 template <typename T, int MODE, int DP>
 static int ck_launch_scalar(CK_ARGS) {
   int cap, passes;
-  ck_plan(MODE, T_, S_, H, G, D, &cap, &passes);
+  ck_plan(MODE, T_, S_, H, G, D, 16, &cap, &passes);
   const bool lstm = MODE == CK_MLSTM;
   float* raw = scratch;
   float* ga = raw + (lstm ? (size_t)T_ * H * (DV + 1) : 0);
@@ -1551,7 +2200,7 @@ static int ck_launch_scalar(CK_ARGS) {
   float* gitems = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
   float* hitems = gitems + (size_t)cap * G * CkGroup<DP>::TOTAL;
   const int ncb = (DV + (lstm ? 1 : 0) + 31) / 32;
-  const int parts = ck_parts(MODE, T_, S_, H, DV);
+  const int parts = ck_parts(MODE, T_, S_, H, DV, 16);
   float* part = hitems + (((size_t)cap * H * CkHead::TOTAL + 3) & ~(size_t)3);
   if (lstm)
     hipLaunchKernelGGL((ck_gates_kernel<T>), dim3(S_ * H), dim3(64), 0,
@@ -1584,12 +2233,66 @@ static int ck_launch_scalar(CK_ARGS) {
   return 0;
 }
 
+template <int MODE, int DP>
+static int ck_launch_wide(CK_ARGS) {
+  int cap, passes;
+  ck_plan(MODE, T_, S_, H, G, D, CK_WIDE, &cap, &passes);
+  const bool lstm = MODE == CK_MLSTM;
+  float* raw = scratch;
+  float* ga = raw + (lstm ? (size_t)T_ * H * (DV + 1) : 0);
+  float* gw = ga + (lstm ? (size_t)T_ * H : 0);
+  float* ge = gw + (lstm ? (size_t)T_ * H : 0);
+  float* gitems = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
+  float* hitems = gitems + (size_t)cap * G * (CkWide<DP>::TOTAL / 4);
+  const int tiles = (DV + (lstm ? 1 : 0) + 15) / 16;
+  const int parts = ck_parts(MODE, T_, S_, H, DV, CK_WIDE);
+  float* part = hitems + (size_t)cap * H * CkWideHead::TOTAL;
+  if (lstm)
+    hipLaunchKernelGGL((ck_gates_kernel<mx_bf16>), dim3(S_ * H), dim3(64), 0,
+                       stream, ga, gw, ge, (const mx_bf16*)in.a, in.lda,
+                       (const mx_bf16*)in.dec, in.lddec, in.p0, in.p1,
+                       (float*)aux, (const int*)seq_rows, H, D, c0f);
+  // a group's heads over a few blocks where there are many
+  const int slices = (H / G + 31) / 32;
+  for (int p = 0; p < passes; ++p) {
+    hipLaunchKernelGGL((ck_prep_wide_kernel<MODE, DP>), dim3(cap, G, slices),
+                       dim3(256), 0, stream, (char*)gitems, hitems, in, ga,
+                       gw, (const int*)seq_rows, S_, H, G, D, scale, p * cap);
+#define CK_SWEEP_NW(PART, RUNS, NW)                                          \
+  hipLaunchKernelGGL((ck_sweep_wide_kernel<MODE, DP, PART, NW>),             \
+                     dim3(S_ * H * ((tiles + NW - 1) / NW) * (RUNS)),        \
+                     dim3(64 * NW * (DP % 64 == 0 ? 2 : 1)), 0, stream,      \
+                     lstm ? raw : (float*)out,                               \
+                     lstm ? H * (DV + 1) : ldo, (const char*)gitems, hitems, \
+                     cap, in, (const float*)p2, (float*)state, (float*)aux,  \
+                     (const int*)seq_rows, S_, H, G, D, DV, p * cap, part,   \
+                     parts)
+#define CK_SWEEP(PART, RUNS)                                                 \
+  if (ck_wide_tiles(tiles) == 3)                                             \
+    CK_SWEEP_NW(PART, RUNS, 3);                                              \
+  else                                                                       \
+    CK_SWEEP_NW(PART, RUNS, 4)
+    if (parts > 1) {
+      CK_SWEEP(1, parts - 1);
+      CK_SWEEP(2, parts);
+    } else {
+      CK_SWEEP(0, 1);
+    }
+#undef CK_SWEEP
+#undef CK_SWEEP_NW
+  }
+  if constexpr (MODE == CK_MLSTM) ck_read<mx_bf16, MODE>(CK_PASS, raw, ge);
+  return 0;
+}
+
 template <typename T, int MODE>
 static int ck_dispatch(CK_ARGS) {
   switch (ck_pad(D)) {
 #define CK_CASE(DP)                                                         \
   case DP:                                                                  \
-    if constexpr (MODE >= CK_SSD)                                           \
+    if constexpr (ck_wide<T, MODE>())                                       \
+      return ck_launch_wide<MODE, DP>(CK_PASS);                             \
+    else if constexpr (MODE >= CK_SSD)                                      \
       return ck_launch_scalar<T, MODE, DP>(CK_PASS);                        \
     else                                                                    \
       return ck_launch<T, MODE, DP>(CK_PASS);
@@ -1637,11 +2340,18 @@ CK_UNIT(ck_mlstm) CK_BODY(CK_MLSTM)
 extern "C" long mx_chunk_scratch(int mode, int T_, int S_, int H, int G,
                                  int D, int DV) {
   if (S_ <= 0 || T_ - S_ + 1 < 16 || ck_pad(D) == 0 || DV > 256) return 0;
-  int cap, passes;
-  ck_plan(mode, T_, S_, H, G, D, &cap, &passes);
-  return ((ck_rows_floats(mode, T_, H, DV) + 3) & ~3l) +
-         ((cap * ck_chunk_floats(mode, ck_pad(D), H, G) + 3) & ~3l) +
-         ck_part_floats(mode, T_, S_, H, D, DV);
+  // of both element types' forms the larger
+  long need = 0;
+  for (int L = 16; L <= (mode >= CK_SSD ? CK_WIDE : 16); L += 16) {
+    int cap, passes;
+    ck_plan(mode, T_, S_, H, G, D, L, &cap, &passes);
+    const long x =
+        ((ck_rows_floats(mode, T_, H, DV) + 3) & ~3l) +
+        ((cap * ck_chunk_floats(mode, ck_pad(D), H, G, L) + 3) & ~3l) +
+        ck_part_floats(mode, T_, S_, H, D, DV, L);
+    if (x > need) need = x;
+  }
+  return need;
 }
 
 extern "C" int mx_chunk_delta(void* out, int ldo, const void* r, int ldr,

@@ -55,3 +55,59 @@ PS_DEV float ck_softplus(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 PS_DEV float ck_log_sigmoid(float z) {
   return fminf(z, 0.f) - log1pf(expf(-fabsf(z)));
 }
+
+// fp32 numbers on the bf16 matrix unit: each is exactly the sum of three bf16
+// terms (h, m, l: 8 bits each; the first one is cut off and not rounded, so
+// that the largest numbers stay finite). Beside an operand that is bf16 already
+// every product is exact, and the unit takes 3 / 16 of the fp32 unit's time.
+typedef __attribute__((ext_vector_type(2))) unsigned ck_u32x2;
+typedef __attribute__((ext_vector_type(4))) unsigned ck_u32x4;
+typedef __attribute__((ext_vector_type(8))) __bf16 ck_bf16x8;
+
+struct CkTerms4 {  // of four numbers
+  ck_u32x2 h, m, l;
+};
+struct CkTerms8 {
+  ck_u32x4 h, m, l;
+};
+
+PS_DEV unsigned ck_pack_high(float a, float b) {  // upper halves, a the low one
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a),
+                               0x07060302u);
+}
+
+PS_DEV void ck_split2(float a, float b, unsigned* h, unsigned* m,
+                      unsigned* l) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  const unsigned top = 0xffff0000u;
+  *h = ck_pack_high(a, b);
+  const f32x2 r = {a - __uint_as_float(__float_as_uint(a) & top),
+                   b - __uint_as_float(__float_as_uint(b) & top)};
+  *m = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+  const f32x2 q = {r[0] - __uint_as_float(*m << 16),
+                   r[1] - __uint_as_float(*m & top)};
+  *l = __builtin_bit_cast(unsigned, __builtin_convertvector(q, bf16x2));
+}
+
+PS_DEV CkTerms4 ck_split(ck_f32x4 x) {
+  unsigned h[2], m[2], l[2];
+  ck_split2(x[0], x[1], &h[0], &m[0], &l[0]);
+  ck_split2(x[2], x[3], &h[1], &m[1], &l[1]);
+  return {{h[0], h[1]}, {m[0], m[1]}, {l[0], l[1]}};
+}
+
+PS_DEV ck_u32x4 ck_join(ck_u32x2 a, ck_u32x2 b) {
+  return {a[0], a[1], b[0], b[1]};
+}
+
+PS_DEV CkTerms8 ck_split(ck_f32x4 a, ck_f32x4 b) {
+  const CkTerms4 x = ck_split(a), y = ck_split(b);
+  return {ck_join(x.h, y.h), ck_join(x.m, y.m), ck_join(x.l, y.l)};
+}
+
+PS_DEV ck_f32x4 ck_mfma(ck_u32x4 a, ck_u32x4 b, ck_f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+      __builtin_bit_cast(ck_bf16x8, a), __builtin_bit_cast(ck_bf16x8, b), c, 0,
+      0, 0);
+}
