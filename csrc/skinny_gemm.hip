@@ -1,21 +1,10 @@
 // Skinny-batch GEMM for decode steps: out[M, N] = x[M, K] @ W[N, K]^T,
 // bf16 inputs, fp32 accumulation, M <= 256.
 //
-// Why it exists: hipBLASLt's tile selection for the decode-shaped GEMMs
-// (qkv [M,4096]x[6144,4096], o, down) streams weights at only 1.4-2 TB/s at
-// M in 16..128 (profiles/gemm_plain.log) when the op is purely
-// weight-bandwidth-bound (~6 TB/s available). This kernel is built around
-// streaming W exactly once:
-//   grid = (N/64, SPLITS): workgroup owns 64 N-rows x a K-range.
-//   4 waves x 16 N-rows each; B-frags are direct 16-B lane loads from W
-//   (lane's col = its N-row, contiguous dims) -- W bytes are read once
-//   across the whole grid.
-//   x (tiny) is staged per 64-wide K-chunk in XOR-swizzled LDS and consumed
-//   as A-frags for ceil(M/16) m-tiles; per-k-chunk MFMA count scales with
-//   m-tiles while W traffic stays fixed.
-//   Split-K partials go to an fp32 workspace that a second kernel adds up.
-// That is the form for 17 to 256 rows, and for 9 to 16 where W has more than
-// 32768; fewer have one of their own, below.
+// Why it exists: the library's tiles for the products of a decode batch leave
+// the read of W, which bounds them, at a third to a half of the rate that memory
+// gives. Up to 16 rows (8 of a W of more than 32768) go without splits, more
+// by the tiled form below; figures stand at both.
 // mfma_f32_16x16x32_bf16; operand k-pattern as verified in
 // csrc/tools/mfma_probe.hip.
 #include "ps_common.h"
@@ -115,84 +104,160 @@ __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
   }
 }
 
-template <int M_TILES>
-__global__ __launch_bounds__(256, 4) void skinny_gemm_kernel(
-    unsigned short* __restrict__ out_bf16,  // [M, N] (splits == 1)
-    float* __restrict__ ws,                 // [S, M, N] (splits > 1)
-    const unsigned short* __restrict__ x,   // [M, K]
-    const unsigned short* __restrict__ w,   // [N, K]
-    int M, int N, int K, long x_stride /* row stride of x, elems */) {
-  constexpr int MP = M_TILES * 16;  // padded M
-  const int n0 = blockIdx.x * 64;
-  const int splits = gridDim.y;
-  const int kchunks = K / 64;
-  const int per_split = (kchunks + splits - 1) / splits;
-  const int kc_begin = blockIdx.y * per_split;
-  const int kc_end = min(kchunks, kc_begin + per_split);
-  if (kc_begin >= kc_end) return;
+// 17 to 256 rows of x (and 9 to 16 of a W of more than 32768): a workgroup owns
+// 64 NC rows of W, all rows of x and a range of K, in steps of 128 columns. x
+// passes through LDS, two steps' buffers with one barrier a step; W goes from
+// memory straight into left operands, WD steps ahead. The eight waves are four by
+// rows of W times two by halves of a step, which add up in LDS at the end.
+// Partial sums of the ranges go to memory and are added by skinny_combine.
+//
+// Bound by the read of W while a range is long enough to hide its start, and by
+// the reads of x from LDS with many rows (each wave reads all of x: 16 NC rows of
+// W share a read). us, distinct weights, this / the form it replaces (a barrier
+// on each side of 64 columns, loads not ahead) / the library's kernel:
+//   4096 x 14336   64 rows 31 / 48 / 39, 128 rows 37 / 66 / 74, 192 43 / 83 / 106
+//   4096 x 4096    64 rows 14 / 22 / 14, 192 rows 23 / 39 / 31
+//   28672 x 4096   64 rows 56 / 96 / 52, 192 rows 71 / 150 / 61
+//   2048 x 8192    64 rows 14 / 25,      192 rows 23 / 39
+// Waves split by rows of x as well read W twice: 10 to 40 % slower.
+template <int MT, int NC>
+__global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
+    unsigned short* __restrict__ out,      // [M, N] (one split)
+    float* __restrict__ ws,                // [splits, M, N]
+    const unsigned short* __restrict__ x,  // [M, K], rows x_stride apart
+    const unsigned short* __restrict__ w,  // [N, K]
+    int M, int N, int K, long x_stride, int splits) {
+  constexpr int BN = 64 * NC;
+  constexpr int WD = NC == 1 ? 4 : 3;       // steps of W in flight
+  constexpr int XL = (MT + 1) / 2;          // pieces of x a thread stages
+  constexpr int XB = (MT + MT % 2) * 2048;  // entries of one buffer
+  constexpr int PN = BN + 4;                // pitch of a row of sums
+  // sums in two halves of the rows where all are more than the buffers
+  constexpr int MH = MT * 32 * PN > 2 * XB && MT > 1 ? MT / 2 : MT;
+  constexpr int LDS = MH * 32 * PN > 2 * XB ? MH * 32 * PN : 2 * XB;
+  __shared__ __align__(16) unsigned short lds[LDS];
+  // the ranges of one tile side by side: an XCD reads few ranges of x
+  const int split = blockIdx.x % splits, n0 = blockIdx.x / splits * BN;
+  const int chunks = K / 64, per = (chunks + splits - 1) / splits;
+  const int c0 = split * per, c1 = min(chunks, c0 + per);
+  const int steps = (c1 - c0 + 1) / 2;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave >> 2, wn = wave & 3;  // half of a step, rows of W
+  const int rc = lane & 15, g = lane >> 4;
 
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
-  const int g = lane >> 4;
-  const int rc = lane & 15;
-  const int nrow = n0 + wave * 16 + rc;  // this lane's W row (B col)
-
-  // x chunk [MP][64] staged with 16-B slot XOR swizzle (slot ^= row&7)
-  __shared__ __align__(16) unsigned short x_lds[MP][64];
-
-  ps_gf32x4 acc[M_TILES];
+  const unsigned short* wp[NC];
 #pragma unroll
-  for (int mt = 0; mt < M_TILES; mt++) acc[mt] = {0.f, 0.f, 0.f, 0.f};
-
-  for (int kc = kc_begin; kc < kc_end; kc++) {
-    // ---- cooperative x staging: MP*8 16-B slots over 256 threads ----
-    for (int u = tid; u < MP * 8; u += 256) {
-      const int row = u >> 3;
-      const int slot = u & 7;
-      ps_bf16x8 v = {};
-      if (row < M)
-        v = *(const ps_bf16x8*)(x + (long)row * x_stride + kc * 64 +
-                                slot * 8);
-      *(ps_bf16x8*)(&x_lds[row][(slot ^ (row & 7)) * 8]) = v;
-    }
-    __syncthreads();
-    // ---- B-frags: W rows streamed once ----
-    const unsigned short* wr = w + (long)nrow * K + kc * 64;
-    ps_gbf16x8 b0 = ps_as_gbf16(*(const ps_bf16x8*)(wr + g * 8));
-    ps_gbf16x8 b1 = ps_as_gbf16(*(const ps_bf16x8*)(wr + 32 + g * 8));
-    __builtin_amdgcn_s_setprio(1);
+  for (int c = 0; c < NC; ++c)
+    wp[c] = w + (long)(n0 + (wn * NC + c) * 16 + rc) * K + g * 8;
+  ps_gbf16x8 wf[WD][NC][2];
+  // steps past the end repeat the last chunk and are not multiplied
+  auto load_w = [&](int u, int t) {
+    const int k = min(c0 + 2 * t + kg, c1 - 1) * 64;
 #pragma unroll
-    for (int mt = 0; mt < M_TILES; mt++) {
-      const int row = mt * 16 + rc;
-      ps_gbf16x8 a0 = ps_as_gbf16(
-          *(const ps_bf16x8*)(&x_lds[row][(g ^ (row & 7)) * 8]));
-      ps_gbf16x8 a1 = ps_as_gbf16(
-          *(const ps_bf16x8*)(&x_lds[row][((4 + g) ^ (row & 7)) * 8]));
-      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[mt],
-                                                        0, 0, 0);
-      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[mt],
-                                                        0, 0, 0);
-    }
-    __builtin_amdgcn_s_setprio(0);
-    __syncthreads();
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        wf[u][c][h] = *(const ps_gbf16x8*)(wp[c] + k + 32 * h);
+  };
+  // x: a thread takes one of a row's 16 slots of 16 bytes in XL rows, swizzled
+  // by the row so that reads of 16 rows spread over the banks
+  const int xs = tid & 15;
+  ps_bf16x8 xf[2][XL];
+  const unsigned short* xp[XL];
+  int xd[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int row = i * 32 + (tid >> 4);
+    xp[i] = x + (long)min(row, M - 1) * x_stride;
+    xd[i] = row * 128 + (xs ^ (row & 7)) * 8;
   }
-
-  // ---- epilogue (C layout: row=(g*4+r), col=rc of each 16x16 tile).
-  // splits==1 writes bf16 output directly; otherwise each split streams
-  // its fp32 partial to ws[split][M][N] and a combine kernel reduces —
-  // device atomicAdd RMW traffic (M*N*splits) was the measured 1/M
-  // throughput wall of the earlier design.
+  auto load_x = [&](int u, int t) {
+    const int k = min(c0 + 2 * t + (xs >> 3), c1 - 1) * 64 + (xs & 7) * 8;
 #pragma unroll
-  for (int mt = 0; mt < M_TILES; mt++) {
+    for (int i = 0; i < XL; ++i) xf[u][i] = *(const ps_bf16x8*)(xp[i] + k);
+  };
+  auto put_x = [&](int u) {
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int m = mt * 16 + g * 4 + r;
-      if (m >= M) continue;
-      if (gridDim.y == 1) {
-        out_bf16[(long)m * N + nrow] = ps_f32_to_bf16(acc[mt][r]);
-      } else {
-        ws[((long)blockIdx.y * M + m) * N + nrow] = acc[mt][r];
+    for (int i = 0; i < XL; ++i)
+      *(ps_bf16x8*)(lds + u * XB + xd[i]) = xf[u][i];
+  };
+  ps_gf32x4 acc[NC][MT];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[c][i] = {0.f, 0.f, 0.f, 0.f};
+  load_x(0, 0);
+#pragma unroll
+  for (int u = 0; u < WD; ++u) load_w(u, u);
+  load_x(1, 1);
+  put_x(0);
+  load_x(0, 2);
+  __syncthreads();
+  const int xr0 = rc * 128 + ((kg * 8 + g) ^ (rc & 7)) * 8;
+  const int xr1 = rc * 128 + ((kg * 8 + 4 + g) ^ (rc & 7)) * 8;
+  constexpr int UN = WD % 2 == 0 ? WD : 2 * WD;
+  for (int t = 0; t < steps; t += UN) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      if (t + u < steps) {
+        const unsigned short* buf = lds + (u & 1) * XB;
+        // the other buffer was read before the last barrier
+        put_x((u + 1) & 1);
+        load_x((u + 1) & 1, t + u + 3);
+        if (c0 + 2 * (t + u) + kg < c1) {
+#pragma unroll
+          for (int i = 0; i < MT; ++i) {
+            const ps_gbf16x8 b0 = *(const ps_gbf16x8*)(buf + i * 2048 + xr0);
+            const ps_gbf16x8 b1 = *(const ps_gbf16x8*)(buf + i * 2048 + xr1);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+              acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  wf[u % WD][c][0], b0, acc[c][i], 0, 0, 0);
+              acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  wf[u % WD][c][1], b1, acc[c][i], 0, 0, 0);
+            }
+          }
+        }
+        load_w(u % WD, t + u + WD);
+        __syncthreads();
+      }
+    }
+  }
+  // acc[c][i][r]: row 16 i + rc of x, row n0 + (wn NC + c) 16 + 4 g + r of W
+  float* sum = (float*)lds;
+#pragma unroll
+  for (int h = 0; h < MT; h += MH) {
+    if (h > 0) __syncthreads();
+    if (kg == 1) {
+#pragma unroll
+      for (int i = 0; i < MH; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          *(ps_gf32x4*)(sum + (i * 16 + rc) * PN + (wn * NC + c) * 16 +
+                        4 * g) = acc[c][h + i];
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+      for (int i = 0; i < MH; ++i) {
+        const int m = (h + i) * 16 + rc;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const int n = (wn * NC + c) * 16 + 4 * g;
+          const ps_gf32x4 v =
+              acc[c][h + i] +
+              *(const ps_gf32x4*)(sum + (i * 16 + rc) * PN + n);
+          if (m >= M) continue;
+          if (splits > 1)
+            *(ps_gf32x4*)(ws + ((long)split * M + m) * N + n0 + n) = v;
+          else
+            *(uint2*)(out + (long)m * N + n0 + n) = make_uint2(
+                (unsigned int)ps_f32_to_bf16(v[0]) |
+                    ((unsigned int)ps_f32_to_bf16(v[1]) << 16),
+                (unsigned int)ps_f32_to_bf16(v[2]) |
+                    ((unsigned int)ps_f32_to_bf16(v[3]) << 16));
+        }
       }
     }
   }
@@ -201,15 +266,53 @@ __global__ __launch_bounds__(256, 4) void skinny_gemm_kernel(
 __global__ __launch_bounds__(256) void skinny_combine_kernel(
     unsigned short* __restrict__ out,  // [M, N] bf16
     const float* __restrict__ ws,      // [S, M, N] fp32
-    long MN, int splits) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    long MN, int splits) {             // MN: a multiple of 64
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= MN) return;
-  float acc = 0.f;
-  for (int s = 0; s < splits; s++) acc += ws[(long)s * MN + i];
-  out[i] = ps_f32_to_bf16(acc);
+  ps_gf32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < splits; s++)
+    a += *(const ps_gf32x4*)(ws + (long)s * MN + i);
+  *(uint2*)(out + i) =
+      make_uint2((unsigned int)ps_f32_to_bf16(a[0]) |
+                     ((unsigned int)ps_f32_to_bf16(a[1]) << 16),
+                 (unsigned int)ps_f32_to_bf16(a[2]) |
+                     ((unsigned int)ps_f32_to_bf16(a[3]) << 16));
 }
 
-
+// Tiles of 64 or 128 rows of W and the ranges of K: as many workgroups as there
+// are CUs, or as few more as one wave of narrow tiles takes. A range has four
+// chunks at least, or its start is most of it. Of the two widths the one that
+// fills more CUs; at as many the wide one for long rows (its reads of x from LDS
+// go to twice the products), the narrow one for short ones (its partial sums are
+// half). us at 192 rows, narrow / wide: 6144 x 4096 32 (192 workgroups) / 29
+// (240), 4096 x 4096 23 / 24, 4096 x 14336 48 / 43, 2560 x 10240 33 (200) / 33
+// (160), 18944 x 3584 82 (296) / 58 (148), 16384 x 2048 30 / 37. Above 192 rows
+// the wide tile's sums do not fit in the registers.
+struct PsSkinnyPlan {
+  bool wide;
+  int splits;
+};
+static PsSkinnyPlan ps_skinny_plan(int M, int N, int K) {
+  const int chunks = K / 64, most = chunks / 4 > 1 ? chunks / 4 : 1;
+  int splits[2], used[2];
+  for (int wide = 0; wide < 2; ++wide) {
+    const int tiles = wide ? (N + 127) / 128 : N / 64;
+    int s = 256 / tiles;
+    if (s > most) s = most;
+    if (s < 1) s = 1;
+    // whole ranges of ceil(chunks / s) chunks are handed out: count those that
+    // are not empty, since an empty one would write no partial sums
+    const int per = (chunks + s - 1) / s;
+    splits[wide] = (chunks + per - 1) / per;
+    // workgroups past the CUs wait for a second turn
+    used[wide] = tiles > 256 ? 128 : tiles * splits[wide];
+  }
+  const bool wide = N % 128 == 0 && M <= 192 &&
+                    (used[1] > used[0] ||
+                     (used[1] == used[0] && (K >= 8192 || N > 32768)));
+  return {wide, splits[wide]};
+}
 
 // Whether the kernel without splits takes it; its byte offsets are 31 bits.
 // More than 8 rows reread x too often where the other form needs no splits
@@ -264,45 +367,44 @@ int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
 // the fp32 workspace.
 int ps_skinny_gemm_splits(int M, int N, int K) {
   if (N < 64 || K < 64 || N % 64 != 0 || K % 64 != 0 || M > 256) return -1;
-  if (M <= 16) return 1;
-  const int kchunks = K / 64;
-  const int target_wgs = 1024;
-  int splits = target_wgs / (N / 64);
-  if (splits < 1) splits = 1;
-  if (splits > kchunks) splits = kchunks;
-  // the kernel hands out whole ranges of ceil(kchunks / splits) chunks: count
-  // the ranges that are not empty, since an empty one writes no partial and
-  // the combine pass would add what its workspace happened to hold
-  const int per_split = (kchunks + splits - 1) / splits;
-  return (kchunks + per_split - 1) / per_split;
+  if (M <= 16 && N <= 32768) return 1;
+  return ps_skinny_plan(M, N, K).splits;
 }
 
 int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
                    int M, int N, int K, long x_stride, hipStream_t stream) {
-  int splits = ps_skinny_gemm_splits(M, N, K);
-  if (splits < 0) return -1;
+  if (ps_skinny_gemm_splits(M, N, K) < 0) return -1;
   if (M < 1) return 0;  // no rows: their size in bytes would wrap below
   if (ps_skinny_rows(M, N, K, x_stride)) {
     ps_skinny_rows_go<false>(out_bf16, x, w, M, N, K, x_stride, stream);
     return 0;
   }
-  if (ws == nullptr) splits = 1;
-  dim3 grid(N / 64, splits);
-  dim3 block(256);
-#define PS_SG(MT)                                                           \
-  skinny_gemm_kernel<MT><<<grid, block, 0, stream>>>(                       \
-      (unsigned short*)out_bf16, (float*)ws, (const unsigned short*)x,      \
-      (const unsigned short*)w, M, N, K, x_stride)
-  if (M <= 16) PS_SG(1);
-  else if (M <= 32) PS_SG(2);
-  else if (M <= 64) PS_SG(4);
-  else if (M <= 128) PS_SG(8);
-  else PS_SG(16);
+  PsSkinnyPlan plan = ps_skinny_plan(M, N, K);
+  if (ws == nullptr) plan.splits = 1;
+#define PS_SG(MT, NC)                                                       \
+  skinny_tile_kernel<MT, NC>                                                \
+      <<<dim3(N / (64 * NC) * plan.splits), dim3(512), 0, stream>>>(        \
+          (unsigned short*)out_bf16, (float*)ws, (const unsigned short*)x,  \
+          (const unsigned short*)w, M, N, K, x_stride, plan.splits)
+#define PS_SG2(MT)                                                          \
+  do {                                                                      \
+    if (plan.wide)                                                          \
+      PS_SG(MT, 2);                                                         \
+    else                                                                    \
+      PS_SG(MT, 1);                                                         \
+  } while (0)
+  if (M <= 16) PS_SG2(1);
+  else if (M <= 32) PS_SG2(2);
+  else if (M <= 64) PS_SG2(4);
+  else if (M <= 128) PS_SG2(8);
+  else if (M <= 192) PS_SG2(12);
+  else PS_SG(16, 1);
+#undef PS_SG2
 #undef PS_SG
-  if (splits > 1) {
+  if (plan.splits > 1) {
     const long MN = (long)M * N;
-    skinny_combine_kernel<<<dim3((MN + 255) / 256), 256, 0, stream>>>(
-        (unsigned short*)out_bf16, (const float*)ws, MN, splits);
+    skinny_combine_kernel<<<dim3((MN / 4 + 255) / 256), 256, 0, stream>>>(
+        (unsigned short*)out_bf16, (const float*)ws, MN, plan.splits);
   }
   return 0;
 }

@@ -246,8 +246,8 @@ def kv_dequant(
 
 
 def skinny_gemm(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """out = x @ w.T for decode-shaped M<=128 (weight-stream-bound GEMMs
-    where hipBLASLt tiles poorly — see csrc/skinny_gemm.hip). GPU only."""
+    """out = x @ w.T for up to 256 rows of x (csrc/skinny_gemm.hip). GPU
+    only."""
     _require_ext()
     out = torch.empty(
         (x.shape[0], w.shape[0]), dtype=torch.bfloat16, device=x.device

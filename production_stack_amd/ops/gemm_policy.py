@@ -1,10 +1,9 @@
 """Per-shape GEMM dispatch: hipBLASLt (torch F.linear) vs the in-house
 skinny split-K MFMA kernel.
 
-hipBLASLt's decode-shaped tiles stream weights at 0.8-2 TB/s for several
-(M<=128, N, K) projections while csrc/skinny_gemm.hip reaches 2.4-5 TB/s at
-M<=32 (profiles/gemm_skinny.log) — but loses at larger M. Instead of a
-hardcoded table, the engine autotunes each (decode bucket M, projection
+The library's decode-shaped tiles leave the read of the weights at a third to
+a half of memory's rate for several projections, csrc/skinny_gemm.hip does for
+others: the engine autotunes each (decode bucket M, projection
 shape) pair once at startup on the actual device and the winner is what the
 hipGraph capture records.
 """
@@ -74,19 +73,12 @@ def tune(weights, buckets, device) -> None:
     )
 
 
-def _few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Untuned shapes that take the in-house kernel: up to 3 rows and rows of
-    W of up to 4096 entries. us, in-house / library: 1 x 2048 x 2048 4.9 / 8.2,
-    1 x 28672 x 4096 46 / 64, 3 x 4096 x 4096 11.0 / 15.8, 3 x 6144 x 4096
-    15.8 / 15.8; past the line 4 x 6144 x 4096 16.2 / 15.7, 1 x 2048 x 8192
-    14.5 / 12.8. Short rows of a wide W are the library's: 3 x 65536 x 1024
-    29.1 / 27.7, 3 x 50304 x 768 19.5 / 18.8 (3 x 51200 x 2560 53 / 52, 1 row 50 /
-    52)."""
+def _fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Operands that the in-house kernel takes as they are."""
     from production_stack_amd import ops
 
-    return (x.dim() == 2 and 0 < x.shape[0] <= 3 and w.shape[1] <= 4096
+    return (x.dim() == 2 and x.shape[0] > 0
             and _eligible(x.shape[0], *w.shape) and x.stride(1) == 1
-            and (w.shape[1] > 1024 or w.shape[0] < 32768)
             and x.shape[1] == w.shape[1] and w.dtype == torch.bfloat16
             and w.is_contiguous() and x.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
@@ -95,12 +87,36 @@ def _few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
                      and (x.requires_grad or w.requires_grad)))
 
 
+def _few_rows(rows: int, N: int, K: int) -> bool:
+    """Up to 3 rows and rows of W of up to 4096 entries. us, in-house /
+    library: 1 x 2048 x 2048 4.9 / 8.2, 1 x 28672 x 4096 46 / 64, 3 x 4096 x 4096
+    11.0 / 15.8, 3 x 6144 x 4096 15.8 / 15.8; past the line 4 x 6144 x 4096 16.2 /
+    15.7, 1 x 2048 x 8192 14.5 / 12.8. Short rows of a wide W are the library's:
+    3 x 65536 x 1024 29.1 / 27.7, 3 x 50304 x 768 19.5 / 18.8 (3 x 51200 x 2560
+    53 / 52, 1 row 50 / 52)."""
+    return rows <= 3 and K <= 4096 and (K > 1024 or N < 32768)
+
+
+def _long_rows(rows: int, N: int, K: int) -> bool:
+    """24 to 192 rows of a W of few long rows, whose tiles fill the chip only in
+    ranges of K. us, in-house / library: 4096 x 14336 with 24 rows 28.5 / 28.7,
+    64 31.7 / 39.0, 128 38.6 / 74.0, 192 44.5 / 101; 2560 x 10240 with 40 20.4 /
+    20.3, 112 25.4 / 34.2; 8192 x 28672 with 72 107 / 189; 2048 x 16384 with 40
+    22.0 / 26.7. Past the lines 6144 x 12288 with 20 36.3 / 34.5, 4096 x 11008
+    with 208 49.8 / 45.5, 1024 x 10240 with 80 19.9 / 18.2, 10240 x 8192 with 64
+    42.6 / 41.4, 4096 x 8192 with 160 31.6 / 32.3 (128 rows 29 / 32)."""
+    return 24 <= rows <= 192 and 2048 <= N <= 8192 and K >= 10240
+
+
 def _choose(x: torch.Tensor, w: torch.Tensor) -> int:
     """0: the library, 1: skinny, 2: 8-phase."""
     if not x.is_cuda or x.dtype != torch.bfloat16:
         return 0
-    impl = _POLICY.get((x.shape[0], w.shape[0], w.shape[1]))
-    return int(_few_rows(x, w)) if impl is None else impl
+    shape = (x.shape[0], w.shape[0], w.shape[1])
+    impl = _POLICY.get(shape)
+    if impl is None:  # untuned
+        impl = int((_few_rows(*shape) or _long_rows(*shape)) and _fits(x, w))
+    return impl
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -925,6 +925,44 @@ def test_skinny_gemm_split_ranges(m, n, k):
         assert err < 2 ** -7, err
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (17, 64, 64), (32, 192, 192), (33, 128, 832), (64, 2112, 576),
+    (65, 256, 640), (128, 128, 12864), (129, 320, 64), (192, 384, 1088),
+    (193, 128, 704), (256, 192, 2112), (16, 33024, 192)])
+def test_skinny_gemm_tiles(M, N, K):
+    """Row counts at and past each tile count, one and two tiles of W a wave,
+    ranges of one chunk, of odd numbers of chunks and of several rounds; x with
+    a row stride and not-a-numbers behind its last row."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    buf = torch.randn(M + 1, K + 8, generator=g, device="cuda").to(
+        torch.bfloat16)
+    buf[M:] = float("nan")
+    buf[:, K:] = float("nan")
+    w = torch.randn(N, K, generator=g, device="cuda").to(torch.bfloat16)
+    got = ops.skinny_gemm(buf[:M, :K], w).double()
+    want = buf[:M, :K].double() @ w.double().t()
+    # one bf16 rounding (2^-9) of an fp32 sum of K products of size 1
+    assert ((got - want).abs() <= want.abs() / 256 + 1e-3 * K ** 0.5 / 8).all()
+
+
+@pytest.mark.parametrize("M,N,K,own", [
+    (23, 2048, 10240, False), (24, 2048, 10240, True),
+    (192, 8192, 10240, True), (193, 2048, 10240, False),
+    (64, 1984, 10240, False), (64, 2048, 10176, False)])
+def test_linear_long_rows(M, N, K, own):
+    """Which untuned products go to the in-house kernel, on either side of
+    each line."""
+    from production_stack_amd.ops import gemm_policy
+
+    gemm_policy.reset()
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    w = torch.randn(N, K, device="cuda").to(torch.bfloat16)
+    assert gemm_policy._choose(x, w) == own
+    assert gemm_policy._choose(x[:, 8:], w[:, 8:]) == 0  # not contiguous
+    want = ops.skinny_gemm(x, w) if own else torch.nn.functional.linear(x, w)
+    assert torch.equal(gemm_policy.linear(x, w), want)
+
+
 def test_skinny_gemm_nothing_to_do():
     """No columns of K are refused for any number of rows, no rows give no
     rows, also where they are a view of a wider matrix."""
