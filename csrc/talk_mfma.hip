@@ -30,8 +30,8 @@
 // of a SIMD's matrix unit, 1024 of them the scores, 2048 the mix, 1536 the
 // output, and 14200 in all: with one workgroup a CU (its LDS) the four barriers
 // between those stages leave the matrix unit waiting. 32/8 heads of 128, 4099
-// rows in two prompts, chunks of 2048: 0.63 ms (11.7 before; 0.65 with a branch
-// around every exponential).
+// rows in two prompts, chunks of 2048: 0.42 ms (11.7 before; 0.63 with the blocks
+// of rows from last to first).
 #include "attn_common.h"
 #include "scan_common.h"
 
@@ -73,6 +73,65 @@ struct TmArgs {
 // A bf16 entry that is an infinity or no number.
 PS_DEV bool tm_odd(unsigned int e) { return (e & 0x7f80u) == 0x7f80u; }
 
+// First row of the workgroups' `rank`-th block of 16: those that see the most
+// keys first, so that the CUs end together. Blocks are one or two a CU and see
+// anything from one to all keys of a chunk; from the last row to the first, a
+// second sequence's longest ones started when others were done (4099 rows of
+// two sequences, chunks of 2048: 632 us, 421 by length). Every wave finds the
+// same: the count of keys that `rank` blocks are above, by halves, then the block
+// among those of that count. Up to 128 blocks all start at once.
+PS_DEV int tm_first_row(const TmArgs& a, int rank, int blocks) {
+  constexpr int PER = 16;
+  if (blocks <= 128 || blocks > 64 * PER) return (blocks - 1 - rank) * 16;
+  const int lane = threadIdx.x & 63;
+  int keys[PER], top = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int b = k * 64 + lane;
+    keys[k] = -1;
+    if (k * 64 < blocks) {
+      const int first = a.token_pos[min(b * 16, a.T - 1)];
+      const int last = a.token_pos[min(b * 16 + 15, a.T - 1)];
+      int low = 0;
+      if (a.chunk > 0) low = first / a.chunk * a.chunk;
+      if (a.window > 0) low = max(low, first - a.window + 1);
+      // of two sequences: to the end of one and from the other's start
+      const int see = last >= first ? last - low : first - low + last;
+      keys[k] = b < blocks ? min(max(see, 0), 0xffffff) : -1;
+      top = max(top, keys[k]);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    top = max(top, __shfl_xor(top, off, 64));
+  // largest v that more than `rank` blocks have at least
+  int v = 0;
+  for (int bit = 31 - __clz(top | 1); bit >= 0; --bit) {
+    const int at = v | 1 << bit;
+    int count = 0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      if (k * 64 < blocks) count += __popcll(__ballot(keys[k] >= at));
+    if (count > rank) v = at;
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+    if (k * 64 < blocks) rank -= __popcll(__ballot(keys[k] > v));
+  int block = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    if (k * 64 < blocks) {
+      const unsigned long long same = __ballot(keys[k] == v);
+      const bool mine =
+          keys[k] == v && __popcll(same & ((1ull << lane) - 1)) == rank;
+      const unsigned long long hit = __ballot(mine);
+      if (hit) block = k * 64 + __ffsll(hit) - 1;
+      rank -= __popcll(same);  // below zero behind the hit: no more
+    }
+  }
+  return block * 16;
+}
+
 // ND = D / 32, NV = DV / 16; CAP: with a score cap
 template <int ND, int NV, bool CAP>
 __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
@@ -92,14 +151,19 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, n = lane & 15;
-  const int hb = blockIdx.y;  // output heads 16 hb ..
+  // the two halves of the output heads (16 hb ..) of a block eight apart: they
+  // share an XCD's L2
+  const int blocks = (a.T + 15) / 16;
+  const int hb = blockIdx.x >> 3 & 1;
+  const int rank = (blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
+  if (rank >= blocks) return;
   const int rep = TM_H / a.G;
   const int grp = wave * 4 / rep;                     // KV head of the scores
   const int vgrp = (16 * hb + (wave >> 1) * 4) / rep;  // and of the output
   sV += (wave >> 1) * TM_KT * PV;  // two waves' values, half a tile from each
 
-  // rows that see the most keys first
-  const int tok0 = (gridDim.x - 1 - blockIdx.x) * 16;
+  const int tok0 =
+      __builtin_amdgcn_readfirstlane(tm_first_row(a, rank, blocks));
   const int ntok = min(16, a.T - tok0);
   if (threadIdx.x < 16) {
     const int t = tok0 + min((int)threadIdx.x, ntok - 1);
@@ -404,8 +468,9 @@ static int tm_launch_as(const TmArgs& a, hipStream_t stream) {
     (void)hipGetLastError();
     return 1;
   }
-  hipLaunchKernelGGL((talk_mfma_kernel<ND, NV, CAP>), dim3((a.T + 15) / 16, 2),
-                     dim3(512), lds, stream, a);
+  // 16 workgroups for eight blocks of rows
+  hipLaunchKernelGGL((talk_mfma_kernel<ND, NV, CAP>),
+                     dim3((a.T + 127) / 128 * 16), dim3(512), lds, stream, a);
   return 0;
 }
 

@@ -390,6 +390,43 @@ def test_talk_attention_matrix_cores(G, D, DV, chunk, window, softcap,
     assert (out[:, H * DV:] == 7.0).all()
 
 
+@pytest.mark.parametrize("lens,chunk,window", [
+    ([2040], 0, 0),                  # 128 blocks: as they come
+    ([1500, 549], 512, 0),           # 129 by length, one of two sequences
+    ([700] * 4, 0, 96),              # equal counts
+    ([4099, 1000, 3], 64, 0)])       # 319, chunks of a few blocks
+def test_talk_attention_block_order(lens, chunk, window):
+    """Blocks of rows start by the keys they see: every row is written once,
+    and as a launch over its own sequence alone writes it."""
+    G, D, bs = 8, 64, 16
+    T = sum(lens)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    per = [-(-n // bs) for n in lens]
+    kc, vc = (torch.randn(sum(per), G, bs, D, generator=g, device="cuda").to(
+        torch.bfloat16) for _ in range(2))
+    q = torch.randn(T, 32 * D, generator=g, device="cuda").to(torch.bfloat16)
+    talk = torch.randn(32, 32, generator=g, device="cuda") * 0.2
+    tables = torch.zeros(len(lens), max(per), dtype=torch.int32)
+    for i, n in enumerate(per):
+        tables[i, :n] = sum(per[:i]) + torch.arange(n)
+    ts = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens))
+    tp = torch.cat([torch.arange(n) for n in lens])
+    tables, ts, tp = (x.int().cuda() for x in (tables, ts, tp))
+
+    def run(a, b):
+        out = torch.full((b - a, 32 * D), 7.0, device="cuda").to(
+            torch.bfloat16)
+        return ops.talk_attention(q[a:b], kc, vc, tables, ts[a:b], tp[a:b],
+                                  D ** -0.5, 32, chunk=chunk, window=window,
+                                  sink=True, talk=talk, out=out, variant=0)
+
+    got, at = run(0, T), 0
+    for n in lens:
+        # bf16 rounding where blocks of 16 begin elsewhere: other tiles of keys
+        assert _rel(got[at:at + n].float(), run(at, at + n).float()) < 3e-3
+        at += n
+
+
 @pytest.mark.parametrize("H,G,D,DV,window,keep,softcap,sink", [
     (8, 2, 128, 128, 0, 0, 0.0, None), (32, 4, 64, 64, 70, 3, 20.0, "zero"),
     (6, 2, 96, 40, 33, 64, 0.0, "heads"), (24, 1, 40, 128, 64, 66, 9.0, None),
