@@ -499,8 +499,14 @@ PS_DEV ck_f32x4 ck_token_terms(float f, float x, ck_f32x4 acc, int lane,
   return acc;
 }
 
+// Row tiles of 16 that a wave has: one up to 64 rows. us, one / two: general
+// delta, 8 heads of 64 x 64, 8000 rows in 2 prompts 296 / 386, 32 heads, 5000 in
+// 4 252 / 290, of 32 x 32 201 / 235; of 96 x 96 452 / 414, of 128 x 128 581 / 462
+// (twice the waves for as many instructions beside the products).
+static constexpr int ck_row_tiles(int dp) { return dp <= 64 ? 1 : 2; }
+
 // Walks the chunks of one (segment, head) for 16 columns of its state: a wave
-// per 32 rows of it, DP / 32 waves. raw [T, H * DV]: S^T r before the
+// per 32 rows of it (16 of up to 64), two to four waves. raw [T, H * DV]: S^T r before the
 // read-out's norm.
 //
 // The chain from one chunk to the next is what bounds this kernel: a prompt
@@ -517,7 +523,8 @@ PS_DEV ck_f32x4 ck_token_terms(float f, float x, ck_f32x4 acc, int lane,
 // segment: no branches in a chunk, and what lies outside reads as zero.
 // Measured (general delta, 128 x 128, one prompt of 336 chunks): 2.13 us a
 // chunk with operands through LDS and 32 columns a workgroup, 1.05 now, of
-// which the products take 0.5.
+// which the products take 0.5; 8 heads, 8000 rows in 2 prompts 698 -> 410 us, 32
+// heads 935 -> 723.
 // Workgroups of one head are H apart, so that they share an XCD's L2 where
 // that is a multiple of 8.
 //
@@ -528,14 +535,19 @@ PS_DEV ck_f32x4 ck_token_terms(float f, float x, ck_f32x4 acc, int lane,
 // the last run's record takes the state before the segment). The second starts
 // each run from what the runs before it leave and writes the outputs.
 template <typename T, int MODE, int DP, int PART>
-__global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
+__global__ __launch_bounds__(DP * 4 / ck_row_tiles(DP),
+                             sizeof(T) == 2 ? 3 : 2) void ck_sweep_kernel(
     float* __restrict__ raw, const float* __restrict__ items, int cap,
     const T* __restrict__ v, int ldv, float* __restrict__ state,
     const int* __restrict__ seq_rows, int S_, int H, int D, int DV, int base,
     float* __restrict__ part, int parts) {
   typedef CkItem<MODE, DP> It;
-  constexpr int NW = DP / 32;          // waves
+  constexpr int RT = ck_row_tiles(DP);   // row tiles of a wave
+  constexpr int NW = DP / 16 / RT;       // waves
   constexpr int NQ = (4 + NW - 1) / NW;  // tokens of four a wave takes
+  // three waves have two tokens' matrix entries each, and three a SIMD would
+  // spill with the written rows on their own and the last chunk's shares early
+  constexpr bool LEAN = NW == 3;
   constexpr int SET = NW * 64;         // shares of one chunk, float4
   __shared__ ck_f32x4 zx[2 * SET], ox[2 * SET];
   __shared__ float tmps[NW * 128];
@@ -584,13 +596,15 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
   const int j = cb * 16 + m16;  // this lane's column
   const bool col = j < DV;
   // row i of row tile t of the state
-  auto row = [&](int t, int i) { return 32 * wave + 16 * t + 4 * g + i; };
+  auto row = [&](int t, int i) {
+    return 16 * (RT * wave + t) + 4 * g + i;
+  };
   float* Sg = state + ((size_t)slot * H + hd) * (size_t)D * DV;
-  ck_f32x4 S[2];
+  ck_f32x4 S[RT];
   const size_t rec = (size_t)D * DV + DP;  // of one run
   float* pt = PART ? part + (size_t)sh * parts * rec : nullptr;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < RT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int d = row(t, i);
@@ -611,7 +625,7 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
 #pragma unroll 2
     for (int q = 0; q < run; ++q)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < RT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int d = row(t, i);
@@ -621,17 +635,21 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
         }
   }
   // product of the decays over the run, this wave's rows
-  ck_f32x4 decay[2] = {{1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}};
+  ck_f32x4 decay[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) decay[t] = {1.f, 1.f, 1.f, 1.f};
 
   // Operands through buffers, too: a uniform base, a uniform offset and a
   // 32-bit one per lane, so that a load is one instruction. `next` is the chunk
   // to fetch (the last one again behind it).
   const char* next = (const char*)(items + ((size_t)first * H + hd) * It::TOTAL);
   const size_t step = (size_t)H * It::TOTAL * sizeof(float);
-  const unsigned at_row0 = ck_row_slot(2 * wave, g, m16) * 16;
-  const unsigned at_row1 = ck_row_slot(2 * wave + 1, g, m16) * 16;
-  const unsigned at_col = ck_col_slot(2 * wave, g, m16) * 16;
-  const unsigned at_gam = (32 * wave + 4 * g) * 4;
+  unsigned at_row[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+    at_row[t] = ck_row_slot(RT * wave + t, g, m16) * 16;
+  const unsigned at_col = ck_col_slot(RT * wave, g, m16) * 16;
+  const unsigned at_gam = (16 * RT * wave + 4 * g) * 4;
   const unsigned at_sq = (lane * 4 + wave) * 4;
   auto operands = [&] {
     return __builtin_amdgcn_make_buffer_rsrc((void*)next, 0, It::TOTAL * 4,
@@ -666,25 +684,25 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
 
   // operands of a chunk: what meets the state before it, and what is written
   struct Reads {
-    ck_f32x4 r[2], u[2];
+    ck_f32x4 r[RT], u[RT];
     float cx[NQ], mx[NQ];  // this wave's tokens of the matrices on V
     T v[4];                // as loaded: a conversion here would wait for them
     float flag;
   };
   struct Writes {
-    ck_f32x4 k[2], b[2], gam[2];
+    ck_f32x4 k[RT], b[RT], gam[RT];
     float zx[NQ];  // this wave's tokens of the matrix on Z (Y)
   };
   constexpr int LASTSQ = MODE == CK_GD ? It::MB : It::M;
   auto fetch_reads = [&](int c, Reads& x) {
     const auto p = operands();
     if constexpr (MODE != CK_GLA) {
-      x.u[0] = load4(p, at_row0, It::U);
-      x.u[1] = load4(p, at_row1, It::U);
+#pragma unroll
+      for (int t = 0; t < RT; ++t) x.u[t] = load4(p, at_row[t], It::U);
     }
     if constexpr (PART != 1) {
-      x.r[0] = load4(p, at_row0, It::R);
-      x.r[1] = load4(p, at_row1, It::R);
+#pragma unroll
+      for (int t = 0; t < RT; ++t) x.r[t] = load4(p, at_row[t], It::R);
       x.flag = ((const float*)next)[It::FLAG];
     }
 #pragma unroll
@@ -707,7 +725,7 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
   auto fetch_writes = [&](int c, Writes& x) {
     const auto p = operands();
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < RT; ++t) {
       x.gam[t] = load4(p, at_gam, It::GAM + t * 16);
       x.k[t] = load4(p, at_col, It::K + t * 256);
       if constexpr (MODE == CK_GD) x.b[t] = load4(p, at_col, It::B + t * 256);
@@ -757,7 +775,9 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
     // the written rows (L) too, so that the larger sums are added last (the
     // state's error against 64 bits is 5.6e-8 so, 7.7e-8 with K V on the state
     // before B Z)
-    ck_f32x4 V, Z[2] = {zero, zero}, O[2] = {zero, zero}, L[2] = {zero, zero};
+    ck_f32x4 V, Z[2] = {zero, zero}, O[2] = {zero, zero}, L[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) L[t] = zero;
 #pragma unroll
     for (int i = 0; i < 4; ++i) V[i] = MxElem<T>::ld(&rd.v[i]);
     // the same in every wave: all have all of V
@@ -776,12 +796,13 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
     auto on_tokens = [&](const float (&f)[NQ], const ck_f32x4& x,
                          ck_f32x4& acc) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q)
-        if (4 % NW == 0 || wave + q * NW < 4)
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              __uint_as_float(__float_as_uint(f[q]) & mask),
-              __uint_as_float(__float_as_uint(pick(x, q)) & mask), acc, 0, 0,
-              0);
+      for (int q = 0; q < NQ; ++q) {
+        // three waves: the fourth token is the first wave's; no branch
+        const unsigned mq = 4 % NW == 0 || wave + q * NW < 4 ? mask : 0;
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            __uint_as_float(__float_as_uint(f[q]) & mq),
+            __uint_as_float(__float_as_uint(pick(x, q)) & mq), acc, 0, 0, 0);
+      }
     };
     // The same term by term, zeros above the diagonal left out: beside a value
     // that is no finite number they would reach earlier tokens. No loads here:
@@ -801,7 +822,7 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
     if constexpr (MODE != CK_GLA) {
       on_tokens(rd.cx, V, Z[1]);
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < RT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           // channel: Y = C V - U S
@@ -812,7 +833,7 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
     if constexpr (PART != 1) {
       if constexpr (MODE != CK_CD) on_tokens(rd.mx, V, O[1]);
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < RT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           O[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(rd.r[t][i], S[t][i],
@@ -835,21 +856,22 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
 #pragma unroll
       for (int w = 0; w < NW; ++w) zr[w] = zs[w * 64 + lane];
     }
-    if constexpr (PART != 1) shares_of(c - 1, so);
+    if constexpr (PART != 1 && !LEAN) shares_of(c - 1, so);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < RT; ++t) {
       S[t] *= wr.gam[t];
       if constexpr (PART == 1) decay[t] *= wr.gam[t];
     }
-    if constexpr (MODE == CK_GD) {
+    auto written = [&](ck_f32x4(&acc)[RT]) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-          L[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr.k[t][i], V[i], L[t],
-                                                      0, 0, 0);
-    }
+        for (int t = 0; t < RT; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr.k[t][i], V[i],
+                                                        acc[t], 0, 0, 0);
+    };
+    if constexpr (MODE == CK_GD && !LEAN) written(L);
     ck_f32x4 Y = V;
     if constexpr (MODE != CK_GLA) {
       Y = NW > 1 ? zr[0] : Z[0] + Z[1];
@@ -860,13 +882,14 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < RT; ++t)
         S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
             MODE == CK_GD ? wr.b[t][i] : wr.k[t][i], Y[i], S[t], 0, 0, 0);
-    if constexpr (MODE == CK_GD) {
-      S[0] += L[0];
-      S[1] += L[1];
+    if constexpr (MODE == CK_GD && !LEAN) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t) S[t] += L[t];
     }
+    if constexpr (MODE == CK_GD && LEAN) written(S);
     if constexpr (MODE != CK_GLA) {
       on_tokens(wr.zx, Y, O[1]);
       __builtin_amdgcn_sched_barrier(0);
@@ -874,6 +897,7 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
     }
     fetch_writes(c + 2, wr);
     if constexpr (PART != 1) {
+      if constexpr (LEAN) shares_of(c - 1, so);
       emit(c - 1, so);
       ox[(c & 1) * SET + wave * 64 + lane] = O[0] + O[1];
     }
@@ -908,7 +932,7 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
     Se = pt + run * rec;
     if (cb == 0 && m16 == 0) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < RT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           Se[(size_t)D * DV + row(t, i)] = decay[t][i];
@@ -916,7 +940,7 @@ __global__ __launch_bounds__(DP * 2, 2) void ck_sweep_kernel(
   }
   if (col && (PART != 2 || last)) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < RT; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (row(t, i) < D) Se[(size_t)row(t, i) * DV + j] = S[t][i];
@@ -2178,10 +2202,11 @@ static int ck_launch(CK_ARGS) {
                        D, scale, c0f, p * cap);
 #define CK_SWEEP(PART, RUNS)                                                 \
   hipLaunchKernelGGL((ck_sweep_kernel<T, MODE, DP, PART>),                   \
-                     dim3(S_ * H * ((DV + 15) / 16) * (RUNS)), dim3(DP * 2), \
-                     0, stream, raw, items, cap, (const T*)in.v, in.ldv,     \
-                     (float*)state, (const int*)seq_rows, S_, H, D, DV,      \
-                     p * cap, part, parts)
+                     dim3(S_ * H * ((DV + 15) / 16) * (RUNS)),               \
+                     dim3(DP * 4 / ck_row_tiles(DP)), 0, stream, raw, items, \
+                     cap, (const T*)in.v, in.ldv, (float*)state,             \
+                     (const int*)seq_rows, S_, H, D, DV, p * cap, part,      \
+                     parts)
     if constexpr (MODE == CK_GLA) {
       if (parts > 1) {
         CK_SWEEP(1, parts - 1);
