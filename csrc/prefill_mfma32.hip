@@ -248,7 +248,7 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
       const bool grew = (m_new > m_run + PS_RESCALE_THR32) ||
                         (m_run == PS_NEG_INF && m_new > PS_NEG_INF);
       if (__any(grew)) {
-        const float corr = exp2f(m_run - m_new);
+        const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
         l_run *= corr;
         m_run = m_new;
         // broadcast corr from the owner lane of each accumulator row
@@ -260,14 +260,21 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
           for (int dt = 0; dt < 4; dt++) o_acc[dt][r] *= c;
         }
       }
+      // Hidden keys, and scores that are no number, have the lowest score and
+      // so a weight of 0, also while nothing is visible (the row's maximum is
+      // then the lowest score itself). Weights below 2^-126 are 0: without the
+      // library function's care for them, and with the hardware's conversion
+      // below, a chunk takes 340 vector instructions a wave for 670.
+      const float m_sub = m_run > PS_NEG_INF ? m_run : 0.f;
       float psum = 0.f;
 #pragma unroll
       for (int kt = 0; kt < 2; kt++) {
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-          const float p = s_frag[kt][r] > PS_NEG_INF
-                              ? exp2f(s_frag[kt][r] - m_run)
-                              : 0.f;
+          // the middle one of the three is the lowest where s is no number
+          const float p = __builtin_amdgcn_exp2f(
+              __builtin_amdgcn_fmed3f(s_frag[kt][r], PS_NEG_INF, INFINITY) -
+              m_sub);
           s_frag[kt][r] = p;
           psum += p;
         }
