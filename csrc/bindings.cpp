@@ -274,7 +274,8 @@ void paged_attn_prefill_mfma(at::Tensor out, at::Tensor q,
     if (splits > 1) {
       ws_o = at::empty({(long)splits * T * QH * HD},
                        q.options().dtype(at::kFloat));
-      ws_ml = at::empty({2L * splits * T * QH},
+      // maxima, denominators, and how many splits a row has
+      ws_ml = at::empty({2L * splits * T * QH + T},
                         q.options().dtype(at::kFloat));
       ws_o_p = ws_o.data_ptr();
       ws_ml_p = ws_ml.data_ptr();

@@ -35,23 +35,70 @@ PS_DEV ps_mbf16x8 ps_as_mbf16_32(ps_bf16x8 u) {
 #define PS_CHUNK32 64    // KV tokens per chunk (4 pages)
 #define PS_TILE32 256    // q rows per workgroup (8 waves x 32)
 
+// The `idx`-th of all tiles' splits, longest first (tile -1: there are fewer).
+// `heads`: workgroups of a tile beside its splits. Every wave finds the same.
+PS_DEV void ps_tile_split(const int* tile_info, int n_tiles, int heads,
+                          int max_splits, int idx, int lane, int* tile,
+                          int* split, int* n_splits) {
+  auto chunks_of = [&](int i) {
+    return (tile_info[i * 4 + 2] + tile_info[i * 4 + 3] + PS_CHUNK32 - 1) /
+           PS_CHUNK32;
+  };
+  int all = 0;
+  for (int i = lane; i < n_tiles; i += 64) all += chunks_of(i);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) all += __shfl_xor(all, off);
+  const int share = max(1, (all * heads + 511) / 512);
+  *tile = -1;
+  if (n_tiles <= 64) {
+    const int c = lane < n_tiles ? chunks_of(lane) : 0;
+    const int s = lane < n_tiles
+                      ? max(1, min(max_splits, (c + share - 1) / share)) : 0;
+    const int len = s > 0 ? (c + s - 1) / s : -1;
+    int before = 0;  // splits of the tiles ahead of this lane's
+    for (int i = 0; i < n_tiles; ++i) {
+      const int li = __builtin_amdgcn_readlane(len, i);
+      const int si = __builtin_amdgcn_readlane(s, i);
+      before += li > len || (li == len && i < lane) ? si : 0;
+    }
+    const unsigned long long hit =
+        __ballot(s > 0 && idx >= before && idx < before + s);
+    if (hit == 0) return;
+    const int l = __ffsll(hit) - 1;
+    *tile = l;
+    *split = idx - __builtin_amdgcn_readlane(before, l);
+    *n_splits = __builtin_amdgcn_readlane(s, l);
+  } else {  // as they come
+    const int i = idx / max_splits;
+    const int s =
+        max(1, min(max_splits, (chunks_of(i) + share - 1) / share));
+    if (idx % max_splits >= s) return;
+    *tile = i;
+    *split = idx % max_splits;
+    *n_splits = s;
+  }
+}
+
 // tile_info: int4 per tile = (seq_row, q_token_start, q_pos_start, n_rows)
 // GQW = GQA q-heads processed per workgroup: the 8 waves split into
 // GQW head-columns x (8/GQW) row-halves, so all GQW heads of a kv-head
 // share ONE K/V staging pass (serving-shape prefill chunks are
 // staging-bound: a 200-row continuation re-reads a 2000+-token context).
 // Tile rows = 32 * (8/GQW).
-// Split-KV (gridDim.y > 1): split s processes kv chunks s, s+S, s+2S...
-// and writes UNNORMALIZED partials (o_acc, m, l) to the workspace; the
-// combine kernel merges them. Strided chunk assignment balances the
-// causal tail across splits. Raises the workgroup count for small
-// serving launches (1-block/CU quantization measured ~25% idle at the
-// 10-seq continuation shape).
+// Split-KV (max_splits > 1): split s of a tile's S processes kv chunks s, s+S,
+// s+2S... and writes UNNORMALIZED partials (o_acc, m, l) to the workspace; the
+// combine kernel merges them. Strided chunk assignment balances the causal
+// tail across splits. A tile has as many splits as it has shares of what two
+// workgroups a CU do on average, up to max_splits, a tile of one share writes
+// its rows itself, and the longest workgroups start first. Three splits for
+// every tile had the continuations of prompts behind 3700 keys take turns of 21
+// chunks beside fresh prompts of two or three (29 tiles of 8 KV heads: 160 us
+// and 35 of merging, 128 and 14 now).
 template <int HEAD_DIM, int GQW, typename KVT>
 __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
     unsigned short* __restrict__ out,            // [T, QH, HD]
     float* __restrict__ ws_o,    // [S, T, QH, HD] (splits > 1)
-    float* __restrict__ ws_ml,   // [2, S, T, QH]
+    float* __restrict__ ws_ml,   // [2, S, T, QH], then int [T]: a row's splits
     long q_tokens,
     const unsigned short* __restrict__ q,        // [T, QH, HD]
     const KVT* __restrict__ k_cache,             // [NB, KH, 16, HD]
@@ -59,9 +106,7 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
     const int* __restrict__ block_tables,  // [S, max_blocks]
     const int* __restrict__ tile_info,     // [NT, 4]
     int max_blocks, float scale, int KH, int GQ, long q_stride,
-    int QH, int n_work, int window) {
-  const int split = blockIdx.y;
-  const int n_splits = gridDim.y;
+    int QH, int n_work, int window, int max_splits) {
   using KVTr = ps_kv_traits<KVT>;
   using kvec8 = typename KVTr::vec8;
   using kvec4 = typename KVTr::vec4;
@@ -70,24 +115,34 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
   constexpr int NKS = D / 16;   // QK k-steps over head dim (8)
   constexpr int ROWH = 8 / GQW; // row-halves (32 rows each) per tile
 
-  // T1 XCD swizzle (same scheme as v3/v4): contiguous work chunks per XCD
-  const int W = n_work;  // n_tiles * KH * (GQ/GQW)
-  const int cpx = (W + 7) >> 3;
-  const int w = (blockIdx.x & 7) * cpx + (blockIdx.x >> 3);
-  if (w >= W) return;
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6;
+  const int lane = tid & 63;
   const int n_grp = GQ / GQW;
-  const int n_tiles = W / (n_grp * KH);
-  const int tile = w % n_tiles;
-  const int g_grp = (w / n_tiles) % n_grp;
-  const int kvh = w / (n_tiles * n_grp);
+  const int n_tiles = n_work / (n_grp * KH);
+  int tile, g_grp, kvh, split = 0, n_splits = 1;
+  if (max_splits > 1) {
+    // a KV head's workgroups eight (or a divisor) apart: one XCD's L2
+    kvh = blockIdx.x % KH;
+    g_grp = blockIdx.x / KH % n_grp;
+    ps_tile_split(tile_info, n_tiles, KH * n_grp, max_splits,
+                  blockIdx.x / (KH * n_grp), lane, &tile, &split, &n_splits);
+    if (tile < 0) return;
+  } else {
+    // T1 XCD swizzle (same scheme as v3/v4): contiguous work chunks per XCD
+    const int W = n_work;  // n_tiles * KH * (GQ/GQW)
+    const int cpx = (W + 7) >> 3;
+    const int w = (blockIdx.x & 7) * cpx + (blockIdx.x >> 3);
+    if (w >= W) return;
+    tile = w % n_tiles;
+    g_grp = (w / n_tiles) % n_grp;
+    kvh = w / (n_tiles * n_grp);
+  }
   const int seq_row = tile_info[tile * 4 + 0];
   const int q_tok0 = tile_info[tile * 4 + 1];
   const int q_pos0 = tile_info[tile * 4 + 2];
   const int n_rows = tile_info[tile * 4 + 3];
 
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
   const int hi = lane >> 5;   // half-wave
   const int rc = lane & 31;   // q row (B/D col) or kv row (A row)
   // wave -> (head column, row half)
@@ -98,6 +153,8 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
   const int ctx_limit = q_pos0 + n_rows;
   const int n_pages = (ctx_limit + BS - 1) / BS;
   const int n_chunks = (ctx_limit + PS_CHUNK32 - 1) / PS_CHUNK32;
+  if (max_splits > 1 && split == 0 && kvh == 0 && g_grp == 0 && tid < n_rows)
+    ((int*)(ws_ml + 2l * max_splits * q_tokens * QH))[q_tok0 + tid] = n_splits;
 
   __shared__ __align__(16) unsigned short k_lds[PS_CHUNK32][D];
   __shared__ __align__(16) unsigned short v_t[D][PS_CHUNK32];
@@ -324,7 +381,7 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
     if (hi == 0 && wq0 + rc < n_rows) {
       const long t = q_tok0 + wq0 + rc;
       ws_ml[((long)split * q_tokens + t) * QH + qh] = m_run;
-      ws_ml[((long)(n_splits + split) * q_tokens + t) * QH + qh] = l_run;
+      ws_ml[((long)(max_splits + split) * q_tokens + t) * QH + qh] = l_run;
     }
 #pragma unroll
     for (int r = 0; r < 16; r++) {
@@ -355,39 +412,53 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
   }
 }
 
-// merge the splits: out = sum_s w_s O_s / sum_s w_s l_s, w_s=exp2(m_s-M)
-__global__ void prefill_split_combine_kernel(
+// merge the splits: out = sum_s w_s O_s / sum_s w_s l_s, w_s=exp2(m_s-M).
+// 32 lanes a (row, head), eight of them a workgroup; rows of one split are
+// written already.
+__global__ __launch_bounds__(256) void prefill_split_combine_kernel(
     unsigned short* __restrict__ out,      // [T, QH, 128]
     const float* __restrict__ ws_o,        // [S, T, QH, 128]
-    const float* __restrict__ ws_ml,       // [2, S, T, QH]
-    long q_tokens, int QH, int n_splits) {
-  const long th = blockIdx.x;  // t * QH + qh
-  if (th >= q_tokens * QH) return;
-  const int d = threadIdx.x;
+    const float* __restrict__ ws_ml,       // [2, S, T, QH], [T]
+    long q_tokens, int QH, int max_splits) {
+  const long t = blockIdx.x;
+  const int qh = blockIdx.y * 8 + (threadIdx.x >> 5);
+  const int d = (threadIdx.x & 31) * 4;
+  // a row outside of every tile has no count
+  const int n_splits =
+      min(((const int*)(ws_ml + 2l * max_splits * q_tokens * QH))[t],
+          max_splits);
+  if (n_splits <= 1 || qh >= QH) return;
+  const long th = t * QH + qh;
   float M = PS_NEG_INF;
   for (int s = 0; s < n_splits; s++)
     M = fmaxf(M, ws_ml[(long)s * q_tokens * QH + th]);
-  float denom = 0.f, acc = 0.f;
+  float denom = 0.f;
+  ps_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int s = 0; s < n_splits; s++) {
     const float m = ws_ml[(long)s * q_tokens * QH + th];
-    const float l = ws_ml[((long)(n_splits + s) * q_tokens) * QH + th];
+    const float l = ws_ml[((long)(max_splits + s) * q_tokens) * QH + th];
     const float w = (m > PS_NEG_INF && l > 0.f) ? exp2f(m - M) : 0.f;
     denom += w * l;
-    acc += w * ws_o[((long)s * q_tokens * QH + th) * 128 + d];
+    acc += w * *(const ps_f32x4*)(ws_o +
+                                  ((long)s * q_tokens * QH + th) * 128 + d);
   }
-  out[th * 128 + d] =
-      ps_f32_to_bf16(denom > 0.f ? acc / denom : 0.f);
+  ps_bf16x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    o[i] = ps_f32_to_bf16(denom > 0.f ? acc[i] / denom : 0.f);
+  *(ps_bf16x4*)(out + th * 128 + d) = o;
 }
 
 extern "C" {
 
-// Split count the launcher will use for a shape (callers size ws with it)
+// Most splits of a tile (callers size ws with it): up to 500 tiles and heads,
+// enough for a few long tiles among short ones.
 int ps_prefill_mfma32_splits(int num_tiles, int KH, int GQ) {
   int gqw = 1;
   while (gqw < 4 && GQ % (gqw * 2) == 0) gqw *= 2;
   const int n_work = num_tiles * KH * (GQ / gqw);
   if (n_work >= 500) return 1;
-  int s = (500 + n_work - 1) / n_work;
+  int s = (1000 + n_work - 1) / n_work;
   return s > 8 ? 8 : s;
 }
 
@@ -409,7 +480,7 @@ int ps_paged_attn_prefill_mfma32(void* out, void* ws_o, void* ws_ml,
   const int n_work = num_tiles * KH * (GQ / gqw);
   int splits = ps_prefill_mfma32_splits(num_tiles, KH, GQ);
   if (ws_o == nullptr) splits = 1;
-  dim3 grid(((n_work + 7) / 8) * 8, splits);
+  dim3 grid(splits > 1 ? n_work * splits : (n_work + 7) / 8 * 8);
 #define PS_PF32_LAUNCH(GQW, KVT)                                          \
   paged_attn_prefill_mfma32_kernel<128, GQW, KVT>                         \
       <<<grid, 512, 0, stream>>>(                                         \
@@ -417,7 +488,7 @@ int ps_paged_attn_prefill_mfma32(void* out, void* ws_o, void* ws_ml,
           (const unsigned short*)q,                                       \
           (const KVT*)k_cache, (const KVT*)v_cache,                       \
           (const int*)block_tables, (const int*)tile_info, max_blocks,    \
-          scale, KH, GQ, q_stride, num_q_heads, n_work, window)
+          scale, KH, GQ, q_stride, num_q_heads, n_work, window, splits)
   if (kv_fp8) {
     if (gqw == 4) PS_PF32_LAUNCH(4, unsigned char);
     else if (gqw == 2) PS_PF32_LAUNCH(2, unsigned char);
@@ -430,7 +501,7 @@ int ps_paged_attn_prefill_mfma32(void* out, void* ws_o, void* ws_ml,
 #undef PS_PF32_LAUNCH
   if (splits > 1) {
     prefill_split_combine_kernel<<<
-        dim3((unsigned)(q_tokens * num_q_heads)), 128, 0, stream>>>(
+        dim3((unsigned)q_tokens, (num_q_heads + 7) / 8), 256, 0, stream>>>(
         (unsigned short*)out, (const float*)ws_o, (const float*)ws_ml,
         q_tokens, num_q_heads, splits);
   }

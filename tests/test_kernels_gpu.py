@@ -616,6 +616,34 @@ def test_prefill_mfma32_v5_vs_reference(qh, kh):
     _close(got, want)
 
 
+@pytest.mark.parametrize("qh,kh,chunks", [
+    (32, 8, [(0, 1950, 70), (1, 0, 3), (2, 0, 200), (3, 500, 64)]),
+    (40, 5, [(0, 0, 5), (1, 0, 1), (2, 1300, 130), (3, 63, 2)]),
+    (4, 1, [(i, 41 * (i % 9) ** 2, 1 + i % 3) for i in range(70)]),
+    (8, 2, [(i, 30 * i, 40) for i in range(64)])])
+def test_prefill_mfma32_uneven_tiles(qh, kh, chunks):
+    """Long tiles among short ones: several splits of some and one of others,
+    two head groups of a KV head, 64 tiles in order of their length and more
+    as they come; every row from its own sequence's keys."""
+    torch.manual_seed(43)
+    hd, bs, n = 128, 16, len(chunks)
+    blocks = max((a + b + bs - 1) // bs for _, a, b in chunks)
+    k_cache, v_cache = _make_cache(n * blocks + 1, kh, bs, hd)
+    tables = torch.arange(1, n * blocks + 1, dtype=torch.int32).reshape(
+        n, blocks)
+    tiles, token_seq, token_pos = _build_tiles(
+        chunks, tile=ops.prefill_tile_rows(qh, kh))
+    q = torch.randn((token_seq.shape[0], qh, hd), dtype=torch.bfloat16,
+                    device="cuda")
+    want = reference.paged_attn_prefill(
+        q.cpu(), k_cache.cpu(), v_cache.cpu(), tables, token_seq, token_pos,
+        1.0 / hd ** 0.5)
+    got = ops.paged_attn_prefill_mfma(
+        q, k_cache, v_cache, tables.cuda(), tiles.cuda(), 1.0 / hd ** 0.5,
+        variant=5)
+    _close(got, want)
+
+
 def test_prefill_mfma32_v5_matches_v3():
     torch.manual_seed(41)
     qh, kh, hd = 32, 8, 128
