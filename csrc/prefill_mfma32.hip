@@ -92,8 +92,8 @@ PS_DEV void ps_tile_split(const int* tile_info, int n_tiles, int heads,
 // workgroups a CU do on average, up to max_splits, a tile of one share writes
 // its rows itself, and the longest workgroups start first. Three splits for
 // every tile had the continuations of prompts behind 3700 keys take turns of 21
-// chunks beside fresh prompts of two or three (29 tiles of 8 KV heads: 160 us
-// and 35 of merging, 128 and 14 now).
+// chunks beside fresh prompts of two or three (29 tiles of 8 KV heads: 164 us
+// and 36 of merging, 127 and 13 now).
 template <int HEAD_DIM, int GQW, typename KVT>
 __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
     unsigned short* __restrict__ out,            // [T, QH, HD]
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
     ps_bf16x8 qs;
 #pragma unroll
     for (int j = 0; j < 8; j++)
-      qs[j] = ps_f32_to_bf16(ps_bf16_to_f32(qv[j]) * qmul);
+      qs[j] = ps_round_bf16(ps_bf16_to_f32(qv[j]) * qmul);
     q_frag[ks] = ps_as_mbf16_32(qs);
   }
 
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
           unsigned short p4[4];
 #pragma unroll
           for (int j = 0; j < 4; j++)
-            p4[j] = ps_f32_to_bf16(s_frag[kt][qd * 4 + j]);
+            p4[j] = ps_round_bf16(s_frag[kt][qd * 4 + j]);
           const int slot = (kt * 4 + qd) ^ (rc & 7);
           *(ps_bf16x4*)(&p_lds[wave][rc][slot * 8 + 4 * hi]) =
               *(const ps_bf16x4*)p4;
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(512, 2) void paged_attn_prefill_mfma32_kernel(
     unsigned short* orow = out + ((long)(q_tok0 + lrow) * QH + qh) * D;
 #pragma unroll
     for (int dt = 0; dt < 4; dt++)
-      orow[dt * 32 + rc] = ps_f32_to_bf16(o_acc[dt][r] * inv);
+      orow[dt * 32 + rc] = ps_round_bf16(o_acc[dt][r] * inv);
   }
 }
 
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(256) void prefill_split_combine_kernel(
   ps_bf16x4 o;
 #pragma unroll
   for (int i = 0; i < 4; i++)
-    o[i] = ps_f32_to_bf16(denom > 0.f ? acc[i] / denom : 0.f);
+    o[i] = ps_round_bf16(denom > 0.f ? acc[i] / denom : 0.f);
   *(ps_bf16x4*)(out + th * 128 + d) = o;
 }
 

@@ -25,9 +25,24 @@ PS_DEV float ps_bf16_to_f32(unsigned short u) {
   return v.f;
 }
 
-// Round to nearest even by the hardware's conversion, one instruction (six by
-// integer arithmetic: a fifth of the prompt attention's vector instructions).
 PS_DEV unsigned short ps_f32_to_bf16(float f) {
+  union {
+    float f;
+    unsigned int i;
+  } v;
+  v.f = f;
+  unsigned int x = v.i;
+  // round-to-nearest-even; NaN flushed to canonical quiet NaN
+  if ((x & 0x7fffffffu) > 0x7f800000u) return 0x7fc0;
+  unsigned int r = (x >> 16) & 1u;
+  x += 0x7fffu + r;
+  return (unsigned short)(x >> 16);
+}
+// The same by the hardware's conversion, one instruction for six: a fifth of the
+// prompt attention's vector instructions. Only where it was timed: in kernels that round a few results behind a long
+// loop it changes that loop's schedule (head-mix attention: prompts 421 us and
+// 440 with it, one token behind 609 keys 90 and 97).
+PS_DEV unsigned short ps_round_bf16(float f) {
   return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
 
