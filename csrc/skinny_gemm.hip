@@ -115,10 +115,10 @@ __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
 // the reads of x from LDS with many rows (each wave reads all of x: 16 NC rows of
 // W share a read). us, distinct weights, this / the form it replaces (a barrier
 // on each side of 64 columns, loads not ahead) / the library's kernel:
-//   4096 x 14336   64 rows 31 / 48 / 39, 128 rows 37 / 66 / 74, 192 43 / 83 / 106
-//   4096 x 4096    64 rows 14 / 22 / 14, 192 rows 23 / 39 / 31
-//   28672 x 4096   64 rows 56 / 96 / 52, 192 rows 71 / 150 / 61
-//   2048 x 8192    64 rows 14 / 25,      192 rows 23 / 39
+//   4096 x 14336   64 rows 32 / 48 / 40, 128 rows 39 / 65 / 74, 192 45 / 82 / 101
+//   4096 x 4096    64 rows 16 / 22 / 14, 192 rows 24 / 40 / 31
+//   28672 x 4096   64 rows 51 / 96 / 53, 192 rows 71 / 150 / 62
+//   2048 x 8192    64 rows 17 / 25 / 21, 192 rows 25 / 40 / 25
 // Waves split by rows of x as well read W twice: 10 to 40 % slower.
 template <int MT, int NC>
 __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
@@ -141,6 +141,18 @@ __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
   const int chunks = K / 64, per = (chunks + splits - 1) / splits;
   const int c0 = split * per, c1 = min(chunks, c0 + per);
   const int steps = (c1 - c0 + 1) / 2;
+  // Every tile begins at another step of its range: rows of W a power of two
+  // apart, read at the same columns by all workgroups, come from few channels of
+  // memory. us, all at the first step / this / the form before: 17 rows of
+  // 128256 x 4096 226 / 184 / 187, 128256 x 2048 116 / 102 / 129, 102400 x 8192
+  // 419 / 333 / 311; 24 rows of 28672 x 4096 57 / 47 / 73, 4096 x 4096 12.8 / 13.6 /
+  // 17.4.
+  const int tile = blockIdx.x / splits;
+  const int turn = steps > 0 ? (tile + tile / 8) % steps : 0;
+  auto place = [&](int t) {
+    const int s = min(t, steps - 1) + turn;
+    return max(s >= steps ? s - steps : s, 0);
+  };
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kg = wave >> 2, wn = wave & 3;  // half of a step, rows of W
@@ -153,7 +165,7 @@ __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
   ps_gbf16x8 wf[WD][NC][2];
   // steps past the end repeat the last chunk and are not multiplied
   auto load_w = [&](int u, int t) {
-    const int k = min(c0 + 2 * t + kg, c1 - 1) * 64;
+    const int k = min(c0 + 2 * place(t) + kg, c1 - 1) * 64;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -173,7 +185,8 @@ __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
     xd[i] = row * 128 + (xs ^ (row & 7)) * 8;
   }
   auto load_x = [&](int u, int t) {
-    const int k = min(c0 + 2 * t + (xs >> 3), c1 - 1) * 64 + (xs & 7) * 8;
+    const int k =
+        min(c0 + 2 * place(t) + (xs >> 3), c1 - 1) * 64 + (xs & 7) * 8;
 #pragma unroll
     for (int i = 0; i < XL; ++i) xf[u][i] = *(const ps_bf16x8*)(xp[i] + k);
   };
@@ -205,7 +218,7 @@ __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
         // the other buffer was read before the last barrier
         put_x((u + 1) & 1);
         load_x((u + 1) & 1, t + u + 3);
-        if (c0 + 2 * (t + u) + kg < c1) {
+        if (c0 + 2 * place(t + u) + kg < c1) {
 #pragma unroll
           for (int i = 0; i < MT; ++i) {
             const ps_gbf16x8 b0 = *(const ps_gbf16x8*)(buf + i * 2048 + xr0);
@@ -316,9 +329,8 @@ static PsSkinnyPlan ps_skinny_plan(int M, int N, int K) {
 
 // Whether the kernel without splits takes it; its byte offsets are 31 bits.
 // More than 8 rows reread x too often where the other form needs no splits
-// (N > 32768; us, this / split, distinct weights: 16 x 128256 x 4096 283 / 213,
-// 16 x 128256 x 2048 151 / 126, 16 x 51200 x 2560 82 / 79; 8 x 128256 x 4096 222 /
-// 236; with splits 16 x 28672 x 4096 68 / 71).
+// (N > 32768; us, this / the tiles, distinct weights: 16 x 128256 x 4096 283 / 183,
+// 16 x 128256 x 2048 151 / 101, 16 x 51200 x 2560 82 / 66).
 static bool ps_skinny_rows(int M, int N, int K, long x_stride) {
   return (M <= 8 || (M <= 16 && N <= 32768)) && x_stride >= 0 &&
          (M - 1) * x_stride + K < (1L << 30);
