@@ -1,6 +1,6 @@
-// Chunk-parallel form of the recurrences with a decay per key channel: whole
-// chunks of 16 tokens go through matrix products instead of one token at a
-// time. Per head the state S is a D x DV fp32 matrix and every token does
+// Chunk-parallel form of the recurrences: whole chunks of 16 tokens (32 in ssd
+// and mlstm of bf16 rows, at the wide kernels below) go through matrix products
+// instead of one token at a time. Per head the state S is a D x DV fp32 matrix and every token does
 //
 //   general delta  w = exp(-scale sigmoid(zw + w0)), a = sigmoid(za + ab),
 //                  u = k / sqrt(sum k^2 + 1e-6)
@@ -33,14 +33,16 @@
 // parallel kernel (one workgroup per chunk and head: the decays' products,
 // the 16 x 16 matrices, the triangular solve), and a second kernel walks the
 // chunks with the state in registers: a wave owns 16 columns of S as D / 16
-// accumulator tiles of v_mfma_f32_16x16x4_f32 (or shares its rows with others). The tiles' register layout (row
-// 4 g + i of a tile in lane group g, register i) is at once the layout of the
-// right operand of the products that read S when the left operand's columns
-// are taken in the order 4 g + i, so the state never leaves its registers; Z
-// and Y pass from one product into the next the same way.
+// accumulator tiles of v_mfma_f32_16x16x4_f32 (or shares its rows with others).
+// The tiles' register layout (row 4 g + i of a tile in lane group g, register i)
+// is at once the layout of the right operand of the products that read S when
+// the left operand's columns are taken in the order 4 g + i, so the state never
+// leaves its registers; Z and Y pass from one product into the next the same
+// way.
 //
 // Arithmetic is fp32 throughout (the matrix unit's fp32 products: fp32 inputs,
-// fp32 accumulation). Ratios W_t / W_s are formed from products counted from
+// fp32 accumulation; the chunks of 32 multiply bf16 rows as they are by fp32
+// numbers cut without loss into three bf16 terms). Ratios W_t / W_s are formed from products counted from
 // the middle of the chunk, so both factors stay in range while either half's
 // product is above 1e-30; chunks beyond that (or with decays that are no
 // numbers) form every ratio on its own.
@@ -2086,7 +2088,7 @@ static long ck_chunk_floats(int mode, int dp, int H, int G, int L) {
 //                                                            5.42 -> 0.55 ms
 //   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.31 ms
 //   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.07 ms
-//   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.84 ms
+//   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.51 ms
 // From 16 rows on a segment goes this way: one chunk costs about 15 us in
 // three launches, 16 tokens one by one 24 us.
 //
