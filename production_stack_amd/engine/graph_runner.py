@@ -16,7 +16,10 @@ state slot that no sequence owns.
 
 from __future__ import annotations
 
+import contextlib
+import gc
 import logging
+import threading
 from typing import Dict, List, Optional, Tuple
 
 import numpy as np
@@ -25,6 +28,29 @@ import torch
 from production_stack_amd.engine.models.llama import BatchMeta
 
 logger = logging.getLogger("engine.graphs")
+
+_CAPTURE = threading.RLock()
+
+
+@contextlib.contextmanager
+def _no_collection():
+    """No cyclic garbage is collected inside. A graph's destructor waits for the
+    device, which a capture that is open forbids: the error leaves a destructor
+    and ends the process. An engine in a reference cycle (a wrapped method is
+    enough) leaves its graphs to the collector, which runs whenever enough
+    objects were made, so what is garbage goes first and the collector rests
+    until the last capture has ended. One thread captures at a time: nobody
+    else wakes the collector before, or finds it off and leaves it so."""
+    with _CAPTURE:
+        gc.collect()
+        enabled = gc.isenabled()
+        gc.disable()
+        try:
+            yield
+        finally:
+            if enabled:
+                gc.enable()
+
 
 BUCKETS = [1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512]
 
@@ -106,10 +132,11 @@ class DecodeGraphRunner:
 
     @torch.no_grad()
     def capture_all(self) -> None:
-        torch.cuda.synchronize()
-        for b in reversed(self.buckets):  # big first: pool sized once
-            self._capture(b)
-        torch.cuda.synchronize()
+        with _no_collection():
+            torch.cuda.synchronize()
+            for b in reversed(self.buckets):  # big first: pool sized once
+                self._capture(b)
+            torch.cuda.synchronize()
         logger.info(
             "captured %d decode graphs (buckets %s)",
             len(self.graphs),

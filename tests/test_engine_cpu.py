@@ -732,3 +732,87 @@ def test_one_token_prompt_chunk_samples_nothing():
     big = make_engine(max_num_batched_tokens=256).generate(prompts, p)
     small = make_engine(max_num_batched_tokens=7).generate(prompts, p)
     assert big == small
+
+
+def test_no_graph_is_collected_during_a_capture(monkeypatch):
+    """Graphs of an engine in a reference cycle are left to the collector. On
+    the device their destructor waits, which ends the process inside a capture:
+    none may run there, nor when a capture fails; and the collector is as it
+    was afterwards."""
+    import contextlib
+    import gc
+
+    import pytest
+
+    from production_stack_amd.engine import graph_runner
+
+    now = dict(capturing=False, inside=0, gone=0)
+
+    class Graph:
+        def __del__(self):
+            now["gone"] += 1
+            now["inside"] += now["capturing"]
+
+        def pool(self):
+            return 1
+
+    @contextlib.contextmanager
+    def capture(g, pool=None):
+        now["capturing"] = True
+        try:
+            yield
+        finally:
+            now["capturing"] = False
+
+    class Stream:
+        def wait_stream(self, other):
+            pass
+
+    class Model:
+        fail = False
+
+        def __call__(self, tokens, meta, caches):
+            if now["capturing"] and gc.isenabled():  # as it may by itself
+                gc.collect()
+            if self.fail and now["capturing"]:
+                raise ValueError("refused")
+            return tokens
+
+        def compute_logits(self, hidden):
+            return hidden
+
+    cuda = graph_runner.torch.cuda
+    monkeypatch.setattr(cuda, "CUDAGraph", Graph)
+    monkeypatch.setattr(cuda, "graph", capture)
+    monkeypatch.setattr(cuda, "Stream", Stream)
+    monkeypatch.setattr(cuda, "current_stream", lambda: Stream())
+    monkeypatch.setattr(cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(cuda, "synchronize", lambda: None)
+    for name in ("zeros", "ones", "full"):  # no pinned memory without a device
+        make = getattr(torch, name)
+        monkeypatch.setattr(
+            torch, name, lambda *a, _make=make, pin_memory=False, **kw:
+            _make(*a, **kw))
+
+    def engine(fail=False):
+        model = Model()
+        model.fail = fail
+        r = graph_runner.DecodeGraphRunner(model, [], 8, 4,
+                                           torch.device("cpu"))
+        r.itself = r  # a cycle, as a wrapped method makes one
+        r.capture_all()
+
+    old = gc.isenabled()
+    try:
+        for on in (True, False):
+            gc.enable() if on else gc.disable()
+            engine()
+            engine()
+            with pytest.raises(ValueError):
+                engine(fail=True)
+            engine()
+            assert gc.isenabled() == on
+            # earlier engines' graphs went between captures
+            assert now["inside"] == 0 and now["gone"] >= 8
+    finally:
+        gc.enable() if old else gc.disable()
