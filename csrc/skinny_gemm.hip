@@ -3,8 +3,9 @@
 //
 // Why it exists: the library's tiles for the products of a decode batch leave
 // the read of W, which bounds them, at a third to a half of the rate that memory
-// gives. Up to 16 rows (8 of a W of more than 32768) go without splits, more
-// by the tiled form below; figures stand at both.
+// gives. Up to 16 rows (8 of a W of more than 32768) go without splits; more go
+// by the tiled form, or by the short form where a workgroup's range of K is
+// short or the tiles leave CUs waiting. Figures stand at each.
 // mfma_f32_16x16x32_bf16; operand k-pattern as verified in
 // csrc/tools/mfma_probe.hip.
 #include "ps_common.h"
@@ -104,17 +105,107 @@ __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
   }
 }
 
-// 17 to 256 rows of x (and 9 to 16 of a W of more than 32768): a workgroup owns
-// 64 NC rows of W, all rows of x and a range of K, in steps of 128 columns. x
-// passes through LDS, two steps' buffers with one barrier a step; W goes from
-// memory straight into left operands, WD steps ahead. The eight waves are four by
-// rows of W times two by halves of a step, which add up in LDS at the end.
-// Partial sums of the ranges go to memory and are added by skinny_combine.
+// The short form: a workgroup owns 64 rows of W, all rows of x and a range of K,
+// in steps of 64 columns: x passes through LDS between two barriers, W goes from
+// memory straight into right operands. Nothing is ahead, so a step costs its
+// latency, but there is nothing to fill either, and up to eight workgroups a CU
+// hide one another: 17 rows of 2048 x 64 3.2 us (tiles 5.7), 17 rows of
+// 128256 x 256 16 (25), 24 rows of 102400 x 4096 161 (175).
+template <int M_TILES>
+__global__ __launch_bounds__(256, 4) void skinny_gemm_kernel(
+    unsigned short* __restrict__ out_bf16,  // [M, N] (splits == 1)
+    float* __restrict__ ws,                 // [S, M, N] (splits > 1)
+    const unsigned short* __restrict__ x,   // [M, K]
+    const unsigned short* __restrict__ w,   // [N, K]
+    int M, int N, int K, long x_stride /* row stride of x, elems */) {
+  constexpr int MP = M_TILES * 16;  // padded M
+  const int n0 = blockIdx.x * 64;
+  const int splits = gridDim.y;
+  const int kchunks = K / 64;
+  const int per_split = (kchunks + splits - 1) / splits;
+  const int kc_begin = blockIdx.y * per_split;
+  const int kc_end = min(kchunks, kc_begin + per_split);
+  if (kc_begin >= kc_end) return;
+
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6;
+  const int lane = tid & 63;
+  const int g = lane >> 4;
+  const int rc = lane & 15;
+  const int nrow = n0 + wave * 16 + rc;  // this lane's W row (B col)
+
+  // x chunk [MP][64] staged with 16-B slot XOR swizzle (slot ^= row&7)
+  __shared__ __align__(16) unsigned short x_lds[MP][64];
+
+  ps_gf32x4 acc[M_TILES];
+#pragma unroll
+  for (int mt = 0; mt < M_TILES; mt++) acc[mt] = {0.f, 0.f, 0.f, 0.f};
+
+  for (int kc = kc_begin; kc < kc_end; kc++) {
+    // ---- cooperative x staging: MP*8 16-B slots over 256 threads ----
+    for (int u = tid; u < MP * 8; u += 256) {
+      const int row = u >> 3;
+      const int slot = u & 7;
+      ps_bf16x8 v = {};
+      if (row < M)
+        v = *(const ps_bf16x8*)(x + (long)row * x_stride + kc * 64 +
+                                slot * 8);
+      *(ps_bf16x8*)(&x_lds[row][(slot ^ (row & 7)) * 8]) = v;
+    }
+    __syncthreads();
+    // ---- B-frags: W rows streamed once ----
+    const unsigned short* wr = w + (long)nrow * K + kc * 64;
+    ps_gbf16x8 b0 = ps_as_gbf16(*(const ps_bf16x8*)(wr + g * 8));
+    ps_gbf16x8 b1 = ps_as_gbf16(*(const ps_bf16x8*)(wr + 32 + g * 8));
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int mt = 0; mt < M_TILES; mt++) {
+      const int row = mt * 16 + rc;
+      ps_gbf16x8 a0 = ps_as_gbf16(
+          *(const ps_bf16x8*)(&x_lds[row][(g ^ (row & 7)) * 8]));
+      ps_gbf16x8 a1 = ps_as_gbf16(
+          *(const ps_bf16x8*)(&x_lds[row][((4 + g) ^ (row & 7)) * 8]));
+      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[mt],
+                                                        0, 0, 0);
+      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[mt],
+                                                        0, 0, 0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __syncthreads();
+  }
+
+  // ---- epilogue (C layout: row=(g*4+r), col=rc of each 16x16 tile).
+  // splits==1 writes bf16 output directly; otherwise each split streams
+  // its fp32 partial to ws[split][M][N] and a combine kernel reduces —
+  // device atomicAdd RMW traffic (M*N*splits) was the measured 1/M
+  // throughput wall of the earlier design.
+#pragma unroll
+  for (int mt = 0; mt < M_TILES; mt++) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = mt * 16 + g * 4 + r;
+      if (m >= M) continue;
+      if (gridDim.y == 1) {
+        out_bf16[(long)m * N + nrow] = ps_f32_to_bf16(acc[mt][r]);
+      } else {
+        ws[((long)blockIdx.y * M + m) * N + nrow] = acc[mt][r];
+      }
+    }
+  }
+}
+
+// The tiled form, for 17 to 256 rows of x (and 9 to 16 of a W of more than
+// 32768): a workgroup owns 64 NC rows of W, all rows of x and a range of K, in
+// steps of 128 columns. x passes through LDS, two steps' buffers with one barrier
+// a step; W goes from memory straight into left operands, WD steps ahead. The
+// eight waves are four by rows of W times two by halves of a step, which add up in
+// LDS at the end. Partial sums of the ranges go to memory and are added by
+// skinny_combine.
 //
 // Bound by the read of W while a range is long enough to hide its start, and by
 // the reads of x from LDS with many rows (each wave reads all of x: 16 NC rows of
-// W share a read). us, distinct weights, this / the form it replaces (a barrier
-// on each side of 64 columns, loads not ahead) / the library's kernel:
+// W share a read). us, distinct weights, this / the short form / the library's
+// kernel:
 //   4096 x 14336   64 rows 32 / 48 / 40, 128 rows 39 / 65 / 74, 192 45 / 82 / 101
 //   4096 x 4096    64 rows 16 / 22 / 14, 192 rows 24 / 40 / 31
 //   28672 x 4096   64 rows 51 / 96 / 53, 192 rows 71 / 150 / 62
@@ -143,7 +234,7 @@ __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
   const int steps = (c1 - c0 + 1) / 2;
   // Every tile begins at another step of its range: rows of W a power of two
   // apart, read at the same columns by all workgroups, come from few channels of
-  // memory. us, all at the first step / this / the form before: 17 rows of
+  // memory. us, all at the first step / this / the short form: 17 rows of
   // 128256 x 4096 226 / 184 / 187, 128256 x 2048 116 / 102 / 129, 102400 x 8192
   // 419 / 333 / 311; 24 rows of 28672 x 4096 57 / 47 / 73, 4096 x 4096 12.8 / 13.6 /
   // 17.4.
@@ -293,38 +384,95 @@ __global__ __launch_bounds__(256) void skinny_combine_kernel(
                      ((unsigned int)ps_f32_to_bf16(a[3]) << 16));
 }
 
+enum PsSkinnyForm { PS_NARROW, PS_WIDE, PS_SHORT };
+struct PsSkinnyPlan {
+  PsSkinnyForm form;
+  int splits;
+};
+
+// Where the short form is the faster one. us, short / tiles:
+// Few sums (up to 32768 rows of W): the tiles' ranges have four chunks at least
+// and start with three or four steps of loads; the more sums, the more the short
+// form pays for its splits. 17 x 512 x 1024 6.1 / 7.7, 17 x 512 x 2048 7.7 / 8.1,
+// 64 x 1024 x 1024 8.7 / 8.8, 64 x 1024 x 1536 10.6 / 9.7, 32 x 4096 x 704 11.2 / 9.3,
+// 64 x 4096 x 768 13.4 / 10.6.
+// A W of more: no splits in either form. The tiles run in turns of the CUs, and
+// what the busiest CU has beyond the mean, and the start of each turn, is the
+// tiles' loss: the line follows the turns of wide tiles (up to one and a half,
+// two, three, the first half of a fourth, all of it, more). 17 x 45056 x 512 15 / 17,
+// x 1024 30 / 26; 17 x 78848 x 1536 54 / 57; 24 x 102400 x 4096 161 / 175; 24 x
+// 128256 x 1536 84 / 90; 64 x 128256 x 1280 86 / 90; 128 x 128256 x 512 62 / 62;
+// 192 x 95232 x 384 56 / 50; 256 x 61440 x 1024 81 / 85. Rows of 2048 columns come from few
+// channels in the short form (17 x 128256 x 2048 129 / 102).
+static bool ps_skinny_short(int M, int N, int K) {
+  if (K < 128) return true;
+  if (N <= 32768) {
+    const long sums = (long)M * N;
+    return K < (sums <= 32768    ? 2048
+                : sums <= 65536  ? 1536
+                : sums <= 131072 ? 640
+                                 : 0);
+  }
+  static const int all = 1 << 30;
+  static const int lines[5][6] = {{768, 896, 3264, all, 3648, 1088},
+                                  {640, 640, 960, 2624, 1344, 704},
+                                  {768, 640, 896, 1600, 640, 768},
+                                  {512, 512, 384, 512, 512, 448},
+                                  {768, 1088, 576, 1024, 1344, 896}};
+  const int rows = M <= 32 ? 0 : M <= 64 ? 1 : M <= 128 ? 2 : M <= 192 ? 3 : 4;
+  const int turn = N <= 49152    ? 0
+                   : N <= 65536  ? 1
+                   : N <= 98304  ? 2
+                   : N <= 114688 ? 3
+                   : N <= 131072 ? 4
+                                 : 5;
+  if (K == 2048 && rows == 0 && turn != 3) return false;
+  return K < lines[rows][turn];
+}
+
 // Tiles of 64 or 128 rows of W and the ranges of K: as many workgroups as there
 // are CUs, or as few more as one wave of narrow tiles takes. A range has four
 // chunks at least, or its start is most of it. Of the two widths the one that
-// fills more CUs; at as many the wide one for long rows (its reads of x from LDS
+// fills more CUs, if that takes no partial sums of short rows (17 x 10240 x 896:
+// three ranges of wide tiles 12.5, one of narrow ones 9.2; x 2048 16.6 / 15.8, x
+// 3072 20.2 / 22.8); at as many the wide one for long rows (its reads of x from LDS
 // go to twice the products), the narrow one for short ones (its partial sums are
 // half). us at 192 rows, narrow / wide: 6144 x 4096 32 (192 workgroups) / 29
 // (240), 4096 x 4096 23 / 24, 4096 x 14336 48 / 43, 2560 x 10240 33 (200) / 33
-// (160), 18944 x 3584 82 (296) / 58 (148), 16384 x 2048 30 / 37. Above 192 rows
-// the wide tile's sums do not fit in the registers.
-struct PsSkinnyPlan {
-  bool wide;
-  int splits;
-};
+// (160), 18944 x 3584 82 (296) / 58 (148), 16384 x 2048 30 / 37. Up to 32 rows of a
+// wide W are bound by its read alone: the narrow one where its busiest CU has an
+// eighth fewer rows (17 rows, narrow / wide: 49152 x 4096 75 / 89, 65664 x 8192 212 /
+// 239; 57344 x 4096 with as many rows 98 / 90, 32 of 136192 x 5120 with a tenth fewer
+// 329 / 316). Above 192 rows the wide tile's sums do not fit in the registers.
 static PsSkinnyPlan ps_skinny_plan(int M, int N, int K) {
-  const int chunks = K / 64, most = chunks / 4 > 1 ? chunks / 4 : 1;
-  int splits[2], used[2];
-  for (int wide = 0; wide < 2; ++wide) {
-    const int tiles = wide ? (N + 127) / 128 : N / 64;
-    int s = 256 / tiles;
+  const int chunks = K / 64;
+  // whole ranges of ceil(chunks / s) chunks are handed out: count those that
+  // are not empty, since an empty one would write no partial sums
+  auto ranges = [&](int s, int most) {
     if (s > most) s = most;
     if (s < 1) s = 1;
-    // whole ranges of ceil(chunks / s) chunks are handed out: count those that
-    // are not empty, since an empty one would write no partial sums
     const int per = (chunks + s - 1) / s;
-    splits[wide] = (chunks + per - 1) / per;
+    return (chunks + per - 1) / per;
+  };
+  if (ps_skinny_short(M, N, K))
+    return {PS_SHORT, ranges(1024 / (N / 64), chunks)};
+  int splits[2], used[2], busiest[2];
+  for (int wide = 0; wide < 2; ++wide) {
+    const int tiles = wide ? (N + 127) / 128 : N / 64;
+    splits[wide] = ranges(256 / tiles, chunks / 4);
     // workgroups past the CUs wait for a second turn
     used[wide] = tiles > 256 ? 128 : tiles * splits[wide];
+    busiest[wide] = (tiles + 255) / 256 * (wide ? 128 : 64);
   }
-  const bool wide = N % 128 == 0 && M <= 192 &&
-                    (used[1] > used[0] ||
-                     (used[1] == used[0] && (K >= 8192 || N > 32768)));
-  return {wide, splits[wide]};
+  bool wide;
+  if (N > 32768 && M <= 32)
+    wide = busiest[0] * 8 > busiest[1] * 7;
+  else
+    wide = (used[1] > used[0] &&
+            (splits[1] == 1 || K > (M <= 64 ? 2048 : 1536))) ||
+           (used[1] == used[0] && (K >= 8192 || N > 32768));
+  wide = wide && N % 128 == 0 && M <= 192;
+  return {wide ? PS_WIDE : PS_NARROW, splits[wide]};
 }
 
 // Whether the kernel without splits takes it; its byte offsets are 31 bits.
@@ -393,25 +541,38 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
   }
   PsSkinnyPlan plan = ps_skinny_plan(M, N, K);
   if (ws == nullptr) plan.splits = 1;
-#define PS_SG(MT, NC)                                                       \
+#define PS_SG(MT)                                                           \
+  skinny_gemm_kernel<MT><<<dim3(N / 64, plan.splits), 256, 0, stream>>>(    \
+      (unsigned short*)out_bf16, (float*)ws, (const unsigned short*)x,      \
+      (const unsigned short*)w, M, N, K, x_stride)
+#define PS_ST(MT, NC)                                                       \
   skinny_tile_kernel<MT, NC>                                                \
       <<<dim3(N / (64 * NC) * plan.splits), dim3(512), 0, stream>>>(        \
           (unsigned short*)out_bf16, (float*)ws, (const unsigned short*)x,  \
           (const unsigned short*)w, M, N, K, x_stride, plan.splits)
-#define PS_SG2(MT)                                                          \
+#define PS_ST2(MT)                                                          \
   do {                                                                      \
-    if (plan.wide)                                                          \
-      PS_SG(MT, 2);                                                         \
+    if (plan.form == PS_WIDE)                                               \
+      PS_ST(MT, 2);                                                         \
     else                                                                    \
-      PS_SG(MT, 1);                                                         \
+      PS_ST(MT, 1);                                                         \
   } while (0)
-  if (M <= 16) PS_SG2(1);
-  else if (M <= 32) PS_SG2(2);
-  else if (M <= 64) PS_SG2(4);
-  else if (M <= 128) PS_SG2(8);
-  else if (M <= 192) PS_SG2(12);
-  else PS_SG(16, 1);
-#undef PS_SG2
+  if (plan.form == PS_SHORT) {
+    if (M <= 16) PS_SG(1);
+    else if (M <= 32) PS_SG(2);
+    else if (M <= 64) PS_SG(4);
+    else if (M <= 128) PS_SG(8);
+    else PS_SG(16);
+  } else {
+    if (M <= 16) PS_ST2(1);
+    else if (M <= 32) PS_ST2(2);
+    else if (M <= 64) PS_ST2(4);
+    else if (M <= 128) PS_ST2(8);
+    else if (M <= 192) PS_ST2(12);
+    else PS_ST(16, 1);
+  }
+#undef PS_ST2
+#undef PS_ST
 #undef PS_SG
   if (plan.splits > 1) {
     const long MN = (long)M * N;

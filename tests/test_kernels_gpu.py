@@ -956,11 +956,22 @@ def test_skinny_gemm_split_ranges(m, n, k):
 @pytest.mark.parametrize("M,N,K", [
     (17, 64, 64), (32, 192, 192), (33, 128, 832), (64, 2112, 576),
     (65, 256, 640), (128, 128, 12864), (129, 320, 64), (192, 384, 1088),
-    (193, 128, 704), (256, 192, 2112), (16, 33024, 192)])
+    (193, 128, 704), (256, 192, 2112), (16, 33024, 192),
+    # the tiled form's edges again past the line of few sums
+    (17, 64, 2112), (32, 2176, 2112), (33, 128, 3136), (64, 2112, 576),
+    (65, 4096, 128), (128, 2560, 2624), (129, 2112, 192), (192, 8192, 1088),
+    (193, 768, 704), (16, 33024, 832), (24, 65664, 3328), (32, 33088, 768),
+    (16, 57344, 960), (24, 20480, 320), (40, 20480, 128), (70, 20480, 192),
+    (150, 20480, 448), (20, 2048, 8256),
+    # and the short form: one to sixteen tiles of rows, splits, none
+    (17, 320, 1984), (31, 1024, 1472), (48, 64, 1984), (100, 1280, 576),
+    (200, 64, 64), (256, 512, 576), (9, 98368, 128), (16, 33024, 704),
+    (20, 102400, 192), (130, 33024, 448), (250, 33024, 128)])
 def test_skinny_gemm_tiles(M, N, K):
     """Row counts at and past each tile count, one and two tiles of W a wave,
     ranges of one chunk, of odd numbers of chunks and of several rounds; x with
-    a row stride and not-a-numbers behind its last row."""
+    a row stride and not-a-numbers behind its last row. On both sides of the lines
+    between the forms."""
     g = torch.Generator(device="cuda").manual_seed(M + K)
     buf = torch.randn(M + 1, K + 8, generator=g, device="cuda").to(
         torch.bfloat16)
