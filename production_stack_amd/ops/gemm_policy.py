@@ -98,14 +98,18 @@ def _few_rows(rows: int, N: int, K: int) -> bool:
 
 
 def _long_rows(rows: int, N: int, K: int) -> bool:
-    """24 to 192 rows of a W of few long rows, whose tiles fill the chip only in
-    ranges of K. us, in-house / library: 4096 x 14336 with 24 rows 28.5 / 28.7,
-    64 31.7 / 39.0, 128 38.6 / 74.0, 192 44.5 / 101; 2560 x 10240 with 40 20.4 /
-    20.3, 112 25.4 / 34.2; 8192 x 28672 with 72 107 / 189; 2048 x 16384 with 40
-    22.0 / 26.7. Past the lines 6144 x 12288 with 20 36.3 / 34.5, 4096 x 11008
-    with 208 49.8 / 45.5, 1024 x 10240 with 80 19.9 / 18.2, 10240 x 8192 with 64
-    42.6 / 41.4, 4096 x 8192 with 160 31.6 / 32.3 (128 rows 29 / 32)."""
-    return 24 <= rows <= 192 and 2048 <= N <= 8192 and K >= 10240
+    """48 to 192 rows (24 where rows of W have 14336 entries) of a W of few long
+    rows, whose tiles fill the chip only in ranges of K. us, in-house / library:
+    4096 x 14336 with 24 rows 28.5 / 31.3, 64 31.3 / 38.3, 128 38.4 / 73.8, 192
+    46.2 / 100; 2560 x 10240 with 48 20.9 / 21.5, 128 26.6 / 54.5; 8192 x 28672 with
+    64 96 / 147; 2048 x 16384 with 40 22.0 / 26.7. Past the lines 2048 x 10240 with
+    40 18.3 / 17.5, 4096 x 12288 with 24 25.8 / 23.9, 8192 x 13824 with 32 47.5 / 45.0,
+    6144 x 12288 with 20 36.3 / 34.5, 4096 x 11008 with 208 49.8 / 45.5, 1024 x 10240
+    with 80 19.9 / 18.2, 10240 x 8192 with 64 42.6 / 41.4, 4096 x 8192 with 160 31.6 /
+    32.3 (128 rows 29 / 32). No wide tiles, so slower, where N is no multiple of
+    128: 6464 x 13568 with 88 70.1 / 56.6, 5184 x 12672 with 184 73.0 / 60.2."""
+    return ((24 if K >= 14336 else 48) <= rows <= 192
+            and 2048 <= N <= 8192 and N % 128 == 0 and K >= 10240)
 
 
 def _choose(x: torch.Tensor, w: torch.Tensor) -> int:

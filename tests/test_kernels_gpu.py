@@ -985,7 +985,9 @@ def test_skinny_gemm_tiles(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,own", [
-    (23, 2048, 10240, False), (24, 2048, 10240, True),
+    (47, 2048, 10240, False), (48, 2048, 10240, True),
+    (23, 2048, 14336, False), (24, 2048, 14336, True),
+    (24, 2048, 14272, False), (48, 2112, 10240, False),
     (192, 8192, 10240, True), (193, 2048, 10240, False),
     (64, 1984, 10240, False), (64, 2048, 10176, False)])
 def test_linear_long_rows(M, N, K, own):
