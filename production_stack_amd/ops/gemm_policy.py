@@ -107,7 +107,8 @@ def _long_rows(rows: int, N: int, K: int) -> bool:
     6144 x 12288 with 20 36.3 / 34.5, 4096 x 11008 with 208 49.8 / 45.5, 1024 x 10240
     with 80 19.9 / 18.2, 10240 x 8192 with 64 42.6 / 41.4, 4096 x 8192 with 160 31.6 /
     32.3 (128 rows 29 / 32). No wide tiles, so slower, where N is no multiple of
-    128: 6464 x 13568 with 88 70.1 / 56.6, 5184 x 12672 with 184 73.0 / 60.2."""
+    128: 6464 x 13568 with 88 70.1 / 56.6, 5184 x 12672 with 184 73.0 / 60.2. The
+    slowest found within: 6784 x 15360 with 28 45.4 / 43.0."""
     return ((24 if K >= 14336 else 48) <= rows <= 192
             and 2048 <= N <= 8192 and N % 128 == 0 and K >= 10240)
 

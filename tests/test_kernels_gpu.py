@@ -999,7 +999,16 @@ def test_linear_long_rows(M, N, K, own):
     x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
     w = torch.randn(N, K, device="cuda").to(torch.bfloat16)
     assert gemm_policy._choose(x, w) == own
-    assert gemm_policy._choose(x[:, 8:], w[:, 8:]) == 0  # not contiguous
+    # the same sizes that the kernel cannot take as they are: rows of W with a
+    # gap, rows of x 2 bytes off a vector, x from a pointer that is, columns apart
+    gap = torch.empty(N, K + 64, device="cuda", dtype=torch.bfloat16)[:, :K]
+    odd = torch.empty(M, K + 1, device="cuda", dtype=torch.bfloat16)[:, :K]
+    off = torch.empty(M * K + 8, device="cuda", dtype=torch.bfloat16)
+    off = off[1:M * K + 1].view(M, K)
+    apart = torch.empty(K, M, device="cuda", dtype=torch.bfloat16).t()
+    assert gemm_policy._choose(x, gap) == 0
+    for other in (odd, off, apart):
+        assert gemm_policy._choose(other, w) == 0
     want = ops.skinny_gemm(x, w) if own else torch.nn.functional.linear(x, w)
     assert torch.equal(gemm_policy.linear(x, w), want)
 
