@@ -1401,6 +1401,8 @@ struct CkWideHead {  // per chunk and head, floats
   static constexpr int SUF = 160; // [16] first half: behind it to 15
   static constexpr int PRE = 176; // [16] second half: from 16, with it
   static constexpr int GAM = 192; // decay over the chunk
+  static constexpr int FLAG = 193; // not 0: a q, k or write scale is no finite
+                                   // number, or so large that q k w might not be
   static constexpr int TOTAL = 196;
 };
 
@@ -1425,20 +1427,22 @@ __global__ __launch_bounds__(256) void ck_prep_wide_kernel(
   const int row0 = seq_rows[4 * seg] + 32 * chunk;
   const int nv = min(32, n - 32 * chunk);
   const int g = lane >> 4, m16 = lane & 15;
+  const mx_bf16* qp = (const mx_bf16*)in.q + grp * D;
+  const mx_bf16* kp = (const mx_bf16*)in.k + grp * D;
+  bool odd = false;
+  for (int i = threadIdx.x; i < 32 * DP; i += 256) {
+    const int t = i / DP, d = i % DP;
+    const size_t row = (size_t)(row0 + min(t, nv - 1));
+    const int dc = min(d, D - 1);
+    const unsigned short q = qp[row * in.ldq + dc].x;
+    const unsigned short k = kp[row * in.ldk + dc].x;
+    const bool live = t < nv && d < D;
+    Q[t * LD + d] = live ? q : 0;
+    K[t * LD + d] = live ? k : 0;
+    odd |= live && max(q & 0x7fff, k & 0x7fff) >= 0x4d80;  // 2^28
+  }
+  odd = __syncthreads_or(odd);
   if (blockIdx.z == 0) {
-    const mx_bf16* qp = (const mx_bf16*)in.q + grp * D;
-    const mx_bf16* kp = (const mx_bf16*)in.k + grp * D;
-    for (int i = threadIdx.x; i < 32 * DP; i += 256) {
-      const int t = i / DP, d = i % DP;
-      const size_t row = (size_t)(row0 + min(t, nv - 1));
-      const int dc = min(d, D - 1);
-      const unsigned short q = qp[row * in.ldq + dc].x;
-      const unsigned short k = kp[row * in.ldk + dc].x;
-      const bool live = t < nv && d < D;
-      Q[t * LD + d] = live ? q : 0;
-      K[t * LD + d] = live ? k : 0;
-    }
-    __syncthreads();
     char* dst = gitems + ((size_t)item * G + grp) * Gi::TOTAL;
     auto rows8 = [&](const unsigned short* x, int tok, int ks) {
       const unsigned short* p = x + tok * LD + 32 * ks + 4 * g;
@@ -1488,6 +1492,7 @@ __global__ __launch_bounds__(256) void ck_prep_wide_kernel(
     }
     a = t < nv ? a : 1.f;
     w = t < nv ? w : 0.f;
+    const unsigned large = __ballot(!(w < 0x1p60f)) >> (threadIdx.x & 32);
     __syncthreads();
     sa[hl][t] = a;
     sw[hl][t] = w;
@@ -1522,7 +1527,10 @@ __global__ __launch_bounds__(256) void ck_prep_wide_kernel(
         dst[Hd::SUF + t] = suf;
       else
         dst[Hd::PRE + t - 16] = pre;
-      if (t == 31) dst[Hd::GAM] = dr;
+      if (t == 31) {
+        dst[Hd::GAM] = dr;
+        *(unsigned*)(dst + Hd::FLAG) = large | odd;
+      }
     }
   }
 }
@@ -1544,21 +1552,49 @@ __global__ __launch_bounds__(256) void ck_prep_wide_kernel(
 // Measured (ssd, 128 heads of 128 x 64, 8192 rows in 2 prompts): 605 us by
 // fp32 products in chunks of 16, 330 with all rows of a tile in one wave (one
 // wave a SIMD: 800 instructions in 5300 cycles), 285 with two.
-template <int MODE, int DP, int PART, int NW>
-__global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_wide_kernel(
-    float* __restrict__ out, int ldo, const char* __restrict__ gitems,
-    const float* __restrict__ hitems, int cap, CkIn in,
-    const float* __restrict__ p2, float* __restrict__ state,
-    float* __restrict__ aux, const int* __restrict__ seq_rows, int S_, int H,
-    int G, int D, int DV, int base, float* __restrict__ part, int parts) {
+// memory that no kernel under way writes: scalar loads
+#define CK_CONST __attribute__((address_space(4)))
+struct CkWideCall {
+  float* out;
+  int ldo;
+  const char* gitems;
+  const float* hitems;
+  int cap;
+  CkIn in;
+  const float* p2;
+  float *state, *aux;
+  const int* seq_rows;
+  int S_, H, G, D, DV, base;
+  float* part;
+  int parts;
+};
+template <int DP, int NW>
+struct CkWideLds {
+  static constexpr int WAVES = NW * (DP % 64 == 0 ? 2 : 1);
+  ck_u32x4 mfrag[2][2][3][64];  // set, token tile, term
+  float vtmp[WAVES][512];
+  ck_f32x4 share[2][DP % 64 == 0 ? WAVES : 1][64];
+};
+
+// The walk; false where something in it came to no finite number (to all waves of
+// the workgroup, or each on its own where PART is 1): then the state is not
+// written. AGAIN: the walk from its start after that, with nothing ahead, for
+// infinities as the fp32 products have them. In the loop itself their branches
+// took 3 to 10 % of the walk.
+template <int MODE, int DP, int PART, int NW, bool AGAIN>
+PS_DEV bool ck_walk_wide(const CkWideCall& a, CkWideLds<DP, NW>& lds) {
   typedef CkWide<DP> Gi;
   typedef CkWideHead Hd;
   constexpr int RH = DP % 64 == 0 ? 2 : 1;   // waves that share a column tile
   constexpr int NT = DP / 16, NK = DP / 32;  // tiles of the state
   constexpr int WT = NT / RH, WK = NK / RH;  // and of a wave
-  __shared__ ck_u32x4 mfrag[2][2][3][64];  // set, token tile, term
-  __shared__ float vtmp[NW * RH][512];
-  __shared__ ck_f32x4 share[2][RH == 2 ? NW * RH : 1][64];
+  auto& mfrag = lds.mfrag;
+  auto& vtmp = lds.vtmp;
+  auto& share = lds.share;
+  const CkIn& in = a.in;
+  const int S_ = a.S_, H = a.H, G = a.G, D = a.D, DV = a.DV, ldo = a.ldo;
+  const int cap = a.cap, base = a.base, parts = a.parts;
+  const int* seq_rows = a.seq_rows;
 
   const int cols = DV + (MODE == CK_MLSTM ? 1 : 0);
   const int ncb = ((cols + 15) / 16 + NW - 1) / NW;
@@ -1566,12 +1602,12 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
   const int rest = blockIdx.x - run * S_ * H * ncb;
   const int hd = rest % H, cb = rest / H % ncb;
   const int seg = ck_by_length(seq_rows, S_, rest / (H * ncb));
-  if (seg < 0) return;
+  if (seg < 0) return true;
   const int sh = seg * H + hd, grp = hd / (H / G);
   int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
   const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
   const int all = ck_count<CK_WIDE>(n);
-  if (all == 0) return;
+  if (all == 0) return true;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int first = 0;
@@ -1583,14 +1619,14 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
   int c0 = max(0, -first);
   int count =
       __builtin_amdgcn_readfirstlane(min(all, cap - first) - c0);
-  if (count <= 0) return;
+  if (count <= 0) return true;
   first += c0;
   const bool old = p0 != 0 || c0 != 0;  // there is a state to start from
   bool last = true;  // this run ends the segment's chunks of the pass
   if constexpr (PART != 0) {
     const int per = (count + parts - 1) / parts;
     last = (run + 1) * per >= count;
-    if (run * per >= count) return;
+    if (run * per >= count) return true;
     first += run * per;
     c0 += run * per;
     count = min(per, count - run * per);
@@ -1606,11 +1642,11 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
   const int j = (cb * NW + wave / RH) * 16 + m16;
   const bool col = j < DV;
   const bool ncol = MODE == CK_MLSTM && j == DV;
-  float* Sg = state + ((size_t)slot * H + hd) * (size_t)D * DV + j;
-  float* Ng = MODE == CK_MLSTM ? aux + ((size_t)slot * H + hd) * (D + 1)
+  float* Sg = a.state + ((size_t)slot * H + hd) * (size_t)D * DV + j;
+  float* Ng = MODE == CK_MLSTM ? a.aux + ((size_t)slot * H + hd) * (D + 1)
                                : nullptr;
   const size_t rec = (size_t)D * cols + 4;  // of one run
-  float* pt = PART ? part + (size_t)sh * parts * rec : nullptr;
+  float* pt = PART ? a.part + (size_t)sh * parts * rec : nullptr;
   ck_f32x4 S[WT];
 #pragma unroll
   for (int t = 0; t < WT; ++t)
@@ -1657,10 +1693,10 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
   const size_t gstep = (size_t)G * Gi::TOTAL;
   const size_t hstep = (size_t)H * Hd::TOTAL * sizeof(float);
   // of the chunk ahead by one, two (the last one again behind it)
-  const char* g1 = gitems + ((size_t)first * G + grp) * Gi::TOTAL;
+  const char* g1 = a.gitems + ((size_t)first * G + grp) * Gi::TOTAL;
   const char* g2 = g1;
   const char* h2 =
-      (const char*)(hitems + ((size_t)first * H + hd) * Hd::TOTAL);
+      (const char*)(a.hitems + ((size_t)first * H + hd) * Hd::TOTAL);
   const unsigned at16 = lane * 16, off = 0x80000000u;
   const unsigned rsv = in.ldv * 2, rsg = in.ldg * 2, rso = ldo * 4;
   const unsigned at_v = col ? 4 * g * rsv + j * 2 : off;
@@ -1673,7 +1709,7 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
           ? (const char*)((const mx_bf16*)in.gate + (size_t)t0 * in.ldg +
                           hd * DV)
           : nullptr;
-  char* oseg = (char*)(out + (size_t)t0 * ldo +
+  char* oseg = (char*)(a.out + (size_t)t0 * ldo +
                        hd * (MODE == CK_SSD ? DV : DV + 1));
   // chunk c's rows (and more, up to the segment's end) of `p`, `rb` bytes
   // apart, `width` bytes of each
@@ -1682,7 +1718,7 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
     return __builtin_amdgcn_make_buffer_rsrc((void*)(p + (size_t)c * 32 * rb),
                                              0, more * rb + width, 0x00020000);
   };
-  const float skip = MODE == CK_SSD ? p2[hd] : 0.f;
+  const float skip = MODE == CK_SSD ? a.p2[hd] : 0.f;
 
   struct Cells {  // of this lane's rows, as loaded
     unsigned short v[8], gt[8 / RH];
@@ -1694,6 +1730,7 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
   struct Scales {
     ck_f32x4 dr[2 / RH], dk[2];
     float gam;
+    unsigned odd;
   };
   // of Q the wave's own token tile first
   ck_u32x4 Q[PART == 1 ? 1 : 2 * WK], K[WT];
@@ -1751,8 +1788,8 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
     x.w = load4(r, g * 16, (Hd::W + b) * 4);
     x.y = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
         r, m16 * 4, (h == 1 ? Hd::PRE : Hd::P + b) * 4, 0));
-    x.u1 = ((const float*)h2)[Hd::P + b + 7];
-    x.u2 = ((const float*)h2)[Hd::P + b + 11];
+    x.u1 = ((CK_CONST const float*)h2)[Hd::P + b + 7];
+    x.u2 = ((CK_CONST const float*)h2)[Hd::P + b + 11];
   };
   auto fetch_scales = [&](Scales& x) {
     const auto r = head_buffer();
@@ -1764,28 +1801,46 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
       x.dk[mt] = load4(r, g * 16, (Hd::DK + 16 * mt) * 4);
-    x.gam = ((const float*)h2)[Hd::GAM];
+    x.gam = ((CK_CONST const float*)h2)[Hd::GAM];
+    x.odd = ((CK_CONST const unsigned*)h2)[Hd::FLAG];
   };
   // a block of M: rows s = 4 g + i of its half, column t = m16 of its own;
   // every decay between them by products of its own
   auto make_block = [&](int h, const Block& x, ck_u32x4* to) {
     h = min(h, 2);
     // no branches: where ways meet, waits are for the latest load of either
-    const int b = h == 1 ? 4 : m16 >> 2;
+    // comparisons made anew, one each: kept, they spill scalar registers within
+    // the loop
+    int t = m16;
+    asm volatile("" : "+v"(t));
+    t = h == 1 ? 19 : t;
+    const int b = t >> 2;
     float tail = b > g ? x.y : 1.f;
-    tail *= g < 1 && (b == 2 || b == 3) ? x.u1 : 1.f;
-    tail *= g < 2 && b == 3 ? x.u2 : 1.f;
+    // the blocks of four between: b 2 and 3 for g 0, b 3 for g 1
+    tail *= (unsigned)(b - 2) < (g < 1 ? 2u : 0u) ? x.u1 : 1.f;
+    tail *= (unsigned)(b - 3) < (g < 2 ? 1u : 0u) ? x.u2 : 1.f;
     ck_f32x4 e;
     e[3] = h == 1 ? tail * x.x[3] : tail;
 #pragma unroll
     for (int i = 2; i >= 0; --i)
       e[i] = h == 1 ? tail * x.x[i]
-                    : e[i + 1] * (4 * g + i + 1 <= m16 ? x.x[i + 1] : 1.f);
+                    : e[i + 1] * (4 * g + i + 1 <= t ? x.x[i + 1] : 1.f);
     ck_f32x4 m;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      m[i] = h == 1 || 4 * g + i <= m16 ? x.qk[i] * e[i] * x.w[i] : 0.f;
-    const CkTerms4 tm = ck_split(m);
+      m[i] = 4 * g + i <= t ? x.qk[i] * e[i] * x.w[i] : 0.f;
+    CkTerms4 tm = ck_split(m);
+    if constexpr (AGAIN) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (!(fabsf(m[i]) < INFINITY)) {  // the first term is all of it
+          const unsigned low = i & 1 ? 0xffffu : 0xffff0000u;
+          const unsigned top = __float_as_uint(m[i] != m[i] ? NAN : m[i]) >> 16;
+          tm.h[i >> 1] = (tm.h[i >> 1] & low) | top << (i & 1) * 16;
+          tm.m[i >> 1] &= low;
+          tm.l[i >> 1] &= low;
+        }
+    }
     // token tile, half of the lane's eight
     ck_u32x2* dst = (ck_u32x2*)(to + (h == 0 ? 0 : 192) + lane) + (h == 2);
     dst[0] = tm.h;
@@ -1793,15 +1848,26 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
     dst[256] = tm.l;
   };
 
+  // a where it is a finite number, else b
+  auto either = [](ck_f32x4 a, ck_f32x4 b) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = fabsf(a[i]) < INFINITY ? a[i] : b[i];
+    return a;
+  };
   const ck_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  // Chunk c; what is used makes room for a later chunk's at once.
+  unsigned odd = 0;  // some chunk's flag
+  // Chunk c; what is used makes room for a later chunk's at once. AGAIN: not, and
+  // what comes to no finite number is made of the numbers themselves. The three
+  // terms of an infinity are not its sum, and an infinite q or k beside a term of
+  // zero makes no number of it, where the fp32 products would be infinite.
   auto walk = [&](int c, Cells& cells, Scales& sc, Block& blk) {
     // the next chunk's M
     if constexpr (PART != 1) {
       make_block(wave, blk, &mfrag[(c + 1) & 1][0][0][0]);
-      fetch_block(wave, blk);
+      if constexpr (!AGAIN) fetch_block(wave, blk);
     }
     ck_f32x4 V[2], W[2], O[2] = {zero, zero}, X[2] = {zero, zero};
+    ck_f32x4 P[2] = {zero, zero};  // O of the numbers themselves
     float gt[8 / RH];
     const int left = n - 32 * c - 4 * g;
 #pragma unroll
@@ -1815,11 +1881,12 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
     for (int i = 0; i < 8 / RH; ++i)
       gt[i] = __uint_as_float((unsigned)cells.gt[i] << 16);
     const Scales s0 = sc;
-    const bool fin =
-        PART == 1 || __all(ck_finite(V[0]) && ck_finite(V[1]));
+    odd |= s0.odd;
     __builtin_amdgcn_sched_barrier(0);
-    fetch_cells(c + 2, cells);
-    fetch_scales(sc);
+    if constexpr (!AGAIN) {
+      fetch_cells(c + 2, cells);
+      fetch_scales(sc);
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) W[mt] = V[mt] * s0.dk[mt];
@@ -1827,7 +1894,7 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
       // values that are no finite numbers are left out here: beside the zeros
       // above M's diagonal they would reach earlier tokens
       ck_f32x4 F[2] = {V[0], V[1]};
-      if (!fin) {
+      if constexpr (AGAIN) {
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           if (!(fabsf(V[i >> 2][i & 3]) < INFINITY)) F[i >> 2][i & 3] = 0.f;
@@ -1841,7 +1908,7 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
 #pragma unroll
         for (int mt = 0; mt < 2 / RH; ++mt)
           X[mt] = ck_mfma(mf[mt + rh][q][lane], vb, X[mt]);
-      if (!fin) {
+      if constexpr (AGAIN) {
         // what the left out values add
         float* tmp = vtmp[wave];
 #pragma unroll
@@ -1884,26 +1951,54 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
         for (int mt = 0; mt < 2; ++mt)
           O[mt] = ck_mfma(Q[mt * WK + ks], ts.h, O[mt]);
       }
+      if constexpr (PART != 1 && AGAIN) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            P[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                ck_bf16(Q[mt * WK + ks], i), S[2 * ks + (i >> 2)][i & 3], P[mt],
+                0, 0, 0);
+      }
       S[2 * ks] *= s0.gam;
       S[2 * ks + 1] *= s0.gam;
     }
+    if constexpr (PART != 1 && AGAIN) {
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) O[mt] = either(O[mt], P[mt]);
+    }
     if constexpr (PART != 1) {
-      fetch_q();
+      if constexpr (!AGAIN) fetch_q();
       if constexpr (RH == 2) share[c & 1][wave][lane] = O[1];
     }
     if constexpr (PART == 1) decay *= s0.gam;
     const CkTerms8 tw = ck_split(W[0], W[1]);
+    if constexpr (AGAIN) {
 #pragma unroll
-    for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.l, S[t]);
+      for (int t = 0; t < WT; ++t) {
+        ck_f32x4 x = S[t];
 #pragma unroll
-    for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.m, S[t]);
+        for (int i = 0; i < 8; ++i)
+          x = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              ck_bf16(K[t], i), W[i >> 2][i & 3], x, 0, 0, 0);
+        S[t] = ck_mfma(K[t], tw.l, S[t]);
+        S[t] = ck_mfma(K[t], tw.m, S[t]);
+        S[t] = either(ck_mfma(K[t], tw.h, S[t]), x);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
 #pragma unroll
-    for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.h, S[t]);
-    fetch_k();
-    g1 = g2;
-    if (c + 3 < count) {
-      g2 += gstep;
-      h2 += hstep;
+      for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.l, S[t]);
+#pragma unroll
+      for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.m, S[t]);
+#pragma unroll
+      for (int t = 0; t < WT; ++t) S[t] = ck_mfma(K[t], tw.h, S[t]);
+      fetch_k();
+      g1 = g2;
+      if (c + 3 < count) {
+        g2 += gstep;
+        h2 += hstep;
+      }
     }
     if constexpr (PART != 1) {
       // also: the next chunk's M is there, this one's is read
@@ -1941,43 +2036,71 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
     make_block(wave, blk, &mfrag[0][0][0][0]);
     __syncthreads();
   }
-  // the order in which a chunk's loads are asked for below: the waits of the
-  // loop are for what is later in either
-  fetch_cells(0, ca);
-  fetch_scales(sa);
-  __builtin_amdgcn_sched_barrier(0);
-  g2 = gn;
-  h2 = hn;
-  if constexpr (PART != 1) fetch_block(wave, blk);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_cells(1, cb2);
-  fetch_scales(sb);
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (PART != 1) fetch_q();
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_k();
-  __builtin_amdgcn_sched_barrier(0);
-  g1 = gn;
-  if (count > 2) {
-    g2 += gstep;
-    h2 += hstep;
-  }
-  int c = 0;
+  if constexpr (AGAIN) {
 #pragma unroll 1
-  for (; c + 1 < count; c += 2) {
-    walk(c, ca, sa, blk);
-    walk(c + 1, cb2, sb, blk);
+    for (int c = 0; c < count; ++c) {
+      g1 = a.gitems + ((size_t)(first + c) * G + grp) * Gi::TOTAL;
+      g2 = g1;
+      h2 = (const char*)(a.hitems + ((size_t)(first + c) * H + hd) * Hd::TOTAL);
+      fetch_cells(c, ca);
+      fetch_scales(sa);
+      fetch_k();
+      if constexpr (PART != 1) {
+        fetch_q();
+        if (c + 1 < count) {
+          g2 += gstep;
+          h2 += hstep;
+        }
+        fetch_block(wave, blk);
+      }
+      walk(c, ca, sa, blk);
+    }
+  } else {
+    // the order in which a chunk's loads are asked for below: the waits of the
+    // loop are for what is later in either
+    fetch_cells(0, ca);
+    fetch_scales(sa);
+    __builtin_amdgcn_sched_barrier(0);
+    g2 = gn;
+    h2 = hn;
+    if constexpr (PART != 1) fetch_block(wave, blk);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_cells(1, cb2);
+    fetch_scales(sb);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (PART != 1) fetch_q();
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_k();
+    __builtin_amdgcn_sched_barrier(0);
+    g1 = gn;
+    if (count > 2) {
+      g2 += gstep;
+      h2 += hstep;
+    }
+    int c = 0;
+#pragma unroll 1
+    for (; c + 1 < count; c += 2) {
+      walk(c, ca, sa, blk);
+      walk(c + 1, cb2, sb, blk);
+    }
+    if (c < count) walk(c, ca, sa, blk);
+    // A value, key or decay that is no finite number leaves none in the state, and
+    // there they stay; the flags tell of the others.
+#pragma unroll
+    for (int t = 0; t < WT; ++t) odd |= !ck_finite(S[t]);
+    if (PART == 1 ? __any(odd) : __syncthreads_or(odd)) return false;
   }
-  if (c < count) walk(c, ca, sa, blk);
   if (PART == 1 && cb == 0 && threadIdx.x == 0)
     pt[run * rec + (size_t)D * cols] = decay;
-  if (PART == 2 && !last) return;
+  if (PART == 2 && !last) return true;
+  int rows = D;  // which rows there are, found again and not kept over the walk
+  asm volatile("" : "+s"(rows));
 #pragma unroll
   for (int t = 0; t < WT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int d = 16 * (WT * rh + t) + 4 * g + i;
-      if (d < D) {
+      if (d < rows) {
         if (PART == 1) {
           if (col || ncol) pt[run * rec + (size_t)d * cols + j] = S[t][i];
         } else {
@@ -1986,6 +2109,24 @@ __global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1), 2) void ck_sweep_
         }
       }
     }
+  return true;
+}
+
+template <int MODE, int DP, int PART, int NW>
+__global__ __launch_bounds__(64 * NW * (DP % 64 == 0 ? 2 : 1),
+                             PART == 1 && DP != 96 ? 4 : 2)  // waves a SIMD
+void ck_sweep_wide_kernel(CkWideCall a) {
+  __shared__ CkWideLds<DP, NW> lds;
+  if (ck_walk_wide<MODE, DP, PART, NW, false>(a, lds)) return;
+  // the arguments once more, so that nothing is kept for this over the first walk:
+  // scalar registers would spill within its loop
+  unsigned long at = (unsigned long)__builtin_amdgcn_kernarg_segment_ptr();
+  unsigned low = at, high = at >> 32;
+  asm volatile("" : "+s"(low), "+s"(high));
+  at = (unsigned)__builtin_amdgcn_readfirstlane(low) |
+       (unsigned long)(unsigned)__builtin_amdgcn_readfirstlane(high) << 32;
+  ck_walk_wide<MODE, DP, PART, NW, true>(
+      *(const CkWideCall*)(CK_CONST const CkWideCall*)at, lds);
 }
 
 // Read-out norm and gate: o / rms_DV(o) * weight * gate for the rows of
@@ -2293,15 +2434,15 @@ static int ck_launch_wide(CK_ARGS) {
     hipLaunchKernelGGL((ck_prep_wide_kernel<MODE, DP>), dim3(cap, G, slices),
                        dim3(256), 0, stream, (char*)gitems, hitems, in, ga,
                        gw, (const int*)seq_rows, S_, H, G, D, scale, p * cap);
+    const CkWideCall call = {
+        lstm ? raw : (float*)out, lstm ? H * (DV + 1) : ldo,
+        (const char*)gitems, hitems, cap, in, (const float*)p2, (float*)state,
+        (float*)aux, (const int*)seq_rows, S_, H, G, D, DV, p * cap, part,
+        parts};
 #define CK_SWEEP_NW(PART, RUNS, NW)                                          \
   hipLaunchKernelGGL((ck_sweep_wide_kernel<MODE, DP, PART, NW>),             \
                      dim3(S_ * H * ((tiles + NW - 1) / NW) * (RUNS)),        \
-                     dim3(64 * NW * (DP % 64 == 0 ? 2 : 1)), 0, stream,      \
-                     lstm ? raw : (float*)out,                               \
-                     lstm ? H * (DV + 1) : ldo, (const char*)gitems, hitems, \
-                     cap, in, (const float*)p2, (float*)state, (float*)aux,  \
-                     (const int*)seq_rows, S_, H, G, D, DV, p * cap, part,   \
-                     parts)
+                     dim3(64 * NW * (DP % 64 == 0 ? 2 : 1)), 0, stream, call)
 #define CK_SWEEP(PART, RUNS)                                                 \
   if (ck_wide_tiles(tiles) == 3)                                             \
     CK_SWEEP_NW(PART, RUNS, 3);                                              \

@@ -56,9 +56,10 @@ PS_DEV float ck_log_sigmoid(float z) {
   return fminf(z, 0.f) - log1pf(expf(-fabsf(z)));
 }
 
-// fp32 numbers on the bf16 matrix unit: each is exactly the sum of three bf16
-// terms (h, m, l: 8 bits each; the first one is cut off and not rounded, so
-// that the largest numbers stay finite). Beside an operand that is bf16 already
+// fp32 numbers on the bf16 matrix unit: each finite one is exactly the sum of
+// three bf16 terms (h, m, l: 8 bits each; the first one is cut off and not
+// rounded, so that the largest numbers stay finite); of an infinity, or what is
+// no number, m and l are no numbers. Beside an operand that is bf16 already
 // every product is exact, and the unit takes 3 / 16 of the fp32 unit's time.
 typedef __attribute__((ext_vector_type(2))) unsigned ck_u32x2;
 typedef __attribute__((ext_vector_type(4))) unsigned ck_u32x4;
@@ -104,6 +105,11 @@ PS_DEV ck_u32x4 ck_join(ck_u32x2 a, ck_u32x2 b) {
 PS_DEV CkTerms8 ck_split(ck_f32x4 a, ck_f32x4 b) {
   const CkTerms4 x = ck_split(a), y = ck_split(b);
   return {ck_join(x.h, y.h), ck_join(x.m, y.m), ck_join(x.l, y.l)};
+}
+
+// Number j of eight bf16.
+PS_DEV float ck_bf16(ck_u32x4 x, int j) {
+  return __uint_as_float(j & 1 ? x[j >> 1] & 0xffff0000u : x[j >> 1] << 16);
 }
 
 PS_DEV ck_f32x4 ck_mfma(ck_u32x4 a, ck_u32x4 b, ck_f32x4 c) {

@@ -281,12 +281,15 @@ def test_recurrence_chunk_edges(mode, H, D, DV, dtype):
         assert _rel(ag, aux) < 2e-6
 
 
+@pytest.mark.parametrize("bad_row", [5, 21])
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("mode", RECURRENCES)
-def test_recurrence_chunk_not_a_number(mode):
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+def test_recurrence_chunk_not_a_number(mode, dtype, bad_row, D):
     """A value, key or decay that is no number reaches no earlier row, not
     even of its own chunk, and no other sequence."""
     rows = _segs([40, 33], [0, 4])
-    x, state, aux, call = _recurrence(mode, 2, 32, 32, rows, torch.float32)
+    x, state, aux, call = _recurrence(mode, 2, D, D, rows, dtype)
     rows = torch.tensor(rows, dtype=torch.int32).cuda()
     xg = _to_gpu(x)
     clean = call(xg, state.cuda(), aux.cuda() if aux is not None else None,
@@ -294,12 +297,72 @@ def test_recurrence_chunk_not_a_number(mode):
     for name, bad in (("v", float("nan")), ("v", float("inf")),
                       ("k", float("nan")), ("dec", float("nan"))):
         y = _to_gpu(x)
-        y[name][21, min(3, y[name].shape[1] - 1)] = bad
+        y[name][bad_row, min(3, y[name].shape[1] - 1)] = bad
         got = call(y, state.cuda(), aux.cuda() if aux is not None else None,
                    rows)
-        assert _rel(got[:21], clean[:21]) < 1e-6, name
+        # other sums within the chunk; rows of bf16 round once more
+        near = 1e-6 if got.dtype == torch.float32 else 2 ** -9
+        assert _rel(got[:bad_row], clean[:bad_row]) < near, name
         assert _rel(got[40:], clean[40:]) < 1e-6, name
-        assert not torch.isfinite(got[21:40]).all(), name
+        assert not torch.isfinite(got[bad_row:40]).all(), name
+
+
+@pytest.mark.parametrize("lens,tokens", [
+    ([75, 33], (5, 21, 37, 64, 74)), ([700], (100, 351))])
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("mode", ["ssd", "mlstm"])
+def test_recurrence_chunk_infinities(mode, D, lens, tokens):
+    """Values, keys, queries and states that are infinite, or no numbers, in
+    either half of a chunk of 32 and in one of several runs: bf16 rows leave
+    infinities and not-a-numbers in the state where fp32 rows of the same values
+    do, whose products are made as they are (k inf is an infinity). Earlier rows
+    and other sequences stay as they are."""
+    H, DV = 2, 40
+    segs = _segs(lens, [3, 4])
+    x, state, aux, call = _recurrence(mode, H, D, DV, segs, torch.bfloat16)
+    rows = torch.tensor(segs, dtype=torch.int32).cuda()
+    base = x["q"]._base.float()
+    wide = {k: (torch.as_strided(base, v.shape, v.stride(),
+                                 v.storage_offset())
+                if v._base is not None else v) for k, v in x.items()}
+
+    def run(x, name, at, bad):
+        x, st = _to_gpu(x), state.clone()
+        if name == "state":  # one entry, which every row of its head meets
+            st[segs[0][3], at % H, 5, 3] = bad
+        elif name:
+            x[name][at, 3] = bad
+        st = st.cuda()
+        ax = aux.cuda() if aux is not None else None
+        out = call(x, st, ax, rows)
+        return [t.float() for t in (out, st, ax) if t is not None]
+
+    def same(a, b):
+        for what in (math.inf, -math.inf):
+            assert torch.equal(a == what, b == what)
+        assert torch.equal(a.isnan(), b.isnan())
+
+    clean = run(x, None, 0, 0.0)
+    near = 1e-6 if mode == "ssd" else 2 ** -9  # other sums, one rounding
+    # (decays over a run may come to zero, which leaves no infinity)
+    for name in ("v", "k", "q") + (("state",) if len(lens) > 1 else ()):
+        for at in tokens:
+            for bad in (math.inf, -math.inf, math.nan):
+                got, want = run(x, name, at, bad), run(wide, name, at, bad)
+                for a, b in zip(got[1:], want[1:]):
+                    same(a, b)
+                if name == "state":
+                    same(got[0], want[0])
+                else:
+                    # sums of several infinities: which chunk they meet in
+                    # says whether they come to one or to none
+                    assert not got[0][at, 3].isfinite()
+                    assert _rel(got[0][:at], clean[0][:at]) < near
+                assert torch.equal(got[0][lens[0]:], clean[0][lens[0]:])
+                # numbers stay: one rounding to bf16, states are fp32
+                for a, b, c in zip(got, want, (6e-3, 2e-6, 2e-6)):
+                    ok = a.isfinite() & b.isfinite()
+                    assert not ok.any() or _rel(a[ok], b[ok]) < c
 
 
 @pytest.mark.parametrize("mode", ["general", "channel", "gla"])
