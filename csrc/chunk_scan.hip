@@ -123,9 +123,14 @@ PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int lane, int* seg,
 // -1 where it has no chunks. Workgroups start in the order of their numbers, so
 // the longest walks start first, and the CU of one takes a shorter one beside
 // it: general delta, 32 heads, prompts of 336 and 166 chunks, 0.60 -> 0.47 ms.
-// Past 64 segments, more than a step has of prompts, they go as they come.
+// Past 32 segments they go as they come: the order would cost a workgroup a
+// load and a turn a segment before its own rows can be asked for, which with
+// many workgroups of a few chunks is more than it gives. us, ordered / as they
+// come: general delta, 32 heads of 96 x 96, 1200 rows in 40 prompts 188 / 161,
+// 3000 in 40 333 / 307, of 64 x 64, 6000 in 60 364 / 343; 8 heads of 128 x 128,
+// 5000 in 24 133 / 140, of 64 x 64, 8000 in 40 114 / 120.
 PS_DEV int ck_by_length(const int* seq_rows, int S_, int rank) {
-  if (S_ > 64 || S_ == 1) return rank;
+  if (S_ > 32 || S_ == 1) return rank;
   const int lane = threadIdx.x & 63;
   const int mine = lane < S_ ? seq_rows[4 * lane + 1] : 0;
   if (rank >= __popcll(__ballot(ck_count(mine) > 0))) return -1;
@@ -507,6 +512,15 @@ PS_DEV ck_f32x4 ck_token_terms(float f, float x, ck_f32x4 acc, int lane,
 // (twice the waves for as many instructions beside the products).
 static constexpr int ck_row_tiles(int dp) { return dp <= 64 ? 1 : 2; }
 
+// Waves that a SIMD has registers for: three, since many short segments are
+// more workgroups than two a SIMD hold; two where three would spill (fp32 rows
+// of 128, either delta: 78 and 25 registers). us, two / three: general delta,
+// 32 fp32 heads of 96 x 96, 1200 rows in 40 prompts 161 / 139, 3000 in 40
+// 307 / 285, 4000 in 8 330 / 327.
+static constexpr int ck_sweep_waves(int mode, int dp, bool wide) {
+  return !wide || dp <= 96 || mode == CK_GLA ? 3 : 2;
+}
+
 // Walks the chunks of one (segment, head) for 16 columns of its state: a wave
 // per 32 rows of it (16 of up to 64), two to four waves. raw [T, H * DV]: S^T r before the
 // read-out's norm.
@@ -538,7 +552,8 @@ static constexpr int ck_row_tiles(int dp) { return dp <= 64 ? 1 : 2; }
 // each run from what the runs before it leave and writes the outputs.
 template <typename T, int MODE, int DP, int PART>
 __global__ __launch_bounds__(DP * 4 / ck_row_tiles(DP),
-                             sizeof(T) == 2 ? 3 : 2) void ck_sweep_kernel(
+                             ck_sweep_waves(MODE, DP, sizeof(T) == 4))
+    void ck_sweep_kernel(
     float* __restrict__ raw, const float* __restrict__ items, int cap,
     const T* __restrict__ v, int ldv, float* __restrict__ state,
     const int* __restrict__ seq_rows, int S_, int H, int D, int DV, int base,
