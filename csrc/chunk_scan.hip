@@ -119,28 +119,71 @@ PS_DEV bool ck_find(const int* seq_rows, int S_, int item, int lane, int* seg,
   return false;
 }
 
-// The segment that `rank` others are longer than (of equal ones the first),
-// -1 where it has no chunks. Workgroups start in the order of their numbers, so
+// A segment's row of seq_rows and its first chunk among those of all.
+struct CkSeg {
+  int seg, t0, n, p0, slot, first;
+};
+
+// The segment that `rank` others are longer than (of equal ones the first), seg
+// -1 where there is none or it has no chunks. Workgroups start in the order of their numbers, so
 // the longest walks start first, and the CU of one takes a shorter one beside
 // it: general delta, 32 heads, prompts of 336 and 166 chunks, 0.60 -> 0.47 ms.
-// Past 32 segments they go as they come: the order would cost a workgroup a
-// load and a turn a segment before its own rows can be asked for, which with
-// many workgroups of a few chunks is more than it gives. us, ordered / as they
-// come: general delta, 32 heads of 96 x 96, 1200 rows in 40 prompts 188 / 161,
-// 3000 in 40 333 / 307, of 64 x 64, 6000 in 60 364 / 343; 8 heads of 128 x 128,
-// 5000 in 24 133 / 140, of 64 x 64, 8000 in 40 114 / 120.
-PS_DEV int ck_by_length(const int* seq_rows, int S_, int rank) {
-  if (S_ > 32 || S_ == 1) return rank;
+// Up to 64 segments every lane asks for one's row, and what is needed of it goes
+// on in scalar registers: one trip to memory before the walk's own. Segments too
+// short for a chunk (single tokens beside prompts) cost no turn: channel delta, 32
+// heads, 6007 rows in 3 prompts beside 37 tokens, 555 us ordered, 586 as they
+// come. Past 32 with chunks, or 64 in all, they go as they come: a turn a segment
+// in each of many short workgroups is more than the order gives. us, ordered / as
+// they come: general delta, 32 fp32 heads of 96 x 96, 1200 rows in 40 prompts
+// 188 / 161, 3000 in 40 333 / 307, of 64 x 64, 6000 in 60 364 / 343; 8 heads of
+// 64 x 64, 8000 in 40 114 / 120.
+template <int L = 16>
+PS_DEV CkSeg ck_by_length(const int* seq_rows, int S_, int rank) {
   const int lane = threadIdx.x & 63;
-  const int mine = lane < S_ ? seq_rows[4 * lane + 1] : 0;
-  if (rank >= __popcll(__ballot(ck_count(mine) > 0))) return -1;
-  int longer = 0;
-  for (int s = 0; s < S_; ++s) {
-    const int n = __builtin_amdgcn_readlane(mine, s);
-    longer += n > mine || (n == mine && s < lane);
+  CkSeg at;
+  int before = 0;
+  at.seg = rank;
+  if (S_ == 1 || S_ > 64) {
+    at.t0 = seq_rows[4 * rank], at.n = seq_rows[4 * rank + 1];
+    if (ck_count<L>(at.n) == 0) {
+      at.seg = -1;
+      return at;
+    }
+    at.p0 = seq_rows[4 * rank + 2], at.slot = seq_rows[4 * rank + 3];
+    for (int s = lane; s < rank; s += 64)
+      before += ck_count<L>(seq_rows[4 * s + 1]);
+  } else {
+    const int* own = seq_rows + 4 * min(lane, S_ - 1);
+    const int t0 = own[0], n = lane < S_ ? own[1] : 0, p0 = own[2],
+              slot = own[3];
+    const unsigned long long live = __ballot(ck_count<L>(n) > 0);
+    const int count = __popcll(live);
+    if (count <= 32) {
+      if (rank >= count) {
+        at.seg = -1;
+        return at;
+      }
+      int longer = 0;
+      for (unsigned long long left = live; left; left &= left - 1) {
+        const int s = __ffsll(left) - 1;
+        const int other = __builtin_amdgcn_readlane(n, s);
+        longer += other > n || (other == n && s < lane);
+      }
+      at.seg = __ffsll((unsigned long long)__ballot(longer == rank) & live) - 1;
+    } else if ((live >> rank & 1) == 0) {
+      at.seg = -1;
+      return at;
+    }
+    at.t0 = __builtin_amdgcn_readlane(t0, at.seg);
+    at.n = __builtin_amdgcn_readlane(n, at.seg);
+    at.p0 = __builtin_amdgcn_readlane(p0, at.seg);
+    at.slot = __builtin_amdgcn_readlane(slot, at.seg);
+    before = lane < at.seg ? ck_count<L>(n) : 0;
   }
-  return __ffsll((unsigned long long)__ballot(lane < S_ && longer == rank)) -
-         1;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+  at.first = __builtin_amdgcn_readfirstlane(before);
+  return at;
 }
 
 template <typename T, int MODE, int DP>
@@ -573,22 +616,15 @@ __global__ __launch_bounds__(DP * 4 / ck_row_tiles(DP),
   const int run = PART ? blockIdx.x / (S_ * H) / ncb : 0;
   const int rest = blockIdx.x - run * S_ * H * ncb;
   const int hd = rest % H, cb = rest / H % ncb;
-  const int seg = ck_by_length(seq_rows, S_, rest / (H * ncb));
-  if (seg < 0) return;
-  const int sh = seg * H + hd;
-  int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
-  const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  const CkSeg at = ck_by_length(seq_rows, S_, rest / (H * ncb));
+  if (at.seg < 0) return;
+  const int sh = at.seg * H + hd;
+  int t0 = at.t0, n = at.n;
+  const int p0 = at.p0, slot = at.slot;
   const int all = ck_count(n);
-  if (all == 0) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // this segment's first chunk among all
-  int first = 0;
-  for (int s = lane; s < seg; s += 64)
-    first += ck_count(seq_rows[4 * s + 1]);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
-  first = __builtin_amdgcn_readfirstlane(first) - base;  // of this pass
+  int first = at.first - base;  // its first chunk of this pass
   int c0 = max(0, -first);
   int count =
       __builtin_amdgcn_readfirstlane(min(all, cap - first) - c0);
@@ -1619,21 +1655,15 @@ PS_DEV bool ck_walk_wide(const CkWideCall& a, CkWideLds<DP, NW>& lds) {
   const int run = PART ? blockIdx.x / (S_ * H) / ncb : 0;
   const int rest = blockIdx.x - run * S_ * H * ncb;
   const int hd = rest % H, cb = rest / H % ncb;
-  const int seg = ck_by_length(seq_rows, S_, rest / (H * ncb));
-  if (seg < 0) return true;
-  const int sh = seg * H + hd, grp = hd / (H / G);
-  int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
-  const int p0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
+  const CkSeg at = ck_by_length<CK_WIDE>(seq_rows, S_, rest / (H * ncb));
+  if (at.seg < 0) return true;
+  const int sh = at.seg * H + hd, grp = hd / (H / G);
+  int t0 = at.t0, n = at.n;
+  const int p0 = at.p0, slot = at.slot;
   const int all = ck_count<CK_WIDE>(n);
-  if (all == 0) return true;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int first = 0;
-  for (int s = lane; s < seg; s += 64)
-    first += ck_count<CK_WIDE>(seq_rows[4 * s + 1]);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off, 64);
-  first = __builtin_amdgcn_readfirstlane(first) - base;  // of this pass
+  int first = at.first - base;  // its first chunk of this pass
   int c0 = max(0, -first);
   int count =
       __builtin_amdgcn_readfirstlane(min(all, cap - first) - c0);

@@ -734,11 +734,14 @@ def test_recurrence_empty_segments(mode):
 @pytest.mark.parametrize("lens", [
     [33, 16, 0, 33, 70, 1, 16], [17 + i // 9 for i in range(32)],
     [16 + i % 3 for i in range(33)], [17] * 64,
+    [1] * 31 + [20, 0, 40] + [7] * 29 + [33],
+    [1, 0] + [16 + i % 3 for i in range(35)],
     [16 + i % 3 for i in range(65)]])
 def test_recurrence_chunk_order(mode, lens, dtype):
-    """Walks start by length, up to 32 segments: equal lengths, empty and
-    single rows among them, one segment more; values end with their segment,
-    columns of the last workgroup beyond the head's."""
+    """Walks start by length, up to 32 segments of a chunk or more and 64 in
+    all: equal lengths, empty and short segments among them, one segment more;
+    values end with their segment, columns of the last workgroup beyond the
+    head's."""
     rows = _segs(lens, [3 * (i % 2) for i in range(len(lens))])
     x, state, aux, call = _recurrence(mode, 2, 40, 40, rows, dtype)
     rows = torch.tensor(rows, dtype=torch.int32)
