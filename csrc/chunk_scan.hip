@@ -556,17 +556,17 @@ PS_DEV ck_f32x4 ck_token_terms(float f, float x, ck_f32x4 acc, int lane,
 static constexpr int ck_row_tiles(int dp) { return dp <= 64 ? 1 : 2; }
 
 // Waves that a SIMD has registers for: three, since many short segments are
-// more workgroups than two a SIMD hold; two where three would spill (fp32 rows
-// of 128, either delta: 78 and 25 registers). us, two / three: general delta,
-// 32 fp32 heads of 96 x 96, 1200 rows in 40 prompts 161 / 139, 3000 in 40
-// 307 / 285, 4000 in 8 330 / 327.
+// more workgroups than two a SIMD hold; two where three would spill more than
+// one register (fp32 rows of 128, either delta: 78 and 25). us, two / three:
+// general delta, 32 fp32 heads of 96 x 96, 1200 rows in 40 prompts 161 / 139,
+// 3000 in 40 307 / 285, 4000 in 8 330 / 327.
 static constexpr int ck_sweep_waves(int mode, int dp, bool wide) {
   return !wide || dp <= 96 || mode == CK_GLA ? 3 : 2;
 }
 
 // Walks the chunks of one (segment, head) for 16 columns of its state: a wave
-// per 32 rows of it (16 of up to 64), two to four waves. raw [T, H * DV]: S^T r before the
-// read-out's norm.
+// per 32 rows of it (16 of up to 64), two to four waves. raw [T, H * DV]: S^T r
+// before the read-out's norm.
 //
 // The chain from one chunk to the next is what bounds this kernel: a prompt
 // has a few hundred chunks, and heads x DV / 16 workgroups are one or two a
@@ -606,7 +606,9 @@ __global__ __launch_bounds__(DP * 4 / ck_row_tiles(DP),
   constexpr int NW = DP / 16 / RT;       // waves
   constexpr int NQ = (4 + NW - 1) / NW;  // tokens of four a wave takes
   // three waves have two tokens' matrix entries each, and three a SIMD would
-  // spill with the written rows on their own and the last chunk's shares early
+  // spill with the written rows on their own and the last chunk's shares early.
+  // Added behind the removed ones (general delta, widths 65 to 96): the state is
+  // 6.9e-8 from 64-bit results, its rows 1.81e-7
   constexpr bool LEAN = NW == 3;
   constexpr int SET = NW * 64;         // shares of one chunk, float4
   __shared__ ck_f32x4 zx[2 * SET], ox[2 * SET];
@@ -1605,7 +1607,8 @@ __global__ __launch_bounds__(256) void ck_prep_wide_kernel(
 // barrier a chunk does for both.
 // Measured (ssd, 128 heads of 128 x 64, 8192 rows in 2 prompts): 605 us by
 // fp32 products in chunks of 16, 330 with all rows of a tile in one wave (one
-// wave a SIMD: 800 instructions in 5300 cycles), 285 with two.
+// wave a SIMD: 800 instructions in 5300 cycles), 285 with two; the whole call
+// 308, and 297 since infinities take a walk of their own.
 // memory that no kernel under way writes: scalar loads
 #define CK_CONST __attribute__((address_space(4)))
 struct CkWideCall {
@@ -2275,9 +2278,9 @@ static long ck_chunk_floats(int mode, int dp, int H, int G, int L) {
 //     (operands 0.24, walk 0.41, read-out 0.08)
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
 //                                                            5.42 -> 0.55 ms
-//   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.31 ms
+//   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.30 ms
 //   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.07 ms
-//   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.51 ms
+//   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.47 ms
 // From 16 rows on a segment goes this way: one chunk costs about 15 us in
 // three launches, 16 tokens one by one 24 us.
 //
