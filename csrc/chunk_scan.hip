@@ -125,18 +125,17 @@ struct CkSeg {
 };
 
 // The segment that `rank` others are longer than (of equal ones the first), seg
-// -1 where there is none or it has no chunks. Workgroups start in the order of their numbers, so
-// the longest walks start first, and the CU of one takes a shorter one beside
-// it: general delta, 32 heads, prompts of 336 and 166 chunks, 0.60 -> 0.47 ms.
-// Up to 64 segments every lane asks for one's row, and what is needed of it goes
-// on in scalar registers: one trip to memory before the walk's own. Segments too
-// short for a chunk (single tokens beside prompts) cost no turn: channel delta, 32
-// heads, 6007 rows in 3 prompts beside 37 tokens, 555 us ordered, 586 as they
-// come. Past 32 with chunks, or 64 in all, they go as they come: a turn a segment
-// in each of many short workgroups is more than the order gives. us, ordered / as
-// they come: general delta, 32 fp32 heads of 96 x 96, 1200 rows in 40 prompts
-// 188 / 161, 3000 in 40 333 / 307, of 64 x 64, 6000 in 60 364 / 343; 8 heads of
-// 64 x 64, 8000 in 40 114 / 120.
+// -1 where there is none or it has no chunks. Workgroups start in the order of
+// their numbers, so the longest walks start first, and the CU of one takes a
+// shorter one beside it: general delta, 32 heads, prompts of 336 and 166 chunks,
+// 0.60 -> 0.47 ms. Up to 64 segments every lane asks for one's row: one trip to
+// memory before the walk's own. Segments too short for a chunk (single tokens
+// beside prompts) cost no turn: channel delta, 32 heads, 6007 rows in 3 prompts
+// beside 37 tokens, 549 us ordered, 565 as they come. Past 32 with chunks, or 64
+// in all, they go as they come: a turn a segment in each of many short workgroups
+// is more than the order gives. us, ordered / as they come: general delta, 32 fp32
+// heads of 96 x 96, 1200 rows in 40 prompts 188 / 161, 3000 in 40 333 / 307, of
+// 64 x 64, 6000 in 60 364 / 343; 8 heads of 64 x 64, 8000 in 40 114 / 120.
 template <int L = 16>
 PS_DEV CkSeg ck_by_length(const int* seq_rows, int S_, int rank) {
   const int lane = threadIdx.x & 63;
@@ -620,9 +619,16 @@ __global__ __launch_bounds__(DP * 4 / ck_row_tiles(DP),
   const int hd = rest % H, cb = rest / H % ncb;
   const CkSeg at = ck_by_length(seq_rows, S_, rest / (H * ncb));
   if (at.seg < 0) return;
-  const int sh = at.seg * H + hd;
-  int t0 = at.t0, n = at.n;
-  const int p0 = at.p0, slot = at.slot;
+  // the same in all lanes, which is not seen through the cases of ck_by_length: in
+  // scalar registers for the loads' addresses (channel delta, 32 fp32 heads, 6007
+  // rows in 3 prompts beside 37 tokens 610 -> 585 us). The three-term walk has none
+  // left for them and keeps them as they are (32 heads of 96 x 40, 2000 rows in 20
+  // prompts 49 us, 53 so)
+  const int sh = __builtin_amdgcn_readfirstlane(at.seg) * H + hd;
+  int t0 = __builtin_amdgcn_readfirstlane(at.t0);
+  int n = __builtin_amdgcn_readfirstlane(at.n);
+  const int p0 = __builtin_amdgcn_readfirstlane(at.p0);
+  const int slot = __builtin_amdgcn_readfirstlane(at.slot);
   const int all = ck_count(n);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
