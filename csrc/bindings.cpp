@@ -74,6 +74,15 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
                    int M, int N, int K, long x_stride, hipStream_t stream);
 int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
                     int K, long x_stride, hipStream_t stream);
+int ps_skinny_norm_gated(void* out, void* res_out, const void* x,
+                         const void* res, const void* nw, const void* w,
+                         int M, int N, int K, float eps, hipStream_t stream);
+int ps_skinny_rope(void* out, void* res_out, const void* x, long x_stride,
+                   const void* res, const void* nw, const void* w, int M,
+                   int N, int K, float eps, const void* positions,
+                   const void* cos_sin, const void* slots, void* k_cache,
+                   void* v_cache, int QH, int KH, int HD, int BS, int kv_fp8,
+                   hipStream_t stream);
 int ps_gemm8p_splits(int M, int N, int K);
 int ps_gemm8p(void* out_bf16, void* ws, const void* x, const void* w, int M,
               int N, int K, long x_stride, hipStream_t stream);
@@ -379,6 +388,85 @@ void skinny_gated(at::Tensor out, at::Tensor x, at::Tensor w) {
               " K=", K);
 }
 
+// what the norm before a product needs: dense rows
+static void check_norm(const at::Tensor& x, const c10::optional<at::Tensor>& res,
+                       const at::Tensor& nw,
+                       const c10::optional<at::Tensor>& res_out) {
+  CHECK_GPU_BF16(x);
+  CHECK_GPU_BF16(nw);
+  TORCH_CHECK(nw.numel() == x.size(1), "norm width mismatch");
+  TORCH_CHECK(res.has_value() == res_out.has_value(),
+              "a residual comes with a buffer for its sum");
+  if (res.has_value()) {
+    CHECK_GPU_BF16(*res);
+    CHECK_GPU_BF16(*res_out);
+    TORCH_CHECK(res->sizes() == x.sizes() && res_out->sizes() == x.sizes(),
+                "residual size mismatch");
+    TORCH_CHECK(res->data_ptr() != res_out->data_ptr() &&
+                    x.data_ptr() != res_out->data_ptr(),
+                "the sum needs a buffer of its own");
+  }
+}
+
+void skinny_norm_gated(at::Tensor out, c10::optional<at::Tensor> res_out,
+                       at::Tensor x, c10::optional<at::Tensor> res,
+                       at::Tensor nw, at::Tensor w, double eps) {
+  CHECK_GPU_BF16(out);
+  CHECK_GPU_BF16(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1),
+              "K mismatch");
+  check_norm(x, res, nw, res_out);
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  TORCH_CHECK(out.numel() == (long)M * (N / 2), "out size mismatch");
+  const int rc = ps_skinny_norm_gated(
+      out.data_ptr(), res ? res_out->data_ptr() : nullptr, x.data_ptr(),
+      res ? res->data_ptr() : nullptr, nw.data_ptr(), w.data_ptr(), M, N, K,
+      (float)eps, current_stream());
+  TORCH_CHECK(rc == 0, "unsupported normed skinny gemm M=", M, " N=", N,
+              " K=", K);
+}
+
+void skinny_rope(at::Tensor out, c10::optional<at::Tensor> res_out,
+                 at::Tensor x, c10::optional<at::Tensor> res,
+                 c10::optional<at::Tensor> nw, at::Tensor w, double eps,
+                 at::Tensor positions, at::Tensor cos_sin, at::Tensor slots,
+                 at::Tensor k_cache, at::Tensor v_cache, int64_t q_heads) {
+  CHECK_GPU_BF16(out);
+  CHECK_GPU_BF16(w);
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
+                  x.dim() == 2 && x.stride(1) == 1,
+              "x must be bf16 rows");
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == x.size(1), "K mismatch");
+  if (nw.has_value()) check_norm(x, res, *nw, res_out);
+  TORCH_CHECK(nw.has_value() || !res.has_value(), "a residual needs a norm");
+  CHECK_GPU_DTYPE(positions, at::kInt);
+  CHECK_GPU_DTYPE(cos_sin, at::kFloat);
+  CHECK_GPU_DTYPE(slots, at::kLong);
+  const int kv_fp8 = cache_fp8(k_cache);
+  TORCH_CHECK(cache_fp8(v_cache) == kv_fp8 &&
+                  v_cache.sizes() == k_cache.sizes(),
+              "caches differ");
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  const int KH = (int)k_cache.size(1), BS = (int)k_cache.size(2),
+            HD = (int)k_cache.size(3);
+  TORCH_CHECK(out.numel() == (long)M * N, "out size mismatch");
+  TORCH_CHECK(positions.numel() == M && slots.numel() == M, "row mismatch");
+  TORCH_CHECK(cos_sin.size(-1) == HD, "rotary width mismatch");
+  TORCH_CHECK((((size_t)cos_sin.data_ptr() | (size_t)k_cache.data_ptr() |
+                (size_t)v_cache.data_ptr() | (size_t)out.data_ptr()) &
+               15) == 0,
+              "rows must be aligned to 16 bytes");
+  const int rc = ps_skinny_rope(
+      out.data_ptr(), res ? res_out->data_ptr() : nullptr, x.data_ptr(),
+      x.stride(0), res ? res->data_ptr() : nullptr,
+      nw ? nw->data_ptr() : nullptr, w.data_ptr(), M, N, K, (float)eps,
+      positions.data_ptr(), cos_sin.data_ptr(), slots.data_ptr(),
+      k_cache.data_ptr(), v_cache.data_ptr(), (int)q_heads, KH, HD, BS,
+      kv_fp8, current_stream());
+  TORCH_CHECK(rc == 0, "unsupported rotary skinny gemm M=", M, " N=", N,
+              " K=", K, " head_dim=", HD);
+}
+
 void rms_norm_fp8(at::Tensor out_q, at::Tensor scales, at::Tensor x,
                   at::Tensor residual, at::Tensor w, double eps,
                   int64_t fused) {
@@ -528,6 +616,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "8-phase deep-pipelined bf16 GEMM (out = x @ w.T)");
   m.def("skinny_gemm", &skinny_gemm,
         "MFMA GEMM for decode-shaped (M<=256) projections");
+  m.def("skinny_norm_gated", &skinny_norm_gated,
+        "Residual sum, RMSNorm, skinny GEMM and gated activation");
+  m.def("skinny_rope", &skinny_rope,
+        "(Residual sum, RMSNorm,) skinny GEMM, RoPE and KV append");
   m.def("skinny_gated", &skinny_gated,
         "silu(x @ wg.T) * (x @ wu.T) of up to 16 rows, w = [wg; wu]");
   m.def("kv_dequant", &kv_dequant, "Row-wise int8 KV dequantization");

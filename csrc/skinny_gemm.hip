@@ -3,15 +3,23 @@
 //
 // Why it exists: the library's tiles for the products of a decode batch leave
 // the read of W, which bounds them, at a third to a half of the rate that memory
-// gives. Up to 16 rows (8 of a W of more than 32768) go without splits; more go
-// by the tiled form, or by the short form where a workgroup's range of K is
+// gives. Up to 16 rows go without splits (x in LDS where it fits, also with the
+// norm before and the activation or rotary embedding behind the products); more
+// go by the tiled form, or by the short form where a workgroup's range of K is
 // short or the tiles leave CUs waiting. Figures stand at each.
 // mfma_f32_16x16x32_bf16; operand k-pattern as verified in
 // csrc/tools/mfma_probe.hip.
 #include "ps_common.h"
+#include <algorithm>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 ps_gbf16x8;
 typedef __attribute__((ext_vector_type(4))) float ps_gf32x4;
+
+// Waves of skinny_lds_kernel, and the most entries of x that it takes: with the
+// norm (their fp32 values stay in registers between its two passes) and without.
+#define SL_WAVES 16
+#define SL_NORM_X 16384
+#define SL_X 65536
 
 PS_DEV ps_gbf16x8 ps_as_gbf16(ps_bf16x8 u) {
   union {
@@ -22,18 +30,25 @@ PS_DEV ps_gbf16x8 ps_as_gbf16(ps_bf16x8 u) {
   return v.bf;
 }
 
-// Up to 16 rows of x (8 of a W of more than 32768): a workgroup owns 16 rows of W
-// and all of K, its NW waves take every NW-th 128-byte piece of them, UC pieces
-// in flight each, and add up in LDS at the end: no second kernel and no partial
-// sums in memory. W goes from memory straight into left operands, x from the
-// caches into right ones (rows past the last read as zeros without an access).
-// Bound by the read of W, at few rows of W by its latency: 1 x 4096 x 4096 in
-// 10.3 us (17.4 with the split kernel, its merge included), 1 x 28672 x 4096 in
-// 46 (79; 5.1 TB/s), 1 x 2048 x 2048 in 5.0 (13.1). Reading x costs as many
-// load instructions as reading W: 16 rows of it make the wide one 68 us.
+// Up to 16 rows of x: a workgroup owns 16 rows of W and all of K, its NW waves
+// take every NW-th 128-byte piece of them, UC pieces in flight each, and add up in
+// LDS at the end: no second kernel and no partial sums in memory. W and x go
+// straight into operands; what lies past the last row of x or the last piece reads
+// as zero without an access (W's last piece again instead: 4096 x 4096 10.8 us, 8.7
+// so). Bound by the read of W, at few rows of W by its latency. Reading x costs as
+// many load instructions as reading W: where x fits in LDS and W is more than a
+// few MB the form below takes over.
 // GATED: W holds N / 2 gate rows, then as many up rows; a workgroup takes eight
 // of each and writes silu(gate) up, both rounded to bf16 first: [M, N / 2].
-template <int UC, int NW, bool GATED>
+// HALF: eight rows of W a workgroup, two pieces of each at a time. Left rows 8 to
+// 15 are the second piece of rows 0 to 7, right columns 8 to 15 that piece of up
+// to eight rows of x; the two diagonal blocks of the product add up, the others
+// are nothing. Where 16 rows a workgroup leave half of the CUs without one (us at
+// one row, 16 rows / 8 / the library: 2048 x 2048 5.4 / 4.5 / 11.0, 2048 x 8192
+// 12.0 / 8.6 / 12.7, 1024 x 4096 7.4 / 5.4 / 14.4).
+// FAR: W by its addresses, where 31-bit offsets do not reach its up rows or it is
+// not aligned to 16 bytes.
+template <int UC, int NW, bool GATED, bool HALF, bool FAR>
 __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
     unsigned short* __restrict__ out, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w, int M, int N, int K, int x_stride) {
@@ -41,25 +56,41 @@ __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
   __shared__ __align__(16) float s_sum[NW][16 * PN];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int rc = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (GATED ? 8 : 16);
-  const int nc = K / 64;  // pieces
-  const int wrow = GATED && rc >= 8 ? N / 2 + n0 + rc - 8 : n0 + rc;
-  const unsigned short* wp = w + (long)wrow * K + g * 8;
+  constexpr int PC = HALF ? 128 : 64;  // columns of a step
+  // rows of W, columns of the result
+  constexpr int NR = HALF ? 8 : 16, NO = GATED ? NR / 2 : NR;
+  const int n0 = blockIdx.x * NO;
+  const int nc = K / PC;  // steps
+  const int r8 = HALF ? rc & 7 : rc;
+  const int k0 = g * 8 + (HALF ? (rc >> 3) * 64 : 0);
+  const int wrow = r8 >= NO ? N / 2 + r8 - NO : r8;
+  const unsigned short* wp = w + (long)(n0 + wrow) * K + k0;
+  // what lies past the end reads as zero without an access
+  const unsigned int off = 0x80000000u;
+  const auto wr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(w + (long)n0 * K), 0, (int)off - 1, 0x00020000);
   const auto xr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)x, 0, ((M - 1) * x_stride + K) * 2, 0x00020000);
+  const unsigned int wo = (unsigned int)(wrow * K + k0) * 2;
   const unsigned int xo =
-      rc < M ? (unsigned int)(rc * x_stride + g * 8) * 2 : 0x80000000u;
+      r8 < M ? (unsigned int)(r8 * x_stride + k0) * 2 : off;
   ps_gf32x4 acc = {0.f, 0.f, 0.f, 0.f};
   ps_gbf16x8 wf[UC][2], xf[UC][2];
-  // pieces past the end repeat the last one and are not multiplied
   auto load = [&](int u, int c) {
-    const int k = min(c, nc - 1) * 64;
+    const unsigned int o = c < nc ? 0u : off;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      wf[u][h] = *(const ps_gbf16x8*)(wp + k + 32 * h);
+      const unsigned int k = c * (2 * PC) + 64 * h;
+      if constexpr (FAR)
+        wf[u][h] =
+            *(const ps_gbf16x8*)(wp + min(c, nc - 1) * PC + 32 * h);
+      else
+        wf[u][h] = __builtin_bit_cast(
+            ps_gbf16x8,
+            __builtin_amdgcn_raw_buffer_load_b128(wr, wo | o, k, 0));
       xf[u][h] = __builtin_bit_cast(
           ps_gbf16x8,
-          __builtin_amdgcn_raw_buffer_load_b128(xr, xo, k * 2 + 64 * h, 0));
+          __builtin_amdgcn_raw_buffer_load_b128(xr, xo | o, k, 0));
     }
   };
   const int w0 = __builtin_amdgcn_readfirstlane(wave);
@@ -68,7 +99,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
   for (int c = w0; c < nc; c += NW * UC) {
 #pragma unroll
     for (int u = 0; u < UC; ++u) {
-      if (c + NW * u < nc) {
+      if (!FAR || c + NW * u < nc) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
           acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][h], xf[u][h],
@@ -86,22 +117,292 @@ __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
 #pragma unroll
     for (int k = 0; k < NW; ++k)
       v += *(const ps_gf32x4*)(&s_sum[k][m * PN + n]);
+    if constexpr (HALF) {
+#pragma unroll
+      for (int k = 0; k < NW; ++k)
+        v += *(const ps_gf32x4*)(
+            &s_sum[k][((m & 7) + 8) * PN + (n & 7) + 8]);
+    }
     if constexpr (GATED) {
-      // the quad of up columns is two lanes on
+      // the quad of up columns is NO / 4 lanes on
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float gv = ps_bf16_to_f32(ps_f32_to_bf16(v[r]));
         const float uv = ps_bf16_to_f32(
-            ps_f32_to_bf16(__shfl_down(v[r], 2, 64)));
+            ps_f32_to_bf16(__shfl_down(v[r], NO / 4, 64)));
         v[r] = gv / (1.f + __expf(-gv)) * uv;
       }
     }
-    if (m < M && (!GATED || n < 8))
+    if (m < M && n < NO)
       *(uint2*)(out + (long)m * (GATED ? N / 2 : N) + n0 + n) = make_uint2(
           (unsigned int)ps_f32_to_bf16(v[0]) |
               ((unsigned int)ps_f32_to_bf16(v[1]) << 16),
           (unsigned int)ps_f32_to_bf16(v[2]) |
               ((unsigned int)ps_f32_to_bf16(v[3]) << 16));
+  }
+}
+
+// What skinny_lds_kernel reads and writes.
+struct SlArgs {
+  unsigned short* out;      // [M, N]; gated [M, N / 2]
+  unsigned short* res_out;  // [M, K] = x + res, where there is a res
+  const unsigned short *x, *res, *nw, *w;  // [M, K], [M, K], [K], [N, K]
+  int M, N, K;
+  int apart;                // rows between the two halves of a tile
+  long x_stride;            // K with the norm
+  float eps;
+  // rotary form
+  const int* positions;     // [M]
+  const float* cos_sin;     // [.., HD]
+  const long* slots;        // [M]
+  void *kc, *vc;            // [blocks, KH, BS, HD]
+  int QH, KH, HD, BS;
+};
+
+// Up to 16 rows of x that LDS holds, with what stands around the products that
+// begin a layer's two halves:
+//   NORM      x <- x + res,  y = x rsqrt(mean x^2 + eps) nw; else y = x
+//             out = y W^T, then
+//   SL_GATED  silu(gate) up
+//   SL_ROPE   the rotary embedding of queries and keys, and keys and values into
+//             the paged cache; W's rows are query heads, key heads, value heads
+// A workgroup a CU reads (and normalises) all of x for itself while its first
+// pieces of W are on their way, and walks tiles of 16 rows of W, every
+// gridDim.x-th; its waves take every NW-th 128-byte piece of a tile, UC pieces in
+// flight each across the tiles' ends. x costs a read from the caches a CU instead
+// of one a tile, the norm and the rotary embedding no launches of their own
+// (3.5 us each and up). The waves' sums of a tile are added by one of them while
+// the others go on. Roundings are those of the separate kernels; x + res goes to
+// a buffer of its own, since other workgroups still read res.
+// Bound by the read of W. us, distinct weights, with the launches it replaces:
+//   norm, 28672 x 4096, silu   1 row 41.3 (before 47.4), 4 rows 43.9 (50.1)
+//   norm, 16384 x 2048, silu   1 row 14.1 (17.9), 8 rows 16.8 (20.1)
+//   norm, 6144 x 4096, rotary  1 row 14.5 (20.6), 4 rows 16.7 (20.6)
+//   norm, 3072 x 2048, rotary  1 row 6.9 (11.1), 8 rows 9.3 (12.4)
+//   28672 x 4096, silu         8 rows 42.6 (52.1), 16 rows 44.9 (60.8; 5.3 TB/s)
+//   6144 x 4096                8 rows 13.2 (15.0), 16 rows 14.4 (18.1)
+// More workgroups a CU read and normalise x more often (28672 x 4096 with the norm,
+// one row 41.3, two 40.7, four rows 43.9 and 46.1, all tiles at once 63), fewer
+// pieces in flight do not cover a tile's end (one 42.3, four 42.0 at one row).
+enum { SL_PLAIN, SL_GATED, SL_ROPE };
+template <int EPI, bool NORM, typename KVT>
+__global__ __launch_bounds__(SL_WAVES * 64) void skinny_lds_kernel(SlArgs a) {
+  constexpr int UC = 2, NW = SL_WAVES;
+  constexpr int PN = 20;  // pitch of a row of sums
+  constexpr int NT = NW * 64;
+  constexpr int VECS = NORM ? SL_NORM_X / 8 : SL_X / 8;
+  constexpr int VP = VECS / NT;  // 16-byte pieces of x a thread has
+  // sums of a tile: with two sets a tile has one barrier, if there is room
+  constexpr int SETS = NORM ? 2 : 1;
+  __shared__ __align__(16) float s_sum[SETS][NW][16 * PN];
+  __shared__ float s_part[NORM ? VECS / 8 : 1], s_inv[16];
+  __shared__ __align__(16) unsigned short s_x[VECS * 8 + 128];  // [M][K + 8]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rc = lane & 15, g = lane >> 4;
+  const int M = a.M, N = a.N, K = a.K, V = K / 8, total = M * V;
+
+  // x first: loads land in the order in which they were asked for
+  ps_bf16x8 xv[VP], rv[VP], nv[VP];
+  int at[VP];  // where a piece goes in s_x
+#pragma unroll
+  for (int u = 0; u < VP; ++u) {
+    const int i = u * NT + tid;
+    if (i < total) {
+      const int m = i / V;
+      at[u] = i * 8 + m * 8;
+      if constexpr (NORM) {
+        xv[u] = *(const ps_bf16x8*)(a.x + i * 8);
+        if (a.res) rv[u] = *(const ps_bf16x8*)(a.res + i * 8);
+        nv[u] = *(const ps_bf16x8*)(a.nw + (i - m * V) * 8);
+      } else {
+        xv[u] = *(const ps_bf16x8*)(a.x + (long)m * a.x_stride +
+                                    (i - m * V) * 8);
+      }
+    }
+  }
+  const int om = lane >> 2, on = (lane & 3) * 4;  // of the last step
+  int pos = 0;
+  long slot = -1;
+  if constexpr (EPI == SL_ROPE) {
+    if (om < M) {
+      pos = a.positions[om];
+      slot = a.slots[om];
+    }
+  }
+  // a tile's rows of W: eight, and the eight that belong to them
+  const int nc = K / 64;  // pieces of a row
+  const int steps = (nc + NW - 1) / NW;
+  const int per = EPI == SL_ROPE ? a.HD / 16 : 1;
+  const int tiles = N / 16;
+  const int apart = a.apart;
+  auto row0 = [&](int tile) {
+    return EPI == SL_ROPE ? tile / per * a.HD + tile % per * 8
+                          : tile * (apart == 8 ? 16 : 8);
+  };
+  // what lies past the end reads as zero without an access
+  const unsigned int off = 0x80000000u;
+  const unsigned int wo =
+      (unsigned int)(((rc & 7) + (rc >> 3) * apart) * K + g * 8) * 2;
+  ps_gbf16x8 wf[UC][2];
+  int lt = blockIdx.x, lj = 0;  // the next step to ask for
+  auto load = [&](int u) {
+    const int c = wave + NW * lj;
+    const unsigned int o = c < nc && lt < tiles ? 0u : off;
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.w + (long)row0(min(lt, tiles - 1)) * K), 0, (int)off - 1,
+        0x00020000);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      wf[u][h] = __builtin_bit_cast(
+          ps_gbf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                          wr, wo | o, c * 128 + 64 * h, 0));
+    if (++lj == steps) lj = 0, lt += gridDim.x;
+  };
+#pragma unroll
+  for (int u = 0; u < UC; ++u) load(u);
+  __builtin_amdgcn_sched_barrier(0);
+
+  if constexpr (!NORM) {
+#pragma unroll
+    for (int u = 0; u < VP; ++u)
+      if (u * NT + tid < total) *(ps_bf16x8*)(s_x + at[u]) = xv[u];
+  } else {
+    float f[VP][8];
+#pragma unroll
+    for (int u = 0; u < VP; ++u) {
+      const int i = u * NT + tid;
+      float ss = 0.f;
+      if (i < total) {
+        ps_bf16x8 sv;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float y = ps_bf16_to_f32(xv[u][j]);
+          if (a.res) y += ps_bf16_to_f32(rv[u][j]);
+          f[u][j] = y;
+          ss += y * y;
+          sv[j] = ps_f32_to_bf16(y);
+        }
+        if (a.res && blockIdx.x == 0) *(ps_bf16x8*)(a.res_out + i * 8) = sv;
+      }
+      // eight lanes have 64 columns of one row
+#pragma unroll
+      for (int d = 1; d < 8; d <<= 1) ss += __shfl_xor(ss, d, 64);
+      if ((lane & 7) == 0 && i < total) s_part[i / 8] = ss;
+    }
+    __syncthreads();
+    for (int m = wave; m < M; m += NW) {
+      float t = 0.f;
+      for (int i = lane; i < nc; i += 64) t += s_part[m * nc + i];
+      t = ps_group_sum<64>(t);
+      if (lane == 0) s_inv[m] = rsqrtf(t / (float)K + a.eps);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < VP; ++u) {
+      const int i = u * NT + tid;
+      if (i < total) {
+        const float inv = s_inv[i / V];
+        ps_bf16x8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          o[j] = ps_f32_to_bf16(f[u][j] * inv * ps_bf16_to_f32(nv[u][j]));
+        *(ps_bf16x8*)(s_x + at[u]) = o;
+      }
+    }
+  }
+  // a tile's angles, on their way during its products
+  ps_gf32x4 cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
+  auto angles = [&](int tile) {
+    if constexpr (EPI == SL_ROPE) {
+      if (om < M && tile / per < a.QH + a.KH) {
+        const float* c =
+            a.cos_sin + (long)pos * a.HD + tile % per * 8 + (on & 7);
+        cs = *(const ps_gf32x4*)c;
+        sn = *(const ps_gf32x4*)(c + a.HD / 2);
+      }
+    }
+  };
+  angles(blockIdx.x);
+  __syncthreads();
+
+  // rows past the last repeat it: their results are left out
+  const unsigned short* xp = s_x + min(rc, M - 1) * (K + 8) + g * 8;
+  ps_gf32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  int tile = blockIdx.x, j = 0, set = 0, turn = 0;
+  // The sums of a tile. acc[r]: row rc of x, row 4 g + r of the tile's.
+  auto finish = [&] {
+    if (SETS == 1 && tile != (int)blockIdx.x) __syncthreads();
+    *(ps_gf32x4*)(&s_sum[set][wave][rc * PN + 4 * g]) = acc;
+    __syncthreads();
+    if (wave != turn) return;
+    ps_gf32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < NW; ++k)
+      v += *(const ps_gf32x4*)(&s_sum[set][k][om * PN + on]);
+    ps_gf32x4 z;  // the eight that belong to these
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      v[r] = ps_bf16_to_f32(ps_f32_to_bf16(v[r]));
+      z[r] = __shfl_xor(v[r], 2, 64);
+    }
+    const int head = tile / per;
+    if constexpr (EPI == SL_GATED) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = v[r] / (1.f + __expf(-v[r])) * z[r];
+    } else if constexpr (EPI == SL_ROPE) {
+      if (head < a.QH + a.KH) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[r] = on < 8 ? v[r] * cs[r] - z[r] * sn[r]
+                        : v[r] * cs[r] + z[r] * sn[r];
+      }
+    }
+    if (om >= M || (EPI == SL_GATED && on >= 8)) return;
+    unsigned short e[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) e[r] = ps_f32_to_bf16(v[r]);
+    const int col = row0(tile) + (on < 8 ? on : apart + on - 8);
+    *(uint2*)(a.out + (long)om * (EPI == SL_GATED ? N / 2 : N) + col) =
+        make_uint2((unsigned int)e[0] | ((unsigned int)e[1] << 16),
+                   (unsigned int)e[2] | ((unsigned int)e[3] << 16));
+    if constexpr (EPI == SL_ROPE) {
+      const int h = head - a.QH;
+      if (h < 0 || slot < 0) return;
+      const bool isv = h >= a.KH;
+      typename ps_kv_traits<KVT>::vec4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[r] = ps_kv_traits<KVT>::from_f32(ps_bf16_to_f32(e[r]));
+      const long row =
+          (slot / a.BS * a.KH + (isv ? h - a.KH : h)) * a.BS + slot % a.BS;
+      *(typename ps_kv_traits<KVT>::vec4*)((KVT*)(isv ? a.vc : a.kc) +
+                                           row * a.HD + col - head * a.HD) = o;
+    }
+  };
+  while (tile < tiles) {
+#pragma unroll
+    for (int u = 0; u < UC; ++u) {
+      if (tile >= tiles) break;
+      const int c = wave + NW * j;
+      if (c < nc) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              wf[u][h], *(const ps_gbf16x8*)(xp + c * 64 + 32 * h), acc, 0, 0,
+              0);
+      }
+      load(u);
+      if (++j == steps) {
+        finish();
+        acc = {0.f, 0.f, 0.f, 0.f};
+        j = 0;
+        tile += gridDim.x;
+        set ^= SETS - 1;
+        turn = turn + 1 == NW ? 0 : turn + 1;
+        if (tile < tiles) angles(tile);
+      }
+    }
   }
 }
 
@@ -475,50 +776,153 @@ static PsSkinnyPlan ps_skinny_plan(int M, int N, int K) {
   return {wide ? PS_WIDE : PS_NARROW, splits[wide]};
 }
 
-// Whether the kernel without splits takes it; its byte offsets are 31 bits.
-// More than 8 rows reread x too often where the other form needs no splits
-// (N > 32768; us, this / the tiles, distinct weights: 16 x 128256 x 4096 283 / 183,
-// 16 x 128256 x 2048 151 / 101, 16 x 51200 x 2560 82 / 66).
-static bool ps_skinny_rows(int M, int N, int K, long x_stride) {
-  return (M <= 8 || (M <= 16 && N <= 32768)) && x_stride >= 0 &&
-         (M - 1) * x_stride + K < (1L << 30);
+// Whether skinny_lds_kernel has room for x and offsets for a tile of W.
+static bool ps_skinny_lds_fits(int M, int N, int K, long x_stride,
+                               const void* x, const void* w, bool norm) {
+  return M >= 1 && M <= 16 && (long)M * K <= (norm ? SL_NORM_X : SL_X) &&
+         N >= 64 && N % 64 == 0 && K >= 64 && K % 64 == 0 &&
+         (long)(N + 32) * K < 1L << 31 && x_stride % 8 == 0 &&
+         (((size_t)x | (size_t)w) & 15) == 0;
+}
+
+template <int EPI, bool NORM, typename KVT = unsigned short>
+static void ps_skinny_lds_go(const SlArgs& a, hipStream_t stream) {
+  skinny_lds_kernel<EPI, NORM, KVT>
+      <<<std::min(a.N / 16, 256), SL_WAVES * 64, 0, stream>>>(a);
+}
+
+// Whether a kernel without splits takes it: up to 8 rows, up to 16 where W has no
+// more than 32768 rows or LDS has room for x. More rows reread x too often where
+// the other form needs no splits (N > 32768; us, rows kernel / tiles, distinct
+// weights: 16 x 128256 x 4096 283 / 183, 16 x 51200 x 2560 82 / 66).
+static bool ps_skinny_rows(int M, int N, int K, long x_stride, const void* x,
+                           const void* w) {
+  return (M <= 8 || (M <= 16 && N <= 32768) ||
+          ps_skinny_lds_fits(M, N, K, x_stride, x, w, false)) &&
+         x_stride >= 0 && (M - 1) * x_stride + K < (1L << 30);
 }
 
 template <bool GATED>
 static void ps_skinny_rows_go(void* out, const void* x, const void* w, int M,
                               int N, int K, long x_stride,
                               hipStream_t stream) {
-#define PS_SR(UC, NW)                                                       \
-  skinny_rows_kernel<UC, NW, GATED><<<N / 16, NW * 64, 0, stream>>>(        \
-      (unsigned short*)out, (const unsigned short*)x,                       \
-      (const unsigned short*)w, M, N, K, (int)x_stride)
-  // long rows: four pieces in flight a wave, else a piece and more waves (us
-  // at one row, 16 waves of one piece against 8 of four: 2048 x 2048 5.0 /
-  // 6.3, 16384 x 2048 16.5 / 20.8, 28672 x 4096 46.2 / 51.6, 4096 x 14336
-  // 28.0 / 25.2). Enough workgroups to fill the chip on short rows want smaller
-  // ones, the more so where 16 waves do not share out the pieces evenly (16 / 8
-  // waves of one piece: 50304 x 768 22.4 / 18.3, 65536 x 1024 33.8 / 27.3, 51200 x
-  // 2560 53.3 / 50.4, 16384 x 2048 17.1 / 16.8; 28672 x 4096 47.0 / 48.8, 18944 x
-  // 3584 29.8 / 31.2, 8192 x 1024 5.7 / 6.2)
-  if (K > 4096)
-    PS_SR(4, 8);
-  else if (N >= 12288 && K <= 3072)
-    PS_SR(1, 8);
+#define PS_SR(UC, NW, HALF, FAR)                                            \
+  skinny_rows_kernel<UC, NW, GATED, HALF, FAR>                              \
+      <<<N / (HALF ? 8 : 16), NW * 64, 0, stream>>>(                        \
+          (unsigned short*)out, (const unsigned short*)x,                   \
+          (const unsigned short*)w, M, N, K, (int)x_stride)
+  if (((size_t)w & 15) != 0 || (GATED && (long)(N + 32) * K >= 1L << 31)) {
+    PS_SR(1, 16, false, true);
+    return;
+  }
+  // 16 rows a workgroup leave half of the CUs without one: eight
+  if (M <= 8 && N <= 2048 && K % 128 == 0) {
+    // us at one row, a step in flight / two: 2048 x 2048 4.5 / 4.5, 512 x 1024
+    // 3.2 / 3.5, 2048 x 4096 6.4 / 5.8, 2048 x 14336 13.5 / 12.7
+    if (K <= 2048)
+      PS_SR(1, 8, true, false);
+    else
+      PS_SR(2, 8, true, false);
+    return;
+  }
+  // Reading x into LDS first takes longer than a short read of W beside it (us at
+  // one row and 16, from memory / from LDS: 4096 x 1024 4.1 / 4.5 and 4.6 / 4.7, 8192
+  // x 768 5.2 / 5.9 and 5.8 / 6.0, 12288 x 768 6.8 / 6.5 and 7.3 / 6.8, 3072 x 2048
+  // 5.6 / 5.3 and 6.3 / 6.3)
+  if ((K >= 2048 || N >= 12288) &&
+      ps_skinny_lds_fits(M, N, K, x_stride, x, w, false)) {
+    SlArgs a = {};
+    a.out = (unsigned short*)out;
+    a.x = (const unsigned short*)x;
+    a.w = (const unsigned short*)w;
+    a.M = M, a.N = N, a.K = K, a.x_stride = x_stride;
+    // Tiles of 16 rows of W side by side, or 8 and the 8 that are N / 2 behind:
+    // 16 rows a power of two apart and 16 KB or more long come from few channels
+    // of memory (us at one row: 4096 x 8192 17.0 / 15.2, 28672 x 8192 89 / 81,
+    // 12288 x 4096 19.8 / 19.9, 28672 x 4096 41.2 / 42.0)
+    a.apart = GATED || (K >= 8192 && K % 4096 == 0) ? N / 2 : 8;
+    ps_skinny_lds_go<GATED ? SL_GATED : SL_PLAIN, false>(a, stream);
+    return;
+  }
+  // us, 8 waves / 16: 16 rows of 4096 x 8192 17.5 / 19.4, of 8192 x 8192 36.6 /
+  // 34.0, 8 rows of 28672 x 8192 104 / 93, one row of 8192 x 1024 5.6 / 6.5
+  if (K < 2048 || (M > 8 && N <= 4096))
+    PS_SR(1, 8, false, false);
   else
-    PS_SR(1, 16);
+    PS_SR(1, 16, false, false);
 #undef PS_SR
 }
 
 extern "C" {
 
-
 // out [M, N / 2] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu]; -1: not built
 int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
                     int K, long x_stride, hipStream_t stream) {
   if (M < 1 || N < 64 || K < 64 || N % 64 != 0 || K % 64 != 0 ||
-      !ps_skinny_rows(M, N, K, x_stride))
+      (M > 8 && N > 32768) || !ps_skinny_rows(M, N, K, x_stride, x, w))
     return -1;
   ps_skinny_rows_go<true>(out, x, w, M, N, K, x_stride, stream);
+  return 0;
+}
+
+// out [M, N / 2] = silu(y Wg^T) * (y Wu^T), y = rms_norm(x + res) nw, res_out =
+// x + res (no res: y = rms_norm(x) nw); -1: not built
+int ps_skinny_norm_gated(void* out, void* res_out, const void* x,
+                         const void* res, const void* nw, const void* w,
+                         int M, int N, int K, float eps, hipStream_t stream) {
+  if (!ps_skinny_lds_fits(M, N, K, K, x, w, true)) return -1;
+  SlArgs a = {};
+  a.out = (unsigned short*)out;
+  a.res_out = (unsigned short*)res_out;
+  a.x = (const unsigned short*)x;
+  a.res = (const unsigned short*)res;
+  a.nw = (const unsigned short*)nw;
+  a.w = (const unsigned short*)w;
+  a.M = M, a.N = N, a.K = K, a.apart = N / 2, a.x_stride = K, a.eps = eps;
+  ps_skinny_lds_go<SL_GATED, true>(a, stream);
+  return 0;
+}
+
+// out [M, N]: query heads, key heads, value heads of y W^T, the first two rotated,
+// the last two in the cache, y as above; without nw y is x. -1: not built
+int ps_skinny_rope(void* out, void* res_out, const void* x, long x_stride,
+                   const void* res, const void* nw, const void* w, int M,
+                   int N, int K, float eps, const void* positions,
+                   const void* cos_sin, const void* slots, void* k_cache,
+                   void* v_cache, int QH, int KH, int HD, int BS, int kv_fp8,
+                   hipStream_t stream) {
+  if (HD < 16 || HD % 16 != 0 || N != (QH + 2 * KH) * HD ||
+      !ps_skinny_lds_fits(M, N, K, x_stride, x, w, nw != nullptr))
+    return -1;
+  const SlArgs a = {(unsigned short*)out,
+                    (unsigned short*)res_out,
+                    (const unsigned short*)x,
+                    (const unsigned short*)res,
+                    (const unsigned short*)nw,
+                    (const unsigned short*)w,
+                    M,
+                    N,
+                    K,
+                    HD / 2,
+                    x_stride,
+                    eps,
+                    (const int*)positions,
+                    (const float*)cos_sin,
+                    (const long*)slots,
+                    k_cache,
+                    v_cache,
+                    QH,
+                    KH,
+                    HD,
+                    BS};
+  if (nw != nullptr && kv_fp8)
+    ps_skinny_lds_go<SL_ROPE, true, unsigned char>(a, stream);
+  else if (nw != nullptr)
+    ps_skinny_lds_go<SL_ROPE, true>(a, stream);
+  else if (kv_fp8)
+    ps_skinny_lds_go<SL_ROPE, false, unsigned char>(a, stream);
+  else
+    ps_skinny_lds_go<SL_ROPE, false>(a, stream);
   return 0;
 }
 
@@ -535,7 +939,7 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
                    int M, int N, int K, long x_stride, hipStream_t stream) {
   if (ps_skinny_gemm_splits(M, N, K) < 0) return -1;
   if (M < 1) return 0;  // no rows: their size in bytes would wrap below
-  if (ps_skinny_rows(M, N, K, x_stride)) {
+  if (ps_skinny_rows(M, N, K, x_stride, x, w)) {
     ps_skinny_rows_go<false>(out_bf16, x, w, M, N, K, x_stride, stream);
     return 0;
   }

@@ -181,6 +181,15 @@ class LlamaLayer(nn.Module):
         fuse_q = (fp8 is not None and hidden.is_cuda
                   and meta.lora_idx is None and not meta.lora_groups
                   and ops.fp8_rowwise_supported(hidden.device))
+        slots = getattr(self, "lora_slots", None)
+        lora = bool(meta.lora_groups) or (slots is not None
+                                          and meta.lora_idx is not None)
+        # few rows: the rotary embedding and the cache's rows (and the norm)
+        # in the launch of the projection
+        fuse_rope = 0
+        if (fp8 is None and not lora and self.qkv_bias is None
+                and self.head_dim % 16 == 0):
+            fuse_rope = gemm_policy.fused(hidden, self.qkv_proj)
         if fuse_q:
             if residual is None:
                 residual = hidden.clone()
@@ -191,6 +200,12 @@ class LlamaLayer(nn.Module):
                     hidden, self.input_norm, cfg.rms_norm_eps,
                     residual=residual)
             qkv = ops.fp8_linear_rowwise(xq, sx, *fp8["qkv"])
+        elif fuse_rope == 2:
+            qkv, residual = ops.skinny_rope(
+                hidden, self.qkv_proj, meta.positions, cos_sin,
+                meta.slot_mapping, *kv_cache, self.q_heads,
+                residual=residual, norm_w=self.input_norm,
+                eps=cfg.rms_norm_eps)
         else:
             if residual is None:
                 residual = hidden
@@ -202,13 +217,16 @@ class LlamaLayer(nn.Module):
                 )
             if fp8 is not None:
                 qkv = ops.fp8_linear(hidden, *fp8["qkv"])
+            elif fuse_rope:
+                qkv, _ = ops.skinny_rope(
+                    hidden, self.qkv_proj, meta.positions, cos_sin,
+                    meta.slot_mapping, *kv_cache, self.q_heads)
             else:
                 qkv = gemm_policy.linear(hidden, self.qkv_proj)
         if self.qkv_bias is not None:
             qkv = qkv + self.qkv_bias
         qs = self.q_heads * self.head_dim
         kvs = self.kv_heads * self.head_dim
-        slots = getattr(self, "lora_slots", None)
         if slots is not None and meta.lora_idx is not None:
             li = self.layer_idx
             slots.apply("q", li, qkv, hidden, meta.lora_idx)
@@ -225,7 +243,9 @@ class LlamaLayer(nn.Module):
             )
         T = qkv.shape[0]
         k_cache, v_cache = kv_cache
-        if qkv.is_cuda:
+        if fuse_rope:
+            qh = qkv.view(T, -1, self.head_dim)[:, : self.q_heads]
+        elif qkv.is_cuda:
             # fused in-place RoPE + KV append straight on the packed qkv;
             # attention consumes the q heads as a strided view (no copies)
             ops.fused_rope_cache(
@@ -321,17 +341,20 @@ class LlamaLayer(nn.Module):
                 residual=residual)
             hidden = attn_out  # bf16 normed not materialized on this path
             gate_up = ops.fp8_linear_rowwise(xq, sx, *fp8["gate_up"])
+        elif fp8 is None and not lora:
+            # no adapter reads the two halves
+            act, residual = gemm_policy.norm_silu_mul(
+                attn_out, residual, self.post_attn_norm, cfg.rms_norm_eps,
+                self.gate_up_proj)
+            gate_up = None
         else:
             hidden, residual = ops.fused_add_rms_norm(
                 attn_out, residual, self.post_attn_norm, cfg.rms_norm_eps
             )
             if fp8 is not None:
                 gate_up = ops.fp8_linear(hidden, *fp8["gate_up"])
-            elif meta.lora_groups or (slots is not None
-                                      and meta.lora_idx is not None):
-                gate_up = gemm_policy.linear(hidden, self.gate_up_proj)
             else:
-                gate_up = None  # no adapter reads the two halves
+                gate_up = gemm_policy.linear(hidden, self.gate_up_proj)
         if slots is not None and meta.lora_idx is not None:
             slots.apply("gate", self.layer_idx, gate_up, hidden,
                         meta.lora_idx)
@@ -351,8 +374,8 @@ class LlamaLayer(nn.Module):
             act = gate_up[:, : self.inter]  # only LoRA reads act; unused
             mlp_out = ops.fp8_linear_rowwise(aq, sa, *fp8["down"])
         else:
-            act = (gemm_policy.silu_mul(hidden, self.gate_up_proj)
-                   if gate_up is None else ops.silu_and_mul(gate_up))
+            if gate_up is not None:
+                act = ops.silu_and_mul(gate_up)
             if fp8 is not None:
                 mlp_out = ops.fp8_linear(act, *fp8["down"])
             else:

@@ -268,6 +268,42 @@ def skinny_gated(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def skinny_norm_gated(x: torch.Tensor, residual, norm_w: torch.Tensor,
+                      eps: float, w: torch.Tensor):
+    """(silu(y @ wg.T) * (y @ wu.T), x + residual) with y the RMSNorm of x +
+    residual and w = [wg; wu], for few rows of x: one launch for
+    fused_add_rms_norm and skinny_gated, same roundings. x and residual stay as
+    they are; without a residual x itself is the sum. GPU only."""
+    _require_ext()
+    out = torch.empty(
+        (x.shape[0], w.shape[0] // 2), dtype=torch.bfloat16, device=x.device
+    )
+    summed = None if residual is None else torch.empty_like(x)
+    _C.skinny_norm_gated(out, summed, x, residual, norm_w, w, eps)
+    return out, x if residual is None else summed
+
+
+def skinny_rope(x: torch.Tensor, w: torch.Tensor, positions: torch.Tensor,
+                cos_sin: torch.Tensor, slots: torch.Tensor,
+                k_cache: torch.Tensor, v_cache: torch.Tensor, q_heads: int,
+                residual=None, norm_w=None, eps: float = 0.0):
+    """(qkv, x + residual): x @ w.T for few rows of x with queries and keys
+    rotated, keys and values in the cache; with norm_w of the RMSNorm of x +
+    residual. One launch for (fused_add_rms_norm,) skinny_gemm and
+    fused_rope_cache, same roundings; x and residual stay as they are. GPU
+    only."""
+    _require_ext()
+    out = torch.empty(
+        (x.shape[0], w.shape[0]), dtype=torch.bfloat16, device=x.device
+    )
+    summed = None if residual is None else torch.empty_like(x)
+    _C.skinny_rope(
+        out, summed, x, residual, norm_w, w, eps, positions, cos_sin, slots,
+        k_cache, v_cache, q_heads,
+    )
+    return out, x if residual is None else summed
+
+
 def cachegen_encode(q: torch.Tensor) -> torch.Tensor:
     """Entropy-encode int8 KV (CPU adaptive range coder, per-channel
     contexts). Falls back to a pure-Python reference when the extension

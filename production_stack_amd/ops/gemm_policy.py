@@ -11,6 +11,7 @@ hipGraph capture records.
 from __future__ import annotations
 
 import logging
+import math
 import time
 from typing import Dict, Tuple
 
@@ -87,14 +88,28 @@ def _fits(x: torch.Tensor, w: torch.Tensor) -> bool:
                      and (x.requires_grad or w.requires_grad)))
 
 
+# entries of x that the kernel with x in LDS takes, with the norm and without
+_LDS_X, _LDS_NORM_X = 65536, 16384
+
+
 def _few_rows(rows: int, N: int, K: int) -> bool:
-    """Up to 3 rows and rows of W of up to 4096 entries. us, in-house /
-    library: 1 x 2048 x 2048 4.9 / 8.2, 1 x 28672 x 4096 46 / 64, 3 x 4096 x 4096
-    11.0 / 15.8, 3 x 6144 x 4096 15.8 / 15.8; past the line 4 x 6144 x 4096 16.2 /
-    15.7, 1 x 2048 x 8192 14.5 / 12.8. Short rows of a wide W are the library's:
-    3 x 65536 x 1024 29.1 / 27.7, 3 x 50304 x 768 19.5 / 18.8 (3 x 51200 x 2560
-    53 / 52, 1 row 50 / 52)."""
-    return rows <= 3 and K <= 4096 and (K > 1024 or N < 32768)
+    """Up to 16 rows, x of up to 65536 entries. Rows of W of up to 4096 entries
+    (us, in-house / library: 1 x 2048 x 2048 4.5 / 11.0, 1 x 28672 x 4096 41 / 63,
+    16 x 28672 x 4096 45 / 64, 16 x 4096 x 4096 10.6 / 15.4, 16 x 6144 x 4096 14.4 /
+    15.5, 16 x 6144 x 2560 10.1 / 10.5, 8 x 51200 x 768 18.7 / 18.9; the narrowest),
+    and longer ones of up to 2048 rows of W (8 x 2048 x 8192 10.5 / 12.6, 8 x 512 x
+    8192 10.0 / 11.4; 16 x 2048 x 8192 16.8 / 12.9) or, up to 4 rows, of as many as
+    give all CUs nearly as much to do (4 x 4096 x 14336 25.8 / 27.0, 4 x 28672 x 8192
+    82 / 122, 1 x 4096 x 8192 15.2 / 16.2; past the line 4 x 6144 x 8192 24 / 22, 4 x
+    5120 x 8192 23 / 20)."""
+    if rows > 16 or rows * K > _LDS_X:
+        return False
+    if K <= 4096:
+        return True
+    if N <= 2048:
+        return rows <= 8 and K % 128 == 0
+    turns = N / 4096
+    return rows <= 4 and turns >= 0.8 * math.ceil(turns)
 
 
 def _long_rows(rows: int, N: int, K: int) -> bool:
@@ -135,6 +150,19 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.linear(x, w)
 
 
+def fused(x: torch.Tensor, w: torch.Tensor) -> int:
+    """What the launch of x @ w.T may have around it: 0 nothing, 1 the rotary
+    embedding and the cache's rows behind it, 2 the residual's sum and the norm
+    before it too. That is as many rows as LDS has room for (a launch of its own
+    costs a decode step 3.5 us and up; the norm in every workgroup of 8 x 4096
+    entries as much)."""
+    entries = x.shape[0] * x.shape[-1]
+    if (x.shape[0] > 16 or entries > _LDS_X or _choose(x, w) != 1
+            or not _fits(x, w) or (w.shape[0] + 32) * w.shape[1] >= 1 << 31):
+        return 0
+    return 2 if entries <= _LDS_NORM_X and x.is_contiguous() else 1
+
+
 def silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu_and_mul(linear(x, w)). Up to 16 rows (8 of a W of more than 32768)
     that take the skinny kernel without splits have the activation in its last
@@ -145,6 +173,18 @@ def silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if x.shape[0] <= rows and _choose(x, w) == 1:
         return ops.skinny_gated(x, w)
     return ops.silu_and_mul(linear(x, w))
+
+
+def norm_silu_mul(x: torch.Tensor, residual: torch.Tensor,
+                  norm_w: torch.Tensor, eps: float, w: torch.Tensor):
+    """(silu_mul(y, w), x + residual), y the RMSNorm of x + residual; x and
+    residual may be overwritten."""
+    from production_stack_amd import ops
+
+    if fused(x, w) == 2 and residual.is_contiguous():
+        return ops.skinny_norm_gated(x, residual, norm_w, eps, w)
+    x, residual = ops.fused_add_rms_norm(x, residual, norm_w, eps)
+    return silu_mul(x, w), residual
 
 
 def reset() -> None:

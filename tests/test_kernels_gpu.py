@@ -1013,6 +1013,118 @@ def test_linear_long_rows(M, N, K, own):
     assert torch.equal(gemm_policy.linear(x, w), want)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 128), (8, 2048, 256), (9, 2048, 256), (8, 2112, 2176),
+    (7, 2048, 4224), (1, 128, 65536), (16, 192, 4096), (13, 192, 4160),
+    (16, 4160, 2048), (5, 4224, 8192), (1, 12288, 1088), (16, 33024, 64)])
+def test_skinny_gemm_lds(M, N, K):
+    """Eight rows of W a workgroup and sixteen, x from memory and from LDS up to
+    its last entry and past it, more tiles than workgroups with a remainder,
+    tiles in two halves, ranges of pieces that the waves do not share evenly;
+    rows of x with a gap and off their alignment, W off its own."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    buf = torch.randn(M + 1, K + 8, generator=g, device="cuda").to(
+        torch.bfloat16)
+    buf[M:] = float("nan")
+    flat = torch.empty(N * K + 1, device="cuda", dtype=torch.bfloat16)
+    flat.normal_(generator=g)
+    odd = flat[1:].view(N, K)
+    w = odd.clone()
+    for x in (buf[:M, :K], buf[:M, 2:K + 2]):
+        want = x.double() @ w.double().t()
+        for m in (w, odd):
+            got = ops.skinny_gemm(x, m).double()
+            # fp32 up to the bf16 rounding of the result (2^-9 at most each); a
+            # sum of K products has an error of sqrt(K) steps of its terms
+            assert ((got - want).abs()
+                    <= want.abs() / 256 + 4e-5 * K ** 0.5).all()
+        if N <= 32768 or M <= 8:
+            for m in (w, odd):
+                act = ops.skinny_gated(x, m)
+                assert torch.equal(act,
+                                   ops.silu_and_mul(ops.skinny_gemm(x, m)))
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 64), (16, 4224, 1024), (4, 8256, 4096), (3, 192, 5184),
+    (7, 320, 2304), (1, 128, 16384)])
+@pytest.mark.parametrize("res", [True, False])
+def test_skinny_norm_gated(M, N, K, res):
+    """The sum and the norm before the products: one row and as many as fit,
+    a width of no whole vectors a thread, several tiles a workgroup. Same
+    roundings as the separate kernels, sums in another order."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x, r = (torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+            for _ in range(2))
+    nw = torch.randn(K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(
+        torch.bfloat16)
+    x0, r0 = x.clone(), r.clone()
+    got, summed = ops.skinny_norm_gated(x, r if res else None, nw, 1e-5, w)
+    assert torch.equal(x, x0) and torch.equal(r, r0)
+    if res:
+        h, r = ops.fused_add_rms_norm(x0, r0, nw, 1e-5)
+        assert torch.equal(summed, r)
+    else:
+        h = ops.rms_norm(x0, nw, 1e-5)
+        assert summed is x
+    want = ops.silu_and_mul(ops.skinny_gemm(h, w)).double()
+    # a row's factor may be a step of fp32 off, which moves few entries of y
+    # over a rounding step
+    assert (got.double() - want).norm() <= 2e-3 * want.norm()
+
+
+@pytest.mark.parametrize("M,qh,kh,hd,K,fp8", [
+    (1, 32, 8, 64, 2048, False), (4, 7, 1, 128, 4096, True),
+    (8, 4, 4, 16, 2048, False), (3, 6, 2, 96, 1088, True),
+    (16, 32, 8, 128, 4096, True), (16, 66, 2, 64, 1024, False),
+    (4, 6, 1, 48, 4096, False)])
+@pytest.mark.parametrize("norm", [True, False])
+def test_skinny_rope(M, qh, kh, hd, K, fp8, norm):
+    """The rotary embedding and the cache's rows behind the products, with and
+    without the norm: head widths of one tile and more, more tiles than
+    workgroups, tokens without a slot, both caches."""
+    if norm and M * K > 16384:
+        with pytest.raises(RuntimeError, match="unsupported"):
+            _skinny_rope(M, qh, kh, hd, K, fp8, norm)
+        return
+    _skinny_rope(M, qh, kh, hd, K, fp8, norm)
+
+
+def _skinny_rope(M, qh, kh, hd, K, fp8, norm):
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    bs, nb = 16, 3
+    n = (qh + 2 * kh) * hd
+    x, r = (torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+            for _ in range(2))
+    nw = torch.randn(K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(n, K, generator=g, device="cuda") * K ** -0.5).to(
+        torch.bfloat16)
+    cs = torch.randn(300, hd, generator=g, device="cuda")
+    pos = torch.randint(0, 300, (M,), generator=g, device="cuda",
+                        dtype=torch.int32)
+    slots = torch.randperm(nb * bs, generator=g, device="cuda")[:M].clone()
+    slots[M // 2] = -1
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    got = [torch.zeros(nb, kh, bs, hd, device="cuda").to(dt)
+           for _ in range(2)]
+    want = [c.clone() for c in got]
+    kw = dict(residual=r, norm_w=nw, eps=1e-5) if norm else {}
+    qkv, summed = ops.skinny_rope(x, w, pos, cs, slots, *got, qh, **kw)
+    h = x
+    if norm:
+        h, r2 = ops.fused_add_rms_norm(x.clone(), r.clone(), nw, 1e-5)
+        assert torch.equal(summed, r2)
+    ref = ops.skinny_gemm(h, w)
+    ops.fused_rope_cache(ref, pos, cs, slots, *want, qh, hd)
+    # sums in another order move few entries over a rounding step (2^-8, 2^-3 in
+    # e4m3) before the rotation
+    assert (qkv.double() - ref.double()).norm() <= 2e-3 * ref.double().norm()
+    tol = 0.03 if fp8 else 2e-3
+    for a, b in zip(got, want):
+        assert (a.double() - b.double()).norm() <= tol * b.double().norm()
+
+
 def test_skinny_gemm_nothing_to_do():
     """No columns of K are refused for any number of rows, no rows give no
     rows, also where they are a view of a wider matrix."""
