@@ -548,4 +548,4 @@ class LlamaForCausalLM(nn.Module):
 
     @torch.no_grad()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden, self.lm_head)
+        return gemm_policy.linear(hidden, self.lm_head)

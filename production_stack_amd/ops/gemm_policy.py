@@ -96,8 +96,8 @@ def _few_rows(rows: int, N: int, K: int) -> bool:
     """Up to 16 rows, x of up to 65536 entries. Rows of W of up to 4096 entries
     (us, in-house / library: 1 x 2048 x 2048 4.5 / 11.0, 1 x 28672 x 4096 41 / 63,
     16 x 28672 x 4096 45 / 64, 16 x 4096 x 4096 10.6 / 15.4, 16 x 6144 x 4096 14.4 /
-    15.5, 16 x 6144 x 2560 10.1 / 10.5, 8 x 51200 x 768 18.7 / 18.9; the narrowest),
-    and longer ones of up to 2048 rows of W (8 x 2048 x 8192 10.5 / 12.6, 8 x 512 x
+    15.5, 16 x 6144 x 2560 10.1 / 10.5, 16 x 128256 x 4096 189 / 191; the narrowest;
+    past the line 1 x 50304 x 768 18.1 / 15.8, 16 x 50304 x 768 19.1 / 16.0), and longer ones of up to 2048 rows of W (8 x 2048 x 8192 10.5 / 12.6, 8 x 512 x
     8192 10.0 / 11.4; 16 x 2048 x 8192 16.8 / 12.9) or, up to 4 rows, of as many as
     give all CUs nearly as much to do (4 x 4096 x 14336 25.8 / 27.0, 4 x 28672 x 8192
     82 / 122, 1 x 4096 x 8192 15.2 / 16.2; past the line 4 x 6144 x 8192 24 / 22, 4 x
@@ -105,7 +105,7 @@ def _few_rows(rows: int, N: int, K: int) -> bool:
     if rows > 16 or rows * K > _LDS_X:
         return False
     if K <= 4096:
-        return True
+        return K > 1024 or N < 32768
     if N <= 2048:
         return rows <= 8 and K % 128 == 0
     turns = N / 4096

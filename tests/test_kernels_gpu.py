@@ -985,6 +985,26 @@ def test_skinny_gemm_tiles(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,own", [
+    (16, 256, 4096, True), (17, 256, 4096, False), (16, 256, 4160, False),
+    (15, 2048, 4160, False), (8, 2048, 8192, True), (9, 2048, 4224, False),
+    (8, 2048, 4160, False), (4, 4096, 8192, True), (5, 4096, 8192, False),
+    (1, 5120, 8192, False), (1, 32768, 1024, False), (1, 32704, 1024, True),
+    (1, 32768, 1088, True), (2, 128, 65536, False)])
+def test_linear_few_rows(M, N, K, own):
+    """Which untuned products of few rows go to the in-house kernel, on either
+    side of each line, and what it says of the launches around them."""
+    from production_stack_amd.ops import gemm_policy
+
+    gemm_policy.reset()
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    w = torch.empty(N, K, device="cuda", dtype=torch.bfloat16).normal_()
+    assert gemm_policy._choose(x, w) == own
+    around = 0 if not own or M * K > 65536 else 1 + (M * K <= 16384)
+    assert gemm_policy.fused(x, w) == around
+    assert gemm_policy.fused(x[:, :K // 2], w[:, :K // 2]) == 0
+
+
+@pytest.mark.parametrize("M,N,K,own", [
     (47, 2048, 10240, False), (48, 2048, 10240, True),
     (23, 2048, 14336, False), (24, 2048, 14336, True),
     (24, 2048, 14272, False), (48, 2112, 10240, False),
