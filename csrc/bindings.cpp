@@ -74,6 +74,18 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
                    int M, int N, int K, long x_stride, hipStream_t stream);
 int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
                     int K, long x_stride, hipStream_t stream);
+int ps_skinny_parts(void* ws, const void* x, const void* w, int M, int N,
+                    int K, long x_stride, hipStream_t stream);
+int ps_skinny_gated_tiles(void* out, const void* x, const void* w, int M,
+                          int N, int K, long x_stride, hipStream_t stream);
+void ps_rms_norm_parts(void* out, const void* parts, int S, void* residual,
+                       const void* w, float eps, long T, int D,
+                       hipStream_t stream);
+int ps_rope_cache_parts(void* q, const void* parts, int S,
+                        const void* positions, const void* cos_sin,
+                        const void* slot_mapping, void* k_cache, void* v_cache,
+                        long T, int QH, int KH, int HD, int BS, int kv_fp8,
+                        hipStream_t stream);
 int ps_skinny_norm_gated(void* out, void* res_out, const void* x,
                          const void* res, const void* nw, const void* w,
                          int M, int N, int K, float eps, hipStream_t stream);
@@ -388,6 +400,88 @@ void skinny_gated(at::Tensor out, at::Tensor x, at::Tensor w) {
               " K=", K);
 }
 
+// fp32 partial sums [splits, M, N]; no tensor where the product has only one
+c10::optional<at::Tensor> skinny_parts(at::Tensor x, at::Tensor w) {
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16,
+              "x must be bf16");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "x must be 2D row-major");
+  CHECK_GPU_BF16(w);
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  TORCH_CHECK(w.size(1) == K, "K mismatch");
+  const int splits = M > 16 ? ps_skinny_gemm_splits(M, N, K) : 0;
+  if (splits < 2) return c10::nullopt;
+  at::Tensor ws = at::empty({(long)splits, (long)M, (long)N},
+                            x.options().dtype(at::kFloat));
+  const int rc = ps_skinny_parts(ws.data_ptr(), x.data_ptr(), w.data_ptr(), M,
+                                 N, K, x.stride(0), current_stream());
+  TORCH_CHECK(rc == 0, "skinny gemm launch failed");
+  return ws;
+}
+
+// false where tiles have only a range of K each
+bool skinny_gated_tiles(at::Tensor out, at::Tensor x, at::Tensor w) {
+  CHECK_GPU_BF16(out);
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16,
+              "x must be bf16");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "x must be 2D row-major");
+  CHECK_GPU_BF16(w);
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  TORCH_CHECK(w.size(1) == K, "K mismatch");
+  TORCH_CHECK(out.numel() == (long)M * (N / 2), "out size mismatch");
+  return ps_skinny_gated_tiles(out.data_ptr(), x.data_ptr(), w.data_ptr(), M,
+                               N, K, x.stride(0), current_stream()) == 0;
+}
+
+// parts [S, T, D]
+void rms_norm_parts(at::Tensor out, at::Tensor parts, at::Tensor residual,
+                    at::Tensor w, double eps) {
+  CHECK_GPU_BF16(out);
+  CHECK_GPU_BF16(residual);
+  CHECK_GPU_BF16(w);
+  CHECK_GPU_DTYPE(parts, at::kFloat);
+  TORCH_CHECK(parts.dim() == 3 && parts.size(0) > 0, "parts must be [S, T, D]");
+  const long T = parts.size(1);
+  const int D = (int)parts.size(2);
+  TORCH_CHECK(out.numel() == T * D && residual.numel() == T * D &&
+                  w.numel() == D && D % 8 == 0 && D <= 32768,
+              "size mismatch");
+  if (T > 0)
+    ps_rms_norm_parts(out.data_ptr(), parts.data_ptr(), (int)parts.size(0),
+                      residual.data_ptr(), w.data_ptr(), (float)eps, T, D,
+                      current_stream());
+}
+
+void rope_cache_parts(at::Tensor q, at::Tensor parts, at::Tensor positions,
+                      at::Tensor cos_sin, at::Tensor slots,
+                      at::Tensor k_cache, at::Tensor v_cache,
+                      int64_t q_heads) {
+  CHECK_GPU_BF16(q);
+  CHECK_GPU_DTYPE(parts, at::kFloat);
+  CHECK_GPU_DTYPE(positions, at::kInt);
+  CHECK_GPU_DTYPE(cos_sin, at::kFloat);
+  CHECK_GPU_DTYPE(slots, at::kLong);
+  const int kv_fp8 = cache_fp8(k_cache);
+  TORCH_CHECK(cache_fp8(v_cache) == kv_fp8 &&
+                  v_cache.sizes() == k_cache.sizes(),
+              "caches differ");
+  const int KH = (int)k_cache.size(1), BS = (int)k_cache.size(2),
+            HD = (int)k_cache.size(3);
+  TORCH_CHECK(parts.dim() == 3 &&
+                  parts.size(2) == (q_heads + 2 * KH) * HD,
+              "parts must be [S, T, (q heads + 2 kv heads) head_dim]");
+  const long T = parts.size(1);
+  TORCH_CHECK(q.numel() == T * q_heads * HD && positions.numel() == T &&
+                  slots.numel() == T && cos_sin.size(-1) == HD,
+              "size mismatch");
+  if (T == 0) return;
+  const int rc = ps_rope_cache_parts(
+      q.data_ptr(), parts.data_ptr(), (int)parts.size(0),
+      positions.data_ptr(), cos_sin.data_ptr(), slots.data_ptr(),
+      k_cache.data_ptr(), v_cache.data_ptr(), T, (int)q_heads, KH, HD, BS,
+      kv_fp8, current_stream());
+  TORCH_CHECK(rc == 0, "unsupported head width ", HD);
+}
+
 // what the norm before a product needs: dense rows
 static void check_norm(const at::Tensor& x, const c10::optional<at::Tensor>& res,
                        const at::Tensor& nw,
@@ -616,6 +710,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "8-phase deep-pipelined bf16 GEMM (out = x @ w.T)");
   m.def("skinny_gemm", &skinny_gemm,
         "MFMA GEMM for decode-shaped (M<=256) projections");
+  m.def("skinny_parts", &skinny_parts,
+        "Partial sums of a split skinny GEMM, or None");
+  m.def("skinny_gated_tiles", &skinny_gated_tiles,
+        "Tiled skinny GEMM with the gated activation; false: not built");
+  m.def("rms_norm_parts", &rms_norm_parts,
+        "Residual add and RMSNorm of partial sums");
+  m.def("rope_cache_parts", &rope_cache_parts,
+        "RoPE and KV append of partial sums");
   m.def("skinny_norm_gated", &skinny_norm_gated,
         "Residual sum, RMSNorm, skinny GEMM and gated activation");
   m.def("skinny_rope", &skinny_rope,

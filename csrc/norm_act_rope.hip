@@ -9,6 +9,21 @@
 // where possible.
 #include "ps_common.h"
 
+// Eight columns of partial sums that lie `apart` entries apart, added in order.
+PS_DEV void ps_sum_parts(const float* p, int S, long apart, float* sum) {
+  ps_f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+#pragma unroll 8
+  for (int s = 0; s < S; ++s) {
+    a += *(const ps_f32x4*)(p + s * apart);
+    b += *(const ps_f32x4*)(p + s * apart + 4);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    sum[j] = a[j];
+    sum[4 + j] = b[j];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // RMSNorm:  out[t, :] = x[t, :] * rsqrt(mean(x^2) + eps) * w
 // with ADD (the per-layer hot path)
@@ -77,6 +92,67 @@ __global__ __launch_bounds__(BLOCK) void rms_norm_kernel(
       for (int j = 0; j < 8; j++)
         ov[j] = ps_f32_to_bf16(vals[u][j] * inv * ps_bf16_to_f32(wv[u][j]));
       *(ps_bf16x8*)(orow + i) = ov;
+    }
+  }
+}
+
+// The same where x comes as partial sums of a product, [S, T, D] in fp32: their
+// sum, rounded as the product's own last step does, is what the norm adds to the
+// residual. That step has no launch of its own then (4.8 to 5.4 us a product of a
+// decode batch). More threads a row than above, since each has S times the loads.
+template <int BLOCK, int VPT>
+__global__ __launch_bounds__(BLOCK) void rms_norm_parts_kernel(
+    unsigned short* __restrict__ out,       // [T, D]
+    const float* __restrict__ parts,        // [S, T, D]
+    int S, unsigned short* __restrict__ residual,  // [T, D]
+    const unsigned short* __restrict__ w,   // [D]
+    float eps, int D) {
+  const long row = blockIdx.x * (long)D, TD = gridDim.x * (long)D;
+  ps_bf16x8 rv[VPT], wv[VPT];
+  float vals[VPT][8];
+#pragma unroll
+  for (int u = 0; u < VPT; u++) {
+    const int i = (u * BLOCK + (int)threadIdx.x) * 8;
+    if (i < D) {
+      rv[u] = *(const ps_bf16x8*)(residual + row + i);
+      wv[u] = *(const ps_bf16x8*)(w + i);
+      ps_sum_parts(parts + row + i, S, TD, vals[u]);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < VPT; u++) {
+    const int i = (u * BLOCK + (int)threadIdx.x) * 8;
+    if (i < D) {
+      ps_bf16x8 sv;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float f = ps_bf16_to_f32(ps_f32_to_bf16(vals[u][j])) +
+                        ps_bf16_to_f32(rv[u][j]);
+        vals[u][j] = f;
+        ss += f * f;
+        sv[j] = ps_f32_to_bf16(f);
+      }
+      *(ps_bf16x8*)(residual + row + i) = sv;
+    }
+  }
+  __shared__ float red[BLOCK / 64];
+  ss = ps_group_sum<64>(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  float tot = 0.f;
+#pragma unroll
+  for (int k = 0; k < BLOCK / 64; k++) tot += red[k];
+  const float inv = rsqrtf(tot / (float)D + eps);
+#pragma unroll
+  for (int u = 0; u < VPT; u++) {
+    const int i = (u * BLOCK + (int)threadIdx.x) * 8;
+    if (i < D) {
+      ps_bf16x8 ov;
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        ov[j] = ps_f32_to_bf16(vals[u][j] * inv * ps_bf16_to_f32(wv[u][j]));
+      *(ps_bf16x8*)(out + row + i) = ov;
     }
   }
 }
@@ -169,6 +245,22 @@ void ps_fused_add_rms_norm(void* out, void* residual, const void* w,
 }
 #undef PS_NORM_WIDTH
 #undef PS_NORM
+
+void ps_rms_norm_parts(void* out, const void* parts, int S, void* residual,
+                       const void* w, float eps, long T, int D,
+                       hipStream_t stream) {
+#define PS_NORM(VPT)                                                         \
+  rms_norm_parts_kernel<512, VPT><<<dim3((unsigned)T), 512, 0, stream>>>(    \
+      (unsigned short*)out, (const float*)parts, S,                          \
+      (unsigned short*)residual, (const unsigned short*)w, eps, D)
+  if (D <= 4096)
+    PS_NORM(1);
+  else if (D <= 8192)
+    PS_NORM(2);
+  else
+    PS_NORM(8);
+#undef PS_NORM
+}
 
 void ps_silu_and_mul(void* out, const void* x, long T, int D,
                      hipStream_t stream) {
@@ -312,6 +404,71 @@ __global__ __launch_bounds__(256) void fused_rope_cache_vec_kernel(
   }
 }
 
+// The same from partial sums of a product, [S, T, (QH + 2 KH) HD] in fp32, each
+// column's sum rounded as the product's own last step does: queries to rows of
+// their own, keys and values to the cache. Four columns of each half a thread, all
+// splits' loads on their way at once: bound by their latency. us with the product
+// before it, 32/8 heads of 128 of 4096: 192 rows 32.0 (the library's product and
+// the kernel above 37.0), 128 rows 27.0 (28.6), 64 rows 22.9 (20.9).
+template <typename KVT>
+__global__ __launch_bounds__(256) void rope_parts_kernel(
+    unsigned short* __restrict__ q, const float* __restrict__ parts, int S,
+    const int* __restrict__ positions, const float* __restrict__ cos_sin,
+    const long* __restrict__ slot_mapping, KVT* __restrict__ k_cache,
+    KVT* __restrict__ v_cache, int QH, int KH, int HD, int BS) {
+  const long t = blockIdx.x;
+  const long N = (long)(QH + 2 * KH) * HD, TN = gridDim.x * N;
+  const long slot = slot_mapping[t];
+  const int half = HD / 2, nr = half / 4;
+  const int rot = (QH + KH) * nr;  // pairs to rotate, then the values
+  const int i = blockIdx.y * blockDim.x + threadIdx.x;
+  auto sum = [&](long col) {
+    const float* p = parts + t * N + col;
+    ps_f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int s = 0; s < S; ++s) a += *(const ps_f32x4*)(p + s * TN);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] = ps_bf16_to_f32(ps_f32_to_bf16(a[j]));
+    return a;
+  };
+  auto put = [&](KVT* cache, int h, int d, const unsigned short(&v)[4]) {
+    typename ps_kv_traits<KVT>::vec4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[j] = ps_kv_traits<KVT>::from_f32(ps_bf16_to_f32(v[j]));
+    *(typename ps_kv_traits<KVT>::vec4*)(
+        cache + ((slot / BS * KH + h) * BS + slot % BS) * HD + d) = o;
+  };
+  if (i < rot) {
+    const int h = i / nr, r = i % nr * 4;
+    const float* cs = cos_sin + (long)positions[t] * HD;
+    const ps_f32x4 c = *(const ps_f32x4*)(cs + r);
+    const ps_f32x4 s = *(const ps_f32x4*)(cs + half + r);
+    const ps_f32x4 a = sum((long)h * HD + r), b = sum((long)h * HD + half + r);
+    unsigned short x[4], y[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      x[j] = ps_f32_to_bf16(a[j] * c[j] - b[j] * s[j]);
+      y[j] = ps_f32_to_bf16(b[j] * c[j] + a[j] * s[j]);
+    }
+    if (h < QH) {
+      unsigned short* out = q + (t * QH + h) * HD + r;
+      *(ps_bf16x4*)out = ps_bf16x4{x[0], x[1], x[2], x[3]};
+      *(ps_bf16x4*)(out + half) = ps_bf16x4{y[0], y[1], y[2], y[3]};
+    } else if (slot >= 0) {
+      put(k_cache, h - QH, r, x);
+      put(k_cache, h - QH, r + half, y);
+    }
+  } else if (i < rot + KH * HD / 4 && slot >= 0) {
+    const int col = (i - rot) * 4;
+    const ps_f32x4 a = sum((long)(QH + KH) * HD + col);
+    unsigned short x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = ps_f32_to_bf16(a[j]);
+    put(v_cache, col / HD, col % HD, x);
+  }
+}
+
 extern "C" void ps_fused_rope_cache(void* qkv, const void* positions,
                                     const void* cos_sin,
                                     const void* slot_mapping, void* k_cache,
@@ -353,6 +510,34 @@ extern "C" void ps_fused_rope_cache(void* qkv, const void* positions,
             (const float*)cos_sin, (const long*)slot_mapping,
             (unsigned short*)k_cache, (unsigned short*)v_cache, QH, KH, HD,
             ROT, qkv_stride, BS);
+}
+
+// From partial sums [S, T, (QH + 2 KH) HD]: queries to q [T, QH HD], keys and
+// values to the cache; whole heads are rotated. -1: not built
+extern "C" int ps_rope_cache_parts(void* q, const void* parts, int S,
+                                   const void* positions, const void* cos_sin,
+                                   const void* slot_mapping, void* k_cache,
+                                   void* v_cache, long T, int QH, int KH,
+                                   int HD, int BS, int kv_fp8,
+                                   hipStream_t stream) {
+  if (HD % 8 != 0 || S < 1 ||
+      (((size_t)q | (size_t)parts | (size_t)cos_sin | (size_t)k_cache |
+        (size_t)v_cache) &
+       15) != 0)
+    return -1;
+  const int work = (QH + KH) * (HD / 8) + KH * HD / 4;
+  const dim3 grid((unsigned)T, (work + 255) / 256);
+#define PS_ROPE(KVT)                                                         \
+  rope_parts_kernel<KVT><<<grid, 256, 0, stream>>>(                          \
+      (unsigned short*)q, (const float*)parts, S, (const int*)positions,     \
+      (const float*)cos_sin, (const long*)slot_mapping, (KVT*)k_cache,       \
+      (KVT*)v_cache, QH, KH, HD, BS)
+  if (kv_fp8)
+    PS_ROPE(unsigned char);
+  else
+    PS_ROPE(unsigned short);
+#undef PS_ROPE
+  return 0;
 }
 
 // ---------------------------------------------------------------------------

@@ -512,7 +512,10 @@ __global__ __launch_bounds__(256, 4) void skinny_gemm_kernel(
 //   28672 x 4096   64 rows 51 / 96 / 53, 192 rows 71 / 150 / 62
 //   2048 x 8192    64 rows 17 / 25 / 21, 192 rows 25 / 40 / 25
 // Waves split by rows of x as well read W twice: 10 to 40 % slower.
-template <int MT, int NC>
+// GATED (one range): W holds N / 2 gate rows, then as many up rows; 16 rows of a
+// tile are eight of each, which are two lane groups apart, and out [M, N / 2] is
+// silu(gate) up, both rounded to bf16 first.
+template <int MT, int NC, bool GATED>
 __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
     unsigned short* __restrict__ out,      // [M, N] (one split)
     float* __restrict__ ws,                // [splits, M, N]
@@ -552,8 +555,14 @@ __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
 
   const unsigned short* wp[NC];
 #pragma unroll
-  for (int c = 0; c < NC; ++c)
-    wp[c] = w + (long)(n0 + (wn * NC + c) * 16 + rc) * K + g * 8;
+  for (int c = 0; c < NC; ++c) {
+    const int row = n0 + (wn * NC + c) * 16;
+    wp[c] = w + g * 8 +
+            (long)(!GATED   ? row + rc
+                   : rc < 8 ? row / 2 + rc
+                            : (N + row) / 2 + rc - 8) *
+                K;
+  }
   ps_gbf16x8 wf[WD][NC][2];
   // steps past the end repeat the last chunk and are not multiplied
   auto load_w = [&](int u, int t) {
@@ -653,6 +662,22 @@ __global__ __launch_bounds__(512, MT* NC <= 8 ? 4 : 2) void skinny_tile_kernel(
           const ps_gf32x4 v =
               acc[c][h + i] +
               *(const ps_gf32x4*)(sum + (i * 16 + rc) * PN + n);
+          if constexpr (GATED) {
+            unsigned short e[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float gv = ps_bf16_to_f32(ps_f32_to_bf16(v[r]));
+              const float uv = ps_bf16_to_f32(
+                  ps_f32_to_bf16(__shfl_xor(v[r], 32, 64)));
+              e[r] = ps_f32_to_bf16(gv / (1.f + __expf(-gv)) * uv);
+            }
+            if (m < M && g < 2)
+              *(uint2*)(out + (long)m * (N / 2) +
+                        (n0 + (wn * NC + c) * 16) / 2 + 4 * g) =
+                  make_uint2((unsigned int)e[0] | ((unsigned int)e[1] << 16),
+                             (unsigned int)e[2] | ((unsigned int)e[3] << 16));
+            continue;
+          }
           if (m >= M) continue;
           if (splits > 1)
             *(ps_gf32x4*)(ws + ((long)split * M + m) * N + n0 + n) = v;
@@ -935,14 +960,10 @@ int ps_skinny_gemm_splits(int M, int N, int K) {
   return ps_skinny_plan(M, N, K).splits;
 }
 
-int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
-                   int M, int N, int K, long x_stride, hipStream_t stream) {
-  if (ps_skinny_gemm_splits(M, N, K) < 0) return -1;
-  if (M < 1) return 0;  // no rows: their size in bytes would wrap below
-  if (ps_skinny_rows(M, N, K, x_stride, x, w)) {
-    ps_skinny_rows_go<false>(out_bf16, x, w, M, N, K, x_stride, stream);
-    return 0;
-  }
+// The tiles or the short form; `parts`: the partial sums are the result.
+static int ps_skinny_splits_go(void* out_bf16, void* ws, const void* x,
+                               const void* w, int M, int N, int K,
+                               long x_stride, bool parts, hipStream_t stream) {
   PsSkinnyPlan plan = ps_skinny_plan(M, N, K);
   if (ws == nullptr) plan.splits = 1;
 #define PS_SG(MT)                                                           \
@@ -950,7 +971,7 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
       (unsigned short*)out_bf16, (float*)ws, (const unsigned short*)x,      \
       (const unsigned short*)w, M, N, K, x_stride)
 #define PS_ST(MT, NC)                                                       \
-  skinny_tile_kernel<MT, NC>                                                \
+  skinny_tile_kernel<MT, NC, false>                                              \
       <<<dim3(N / (64 * NC) * plan.splits), dim3(512), 0, stream>>>(        \
           (unsigned short*)out_bf16, (float*)ws, (const unsigned short*)x,  \
           (const unsigned short*)w, M, N, K, x_stride, plan.splits)
@@ -978,11 +999,59 @@ int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
 #undef PS_ST2
 #undef PS_ST
 #undef PS_SG
-  if (plan.splits > 1) {
+  if (plan.splits > 1 && !parts) {
     const long MN = (long)M * N;
     skinny_combine_kernel<<<dim3((MN / 4 + 255) / 256), 256, 0, stream>>>(
         (unsigned short*)out_bf16, (const float*)ws, MN, plan.splits);
   }
+  return 0;
+}
+
+int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
+                   int M, int N, int K, long x_stride, hipStream_t stream) {
+  if (ps_skinny_gemm_splits(M, N, K) < 0) return -1;
+  if (M < 1) return 0;  // no rows: their size in bytes would wrap below
+  if (ps_skinny_rows(M, N, K, x_stride, x, w)) {
+    ps_skinny_rows_go<false>(out_bf16, x, w, M, N, K, x_stride, stream);
+    return 0;
+  }
+  return ps_skinny_splits_go(out_bf16, ws, x, w, M, N, K, x_stride, false,
+                             stream);
+}
+
+// Partial sums [splits, M, N] in fp32 of more than 16 rows, for a kernel behind
+// this one that adds them; -1: not built, or there is only one
+int ps_skinny_parts(void* ws, const void* x, const void* w, int M, int N,
+                    int K, long x_stride, hipStream_t stream) {
+  if (M <= 16 || ps_skinny_gemm_splits(M, N, K) < 2) return -1;
+  return ps_skinny_splits_go(nullptr, ws, x, w, M, N, K, x_stride, true,
+                             stream);
+}
+
+// As ps_skinny_gated for 17 to 192 rows, in tiles that have all of K
+int ps_skinny_gated_tiles(void* out, const void* x, const void* w, int M,
+                          int N, int K, long x_stride, hipStream_t stream) {
+  if (M <= 16 || M > 192 || ps_skinny_gemm_splits(M, N, K) != 1) return -1;
+  const PsSkinnyPlan plan = ps_skinny_plan(M, N, K);
+  if (plan.form == PS_SHORT) return -1;
+#define PS_ST(MT, NC)                                                       \
+  skinny_tile_kernel<MT, NC, true>                                          \
+      <<<dim3(N / (64 * NC)), dim3(512), 0, stream>>>(                      \
+          (unsigned short*)out, nullptr, (const unsigned short*)x,          \
+          (const unsigned short*)w, M, N, K, x_stride, 1)
+#define PS_ST2(MT)                                                          \
+  do {                                                                      \
+    if (plan.form == PS_WIDE)                                               \
+      PS_ST(MT, 2);                                                         \
+    else                                                                    \
+      PS_ST(MT, 1);                                                         \
+  } while (0)
+  if (M <= 32) PS_ST2(2);
+  else if (M <= 64) PS_ST2(4);
+  else if (M <= 128) PS_ST2(8);
+  else PS_ST2(12);
+#undef PS_ST2
+#undef PS_ST
   return 0;
 }
 

@@ -115,6 +115,7 @@ class LlamaLayer(nn.Module):
         super().__init__()
         self.cfg = cfg
         self.layer_idx = layer_idx
+        self.tp = tp
         assert cfg.num_q_heads % tp == 0, "q heads must divide TP"
         assert cfg.num_kv_heads % tp == 0 or tp % cfg.num_kv_heads == 0
         self.q_heads = cfg.num_q_heads // tp
@@ -166,11 +167,12 @@ class LlamaLayer(nn.Module):
 
     def forward(
         self,
-        hidden: torch.Tensor,  # [T, H]
+        hidden: torch.Tensor,  # [T, H], or partial sums [S, T, H] of it
         residual: Optional[torch.Tensor],
         meta: BatchMeta,
         kv_cache: tuple,  # (k_cache, v_cache) [NB, KH, BS, HD]
         cos_sin: torch.Tensor,
+        parts_out: bool = False,  # the caller takes partial sums
     ) -> tuple:
         cfg = self.cfg
         fp8 = getattr(self, "fp8_w", None)
@@ -186,10 +188,14 @@ class LlamaLayer(nn.Module):
                                           and meta.lora_idx is not None)
         # few rows: the rotary embedding and the cache's rows (and the norm)
         # in the launch of the projection
+        plain = fp8 is None and not lora
+        few = plain and hidden.shape[-2] <= gemm_policy.MAX_ROWS
+        rope_behind = (few and self.qkv_bias is None
+                       and self.head_dim % 16 == 0)
         fuse_rope = 0
-        if (fp8 is None and not lora and self.qkv_bias is None
-                and self.head_dim % 16 == 0):
+        if rope_behind and hidden.dim() == 2:
             fuse_rope = gemm_policy.fused(hidden, self.qkv_proj)
+        qkv_parts = None
         if fuse_q:
             if residual is None:
                 residual = hidden.clone()
@@ -212,10 +218,16 @@ class LlamaLayer(nn.Module):
                 hidden = ops.rms_norm(hidden, self.input_norm,
                                       cfg.rms_norm_eps)
             else:
-                hidden, residual = ops.fused_add_rms_norm(
+                add_norm = (ops.fused_add_rms_norm if hidden.dim() == 2
+                            else ops.add_rms_norm_parts)
+                hidden, residual = add_norm(
                     hidden, residual, self.input_norm, cfg.rms_norm_eps
                 )
-            if fp8 is not None:
+            if rope_behind:
+                qkv_parts = gemm_policy.parts(hidden, self.qkv_proj, "rope")
+            if qkv_parts is not None:
+                qkv = None
+            elif fp8 is not None:
                 qkv = ops.fp8_linear(hidden, *fp8["qkv"])
             elif fuse_rope:
                 qkv, _ = ops.skinny_rope(
@@ -241,9 +253,13 @@ class LlamaLayer(nn.Module):
             apply_lora_slice(
                 qkv, hidden, meta.lora_groups, li, "v", qs + kvs, kvs
             )
-        T = qkv.shape[0]
+        T = hidden.shape[0]
         k_cache, v_cache = kv_cache
-        if fuse_rope:
+        if qkv_parts is not None:
+            qh = ops.rope_cache_parts(
+                qkv_parts, meta.positions, cos_sin, meta.slot_mapping,
+                k_cache, v_cache, self.q_heads)
+        elif fuse_rope:
             qh = qkv.view(T, -1, self.head_dim)[:, : self.q_heads]
         elif qkv.is_cuda:
             # fused in-place RoPE + KV append straight on the packed qkv;
@@ -313,7 +329,12 @@ class LlamaLayer(nn.Module):
                 )
             )
         attn = torch.cat(outs, dim=0) if len(outs) > 1 else outs[0]
-        if getattr(self, "fp8_w", None) is not None:
+        attn_out = None
+        if few and self.tp == 1 and not self.n_experts:
+            attn_out = gemm_policy.parts(attn.view(T, qs), self.o_proj, "norm")
+        if attn_out is not None:
+            pass  # the norm behind adds the sums
+        elif getattr(self, "fp8_w", None) is not None:
             attn_out = ops.fp8_linear(attn.reshape(T, qs),
                                       *self.fp8_w["o"])
         else:
@@ -326,7 +347,8 @@ class LlamaLayer(nn.Module):
                 attn_out, attn.view(T, qs), meta.lora_groups,
                 self.layer_idx, "o",
             )
-        attn_out = pstate.tp_all_reduce(attn_out)
+        if attn_out.dim() == 2:
+            attn_out = pstate.tp_all_reduce(attn_out)
 
         if self.n_experts:
             hidden, residual = ops.fused_add_rms_norm(
@@ -341,7 +363,7 @@ class LlamaLayer(nn.Module):
                 residual=residual)
             hidden = attn_out  # bf16 normed not materialized on this path
             gate_up = ops.fp8_linear_rowwise(xq, sx, *fp8["gate_up"])
-        elif fp8 is None and not lora:
+        elif few:
             # no adapter reads the two halves
             act, residual = gemm_policy.norm_silu_mul(
                 attn_out, residual, self.post_attn_norm, cfg.rms_norm_eps,
@@ -353,6 +375,9 @@ class LlamaLayer(nn.Module):
             )
             if fp8 is not None:
                 gate_up = ops.fp8_linear(hidden, *fp8["gate_up"])
+            elif plain:
+                act = gemm_policy.silu_mul(hidden, self.gate_up_proj)
+                gate_up = None
             else:
                 gate_up = gemm_policy.linear(hidden, self.gate_up_proj)
         if slots is not None and meta.lora_idx is not None:
@@ -376,6 +401,10 @@ class LlamaLayer(nn.Module):
         else:
             if gate_up is not None:
                 act = ops.silu_and_mul(gate_up)
+            elif few and parts_out and self.tp == 1:
+                sums = gemm_policy.parts(act, self.down_proj, "norm")
+                if sums is not None:
+                    return sums, residual
             if fp8 is not None:
                 mlp_out = ops.fp8_linear(act, *fp8["down"])
             else:
@@ -533,15 +562,19 @@ class LlamaForCausalLM(nn.Module):
             residual = None
         else:
             hidden = token_ids  # mid-pipeline: activations from prev stage
-        for layer, cache in zip(self.layers, kv_caches):
+        for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):
             hidden, residual = layer(
-                hidden, residual, meta, cache, self.cos_sin
+                hidden, residual, meta, cache, self.cos_sin,
+                # norms add partial sums; the next stage asks for rows
+                parts_out=self.is_last or i + 1 < len(self.layers),
             )
         if not self.is_last:
             # caller ships (hidden, residual) to the next stage
             return torch.stack([hidden, residual])
         # final residual add + norm
-        hidden, _ = ops.fused_add_rms_norm(
+        add_norm = (ops.fused_add_rms_norm if hidden.dim() == 2
+                    else ops.add_rms_norm_parts)
+        hidden, _ = add_norm(
             hidden, residual, self.final_norm, self.cfg.rms_norm_eps
         )
         return hidden

@@ -52,6 +52,16 @@ def fused_add_rms_norm(
     return normed, summed
 
 
+def add_rms_norm_parts(parts: torch.Tensor, residual: torch.Tensor,
+                       w: torch.Tensor, eps: float):
+    """fused_add_rms_norm of a product's partial sums (skinny_parts): (normed,
+    residual), the residual in place. GPU only."""
+    _require_ext()
+    out = torch.empty_like(residual)
+    _C.rms_norm_parts(out, parts, residual, w, eps)
+    return out, residual
+
+
 def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     if x.is_cuda:
         _require_ext()
@@ -93,6 +103,25 @@ def fused_rope_cache(
         qkv, positions, cos_sin, slot_mapping, k_cache, v_cache, q_heads,
         head_dim,
     )
+
+
+def rope_cache_parts(
+    parts: torch.Tensor,
+    positions: torch.Tensor,
+    cos_sin: torch.Tensor,
+    slot_mapping: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    q_heads: int,
+) -> torch.Tensor:
+    """fused_rope_cache of a product's partial sums (skinny_parts): the rotated
+    queries [T, q_heads, head_dim]. GPU only."""
+    _require_ext()
+    q = torch.empty((parts.shape[1], q_heads, k_cache.shape[3]),
+                    dtype=torch.bfloat16, device=parts.device)
+    _C.rope_cache_parts(q, parts, positions, cos_sin, slot_mapping, k_cache,
+                        v_cache, q_heads)
+    return q
 
 
 def reshape_and_cache(
@@ -266,6 +295,24 @@ def skinny_gated(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     )
     _C.skinny_gated(out, x, w)
     return out
+
+
+def skinny_parts(x: torch.Tensor, w: torch.Tensor):
+    """x @ w.T for 17 to 256 rows of x as fp32 partial sums [splits, rows,
+    columns] for a kernel behind it to add, or None where the kernel that takes
+    these sizes has no splits. GPU only."""
+    _require_ext()
+    return _C.skinny_parts(x, w)
+
+
+def skinny_gated_tiles(x: torch.Tensor, w: torch.Tensor):
+    """skinny_gated for 17 to 192 rows, or None where the kernel that takes these
+    sizes has splits. GPU only."""
+    _require_ext()
+    out = torch.empty(
+        (x.shape[0], w.shape[0] // 2), dtype=torch.bfloat16, device=x.device
+    )
+    return out if _C.skinny_gated_tiles(out, x, w) else None
 
 
 def skinny_norm_gated(x: torch.Tensor, residual, norm_w: torch.Tensor,

@@ -24,8 +24,11 @@ logger = logging.getLogger("ops.gemm_policy")
 _POLICY: Dict[Tuple[int, int, int], int] = {}
 
 
+MAX_ROWS = 256  # of the skinny kernels
+
+
 def _eligible(M: int, N: int, K: int) -> bool:
-    return M <= 256 and N % 64 == 0 and K % 64 == 0
+    return M <= MAX_ROWS and N % 64 == 0 and K % 64 == 0
 
 
 def _eligible_8p(M: int, N: int, K: int) -> bool:
@@ -128,15 +131,70 @@ def _long_rows(rows: int, N: int, K: int) -> bool:
             and 2048 <= N <= 8192 and N % 128 == 0 and K >= 10240)
 
 
-def _choose(x: torch.Tensor, w: torch.Tensor) -> int:
-    """0: the library, 1: skinny, 2: 8-phase."""
+def _rows_before_norm(rows: int, N: int, K: int) -> bool:
+    """17 to 192 rows whose partial sums the norm behind them adds. us with that
+    norm, in-house / library: 17 x 2048 x 2048 10.1 / 13.8, 64 x 2048 x 8192 18.4 /
+    25.2, 64 x 4096 x 4096 17.0 / 18.4, 192 x 4096 x 4096 24.9 / 36.3, 64 x 4096 x
+    14336 32.7 / 42.5, 96 x 3584 x 4096 20.1 / 25.3, 128 x 6144 x 4096 27.2 / 29.6,
+    192 x 8192 x 14336 78 / 117. Past the lines 64 x 6144 x 4096 22.7 / 22.0, 17 x
+    2048 x 8192 16.8 / 16.5, 96 x 2560 x 4096 19.4 / 16.3, 160 x 3072 x 4096 22.5 /
+    20.2, 128 x 4096 x 2048 18.8 / 18.7, 256 x 4096 x 8192 45.6 / 40.1. The slowest
+    found within: 48 x 2560 x 2560 13.7 / 12.7."""
+    if not 17 <= rows <= 192 or not 1024 <= N <= 8192 or K < 1024:
+        return False
+    if K >= 10240:
+        return True
+    if rows > 64:
+        return 3584 <= N <= 6144 and K >= 4096
+    return N <= 4096 and (K <= 5120 or (rows >= 48 and N >= 1536))
+
+
+def _rows_before_rope(rows: int, N: int, K: int) -> bool:
+    """As above with the rotary embedding and the cache's rows behind: 128 x 6144 x
+    4096 27.0 / 28.6, 192 32.0 / 37.0, 128 x 7168 x 5120 35.3 / 36.7, 128 x 4608 x 3584
+    24.6 / 26.1; past the lines 96 x 4608 x 3584 23.6 / 23.4, 192 x 6144 x 2048 26.2 /
+    25.8, 160 x 3072 x 2048 21.6 / 15.9."""
+    return 128 <= rows <= 192 and 4608 <= N <= 10240 and K >= 3584
+
+
+def _rows_before_gate(rows: int, N: int, K: int) -> bool:
+    """As above with the activation behind, in tiles that have all of K and fill
+    the CUs once, rows of W a power of two apart or nearly (where the library is
+    slow): 17 x 28672 x 4096 49.5 / 56.4, 64 51.7 / 55.4, 64 x 28672 x 2048 30.7 / 33.1,
+    64 x 32768 x 8192 105 / 123; past the lines 96 x 28672 x 4096 59.5 / 56.3, 64 x
+    24576 x 4096 50.8 / 49.0, 17 x 28672 x 2560 36.6 / 31.7, 64 x 57344 x 4096 106 /
+    102."""
+    return 17 <= rows <= 64 and 28160 <= N <= 32768 and K % 2048 == 0
+
+
+_UNTUNED = {"": (_few_rows, _long_rows),
+            "norm": (_rows_before_norm,),
+            "rope": (_rows_before_rope,),
+            "gate": (_few_rows, _long_rows, _rows_before_gate)}
+
+
+def _choose(x: torch.Tensor, w: torch.Tensor, behind: str = "") -> int:
+    """0: the library, 1: skinny, 2: 8-phase. behind: what the product's last step
+    shares a launch with."""
     if not x.is_cuda or x.dtype != torch.bfloat16:
         return 0
     shape = (x.shape[0], w.shape[0], w.shape[1])
     impl = _POLICY.get(shape)
     if impl is None:  # untuned
-        impl = int((_few_rows(*shape) or _long_rows(*shape)) and _fits(x, w))
+        impl = int(any(rule(*shape) for rule in _UNTUNED[behind])
+                   and _fits(x, w))
     return impl
+
+
+def parts(x: torch.Tensor, w: torch.Tensor, behind: str):
+    """linear(x, w) as partial sums in fp32 [splits, rows, columns] for "norm"
+    (ops.add_rms_norm_parts) or "rope" (ops.rope_cache_parts) to add, or None
+    where linear is to be called."""
+    from production_stack_amd import ops
+
+    if 16 < x.shape[0] <= MAX_ROWS and _choose(x, w, behind) == 1 and _fits(x, w):
+        return ops.skinny_parts(x, w)
+    return None
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -156,8 +214,10 @@ def fused(x: torch.Tensor, w: torch.Tensor) -> int:
     before it too. That is as many rows as LDS has room for (a launch of its own
     costs a decode step 3.5 us and up; the norm in every workgroup of 8 x 4096
     entries as much)."""
+    if x.shape[0] > 16:
+        return 0
     entries = x.shape[0] * x.shape[-1]
-    if (x.shape[0] > 16 or entries > _LDS_X or _choose(x, w) != 1
+    if (entries > _LDS_X or _choose(x, w) != 1
             or not _fits(x, w) or (w.shape[0] + 32) * w.shape[1] >= 1 << 31):
         return 0
     return 2 if entries <= _LDS_NORM_X and x.is_contiguous() else 1
@@ -165,25 +225,33 @@ def fused(x: torch.Tensor, w: torch.Tensor) -> int:
 
 def silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu_and_mul(linear(x, w)). Up to 16 rows (8 of a W of more than 32768)
-    that take the skinny kernel without splits have the activation in its last
-    step (a launch of its own costs a decode step 4.5 us a layer)."""
+    that take the skinny kernel, and more where its tiles have all of K, have the
+    activation in its last step (a launch of its own costs a decode step 4.5 us
+    a layer and more)."""
     from production_stack_amd import ops
 
     rows = 8 if w.shape[0] > 32768 else 16
-    if x.shape[0] <= rows and _choose(x, w) == 1:
-        return ops.skinny_gated(x, w)
+    if _choose(x, w, "gate") == 1:
+        if x.shape[0] <= rows:
+            return ops.skinny_gated(x, w)
+        if 16 < x.shape[0] <= 192 and _fits(x, w):
+            act = ops.skinny_gated_tiles(x, w)
+            if act is not None:
+                return act
     return ops.silu_and_mul(linear(x, w))
 
 
 def norm_silu_mul(x: torch.Tensor, residual: torch.Tensor,
                   norm_w: torch.Tensor, eps: float, w: torch.Tensor):
-    """(silu_mul(y, w), x + residual), y the RMSNorm of x + residual; x and
-    residual may be overwritten."""
+    """(silu_mul(y, w), x + residual), y the RMSNorm of x + residual; x may be
+    partial sums; x and residual may be overwritten."""
     from production_stack_amd import ops
 
-    if fused(x, w) == 2 and residual.is_contiguous():
+    if x.dim() == 2 and fused(x, w) == 2 and residual.is_contiguous():
         return ops.skinny_norm_gated(x, residual, norm_w, eps, w)
-    x, residual = ops.fused_add_rms_norm(x, residual, norm_w, eps)
+    add_norm = (ops.fused_add_rms_norm if x.dim() == 2
+                else ops.add_rms_norm_parts)
+    x, residual = add_norm(x, residual, norm_w, eps)
     return silu_mul(x, w), residual
 
 

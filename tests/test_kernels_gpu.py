@@ -1145,6 +1145,131 @@ def _skinny_rope(M, qh, kh, hd, K, fp8, norm):
         assert (a.double() - b.double()).norm() <= tol * b.double().norm()
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (17, 64, 128), (61, 4096, 4096), (192, 1024, 2176), (256, 4160, 4096),
+    (33, 8256, 1024), (20, 16448, 512)])
+def test_skinny_parts_norm(M, N, K):
+    """Partial sums that the norm adds, from the short form and from tiles, up to
+    rows of more than one vector a thread: bit for bit the residual of the
+    separate kernels; None where there is one range."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x, r = (torch.randn(M, n, generator=g, device="cuda").to(torch.bfloat16)
+            for n in (K, N))
+    nw = torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(
+        torch.bfloat16)
+    parts = ops.skinny_parts(x, w)
+    want, wr = ops.fused_add_rms_norm(ops.skinny_gemm(x, w), r.clone(), nw,
+                                      1e-5)
+    if parts is None:
+        assert N > 8192
+        parts = torch.stack([x.float() @ w.float().t(),
+                             torch.zeros(M, N, device="cuda")])
+        exact = False
+    else:
+        assert parts.shape[0] > 1 and parts.shape[1:] == (M, N)
+        exact = True
+    got, gr = ops.add_rms_norm_parts(parts, r, nw, 1e-5)
+    assert gr is r
+    if exact:
+        assert torch.equal(gr, wr)
+    # the row's sum of squares in another order
+    assert (got.double() - want.double()).norm() <= 2e-3 * want.double().norm()
+
+
+@pytest.mark.parametrize("M,qh,kh,hd,K,fp8", [
+    (17, 32, 8, 64, 2048, False), (192, 7, 1, 128, 4096, True),
+    (130, 4, 4, 16, 1024, False), (33, 6, 2, 96, 1088, True)])
+def test_rope_cache_parts(M, qh, kh, hd, K, fp8):
+    """Rotary embedding and cache rows of partial sums: the separate kernels'
+    values, tokens without a slot, both caches."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    bs, nb = 16, 16
+    n = (qh + 2 * kh) * hd
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(n, K, generator=g, device="cuda") * K ** -0.5).to(
+        torch.bfloat16)
+    cs = torch.randn(300, hd, generator=g, device="cuda")
+    pos = torch.randint(0, 300, (M,), generator=g, device="cuda",
+                        dtype=torch.int32)
+    slots = torch.randperm(nb * bs, generator=g, device="cuda")[:M].clone()
+    slots[M // 2] = -1
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    got = [torch.zeros(nb, kh, bs, hd, device="cuda").to(dt)
+           for _ in range(2)]
+    want = [c.clone() for c in got]
+    q = ops.rope_cache_parts(ops.skinny_parts(x, w), pos, cs, slots, *got, qh)
+    ref = ops.skinny_gemm(x, w)
+    ops.fused_rope_cache(ref, pos, cs, slots, *want, qh, hd)
+    # an angle's two products and their sum may round apart by a step of fp32,
+    # so that few entries move over a step of their type
+    ref = ref[:, :qh * hd].double()
+    assert (q.view(M, -1).double() - ref).norm() <= 1e-3 * ref.norm()
+    for a, b in zip(got, want):
+        assert ((a.double() - b.double()).norm()
+                <= (2e-2 if fp8 else 1e-3) * b.double().norm())
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (17, 28672, 2048), (64, 32768, 256), (65, 16384, 1088), (192, 28672, 192),
+    (100, 49152, 128)])
+def test_skinny_gated_tiles(M, N, K):
+    """Tiles of gate and up rows with the activation behind, both widths."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(
+        torch.bfloat16)
+    got = ops.skinny_gated_tiles(x, w)
+    want = ops.silu_and_mul(ops.skinny_gemm(x, w)).double()
+    if got is None:  # the short form
+        assert K <= 1088
+        return
+    # ranges begin at other steps: sums in another order, roundings the same
+    assert (got.double() - want).norm() <= 2e-3 * want.norm()
+
+
+@pytest.mark.parametrize("behind,M,N,K,own", [
+    ("norm", 17, 1024, 1024, True), ("norm", 16, 1024, 2048, False),
+    ("norm", 64, 4096, 5120, True), ("norm", 64, 4160, 4096, False),
+    ("norm", 65, 3584, 4096, True), ("norm", 65, 3520, 4096, False),
+    ("norm", 192, 6144, 4096, True), ("norm", 193, 6144, 4096, False),
+    ("norm", 96, 4096, 4032, False), ("norm", 47, 4096, 8192, False),
+    ("norm", 48, 4096, 8192, True), ("norm", 48, 1472, 8192, False),
+    ("norm", 17, 8192, 10240, True), ("norm", 17, 960, 10240, False),
+    ("norm", 65, 6208, 4096, False),
+    ("rope", 128, 4608, 3584, True), ("rope", 127, 4608, 3584, False),
+    ("rope", 192, 10240, 3584, True), ("rope", 192, 4544, 3584, False)])
+def test_parts_dispatch(behind, M, N, K, own):
+    """Which untuned products leave their partial sums, on either side of each
+    line."""
+    from production_stack_amd.ops import gemm_policy
+
+    gemm_policy.reset()
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    w = torch.empty(N, K, device="cuda", dtype=torch.bfloat16).normal_()
+    got = gemm_policy.parts(x, w, behind)
+    assert (got is not None) == own
+    assert gemm_policy.parts(x[:, :-64], w[:, :-64], behind) is None
+
+
+@pytest.mark.parametrize("M,N,K,own", [
+    (17, 28160, 2048, True), (64, 32768, 2048, True), (65, 28672, 2048, False),
+    (17, 28096, 2048, False), (17, 32832, 2048, False),
+    (17, 28672, 1024, False)])
+def test_gate_dispatch(M, N, K, own):
+    """Which untuned gated products of 17 rows and more are in-house."""
+    from production_stack_amd.ops import gemm_policy
+
+    gemm_policy.reset()
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    w = (torch.empty(N, K, device="cuda").normal_() * K ** -0.5).to(
+        torch.bfloat16)
+    assert gemm_policy._choose(x, w, "gate") == own
+    want = (ops.skinny_gated_tiles(x, w) if own else
+            ops.silu_and_mul(torch.nn.functional.linear(x, w)))
+    assert torch.equal(gemm_policy.silu_mul(x, w), want)
+
+
 def test_skinny_gemm_nothing_to_do():
     """No columns of K are refused for any number of rows, no rows give no
     rows, also where they are a view of a wider matrix."""
