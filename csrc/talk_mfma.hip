@@ -6,32 +6,36 @@
 // talk_attention.hip; 32 heads, head widths 64 or 128.
 //
 // A workgroup of eight waves owns 16 consecutive rows and 16 output heads and
-// walks tiles of 32 keys:
-//   scores   of all 32 heads: wave w has heads 4 w .. 4 w + 3 (one KV head),
-//            K Q^T as 16 x 16 tiles, keys straight from the cache as left
-//            operands (no other wave reads them), queries in registers for the
-//            whole walk. The other 16 output heads' workgroup repeats them:
+// walks tiles of 32 keys by halves of 16, one barrier each. Between two barriers
+//   scores   of the next half, all 32 heads: wave w has heads 4 w .. 4 w + 3 (one
+//            KV head), K Q^T as 16 x 16 tiles, keys straight from the cache as
+//            left operands (no other wave reads them), queries in registers for
+//            the whole walk. The other 16 output heads' workgroup repeats them:
 //            an eighth of the work, and with 32 output heads the accumulators
 //            alone would fill half the registers;
-//   mix      through LDS as fp32 [head][row][key], since every output head
-//            needs all of them: wave w mixes the 16 output heads for 4 keys,
-//            the matrix and the scores as fp32 operands of
+//   mix      of this half through LDS as fp32 [head][row][key], since every
+//            output head needs all of them: wave w mixes the 16 output heads for
+//            2 keys, the matrix and the scores as fp32 operands of
 //            v_mfma_f32_16x16x4_f32 (no term of either is rounded);
-//   softmax  a lane then holds one row's scores of 4 heads over 4 keys: the
-//            maximum meets the other seven key shares in LDS, the
-//            denominator stays a partial sum per share to the end;
-//   output   the weights go back through the same LDS rows to the wave of
-//            their head (wave w: two of the 16), there cut into three bf16
-//            terms (exact products, fp32 accumulation), values through LDS
-//            with transposed reads.
-// A thread-per-(head, row) kernel on the vector pipe did this before (it
-// remains for fp32 and other shapes): 13 TF/s, every product of the mix and of
-// both contractions an fp32 multiply-add. Here a tile takes about 4600 cycles
-// of a SIMD's matrix unit, 1024 of them the scores, 2048 the mix, 1536 the
-// output, and 14200 in all: with one workgroup a CU (its LDS) the four barriers
-// between those stages leave the matrix unit waiting. 32/8 heads of 128, 4099
-// rows in two prompts, chunks of 2048: 0.42 ms (11.7 before; 0.63 with the blocks
-// of rows from last to first).
+//   softmax  a lane then holds one row's scores of 4 heads over 2 keys, whose
+//            weights are relative to a reference that all waves share, not to the
+//            half's own maximum: it moves, by an exchange behind the barrier, only
+//            where a score is more than TM_FAR above it. The denominator stays a
+//            partial sum per key share to the end;
+//   output   of the tile before, in every other half: the weights go through LDS
+//            to the wave of their head (wave w: two of the 16), there cut into
+//            three bf16 terms (exact products, fp32 accumulation), values through
+//            LDS with transposed reads.
+// Scores have two halves in LDS, weights three, so that none of this waits for
+// another wave. A tile takes about 4600 cycles of a SIMD's matrix unit, 1024 of
+// them the scores, 2048 the mix, 1536 the output, 4000 of vector instructions, and
+// 12000 in all (14200 with four barriers a tile of 32 and the maximum through LDS
+// in each): both waves of a SIMD come to the products and to the softmax at about
+// the same time. 32/8 heads of 128, 4099 rows in two prompts, chunks of 2048: 0.32
+// ms (0.42 with four barriers, 0.63 with the blocks of rows from last to first, 11.7
+// on the vector pipe, whose kernel remains for fp32 and other shapes). Sixteen waves
+// spill at widths of 128 and are no faster at 64 (284 us, 272 with eight); orders of
+// the four parts that differ between the two waves of a SIMD spill as well.
 #include "attn_common.h"
 #include "scan_common.h"
 
@@ -50,7 +54,9 @@ union TmPack {
 
 #define TM_H 32
 #define TM_KT 32
-#define TM_PS 36  // LDS pitch of a row's keys: 16-byte units 9 apart
+// how far scores, in powers of two, may be above the reference that weights are
+// relative to
+#define TM_FAR 8.f
 
 struct TmArgs {
   unsigned short* out;
@@ -132,6 +138,12 @@ PS_DEV int tm_first_row(const TmArgs& a, int rank, int blocks) {
   return block * 16;
 }
 
+// Where a (row, unit) of LDS rows of 16 keys is: units of two keys, turned by the
+// row and one bit of the head so that the 32 lanes of a pass meet all banks.
+PS_DEV int tm_at(int head, int row, int unit, int bit) {
+  return (head * 16 + row) * 16 + 2 * (unit ^ (row >> 2 | (bit & 1) << 2));
+}
+
 // ND = D / 32, NV = DV / 16; CAP: with a score cap
 template <int ND, int NV, bool CAP>
 __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
@@ -140,14 +152,17 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   constexpr int PR = DV / 8;          // 16-byte pieces of a value row
   constexpr int RI = 64 / PR;         // value rows per load of a wave
   constexpr int NL = TM_KT / 2 / RI;
+  constexpr int SS = TM_H * 256, SP = 16 * 256;
   extern __shared__ __align__(16) float lds[];
-  float* sS = lds;                                 // [32][16][TM_PS]
-  float* sPM = sS + TM_H * 16 * TM_PS;             // [8][16][16]
+  float* sS = lds;                                 // [2][32][16][16 keys]
+  float* sP = sS + 2 * SS;                         // [3][16][16][16 keys]
+  float* sPM = sP + 3 * SP;                        // [8][16][16]
   float* sAL = sPM + 8 * 256;                      // [16][16]
   unsigned short* sV = (unsigned short*)(sAL + 256);  // [4][32][PV]
   __shared__ int s_seq[16], s_pos[16];
   // first and last tile of a run whose values (of two waves) are not all finite
   __shared__ int s_odd[4][2];
+  __shared__ int s_high[3];  // a half's scores are too far above the reference
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, n = lane & 15;
@@ -181,10 +196,13 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
       for (int d = 0; d < ND; ++d)
         qf[h][d].q = *(const tm_u4*)(qp + h * D + 32 * d);
   }
-  float ta[8];  // left operand of the mix: step j takes heads 4 j + g
+  // left operand of the mix: step j takes heads 4 j + g. Scores in powers of two
+  // (with a cap behind it).
+  float ta[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j)
-    ta[j] = a.talk[(16 * hb + n) * TM_H + 4 * j + g];
+    ta[j] = a.talk[(16 * hb + n) * TM_H + 4 * j + g] *
+            (CAP ? a.scale : a.scale * KV_LOG2E);
   __syncthreads();
 
   const int pos = s_pos[n];
@@ -194,7 +212,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     m[i] = a.sink ? (a.sink_vals != nullptr
-                         ? fmaxf(a.sink_vals[h0 + i], PS_NEG_INF)
+                         ? fmaxf(a.sink_vals[h0 + i] * KV_LOG2E, PS_NEG_INF)
                          : 0.f)
                   : PS_NEG_INF;
     l[i] = a.sink && wave == 0 ? 1.f : 0.f;
@@ -205,6 +223,9 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
 #pragma unroll
     for (int t = 0; t < NV; ++t) acc[h][t] = ck_f32x4{0.f, 0.f, 0.f, 0.f};
 
+  // one of the two waves of a SIMD first, so that its softmax comes beside
+  // products of the other (324 -> 320 us)
+  if (ND == 4 && wave < 4) __builtin_amdgcn_s_setprio(1);
   int rs = 0;
   while (rs < ntok) {
     // batch rows rs .. re - 1 continue one sequence
@@ -229,38 +250,16 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
       const int j = min(kmin + t * TM_KT + (lane & 31), kmax);
       return table[j / a.BS] * a.G * a.BS + j % a.BS;
     };
-    TmPack kf[2][ND];
-    auto fetch_k = [&](int ridx) {
+    TmPack kf[ND];  // keys of a half: left operands
+    auto fetch_k = [&](int ridx, int half) {
+      const unsigned short* kp =
+          a.kc +
+          (int64_t)(__shfl(ridx, 16 * half + n, 64) + grp * a.BS) * D + 8 * g;
 #pragma unroll
-      for (int kh = 0; kh < 2; ++kh) {
-        const unsigned short* kp =
-            a.kc + (int64_t)(__shfl(ridx, 16 * kh + n, 64) + grp * a.BS) * D +
-            8 * g;
-#pragma unroll
-        for (int d = 0; d < ND; ++d)
-          kf[kh][d].q = *(const tm_u4*)(kp + 32 * d);
-      }
+      for (int d = 0; d < ND; ++d) kf[d].q = *(const tm_u4*)(kp + 32 * d);
     };
-    int ridx = row_of(0);
-    fetch_k(ridx);
-    int rnext = row_of(min(1, nt - 1));
-    for (int t = 0; t < nt; ++t) {
-      const int j0 = kmin + t * TM_KT;
-      // raw scores: lane (g, n) has keys 16 kh + 4 g + i of row n
-#pragma unroll
-      for (int h = 0; h < 4; ++h)
-#pragma unroll
-        for (int kh = 0; kh < 2; ++kh) {
-          ck_f32x4 st = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int d = 0; d < ND; ++d)
-            st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                kf[kh][d].v, qf[h][d].v, st, 0, 0, 0);
-          *(ck_f32x4*)(sS + ((wave * 4 + h) * 16 + n) * TM_PS + 16 * kh +
-                       4 * g) = st * a.scale;
-        }
-      // values: on their way during the mix
-      tm_u4 vr[NL];
+    tm_u4 vr[NL];
+    auto fetch_v = [&](int ridx) {
 #pragma unroll
       for (int u = 0; u < NL; ++u)
         vr[u] = *(const tm_u4*)(
@@ -269,71 +268,103 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
                       vgrp * a.BS) *
                 a.vr +
             (lane % PR) * 8);
-      __syncthreads();
-      if (t == 0 && threadIdx.x < 4) {  // read by all for the run before
-        s_odd[threadIdx.x][0] = nt;
-        s_odd[threadIdx.x][1] = -1;
-      }
-
-      // mixed scores x[e][i]: key 4 wave + e, head h0 + i, row n
-      ck_f32x4 x[4];
+    };
+    // raw scores of a half: lane (g, n) has keys 4 g + i of row n
+    auto scores = [&](int half) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = ck_f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int h = 0; h < 4; ++h) {
+        ck_f32x4 st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+          st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[d].v, qf[h][d].v, st,
+                                                       0, 0, 0);
+        float* to = sS + half * SS;
+        *(float2*)(to + tm_at(wave * 4 + h, n, 2 * g, h)) =
+            make_float2(st[0], st[1]);
+        *(float2*)(to + tm_at(wave * 4 + h, n, 2 * g + 1, h)) =
+            make_float2(st[2], st[3]);
+      }
+    };
+    // mixed scores x[e][i]: key 2 wave + e of a half, head h0 + i, row n
+    auto mix = [&](int t, int half, ck_f32x4(&x)[2]) {
+      x[0] = x[1] = ck_f32x4{0.f, 0.f, 0.f, 0.f};
+      float2 b[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        b[j] = *(const float2*)(sS + half * SS + tm_at(4 * j + g, n, wave, g));
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const ck_f32x4 b = *(const ck_f32x4*)(
-            sS + ((4 * j + g) * 16 + n) * TM_PS + 4 * wave);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          x[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta[j], b[e], x[e], 0, 0,
-                                                      0);
-      }
-      if constexpr (CAP) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            x[e][i] = a.softcap * tanhf(x[e][i] / a.softcap);
+        x[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta[j], b[j].x, x[0], 0, 0,
+                                                    0);
+        x[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta[j], b[j].y, x[1], 0, 0,
+                                                    0);
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int j = j0 + 4 * wave + e;
+      for (int e = 0; e < 2; ++e) {
+        const int j = kmin + t * TM_KT + 16 * half + 2 * wave + e;
         const bool vis = j >= my_lo && j <= my_hi;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)  // no number counts as hidden
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (CAP)
+            x[e][i] = a.softcap * KV_LOG2E * tanhf(x[e][i] / a.softcap);
+          // no number counts as hidden
           x[e][i] = vis ? fmaxf(x[e][i], PS_NEG_INF) : PS_NEG_INF;
+        }
       }
+    };
+    // weights of a half, its third of sP, their sums
+    auto weigh = [&](ck_f32x4(&x)[2], float* to, float(&sum)[4]) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        // nothing visible yet: weights of 0, whatever is subtracted
+        const float ms = m[i] > PS_NEG_INF ? m[i] : 0.f;
+        const float p0 = __builtin_amdgcn_exp2f(x[0][i] - ms);
+        const float p1 = __builtin_amdgcn_exp2f(x[1][i] - ms);
+        sum[i] = p0 + p1;
+        *(float2*)(to + tm_at(4 * g + i, n, wave, g)) = make_float2(p0, p1);
+      }
+    };
+    // A half whose scores are more than TM_FAR above the reference, behind the
+    // barrier that ends its turn: the reference moves to the largest, and with it
+    // what was made by the one before: the half's weights, those of the other
+    // half of an unfinished tile, sums and outputs.
+    auto raise = [&](int t, int half, int third, float(&sum)[4]) {
+      ck_f32x4 x[2];
+      mix(t, half, x);
       float* pm = sPM + 4 * g * 16 + n;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        pm[wave * 256 + i * 16] =
-            fmaxf(fmaxf(x[0][i], x[1][i]), fmaxf(x[2][i], x[3][i]));
-      __syncthreads();  // also: the raw scores are read
-
+        pm[wave * 256 + i * 16] = fmaxf(x[0][i], x[1][i]);
+      __syncthreads();
+      float* other = sP + (third + 2) % 3 * SP;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float mn = m[i];
 #pragma unroll
         for (int k = 0; k < 8; ++k) mn = fmaxf(mn, pm[k * 256 + i * 16]);
-        // nothing visible yet: weights of 0 below, whatever is subtracted
-        // (ck_exp of minus infinity; no branches around it)
-        const float ms = mn > PS_NEG_INF ? mn : 0.f;
-        const float al = ck_exp(m[i] - ms);
+        const float al =
+            __builtin_amdgcn_exp2f(m[i] - (mn > PS_NEG_INF ? mn : 0.f));
         m[i] = mn;
+        l[i] *= al;
         if (wave == 0) sAL[(4 * g + i) * 16 + n] = al;
-        float sum = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[e][i] = ck_exp(x[e][i] - ms);
-          sum += x[e][i];
+        if (half == 1) {
+          float2* p = (float2*)(other + tm_at(4 * g + i, n, wave, g));
+          *p = make_float2(p->x * al, p->y * al);
         }
-        l[i] = l[i] * al + sum;
-        *(ck_f32x4*)(sS + ((4 * g + i) * 16 + n) * TM_PS + 4 * wave) =
-            ck_f32x4{x[0][i], x[1][i], x[2][i], x[3][i]};
       }
-      // Values that are not finite stay out of the products, where a hidden
-      // key's weight of zero would carry them to rows that do not see it (rows
-      // of other sequences among them); they join behind the walk.
+      weigh(x, sP + third * SP, sum);
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float al = sAL[(wave * 2 + h) * 16 + n];
+#pragma unroll
+        for (int c = 0; c < NV; ++c) acc[h][c] *= al;
+      }
+    };
+    // Values that are not finite stay out of the products, where a hidden
+    // key's weight of zero would carry them to rows that do not see it (rows
+    // of other sequences among them); they join behind the walk.
+    auto put_v = [&](int t) {
       tm_us2 top = {0, 0};
 #pragma unroll
       for (int u = 0; u < NL; ++u)
@@ -359,10 +390,9 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
       for (int u = 0; u < NL; ++u)
         *(tm_u4*)(sV + ((wave & 1) * 16 + u * RI + lane / PR) * PV +
                   (lane % PR) * 8) = vr[u];
-      ridx = rnext;
-      rnext = row_of(min(t + 2, nt - 1));
-      __syncthreads();
-
+    };
+    // a tile's output: its weights are in thirds `first` and the next
+    auto output = [&](int first) {
       TmPack vf[NV];  // left operands: columns 16 c .., keys 8 g + i
       const unsigned short* va =
           sV + (8 * g + (n >> 2)) * PV + 4 * (n & 3);
@@ -372,22 +402,17 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
         for (int h = 0; h < 2; ++h)
           vf[c].h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
               (tm_lds_s4*)(va + 4 * h * PV + 16 * c));
+      const float* from = sP + (first + (g >> 1)) % 3 * SP;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int head = wave * 2 + h;  // of the 16
-        const float al = sAL[head * 16 + n];
-        if (__any(al != 1.f)) {
-#pragma unroll
-          for (int c = 0; c < NV; ++c) acc[h][c] *= al;
-        }
-        const float* ps = sS + (head * 16 + n) * TM_PS + 8 * g;
-        const ck_f32x4 pa = *(const ck_f32x4*)ps;
-        const ck_f32x4 pb = *(const ck_f32x4*)(ps + 4);
         TmPack b0, b1, b2;
-        kv_split(pa[0], pa[1], &b0.w[0], &b1.w[0], &b2.w[0]);
-        kv_split(pa[2], pa[3], &b0.w[1], &b1.w[1], &b2.w[1]);
-        kv_split(pb[0], pb[1], &b0.w[2], &b1.w[2], &b2.w[2]);
-        kv_split(pb[2], pb[3], &b0.w[3], &b1.w[3], &b2.w[3]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float2 p = *(const float2*)(
+              from + tm_at(head, n, 4 * (g & 1) + q, head >> 2));
+          kv_split(p.x, p.y, &b0.w[q], &b1.w[q], &b2.w[q]);
+        }
 #pragma unroll
         for (int c = 0; c < NV; ++c) {
           acc[h][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -398,10 +423,70 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
               vf[c].v, b2.v, acc[h][c], 0, 0, 0);
         }
       }
-      // not before: beside the value operands they would spill
-      fetch_k(ridx);
-      __syncthreads();  // the weights are read
+    };
+
+    int rcur = row_of(0), rnext = row_of(min(1, nt - 1));
+    fetch_k(rcur, 0);
+    if (threadIdx.x < 4) {
+      s_odd[threadIdx.x][0] = nt;
+      s_odd[threadIdx.x][1] = -1;
     }
+    if (threadIdx.x < 3) s_high[threadIdx.x] = 0;
+    scores(0);
+    fetch_k(rcur, 1);
+    __syncthreads();
+    float sum[4];
+    int third = 0;  // of sP for the coming half
+    // One half: its weights, the scores of the next one, beside either the output
+    // of the tile before or the writing of this one's values.
+    auto turn = [&](int t, int half) {
+      // read before the last barrier; set again behind the next
+      if (threadIdx.x == 0) s_high[(third + 1) % 3] = 0;
+      auto weights = [&] {
+        ck_f32x4 x[2];
+        mix(t, half, x);
+        bool high = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          high |= fmaxf(x[0][i], x[1][i]) > m[i] + TM_FAR;
+        if (__any(high) && lane == 0) s_high[third] = 1;
+        weigh(x, sP + third * SP, sum);
+      };
+      auto others = [&] {
+        scores(half ^ 1);
+        if (half == 0) {
+          if (t > 0) output((third + 1) % 3);
+          // not before: beside the value operands they would spill
+          __builtin_amdgcn_sched_barrier(0);
+          fetch_k(rnext, 0);
+          fetch_v(rcur);
+        } else {
+          put_v(t);
+          rcur = rnext;
+          rnext = row_of(min(t + 2, nt - 1));
+          fetch_k(rcur, 1);
+        }
+      };
+      // us, weights first / last: heads of 128 329 / 324, of 64 262 / 277
+      if constexpr (ND == 4) {
+        others();
+        weights();
+      } else {
+        weights();
+        others();
+      }
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(s_high[third]))
+        raise(t, half, third, sum);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) l[i] += sum[i];
+      third = third == 2 ? 0 : third + 1;
+    };
+    for (int t = 0; t < nt; ++t) {
+      turn(t, 0);
+      turn(t, 1);
+    }
+    output((third + 1) % 3);
     // values that are not finite, to the rows that see their keys: whatever
     // the weight, which is above zero, they decide the sum
     const int odd0 = s_odd[wave >> 1][0], odd1 = s_odd[wave >> 1][1];
@@ -424,6 +509,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    __syncthreads();  // the run's LDS is read
     rs = re;
   }
 
@@ -460,7 +546,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
 
 template <int ND, int NV, bool CAP>
 static int tm_launch_as(const TmArgs& a, hipStream_t stream) {
-  const size_t lds = (size_t)(TM_H * 16 * TM_PS + 9 * 256) * 4 +
+  const size_t lds = (size_t)(2 * TM_H * 256 + 3 * 16 * 256 + 9 * 256) * 4 +
                      (size_t)4 * TM_KT * (NV * 16 + 8) * 2;
   if (hipFuncSetAttribute((const void*)talk_mfma_kernel<ND, NV, CAP>,
                           hipFuncAttributeMaxDynamicSharedMemorySize,

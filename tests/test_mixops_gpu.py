@@ -489,6 +489,44 @@ def test_talk_attention_matrix_cores(G, D, DV, chunk, window, softcap,
     assert (out[:, H * DV:] == 7.0).all()
 
 
+@pytest.mark.parametrize("sink", [True, False])
+@pytest.mark.parametrize("shape", ["up", "down", "steps"])
+def test_talk_attention_scores_climb(shape, sink):
+    """Scores that climb past the reference of the weights in nearly every half
+    of a tile, once at its start, or in steps within first and second halves;
+    rows of two sequences whose scores move by different amounts."""
+    g = torch.Generator().manual_seed(19)
+    H, G, D, DV, bs, L = 32, 8, 128, 128, 16, 170
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.bfloat16, g, 2)
+    pos = torch.arange(tables.shape[1] * bs).float()
+    grow = {"up": 0.05 * pos, "down": 8.0 - 0.05 * pos,
+            "steps": 2.0 * (pos // 21)}[shape]
+    for s in range(2):
+        # all heads' queries look along one direction, keys of sequence 1 less so
+        f = grow * (1.0 if s == 0 else 0.4)
+        for j in range(tables.shape[1]):
+            kc[tables[s, j], :, :, 0] += f[j * bs:(j + 1) * bs].to(
+                torch.bfloat16)
+    ts = torch.tensor([0] * 25 + [1] * 12, dtype=torch.int32)
+    tp = torch.tensor(list(range(140, 165)) + list(range(100, 112)),
+                      dtype=torch.int32)
+    T = len(ts)
+    q = torch.randn(T, H, D, generator=g)
+    q[:, :, 0] = 10.0 + q[:, :, 0].abs()
+    q = q.to(torch.bfloat16)
+    talk = torch.eye(H) + 0.1 * torch.randn(H, H, generator=g)
+    want = reference.talk_attention(
+        q.float(), kc.float(), vc.float(), tables, ts, tp, D ** -0.5, 0, 0,
+        sink, talk)
+    got = ops.talk_attention(
+        q.cuda().view(T, H * D), kc.cuda(), vc.cuda(), tables.cuda(),
+        ts.cuda(), tp.cuda(), D ** -0.5, H, sink=sink, talk=talk.cuda(),
+        variant=10)
+    # fp32 up to the bf16 rounding of the result; scores of up to 60 in sums of
+    # 128 and 32 terms are 2e-5 off, and their weights with them
+    assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
+
+
 @pytest.mark.parametrize("lens,chunk,window", [
     ([2040], 0, 0),                  # 128 blocks: as they come
     ([1500, 549], 512, 0),           # 129 by length, one of two sequences
