@@ -2255,6 +2255,68 @@ __global__ __launch_bounds__(256) void ck_readout_kernel(
   }
 }
 
+// The same for heads of 8 LPH columns whose rows lie on 16-byte borders (not the
+// matrix LSTM's): a lane has eight neighbouring columns, LPH lanes a head, so that
+// every access is 16 bytes. Whether the rows are this kernel's is asked while they
+// are on their way. Bound by memory; us, a lane with one to four columns of four
+// heads / this: 8011 rows of 32 bf16 heads of 128 80 / 42 (6.2 TB/s), 6007 rows 55 /
+// 33, 1501 rows of 8 heads of 256 15.8 / 7.0.
+template <typename T, int MODE, int LPH>
+__global__ __launch_bounds__(256) void ck_readout_wide_kernel(
+    T* __restrict__ out, int ldo, const float* __restrict__ raw,
+    const T* __restrict__ gate, int ldg, const float* __restrict__ normw,
+    const int* __restrict__ seq_rows, int S_, int T_, int H, float eps) {
+  constexpr int DV = 8 * LPH;
+  struct alignas(16) vec8 {
+    T e[8];
+  };
+  const unsigned units = H * LPH;  // of eight columns
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  const unsigned last = (unsigned)T_ * units - 1;
+  const unsigned at = min(i, last);
+  const int t = at / units, c = (at - t * units) * 8;
+  const float* r = raw + (size_t)t * (H * DV) + c;
+  const ck_f32x4 oa = *(const ck_f32x4*)r, ob = *(const ck_f32x4*)(r + 4);
+  const vec8 gv = *(const vec8*)(gate + (size_t)t * ldg + c);
+  const float* w = normw + (MODE == CK_GD ? c : c % DV);
+  const ck_f32x4 wa = *(const ck_f32x4*)w, wb = *(const ck_f32x4*)(w + 4);
+  // rows of short segments are not this kernel's; a wave has one row or a few
+  const int lane = threadIdx.x & 63;
+  bool mine = false;
+  for (int s0 = 0; s0 < S_; s0 += 64) {
+    const int s = min(s0 + lane, S_ - 1);
+    const int a = seq_rows[4 * s], n = seq_rows[4 * s + 1];
+    unsigned long long left =
+        __ballot(s0 + lane < S_ && n >= 16 &&
+                 a + n > __builtin_amdgcn_readfirstlane(t));
+    while (left) {
+      const int k = __ffsll((long long)left) - 1;
+      const int first = __builtin_amdgcn_readlane(a, k);
+      const int rows = __builtin_amdgcn_readlane(n, k);
+      mine |= t >= first && t < first + rows;
+      left &= left - 1;
+      if (__all(mine)) break;
+    }
+    if (__all(mine)) break;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) ss += oa[u] * oa[u] + ob[u] * ob[u];
+#pragma unroll
+  for (int d = 1; d < LPH; d <<= 1) ss += __shfl_xor(ss, d, 64);
+  const float inv = 1.0f / sqrtf(ss / (float)DV + eps);
+  vec8 y;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const float g = MxElem<T>::ld(&gv.e[u]);
+    float gt = ck_sigmoid(g);
+    if (MODE == CK_GLA) gt *= g;
+    MxElem<T>::st(&y.e[u], (u < 4 ? oa[u & 3] : ob[u & 3]) * inv *
+                               (u < 4 ? wa[u & 3] : wb[u & 3]) * gt);
+  }
+  if (mine && i <= last) *(vec8*)(out + (size_t)t * ldo + c) = y;
+}
+
 // Key width as the kernels pad it (0: not built).
 static int ck_pad(int D) {
   const int pads[] = {32, 64, 96, 128};
@@ -2280,12 +2342,12 @@ static long ck_chunk_floats(int mode, int dp, int H, int G, int L) {
 }
 
 // Measured (bf16, one MI355X, whole operation; token by token -> this form):
-//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.74 ms
-//     (operands 0.24, walk 0.41, read-out 0.08)
+//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.70 ms
+//     (operands 0.24, walk 0.41, read-out 0.04)
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
-//                                                            5.42 -> 0.55 ms
+//                                                            5.42 -> 0.53 ms
 //   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.30 ms
-//   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.07 ms
+//   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.06 ms
 //   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.47 ms
 // From 16 rows on a segment goes this way: one chunk costs about 15 us in
 // three launches, 16 tokens one by one 24 us.
@@ -2372,6 +2434,29 @@ static long ck_rows_floats(int mode, int T_, int H, int DV) {
 
 template <typename T, int MODE>
 static void ck_read(CK_ARGS, const float* raw, const float* gx) {
+  if constexpr (MODE != CK_MLSTM) {
+    const int border = 16 / sizeof(T);
+    const size_t at = (size_t)out | (size_t)in.gate | (size_t)normw |
+                      (size_t)raw;
+    if (at % 16 == 0 && ldo % border == 0 && in.ldg % border == 0 &&
+        (long)T_ * H * DV < 1l << 32) {
+#define CK_READ(LPH)                                                         \
+  case 8 * LPH:                                                              \
+    hipLaunchKernelGGL((ck_readout_wide_kernel<T, MODE, LPH>),               \
+                       dim3(((long)T_ * H * LPH + 255) / 256), dim3(256), 0, \
+                       stream, (T*)out, ldo, raw, (const T*)in.gate, in.ldg, \
+                       (const float*)normw, (const int*)seq_rows, S_, T_, H, \
+                       eps);                                                 \
+    return;
+      switch (DV) {
+        CK_READ(4)
+        CK_READ(8)
+        CK_READ(16)
+        CK_READ(32)
+      }
+#undef CK_READ
+    }
+  }
 #define CK_READ(VEC)                                                         \
   hipLaunchKernelGGL((ck_readout_kernel<T, MODE, VEC>),                      \
                      dim3(T_, (H + 15) / 16), dim3(256), 0, stream, (T*)out, \

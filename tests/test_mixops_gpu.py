@@ -527,6 +527,44 @@ def test_talk_attention_scores_climb(shape, sink):
     assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,D", [(1, 32), (3, 32), (3, 64), (2, 128), (5, 96)])
+def test_recurrence_readout_borders(H, D, dtype):
+    """The read-out on 16-byte borders and off them (rows of the gate or of the
+    result moved by one entry): several rows in a wave and several waves a row,
+    rows of short segments between, before and behind those of chunks."""
+    g = torch.Generator(device="cuda").manual_seed(23)
+    rows = torch.tensor([[1, 40, 5, 2], [41, 3, 2, 0], [44, 17, 0, 1],
+                         [0, 1, 4, 3], [61, 1, 9, 4]], dtype=torch.int32,
+                        device="cuda")
+    T, HD = 62, H * D
+    v = [torch.randn(T, HD, generator=g, device="cuda").to(dtype)
+         for _ in range(5)]
+    par = [torch.randn(HD, generator=g, device="cuda") for _ in range(3)]
+    gate = torch.randn(T, HD, generator=g, device="cuda").to(dtype)
+    start = torch.randn(5, H, D, D, generator=g, device="cuda")
+
+    def run(pitch, lead, out_lead):
+        gp = torch.zeros(T, HD + pitch, dtype=dtype, device="cuda")
+        gp[:, lead:lead + HD] = gate
+        out = torch.full((T, HD + 16), 7.0, dtype=dtype, device="cuda")
+        state = start.clone()
+        ops.delta_rule(*v, gp[:, lead:lead + HD], *par, state, rows, H, 1e-5,
+                       0.6, out=out[:, out_lead:out_lead + HD])
+        assert (out[:, :out_lead] == 7.0).all()
+        assert (out[:, out_lead + HD:] == 7.0).all()
+        return out[:, out_lead:out_lead + HD].double(), state
+
+    want, ws = run(16, 0, 0)
+    for args in ((16, 1, 0), (17, 0, 0), (16, 0, 1)):
+        got, st = run(*args)
+        assert torch.equal(st, ws)
+        # the squares' sum in another order: a step of fp32, or one of bf16 where
+        # that crosses a border
+        tol = 2e-6 if dtype == torch.float32 else 2 ** -7
+        assert ((got - want).abs() <= tol * want.abs() + 1e-6).all()
+
+
 @pytest.mark.parametrize("lens,chunk,window", [
     ([2040], 0, 0),                  # 128 blocks: as they come
     ([1500, 549], 512, 0),           # 129 by length, one of two sequences
