@@ -185,6 +185,29 @@ PS_DEV CkSeg ck_by_length(const int* seq_rows, int S_, int rank) {
   return at;
 }
 
+// Sums of eight values over the wave: lanes 8 e .. 8 e + 7 return that of x[e].
+// Every step of the first three adds two halves of the lanes and keeps half of the
+// values in each, so that ten exchanges take the place of 48 one after the other.
+PS_DEV float ck_wave_sums(const float (&x)[8]) {
+  const int lane = threadIdx.x & 63;
+  float a[4], b[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const bool up = lane & 32;
+    a[i] = (up ? x[4 + i] : x[i]) + __shfl_xor(up ? x[i] : x[4 + i], 32, 64);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const bool up = lane & 16;
+    b[i] = (up ? a[2 + i] : a[i]) + __shfl_xor(up ? a[i] : a[2 + i], 16, 64);
+  }
+  const bool up = lane & 8;
+  float s = (up ? b[1] : b[0]) + __shfl_xor(up ? b[0] : b[1], 8, 64);
+#pragma unroll
+  for (int d = 4; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
+  return s;
+}
+
 template <typename T, int MODE, int DP>
 __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
     float* __restrict__ items, CkIn in, const int* __restrict__ seq_rows,
@@ -259,14 +282,19 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
 
   // unit vectors
   if (MODE != CK_GLA) {
+    float sq[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float k2 = mx_wave_sum(kv[e] * kv[e]);
-      const float r2 = MODE == CK_CD ? mx_wave_sum(rv[e] * rv[e]) : 0.f;
-      if (lane == 0) {
-        red[0][half * 8 + e][wave & 1] = k2;
-        red[1][half * 8 + e][wave & 1] = r2;
-      }
+    for (int e = 0; e < 8; ++e) sq[e] = kv[e] * kv[e];
+    const float k2 = ck_wave_sums(sq);
+    float r2 = 0.f;
+    if (MODE == CK_CD) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sq[e] = rv[e] * rv[e];
+      r2 = ck_wave_sums(sq);
+    }
+    if ((lane & 7) == 0) {
+      red[0][half * 8 + (lane >> 3)][wave & 1] = k2;
+      red[1][half * 8 + (lane >> 3)][wave & 1] = r2;
     }
   }
   // products of the decays within the half
@@ -2345,7 +2373,8 @@ static long ck_chunk_floats(int mode, int dp, int H, int G, int L) {
 //   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.70 ms
 //     (operands 0.24, walk 0.41, read-out 0.04)
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
-//                                                            5.42 -> 0.53 ms
+//                                                            5.42 -> 0.49 ms
+//     (its operands' logarithms and wave sums 0.04 less than before)
 //   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.30 ms
 //   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.06 ms
 //   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.47 ms

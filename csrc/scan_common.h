@@ -50,10 +50,31 @@ PS_DEV float ck_sigmoid(float x) {
   return ck_rcp(1.f + ck_exp(x < -80.f ? 80.f : -x));
 }
 
-PS_DEV float ck_softplus(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+// log(1 + exp(-|z|)) as 2 artanh(s), s = e / (2 + e) <= 1 / 3, by its series up to
+// s^13 (what is left is below 2e-8 of it), s with its rounding error beside it. Its
+// errors are those of log1pf(expf()) (softplus: 2.24 units of 2^-24 at most, 0.42 in
+// the mean), in a third of the instructions; they were half of those that laid down
+// the channel delta's operands (6007 rows of 32 x 128x128: 531 -> 495 us in all).
+PS_DEV float ck_log1p_exp(float z) {
+  const float e = expf(-fabsf(z));
+  const float d = 2.f + e, de = (2.f - d) + e;  // d + de = 2 + e
+  const float r = __builtin_amdgcn_rcpf(d);
+  float s = e * r;
+  s = fmaf(fmaf(-s, de, fmaf(-d, s, e)), r, s);
+  const float lo = fmaf(-s, de, fmaf(-d, s, e)) * r;
+  const float q = s * s;
+  float p = fmaf(q, 1.f / 13.f, 1.f / 11.f);
+  p = fmaf(q, p, 1.f / 9.f);
+  p = fmaf(q, p, 1.f / 7.f);
+  p = fmaf(q, p, 1.f / 5.f);
+  p = fmaf(q, p, 1.f / 3.f);
+  return 2.f * (fmaf(s * q, p, lo) + s);
+}
+
+PS_DEV float ck_softplus(float z) { return fmaxf(z, 0.f) + ck_log1p_exp(z); }
 
 PS_DEV float ck_log_sigmoid(float z) {
-  return fminf(z, 0.f) - log1pf(expf(-fabsf(z)));
+  return fminf(z, 0.f) - ck_log1p_exp(z);
 }
 
 // fp32 numbers on the bf16 matrix unit: each finite one is exactly the sum of

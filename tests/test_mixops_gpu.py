@@ -565,6 +565,30 @@ def test_recurrence_readout_borders(H, D, dtype):
         assert ((got - want).abs() <= tol * want.abs() + 1e-6).all()
 
 
+def test_recurrence_softplus_range():
+    """Step sizes of the state-space scan from the smallest to the largest argument,
+    read from the state that one row of ones leaves: 2.3 steps of fp32 (as
+    log1pf(expf()) has at most), and one more where the sum is rounded."""
+    z = torch.cat([torch.linspace(-87, 100, 3000), torch.linspace(-4, 4, 1086),
+                   torch.tensor([0.0, -0.0, 1e-30, -1e-30, 20.0, 2e4, 3e38,
+                                 -3e38, float("inf"), float("-inf")])])
+    H = z.numel()
+    one = torch.ones(1, 1, device="cuda")
+    state = torch.zeros(1, H, 1, 1, device="cuda")
+    rows = torch.tensor([[0, 1, 0, 0]], dtype=torch.int32, device="cuda")
+    zero = torch.zeros(H, device="cuda")
+    ops.linear_scan("ssd", one, one, one.expand(1, H).contiguous(),
+                    z.cuda()[None], zero[None], state, rows, H, 1, 1e-5,
+                    p0=zero, p1=zero, p2=zero, normw=one[0])
+    got, z = state.flatten().cpu().double(), z.double()
+    want = z.clamp(min=0) + torch.log1p(torch.exp(-z.abs()))
+    fin = torch.isfinite(want)
+    assert torch.equal(got[~fin], want[~fin])
+    got, want = got[fin], want[fin]
+    # below 2^-126 a step no longer follows the number
+    assert ((got - want).abs() <= 3.3 * 2 ** -24 * want + 2.0 ** -148).all()
+
+
 @pytest.mark.parametrize("lens,chunk,window", [
     ([2040], 0, 0),                  # 128 blocks: as they come
     ([1500, 549], 512, 0),           # 129 by length, one of two sequences
