@@ -22,9 +22,14 @@
 // wider values and odd widths) staged 32 keys between two barriers with nothing
 // in flight and read values as single 16-bit words. 32/8 heads of 128, two
 // prompts of 2048: 159 us, 159 with a window of 1024 and a cap (598 and 408
-// before; 182 with the cap's subtraction of the running maximum on its own); 256
-// rows behind 2048 keys 91 (302). Raised wave priority during the products made
-// it 5 % slower.
+// before; 182 with the cap's subtraction of the reference on its own); 256
+// rows behind 2048 keys 91 (302). A reference that stays while no score passes it
+// by 16 times: 8069 rows of two prompts, window 2048 and a cap, 530 -> 503 us, 32/8
+// heads of 64 86 -> 72. (Matrix pipe busy 48 % of it, each wave issuing 45 %.)
+// Raised wave priority during the products made it 5 % slower, the bf16
+// dot product in the weights' cut 2 %; bank conflicts in half the value reads, gone
+// with the row pitch, and the first 32 keys' scores beside the second 32 keys'
+// products cost and gave nothing.
 // The token form is bound by the keys and values it reads, at few tokens by the
 // latency of its tiles: 64 tokens x 4001 keys 177 us, 5.9 TB/s (424 before);
 // window 1024 42 us (119); 8 tokens of it 16 us (32).
@@ -67,7 +72,8 @@ PS_DEV float wa_score(const WaArgs& a, float st, float base, float top) {
 // DK: 16-entry steps of a key (D <= 16 DK), VB: 32-column blocks of a value
 template <int DK, int VB, bool CAP>
 __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
-  constexpr int PK = DK * 16 + 8, PV = VB * 32 + 8;
+  // values: the four rows of a transposed read lie 16 banks apart
+  constexpr int PK = DK * 16 + 8, PV = VB * 32 + 32;
   __shared__ __align__(16) unsigned short sK[2][WA_KT * PK];
   __shared__ __align__(16) unsigned short sV[2][WA_KT * PV];
   __shared__ int s_row[2][WA_KT];

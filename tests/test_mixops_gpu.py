@@ -527,6 +527,38 @@ def test_talk_attention_scores_climb(shape, sink):
     assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
 
 
+@pytest.mark.parametrize("grow", [0.03, 0.2, -0.1])
+@pytest.mark.parametrize("softcap", [0.0, 50.0])
+def test_window_attention_scores_climb(grow, softcap):
+    """Scores that climb by less than the weights' reference waits for in a tile,
+    by more than that in each, or fall from the first key on: as portions and as
+    single tokens with one and several shares."""
+    g = torch.Generator().manual_seed(29)
+    H, G, D, bs, L = 8, 2, 64, 16, 330
+    kc, vc, tables = _paged(L, G, D, D, bs, torch.bfloat16, g, 2)
+    f = grow * torch.arange(tables.shape[1] * bs).float()
+    for j in range(tables.shape[1]):
+        kc[tables[0, j], :, :, 0] += f[j * bs:(j + 1) * bs].to(torch.bfloat16)
+    ts = torch.tensor([0] * 40 + [1] * 12, dtype=torch.int32)
+    tp = torch.tensor(list(range(280, 320)) + list(range(100, 112)),
+                      dtype=torch.int32)
+    T = len(ts)
+    q = torch.randn(T, H, D, generator=g)
+    q[:, :, 0] = 8.0 + q[:, :, 0].abs()
+    q = q.to(torch.bfloat16)
+    want = reference.talk_attention(
+        q.float(), kc.float(), vc.float(), tables, ts, tp, D ** -0.5, 0, 250,
+        True, None, softcap=softcap, keep_first=70)
+    dev = [x.cuda() for x in (q.view(T, H * D), kc, vc, tables, ts, tp)]
+    for kw in ({"variant": 0}, {"variant": 3},
+               {"variant": 3, "splits": 3}):
+        got = ops.talk_attention(*dev, D ** -0.5, H, window=250, sink=True,
+                                 softcap=softcap, keep_first=70, **kw)
+        # fp32 up to the bf16 rounding of the result; scores of up to 70 in sums
+        # of 64 terms are 2e-5 off, and their weights with them
+        assert _rel(got.float().cpu().reshape(T, H, D), want) < 3e-3, kw
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,D", [(1, 32), (3, 32), (3, 64), (2, 128), (5, 96)])
 def test_recurrence_readout_borders(H, D, dtype):
