@@ -229,55 +229,66 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
 
   // which chunk of which segment
   const int item = blockIdx.x, hd = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int seg, chunk;
   if (!ck_find(seq_rows, S_, base + item, lane, &seg, &chunk)) return;
+  // the same in all lanes: rows' addresses are a scalar and one offset per lane,
+  // and what depends on the half a branch
+  seg = __builtin_amdgcn_readfirstlane(seg);
+  chunk = __builtin_amdgcn_readfirstlane(chunk);
   const int n = seq_rows[4 * seg + 1];
   const int row0 = seq_rows[4 * seg] + 16 * chunk;
   const int nv = min(16, n - 16 * chunk);
 
-  const int half = threadIdx.x >> 7, d = threadIdx.x & 127;
+  const int half = wave >> 1, d = threadIdx.x & 127;
   const bool on = d < DP, real = d < D;
   const int grp = hd / (H / G);
-  const int hk = MODE == CK_GD ? hd * D + d : grp * D + d;
-  const int hz = hd * D + d;
 
-  const T* qp = (const T*)in.q;
-  const T* kp = (const T*)in.k;
-  const T* zp = (const T*)in.dec;
-  const T* ap = (const T*)in.a;
-  float kv[8], rv[8], wv[8], av[8];
   // all loads ahead of any use, from a row and a channel that exist
-  const int dc = real ? 0 : -d;
+  const int dc = real ? d : 0;
+  const unsigned at_c = dc * sizeof(T);
+  const size_t h0 = (size_t)hd * D;
+  const size_t k0 = MODE == CK_GD ? h0 : (size_t)grp * D;
+  auto get = [&](const void* p, size_t row, int ld, size_t c, unsigned at) {
+    return MxElem<T>::ld(
+        (const T*)((const char*)((const T*)p + row * ld + c) + at));
+  };
+  float kv[8], rv[8], wv[8], av[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const size_t row = (size_t)(row0 + min(half * 8 + e, nv - 1));
-    kv[e] = MxElem<T>::ld(kp + row * in.ldk + hk + dc);
-    rv[e] = MxElem<T>::ld(qp + row * in.ldq + hk + dc);
-    wv[e] = MxElem<T>::ld(zp + row * in.lddec + hz + dc);
+    kv[e] = get(in.k, row, in.ldk, k0, at_c);
+    rv[e] = get(in.q, row, in.ldq, k0, at_c);
+    wv[e] = get(in.dec, row, in.lddec, h0, at_c);
     av[e] = 0.f;
-    if (MODE == CK_GD) av[e] = MxElem<T>::ld(ap + row * in.lda + hz + dc);
-    if (MODE == CK_CD) av[e] = MxElem<T>::ld(ap + row * in.lda + hd);
+    if (MODE == CK_GD) av[e] = get(in.a, row, in.lda, h0, at_c);
+    if (MODE == CK_CD) av[e] = get(in.a, row, in.lda, hd, 0);
   }
-  const float c0z = in.p0[hz + dc];
+  const float c0z = in.p0[h0 + dc];
   float c1 = 0.f;
-  if (MODE == CK_GD) c1 = in.p1[hz + dc];
+  if (MODE == CK_GD) c1 = in.p1[h0 + dc];
   if (MODE == CK_CD) c1 = expf(in.p1[hd]);
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const bool live = real && half * 8 + e < nv;
-    float w;
     if (MODE == CK_GD) {
-      w = ck_exp(-scale * ck_sigmoid(wv[e] + c0z));
+      wv[e] = ck_exp(-scale * ck_sigmoid(wv[e] + c0z));
       av[e] = ck_sigmoid(av[e] + c1);
     } else if (MODE == CK_CD) {
-      w = ck_exp(-c1 * ck_softplus(wv[e] + c0z));
+      wv[e] = ck_exp(-c1 * ck_softplus(wv[e] + c0z));
       av[e] = ck_sigmoid(av[e]);
     } else {
-      w = ck_exp(ck_log_sigmoid(wv[e] + c0z) * c0f);
+      wv[e] = ck_exp(ck_log_sigmoid(wv[e] + c0z) * c0f);
     }
-    wv[e] = live ? w : 1.f;  // rows past the segment's end change nothing
-    if (!live) kv[e] = rv[e] = av[e] = 0.f;
+  }
+  // rows past the segment's end and channels past the head's change nothing
+  if (DP != 128 || D != DP || nv != 16) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const bool live = real && half * 8 + e < nv;
+      wv[e] = live ? wv[e] : 1.f;
+      if (!live) kv[e] = rv[e] = av[e] = 0.f;
+    }
   }
 
   // unit vectors
@@ -321,8 +332,8 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
     mag += fabsf(kv[e]) + fabsf(rv[e]) + fabsf(wv[e]) + fabsf(av[e]);
   const bool odd = __syncthreads_or(!(mag < INFINITY));
   // out of range (or no number): ratios are formed one by one
-  const bool slow =
-      __syncthreads_or(on && !(pin[7] > 1e-30f && pin[7] < 1e30f));
+  const bool slow = __builtin_amdgcn_readfirstlane(
+      __syncthreads_or(on && !(pin[7] > 1e-30f && pin[7] < 1e30f)));
   const float other = half_prod[half ^ 1][d];
 
   float uv[8], bv[8];  // u (GD) / k^ (CD); b
@@ -346,30 +357,46 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
   }
 
   if (on) {
-    // W_t counted from the middle (W_7 = 1) and its inverse; general delta's
-    // reading rows take W_{t-1}
-    float inv[8];
+    // operand rows of token e: wt, iw W_t counted from the middle (W_7 = 1) and
+    // its inverse; general delta's reading rows take W_{t-1} (wp)
+    auto put = [&](int e, float wt, float iw, float wp) {
+      const int at = (half * 8 + e) * LD + d;
+      if (MODE == CK_GD) X0[at] = uv[e] * wp;
+      if (MODE == CK_CD) X0[at] = uv[e] * wt;
+      X1[at] = rv[e] * wt;
+      if (MODE == CK_GD) Y0[at] = bv[e] * iw;
+      Y1[at] = kv[e] * iw;
+    };
+    // what reads the state before the chunk: products from its start
+    auto reads = [&](int e, float before, float to) {
+      if (MODE == CK_GD) su[(half * 8 + e) * LD + d] = uv[e] * before;
+      if (MODE == CK_CD) su[(half * 8 + e) * LD + d] = uv[e] * to;
+    };
+    if (half == 0) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) inv[e] = ck_rcp(half == 0 ? suf[e] : pin[e]);
-    const float from = half == 0 ? 1.f : other;
+      for (int e = 0; e < 8; ++e)
+        reads(e, e > 0 ? pin[e > 0 ? e - 1 : 0] : 1.f, pin[e]);
+    } else {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int tt = half * 8 + e;
-      float wt = half == 0 ? inv[e] : pin[e];
-      float iw = half == 0 ? suf[e] : inv[e];
-      float wp = half == 0 ? (e > 0 ? inv[e > 0 ? e - 1 : 0] : 0.f)
-                           : (e > 0 ? pin[e > 0 ? e - 1 : 0] : 1.f);
-      if (slow) wt = iw = wp = 1.f;
-      if (MODE == CK_GD) X0[tt * LD + d] = uv[e] * wp;
-      if (MODE == CK_CD) X0[tt * LD + d] = uv[e] * wt;
-      X1[tt * LD + d] = rv[e] * wt;
-      if (MODE == CK_GD) Y0[tt * LD + d] = bv[e] * iw;
-      Y1[tt * LD + d] = kv[e] * iw;
-      // what reads the state before the chunk: products from its start
-      if (MODE == CK_GD)
-        su[tt * LD + d] =
-            uv[e] * (e > 0 ? from * pin[e > 0 ? e - 1 : 0] : from);
-      if (MODE == CK_CD) su[tt * LD + d] = uv[e] * (from * pin[e]);
+      for (int e = 0; e < 8; ++e)
+        reads(e, e > 0 ? other * pin[e > 0 ? e - 1 : 0] : other,
+              other * pin[e]);
+    }
+    if (slow) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) put(e, 1.f, 1.f, 1.f);
+    } else if (half == 0) {
+      float before = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float inv = ck_rcp(suf[e]);
+        put(e, inv, suf[e], before);
+        before = inv;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        put(e, pin[e], ck_rcp(pin[e]), e > 0 ? pin[e > 0 ? e - 1 : 0] : 1.f);
     }
   }
   __syncthreads();
@@ -455,14 +482,17 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
   if (on) {
     const int t = d >> 4, dg = (d & 15) >> 2, di = d & 3;
     float kf[8], bf[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int tt = half * 8 + e;
-      const float from = half == 0 ? pin[e] : other * pin[e];
-      const float to = half == 0 ? suf[e] * other : suf[e];
-      stage[It::R + ck_row_slot(t, dg, tt) * 4 + di] = rv[e] * from;
+    auto scaled = [&](int e, float from, float to) {
+      stage[It::R + ck_row_slot(t, dg, half * 8 + e) * 4 + di] = rv[e] * from;
       kf[e] = kv[e] * to;
       bf[e] = bv[e] * to;
+    };
+    if (half == 0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) scaled(e, pin[e], suf[e] * other);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) scaled(e, other * pin[e], suf[e]);
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -2370,8 +2400,8 @@ static long ck_chunk_floats(int mode, int dp, int H, int G, int L) {
 }
 
 // Measured (bf16, one MI355X, whole operation; token by token -> this form):
-//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.70 ms
-//     (operands 0.24, walk 0.41, read-out 0.04)
+//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.68 ms
+//     (operands 0.22, walk 0.41, read-out 0.04)
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
 //                                                            5.42 -> 0.49 ms
 //     (its operands' logarithms and wave sums 0.04 less than before)
