@@ -153,6 +153,47 @@ def test_paged_attn_decode_many_heads(S, qh, kh, hd, window, fp8):
     _close(got.cpu()[some], want)
 
 
+@pytest.mark.parametrize("S,qh,kh,hd,window,fp8,longest", [
+    (33, 16, 8, 128, 0, False, 1100),   # one sequence past the CUs' first round
+    (64, 16, 8, 128, 0, True, 5000),    # second round full, a split of the longest
+    (66, 32, 32, 128, 0, False, 1100),  # a wave per head among long ones
+    (257, 8, 1, 64, 0, False, 1100),    # one head, five counts a lane
+    (320, 8, 8, 128, 2100, False, 2300),
+    (321, 8, 8, 128, 0, False, 1100),   # as they come
+    (64, 16, 8, 128, 0, False, -1100)])  # within an eighth: as they come
+def test_paged_attn_decode_by_length(S, qh, kh, hd, window, fp8, longest):
+    """Sequences that workgroups take by their lengths: equal lengths, empty ones
+    and ones of a few tiles between long ones. Every row is written, as a launch
+    over few sequences (too few to be ordered) writes it."""
+    g = torch.Generator().manual_seed(S)
+    nb, max_blocks = 400, -(-abs(longest) // 16)
+    if longest < 0:
+        lens = torch.randint(1020, -longest, (S,), generator=g).int()
+    else:
+        edges = [0, 1, 32, 33, 64, 65, 128, 129, 512, 513, 700, 700, 1024]
+        lens = torch.tensor([edges[i] for i in torch.randint(
+            0, len(edges), (S,), generator=g)], dtype=torch.int32)
+        lens[S // 3] = lens[S - 1] = longest
+    k_cache, v_cache = _make_cache(nb, kh, 16, hd)
+    if fp8:
+        k_cache, v_cache = (c.to(torch.float8_e4m3fn)
+                            for c in (k_cache, v_cache))
+    tables = torch.randint(0, nb, (S, max_blocks), generator=g).int().cuda()
+    q = torch.randn((S, qh, hd), generator=g).to(torch.bfloat16).cuda()
+    lens = lens.cuda()
+
+    def run(a, b):
+        return ops.paged_attn_decode(q[a:b], k_cache, v_cache, tables[a:b],
+                                     lens[a:b], hd ** -0.5, window=window)
+
+    got = run(0, S)
+    few = max(1, 256 // kh)
+    want = torch.cat([run(a, min(a + few, S)) for a in range(0, S, few)])
+    assert not got[lens == 0].any()
+    # sums split at other keys: fp32 up to the bf16 rounding of the result
+    _close(got, want.cpu())
+
+
 @pytest.mark.parametrize("num_splits", [1, 2, 4, 8, 32])
 def test_paged_attn_decode_split_kv(num_splits):
     """All split factors must agree with the reference (incl. splits that
