@@ -816,3 +816,49 @@ def test_no_graph_is_collected_during_a_capture(monkeypatch):
             assert now["inside"] == 0 and now["gone"] >= 8
     finally:
         gc.enable() if old else gc.disable()
+
+
+def test_graph_inputs_in_one_transfer(monkeypatch):
+    """A step's inputs lie in one buffer: every one of the replayed bucket
+    arrives, rows past the step's are padding, in odd sizes of batch and table
+    and after steps of other buckets."""
+    import numpy as np
+
+    from production_stack_amd.engine import graph_runner
+
+    make = torch.zeros
+    monkeypatch.setattr(torch, "zeros", lambda *a, pin_memory=False, **kw:
+                        make(*a, **kw))
+
+    class Model:
+        needs_seq_meta = True
+        lora_slots = object()
+
+    class Graph:
+        def replay(self):
+            pass
+
+    r = graph_runner.DecodeGraphRunner(Model(), [], 5, 3,
+                                       torch.device("cpu"), 77)
+    assert r.buckets == [1, 2, 4, 5]
+    for b in r.buckets:
+        r.graphs[b], r.logits[b] = Graph(), torch.empty(b, 1)
+    for n in (5, 3, 1, 4, 2):
+        b = r.bucket_for(n)
+        i = np.arange(n)
+        tables = [[10 * n + k] * (1 + k % 3) for k in range(n)]
+        r.run(100 + i, 7 * i + n, 1000 + i, i + 2, tables, lora_idx=i % 2,
+              state_slots=i + 30)
+        pad = b - n
+        for got, want, fill in (
+                (r.tokens, 100 + i, 0), (r.positions, 7 * i + n, 0),
+                (r.slots, 1000 + i, -1), (r.seq_lens, i + 2, 1),
+                (r.lora_idx, i % 2, -1), (r.seq_rows[:, 0], i, n),
+                (r.seq_rows[:, 1], i * 0 + 1, 1),
+                (r.seq_rows[:, 2], 7 * i + n, 0),
+                (r.seq_rows[:, 3], i + 30, 77)):
+            assert got[:b].tolist() == want.tolist() + [fill] * pad
+        for k, t in enumerate(tables):
+            assert r.block_tables[k, :len(t)].tolist() == t
+        if pad:
+            assert (r.block_tables[n:b, 0] == 0).all()
