@@ -284,51 +284,49 @@ class LlamaLayer(nn.Module):
                 meta.slot_mapping,
             )
             qh = q.view(T, self.q_heads, self.head_dim)
-        outs: List[torch.Tensor] = []
+        # both kinds of rows of a mixed step into one buffer
         tp = meta.num_prefill_tokens
+        attn = torch.empty((T, self.q_heads, self.head_dim), dtype=qh.dtype,
+                           device=qh.device)
         if tp > 0:
             if (
                 qh.is_cuda
                 and self.head_dim == 128
                 and meta.prefill_tiles is not None
             ):
-                outs.append(
-                    ops.paged_attn_prefill_mfma(
-                        qh[:tp],
-                        k_cache,
-                        v_cache,
-                        meta.prefill_block_tables,
-                        meta.prefill_tiles,
-                        self.scale,
-                        self.window,
-                    )
-                )
-            else:
-                outs.append(
-                    ops.paged_attn_prefill(
-                        qh[:tp] if qh.is_cuda else qh[:tp].contiguous(),
-                        k_cache,
-                        v_cache,
-                        meta.prefill_block_tables,
-                        meta.prefill_token_seq,
-                        meta.prefill_token_pos,
-                        self.scale,
-                        self.window,
-                    )
-                )
-        if meta.num_decode_seqs > 0:
-            outs.append(
-                ops.paged_attn_decode(
-                    qh[tp:] if qh.is_cuda else qh[tp:].contiguous(),
+                ops.paged_attn_prefill_mfma(
+                    qh[:tp],
                     k_cache,
                     v_cache,
-                    meta.decode_block_tables,
-                    meta.decode_seq_lens,
+                    meta.prefill_block_tables,
+                    meta.prefill_tiles,
                     self.scale,
                     self.window,
+                    out=attn[:tp],
                 )
+            else:
+                ops.paged_attn_prefill(
+                    qh[:tp] if qh.is_cuda else qh[:tp].contiguous(),
+                    k_cache,
+                    v_cache,
+                    meta.prefill_block_tables,
+                    meta.prefill_token_seq,
+                    meta.prefill_token_pos,
+                    self.scale,
+                    self.window,
+                    out=attn[:tp],
+                )
+        if meta.num_decode_seqs > 0:
+            ops.paged_attn_decode(
+                qh[tp:] if qh.is_cuda else qh[tp:].contiguous(),
+                k_cache,
+                v_cache,
+                meta.decode_block_tables,
+                meta.decode_seq_lens,
+                self.scale,
+                self.window,
+                out=attn[tp:],
             )
-        attn = torch.cat(outs, dim=0) if len(outs) > 1 else outs[0]
         attn_out = None
         if few and self.tp == 1 and not self.n_experts:
             attn_out = gemm_policy.parts(attn.view(T, qs), self.o_proj, "norm")

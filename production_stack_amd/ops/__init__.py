@@ -149,18 +149,21 @@ def paged_attn_decode(
     seq_lens: torch.Tensor,
     scale: float,
     window: int = 0,
+    out: torch.Tensor = None,
 ) -> torch.Tensor:
     if q.is_cuda:
         _require_ext()
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        if out is None:
+            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         _C.paged_attn_decode(
             out, q, k_cache, v_cache, block_tables, seq_lens, scale, 0, 0,
             window
         )
         return out
-    return reference.paged_attn_decode(
+    want = reference.paged_attn_decode(
         q, k_cache, v_cache, block_tables, seq_lens, scale, window
     )
+    return want if out is None else out.copy_(want)
 
 
 def paged_attn_prefill(
@@ -172,19 +175,22 @@ def paged_attn_prefill(
     token_pos: torch.Tensor,
     scale: float,
     window: int = 0,
+    out: torch.Tensor = None,
 ) -> torch.Tensor:
     if q.is_cuda:
         _require_ext()
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        if out is None:
+            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         _C.paged_attn_prefill(
             out, q, k_cache, v_cache, block_tables, token_seq, token_pos,
             scale, window
         )
         return out
-    return reference.paged_attn_prefill(
+    want = reference.paged_attn_prefill(
         q, k_cache, v_cache, block_tables, token_seq, token_pos, scale,
         window
     )
+    return want if out is None else out.copy_(want)
 
 
 # Default MFMA prefill variant: 5 = 8-wave 32x32 swapped-QK^T kernel
@@ -215,12 +221,14 @@ def paged_attn_prefill_mfma(
     scale: float,
     window: int = 0,
     variant: int = None,
+    out: torch.Tensor = None,
 ) -> torch.Tensor:
     """MFMA-tiled chunked prefill (GPU, head_dim 128 only). tile_info rows
     must be built with n_rows <= prefill_tile_rows() for the active
     variant."""
     _require_ext()
-    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    if out is None:
+        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     # v5's split-KV (up to 8 kv-splits) keeps CUs filled at small
     # serving launches, where it now beats v3 at the canonical shapes
     # (12-seq x 200-row continuation at hist 4600: 305 vs 263 TF; fresh
