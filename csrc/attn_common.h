@@ -104,3 +104,74 @@ PS_DEV void kv_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
+
+// Which of `count` sequences a workgroup at place `pos` of as many has: the longest
+// ones first, so that none starts late, but the second of two rounds of the CUs
+// (`half` places each) from the shortest on, as its workgroups join the first
+// round's on their CUs: every CU then has about as many keys to read, and all of
+// them stay busy to the end. As sequences come, a CU has two long ones while another
+// is done with two short ones.
+// Found without a sort: the tile count (at most `most`) that `rank` sequences exceed,
+// bit by bit, among counts that the lanes hold. All keep their places where none has
+// more than KV_SHORT tiles or every one as many as the first, within an eighth. In
+// more than four rounds, where workgroups start as others end, those of up to
+// KV_SHORT tiles keep theirs (`mine` is the place's own count) and do not wait for
+// the others' lengths (32/8 heads, 256 x 20 to 300 keys 37 us, 41 otherwise); in few
+// they have to pair with long ones (61 of 300 to 4000 98 us, 109 otherwise).
+#define KV_ORDER 320  // sequences at most
+#define KV_SHORT 16
+template <typename F>
+PS_DEV int kv_order(F tiles_of, int count, int pos, int lane, int half,
+                    int mine, int most) {
+  const int skip = count > 4 * half ? KV_SHORT : 0;
+  if (mine <= skip) return pos;
+  int tiles[KV_ORDER / 64];
+#pragma unroll
+  for (int j = 0; j < KV_ORDER / 64; ++j) {
+    const int s = j * 64 + lane;
+    tiles[j] = s < count ? tiles_of(s) : -1;
+  }
+  auto above = [&](int t) {  // sequences of more than t tiles
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < KV_ORDER / 64; ++j)
+      if (j * 64 < count) n += __popcll(__ballot(tiles[j] > t));
+    return n;
+  };
+  const int first = __builtin_amdgcn_readfirstlane(tiles[0]);
+  bool even = true;  // all within an eighth of the first one
+#pragma unroll
+  for (int j = 0; j < KV_ORDER / 64; ++j)
+    if (j * 64 < count)
+      even &= __all(tiles[j] < 0 || abs(tiles[j] - first) <= first / 8);
+  int seq = pos;
+  if (!even && above(KV_SHORT) > 0) {
+    int rank = 0;  // of this place among those of longer ones
+#pragma unroll
+    for (int j = 0; j < KV_ORDER / 64; ++j) {
+      const int at = min(pos - 64 * j, 64);
+      if (at > 0)
+        rank += __popcll(__ballot(tiles[j] > skip && lane < at));
+    }
+    const int end = min(2 * half, above(skip));
+    if (rank >= half && rank < end) rank = half + end - 1 - rank;
+    int t = 0;
+    for (int b = 31 - __clz(most | 1); b >= 0; --b)
+      if (above(t + (1 << b) - 1) > rank) t += 1 << b;
+    int left = rank - above(t);  // which of those of t tiles
+#pragma unroll
+    for (int j = 0; j < KV_ORDER / 64; ++j) {
+      const unsigned long long m = __ballot(tiles[j] == t);
+      const int n = __popcll(m);
+      if (left >= 0 && left < n) {
+        const int before = __builtin_amdgcn_mbcnt_hi(
+            (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+        seq = j * 64 + __ffsll((unsigned long long)__ballot(
+                           tiles[j] == t && before == left)) - 1;
+      }
+      left -= n;
+    }
+    seq = __builtin_amdgcn_readfirstlane(seq);
+  }
+  return seq;
+}

@@ -61,79 +61,15 @@ PS_DEV int da_tiles(const DaArgs& a, int ctx) {
   return ((a.window > 0 ? min(ctx, a.window) : ctx) + TT - 1) / TT;
 }
 
-// Which sequence a workgroup at place `pos` of 0 .. seqs - 1 has: the longest
-// ones first, so that none starts late, but the second of two rounds of the CUs
-// from the shortest on, as its workgroups join the first round's on their CUs:
-// every CU then has about as many keys to read, and all of them stay busy to the
-// end. As the sequences came, a CU had two long ones while another was done with
-// two short ones (32/8 heads of 128, us, as they come / longest first / this / all
-// of one length: 61 sequences of 300 to 4000 keys 117 / 105 / 93 / 92, 100 of 500
-// to 3000 157 / 136 / 131 / 142; fp8, 192 of 1200 to 5500 250 / 228 / 227 / 227).
-// Found without a sort: the tile count that `rank` sequences exceed, bit by bit,
-// among counts that the lanes hold. Empty sequences and those of a wave per head (up
-// to a.packed tiles) keep their places, and so do all where none has more than
-// DA_SHORT tiles or every one as many as the first, within an eighth.
-#define DA_ORDER 320  // sequences at most
-#define DA_SHORT 16
+// The sequence of a place (see kv_order). 32/8 heads of 128, us, as they come /
+// longest first / this / all of one length: 61 sequences of 300 to 4000 keys 117 /
+// 105 / 93 / 92, 100 of 500 to 3000 157 / 136 / 131 / 142; fp8, 192 of 1200 to 5500
+// 250 / 228 / 227 / 227.
 template <int TT>
-PS_DEV int da_order(const DaArgs& a, int pos, int lane) {
-  int tiles[DA_ORDER / 64];
-#pragma unroll
-  for (int j = 0; j < DA_ORDER / 64; ++j) {
-    const int s = j * 64 + lane;
-    tiles[j] = s < a.seqs ? da_tiles<TT>(a, a.seq_lens[s]) : -1;
-  }
-  auto above = [&](int t) {  // sequences of more than t tiles
-    int n = 0;
-#pragma unroll
-    for (int j = 0; j < DA_ORDER / 64; ++j)
-      if (j * 64 < a.seqs) n += __popcll(__ballot(tiles[j] > t));
-    return n;
-  };
-  const int first = __builtin_amdgcn_readfirstlane(tiles[0]);
-  bool even = true;  // all within an eighth of the first one
-#pragma unroll
-  for (int j = 0; j < DA_ORDER / 64; ++j)
-    if (j * 64 < a.seqs)
-      even &= __all(tiles[j] < 0 || abs(tiles[j] - first) <= first / 8);
-  int seq = pos;
-  if (!even && above(DA_SHORT) > 0) {
-    int rank = 0;       // of this place among those of more than a.packed tiles
-    bool moves = false;  // whether it is one of them
-#pragma unroll
-    for (int j = 0; j < DA_ORDER / 64; ++j) {
-      const unsigned long long m = __ballot(tiles[j] > a.packed);
-      const int at = pos - 64 * j;
-      if (at >= 64) {
-        rank += __popcll(m);
-      } else if (at >= 0) {
-        rank += __popcll(m & ((1ull << at) - 1));
-        moves = m >> at & 1;
-      }
-    }
-    if (!moves) return pos;
-    const int half = 256 / a.KH;  // sequences of one round of the CUs
-    const int end = min(2 * half, above(a.packed));
-    if (rank >= half && rank < end) rank = half + end - 1 - rank;
-    int t = 0;
-    for (int b = 31 - __clz((a.max_blocks * 16 + TT - 1) / TT | 1); b >= 0; --b)
-      if (above(t + (1 << b) - 1) > rank) t += 1 << b;
-    int left = rank - above(t);  // which of those of t tiles
-#pragma unroll
-    for (int j = 0; j < DA_ORDER / 64; ++j) {
-      const unsigned long long m = __ballot(tiles[j] == t);
-      const int n = __popcll(m);
-      if (left >= 0 && left < n) {
-        const int before = __builtin_amdgcn_mbcnt_hi(
-            (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
-        seq = j * 64 + __ffsll((unsigned long long)__ballot(
-                           tiles[j] == t && before == left)) - 1;
-      }
-      left -= n;
-    }
-    seq = __builtin_amdgcn_readfirstlane(seq);
-  }
-  return seq;
+PS_DEV int da_order(const DaArgs& a, int pos, int ctx, int lane) {
+  return kv_order([&](int s) { return da_tiles<TT>(a, a.seq_lens[s]); }, a.seqs,
+                  pos, lane, 256 / a.KH, da_tiles<TT>(a, ctx),
+                  (a.max_blocks * 16 + TT - 1) / TT);
 }
 
 // 8 fp8 entries as bf16
@@ -181,8 +117,8 @@ __global__ __launch_bounds__(256, WPE) void paged_attn_decode_kernel(DaArgs a) {
   const int split = r / a.seqs;
   const int pos = (r - split * a.seqs + split) % a.seqs;
   int seq = pos, ctx = a.seq_lens[pos];
-  if (a.order && (a.packed == 0 || da_tiles<TT>(a, ctx) > a.packed)) {
-    seq = da_order<TT>(a, pos, lane);
+  if (a.order) {
+    seq = da_order<TT>(a, pos, ctx, lane);
     if (seq != pos) ctx = a.seq_lens[seq];
   }
   const int lo = a.window > 0 && ctx > a.window ? ctx - a.window : 0;
@@ -480,7 +416,7 @@ extern "C" int ps_paged_attn_decode(
   const int width =
       window > 0 ? std::min(window, max_blocks * 16) : max_blocks * 16;
   const int order =
-      num_seqs * KH > 256 && num_seqs <= DA_ORDER &&
+      num_seqs * KH > 256 && num_seqs <= KV_ORDER &&
       width > (window > 0 ? 2048 : 1024);
   const DaArgs a = {(unsigned short*)out,
                     (float*)ws_acc,

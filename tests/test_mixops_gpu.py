@@ -527,6 +527,35 @@ def test_talk_attention_scores_climb(shape, sink):
     assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
 
 
+@pytest.mark.parametrize("T,G,window", [(33, 8, 0), (70, 8, 1500),
+                                        (150, 8, 0), (320, 1, 0), (321, 1, 0)])
+def test_window_attention_token_order(T, G, window):
+    """Single tokens that workgroups take by their keys (a round of the CUs and
+    one, two and a remainder, more than four, at the most and past it): every row
+    is written, as a launch over few tokens (as they come) writes it."""
+    g = torch.Generator().manual_seed(T)
+    H, D, bs, nb = 2 * G, 64, 16, 300
+    n = torch.tensor([1, 31, 32, 33, 500, 512, 513, 1000, 1000, 1600])
+    pos = (n[torch.randint(0, 10, (T,), generator=g)] - 1).int()
+    pos[T // 2] = 1599
+    kc, vc = (torch.randn(nb, G, bs, D, generator=g).to(torch.bfloat16).cuda()
+              for _ in range(2))
+    tables = torch.randint(0, nb, (T, 100), generator=g).int().cuda()
+    q = torch.randn(T, H * D, generator=g).to(torch.bfloat16).cuda()
+    pos, seq = pos.cuda(), torch.arange(T, dtype=torch.int32).cuda()
+
+    def run(a, b):
+        return ops.talk_attention(
+            q[a:b], kc, vc, tables, seq[a:b], pos[a:b], D ** -0.5, H,
+            window=window, sink=True, keep_first=3 if window else 0, variant=3,
+            splits=1).float()
+
+    got, few = run(0, T), 256 // G
+    # the same tiles in the same waves
+    assert torch.equal(got, torch.cat([run(a, min(a + few, T))
+                                       for a in range(0, T, few)]))
+
+
 @pytest.mark.parametrize("grow", [0.03, 0.2, -0.1])
 @pytest.mark.parametrize("softcap", [0.0, 50.0])
 def test_window_attention_scores_climb(grow, softcap):
