@@ -1,8 +1,11 @@
 """Llama-family causal LM built on the MI355X op set.
 
 Compute mapping (MI355X-first):
-  * plain GEMMs (qkv / o / gate-up / down / lm_head) -> torch F.linear, which
-    lowers to hipBLASLt on ROCm;
+  * GEMMs (qkv / o / gate-up / down / lm_head) of up to 16 rows, and the
+    others of steps up to gemm_policy.MAX_ROWS rows where they are faster ->
+    the few-row kernels, with norm, rope and SiLU-mul in their launches or
+    adding up their sums; larger ones -> torch F.linear, which lowers to
+    hipBLASLt on ROCm;
   * everything else on the hot path is a hand-written HIP kernel via
     production_stack_amd.ops: fused residual-add RMSNorm, fused rope over
     q+k, paged-KV append, paged attention (prefill + decode), SiLU-mul.
@@ -11,7 +14,7 @@ Compute mapping (MI355X-first):
 
 Supports tensor parallelism: q/kv heads and the MLP intermediate dim are
 sharded across the TP group; o_proj and down_proj outputs are all-reduced
-(RCCL over xGMI on the GPU box, gloo in CPU tests).
+(RCCL over xGMI, gloo in CPU tests).
 """
 
 from __future__ import annotations
