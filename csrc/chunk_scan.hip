@@ -208,24 +208,31 @@ PS_DEV float ck_wave_sums(const float (&x)[8]) {
   return s;
 }
 
+// Lays down a chunk's operands: a workgroup per (chunk, head), a lane per channel
+// of eight rows. Bound by its vector instructions (1190 a wave for the general
+// delta, three waves a SIMD: registers), beside a write of 32 KB. Four workgroups a
+// CU spill for the channel delta (480 -> 500 us of its whole operation).
 template <typename T, int MODE, int DP>
-__global__ __launch_bounds__(256, 3) void ck_prep_kernel(
+__global__ __launch_bounds__(256, MODE == CK_GLA ? 4 : 3) void ck_prep_kernel(
     float* __restrict__ items, CkIn in, const int* __restrict__ seq_rows,
     int S_, int H, int G, int D, float scale, float c0f, int base) {
   typedef CkItem<MODE, DP> It;
   constexpr int LD = DP + 4;
-  // operand rows in channel order; reused for the fragments once the 16 x 16
-  // products are done
+  // operand rows in channel order; reused for the fragments that are not stored
+  // from registers (rows R and U, then what lies behind the rows) once the
+  // 16 x 16 products are done
+  constexpr int ROWS = MODE == CK_GD ? 4 : (MODE == CK_CD ? 3 : 2);
+  constexpr int SU = It::ROW, SO = (MODE == CK_GLA ? 1 : 2) * It::ROW - It::M;
   __shared__ __align__(16) float stage[
-      It::TOTAL > 4 * 16 * LD ? It::TOTAL : 4 * 16 * LD];
+      It::TOTAL + SO > ROWS * 16 * LD ? It::TOTAL + SO : ROWS * 16 * LD];
   __shared__ __align__(16) float su[MODE == CK_GLA ? 4 : 16 * LD];
   __shared__ __align__(16) float sm[4][16][20];
   __shared__ float red[2][16][2];
   __shared__ float half_prod[2][128];
-  float* X0 = stage;              // rows that read the state for Z
-  float* X1 = X0 + 16 * LD;       // rows that read it for the output
-  float* Y0 = X1 + 16 * LD;       // columns written with Z
-  float* Y1 = Y0 + 16 * LD;       // columns written with V
+  float* X1 = stage;              // rows that read the state for the output
+  float* Y1 = X1 + 16 * LD;       // columns written with V
+  float* X0 = Y1 + 16 * LD;       // rows that read it for Z
+  float* Y0 = X0 + 16 * LD;       // columns written with Z
 
   // which chunk of which segment
   const int item = blockIdx.x, hd = blockIdx.y;
@@ -263,8 +270,11 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
     wv[e] = get(in.dec, row, in.lddec, h0, at_c);
     av[e] = 0.f;
     if (MODE == CK_GD) av[e] = get(in.a, row, in.lda, h0, at_c);
-    if (MODE == CK_CD) av[e] = get(in.a, row, in.lda, hd, 0);
   }
+  // one number per row: each of eight lanes has one, and all take it from there
+  float ar = 0.f;
+  if (MODE == CK_CD)
+    ar = get(in.a, row0 + min(half * 8 + (lane & 7), nv - 1), in.lda, hd, 0);
   const float c0z = in.p0[h0 + dc];
   float c1 = 0.f;
   if (MODE == CK_GD) c1 = in.p1[h0 + dc];
@@ -276,10 +286,16 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
       av[e] = ck_sigmoid(av[e] + c1);
     } else if (MODE == CK_CD) {
       wv[e] = ck_exp(-c1 * ck_softplus(wv[e] + c0z));
-      av[e] = ck_sigmoid(av[e]);
     } else {
       wv[e] = ck_exp(ck_log_sigmoid(wv[e] + c0z) * c0f);
     }
+  }
+  if (MODE == CK_CD) {
+    ar = half * 8 + (lane & 7) < nv ? ck_sigmoid(ar) : 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      av[e] = __uint_as_float(
+          __builtin_amdgcn_readlane(__float_as_uint(ar), e));
   }
   // rows past the segment's end and channels past the head's change nothing
   if (DP != 128 || D != DP || nv != 16) {
@@ -287,7 +303,8 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
     for (int e = 0; e < 8; ++e) {
       const bool live = real && half * 8 + e < nv;
       wv[e] = live ? wv[e] : 1.f;
-      if (!live) kv[e] = rv[e] = av[e] = 0.f;
+      if (!live) kv[e] = rv[e] = 0.f;
+      if (MODE == CK_GD && !live) av[e] = 0.f;
     }
   }
 
@@ -477,13 +494,15 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
     __syncthreads();
   }
 
-  // fragments (over the operand rows, which nothing reads any more)
+  // Fragments over the operand rows, which nothing reads any more; those of 16
+  // bytes go to memory at once, on their way during the substitution.
+  float* dst = items + ((size_t)item * H + hd) * It::TOTAL;
   constexpr int LAST = MODE == CK_GD ? 3 : (MODE == CK_CD ? 1 : 0);
   if (on) {
     const int t = d >> 4, dg = (d & 15) >> 2, di = d & 3;
     float kf[8], bf[8];
     auto scaled = [&](int e, float from, float to) {
-      stage[It::R + ck_row_slot(t, dg, half * 8 + e) * 4 + di] = rv[e] * from;
+      stage[ck_row_slot(t, dg, half * 8 + e) * 4 + di] = rv[e] * from;
       kf[e] = kv[e] * to;
       bf[e] = bv[e] * to;
     };
@@ -497,20 +516,20 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int at = ck_col_slot(t, half * 2 + h, d & 15) * 4;
-      *(ck_f32x4*)(stage + It::K + at) =
+      *(ck_f32x4*)(dst + It::K + at) =
           ck_f32x4{kf[4 * h], kf[4 * h + 1], kf[4 * h + 2], kf[4 * h + 3]};
       if (MODE == CK_GD)
-        *(ck_f32x4*)(stage + It::B + at) =
+        *(ck_f32x4*)(dst + It::B + at) =
             ck_f32x4{bf[4 * h], bf[4 * h + 1], bf[4 * h + 2], bf[4 * h + 3]};
     }
-    if (half == 0) stage[It::GAM + d] = pin[7] * other;
-    if (threadIdx.x < 4) stage[It::FLAG + threadIdx.x] = odd ? 1.f : 0.f;
+    if (half == 0) stage[SO + It::GAM + d] = pin[7] * other;
+    if (threadIdx.x < 4) stage[SO + It::FLAG + threadIdx.x] = odd ? 1.f : 0.f;
   }
   if (wave == 3)
-    *(ck_f32x4*)(stage + It::M + lane * 4) =
+    *(ck_f32x4*)(stage + SO + It::M + lane * 4) =
         *(const ck_f32x4*)(&sm[LAST][m16][g * 4]);
   if (MODE == CK_GD && wave == 2)
-    *(ck_f32x4*)(stage + It::MB + lane * 4) =
+    *(ck_f32x4*)(stage + SO + It::MB + lane * 4) =
         *(const ck_f32x4*)(&sm[2][m16][g * 4]);
   if (MODE != CK_GLA) {
     // forward substitution, one thread per column of [U | Km] (general) or
@@ -542,19 +561,28 @@ __global__ __launch_bounds__(256, 3) void ck_prep_kernel(
         const int t = col >> 4, dg = (col & 15) >> 2, di = col & 3;
 #pragma unroll
         for (int tt = 0; tt < 16; ++tt)
-          stage[It::U + ck_row_slot(t, dg, tt) * 4 + di] = x[tt];
+          stage[SU + ck_row_slot(t, dg, tt) * 4 + di] = x[tt];
       } else {
         const int s = col - DP;
 #pragma unroll
         for (int tt = 0; tt < 16; ++tt)
-          stage[It::C + ((s >> 2) * 16 + tt) * 4 + (s & 3)] = x[tt];
+          stage[SO + It::C + ((s >> 2) * 16 + tt) * 4 + (s & 3)] = x[tt];
       }
     }
   }
   __syncthreads();
-  float* dst = items + ((size_t)item * H + hd) * It::TOTAL;
-  for (int i = threadIdx.x; i < It::TOTAL / 4; i += 256)
-    *(ck_f32x4*)(dst + i * 4) = *(const ck_f32x4*)(stage + i * 4);
+  auto copy = [&](int from, int to, int shift) {
+#pragma unroll
+    for (int i = from / 4; i < to / 4; i += 256) {
+      const int at = i + threadIdx.x;
+      if (at < to / 4)
+        *(ck_f32x4*)(dst + at * 4) =
+            *(const ck_f32x4*)(stage + shift + at * 4);
+    }
+  };
+  copy(It::R, It::R + It::ROW, 0);
+  if (MODE != CK_GLA) copy(It::U, It::U + It::ROW, SU - It::U);
+  copy(It::M, It::TOTAL, SO);
 }
 
 PS_DEV bool ck_finite(ck_f32x4 a) {
@@ -2400,11 +2428,11 @@ static long ck_chunk_floats(int mode, int dp, int H, int G, int L) {
 }
 
 // Measured (bf16, one MI355X, whole operation; token by token -> this form):
-//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.68 ms
-//     (operands 0.22, walk 0.41, read-out 0.04)
+//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.67 ms
+//     (operands 0.21, walk 0.41, read-out 0.04)
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
-//                                                            5.42 -> 0.49 ms
-//     (its operands' logarithms and wave sums 0.04 less than before)
+//                                                            5.42 -> 0.48 ms
+//     (operands 0.14, walk 0.27, tokens 0.03)
 //   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.30 ms
 //   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.06 ms
 //   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.47 ms
