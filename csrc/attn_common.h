@@ -14,12 +14,13 @@ typedef __attribute__((address_space(3))) kv_s4 kv_lds_s4;
 
 #define KV_LOG2E 1.44269504f
 #define KV_LOW (-3.0e38f)
-// Powers of two by which a tile's scores may exceed the reference of the weights
-// before it moves: what moves it, in a tile where any of a wave's rows does, is a
-// product per accumulated number (96 of 560 instructions of the prompt form of
-// window_attention.hip, in most tiles, as a sequence's 32nd tile still holds the
-// largest score so far of one of 32 rows with 60 %). A weight then is at most 16,
-// its exponent at most one unit of 2^-24 more off than one below 1.
+// Powers of two by which a tile's scores may exceed those that set the reference of
+// the weights before it moves: what moves it, in a tile where any of a wave's rows
+// does, is a product per accumulated number (96 of 560 instructions of the prompt
+// form of window_attention.hip, in most tiles, as a sequence's 32nd tile still holds
+// the largest score so far of one of 32 rows with 60 %). The reference is as much
+// above the score that set it, so that no weight is above 1 and sums of weighted
+// values have the range that they have with the maximum itself as reference.
 #define KV_FAR 4.f
 
 union KvPack {
@@ -45,23 +46,24 @@ PS_DEV void kv_split(float p0, float p1, unsigned int* a, unsigned int* b,
   *c = __builtin_amdgcn_perm(z1, z0, 0x07060302u);
 }
 
-// One online-softmax step of a lane's N scores v (relative to the reference m, the
-// largest score when it last moved, or absolute while m is KV_LOW): weights into
-// v, their sum into l, a new reference into m; returns the factor for what was
-// accumulated before. mx: the largest v over all lanes of the row. The factor is
-// 1 for every lane (and *moved false) when no reference of the wave moves. sink2: a sink in powers
-// of two that joins with the row's first maximum, of which this lane has
-// `share` (the alternative to kv_sink where what lives past the walk costs).
+// One online-softmax step of a lane's N scores v (relative to the reference m, which
+// was KV_FAR above the largest score when it last moved, or absolute while m is
+// KV_LOW): weights into v, their sum into l, a new reference into m; returns the
+// factor for what was accumulated before. mx: the largest v over all lanes of the
+// row. The factor is 1 for every lane (and *moved false) when no reference of the
+// wave moves. sink2: a sink in powers of two that joins with the row's first
+// maximum, of which this lane has `share` (the alternative to kv_sink where what
+// lives past the walk costs).
 template <int N>
 PS_DEV float kv_softmax(float* v, float mx, float* m, float* l, bool* moved,
                         float sink2 = -INFINITY, float share = 0.f) {
   const bool fresh = *m == KV_LOW;
-  *moved = __any(mx > KV_FAR || (fresh && mx > -INFINITY));
+  *moved = __any(mx > 0.f || (fresh && mx > -INFINITY));
   float alpha = 1.f;
   if (*moved) {
     const float top = share != 0.f ? fmaxf(mx, sink2) : mx;
     const float d =
-        fresh ? (mx > -INFINITY ? top : 0.f) : fmaxf(mx, 0.f);
+        fresh ? (mx > -INFINITY ? top + KV_FAR : 0.f) : fmaxf(mx + KV_FAR, 0.f);
     if (!fresh) {
       alpha = __builtin_amdgcn_exp2f(-d);
       *m += d;
@@ -82,7 +84,7 @@ PS_DEV float kv_softmax(float* v, float mx, float* m, float* l, bool* moved,
   return alpha;
 }
 
-// A sink (natural log units) joins a finished row of maximum m and denominator
+// A sink (natural log units) joins a finished row of reference m and denominator
 // l; returns the factor for the row's sums. It comes last: scores relative to
 // a sink far below them would lose their digits, and to one of minus infinity
 // be no numbers.

@@ -19,9 +19,9 @@
 //            v_mfma_f32_16x16x4_f32 (no term of either is rounded);
 //   softmax  a lane then holds one row's scores of 4 heads over 2 keys, whose
 //            weights are relative to a reference that all waves share, not to the
-//            half's own maximum: it moves, by an exchange behind the barrier, only
-//            where a score is more than TM_FAR above it. The denominator stays a
-//            partial sum per key share to the end;
+//            half's own maximum: it lies TM_FAR above the score that set it and
+//            moves, by an exchange behind the barrier, only where a score is above
+//            it. The denominator stays a partial sum per key share to the end;
 //   output   of the tile before, in every other half: the weights go through LDS
 //            to the wave of their head (wave w: two of the 16), there cut into
 //            three bf16 terms (exact products, fp32 accumulation), values through
@@ -54,8 +54,8 @@ union TmPack {
 
 #define TM_H 32
 #define TM_KT 32
-// how far scores, in powers of two, may be above the reference that weights are
-// relative to
+// How far scores, in powers of two, may be above those that set the reference that
+// weights are relative to. The reference is as much above them: no weight is above 1.
 #define TM_FAR 8.f
 
 struct TmArgs {
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   __shared__ int s_seq[16], s_pos[16];
   // first and last tile of a run whose values (of two waves) are not all finite
   __shared__ int s_odd[4][2];
-  __shared__ int s_high[3];  // a half's scores are too far above the reference
+  __shared__ int s_high[3];  // a half has scores above the reference
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, n = lane & 15;
@@ -213,9 +213,9 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   for (int i = 0; i < 4; ++i) {
     m[i] = a.sink ? (a.sink_vals != nullptr
                          ? fmaxf(a.sink_vals[h0 + i] * KV_LOG2E, PS_NEG_INF)
-                         : 0.f)
+                         : 0.f) + TM_FAR
                   : PS_NEG_INF;
-    l[i] = a.sink && wave == 0 ? 1.f : 0.f;
+    l[i] = a.sink && wave == 0 ? __builtin_amdgcn_exp2f(-TM_FAR) : 0.f;
   }
   ck_f32x4 acc[2][NV];
 #pragma unroll
@@ -324,8 +324,8 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
         *(float2*)(to + tm_at(4 * g + i, n, wave, g)) = make_float2(p0, p1);
       }
     };
-    // A half whose scores are more than TM_FAR above the reference, behind the
-    // barrier that ends its turn: the reference moves to the largest, and with it
+    // A half with scores above the reference, behind the barrier that ends its
+    // turn: the reference moves to TM_FAR above the largest, and with it
     // what was made by the one before: the half's weights, those of the other
     // half of an unfinished tile, sums and outputs.
     auto raise = [&](int t, int half, int third, float(&sum)[4]) {
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
       for (int i = 0; i < 4; ++i) {
         float mn = m[i];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) mn = fmaxf(mn, pm[k * 256 + i * 16]);
+        for (int k = 0; k < 8; ++k) mn = fmaxf(mn, pm[k * 256 + i * 16] + TM_FAR);
         const float al =
             __builtin_amdgcn_exp2f(m[i] - (mn > PS_NEG_INF ? mn : 0.f));
         m[i] = mn;
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
         bool high = false;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          high |= fmaxf(x[0][i], x[1][i]) > m[i] + TM_FAR;
+          high |= fmaxf(x[0][i], x[1][i]) > m[i];
         if (__any(high) && lane == 0) s_high[third] = 1;
         weigh(x, sP + third * SP, sum);
       };

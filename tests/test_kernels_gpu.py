@@ -117,6 +117,31 @@ def test_paged_attn_decode(qh, kh, hd):
     _close(got, want)
 
 
+@pytest.mark.parametrize("S,qh,hd", [(33, 32, 128), (33, 16, 64), (1, 32, 128)])
+@pytest.mark.parametrize("grow", [0.9, 5.0])
+def test_paged_attn_decode_largest_values(S, qh, hd, grow):
+    """A key whose score lies above the earlier ones by less than the weights'
+    reference waits for (four powers of two), or by more, and whose value is near
+    the end of bf16's range: weights stay at most 1, so the sums do not
+    overflow, with one range of keys a sequence and several."""
+    kh, bs, L = 8, 16, 400
+    kc = torch.zeros(L // bs, kh, bs, hd, dtype=torch.bfloat16)
+    vc = torch.ones(L // bs, kh, bs, hd, dtype=torch.bfloat16)
+    at = 389                                # no wave's first tile
+    kc[at // bs, :, at % bs, 0] = grow * 4 * 0.6931
+    vc[at // bs, :, at % bs, 5] = 1e38
+    tables = torch.arange(L // bs, dtype=torch.int32).repeat(S, 1)
+    lens = (L - torch.arange(S) % 8).int()
+    q = torch.zeros(S, qh, hd, dtype=torch.bfloat16)
+    q[:, :, 0] = 8.0
+    want = reference.paged_attn_decode(q.float(), kc.float(), vc.float(), tables,
+                                       lens, 0.125)
+    got = ops.paged_attn_decode(q.cuda(), kc.cuda(), vc.cuda(), tables.cuda(),
+                                lens.cuda(), 0.125).cpu()
+    # the bf16 rounding of the result, entry by entry
+    assert float(((got.double() - want).abs() / want).max()) < 5e-3
+
+
 @pytest.mark.parametrize("S,qh,kh,hd,window,fp8", [
     (66, 32, 32, 128, 0, False),    # a wave per head up to two tiles
     (66, 32, 32, 128, 0, True),     # (four of fp8)

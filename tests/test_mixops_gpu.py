@@ -588,6 +588,36 @@ def test_window_attention_scores_climb(grow, softcap):
         assert _rel(got.float().cpu().reshape(T, H, D), want) < 3e-3, kw
 
 
+@pytest.mark.parametrize("variant,splits,far", [
+    (10, 0, 8), (11, 0, 4), (12, 1, 4), (12, 3, 4)])
+@pytest.mark.parametrize("sink", [True, False])
+def test_attention_largest_values(variant, splits, far, sink):
+    """Values near the end of bf16's range at a key whose score lies nearly as
+    far above the earlier ones as the weights' reference waits for (far powers of
+    two): weights stay at most 1, so the sums do not overflow."""
+    H, G, D, bs, L = 32, 8, 64, 16, 400
+    kc = torch.zeros(L // bs, G, bs, D, dtype=torch.bfloat16)
+    vc = torch.ones(L // bs, G, bs, D, dtype=torch.bfloat16)
+    at = 389                                # no wave's first tile
+    kc[at // bs, :, at % bs, 0] = 0.9 * far * math.log(2.0)
+    vc[at // bs, :, at % bs, 5] = 1e38
+    tables = torch.arange(L // bs, dtype=torch.int32).view(1, -1)
+    tp = torch.arange(L - 8, L, dtype=torch.int32)
+    ts = torch.zeros(8, dtype=torch.int32)
+    q = torch.zeros(8, H, D, dtype=torch.bfloat16)
+    q[:, :, 0] = 8.0
+    talk = torch.eye(H) if variant == 10 else None
+    want = reference.talk_attention(q.float(), kc.float(), vc.float(), tables,
+                                    ts, tp, D ** -0.5, 0, 0, sink, talk)
+    got = ops.talk_attention(
+        q.view(8, H * D).cuda(), kc.cuda(), vc.cuda(), tables.cuda(), ts.cuda(),
+        tp.cuda(), D ** -0.5, H, sink=sink, variant=variant, splits=splits,
+        talk=talk.cuda() if talk is not None else None)
+    # the bf16 rounding of the result, entry by entry
+    err = (got.cpu().double().view(8, H, D) - want).abs() / want
+    assert float(err.max()) < 5e-3
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,D", [(1, 32), (3, 32), (3, 64), (2, 128), (5, 96)])
 def test_recurrence_readout_borders(H, D, dtype):

@@ -532,6 +532,41 @@ def test_keyval_token_kernel(shape, splits):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("variant,splits", [(8, 0), (9, 1), (9, 3)])
+@pytest.mark.parametrize("at", [5, 389])
+@pytest.mark.parametrize("grow", [0.9, 5.0])
+@pytest.mark.parametrize("sink", [True, False])
+def test_keyval_score_steps(variant, splits, at, grow, sink):
+    """A key whose score lies above the others by less than the weights'
+    reference waits for, or by more, and whose value is near the end of bf16's
+    range, in the first tile of a walk or the last: weights stay at most 1, so
+    the sums do not overflow."""
+    H, G, D, bs, L = 8, 2, 64, 16, 400
+    c = torch.zeros(L // bs, G, bs, D, dtype=torch.bfloat16)
+    c[..., 5] = 1.0
+    c[at // bs, :, at % bs, 0] = grow * 4 * math.log(2.0)
+    c[at // bs, :, at % bs, 5] = 1e38
+    tables = torch.arange(L // bs, dtype=torch.int32).view(1, -1)
+    pos = torch.arange(L - 8, L, dtype=torch.int32)
+    seq = torch.zeros(8, dtype=torch.int32)
+    f = torch.ones(L // bs, G, bs)
+    q = torch.zeros(8, H, D, dtype=torch.bfloat16)
+    q[:, :, 0] = 8.0
+    want = R.talk_attention(q.float(), c.float(), c.float(), tables, seq, pos,
+                            D ** -0.5, 0, 0, sink, None, 0, 0.0, None, D, None,
+                            f)[..., 5]
+    cc = c.cuda()
+    got = ops.talk_attention(
+        q.view(8, H * D).cuda(), cc, cc, tables.cuda(), seq.cuda(), pos.cuda(),
+        D ** -0.5, H, sink=sink, variant=variant, splits=splits, vdim=D,
+        key_scale=f.cuda()).cpu().view(8, H, D)
+    assert torch.isfinite(got).all()
+    # the bf16 rounding of the result, entry by entry
+    err = (got[..., 5].double() - want).abs() / want
+    assert float(err.max()) < 5e-3
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape", KERNEL_SHAPES + [
     (130, 1, 16, 40, "learned", 16, True, True)])
 def test_keyval_prompt_kernel(shape):
