@@ -5,7 +5,9 @@ The library's decode-shaped tiles leave the read of the weights at a third to
 a half of memory's rate for several projections, csrc/skinny_gemm.hip does for
 others: the engine autotunes each (decode bucket M, projection
 shape) pair once at startup on the actual device and the winner is what the
-hipGraph capture records.
+hipGraph capture records. That times bare products. Where a launch before or
+behind one can be joined with it, the rules below, which were measured with those
+launches, decide first.
 """
 
 from __future__ import annotations
@@ -13,15 +15,16 @@ from __future__ import annotations
 import logging
 import math
 import time
-from typing import Dict, Tuple
+from typing import Dict
 
 import torch
 import torch.nn.functional as F
 
 logger = logging.getLogger("ops.gemm_policy")
 
-# (M, N, K) -> winning impl: 0 = hipBLASLt, 1 = skinny split-K, 2 = 8-phase
-_POLICY: Dict[Tuple[int, int, int], int] = {}
+# (M, N, K) -> winning impl: 0 = hipBLASLt, 1 = skinny split-K, 2 = 8-phase;
+# (M, N, K, behind) -> that of a product joined with other launches
+_POLICY: Dict[tuple, int] = {}
 
 
 MAX_ROWS = 256  # of the skinny kernels
@@ -66,14 +69,19 @@ def tune(weights, buckets, device) -> None:
                 cands.append((2, _time_fn(lambda: ops.gemm8p(x, w))))
             impl, t = min(cands, key=lambda c: c[1])
             _POLICY[(M, N, K)] = impl
+            for behind, rules in _UNTUNED.items():
+                if behind:
+                    _POLICY[(M, N, K, behind)] = (
+                        1 if any(rule(M, N, K) for rule in rules) else impl)
             if impl:
                 logger.info(
                     "gemm M=%d N=%d K=%d: impl %s wins at %.1fus",
                     M, N, K, ("blas", "skinny", "8p")[impl], t * 1e6,
                 )
+    cells = [v for key, v in _POLICY.items() if len(key) == 3]
     logger.info(
         "gemm autotune done: %d/%d cells use an in-house kernel",
-        sum(1 for v in _POLICY.values() if v), len(_POLICY),
+        sum(1 for v in cells if v), len(cells),
     )
 
 
@@ -168,6 +176,7 @@ def _rows_before_gate(rows: int, N: int, K: int) -> bool:
 
 
 _UNTUNED = {"": (_few_rows, _long_rows),
+            "around": (_few_rows,),
             "norm": (_rows_before_norm,),
             "rope": (_rows_before_rope,),
             "gate": (_few_rows, _long_rows, _rows_before_gate)}
@@ -175,11 +184,14 @@ _UNTUNED = {"": (_few_rows, _long_rows),
 
 def _choose(x: torch.Tensor, w: torch.Tensor, behind: str = "") -> int:
     """0: the library, 1: skinny, 2: 8-phase. behind: what the product's last step
-    shares a launch with."""
+    shares a launch with ("around": its first one too). A choice that was made for
+    the bare product alone holds for that as well."""
     if not x.is_cuda or x.dtype != torch.bfloat16:
         return 0
     shape = (x.shape[0], w.shape[0], w.shape[1])
-    impl = _POLICY.get(shape)
+    impl = _POLICY.get(shape + (behind,) if behind else shape)
+    if impl is None:
+        impl = _POLICY.get(shape)
     if impl is None:  # untuned
         impl = int(any(rule(*shape) for rule in _UNTUNED[behind])
                    and _fits(x, w))
@@ -217,7 +229,7 @@ def fused(x: torch.Tensor, w: torch.Tensor) -> int:
     if x.shape[0] > 16:
         return 0
     entries = x.shape[0] * x.shape[-1]
-    if (entries > _LDS_X or _choose(x, w) != 1
+    if (entries > _LDS_X or _choose(x, w, "around") != 1
             or not _fits(x, w) or (w.shape[0] + 32) * w.shape[1] >= 1 << 31):
         return 0
     return 2 if entries <= _LDS_NORM_X and x.is_contiguous() else 1
@@ -231,10 +243,10 @@ def silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     from production_stack_amd import ops
 
     rows = 8 if w.shape[0] > 32768 else 16
-    if _choose(x, w, "gate") == 1:
+    if _choose(x, w, "gate") == 1 and _fits(x, w):
         if x.shape[0] <= rows:
             return ops.skinny_gated(x, w)
-        if 16 < x.shape[0] <= 192 and _fits(x, w):
+        if 16 < x.shape[0] <= 192:
             act = ops.skinny_gated_tiles(x, w)
             if act is not None:
                 return act

@@ -1336,6 +1336,61 @@ def test_gate_dispatch(M, N, K, own):
     assert torch.equal(gemm_policy.silu_mul(x, w), want)
 
 
+@pytest.mark.parametrize("M,N,K,behind,own", [
+    (1, 3072, 2048, "around", True), (16, 3072, 2048, "around", True),
+    (4, 16384, 2048, "gate", True), (17, 28160, 2048, "gate", True),
+    (65, 28672, 2048, "gate", False), (64, 4096, 4096, "norm", True),
+    (64, 4160, 4096, "norm", False), (128, 4608, 3584, "rope", True),
+    (127, 4608, 3584, "rope", False)])
+@pytest.mark.parametrize("bare", [0, 1, 2])
+def test_tuned_bare_products(M, N, K, behind, own, bare, monkeypatch):
+    """The choice that start-up timing of bare products leaves: where the product
+    joins its neighbours' launches by the rules measured with them, it does
+    whatever won alone; elsewhere it follows the bare product."""
+    from production_stack_amd.ops import gemm_policy
+
+    w = (torch.empty(N, K, device="cuda").normal_() * K ** -0.5).to(
+        torch.bfloat16)
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    order = [1.0, 1.0, 1.0]
+    order[bare] = 0.5
+    times = iter(order)
+    monkeypatch.setattr(gemm_policy, "_time_fn", lambda fn: next(times))
+    gemm_policy.reset()
+    try:
+        gemm_policy.tune([w], [M], torch.device("cuda"))
+        wide = N % 256 == 0 and K % 128 == 0
+        bare = bare if bare < 2 or wide else 0
+        assert gemm_policy._choose(x, w) == bare
+        joins = own or bare == 1
+        if behind == "around":
+            assert gemm_policy.fused(x, w) == (
+                0 if not joins else 2 if M * K <= 16384 else 1)
+        elif behind == "gate":
+            got = gemm_policy.silu_mul(x, w)
+            kernel = None
+            if joins:
+                kernel = (ops.skinny_gated if M <= 16
+                          else ops.skinny_gated_tiles)(x, w)
+            if kernel is None:
+                kernel = ops.silu_and_mul(gemm_policy.linear(x, w))
+            assert torch.equal(got, kernel)
+        else:
+            got = gemm_policy.parts(x, w, behind)
+            assert (got is not None) == joins
+        # operands that the kernels do not take as they are: no joined launch
+        odd = torch.empty(M * K + 8, device="cuda", dtype=torch.bfloat16)
+        odd = odd[1:M * K + 1].view(M, K)
+        assert gemm_policy.fused(odd, w) == 0
+        assert gemm_policy.parts(odd, w, behind) is None
+        if bare == 0:
+            odd.copy_(x)
+            assert torch.equal(gemm_policy.silu_mul(odd, w), ops.silu_and_mul(
+                torch.nn.functional.linear(odd, w)))
+    finally:
+        gemm_policy.reset()
+
+
 def test_skinny_gemm_nothing_to_do():
     """No columns of K are refused for any number of rows, no rows give no
     rows, also where they are a view of a wider matrix."""
