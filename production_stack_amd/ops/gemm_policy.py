@@ -106,21 +106,34 @@ _LDS_X, _LDS_NORM_X = 65536, 16384
 def _few_rows(rows: int, N: int, K: int) -> bool:
     """Up to 16 rows, x of up to 65536 entries. Rows of W of up to 4096 entries
     (us, in-house / library: 1 x 2048 x 2048 4.5 / 11.0, 1 x 28672 x 4096 41 / 63,
-    16 x 28672 x 4096 45 / 64, 16 x 4096 x 4096 10.6 / 15.4, 16 x 6144 x 4096 14.4 /
-    15.5, 16 x 6144 x 2560 10.1 / 10.5, 16 x 128256 x 4096 189 / 191; the narrowest;
-    past the line 1 x 50304 x 768 18.1 / 15.8, 16 x 50304 x 768 19.1 / 16.0), and longer ones of up to 2048 rows of W (8 x 2048 x 8192 10.5 / 12.6, 8 x 512 x
-    8192 10.0 / 11.4; 16 x 2048 x 8192 16.8 / 12.9) or, up to 4 rows, of as many as
-    give all CUs nearly as much to do (4 x 4096 x 14336 25.8 / 27.0, 4 x 28672 x 8192
-    82 / 122, 1 x 4096 x 8192 15.2 / 16.2; past the line 4 x 6144 x 8192 24 / 22, 4 x
-    5120 x 8192 23 / 20)."""
+    16 x 28672 x 4096 45 / 64, 16 x 4096 x 4096 10.6 / 15.4, 16 x 6144 x 2560 10.1 /
+    10.5, 16 x 128256 x 4096 189 / 191; the narrowest), without short rows of a wide
+    W (1 x 50304 x 768 18.1 / 15.8, 16 x 28672 x 256 9.6 / 8.3, 16 x 18432 x 192 7.0 /
+    6.0), from 4 rows on also
+    of other lengths than whole 1024 (16 x 128256 x 1536 82.7 / 74.3, 16 x 50304 x
+    3584 69.6 / 65.2). Longer ones of up to 2048 rows of W (8 x 2048 x 8192 10.5 /
+    12.6; 16 x 2048 x 8192 16.8 / 12.9, 8 x 256 x 8192 9.7 / 8.4) or, up to 4 rows, of
+    as many as give all CUs nearly as much to do (4 x 4096 x 14336 25.8 / 27.0, 4 x
+    28672 x 8192 82 / 122, 1 x 4096 x 8192 15.2 / 16.2; past the line 4 x 6144 x 8192
+    24 / 22, 4 x 5120 x 8192 23 / 20)."""
     if rows > 16 or rows * K > _LDS_X:
         return False
     if K <= 4096:
-        return K > 1024 or N < 32768
+        if N >= 32768:
+            return K > 1024 and (rows <= 3 or K % 1024 == 0)
+        return K >= 512 or N < (24576 if K >= 256 else 14336)
     if N <= 2048:
-        return rows <= 8 and K % 128 == 0
+        return rows <= (8 if N >= 1024 else 5) and K % 128 == 0
     turns = N / 4096
     return rows <= 4 and turns >= 0.8 * math.ceil(turns)
+
+
+def _few_rows_alone(rows: int, N: int, K: int) -> bool:
+    """As above where nothing else shares the launch: at 13 to 16 rows, tiles that
+    are more than the CUs and not many times as many (16 x 5120 x 4096 14.3 / 13.9, x
+    3584 13.1 / 12.6, 16 x 8192 x 3584 14.4 / 14.0) are the library's."""
+    return (_few_rows(rows, N, K)
+            and not (rows > 12 and 4096 < N <= 8192 and K > 3072))
 
 
 def _long_rows(rows: int, N: int, K: int) -> bool:
@@ -141,28 +154,61 @@ def _long_rows(rows: int, N: int, K: int) -> bool:
 
 def _rows_before_norm(rows: int, N: int, K: int) -> bool:
     """17 to 192 rows whose partial sums the norm behind them adds. us with that
-    norm, in-house / library: 17 x 2048 x 2048 10.1 / 13.8, 64 x 2048 x 8192 18.4 /
-    25.2, 64 x 4096 x 4096 17.0 / 18.4, 192 x 4096 x 4096 24.9 / 36.3, 64 x 4096 x
-    14336 32.7 / 42.5, 96 x 3584 x 4096 20.1 / 25.3, 128 x 6144 x 4096 27.2 / 29.6,
-    192 x 8192 x 14336 78 / 117. Past the lines 64 x 6144 x 4096 22.7 / 22.0, 17 x
-    2048 x 8192 16.8 / 16.5, 96 x 2560 x 4096 19.4 / 16.3, 160 x 3072 x 4096 22.5 /
-    20.2, 128 x 4096 x 2048 18.8 / 18.7, 256 x 4096 x 8192 45.6 / 40.1. The slowest
-    found within: 48 x 2560 x 2560 13.7 / 12.7."""
+    norm, in-house / library; the library's time jumps up at whole 32 rows, and
+    between its tuned sizes in N and K it is some other kernel's.
+    Long rows: 64 x 4096 x 14336 33.3 / 43.7, 17 x 8192 x 10240 41.7 / 42.1, but 20 x
+    8192 x 13824 51.3 / 47.0, 17 x 4096 x 12288 28.1 / 26.8, 104 x 1024 x 10240 21.6 /
+    19.2.
+    More than 64 rows: 96 x 4096 x 4096 21.4 / 25.3, 192 24.8 / 36.3, but 80 21.0 / 19.9,
+    112 22.0 / 20.0; 144 24.0 / 25.5; 80 x 5120 x 4096 25.2 / 21.4, 112 26.1 / 27.7, 149 x
+    5376 x 4096 28.4 / 27.1; 80 x 6144 x 4096 25.9 / 27.5, 144 30.8 / 43.8, 176 1.02 times.
+    Fewer: few rows of W (17 x 2048 x 2048 10.1 / 13.7, 63 x 2048 x 4096 14.2 / 15.0, 48
+    x 2560 x 2048 13.5 / 14.8; 25 x 2048 x 1024 9.0 / 8.4, 60 x 1024 x 1280 up to 1.2
+    times, 48 x 2560 x 2560 14.5 / 12.7), of more 64 x 4096 x 4096 17.6 / 18.6 and 32 x
+    4096 x 4096 16.0 / 16.3, but 63 x 4096 x 4096 17.7 / 17.2, 32 x 4096 x 3072 14.7 /
+    14.1, 64 x 3584 x 3328 18.2 / 16.7. Of 1950 drawn sizes within the slowest, 63 x
+    1536 x 3072, takes 13.5 / 12.8."""
     if not 17 <= rows <= 192 or not 1024 <= N <= 8192 or K < 1024:
         return False
+    whole = rows % 32 == 0
     if K >= 10240:
-        return True
+        return ((N >= 1536 or K >= 14336) and
+                (rows >= 32 or (K % 2048 == 0 and
+                                (K >= 14336 or not 3072 < N < 4608))))
     if rows > 64:
-        return 3584 <= N <= 6144 and K >= 4096
-    return N <= 4096 and (K <= 5120 or (rows >= 48 and N >= 1536))
+        if not 3584 <= N <= 6144 or K < 4096:
+            return False
+        if whole or K >= 8192:
+            return True
+        if N <= 4096:
+            return rows > 128 or K >= 6144
+        if N < 5632:
+            return 96 < rows < 128
+        return rows <= 160 or K >= 5120
+    if N > 4096:
+        return False
+    if K < 3072:
+        return K == 2048 or (K == 1024 and not 1536 < N < 2560)
+    if K > 5120:
+        return rows >= 48 and (N >= 3072 or (whole and N >= 1536))
+    return (N <= 2048 or (rows == 64 and K % 512 == 0)
+            or (rows <= 32 and K >= 4096))
 
 
 def _rows_before_rope(rows: int, N: int, K: int) -> bool:
     """As above with the rotary embedding and the cache's rows behind: 128 x 6144 x
-    4096 27.0 / 28.6, 192 32.0 / 37.0, 128 x 7168 x 5120 35.3 / 36.7, 128 x 4608 x 3584
-    24.6 / 26.1; past the lines 96 x 4608 x 3584 23.6 / 23.4, 192 x 6144 x 2048 26.2 /
-    25.8, 160 x 3072 x 2048 21.6 / 15.9."""
-    return 128 <= rows <= 192 and 4608 <= N <= 10240 and K >= 3584
+    4096 27.1 / 28.5, 192 32.0 / 36.8, 144 29.9 / 42.4 (176 31.3 / 29.2), 128 x 7168 x
+    5120 35.6 / 36.6, 192 x 10240 x 3584 37.9 / 42.0, 144 x 8192 x 8192 47.4 / 50.4;
+    past the lines 96 x 4608 x 3584 23.6 / 23.4, 144 x 4608 x 4096 27.3 / 25.5, 135 x
+    5376 x 4096 28.7 / 26.4, 128 x 8192 x 4096 32.5 / 30.0, 144 34.9 / 29.2, 128 x 10240
+    x 3584 32.1 / 31.5."""
+    if not 128 <= rows <= 192 or not 4608 <= N <= 10240 or K < 3584:
+        return False
+    if rows % 32 == 0:
+        return N <= 6144 or K >= 5120 or (N >= 9216 and rows * K >= 1 << 19)
+    if N < 5632:
+        return False
+    return K >= 8192 or (N <= 6144 and (rows <= 160 or K >= 5120))
 
 
 def _rows_before_gate(rows: int, N: int, K: int) -> bool:
@@ -171,11 +217,12 @@ def _rows_before_gate(rows: int, N: int, K: int) -> bool:
     slow): 17 x 28672 x 4096 49.5 / 56.4, 64 51.7 / 55.4, 64 x 28672 x 2048 30.7 / 33.1,
     64 x 32768 x 8192 105 / 123; past the lines 96 x 28672 x 4096 59.5 / 56.3, 64 x
     24576 x 4096 50.8 / 49.0, 17 x 28672 x 2560 36.6 / 31.7, 64 x 57344 x 4096 106 /
-    102."""
-    return 17 <= rows <= 64 and 28160 <= N <= 32768 and K % 2048 == 0
+    102; no wide tiles where N is no multiple of 128: 63 x 28224 x 4096 61.4 / 55.3."""
+    return (17 <= rows <= 64 and 28160 <= N <= 32768 and N % 128 == 0
+            and K % 2048 == 0)
 
 
-_UNTUNED = {"": (_few_rows, _long_rows),
+_UNTUNED = {"": (_few_rows_alone, _long_rows),
             "around": (_few_rows,),
             "norm": (_rows_before_norm,),
             "rope": (_rows_before_rope,),

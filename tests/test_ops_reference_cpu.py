@@ -4,6 +4,7 @@ The paged references are checked against dense (non-paged) attention so the
 GPU kernel tests compare against a trustworthy baseline.
 """
 
+import pytest
 import torch
 
 from production_stack_amd.ops import reference
@@ -87,3 +88,68 @@ def test_rope_preserves_tail_dims():
         atol=1e-2,
         rtol=1e-2,
     )
+
+
+@pytest.mark.parametrize("rule,shape,own", [
+    # rows, rows of W, entries of each: on either side of each line
+    ("few_rows", (1, 28672, 512), True), ("few_rows", (1, 28672, 256), False),
+    ("few_rows", (1, 16384, 256), True), ("few_rows", (1, 16384, 192), False), ("few_rows", (3, 50304, 1536), True),
+    ("few_rows", (4, 50304, 1536), False), ("few_rows", (16, 50304, 2048), True),
+    ("few_rows", (8, 1024, 8192), True), ("few_rows", (8, 512, 8192), False),
+    ("few_rows", (5, 512, 8192), True), ("few_rows", (16, 6144, 4096), True),
+    ("few_rows_alone", (16, 6144, 4096), False),
+    ("few_rows_alone", (12, 6144, 4096), True),
+    ("few_rows_alone", (16, 4096, 4096), True),
+    ("few_rows_alone", (16, 8256, 4096), True),
+    ("few_rows_alone", (16, 6144, 3072), True),
+    ("few_rows_alone", (17, 4096, 2048), False),
+    ("rows_before_norm", (60, 2048, 1280), False),
+    ("rows_before_norm", (60, 2048, 2048), True),
+    ("rows_before_norm", (63, 2048, 3584), True),
+    ("rows_before_norm", (63, 4096, 4096), False),
+    ("rows_before_norm", (64, 4096, 4096), True),
+    ("rows_before_norm", (32, 4096, 4096), True),
+    ("rows_before_norm", (32, 4096, 3584), False),
+    ("rows_before_norm", (63, 2560, 8192), False),
+    ("rows_before_norm", (64, 2560, 8192), True),
+    ("rows_before_norm", (96, 4096, 4096), True),
+    ("rows_before_norm", (112, 4096, 4096), False),
+    ("rows_before_norm", (129, 4096, 4096), True),
+    ("rows_before_norm", (112, 4096, 6144), True),
+    ("rows_before_norm", (80, 5120, 6144), False),
+    ("rows_before_norm", (112, 5120, 4096), True),
+    ("rows_before_norm", (144, 5120, 6144), False),
+    ("rows_before_norm", (144, 6144, 4096), True),
+    ("rows_before_norm", (176, 6144, 4096), False),
+    ("rows_before_norm", (176, 6144, 5120), True),
+    ("rows_before_norm", (176, 5120, 8192), True),
+    ("rows_before_norm", (24, 4096, 12288), False),
+    ("rows_before_norm", (24, 4096, 14336), True),
+    ("rows_before_norm", (24, 8192, 13824), False),
+    ("rows_before_norm", (32, 8192, 13824), True),
+    ("rows_before_norm", (104, 1024, 10240), False),
+    ("rows_before_norm", (104, 1024, 14336), True),
+    ("rows_before_norm", (80, 5376, 5120), False),
+    ("rows_before_norm", (80, 5632, 5120), True),
+    ("rows_before_norm", (24, 2048, 1024), False),
+    ("rows_before_norm", (24, 2560, 1024), True),
+    ("rows_before_norm", (64, 3584, 3328), False),
+    ("rows_before_norm", (64, 3584, 3584), True),
+    ("rows_before_norm", (32, 4096, 12288), True),
+    ("rows_before_rope", (144, 6144, 4096), True),
+    ("rows_before_rope", (176, 6144, 4096), False),
+    ("rows_before_rope", (176, 6144, 5120), True),
+    ("rows_before_rope", (144, 5120, 4096), False),
+    ("rows_before_rope", (160, 8192, 4096), False),
+    ("rows_before_rope", (160, 8192, 5120), True),
+    ("rows_before_rope", (144, 8192, 8192), True),
+    ("rows_before_rope", (144, 5376, 8192), False),
+    ("rows_before_gate", (48, 28288, 2048), True),
+    ("rows_before_gate", (48, 28224, 2048), False),
+    ("rows_before_rope", (128, 9216, 3584), False),
+    ("rows_before_rope", (160, 9216, 3584), True)])
+def test_gemm_policy_lines(rule, shape, own):
+    """Which untuned products are in-house, by the lines that were measured."""
+    from production_stack_amd.ops import gemm_policy
+
+    assert getattr(gemm_policy, "_" + rule)(*shape) == own
