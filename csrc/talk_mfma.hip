@@ -211,8 +211,11 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   float m[4], l[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
+    // the product may be past the largest float
     m[i] = a.sink ? (a.sink_vals != nullptr
-                         ? fmaxf(a.sink_vals[h0 + i] * KV_LOG2E, PS_NEG_INF)
+                         ? fminf(fmaxf(a.sink_vals[h0 + i] * KV_LOG2E,
+                                       PS_NEG_INF),
+                                 -KV_LOW)
                          : 0.f) + TM_FAR
                   : PS_NEG_INF;
     l[i] = a.sink && wave == 0 ? __builtin_amdgcn_exp2f(-TM_FAR) : 0.f;

@@ -839,6 +839,37 @@ def test_window_attention_far_sinks(low, softcap):
             assert _rel(out[:, 1::2], want[:, 1::2]) < 3e-3
 
 
+@pytest.mark.parametrize("low", [-math.inf, -3.4e38, -1e9, -1e4, 1e9, 2.3e38,
+                                 3.4e38])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_talk_attention_far_sinks(low, softcap):
+    """Sinks far from every mixed score, beside ordinary ones: a low one takes
+    nothing, a high one everything, up to the largest number."""
+    g = torch.Generator().manual_seed(16)
+    H, G, D, bs, L = 32, 8, 64, 16, 100
+    kc, vc, tables = _paged(L, G, D, D, bs, torch.bfloat16, g, 2)
+    ts = torch.tensor([0] * 30 + [1] * 3, dtype=torch.int32)
+    tp = torch.tensor(list(range(60, 90)) + [0, 1, 95], dtype=torch.int32)
+    T = len(ts)
+    q = torch.randn(T, H * D, generator=g).to(torch.bfloat16)
+    talk = torch.eye(H) + 0.1 * torch.randn(H, H, generator=g)
+    sinks = torch.randn(H, generator=g)
+    sinks[1::2] = low
+    want = reference.talk_attention(
+        q.float().reshape(T, H, D), kc.float(), vc.float(), tables, ts, tp,
+        D ** -0.5, 0, 0, True, talk, 0, softcap, sinks)
+    out = ops.talk_attention(
+        q.cuda(), kc.cuda(), vc.cuda(), tables.cuda(), ts.cuda(), tp.cuda(),
+        D ** -0.5, H, sink=True, softcap=softcap, talk=talk.cuda(), variant=10,
+        sink_vals=sinks.cuda()).float().cpu().reshape(T, H, D)
+    # fp32 up to the bf16 rounding of the result, head by head
+    assert _rel(out[:, ::2], want[:, ::2]) < 3e-3
+    if low > 0:
+        assert (out[:, 1::2] == 0).all()
+    else:
+        assert _rel(out[:, 1::2], want[:, 1::2]) < 3e-3
+
+
 @pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
 @pytest.mark.parametrize("G,D,DV", [(8, 128, 128), (2, 64, 64)])
 def test_talk_attention_value_no_number(G, D, DV, bad):
