@@ -622,12 +622,17 @@ int mx_window_attention(void* out, int ldout, const void* q, int ldq,
     a.hpb = 16;
     a.hblocks = (rep + 15) / 16;
     const long groups = (long)T_ * G * a.hblocks;
-    // By keys (kv_order) under the same rule as the paged decode kernel's. 32/8
-    // heads of 128, us, as they come -> so: 61 tokens of 300 to 4000 keys 127 -> 108,
-    // 100 of 50 to 8000 365 -> 327, 313 of 1000 to 4000 587 -> 562, 64 of 4000 184.
+    // By keys (kv_order) where CUs have more than one workgroup and enough keys may
+    // be visible, with two or less a CU in a longer window than with more. 32/8
+    // heads of 128, us, as they come -> so: 61 tokens of 300 to 4000 keys 114 -> 91,
+    // window 2048 77.6 -> 76.3, 1500 54.6 -> 56.4 (50 tokens 47.6 -> 50.1, 1800 57.0 ->
+    // 57.7; 40 tokens 44.8 -> 41.1, 64 of 100 to 2500 45.4 -> 43.1); 70 tokens, window
+    // 1100 59.4 -> 53.6, 1024 53.3; 100 of 50 to 8000 365 -> 301, 313 of 1000 to 4000
+    // 561 -> 536, window 1280 279 -> 278; 64 of 4000 178 -> 176.
     // (Heads first, without an order, 512 of 300 to 3000, window 2048 560 -> 542.)
     a.order = a.KS == 1 && groups > 256 && T_ <= KV_ORDER &&
-              max_blocks * BS > 1024 && (window <= 0 || window > 1024);
+              max_blocks * BS > 1024 &&
+              (window <= 0 || window > (groups > 512 ? 1024 : 1536));
     grid = dim3((unsigned)(groups * a.KS));
   }
 #define WA_GO(DK, VB, CAP)                                                   \
