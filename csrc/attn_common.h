@@ -115,7 +115,9 @@ PS_DEV void kv_wave_sync() {
 // is done with two short ones.
 // Found without a sort: the tile count (at most `most`) that `rank` sequences exceed,
 // bit by bit, among counts that the lanes hold. All keep their places where none has
-// more than KV_SHORT tiles or every one as many as the first, within an eighth. In
+// more than KV_SHORT tiles, every one as many as the first, within an eighth, or one
+// more than `whole` tiles, which are several workgroups' (counts say nothing of their
+// work then). In
 // more than four rounds, where workgroups start as others end, those of up to
 // KV_SHORT tiles keep theirs (`mine` is the place's own count) and do not wait for
 // the others' lengths (32/8 heads, 256 x 20 to 300 keys 37 us, 41 otherwise); in few
@@ -124,7 +126,7 @@ PS_DEV void kv_wave_sync() {
 #define KV_SHORT 16
 template <typename F>
 PS_DEV int kv_order(F tiles_of, int count, int pos, int lane, int half,
-                    int mine, int most) {
+                    int mine, int most, int whole = 0x7fffffff) {
   const int skip = count > 4 * half ? KV_SHORT : 0;
   if (mine <= skip) return pos;
   int tiles[KV_ORDER / 64];
@@ -147,7 +149,7 @@ PS_DEV int kv_order(F tiles_of, int count, int pos, int lane, int half,
     if (j * 64 < count)
       even &= __all(tiles[j] < 0 || abs(tiles[j] - first) <= first / 8);
   int seq = pos;
-  if (!even && above(KV_SHORT) > 0) {
+  if (!even && above(KV_SHORT) > 0 && above(whole) == 0) {
     int rank = 0;  // of this place among those of longer ones
 #pragma unroll
     for (int j = 0; j < KV_ORDER / 64; ++j) {
