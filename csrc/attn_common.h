@@ -112,16 +112,19 @@ PS_DEV void kv_wave_sync() {
 // (`half` places each) from the shortest on, as its workgroups join the first
 // round's on their CUs: every CU then has about as many keys to read, and all of
 // them stay busy to the end. As sequences come, a CU has two long ones while another
-// is done with two short ones.
+// is done with two short ones. Where the second round is not full, the first places,
+// which it joins, have the shortest ones of the first (us, as they come / the longest
+// ones there / so: 33 of 2000 to 4000 keys 91 / 101 / 83, fp8 40 / 46 / 40; 40 of 300
+// to 4000 93 / 71 / 68).
 // Found without a sort: the tile count (at most `most`) that `rank` sequences exceed,
 // bit by bit, among counts that the lanes hold. All keep their places where none has
 // more than KV_SHORT tiles, every one as many as the first, within an eighth, or one
 // more than `whole` tiles, which are several workgroups' (counts say nothing of their
-// work then). In
-// more than four rounds, where workgroups start as others end, those of up to
-// KV_SHORT tiles keep theirs (`mine` is the place's own count) and do not wait for
-// the others' lengths (32/8 heads, 256 x 20 to 300 keys 37 us, 41 otherwise); in few
-// they have to pair with long ones (61 of 300 to 4000 98 us, 109 otherwise).
+// work then). In more than four rounds, where workgroups start as others end, those
+// of up to KV_SHORT tiles keep theirs (`mine` is the place's own count) and do not
+// wait for the others' lengths (32/8 heads, 256 x 20 to 300 keys 37 us, 41
+// otherwise); in few they have to pair with long ones (61 of 300 to 4000 98 us, 109
+// otherwise).
 #define KV_ORDER 320  // sequences at most
 #define KV_SHORT 16
 template <typename F>
@@ -158,7 +161,11 @@ PS_DEV int kv_order(F tiles_of, int count, int pos, int lane, int half,
         rank += __popcll(__ballot(tiles[j] > skip && lane < at));
     }
     const int end = min(2 * half, above(skip));
-    if (rank >= half && rank < end) rank = half + end - 1 - rank;
+    const int pairs = skip > 0 ? half : end - half;  // CUs that get a second one
+    if (rank >= half && rank < end)
+      rank = half + end - 1 - rank;
+    else if (rank < half && pairs > 0)
+      rank += rank < pairs ? half - pairs : -pairs;
     int t = 0;
     for (int b = 31 - __clz(most | 1); b >= 0; --b)
       if (above(t + (1 << b) - 1) > rank) t += 1 << b;

@@ -186,6 +186,7 @@ def test_paged_attn_decode_many_heads(S, qh, kh, hd, window, fp8):
     (320, 8, 8, 128, 2100, False, 2300),
     (321, 8, 8, 128, 0, False, 1100),   # as they come
     (64, 16, 8, 128, 0, True, 4000),    # no split of the longest
+    (45, 16, 8, 128, 0, False, 1100),   # second round partly full
     (64, 16, 8, 128, 0, False, -1100)])  # within an eighth: as they come
 def test_paged_attn_decode_by_length(S, qh, kh, hd, window, fp8, longest):
     """Sequences that workgroups take by their lengths: equal lengths, empty ones

@@ -527,7 +527,7 @@ def test_talk_attention_scores_climb(shape, sink):
     assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
 
 
-@pytest.mark.parametrize("T,G,window", [(33, 8, 0), (33, 8, 1500),
+@pytest.mark.parametrize("T,G,window", [(33, 8, 0), (45, 8, 0), (33, 8, 1500),
                                         (33, 8, 1550), (70, 8, 1500),
                                         (150, 8, 0), (320, 1, 0), (321, 1, 0)])
 def test_window_attention_token_order(T, G, window):
