@@ -194,7 +194,7 @@ void paged_attn_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
                        at::Tensor seq_lens, double scale, int64_t num_splits,
                        int64_t variant, int64_t window) {
   CHECK_GPU_BF16(out);
-  TORCH_CHECK(out.sizes() == q.sizes(), "out must have q's shape");
+  TORCH_CHECK(out.numel() == q.numel(), "out must have q's size");
   const int kv_fp8 = cache_fp8(k_cache);
   cache_fp8(v_cache);
   CHECK_GPU_DTYPE(block_tables, at::kInt);
@@ -247,7 +247,7 @@ void paged_attn_prefill(at::Tensor out, at::Tensor q, at::Tensor k_cache,
                         at::Tensor token_seq, at::Tensor token_pos,
                         double scale, int64_t window) {
   CHECK_GPU_BF16(out);
-  TORCH_CHECK(out.sizes() == q.sizes(), "out must have q's shape");
+  TORCH_CHECK(out.numel() == q.numel(), "out must have q's size");
   CHECK_GPU_BF16(k_cache);
   CHECK_GPU_BF16(v_cache);
   CHECK_GPU_DTYPE(block_tables, at::kInt);
@@ -275,7 +275,7 @@ void paged_attn_prefill_mfma(at::Tensor out, at::Tensor q,
                              at::Tensor block_tables, at::Tensor tile_info,
                              double scale, int64_t variant, int64_t window) {
   CHECK_GPU_BF16(out);
-  TORCH_CHECK(out.sizes() == q.sizes(), "out must have q's shape");
+  TORCH_CHECK(out.numel() == q.numel(), "out must have q's size");
   const int kv_fp8 = cache_fp8(k_cache);
   cache_fp8(v_cache);
   CHECK_GPU_DTYPE(block_tables, at::kInt);

@@ -221,6 +221,28 @@ def test_paged_attn_decode_by_length(S, qh, kh, hd, window, fp8, longest):
     _close(got, want.cpu())
 
 
+def test_paged_attn_out_rows():
+    """A result buffer of one row a token, all heads side by side, is taken as
+    one of q's shape is; one of another size is refused."""
+    S, qh, kh, hd = 5, 8, 2, 128
+    kc, vc = _make_cache(40, kh, 16, hd)
+    tables = torch.randint(0, 40, (S, 8), dtype=torch.int32, device="cuda")
+    lens = torch.tensor([1, 17, 33, 100, 128], dtype=torch.int32, device="cuda")
+    seq = torch.arange(S, dtype=torch.int32, device="cuda")
+    tiles = torch.tensor([[i, i, int(n) - 1, 1] for i, n in enumerate(lens)],
+                         dtype=torch.int32, device="cuda")
+    q = torch.randn(S, qh, hd, device="cuda").to(torch.bfloat16)
+    for fn, args in ((ops.paged_attn_decode, (tables, lens)),
+                     (ops.paged_attn_prefill, (tables, seq, lens - 1)),
+                     (ops.paged_attn_prefill_mfma, (tables, tiles))):
+        want = fn(q, kc, vc, *args, hd ** -0.5)
+        rows = torch.empty(S, qh * hd, dtype=torch.bfloat16, device="cuda")
+        fn(q, kc, vc, *args, hd ** -0.5, out=rows)
+        assert torch.equal(rows.view(S, qh, hd), want)
+        with pytest.raises(RuntimeError, match="size"):
+            fn(q, kc, vc, *args, hd ** -0.5, out=rows[:-1])
+
+
 @pytest.mark.parametrize("num_splits", [1, 2, 4, 8, 32])
 def test_paged_attn_decode_split_kv(num_splits):
     """All split factors must agree with the reference (incl. splits that
