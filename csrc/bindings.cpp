@@ -485,7 +485,7 @@ void rope_cache_parts(at::Tensor q, at::Tensor parts, at::Tensor positions,
   TORCH_CHECK(rc == 0, "unsupported head width ", HD);
 }
 
-// what the norm before a product needs: dense rows
+// what the norm before a product needs: dense rows on 16-byte borders
 static void check_norm(const at::Tensor& x, const c10::optional<at::Tensor>& res,
                        const at::Tensor& nw,
                        const c10::optional<at::Tensor>& res_out) {
@@ -494,6 +494,11 @@ static void check_norm(const at::Tensor& x, const c10::optional<at::Tensor>& res
   TORCH_CHECK(nw.numel() == x.size(1), "norm width mismatch");
   TORCH_CHECK(res.has_value() == res_out.has_value(),
               "a residual comes with a buffer for its sum");
+  TORCH_CHECK((((size_t)nw.data_ptr() |
+                (size_t)(res ? res->data_ptr() : nullptr) |
+                (size_t)(res ? res_out->data_ptr() : nullptr)) &
+               15) == 0,
+              "rows must be aligned to 16 bytes");
   if (res.has_value()) {
     CHECK_GPU_BF16(*res);
     CHECK_GPU_BF16(*res_out);

@@ -194,10 +194,12 @@ class LlamaLayer(nn.Module):
         plain = fp8 is None and not lora
         few = plain and hidden.shape[-2] <= gemm_policy.MAX_ROWS
         rope_behind = (few and self.qkv_bias is None
-                       and self.head_dim % 16 == 0)
+                       and self.head_dim % 16 == 0
+                       and gemm_policy.dense(cos_sin, *kv_cache))
         fuse_rope = 0
         if rope_behind and hidden.dim() == 2:
-            fuse_rope = gemm_policy.fused(hidden, self.qkv_proj)
+            fuse_rope = gemm_policy.fused(hidden, self.qkv_proj, residual,
+                                          self.input_norm)
         qkv_parts = None
         if fuse_q:
             if residual is None:

@@ -267,19 +267,25 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.linear(x, w)
 
 
-def fused(x: torch.Tensor, w: torch.Tensor) -> int:
+def dense(*tensors) -> bool:
+    """Dense tensors (or None) that may be accessed 16 bytes at a time."""
+    return all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0)
+               for t in tensors)
+
+
+def fused(x: torch.Tensor, w: torch.Tensor, *before) -> int:
     """What the launch of x @ w.T may have around it: 0 nothing, 1 the rotary
     embedding and the cache's rows behind it, 2 the residual's sum and the norm
-    before it too. That is as many rows as LDS has room for (a launch of its own
-    costs a decode step 3.5 us and up; the norm in every workgroup of 8 x 4096
-    entries as much)."""
+    (of `before`: residual and weights) before it too. That is as many rows as
+    LDS has room for (a launch of its own costs a decode step 3.5 us and up; the
+    norm in every workgroup of 8 x 4096 entries as much)."""
     if x.shape[0] > 16:
         return 0
     entries = x.shape[0] * x.shape[-1]
     if (entries > _LDS_X or _choose(x, w, "around") != 1
             or not _fits(x, w) or (w.shape[0] + 32) * w.shape[1] >= 1 << 31):
         return 0
-    return 2 if entries <= _LDS_NORM_X and x.is_contiguous() else 1
+    return 2 if entries <= _LDS_NORM_X and dense(x, *before) else 1
 
 
 def silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -306,7 +312,7 @@ def norm_silu_mul(x: torch.Tensor, residual: torch.Tensor,
     partial sums; x and residual may be overwritten."""
     from production_stack_amd import ops
 
-    if x.dim() == 2 and fused(x, w) == 2 and residual.is_contiguous():
+    if x.dim() == 2 and fused(x, w, residual, norm_w) == 2:
         return ops.skinny_norm_gated(x, residual, norm_w, eps, w)
     add_norm = (ops.fused_add_rms_norm if x.dim() == 2
                 else ops.add_rms_norm_parts)

@@ -1184,6 +1184,32 @@ def test_skinny_norm_gated(M, N, K, res):
     assert (got.double() - want).norm() <= 2e-3 * want.norm()
 
 
+def test_skinny_norm_borders():
+    """A residual or norm weights off 16-byte borders: not the dispatch's for the
+    launch that has the norm in it, and refused there before anything runs."""
+    from production_stack_amd.ops import gemm_policy
+
+    gemm_policy.reset()
+    M, N, K = 4, 4096, 2048
+    x, r = (torch.randn(M, K, device="cuda").to(torch.bfloat16)
+            for _ in range(2))
+    nw = torch.randn(K, device="cuda").to(torch.bfloat16)
+    w = torch.randn(N, K, device="cuda").to(torch.bfloat16)
+
+    def off(t):
+        buf = torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")
+        return buf[1:t.numel() + 1].view(t.shape).copy_(t)
+
+    assert gemm_policy.fused(x, w, r, nw) == 2
+    assert gemm_policy.fused(x, w, None, nw) == 2
+    for args in ((off(r), nw), (r, off(nw)), (None, off(nw)),
+                 (torch.cat([r, r], 1)[:, :K], nw)):
+        assert gemm_policy.fused(x, w, *args) == 1
+    for args in ((off(r), nw), (r, off(nw)), (None, off(nw))):
+        with pytest.raises(RuntimeError, match="aligned"):
+            ops.skinny_norm_gated(x, *args, 1e-5, w)
+
+
 @pytest.mark.parametrize("M,qh,kh,hd,K,fp8", [
     (1, 32, 8, 64, 2048, False), (4, 7, 1, 128, 4096, True),
     (8, 4, 4, 16, 2048, False), (3, 6, 2, 96, 1088, True),
