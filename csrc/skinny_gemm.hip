@@ -46,8 +46,8 @@ PS_DEV ps_gbf16x8 ps_as_gbf16(ps_bf16x8 u) {
 // are nothing. Where 16 rows a workgroup leave half of the CUs without one (us at
 // one row, 16 rows / 8 / the library: 2048 x 2048 5.4 / 4.5 / 11.0, 2048 x 8192
 // 12.0 / 8.6 / 12.7, 1024 x 4096 7.4 / 5.4 / 14.4).
-// FAR: W by its addresses, where 31-bit offsets do not reach its up rows or it is
-// not aligned to 16 bytes.
+// FAR: W by its addresses, where 31-bit offsets do not reach a tile's last row or
+// it is not aligned to 16 bytes.
 template <int UC, int NW, bool GATED, bool HALF, bool FAR>
 __global__ __launch_bounds__(NW * 64) void skinny_rows_kernel(
     unsigned short* __restrict__ out, const unsigned short* __restrict__ x,
@@ -836,7 +836,8 @@ static void ps_skinny_rows_go(void* out, const void* x, const void* w, int M,
       <<<N / (HALF ? 8 : 16), NW * 64, 0, stream>>>(                        \
           (unsigned short*)out, (const unsigned short*)x,                   \
           (const unsigned short*)w, M, N, K, (int)x_stride)
-  if (((size_t)w & 15) != 0 || (GATED && (long)(N + 32) * K >= 1L << 31)) {
+  // offsets from a tile's first row reach 15 rows on, gated those N / 2 behind
+  if (((size_t)w & 15) != 0 || (GATED ? N + 32L : 32L) * K >= 1L << 31) {
     PS_SR(1, 16, false, true);
     return;
   }

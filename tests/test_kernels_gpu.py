@@ -1184,6 +1184,20 @@ def test_skinny_norm_gated(M, N, K, res):
     assert (got.double() - want).norm() <= 2e-3 * want.norm()
 
 
+def test_skinny_gemm_longest_rows():
+    """Rows of W so long that 31-bit offsets do not reach the last of 16: every
+    row's last entries are multiplied."""
+    N, K = 64, 72 << 20
+    w = torch.zeros(N, K, dtype=torch.bfloat16, device="cuda")
+    x = torch.zeros(9, K, dtype=torch.bfloat16, device="cuda")
+    w[:, -1] = torch.arange(1, N + 1, device="cuda").to(torch.bfloat16)
+    w[:, 1] = 1.0
+    x[8, 1] = x[8, -1] = 2.0
+    want = 2.0 * torch.arange(1, N + 1, device="cuda") + 2.0
+    got = ops.skinny_gemm(x, w).float()
+    assert torch.equal(got[8], want) and not got[:8].any()
+
+
 def test_skinny_norm_borders():
     """A residual or norm weights off 16-byte borders: not the dispatch's for the
     launch that has the norm in it, and refused there before anything runs."""
