@@ -113,6 +113,14 @@ def build_cos_sin_cache(
     return torch.cat([freqs.cos(), freqs.sin()], dim=-1).float().contiguous()
 
 
+def _hooked(module: nn.Module) -> bool:
+    """Something looks at what the module takes or returns."""
+    every = nn.modules.module
+    return bool(module._forward_hooks or module._forward_pre_hooks
+                or every._global_forward_hooks
+                or every._global_forward_pre_hooks)
+
+
 class LlamaLayer(nn.Module):
     def __init__(self, cfg: ModelConfig, tp: int, layer_idx: int = 0) -> None:
         super().__init__()
@@ -565,11 +573,12 @@ class LlamaForCausalLM(nn.Module):
             residual = None
         else:
             hidden = token_ids  # mid-pipeline: activations from prev stage
+        # norms add partial sums; hooks and the next stage ask for rows
+        rows = [_hooked(layer) for layer in self.layers] + [not self.is_last]
         for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):
             hidden, residual = layer(
                 hidden, residual, meta, cache, self.cos_sin,
-                # norms add partial sums; the next stage asks for rows
-                parts_out=self.is_last or i + 1 < len(self.layers),
+                parts_out=not (rows[i] or rows[i + 1]),
             )
         if not self.is_last:
             # caller ships (hidden, residual) to the next stage

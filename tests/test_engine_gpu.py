@@ -509,3 +509,82 @@ def test_logprobs_and_prompt_logprobs_gpu():
     assert all(v <= 0 for v in plp[1:])
     for row, chosen in zip(tops, lps):
         assert abs(max(v for _, v in row) - chosen) < 1e-4
+
+
+@pytest.fixture(scope="module")
+def wide_llama():
+    """Three layers of an 8b-sized stack."""
+    import dataclasses
+
+    from production_stack_amd.engine.config import ARCHITECTURES
+    from production_stack_amd.engine.models.llama import LlamaForCausalLM
+
+    cfg = dataclasses.replace(ARCHITECTURES["llama-3-8b"], num_layers=3,
+                              vocab_size=512, max_position=256)
+    with torch.device("cuda"):
+        model = LlamaForCausalLM(cfg)
+    model.random_init(3)
+    return model
+
+
+def _wide_step(model, rows, prompt, kv):
+    """(tokens, meta, caches) of a step of `rows` rows, the first `prompt` of
+    them of one prompt behind 20 positions, the others single tokens."""
+    from production_stack_amd import ops
+    from production_stack_amd.engine.models.llama import BatchMeta
+
+    cfg, bs, per = model.cfg, 16, 12
+    g = torch.Generator().manual_seed(rows)
+    seqs = rows - prompt + (1 if prompt else 0)
+    tables = torch.randperm(seqs * per, generator=g).int().view(seqs, per)
+    lens = torch.randint(1, per * bs - 1, (rows - prompt,), generator=g)
+    pos = torch.cat([torch.arange(20, 20 + prompt), lens - 1])
+    seq = torch.cat([torch.zeros(prompt, dtype=torch.long),
+                     torch.arange(seqs - len(lens), seqs)])
+    slots = tables[seq, pos // bs].long() * bs + pos % bs
+    tile = ops.prefill_tile_rows(cfg.num_q_heads, cfg.num_kv_heads)
+    tiles = [(0, t, 20 + t, min(tile, prompt - t))
+             for t in range(0, prompt, tile)]
+    first = 1 if prompt else 0
+
+    def dev(x, dtype=torch.int32):
+        return x.to(dtype).cuda()
+
+    meta = BatchMeta(
+        positions=dev(pos), slot_mapping=dev(slots, torch.long),
+        num_prefill_tokens=prompt,
+        prefill_token_seq=dev(seq[:prompt]) if prompt else None,
+        prefill_token_pos=dev(pos[:prompt]) if prompt else None,
+        prefill_block_tables=dev(tables[:1]) if prompt else None,
+        num_decode_seqs=len(lens), decode_seq_lens=dev(lens),
+        decode_block_tables=dev(tables[first:]),
+        prefill_tiles=dev(torch.tensor(tiles)) if prompt else None)
+    shape = (seqs * per, cfg.num_kv_heads, bs, cfg.head_dim)
+    dt = torch.float8_e4m3fn if kv == "fp8" else torch.bfloat16
+    caches = [tuple(torch.randn(shape, generator=g).cuda().to(dt)
+                    for _ in range(2)) for _ in model.layers]
+    tokens = torch.randint(0, cfg.vocab_size, (rows,), generator=g).cuda()
+    return tokens, meta, caches
+
+
+def test_joined_launches_hooks(wide_llama):
+    """A hook on a layer sees hidden rows, as without joined launches, and the
+    rows behind it are the same."""
+    from production_stack_amd.ops import gemm_policy
+
+    gemm_policy.reset()
+    tokens, meta, caches = _wide_step(wide_llama, 64, 0, "auto")
+    want = wide_llama(tokens, meta, caches)
+    seen = []
+    hooks = [
+        wide_llama.layers[0].register_forward_hook(
+            lambda m, a, out: seen.append(out[0].shape)),
+        wide_llama.layers[2].register_forward_pre_hook(
+            lambda m, a: seen.append(a[0].shape))]
+    try:
+        got = wide_llama(tokens, meta, caches)
+    finally:
+        for h in hooks:
+            h.remove()
+    assert seen == [want.shape, want.shape]
+    assert (got.double() - want.double()).norm() <= 0.03 * want.double().norm()
