@@ -567,6 +567,70 @@ def _wide_step(model, rows, prompt, kv):
     return tokens, meta, caches
 
 
+# per layer: launches joined with a product at these row counts
+_JOINED = {
+    1: dict(skinny_rope=1, skinny_norm_gated=1),
+    4: dict(skinny_rope=1, skinny_norm_gated=1),
+    8: dict(skinny_rope=1, skinny_gated=1),
+    16: dict(skinny_rope=1, skinny_gated=1),
+    17: dict(skinny_parts=2, skinny_gated_tiles=1, add_rms_norm_parts=2),
+    63: dict(skinny_parts=1, skinny_gated_tiles=1, add_rms_norm_parts=1),
+    64: dict(skinny_parts=2, skinny_gated_tiles=1, add_rms_norm_parts=2),
+    96: dict(skinny_parts=2, add_rms_norm_parts=2),
+    128: dict(skinny_parts=3, add_rms_norm_parts=2, rope_cache_parts=1),
+    192: dict(skinny_parts=3, add_rms_norm_parts=2, rope_cache_parts=1),
+    193: {},
+}
+
+
+@pytest.mark.parametrize("rows", list(_JOINED))
+@pytest.mark.parametrize("prompt,kv", [(0, "auto"), (0, "fp8"), (40, "auto")])
+def test_joined_launches(wide_llama, rows, prompt, kv, monkeypatch):
+    """A stack whose products share launches with the norms, rotary embeddings
+    and activations around them, in each of the ways that the row counts pick,
+    against the library's products and the separate kernels: hidden rows and
+    the caches' new rows of every layer."""
+    from production_stack_amd import ops
+    from production_stack_amd.ops import gemm_policy
+
+    if prompt >= rows:
+        pytest.skip("no room for the prompt")
+    gemm_policy.reset()
+    calls = {}
+    for name in {n for d in _JOINED.values() for n in d}:
+        def count(*a, _fn=getattr(ops, name), _name=name, **kw):
+            calls[_name] = calls.get(_name, 0) + 1
+            return _fn(*a, **kw)
+        monkeypatch.setattr(ops, name, count)
+    tokens, meta, caches = _wide_step(wide_llama, rows, prompt, kv)
+    plain = [tuple(c.clone() for c in kv) for kv in caches]
+    got = wide_llama(tokens, meta, caches)
+    layers = len(wide_llama.layers)
+    assert calls == {n: layers * c for n, c in _JOINED[rows].items()}
+    logits = wide_llama.compute_logits(got)
+    calls.clear()
+    monkeypatch.setattr(gemm_policy, "_choose", lambda *a: 0)
+    want = wide_llama(tokens, meta, plain)
+    assert not calls
+
+    def far(a, b):
+        return float((a.double() - b.double()).norm() / b.double().norm())
+
+    # bf16 roundings of sums in another order, layer after layer: hidden rows
+    # differ by 0.007, the last layer's keys and values by 0.006, in steps of
+    # e4m3 by 0.016; four times that
+    at = meta.slot_mapping
+    for mine, theirs in zip(caches, plain):
+        for a, b in zip(mine, theirs):
+            a, b = (c.transpose(1, 2).reshape(-1, *c.shape[1::2])
+                    .to(torch.bfloat16) for c in (a, b))
+            assert far(a[at], b[at]) <= (0.065 if kv == "fp8" else 0.025)
+            a[at] = b[at]
+            assert torch.equal(a, b)            # no other row was written
+    assert got.shape == want.shape and far(got, want) <= 0.03
+    assert far(logits, wide_llama.compute_logits(want)) <= 0.03
+
+
 def test_joined_launches_hooks(wide_llama):
     """A hook on a layer sees hidden rows, as without joined launches, and the
     rows behind it are the same."""
