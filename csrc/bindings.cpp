@@ -72,6 +72,7 @@ void ps_kv_dequant(void* out, const void* in, const void* scales, long rows,
 int ps_skinny_gemm_splits(int M, int N, int K);
 int ps_skinny_gemm(void* out_bf16, void* ws, const void* x, const void* w,
                    int M, int N, int K, long x_stride, hipStream_t stream);
+void ps_skinny_limits(int* most);
 int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
                     int K, long x_stride, hipStream_t stream);
 int ps_skinny_parts(void* ws, const void* x, const void* w, int M, int N,
@@ -718,6 +719,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "8-phase deep-pipelined bf16 GEMM (out = x @ w.T)");
   m.def("skinny_gemm", &skinny_gemm,
         "MFMA GEMM for decode-shaped (M<=256) projections");
+  m.def("skinny_limits", [] {
+    int most[2];
+    ps_skinny_limits(most);
+    return std::make_pair(most[0], most[1]);
+  }, "Most entries of x in LDS, without the norm and with it");
   m.def("skinny_parts", &skinny_parts,
         "Partial sums of a split skinny GEMM, or None");
   m.def("skinny_gated_tiles", &skinny_gated_tiles,

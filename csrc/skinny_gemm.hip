@@ -495,8 +495,8 @@ __global__ __launch_bounds__(256, 4) void skinny_gemm_kernel(
   }
 }
 
-// The tiled form, for 17 to 256 rows of x (and 9 to 16 of a W of more than
-// 32768): a workgroup owns 64 NC rows of W, all rows of x and a range of K, in
+// The tiled form, for 17 to 256 rows of x (and 9 to 16 of a W of more than 32768
+// where LDS has no room for x): a workgroup owns 64 NC rows of W, all rows of x and a range of K, in
 // steps of 128 columns. x passes through LDS, two steps' buffers with one barrier
 // a step; W goes from memory straight into left operands, WD steps ahead. The
 // eight waves are four by rows of W times two by halves of a step, which add up in
@@ -728,8 +728,8 @@ struct PsSkinnyPlan {
 // two, three, the first half of a fourth, all of it, more). 17 x 45056 x 512 15 / 17,
 // x 1024 30 / 26; 17 x 78848 x 1536 54 / 57; 24 x 102400 x 4096 161 / 175; 24 x
 // 128256 x 1536 84 / 90; 64 x 128256 x 1280 86 / 90; 128 x 128256 x 512 62 / 62;
-// 192 x 95232 x 384 56 / 50; 256 x 61440 x 1024 81 / 85. Rows of 2048 columns come from few
-// channels in the short form (17 x 128256 x 2048 129 / 102).
+// 192 x 95232 x 384 56 / 50; 256 x 61440 x 1024 81 / 85. Rows of 2048 columns come
+// from few channels in the short form (17 x 128256 x 2048 129 / 102).
 static bool ps_skinny_short(int M, int N, int K) {
   if (K < 128) return true;
   if (N <= 32768) {
@@ -881,7 +881,9 @@ static void ps_skinny_rows_go(void* out, const void* x, const void* w, int M,
 
 extern "C" {
 
-// out [M, N / 2] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu]; -1: not built
+// out [M, N / 2] = silu(x Wg^T) * (x Wu^T), W = [Wg; Wu]; -1: not built. Of a W of
+// more than 32768 rows only up to 8 rows of x: callers take the plain product and
+// the activation for more.
 int ps_skinny_gated(void* out, const void* x, const void* w, int M, int N,
                     int K, long x_stride, hipStream_t stream) {
   if (M < 1 || N < 64 || K < 64 || N % 64 != 0 || K % 64 != 0 ||
@@ -950,6 +952,12 @@ int ps_skinny_rope(void* out, void* res_out, const void* x, long x_stride,
   else
     ps_skinny_lds_go<SL_ROPE, false>(a, stream);
   return 0;
+}
+
+// Most entries of x that LDS has room for, without the norm and with it.
+void ps_skinny_limits(int* most) {
+  most[0] = SL_X;
+  most[1] = SL_NORM_X;
 }
 
 // ws == nullptr forces splits = 1. ps_skinny_gemm_splits reports the

@@ -99,7 +99,8 @@ def _fits(x: torch.Tensor, w: torch.Tensor) -> bool:
                      and (x.requires_grad or w.requires_grad)))
 
 
-# entries of x that the kernel with x in LDS takes, with the norm and without
+# entries of x that the kernel with x in LDS takes, without the norm and with it
+# (what _C.skinny_limits() says)
 _LDS_X, _LDS_NORM_X = 65536, 16384
 
 
@@ -159,9 +160,10 @@ def _rows_before_norm(rows: int, N: int, K: int) -> bool:
     Long rows: 64 x 4096 x 14336 33.3 / 43.7, 17 x 8192 x 10240 41.7 / 42.1, but 20 x
     8192 x 13824 51.3 / 47.0, 17 x 4096 x 12288 28.1 / 26.8, 104 x 1024 x 10240 21.6 /
     19.2.
-    More than 64 rows: 96 x 4096 x 4096 21.4 / 25.3, 192 24.8 / 36.3, but 80 21.0 / 19.9,
-    112 22.0 / 20.0; 144 24.0 / 25.5; 80 x 5120 x 4096 25.2 / 21.4, 112 26.1 / 27.7, 149 x
-    5376 x 4096 28.4 / 27.1; 80 x 6144 x 4096 25.9 / 27.5, 144 30.8 / 43.8, 176 1.02 times.
+    More than 64 rows: 96 x 4096 x 4096 21.4 / 25.3, 192 24.8 / 36.3, but 80 21.0 /
+    19.9, 112 22.0 / 20.0; 144 24.0 / 25.5; 80 x 5120 x 4096 25.2 / 21.4, 112 26.1 /
+    27.7, 149 x 5376 x 4096 28.4 / 27.1; 80 x 6144 x 4096 25.9 / 27.5, 144 30.8 /
+    43.8, 176 1.02 times.
     Fewer: few rows of W (17 x 2048 x 2048 10.1 / 13.7, 63 x 2048 x 4096 14.2 / 15.0, 48
     x 2560 x 2048 13.5 / 14.8; 25 x 2048 x 1024 9.0 / 8.4, 60 x 1024 x 1280 up to 1.2
     times, 48 x 2560 x 2560 14.5 / 12.7), of more 64 x 4096 x 4096 17.6 / 18.6 and 32 x

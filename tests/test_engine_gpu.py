@@ -583,8 +583,9 @@ _JOINED = {
 }
 
 
-@pytest.mark.parametrize("rows", list(_JOINED))
-@pytest.mark.parametrize("prompt,kv", [(0, "auto"), (0, "fp8"), (40, "auto")])
+@pytest.mark.parametrize("rows,prompt,kv", [
+    (rows, *case) for case in ((0, "auto"), (0, "fp8"), (40, "auto"))
+    for rows in _JOINED if rows > case[0]])
 def test_joined_launches(wide_llama, rows, prompt, kv, monkeypatch):
     """A stack whose products share launches with the norms, rotary embeddings
     and activations around them, in each of the ways that the row counts pick,
@@ -593,8 +594,6 @@ def test_joined_launches(wide_llama, rows, prompt, kv, monkeypatch):
     from production_stack_amd import ops
     from production_stack_amd.ops import gemm_policy
 
-    if prompt >= rows:
-        pytest.skip("no room for the prompt")
     gemm_policy.reset()
     calls = {}
     for name in {n for d in _JOINED.values() for n in d}:

@@ -1275,10 +1275,11 @@ def _skinny_rope(M, qh, kh, hd, K, fp8, norm):
         assert (a.double() - b.double()).norm() <= tol * b.double().norm()
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (17, 64, 128), (61, 4096, 4096), (192, 1024, 2176), (256, 4160, 4096),
-    (33, 8256, 1024), (20, 16448, 512)])
-def test_skinny_parts_norm(M, N, K):
+@pytest.mark.parametrize("M,N,K,own", [
+    (17, 64, 128, True), (61, 4096, 4096, True), (192, 1024, 2176, True),
+    (256, 4160, 4096, True), (20, 9216, 8192, True), (33, 8256, 1024, False),
+    (20, 16448, 512, False)])
+def test_skinny_parts_norm(M, N, K, own):
     """Partial sums that the norm adds, from the short form and from tiles, up to
     rows of more than one vector a thread: bit for bit the residual of the
     separate kernels; None where there is one range."""
@@ -1291,8 +1292,8 @@ def test_skinny_parts_norm(M, N, K):
     parts = ops.skinny_parts(x, w)
     want, wr = ops.fused_add_rms_norm(ops.skinny_gemm(x, w), r.clone(), nw,
                                       1e-5)
+    assert (parts is not None) == own
     if parts is None:
-        assert N > 8192
         parts = torch.stack([x.float() @ w.float().t(),
                              torch.zeros(M, N, device="cuda")])
         exact = False
@@ -1340,19 +1341,23 @@ def test_rope_cache_parts(M, qh, kh, hd, K, fp8):
                 <= (2e-2 if fp8 else 1e-3) * b.double().norm())
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (17, 28672, 2048), (64, 32768, 256), (65, 16384, 1088), (192, 28672, 192),
-    (100, 49152, 128)])
-def test_skinny_gated_tiles(M, N, K):
-    """Tiles of gate and up rows with the activation behind, both widths."""
+@pytest.mark.parametrize("M,N,K,own", [
+    (17, 28672, 2048, True), (64, 32768, 256, True), (65, 16384, 1088, True),
+    (192, 28672, 192, True), (32, 28736, 1024, True), (128, 28672, 1024, True),
+    (100, 49152, 128, False), (193, 28672, 1024, False),
+    (64, 4096, 4096, False)])
+def test_skinny_gated_tiles(M, N, K, own):
+    """Tiles of gate and up rows with the activation behind, both widths at all
+    heights; None in the short form, past 192 rows and where tiles have a range
+    of K."""
     g = torch.Generator(device="cuda").manual_seed(M + K)
     x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(
         torch.bfloat16)
     got = ops.skinny_gated_tiles(x, w)
     want = ops.silu_and_mul(ops.skinny_gemm(x, w)).double()
-    if got is None:  # the short form
-        assert K <= 1088
+    assert (got is not None) == own
+    if got is None:
         return
     # ranges begin at other steps: sums in another order, roundings the same
     assert (got.double() - want).norm() <= 2e-3 * want.norm()

@@ -90,6 +90,17 @@ def test_rope_preserves_tail_dims():
     )
 
 
+def test_gemm_policy_limits():
+    """The dispatch's idea of what fits in LDS is the kernel's."""
+    from production_stack_amd import ops
+    from production_stack_amd.ops import gemm_policy
+
+    if not ops.HAVE_EXT:
+        pytest.skip("extension not built")
+    assert ops._C.skinny_limits() == (gemm_policy._LDS_X,
+                                      gemm_policy._LDS_NORM_X)
+
+
 @pytest.mark.parametrize("rule,shape,own", [
     # rows, rows of W, entries of each: on either side of each line
     ("few_rows", (1, 28672, 512), True), ("few_rows", (1, 28672, 256), False),
