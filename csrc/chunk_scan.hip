@@ -209,7 +209,7 @@ PS_DEV float ck_wave_sums(const float (&x)[8]) {
 }
 
 // Lays down a chunk's operands: a workgroup per (chunk, head), a lane per channel
-// of eight rows. Bound by its vector instructions (1190 a wave for the general
+// of eight rows. Bound by its vector instructions (1100 a wave for the general
 // delta, three waves a SIMD: registers), beside a write of 32 KB. Four workgroups a
 // CU spill for the channel delta (480 -> 500 us of its whole operation).
 template <typename T, int MODE, int DP>
@@ -2428,11 +2428,11 @@ static long ck_chunk_floats(int mode, int dp, int H, int G, int L) {
 }
 
 // Measured (bf16, one MI355X, whole operation; token by token -> this form):
-//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.67 ms
-//     (operands 0.21, walk 0.41, read-out 0.04)
+//   general delta 32 heads 128x128, 8011 rows in 2 prompts   12.3 -> 0.68 ms
+//     (operands 0.19, walk 0.45, read-out 0.04)
 //   channel delta 32 x 128x128, 6007 rows in 3 prompts, 37 single tokens
 //                                                            5.42 -> 0.48 ms
-//     (operands 0.14, walk 0.27, tokens 0.03)
+//     (operands 0.15, walk 0.27, tokens 0.03, read-out 0.03)
 //   ssd 128 heads 128x64, 8192 rows in 2 prompts             6.91 -> 0.30 ms
 //   gla 8 heads 128x256, 1501 rows                           2.12 -> 0.06 ms
 //   mlstm 32 heads 128x128, 8192 rows in 2 prompts           6.41 -> 0.47 ms

@@ -435,9 +435,10 @@ extern "C" int ps_paged_attn_decode(
   // more than 1024 keys: below, the trip to memory for all lengths costs more than
   // the order gives (64 sequences of up to 1000 keys 33.6 us, 30.5 ordered, but 256
   // of up to 500 60.7 / 63.5; 64 of one length 94 / 95; 61 of up to 4000 of which a
-  // window shows 1500 54 / 56). Over 320 sequences fill the
-  // CUs five times over, and the order's counts take their time in each workgroup
-  // (fp8, 512 of up to 1000 keys 111 / 120, 400 of 1000 to 8000 689 / 649).
+  // window shows 1500 54 / 56). Over 320 sequences fill the CUs five times over, and
+  // the order's counts take their time in each workgroup: fp8, 512 of up to 1000
+  // keys 111 / 120. Long ones would gain even so (400 of 1000 to 8000 689 / 649), but
+  // lengths are not known here, and a lane would hold more counts.
   const int width =
       window > 0 ? std::min(window, max_blocks * 16) : max_blocks * 16;
   const int order =

@@ -628,7 +628,9 @@ int mx_window_attention(void* out, int ldout, const void* q, int ldq,
     // window 2048 77.6 -> 76.3, 1500 54.6 -> 56.4 (50 tokens 47.6 -> 50.1, 1800 57.0 ->
     // 57.7; 40 tokens 44.8 -> 41.1, 64 of 100 to 2500 45.4 -> 43.1); 70 tokens, window
     // 1100 59.4 -> 53.6, 1024 53.3; 100 of 50 to 8000 365 -> 301, 313 of 1000 to 4000
-    // 561 -> 536, window 1280 279 -> 278; 64 of 4000 178 -> 176.
+    // 561 -> 536, window 1280 279 -> 278; 64 of 4000 178 -> 176. Where most of two
+    // rounds' tokens see a whole window it costs up to 5 % (64 of 300 to 4000, window
+    // 2048 76.0 -> 79.8; of 100 to 2500 64.9 -> 56.4).
     // (Heads first, without an order, 512 of 300 to 3000, window 2048 560 -> 542.)
     a.order = a.KS == 1 && groups > 256 && T_ <= KV_ORDER &&
               max_blocks * BS > 1024 &&
