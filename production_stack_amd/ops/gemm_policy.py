@@ -14,7 +14,6 @@ from __future__ import annotations
 
 import logging
 import math
-import time
 from typing import Dict
 
 import torch
@@ -38,15 +37,28 @@ def _eligible_8p(M: int, N: int, K: int) -> bool:
     return N % 256 == 0 and K % 128 == 0
 
 
-def _time_fn(fn, iters: int = 20) -> float:
+_PASSES = 512 << 20  # bytes read between timed calls: twice the last cache
+
+
+def _time_fn(fn, others=None, iters: int = 15) -> float:
+    """Seconds of a call. others: a tensor that is read before each, so that
+    weights come from memory as in a decode step, where the other layers' have
+    passed through the caches. (A matrix that stays there made the skinny kernel
+    win where it loses: steps of 16, 48, 96 and 144 rows of a 1b-sized stack 627,
+    853, 1076 and 1346 us, 598, 823, 1054 and 1254 so.)"""
     for _ in range(3):
         fn()
-    torch.cuda.synchronize()
-    t0 = time.perf_counter()
+    spans = []
     for _ in range(iters):
+        if others is not None:
+            others.max()  # fn is queued before this is done
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
         fn()
+        b.record()
+        spans.append((a, b))
     torch.cuda.synchronize()
-    return (time.perf_counter() - t0) / iters
+    return sorted(a.elapsed_time(b) for a, b in spans)[iters // 2] * 1e-3
 
 
 def tune(weights, buckets, device) -> None:
@@ -58,15 +70,20 @@ def tune(weights, buckets, device) -> None:
     w_by_shape = {}
     for w in weights:
         w_by_shape.setdefault((int(w.shape[0]), int(w.shape[1])), w)
+    try:
+        others = torch.zeros(_PASSES // 4, dtype=torch.int32, device=device)
+    except torch.cuda.OutOfMemoryError:
+        others = None
     for M in buckets:
         for (N, K) in shapes:
             w = w_by_shape[(N, K)]
             x = torch.randn(M, K, dtype=torch.bfloat16, device=device)
-            cands = [(0, _time_fn(lambda: F.linear(x, w)))]
+            cands = [(0, _time_fn(lambda: F.linear(x, w), others))]
             if _eligible(M, N, K):
-                cands.append((1, _time_fn(lambda: ops.skinny_gemm(x, w))))
+                cands.append((1, _time_fn(lambda: ops.skinny_gemm(x, w),
+                                          others)))
             if _eligible_8p(M, N, K):
-                cands.append((2, _time_fn(lambda: ops.gemm8p(x, w))))
+                cands.append((2, _time_fn(lambda: ops.gemm8p(x, w), others)))
             impl, t = min(cands, key=lambda c: c[1])
             _POLICY[(M, N, K)] = impl
             for behind, rules in _UNTUNED.items():
@@ -78,6 +95,8 @@ def tune(weights, buckets, device) -> None:
                     "gemm M=%d N=%d K=%d: impl %s wins at %.1fus",
                     M, N, K, ("blas", "skinny", "8p")[impl], t * 1e6,
                 )
+    del others
+    torch.cuda.empty_cache()
     cells = [v for key, v in _POLICY.items() if len(key) == 3]
     logger.info(
         "gemm autotune done: %d/%d cells use an in-house kernel",

@@ -1424,7 +1424,7 @@ def test_tuned_bare_products(M, N, K, behind, own, bare, monkeypatch):
     order = [1.0, 1.0, 1.0]
     order[bare] = 0.5
     times = iter(order)
-    monkeypatch.setattr(gemm_policy, "_time_fn", lambda fn: next(times))
+    monkeypatch.setattr(gemm_policy, "_time_fn", lambda fn, others: next(times))
     gemm_policy.reset()
     try:
         gemm_policy.tune([w], [M], torch.device("cuda"))
@@ -1458,6 +1458,21 @@ def test_tuned_bare_products(M, N, K, behind, own, bare, monkeypatch):
                 torch.nn.functional.linear(odd, w)))
     finally:
         gemm_policy.reset()
+
+
+def test_tuning_reads_weights_from_memory():
+    """Start-up timing of a product whose W the caches would hold takes as long as
+    reading W from memory does at least."""
+    from production_stack_amd.ops import gemm_policy
+
+    w = torch.randn(8192, 8192, device="cuda").to(torch.bfloat16)  # 134 MB
+    x = torch.randn(1, 8192, device="cuda").to(torch.bfloat16)
+    others = torch.zeros(gemm_policy._PASSES // 4, dtype=torch.int32,
+                         device="cuda")
+    far = gemm_policy._time_fn(lambda: ops.skinny_gemm(x, w), others)
+    near = gemm_policy._time_fn(lambda: ops.skinny_gemm(x, w))
+    # 8 TB/s at most; from the caches it is faster
+    assert far > w.numel() * 2 / 8e12 and far > near
 
 
 def test_skinny_gemm_nothing_to_do():
