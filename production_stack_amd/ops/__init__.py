@@ -758,7 +758,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     portions with a head mix over 32 heads of width 64 or 128 have a
     matrix-core kernel too (variant 0; 10 insists on it). Without a head mix,
     rows of whole 16-byte vectors up to 128 wide take a portion and a token
-    kernel of their own (variants 0 and 3; 11 and 12 insist on them).
+    kernel of their own (variants 0 and 3; 11 and 12 insist on them), and so do
+    fp32 rows of widths in steps of 16 up to 128 (13 and 14 insist on it).
     Returns [T, H*DV]."""
     NB, G, BS, D = k_cache.shape
     VR = v_cache.shape[3]
@@ -893,6 +894,46 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if variant in (11, 12):
         raise RuntimeError(
             "talk_attention: shape or dtype outside the window kernels")
+    # fp32 keys and values of their own, prompt portions or single tokens
+    if (variant in (0, 3, 13, 14) and q.dtype == torch.float32
+            and talk is None and not extra and pool is None):
+        token = variant in (3, 14)
+        rep = H // G
+        keys = block_tables.shape[1] * BS
+        if window > 0:
+            keys = min(keys, window + keep_first)
+        if chunk > 0:
+            keys = min(keys, chunk + keep_first)
+        # 32 columns a wave where those fill the chip twice, else 16 (32/8 heads,
+        # us, 16 / 32: 1000 rows of 128 alone 125 / 122, behind 3000 keys 258 /
+        # 234; 400 rows 26.7 / 28.1; 1000 of 64 37.4 / 43.3)
+        rows = 16
+        if not token and rep <= 32 and max(D, DV) > 64 and (
+                (T + 32 // rep - 1) // (32 // rep) * G >= 512):
+            rows = 32
+        # Several workgroups for a tile's keys where CUs are left: records cost 3
+        # us and 4 bytes a share and entry (1 token x 947 keys 46 us whole, 18.6
+        # in 8 shares; 64 x 1500 162, 157 in 3, 193 in 12; 8 x 300 19.0, 14.5 in
+        # 4; portions: 80 rows behind 334 keys 20.9, 23.9 in 2)
+        tpt = 1 if token else max(1, rows // rep)
+        groups = (T + tpt - 1) // tpt * G
+        shares = splits if splits > 0 else max(1, min(
+            16, (512 if token else 256) // groups,
+            keys // (128 if token else 256)))
+        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
+                            device=q.device) if shares > 1 else None)
+        rc = _mx().mx_attn_f32(
+            _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
+            _p(v_cache), _p(block_tables), block_tables.shape[1],
+            _p(token_seq), _p(token_pos), T, H, G, D, DV, BS, _f(scale),
+            int(chunk), int(window), int(bool(sink)), int(keep_first),
+            _f(softcap), _p(sink_vals), int(VR), int(token), int(rows),
+            int(shares), _p(part), _stream())
+        if rc == 0:
+            return out
+    if variant in (13, 14):
+        raise RuntimeError(
+            "talk_attention: shape or dtype outside the fp32 kernel")
     if variant not in (3, 4, 5, 6):
         splits = 1
     elif splits <= 0:

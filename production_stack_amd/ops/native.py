@@ -10,7 +10,7 @@ shape checks live in the Python wrappers
 
 Groups (one shared library each):
   core    resid32, norm_conv, mixer_prep, talk_attention, talk_mfma,
-          window_attention, mfma_attention, expand_attention, latent_decode, keyval_attention,
+          window_attention, attn_f32, mfma_attention, expand_attention, latent_decode, keyval_attention,
           moe_route, moe_group, mingru_scan -> _mixops.so
   delta   delta_rule                        -> _mixops_delta.so
   gdelta  gated_delta                       -> _mixops_gdelta.so
@@ -51,6 +51,7 @@ GROUPS = {
         ("talk_attention.hip", []),
         ("talk_mfma.hip", []),
         ("window_attention.hip", []),
+        ("attn_f32.hip", []),
         ("mixer_prep.hip", []),
         ("mfma_attention.hip", []),
         ("expand_attention.hip", []),
@@ -104,7 +105,7 @@ INT_RESULT = {
     "mx_add_layer_norm32", "mx_expert_plan", "mx_expand_attention",
     "mx_latent_decode", "mx_keyval_attention", "mx_chunk_delta",
     "mx_chunk_gated", "mx_chunk_scan", "mx_token_scan", "mx_talk_mfma",
-    "mx_window_attention",
+    "mx_window_attention", "mx_attn_f32",
 }
 
 # entry points that return a 64-bit count

@@ -1125,3 +1125,69 @@ def test_recurrence_spans_launches():
     assert forms(15, 1, cells, None) == (False, True, False)
     assert forms(512, 64, cells, (8, 8)) == (False, True, True)
     assert forms(46, 2, cells, (30, -1)) == (True, False, True)
+
+
+@pytest.mark.parametrize("H,G,D,DV,chunk,window,keep,softcap", [
+    (32, 8, 128, 128, 0, 90, 4, 0.0), (32, 8, 64, 64, 0, 0, 0, 30.0),
+    (6, 2, 96, 80, 40, 0, 3, 0.0), (16, 1, 16, 4, 0, 33, 20, 0.0),
+    (3, 3, 112, 128, 0, 0, 0, 0.0)])
+@pytest.mark.parametrize("variant,splits", [(13, 1), (13, 3), (14, 1),
+                                            (14, 4)])
+def test_attention_fp32(H, G, D, DV, chunk, window, keep, softcap, variant,
+                        splits):
+    """The fp32 matrix-core kernel: portions that cross its row groups, rows of
+    several sequences in one group, key counts around its 16-key tiles, shares
+    without a key; a value that is no number and an infinite one, which only the
+    rows that see them may show."""
+    g = torch.Generator().manual_seed(14)
+    bs, L = 16, 150
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.float32, g, 3)
+    ts, tp = [], []
+    for s, a, b in ((0, 0, 35), (1, 60, 66), (2, 31, 34), (1, 95, 98),
+                    (0, 127, 130), (2, 149, 150), (2, 0, 1)):
+        ts += [s] * (b - a)
+        tp += list(range(a, b))
+    T = len(ts)
+    q = torch.randn(T, H * D + 8, generator=g)
+    sinks = torch.randn(H, generator=g)
+    ts = torch.tensor(ts, dtype=torch.int32)
+    tp = torch.tensor(tp, dtype=torch.int32)
+
+    def run(kc, vc):
+        want = reference.talk_attention(
+            q[:, :H * D].reshape(T, H, D), kc, vc, tables, ts, tp, D ** -0.5,
+            chunk, window, True, None, keep, softcap, sinks)
+        out = torch.full((T, H * DV + 4), 7.0, device="cuda")
+        ops.talk_attention(
+            q.cuda()[:, :H * D], kc.cuda(), vc.cuda(), tables.cuda(),
+            ts.cuda(), tp.cuda(), D ** -0.5, H, chunk=chunk, window=window,
+            sink=True, softcap=softcap, variant=variant, keep_first=keep,
+            sink_vals=sinks.cuda(), out=out[:, :H * DV], splits=splits)
+        assert (out[:, H * DV:] == 7.0).all()
+        return out[:, :H * DV].cpu().reshape(T, H, DV), want
+
+    got, want = run(kc, vc)
+    # sums of up to 150 and 128 roundings of 2^-24, scores of up to 5 before exp
+    assert _rel(got, want) < 3e-6
+    vc[tables[0, 128 // bs], 0, 128 % bs, 1] = float("nan")
+    vc[tables[2, 32 // bs], 0, 32 % bs, 2] = float("inf")
+    got, want = run(kc, vc)
+    fin = torch.isfinite(want)
+    assert torch.equal(fin, torch.isfinite(got))
+    assert _rel(got[fin], want[fin]) < 3e-6
+
+
+def test_attention_fp32_wide():
+    """32 columns a wave, which prompts of some length take."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    H, G, D, bs, T = 32, 8, 128, 16, 271
+    kc, vc = (torch.randn(20, G, bs, D, generator=g, device="cuda")
+              for _ in range(2))
+    tables = torch.randperm(20, generator=g, device="cuda").int()[None]
+    q = torch.randn(T, H * D, generator=g, device="cuda")
+    tp = torch.arange(T, dtype=torch.int32, device="cuda") + 20
+    ts = torch.zeros_like(tp)
+    for kw in (dict(window=100, keep_first=5), dict(softcap=20.0)):
+        want, got = (ops.talk_attention(q, kc, vc, tables, ts, tp, D ** -0.5,
+                                        H, variant=v, **kw) for v in (2, 13))
+        assert _rel(got, want) < 3e-6
