@@ -760,6 +760,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     rows of whole 16-byte vectors up to 128 wide take a portion and a token
     kernel of their own (variants 0 and 3; 11 and 12 insist on them), and so do
     fp32 rows of widths in steps of 16 up to 128 (13 and 14 insist on it).
+    Single tokens with a head mix over 32 heads of width 64 or 128 have one as
+    well (variant 3; 15 insists on it).
     Returns [T, H*DV]."""
     NB, G, BS, D = k_cache.shape
     VR = v_cache.shape[3]
@@ -934,6 +936,32 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if variant in (13, 14):
         raise RuntimeError(
             "talk_attention: shape or dtype outside the fp32 kernel")
+    # a head mix over single tokens
+    if (variant in (3, 15) and talk is not None and not extra and pool is None
+            and keep_first == 0):
+        keys = block_tables.shape[1] * BS
+        if window > 0:
+            keys = min(keys, window)
+        if chunk > 0:
+            keys = min(keys, chunk)
+        # one workgroup a CU (bf16 64 tokens of up to 2250 keys in 1 / 2 / 4 / 8
+        # shares 215 / 120 / 78 / 86 us), 48 keys each at least
+        shares = splits if splits > 0 else max(
+            1, min(16, 256 // T, keys // 48))
+        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
+                            device=q.device) if shares > 1 else None)
+        rc = _mx().mx_talk_token(
+            _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
+            _p(v_cache), _p(block_tables), block_tables.shape[1],
+            _p(token_seq), _p(token_pos), _p(talk), T, H, G, D, DV, BS,
+            _f(scale), int(chunk), int(window), int(bool(sink)),
+            _f(softcap), _p(sink_vals), int(VR), _mx_dtype(q.dtype),
+            int(shares), _p(part), _stream())
+        if rc == 0:
+            return out
+    if variant == 15:
+        raise RuntimeError(
+            "talk_attention: shape or dtype outside the head-mix token kernel")
     if variant not in (3, 4, 5, 6):
         splits = 1
     elif splits <= 0:

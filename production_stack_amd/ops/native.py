@@ -10,8 +10,8 @@ shape checks live in the Python wrappers
 
 Groups (one shared library each):
   core    resid32, norm_conv, mixer_prep, talk_attention, talk_mfma,
-          window_attention, attn_f32, mfma_attention, expand_attention, latent_decode, keyval_attention,
-          moe_route, moe_group, mingru_scan -> _mixops.so
+          talk_token, window_attention, attn_f32, mfma_attention,
+          expand_attention, latent_decode, keyval_attention, moe_route, moe_group, mingru_scan -> _mixops.so
   delta   delta_rule                        -> _mixops_delta.so
   gdelta  gated_delta                       -> _mixops_gdelta.so
   scan    linear_scan                       -> _mixops_scan.so
@@ -52,6 +52,7 @@ GROUPS = {
         ("talk_mfma.hip", []),
         ("window_attention.hip", []),
         ("attn_f32.hip", []),
+        ("talk_token.hip", []),
         ("mixer_prep.hip", []),
         ("mfma_attention.hip", []),
         ("expand_attention.hip", []),
@@ -105,7 +106,7 @@ INT_RESULT = {
     "mx_add_layer_norm32", "mx_expert_plan", "mx_expand_attention",
     "mx_latent_decode", "mx_keyval_attention", "mx_chunk_delta",
     "mx_chunk_gated", "mx_chunk_scan", "mx_token_scan", "mx_talk_mfma",
-    "mx_window_attention", "mx_attn_f32",
+    "mx_window_attention", "mx_attn_f32", "mx_talk_token",
 }
 
 # entry points that return a 64-bit count

@@ -1191,3 +1191,51 @@ def test_attention_fp32_wide():
         want, got = (ops.talk_attention(q, kc, vc, tables, ts, tp, D ** -0.5,
                                         H, variant=v, **kw) for v in (2, 13))
         assert _rel(got, want) < 3e-6
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("G,D,DV,chunk,window,softcap,learned", [
+    (8, 128, 128, 64, 0, 0.0, False), (8, 64, 64, 0, 50, 0.0, True),
+    (2, 128, 64, 0, 0, 9.0, True), (1, 64, 128, 33, 20, 0.0, False)])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_talk_attention_tokens(G, D, DV, chunk, window, softcap, learned,
+                               splits, dtype):
+    """The head-mix kernel of single tokens: key counts around its 16-key tiles
+    and a workgroup's 64, shares without a key; a value that is no number and an
+    infinite one, which only the heads and rows that see them may show."""
+    g = torch.Generator().manual_seed(15)
+    H, bs, L = 32, 16, 330
+    kc, vc, tables = _paged(L, G, D, DV, bs, dtype, g, 3)
+    tp = torch.tensor([0, 14, 15, 16, 62, 63, 64, 130, 191, 192, 193, 329],
+                      dtype=torch.int32)
+    T = len(tp)
+    ts = (torch.arange(T) % 3).int()
+    q = torch.randn(T, H * D + 8, generator=g).to(dtype)
+    talk = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)
+    sinks = torch.randn(H, generator=g) if learned else None
+
+    def run(kc, vc):
+        want = reference.talk_attention(
+            q[:, :H * D].float().reshape(T, H, D), kc.float(), vc.float(),
+            tables, ts, tp, D ** -0.5, chunk, window, True, talk, 0, softcap,
+            sinks)
+        out = torch.full((T, H * DV + 4), 7.0, dtype=dtype, device="cuda")
+        ops.talk_attention(
+            q.cuda()[:, :H * D], kc.cuda(), vc.cuda(), tables.cuda(),
+            ts.cuda(), tp.cuda(), D ** -0.5, H, chunk=chunk, window=window,
+            sink=True, talk=talk.cuda(), softcap=softcap, variant=15,
+            sink_vals=sinks.cuda() if learned else None,
+            out=out[:, :H * DV], splits=splits)
+        assert (out[:, H * DV:] == 7.0).all()
+        return out[:, :H * DV].cpu().reshape(T, H, DV), want
+
+    got, want = run(kc, vc)
+    # fp32 sums of up to 330 and 128 terms, or the bf16 rounding of the result
+    bound = 3e-3 if dtype == torch.bfloat16 else 4e-6
+    assert _rel(got, want) < bound
+    vc[tables[1, 129 // bs], 0, 129 % bs, 1] = float("nan")
+    vc[tables[2, 191 // bs], G - 1, 191 % bs, 2] = float("inf")
+    got, want = run(kc, vc)
+    fin = torch.isfinite(want)
+    assert torch.equal(fin, torch.isfinite(got))
+    assert _rel(got[fin], want[fin]) < bound
