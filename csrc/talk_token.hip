@@ -57,6 +57,8 @@ struct TtArgs {
 
 #define TT_H 32
 
+PS_DEV bool tt_odd(float x) { return !(fabsf(x) < INFINITY); }
+
 // How far a score may be above the one that set the reference that weights are
 // relative to, before it moves; the reference is as much above it, so that no weight
 // is above 1. Moving it is a product per sum.
@@ -349,6 +351,296 @@ __global__ __launch_bounds__(512, 2) void talk_token_kernel(TtArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Prompt portions in fp32: as above, four consecutive rows a workgroup, whose eight
+// waves take one tile of 16 keys at a time. A KV head's four heads of four rows are 16
+// rows of one product, one KV head a wave, so that no part of it is idle; the way
+// through LDS hands every wave the scores of its rows (one, or two with half of the
+// value entries at widths of 128) as left operands of the mix. Queries stay in LDS.
+//
+// A tile takes 5100 cycles of a SIMD's matrix unit (8192 of 20000 for the scores, 2048
+// for the mix, 8192 for the output, over four SIMDs) and 64 KB of keys and of values
+// from the L2 each. us, by the vector kernel of talk_attention.hip -> this one, heads of
+// 128: 149 rows behind 817 keys 4390 -> 71, 1000 rows 4520 -> 188 (a third of the fp32
+// matrix rate: the phases between two barriers are the same in all waves), 80 rows
+// behind 334 1800 -> 39; of 64 2460 -> 47, 2550 -> 121, 1010 -> 27.
+// Hidden keys of a row have weights of zero, which values that are not finite would
+// carry into its sums; where sums are not finite the walk goes again with those kept
+// out of the products and added to the rows that see them.
+template <int D, int DV>
+__global__ __launch_bounds__(512, 2) void talk_rows_f32_kernel(TtArgs a) {
+  constexpr int KF = D / 16, P = 4;
+  constexpr int SP = DV / 64;          // waves that share a value row
+  constexpr int TW = SP;               // rows of a wave
+  constexpr int NE = 16, VF = 4;
+  // values when the keys are read, keys when half of the values are: with both a
+  // tile ahead registers spill
+  constexpr bool LATE = TW == 2;
+  constexpr int PQ = D + 4, TQ = TT_H * PQ + 16;
+  extern __shared__ __align__(16) float s_q[];  // [4][TQ]
+  __shared__ __align__(16) kv_f32x4 s_sc[2][4][2][64];
+  __shared__ int s_seq[4], s_pos[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hf = wave >> 2, sp = wave % SP, r0 = wave % 4 / SP * TW;
+  const int g = lane >> 4, n = lane & 15;
+  // rows that see the most keys first
+  const int ks = blockIdx.x % a.KS;
+  const int tok0 = ((a.T + 3) / 4 - 1 - blockIdx.x / a.KS) * 4;
+  const int ntok = min(4, a.T - tok0);
+  const int G = a.G, BS = a.BS, rep = TT_H / G;
+  const float* kc = (const float*)a.kc;
+  const float* vc = (const float*)a.vc;
+  if (tid < 4) {
+    const int t = tok0 + min(tid, ntok - 1);
+    s_seq[tid] = a.token_seq[t];
+    s_pos[tid] = a.token_pos[t];
+  }
+  for (int i = tid; i < 4 * TT_H * D / 4; i += 512) {
+    const int r = i / (TT_H * D / 4), c = i % (TT_H * D / 4);
+    *(float4*)(s_q + r * TQ + c / (D / 4) * PQ + c % (D / 4) * 4) =
+        *(const float4*)((const float*)a.q +
+                         (size_t)(tok0 + min(r, ntok - 1)) * a.ldq + c * 4);
+  }
+  // left operands: row n is head 4 wave + n % 4 of token n / 4
+  const float* sq = s_q + (n >> 2) * TQ + (4 * wave + (n & 3)) * PQ + g * P;
+  float tb[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      tb[h][i] =
+          a.talk[(16 * hf + n) * TT_H + 16 * h + 4 * g + i] * a.scale;
+  __syncthreads();
+
+  auto low = [&](int p) {
+    int lo = 0;
+    if (a.chunk > 0) lo = p / a.chunk * a.chunk;
+    if (a.window > 0) lo = max(lo, p - a.window + 1);
+    return lo;
+  };
+  const int khead = 4 * wave / rep * BS;
+  const int vhead = (16 * hf + (n & 12)) / rep * BS;
+  int my_pos[TW], my_lo[TW];
+#pragma unroll
+  for (int q = 0; q < TW; ++q) {
+    my_pos[q] = __builtin_amdgcn_readfirstlane(s_pos[r0 + q]);
+    my_lo[q] = low(my_pos[q]);
+  }
+  float m[TW], l[TW];
+  kv_f32x4 acc[TW][NE];
+  bool careful = false;
+#pragma unroll 1
+  for (;;) {
+#pragma unroll
+    for (int q = 0; q < TW; ++q) {
+      m[q] = PS_NEG_INF;
+      l[q] = 0.f;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) acc[q][e] = kv_f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    int turn = 0, rs = 0;
+    while (rs < ntok) {
+      // rows rs .. re - 1 continue one sequence
+      int re = rs + 1;
+      while (re < ntok && s_seq[re] == s_seq[rs] &&
+             s_pos[re] == s_pos[re - 1] + 1)
+        ++re;
+      const int* table = a.block_tables + (size_t)s_seq[rs] * a.max_blocks;
+      const int kmin = low(s_pos[rs]), kmax = s_pos[re - 1];
+      const int nt = (kmax - kmin) / 16 + 1;
+      auto key_of = [&](int t) { return min(kmin + t * 16 + n, kmax); };
+      auto row_of = [&](int t, int page) {
+        return page * G * BS + key_of(t) % BS;
+      };
+      float4 kb[KF], vb[4][VF];
+      auto fetch_k = [&](int row) {
+        const float* p = kc + ((int64_t)row + khead) * D + g * P;
+#pragma unroll
+        for (int f = 0; f < KF; ++f) kb[f] = *(const float4*)(p + 4 * f * P);
+      };
+      auto fetch_v = [&](int i, int row) {
+        const float* p =
+            vc + ((int64_t)__shfl(row, 4 * g + i, 64) + vhead) * a.vr + 64 * sp +
+            (n & 3) * P;
+#pragma unroll
+        for (int f = 0; f < VF; ++f)
+          vb[i][f] = *(const float4*)(p + 4 * f * P);
+      };
+      // pages two tiles ahead; tiles past the last repeat it, unread
+      int tn = min(ks, nt - 1);
+      int row = row_of(tn, table[key_of(tn) / BS]);
+      tn = min(ks + a.KS, nt - 1);
+      int page = table[key_of(tn) / BS];
+      fetch_k(row);
+      if constexpr (!LATE)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fetch_v(i, row);
+      for (int t = ks; t < nt; t += a.KS) {
+        const int next = row_of(tn, page);
+        tn = min(t + 2 * a.KS, nt - 1);
+        page = table[key_of(tn) / BS];
+        kv_f32x4 st[4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) st[f] = kv_f32x4{0.f, 0.f, 0.f, 0.f};
+        // sums of every fourth piece: shorter chains of roundings
+#pragma unroll
+        for (int f = 0; f < KF; ++f) {
+          const float4 q = *(const float4*)(sq + 4 * f * P);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            st[f & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                (&q.x)[e], (&kb[f].x)[e], st[f & 3], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // no load earlier, it would spill
+        if constexpr (LATE) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) fetch_v(i, row);
+        } else {
+          fetch_k(next);
+        }
+        // heads 4 wave + i of token g: group wave % 4 of its half's operand
+        s_sc[turn][g][hf][16 * (wave & 3) + n] =
+            (st[0] + st[1]) + (st[2] + st[3]);
+        __syncthreads();
+        const int j0 = kmin + t * 16 + 4 * g;
+        float x[TW][4];
+#pragma unroll
+        for (int q = 0; q < TW; ++q) {
+          const int r = r0 + q;
+          const kv_f32x4 s0 = s_sc[turn][r][0][lane];
+          const kv_f32x4 s1 = s_sc[turn][r][1][lane];
+          kv_f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            y = __builtin_amdgcn_mfma_f32_16x16x4f32(s0[i], tb[0][i], y, 0, 0,
+                                                     0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            y = __builtin_amdgcn_mfma_f32_16x16x4f32(s1[i], tb[1][i], y, 0, 0,
+                                                     0);
+          // keys 4 g + i of head 16 hf + n
+          const int hi = r >= rs && r < re ? my_pos[q] : -1;
+          float mx = PS_NEG_INF;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float v = y[i];
+            if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
+            // no number counts as hidden
+            x[q][i] = j0 + i >= my_lo[q] && j0 + i <= hi && v == v ? v : -INFINITY;
+            mx = fmaxf(mx, x[q][i]);
+          }
+          mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+          mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+          if (__any(mx > m[q])) {
+            const float mn = mx > m[q] ? mx + TT_FAR : m[q];
+            const float al = expf(m[q] - mn);
+            m[q] = mn;
+            l[q] *= al;
+            float f[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) f[i] = tt_quad(al, i);
+#pragma unroll
+            for (int e = 0; e < NE; ++e)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) acc[q][e][i] *= f[i];
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            x[q][i] = expf(x[q][i] - m[q]);
+            l[q] += x[q][i];
+          }
+        }
+        turn ^= 1;
+        if (careful) {
+#pragma unroll
+          for (int q = 0; q < TW; ++q) {
+            const int r = r0 + q;
+            const int hi = r >= rs && r < re ? my_pos[q] : -1;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int e = 0; e < NE; ++e) {
+                const float v = (&vb[i][e / P].x)[e % P];
+                if (tt_odd(v) && j0 + i >= my_lo[q] && j0 + i <= hi)
+                  acc[q][e] += v;
+              }
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+              float& v = (&vb[i][e / P].x)[e % P];
+              if (tt_odd(v)) v = 0.f;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+          for (int e = 0; e < NE; ++e)
+#pragma unroll
+            for (int q = 0; q < TW; ++q)
+              acc[q][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(
+                  x[q][i], (&vb[i][e / P].x)[e % P], acc[q][e], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (!LATE)
+            fetch_v(i, next);
+          else if (i == 1)
+            fetch_k(next);
+        }
+        row = next;
+      }
+      rs = re;
+    }
+    bool odd = false;
+#pragma unroll
+    for (int q = 0; q < TW; ++q)
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) odd |= tt_odd(acc[q][e][i]);
+    if (!__syncthreads_or(odd) || careful) break;
+    careful = true;
+  }
+
+  // a lane group has the sums of one of four heads
+  const int own = (n & 12) + (g & 1) * 2 + g / 2, head = 16 * hf + own;
+  const float sv = a.sink_vals != nullptr ? a.sink_vals[head] : 0.f;
+#pragma unroll
+  for (int q = 0; q < TW; ++q) {
+    float lt = l[q];
+    lt += __shfl_xor(lt, 16, 64);
+    lt += __shfl_xor(lt, 32, 64);
+    lt = __shfl(lt, own, 64);
+    float mt = __shfl(m[q], own, 64), f = 1.f;
+    if (a.sink && ks == 0) {  // the sink is share 0's
+      const float mn = fmaxf(mt, sv);
+      f = expf(mt - mn);
+      lt = lt * f + expf(sv - mn);
+      mt = mn;
+    }
+    const int r = r0 + q, tok = tok0 + r;
+    const int at = 64 * sp + (n & 3) * P;
+    float* rec = a.part + (((size_t)tok * a.KS + ks) * TT_H + head) * (DV + 4);
+    if (a.KS > 1 && at == 0 && r < ntok) {
+      rec[0] = mt;
+      rec[1] = lt;
+    }
+    float* dst = a.KS > 1 ? rec + 4
+                          : (float*)a.out + (size_t)tok * a.ldout + head * DV;
+    if (a.KS == 1) f /= lt;
+#pragma unroll
+    for (int e = 0; e < NE; e += 4) {
+      float o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = tt_gather(acc[q][e + i]) * f;
+      if (r < ntok)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dst[at + e * 4 + i] = o[i];
+    }
+  }
+}
+
 extern "C" void mx_attn_records(void* out, int ldout, const void* part, int T_,
                                 int H, int DV, int KS, int dtype,
                                 void* stream);
@@ -404,5 +696,50 @@ extern "C" int mx_talk_token(
   })
   if (rc == 0 && a.KS > 1)
     mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, dtype, stream);
+  return rc;
+}
+
+template <int D, int DV>
+static int tt_launch_rows(const TtArgs& a, hipStream_t stream) {
+  const size_t lds = (size_t)4 * (TT_H * (D + 4) + 16) * 4;
+  if (hipFuncSetAttribute((const void*)talk_rows_f32_kernel<D, DV>,
+                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return 1;
+  }
+  hipLaunchKernelGGL((talk_rows_f32_kernel<D, DV>), dim3((a.T + 3) / 4 * a.KS),
+                     dim3(512), lds, stream, a);
+  return 0;
+}
+
+// The same for prompt portions, fp32.
+extern "C" int mx_talk_rows_f32(
+    void* out, int ldout, const void* q, int ldq, const void* kc,
+    const void* vc, const void* block_tables, int max_blocks,
+    const void* token_seq, const void* token_pos, const void* talk, int T_,
+    int H, int G, int D, int DV, int BS, float scale, int chunk, int window,
+    int sink, float softcap, const void* sink_vals, int vrow, int splits,
+    void* scratch, void* stream) {
+  if (T_ <= 0) return 0;
+  if (H != TT_H || G < 1 || H % G || H / G % 4 || BS < 1) return 1;
+  if ((D != 64 && D != 128) || (DV != 64 && DV != 128)) return 1;
+  if (ldq % 4 || vrow % 4 || vrow < DV ||
+      (((size_t)q | (size_t)kc | (size_t)vc) & 15))
+    return 1;
+  const TtArgs a = {out, ldout, q, ldq, kc, vc, vrow,
+                    (const int*)block_tables, max_blocks,
+                    (const int*)token_seq, (const int*)token_pos,
+                    (const float*)talk, T_, G, BS, scale, chunk, window, sink,
+                    softcap > 0.f ? softcap : 0.f, (const float*)sink_vals,
+                    splits > 1 && scratch != nullptr ? splits : 1,
+                    (float*)scratch};
+  hipStream_t s = (hipStream_t)stream;
+  const int rc = D == 64 ? (DV == 64 ? tt_launch_rows<64, 64>(a, s)
+                                     : tt_launch_rows<64, 128>(a, s))
+                         : (DV == 64 ? tt_launch_rows<128, 64>(a, s)
+                                     : tt_launch_rows<128, 128>(a, s));
+  if (rc == 0 && a.KS > 1)
+    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, MX_F32, stream);
   return rc;
 }

@@ -761,7 +761,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     kernel of their own (variants 0 and 3; 11 and 12 insist on them), and so do
     fp32 rows of widths in steps of 16 up to 128 (13 and 14 insist on it).
     Single tokens with a head mix over 32 heads of width 64 or 128 have one as
-    well (variant 3; 15 insists on it).
+    well (variant 3; 15 insists on it), and so have fp32 portions with such a
+    mix (variant 0; 16 insists on it).
     Returns [T, H*DV]."""
     NB, G, BS, D = k_cache.shape
     VR = v_cache.shape[3]
@@ -936,6 +937,36 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if variant in (13, 14):
         raise RuntimeError(
             "talk_attention: shape or dtype outside the fp32 kernel")
+    # a head mix over prompt portions in fp32
+    if (variant in (0, 16) and talk is not None and not extra and pool is None
+            and keep_first == 0 and q.dtype == torch.float32):
+        keys = block_tables.shape[1] * BS
+        if window > 0:
+            keys = min(keys, window)
+        if chunk > 0:
+            keys = min(keys, chunk)
+        # Workgroups of a group's keys: one round of the CUs where few rows leave
+        # the groups alike, two where groups see a few keys or all (128, us: 149
+        # rows behind 817 keys in 1 / 6 / 12 shares 277 / 71 / 81; 254, of which 85
+        # behind 1800, in 1 / 4 / 8 528 / 159 / 111; 1000 in 1 / 2 / 4 286 / 188 /
+        # 208; 70 in 1 / 4 33 / 25), a tile of keys each at least
+        groups = (T + 3) // 4
+        shares = splits if splits > 0 else max(1, min(
+            16, (256 if groups <= 48 else 512) // groups, keys // 16))
+        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
+                            device=q.device) if shares > 1 else None)
+        rc = _mx().mx_talk_rows_f32(
+            _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
+            _p(v_cache), _p(block_tables), block_tables.shape[1],
+            _p(token_seq), _p(token_pos), _p(talk), T, H, G, D, DV, BS,
+            _f(scale), int(chunk), int(window), int(bool(sink)),
+            _f(softcap), _p(sink_vals), int(VR), int(shares), _p(part),
+            _stream())
+        if rc == 0:
+            return out
+    if variant == 16:
+        raise RuntimeError(
+            "talk_attention: shape or dtype outside the fp32 head-mix kernel")
     # a head mix over single tokens
     if (variant in (3, 15) and talk is not None and not extra and pool is None
             and keep_first == 0):

@@ -107,6 +107,7 @@ INT_RESULT = {
     "mx_latent_decode", "mx_keyval_attention", "mx_chunk_delta",
     "mx_chunk_gated", "mx_chunk_scan", "mx_token_scan", "mx_talk_mfma",
     "mx_window_attention", "mx_attn_f32", "mx_talk_token",
+    "mx_talk_rows_f32",
 }
 
 # entry points that return a 64-bit count

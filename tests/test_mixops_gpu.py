@@ -1239,3 +1239,53 @@ def test_talk_attention_tokens(G, D, DV, chunk, window, softcap, learned,
     fin = torch.isfinite(want)
     assert torch.equal(fin, torch.isfinite(got))
     assert _rel(got[fin], want[fin]) < bound
+
+
+@pytest.mark.parametrize("G,D,DV,chunk,window,softcap,learned", [
+    (8, 128, 128, 64, 0, 0.0, False), (8, 64, 64, 0, 50, 0.0, True),
+    (2, 128, 64, 0, 0, 9.0, True), (1, 64, 128, 33, 20, 0.0, False)])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_talk_attention_fp32_portions(G, D, DV, chunk, window, softcap,
+                                      learned, splits):
+    """The fp32 head-mix kernel of portions: rows that cross its groups of four,
+    several sequences in one group, key counts around its 16-key tiles, shares
+    without a key; a value that is no number and an infinite one, which only the
+    heads and rows that see them may show."""
+    g = torch.Generator().manual_seed(16)
+    H, bs, L = 32, 16, 150
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.float32, g, 3)
+    ts, tp = [], []
+    for s, a, b in ((0, 0, 35), (1, 60, 66), (2, 31, 34), (1, 95, 98),
+                    (0, 127, 130), (2, 149, 150), (2, 0, 1)):
+        ts += [s] * (b - a)
+        tp += list(range(a, b))
+    T = len(ts)
+    q = torch.randn(T, H * D + 8, generator=g)
+    talk = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)
+    sinks = torch.randn(H, generator=g) if learned else None
+    ts = torch.tensor(ts, dtype=torch.int32)
+    tp = torch.tensor(tp, dtype=torch.int32)
+
+    def run(kc, vc):
+        want = reference.talk_attention(
+            q[:, :H * D].reshape(T, H, D), kc, vc, tables, ts, tp, D ** -0.5,
+            chunk, window, True, talk, 0, softcap, sinks)
+        out = torch.full((T, H * DV + 4), 7.0, device="cuda")
+        ops.talk_attention(
+            q.cuda()[:, :H * D], kc.cuda(), vc.cuda(), tables.cuda(),
+            ts.cuda(), tp.cuda(), D ** -0.5, H, chunk=chunk, window=window,
+            sink=True, talk=talk.cuda(), softcap=softcap, variant=16,
+            sink_vals=sinks.cuda() if learned else None,
+            out=out[:, :H * DV], splits=splits)
+        assert (out[:, H * DV:] == 7.0).all()
+        return out[:, :H * DV].cpu().reshape(T, H, DV), want
+
+    got, want = run(kc, vc)
+    # fp32 sums of up to 150 and 128 terms
+    assert _rel(got, want) < 4e-6
+    vc[tables[0, 128 // bs], 0, 128 % bs, 1] = float("nan")
+    vc[tables[2, 32 // bs], G - 1, 32 % bs, 2] = float("inf")
+    got, want = run(kc, vc)
+    fin = torch.isfinite(want)
+    assert torch.equal(fin, torch.isfinite(got))
+    assert _rel(got[fin], want[fin]) < 4e-6
