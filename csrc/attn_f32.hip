@@ -349,13 +349,15 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
         rec[0] = mh;
         rec[1] = lt;
       }
-      *(float4*)(rec + AF_HEAD + d) = make_float4(o[0], o[1], o[2], o[3]);
+      if (lt != 0.f)  // else no key of this share: no sums
+        *(float4*)(rec + AF_HEAD + d) = make_float4(o[0], o[1], o[2], o[3]);
     }
   }
 }
 
-// Merge of `KS` partial records of every (token, head): 256 threads of four
-// entries each.
+// Merge of `KS` (at most AF_KS) partial records of every (token, head): 256 threads
+// of four entries each. Shares without a key have a denominator of 0 and no sums.
+#define AF_KS 16
 template <typename T>
 __global__ __launch_bounds__(256) void attn_records_kernel(
     T* __restrict__ out, int ldout, const float* __restrict__ part, int H,
@@ -366,20 +368,25 @@ __global__ __launch_bounds__(256) void attn_records_kernel(
   const float* rec =
       part + ((size_t)blockIdx.x * KS * H + h) * (DV + AF_HEAD);
   const size_t step = (size_t)H * (DV + AF_HEAD);
-  float mh = PS_NEG_INF, l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int s = 0; s < KS; ++s) {
-    const float2 ml = *(const float2*)(rec + s * step);
+  float2 ml[AF_KS];
+  float mh = PS_NEG_INF;
+#pragma unroll
+  for (int s = 0; s < AF_KS; ++s) {
+    ml[s] = s < KS ? *(const float2*)(rec + s * step)
+                   : make_float2(PS_NEG_INF, 0.f);
+    if (ml[s].y != 0.f) mh = fmaxf(mh, ml[s].x);
+  }
+  float l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < AF_KS; ++s) {
+    if (ml[s].y == 0.f) continue;
     const float4 v = *(const float4*)(rec + s * step + AF_HEAD + d);
-    if (ml.x == PS_NEG_INF && ml.y == 0.f) continue;  // an empty share
-    const float mn = fmaxf(mh, ml.x);
-    const float was = expf(mh - mn), f = expf(ml.x - mn);
-    mh = mn;
-    l = l * was + ml.y * f;
-    o[0] = o[0] * was + v.x * f;
-    o[1] = o[1] * was + v.y * f;
-    o[2] = o[2] * was + v.z * f;
-    o[3] = o[3] * was + v.w * f;
+    const float f = expf(ml[s].x - mh);
+    l += ml[s].y * f;
+    o[0] += v.x * f;
+    o[1] += v.y * f;
+    o[2] += v.z * f;
+    o[3] += v.w * f;
   }
   const float f = 1.0f / l;
   T* dst = out + (size_t)blockIdx.x * ldout + h * DV + d;
@@ -387,7 +394,7 @@ __global__ __launch_bounds__(256) void attn_records_kernel(
   for (int e = 0; e < 4; ++e) MxElem<T>::st(dst + e, o[e] * f);
 }
 
-// Merge pass over records [T, KS, H, DV + 4] (DV in steps of 4).
+// Merge pass over records [T, KS, H, DV + 4] (DV in steps of 4, KS up to 16).
 extern "C" void mx_attn_records(void* out, int ldout, const void* part, int T_,
                                 int H, int DV, int KS, int dtype,
                                 void* stream) {
@@ -430,6 +437,7 @@ extern "C" int mx_attn_f32(void* out, int ldout, const void* q, int ldq,
                            int rows, int splits, void* scratch,
                            void* stream) {
   if (T_ <= 0) return 0;
+  if (splits > AF_KS) return 1;
   if (G < 1 || H < 1 || H % G || H / G > 16 || BS < 1 || D < 16 || D % 16 ||
       D > 128 || DV < 4 || DV % 4 || DV > 128 || ldq % 4 || vrow % 4 ||
       vrow < DV || (((size_t)q | (size_t)kc | (size_t)vc) & 15))

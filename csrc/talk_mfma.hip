@@ -36,6 +36,9 @@
 // on the vector pipe, whose kernel remains for fp32 and other shapes). Sixteen waves
 // spill at widths of 128 and are no faster at 64 (284 us, 272 with eight); orders of
 // the four parts that differ between the two waves of a SIMD spill as well.
+// Few rows behind many keys are a chain of tiles (3.5 us each) on a few CUs: there
+// several workgroups share a block's keys, and mx_attn_records merges what they have (70
+// rows behind 2000 keys 276 us whole, 50 in 16 shares).
 #include "attn_common.h"
 #include "scan_common.h"
 
@@ -74,6 +77,8 @@ struct TmArgs {
   int chunk, window, sink;
   float softcap;
   const float* sink_vals;
+  int KS;       // workgroups that share a block's keys
+  float* part;  // [T, KS, 32, DV + 4]: maximum, denominator, sums
 };
 
 // A bf16 entry that is an infinity or no number.
@@ -144,8 +149,9 @@ PS_DEV int tm_at(int head, int row, int unit, int bit) {
   return (head * 16 + row) * 16 + 2 * (unit ^ (row >> 2 | (bit & 1) << 2));
 }
 
-// ND = D / 32, NV = DV / 16; CAP: with a score cap
-template <int ND, int NV, bool CAP>
+// ND = D / 32, NV = DV / 16; CAP: with a score cap; PART: several workgroups to a
+// block's keys (as a choice at run time whole blocks took 1 to 2 % longer)
+template <int ND, int NV, bool CAP, bool PART>
 __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   constexpr int D = ND * 32, DV = NV * 16;
   constexpr int PV = DV + 8;          // LDS pitch of a value row
@@ -212,13 +218,14 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     // the product may be past the largest float
-    m[i] = a.sink ? (a.sink_vals != nullptr
+    m[i] = a.sink && (!PART || blockIdx.y == 0)  // the sink is share 0's
+               ? (a.sink_vals != nullptr
                          ? fminf(fmaxf(a.sink_vals[h0 + i] * KV_LOG2E,
                                        PS_NEG_INF),
                                  -KV_LOW)
                          : 0.f) + TM_FAR
                   : PS_NEG_INF;
-    l[i] = a.sink && wave == 0 ? __builtin_amdgcn_exp2f(-TM_FAR) : 0.f;
+    l[i] = a.sink && (!PART || blockIdx.y == 0) && wave == 0 ? __builtin_amdgcn_exp2f(-TM_FAR) : 0.f;
   }
   ck_f32x4 acc[2][NV];
 #pragma unroll
@@ -244,7 +251,17 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
       if (a.window > 0) lo = max(lo, p - a.window + 1);
       return lo;
     };
-    const int kmin = low(s_pos[rs]), kmax = s_pos[re - 1];
+    int kmin = low(s_pos[rs]), kmax = s_pos[re - 1];
+    if constexpr (PART) {  // this share's tiles
+      const int all = (kmax - kmin) / TM_KT + 1, ks = blockIdx.y;
+      const int t0 = all * ks / a.KS, t1 = all * (ks + 1) / a.KS;
+      if (t0 == t1) {
+        rs = re;
+        continue;
+      }
+      kmax = min(kmax, kmin + t1 * TM_KT - 1);
+      kmin += t0 * TM_KT;
+    }
     const int nt = (kmax - kmin) / TM_KT + 1;
     const int my_lo = low(pos), my_hi = mine ? pos : -1;
     // cache row, less its KV head's, of key (lane & 31) of a tile; keys past
@@ -518,7 +535,10 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
 
   // denominators: eight key shares per (head, row)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sPM[wave * 256 + (4 * g + i) * 16 + n] = l[i];
+  for (int i = 0; i < 4; ++i) {
+    sPM[wave * 256 + (4 * g + i) * 16 + n] = l[i];
+    if (PART && wave == 0) sAL[(4 * g + i) * 16 + n] = m[i];
+  }
   __syncthreads();
   if (n >= ntok) return;
   unsigned short* o = a.out + (size_t)(tok0 + n) * a.ldout +
@@ -529,6 +549,21 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
     float lt = 0.f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) lt += sPM[k * 256 + (wave * 2 + h) * 16 + n];
+    if constexpr (PART) {
+      float* rec = a.part + (((size_t)(tok0 + n) * a.KS + blockIdx.y) * TM_H +
+                             16 * hb + wave * 2 + h) * (DV + 4);
+      if (g == 0) {
+        const float mt = sAL[(wave * 2 + h) * 16 + n];
+        rec[0] = lt != 0.f ? mt * 0.693147181f : PS_NEG_INF;
+        rec[1] = lt;
+      }
+      if (lt == 0.f) continue;  // no key of this share: no sums
+#pragma unroll
+      for (int c = 0; c < NV; ++c)
+        *(float4*)(rec + 4 + 16 * c + 4 * g) =
+            make_float4(acc[h][c][0], acc[h][c][1], acc[h][c][2], acc[h][c][3]);
+      continue;
+    }
     const float f = 1.0f / lt;
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
@@ -547,38 +582,47 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   }
 }
 
-template <int ND, int NV, bool CAP>
+template <int ND, int NV, bool CAP, bool PART>
 static int tm_launch_as(const TmArgs& a, hipStream_t stream) {
   const size_t lds = (size_t)(2 * TM_H * 256 + 3 * 16 * 256 + 9 * 256) * 4 +
                      (size_t)4 * TM_KT * (NV * 16 + 8) * 2;
-  if (hipFuncSetAttribute((const void*)talk_mfma_kernel<ND, NV, CAP>,
+  if (hipFuncSetAttribute((const void*)talk_mfma_kernel<ND, NV, CAP, PART>,
                           hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)lds) != hipSuccess) {
     (void)hipGetLastError();
     return 1;
   }
   // 16 workgroups for eight blocks of rows
-  hipLaunchKernelGGL((talk_mfma_kernel<ND, NV, CAP>),
-                     dim3((a.T + 127) / 128 * 16), dim3(512), lds, stream, a);
+  hipLaunchKernelGGL((talk_mfma_kernel<ND, NV, CAP, PART>),
+                     dim3((a.T + 127) / 128 * 16, a.KS), dim3(512), lds, stream, a);
   return 0;
 }
 
 template <int ND, int NV>
 static int tm_launch(const TmArgs& a, hipStream_t stream) {
-  return a.softcap > 0.f ? tm_launch_as<ND, NV, true>(a, stream)
-                         : tm_launch_as<ND, NV, false>(a, stream);
+  if (a.KS > 1)
+    return a.softcap > 0.f ? tm_launch_as<ND, NV, true, true>(a, stream)
+                           : tm_launch_as<ND, NV, false, true>(a, stream);
+  return a.softcap > 0.f ? tm_launch_as<ND, NV, true, false>(a, stream)
+                         : tm_launch_as<ND, NV, false, false>(a, stream);
 }
+
+extern "C" void mx_attn_records(void* out, int ldout, const void* part, int T_,
+                                int H, int DV, int KS, int dtype,
+                                void* stream);
 
 // Returns 0 when launched, 1 when the shape is outside this kernel: 32 heads
 // over at most 8 KV heads (a wave's four heads share one), widths 64 or 128,
-// rows on 16-byte borders.
+// rows on 16-byte borders. scratch fp32 [T, splits, 32, DV + 4] when splits > 1.
 extern "C" int mx_talk_mfma(
     void* out, int ldout, const void* q, int ldq, const void* kc,
     const void* vc, const void* block_tables, int max_blocks,
     const void* token_seq, const void* token_pos, const void* talk, int T_,
     int H, int G, int D, int DV, int BS, float scale, int chunk, int window,
-    int sink, float softcap, const void* sink_vals, int vrow, void* stream) {
+    int sink, float softcap, const void* sink_vals, int vrow, int splits,
+    void* scratch, void* stream) {
   if (T_ <= 0) return 0;
+  if (splits > 16) return 1;
   if (H != TM_H || G < 1 || H % G || H / G % 4) return 1;
   if ((D != 64 && D != 128) || (DV != 64 && DV != 128)) return 1;
   if (ldq % 8 || vrow % 8 || ((size_t)q | (size_t)kc | (size_t)vc) % 16)
@@ -587,9 +631,12 @@ extern "C" int mx_talk_mfma(
               (const unsigned short*)kc, (const unsigned short*)vc, vrow,
               (const int*)block_tables, max_blocks, (const int*)token_seq,
               (const int*)token_pos, (const float*)talk, T_, G, BS, scale,
-              chunk, window, sink, softcap, (const float*)sink_vals};
+              chunk, window, sink, softcap, (const float*)sink_vals,
+              splits > 1 && scratch != nullptr ? splits : 1, (float*)scratch};
   hipStream_t s = (hipStream_t)stream;
-  if (D == 64)
-    return DV == 64 ? tm_launch<2, 4>(a, s) : tm_launch<2, 8>(a, s);
-  return DV == 64 ? tm_launch<4, 4>(a, s) : tm_launch<4, 8>(a, s);
+  const int rc = D == 64 ? (DV == 64 ? tm_launch<2, 4>(a, s) : tm_launch<2, 8>(a, s))
+                         : (DV == 64 ? tm_launch<4, 4>(a, s) : tm_launch<4, 8>(a, s));
+  if (rc == 0 && a.KS > 1)
+    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, MX_BF16, stream);
+  return rc;
 }

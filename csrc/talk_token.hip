@@ -346,7 +346,8 @@ __global__ __launch_bounds__(512, 2) void talk_token_kernel(TtArgs a) {
         rec[0] = mh;
         rec[1] = lt;
       }
-      *(float4*)(rec + 4 + d) = make_float4(o[0], o[1], o[2], o[3]);
+      if (lt != 0.f)  // else no key of this share: no sums
+        *(float4*)(rec + 4 + d) = make_float4(o[0], o[1], o[2], o[3]);
     }
   }
 }
@@ -629,12 +630,13 @@ __global__ __launch_bounds__(512, 2) void talk_rows_f32_kernel(TtArgs a) {
     float* dst = a.KS > 1 ? rec + 4
                           : (float*)a.out + (size_t)tok * a.ldout + head * DV;
     if (a.KS == 1) f /= lt;
+    const bool put = r < ntok && (a.KS == 1 || lt != 0.f);
 #pragma unroll
     for (int e = 0; e < NE; e += 4) {
       float o[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = tt_gather(acc[q][e + i]) * f;
-      if (r < ntok)
+      if (put)
 #pragma unroll
         for (int i = 0; i < 4; ++i) dst[at + e * 4 + i] = o[i];
     }
@@ -672,6 +674,7 @@ extern "C" int mx_talk_token(
     int sink, float softcap, const void* sink_vals, int vrow, int dtype,
     int splits, void* scratch, void* stream) {
   if (T_ <= 0) return 0;
+  if (splits > 16) return 1;
   const int vec = dtype == MX_BF16 ? 8 : 4;
   if (H != TT_H || G < 1 || H % G || H / G % 4 || BS < 1) return 1;
   if ((D != 64 && D != 128) || (DV != 64 && DV != 128)) return 1;
@@ -722,6 +725,7 @@ extern "C" int mx_talk_rows_f32(
     int sink, float softcap, const void* sink_vals, int vrow, int splits,
     void* scratch, void* stream) {
   if (T_ <= 0) return 0;
+  if (splits > 16) return 1;
   if (H != TT_H || G < 1 || H % G || H / G % 4 || BS < 1) return 1;
   if ((D != 64 && D != 128) || (DV != 64 && DV != 128)) return 1;
   if (ldq % 4 || vrow % 4 || vrow < DV ||

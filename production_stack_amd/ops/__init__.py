@@ -993,6 +993,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if variant == 15:
         raise RuntimeError(
             "talk_attention: shape or dtype outside the head-mix token kernel")
+    asked = splits
     if variant not in (3, 4, 5, 6):
         splits = 1
     elif splits <= 0:
@@ -1024,12 +1025,29 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     # a head mix over prompt portions on the matrix cores
     if (variant in (0, 10) and q.dtype == torch.bfloat16 and talk is not None
             and keep_first == 0 and pool is None):
+        # Several workgroups for the keys of 16 rows where CUs are left, 64 keys
+        # each at least: a block of rows' two workgroups are one XCD's, which has
+        # 32 CUs (us, heads of 128, in 1 / 2 / 4 / 8: 132 rows, one portion behind
+        # 2882 keys 140 / 90 / 64 / 52, in 12 75; 400 behind 1500 259 / 150 / 93 /
+        # 112; 1349 behind 1463 279 / 205; 1800 in three prompts 101 / 118)
+        keys = block_tables.shape[1] * BS
+        if window > 0:
+            keys = min(keys, window)
+        if chunk > 0:
+            keys = min(keys, chunk)
+        blocks = (T + 127) // 128           # of an XCD
+        shares = asked if asked > 0 else max(1, min(
+            16 // blocks if blocks < 8 else 2 if blocks < 12 else 1,
+            keys // 64))
+        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
+                            device=q.device) if shares > 1 else None)
         rc = _mx().mx_talk_mfma(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
             _p(token_seq), _p(token_pos), _p(talk), T, H, G, D, DV, BS,
             _f(scale), int(chunk), int(window), int(bool(sink)),
-            _f(softcap), _p(sink_vals), int(VR), _stream())
+            _f(softcap), _p(sink_vals), int(VR), int(shares), _p(part),
+            _stream())
         if rc == 0:
             return out
     if variant == 10:

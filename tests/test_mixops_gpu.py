@@ -1289,3 +1289,32 @@ def test_talk_attention_fp32_portions(G, D, DV, chunk, window, softcap,
     fin = torch.isfinite(want)
     assert torch.equal(fin, torch.isfinite(got))
     assert _rel(got[fin], want[fin]) < 4e-6
+
+
+@pytest.mark.parametrize("splits", [1, 2, 5, 16])
+@pytest.mark.parametrize("D,DV,softcap", [(128, 128, 0.0), (64, 128, 9.0)])
+def test_talk_attention_portion_shares(D, DV, softcap, splits):
+    """The 16-row head-mix kernel with the keys of a block over several
+    workgroups: shares of whole 32-key tiles, without a tile, without a key that
+    a row of the block sees; a sink that counts once."""
+    g = torch.Generator().manual_seed(18)
+    H, G, bs, L, chunk = 32, 8, 16, 330, 200
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.bfloat16, g, 2)
+    ts, tp = [], []
+    for s, a, b in ((0, 190, 215), (1, 0, 7), (1, 321, 330), (0, 31, 34)):
+        ts += [s] * (b - a)
+        tp += list(range(a, b))
+    T = len(ts)
+    q = torch.randn(T, H * D, generator=g).to(torch.bfloat16)
+    talk = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)
+    sinks = torch.randn(H, generator=g)
+    ts, tp = (torch.tensor(x, dtype=torch.int32) for x in (ts, tp))
+    want = reference.talk_attention(
+        q.float().reshape(T, H, D), kc.float(), vc.float(), tables, ts, tp,
+        D ** -0.5, chunk, 0, True, talk, 0, softcap, sinks)
+    got = ops.talk_attention(
+        *[x.cuda() for x in (q, kc, vc, tables, ts, tp)], D ** -0.5, H,
+        chunk=chunk, sink=True, talk=talk.cuda(), softcap=softcap, variant=10,
+        sink_vals=sinks.cuda(), splits=splits)
+    # fp32 up to the bf16 rounding of the result
+    assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
