@@ -677,7 +677,10 @@ void greedy_sample(at::Tensor out, at::Tensor logits) {
 
 }  // namespace
 
+void register_entry_calls(PyObject* module);  // entry_call.cpp
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  register_entry_calls(m.ptr());
   m.def("rms_norm", &rms_norm, "RMSNorm (bf16)");
   m.def("fused_add_rms_norm", &fused_add_rms_norm,
         "Fused residual add + RMSNorm (bf16, in-place)");

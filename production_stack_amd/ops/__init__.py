@@ -12,7 +12,7 @@ import os
 
 import torch
 
-from production_stack_amd.ops import reference
+from production_stack_amd.ops import native, reference
 
 try:
     from production_stack_amd import _C  # type: ignore[attr-defined]
@@ -522,8 +522,6 @@ ACT_KINDS = {"silu": 0, "gelu_tanh": 1, "clamped_swish": 2, "sigmoid": 3,
 
 
 def _mx():
-    from production_stack_amd.ops import native
-
     return native.load()
 
 
@@ -535,16 +533,15 @@ def _mx_dtype(dtype: torch.dtype) -> int:
     raise TypeError(f"mixer kernels take bfloat16 or float32, not {dtype}")
 
 
-def _stream():
-    import ctypes
-
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    """The current stream, as entry points take it (torch.cuda.current_stream
+    makes an object of it, which takes 3 us)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t):
-    import ctypes
-
-    return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+    """A pointer: entry points take tensors, or None."""
+    return t
 
 
 def _rows(t: torch.Tensor, name: str) -> int:
@@ -552,6 +549,9 @@ def _rows(t: torch.Tensor, name: str) -> int:
     if t.dim() != 2 or t.stride(1) != 1:
         raise ValueError(f"{name}: need a 2-D view with unit inner stride")
     return t.stride(0)
+
+
+_rows = getattr(_C, "row_stride", _rows)
 
 
 def embed_scale(tokens: torch.Tensor, embed: torch.Tensor,
@@ -578,10 +578,9 @@ def embed_scale(tokens: torch.Tensor, embed: torch.Tensor,
     return x
 
 
-def _f(v: float):
-    import ctypes
-
-    return ctypes.c_float(v)
+def _f(v) -> float:
+    """A float argument: integers are passed as such."""
+    return float(v)
 
 
 def add_rms_norm32(x32: torch.Tensor, deltas, w32: torch.Tensor, eps: float,

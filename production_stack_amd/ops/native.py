@@ -4,8 +4,9 @@ The fp32-residual / delta-rule / linear-scan / attention kernels expose a
 plain C ABI, so the libraries need hipcc only: no torch headers,
 seconds-to-minutes to build, and a fresh checkout compiles on first use just
 the group of files a model's ops live in, without building the large `_C`
-extension. Launchers receive raw device pointers and the current HIP stream;
-shape checks live in the Python wrappers
+extension (which, where it is built, makes the calls: entry_call.cpp). Launchers
+receive raw device pointers and the current HIP stream; shape checks live in the
+Python wrappers
 (production_stack_amd/ops/__init__.py).
 
 Groups (one shared library each):
@@ -210,6 +211,30 @@ def build(force: bool = False, groups=None) -> str:
     return LIB_PATH
 
 
+def _entry(fn, name: str):
+    """A callable for an entry point, whose arguments are tensors or None (a
+    pointer), integers and floats. The `_C` extension marshals them; without it
+    ctypes does, which takes longer than a launch."""
+    try:
+        from production_stack_amd import _C
+    except ImportError:
+        _C = None
+    if hasattr(_C, "entry"):
+        kind = 1 if name in INT_RESULT else 2 if name in LONG_RESULT else 0
+        return _C.entry(ctypes.cast(fn, ctypes.c_void_p).value, kind, name)
+    fn.restype = (ctypes.c_int if name in INT_RESULT else
+                  ctypes.c_long if name in LONG_RESULT else None)
+
+    def argument(a):
+        if isinstance(a, float):
+            return ctypes.c_float(a)
+        if a is None or isinstance(a, int):
+            return ctypes.c_void_p(a) if not a or a >> 31 else a
+        return ctypes.c_void_p(a.data_ptr())
+
+    return lambda *args: fn(*map(argument, args))
+
+
 class _Libs:
     """Attribute access resolves an entry point in its group's library,
     which is loaded (and built, when it is not there or was built from other
@@ -230,9 +255,8 @@ class _Libs:
     def __getattr__(self, name: str):
         if not name.startswith("mx_"):
             raise AttributeError(name)
-        fn = getattr(self._handle(SYMBOL_GROUP.get(name, "core")), name)
-        fn.restype = (ctypes.c_int if name in INT_RESULT else
-                      ctypes.c_long if name in LONG_RESULT else None)
+        fn = _entry(getattr(self._handle(SYMBOL_GROUP.get(name, "core")),
+                            name), name)
         setattr(self, name, fn)
         return fn
 

@@ -31,6 +31,7 @@ ext = CUDAExtension(
     name="production_stack_amd._C",
     sources=[
         "csrc/bindings.cpp",
+        "csrc/entry_call.cpp",
         "csrc/norm_act_rope.hip",
         "csrc/attention.hip",
         "csrc/decode_attention.hip",

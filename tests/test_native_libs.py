@@ -2,6 +2,7 @@
 types, so a library built from other sources must not be loaded."""
 
 import subprocess
+import sys
 
 import pytest
 
@@ -81,3 +82,81 @@ def test_library_without_sources_is_taken_as_it_is(tree):
     changed()
     assert native.current("core")
     assert native._Libs().mx_answer() == 1 and len(builds) == 1
+
+
+ENTRY_C = """
+#include <stdint.h>
+#define W(i, v) r = r * 31 + (int64_t)(v) * (i)
+long mx_mixed(const float* p, int a, float x, const void* q, long b, float y,
+              int c0, int c1, int c2, int c3, int c4, int c5, int c6, int c7,
+              float z, int d0, int d1, int d2, int d3, int d4, int d5, int d6,
+              int d7, int e0, int e1, int e2, int e3, int e4, int e5, int e6,
+              int e7, float f0, float f1, float f2, float f3, float f4,
+              int last, void* stream) {
+  int64_t r = 0;
+  W(1, p[1]); W(2, a); W(3, x * 4); W(4, q == 0); W(5, b); W(6, y * 4);
+  W(7, c0); W(8, c1); W(9, c2); W(10, c3); W(11, c4); W(12, c5); W(13, c6);
+  W(14, c7); W(15, z * 4); W(16, d0); W(17, d1); W(18, d2); W(19, d3);
+  W(20, d4); W(21, d5); W(22, d6); W(23, d7); W(24, e0); W(25, e1);
+  W(26, e2); W(27, e3); W(28, e4); W(29, e5); W(30, e6); W(31, e7);
+  W(32, f0 * 4); W(33, f1 * 4); W(34, f2 * 4); W(35, f3 * 4); W(36, f4 * 4);
+  W(37, last); W(38, (intptr_t)stream >> 33);
+  return r % 1000003;
+}
+int mx_minus(int a) { return -a; }
+void mx_set(float* p, float v) { *p = v; }
+"""
+
+
+@pytest.mark.parametrize("extension", [True, False])
+def test_entry_points_get_their_arguments(tmp_path, monkeypatch, extension):
+    """Pointers, integers and floats in any order, more than registers hold,
+    through the extension and through ctypes."""
+    import ctypes
+
+    import torch
+
+    import production_stack_amd
+
+    if extension:
+        pytest.importorskip("production_stack_amd._C")
+    else:
+        monkeypatch.setitem(sys.modules, "production_stack_amd._C", None)
+        monkeypatch.delattr(production_stack_amd, "_C", raising=False)
+    src, lib = tmp_path / "e.c", tmp_path / "e.so"
+    src.write_text(ENTRY_C)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-fwrapv", str(src), "-o",
+                    str(lib)], check=True)
+    h = ctypes.CDLL(str(lib))
+    monkeypatch.setattr(native, "LONG_RESULT", {"mx_mixed"})
+    monkeypatch.setattr(native, "INT_RESULT", {"mx_minus"})
+    mixed, minus, put = (native._entry(getattr(h, n), n)
+                         for n in ("mx_mixed", "mx_minus", "mx_set"))
+    t = torch.tensor([1.0, 77.0, 3.0])
+    args = [t, -5, 0.25, None, 1 << 40, -1.5, 1, 2, 3, 4, 5, 6, 7, 8, 2.25, 9,
+            10, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22, 23, True, 0.5,
+            0.75, 1.0, 1.25, 7.5, -3, 0x7f1234567000]
+    terms = [77, -5, 1, 1, 1 << 40, -6, 1, 2, 3, 4, 5, 6, 7, 8, 9, 9, 10, 11,
+             12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22, 23, 1, 2, 3, 4, 5, 30,
+             -3, 0x7f1234567000 >> 33]
+    r = 0
+    for i, v in enumerate(terms):
+        r = r * 31 + v * (i + 1)
+    r = (r + (1 << 63)) % (1 << 64) - (1 << 63)       # as 64 bits have it
+    assert mixed(*args) == (abs(r) % 1000003) * (1 if r >= 0 else -1)
+    assert minus(7) == -7 and minus(-7) == 7
+    assert put(t[2:], 5.5) is None and t[2] == 5.5
+    if extension:
+        with pytest.raises(TypeError):
+            minus("7")
+        with pytest.raises(TypeError):
+            minus(*range(60))
+        with pytest.raises(TypeError):
+            put(t, *[0.5] * 9)
+        from production_stack_amd import _C
+
+        view = torch.zeros(4, 6)[:, 1:3]
+        assert _C.row_stride(view, "x") == 6
+        for bad in (view.t(), t):
+            with pytest.raises(ValueError, match="x: need a 2-D view"):
+                _C.row_stride(bad, "x")
