@@ -1103,6 +1103,10 @@ struct CkGroup {  // per chunk and group: fragments of Q and K
   static constexpr int K = 16 * DP;
   static constexpr int TOTAL = 32 * DP;
 };
+// Floats of a head in a row of the matrix LSTM's outputs before their read-out: its
+// columns, n.q behind them, up to a border of 16 bytes.
+__host__ __device__ constexpr int ck_pitch(int DV) { return (DV + 4) & ~3; }
+
 struct CkHead {  // per chunk and head
   static constexpr int M = 0;     // 16 x 16 on V, fragment order
   static constexpr int DR = 256;  // [16] decay from the chunk's start
@@ -1113,36 +1117,46 @@ struct CkHead {  // per chunk and head
 
 // Gates of the matrix LSTM: i = cap(wr + p0), f = logsigmoid(cap(dec + p1)),
 // m' = max(f + m, i); ga / gw / ge [T, H] = exp(f + m - m'), exp(i - m'),
-// exp(-m'). One wave per (segment, head); the running maximum over 64 tokens
-// is a scan over lanes of the maps m -> max(m + A, B).
+// exp(-m'). The running maximum over 64 tokens is a scan over a wave's lanes of the
+// maps m -> max(m + A, B). A workgroup per (segment, head), whose waves scan 64
+// tokens each at a time; the maps of whole waves go through LDS, where every wave
+// follows m through those before it, so that it is what one wave after another would
+// find. A turn takes 0.8 us whatever its waves (one wave a segment: 16 heads, 4950 rows
+// in 2 prompts 44 us, 9 with 16).
 template <typename T>
-__global__ __launch_bounds__(64) void ck_gates_kernel(
+__global__ __launch_bounds__(1024) void ck_gates_kernel(
     float* __restrict__ ga, float* __restrict__ gw, float* __restrict__ ge,
     const T* __restrict__ wr, int ldwr, const T* __restrict__ dec, int lddec,
     const float* __restrict__ p0, const float* __restrict__ p1,
     float* __restrict__ aux, const int* __restrict__ seq_rows, int H, int D,
     float cap) {
-  const int seg = blockIdx.x / H, hd = blockIdx.x % H, lane = threadIdx.x;
+  __shared__ float2 s_map[2][16];
+  const int seg = blockIdx.x / H, hd = blockIdx.x % H;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int waves = blockDim.x >> 6;
   const int t0 = seq_rows[4 * seg], n = seq_rows[4 * seg + 1];
   const int pos0 = seq_rows[4 * seg + 2], slot = seq_rows[4 * seg + 3];
   if (n < 16) return;
   float* mp = aux + ((size_t)slot * H + hd) * (D + 1) + D;
-  float m = pos0 != 0 ? *mp : 0.f;
+  float m = pos0 != 0 ? *mp : 0.f;  // before the turn's first token
   const float bi = p0[hd], bf = p1[hd];
-  // the next 64 tokens' inputs are asked for before these are used: a wave
-  // alone on its SIMD has nothing else to wait beside
-  auto fetch = [&](int tb, float* zi, float* zf) {
-    const size_t row = (size_t)(t0 + min(tb + lane, n - 1));
+  // the next turn's inputs are asked for before these are used: few waves have
+  // nothing else to wait beside
+  auto fetch = [&](int t, float* zi, float* zf) {
+    const size_t row = (size_t)(t0 + min(t, n - 1));
     *zi = MxElem<T>::ld(wr + row * ldwr + hd);
     *zf = MxElem<T>::ld(dec + row * lddec + hd);
   };
   float zi, zf, ni, nf;
-  fetch(0, &ni, &nf);
-  for (int tb = 0; tb < n; tb += 64) {
-    const size_t row = (size_t)(t0 + min(tb + lane, n - 1));
+  fetch(wave * 64 + lane, &ni, &nf);
+  int turn = 0;
+  for (int tb = 0; tb < n; tb += 64 * waves) {
+    const int t = tb + wave * 64 + lane;
+    const size_t row = (size_t)(t0 + min(t, n - 1));
     zi = ni + bi;
     zf = nf + bf;
-    fetch(tb + 64, &ni, &nf);
+    fetch(t + 64 * waves, &ni, &nf);
     const float ig = cap * tanhf(zi / cap);
     const float fg = ck_log_sigmoid(cap * tanhf(zf / cap));
     float A = fg, B = ig;
@@ -1154,17 +1168,34 @@ __global__ __launch_bounds__(64) void ck_gates_kernel(
         A += a1;
       }
     }
-    const float mn = fmaxf(m + A, B);
+    if (lane == 63) s_map[turn][wave] = make_float2(A, B);
+    __syncthreads();
+    float mw = m;  // before this wave's first token
+    for (int w = 0; w < waves; ++w) {
+      const float2 ab = s_map[turn][w];
+      if (w == wave) mw = m;
+      m = fmaxf(m + ab.x, ab.y);
+    }
+    turn ^= 1;
+    const float mn = fmaxf(mw + A, B);
     float mo = __shfl_up(mn, 1, 64);
-    if (lane == 0) mo = m;
-    if (tb + lane < n) {
+    if (lane == 0) mo = mw;
+    if (t < n) {
       ga[row * H + hd] = expf(fg + mo - mn);
       gw[row * H + hd] = expf(ig - mn);
       ge[row * H + hd] = expf(-mn);
     }
-    m = __shfl(mn, min(63, n - 1 - tb), 64);
+    if (t == n - 1) *mp = mn;
   }
-  if (lane == 0) *mp = m;
+}
+
+// Waves of a workgroup of the gates: as many as a segment of all rows has 64s of,
+// fewer where the segments' heads are many (a workgroup of a segment of a few rows has
+// nothing to do, whatever its size).
+static int ck_gate_waves(int T_, int S_, int H) {
+  const long most = 8192l / ((long)S_ * H);
+  const int want = (T_ + 63) / 64 < 16 ? (T_ + 63) / 64 : 16;
+  return most < 1 ? 1 : most < want ? (int)most : want;
 }
 
 template <typename T, int MODE, int DP>
@@ -1279,7 +1310,7 @@ __global__ __launch_bounds__(256) void ck_prep_scalar_kernel(
 
 // The walk of ck_sweep_kernel for one decay per head and token. out: the
 // finished fp32 rows of ssd, (o + skip v) silu(gate), or the raw read-outs
-// [T, H * (DV + 1)] of mlstm, whose column DV is the normaliser's (its values
+// [T, H * ck_pitch(DV)] of mlstm, whose column DV is the normaliser's (its values
 // are 1, its state lies in aux). PART, part and parts as there; a record is the
 // D x (DV, with the normaliser DV + 1) state and one decay.
 template <typename T, int MODE, int DP, int PART>
@@ -1483,7 +1514,7 @@ __global__ __launch_bounds__(256, 2) void ck_sweep_scalar_kernel(
             out[(row + i) * ldo + hv] =
                 (O[i] + skip * V[i]) * gt[i] * ck_sigmoid(gt[i]);
           else
-            out[(row + i) * ldo + hd * (DV + 1) + j] = O[i];
+            out[(row + i) * ldo + hd * ck_pitch(DV) + j] = O[i];
         }
       }
     }
@@ -1853,7 +1884,7 @@ PS_DEV bool ck_walk_wide(const CkWideCall& a, CkWideLds<DP, NW>& lds) {
                           hd * DV)
           : nullptr;
   char* oseg = (char*)(a.out + (size_t)t0 * ldo +
-                       hd * (MODE == CK_SSD ? DV : DV + 1));
+                       hd * (MODE == CK_SSD ? DV : ck_pitch(DV)));
   // chunk c's rows (and more, up to the segment's end) of `p`, `rb` bytes
   // apart, `width` bytes of each
   auto rows_from = [&](const char* p, int c, unsigned rb, unsigned width) {
@@ -2282,7 +2313,7 @@ __global__ __launch_bounds__(256) void ck_readout_kernel(
     const int* __restrict__ seq_rows, int S_, int H, int DV, float eps,
     const float* __restrict__ ge) {
   // the matrix LSTM's rows carry n.q behind a head's columns
-  constexpr int EXTRA = MODE == CK_MLSTM ? 1 : 0;
+  const int pitch = MODE == CK_MLSTM ? ck_pitch(DV) : DV;
   const int t = blockIdx.x, lane = threadIdx.x & 63;
   const int h0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * 4;
   // rows of short segments are not this kernel's
@@ -2297,7 +2328,7 @@ __global__ __launch_bounds__(256) void ck_readout_kernel(
     mine = __any(hit);
   }
   if (!mine) return;
-  const float* r = raw + (size_t)t * ((size_t)H * (DV + EXTRA));
+  const float* r = raw + (size_t)t * ((size_t)H * pitch);
   const T* gp = gate + (size_t)t * ldg;
   T* op = out + (size_t)t * ldo;
   const int c0 = lane * VEC;
@@ -2308,13 +2339,13 @@ __global__ __launch_bounds__(256) void ck_readout_kernel(
 #pragma unroll
     for (int u = 0; u < VEC; ++u) {
       const int c = min(c0 + u, DV - 1);
-      o[h][u] = r[hd * (DV + EXTRA) + c];
+      o[h][u] = r[hd * pitch + c];
       gv[h][u] = MxElem<T>::ld(gp + hd * DV + c);
       nw[h][u] =
           normw[(MODE == CK_GD || MODE == CK_MLSTM ? hd * DV : 0) + c];
     }
     if (MODE == CK_MLSTM)
-      den[h] = fmaxf(fabsf(r[hd * (DV + 1) + DV]), ge[(size_t)t * H + hd]) +
+      den[h] = fmaxf(fabsf(r[hd * pitch + DV]), ge[(size_t)t * H + hd]) +
                1e-6f;
   }
 #pragma unroll
@@ -2341,8 +2372,7 @@ __global__ __launch_bounds__(256) void ck_readout_kernel(
   }
 }
 
-// The same for heads of 8 LPH columns whose rows lie on 16-byte borders (not the
-// matrix LSTM's): a lane has eight neighbouring columns, LPH lanes a head, so that
+// The same for heads of 8 LPH columns whose rows lie on 16-byte borders: a lane has eight neighbouring columns, LPH lanes a head, so that
 // every access is 16 bytes. Whether the rows are this kernel's is asked while they
 // are on their way. Bound by memory; us, a lane with one to four columns of four
 // heads / this: 8011 rows of 32 bf16 heads of 128 80 / 42 (6.2 TB/s), 6007 rows 55 /
@@ -2351,8 +2381,10 @@ template <typename T, int MODE, int LPH>
 __global__ __launch_bounds__(256) void ck_readout_wide_kernel(
     T* __restrict__ out, int ldo, const float* __restrict__ raw,
     const T* __restrict__ gate, int ldg, const float* __restrict__ normw,
-    const int* __restrict__ seq_rows, int S_, int T_, int H, float eps) {
+    const int* __restrict__ seq_rows, int S_, int T_, int H, float eps,
+    const float* __restrict__ ge) {
   constexpr int DV = 8 * LPH;
+  constexpr int PITCH = MODE == CK_MLSTM ? ck_pitch(DV) : DV;
   struct alignas(16) vec8 {
     T e[8];
   };
@@ -2361,10 +2393,16 @@ __global__ __launch_bounds__(256) void ck_readout_wide_kernel(
   const unsigned last = (unsigned)T_ * units - 1;
   const unsigned at = min(i, last);
   const int t = at / units, c = (at - t * units) * 8;
-  const float* r = raw + (size_t)t * (H * DV) + c;
-  const ck_f32x4 oa = *(const ck_f32x4*)r, ob = *(const ck_f32x4*)(r + 4);
+  const unsigned hd = c / DV;
+  const float* rh = raw + (size_t)t * (H * PITCH) + hd * PITCH;
+  const float* r = rh + c % DV;
+  ck_f32x4 oa = *(const ck_f32x4*)r, ob = *(const ck_f32x4*)(r + 4);
+  float den = 1.f;
+  if (MODE == CK_MLSTM)
+    den = fmaxf(fabsf(rh[DV]), ge[(size_t)t * H + hd]) + 1e-6f;
   const vec8 gv = *(const vec8*)(gate + (size_t)t * ldg + c);
-  const float* w = normw + (MODE == CK_GD ? c : c % DV);
+  const float* w =
+      normw + (MODE == CK_GD || MODE == CK_MLSTM ? c : c % DV);
   const ck_f32x4 wa = *(const ck_f32x4*)w, wb = *(const ck_f32x4*)(w + 4);
   // rows of short segments are not this kernel's; a wave has one row or a few
   const int lane = threadIdx.x & 63;
@@ -2384,6 +2422,10 @@ __global__ __launch_bounds__(256) void ck_readout_wide_kernel(
       if (__all(mine)) break;
     }
     if (__all(mine)) break;
+  }
+  if (MODE == CK_MLSTM) {
+    oa /= den;
+    ob /= den;
   }
   float ss = 0.f;
 #pragma unroll
@@ -2516,33 +2558,31 @@ static long ck_part_floats(int mode, int T_, int S_, int H, int D, int DV,
 // Floats of scratch per row: raw read-outs, and the matrix LSTM's gates.
 static long ck_rows_floats(int mode, int T_, int H, int DV) {
   if (mode == CK_SSD) return 0;
-  return (long)T_ * H * (mode == CK_MLSTM ? DV + 4 : DV);
+  return (long)T_ * H * (mode == CK_MLSTM ? ck_pitch(DV) + 3 : DV);
 }
 
 template <typename T, int MODE>
 static void ck_read(CK_ARGS, const float* raw, const float* gx) {
-  if constexpr (MODE != CK_MLSTM) {
-    const int border = 16 / sizeof(T);
-    const size_t at = (size_t)out | (size_t)in.gate | (size_t)normw |
-                      (size_t)raw;
-    if (at % 16 == 0 && ldo % border == 0 && in.ldg % border == 0 &&
-        (long)T_ * H * DV < 1l << 32) {
+  const int border = 16 / sizeof(T);
+  const size_t at = (size_t)out | (size_t)in.gate | (size_t)normw |
+                    (size_t)raw;
+  if (at % 16 == 0 && ldo % border == 0 && in.ldg % border == 0 &&
+      (long)T_ * H * DV < 1l << 32) {
 #define CK_READ(LPH)                                                         \
   case 8 * LPH:                                                              \
     hipLaunchKernelGGL((ck_readout_wide_kernel<T, MODE, LPH>),               \
                        dim3(((long)T_ * H * LPH + 255) / 256), dim3(256), 0, \
                        stream, (T*)out, ldo, raw, (const T*)in.gate, in.ldg, \
                        (const float*)normw, (const int*)seq_rows, S_, T_, H, \
-                       eps);                                                 \
+                       eps, gx);                                             \
     return;
-      switch (DV) {
-        CK_READ(4)
-        CK_READ(8)
-        CK_READ(16)
-        CK_READ(32)
-      }
-#undef CK_READ
+    switch (DV) {
+      CK_READ(4)
+      CK_READ(8)
+      CK_READ(16)
+      CK_READ(32)
     }
+#undef CK_READ
   }
 #define CK_READ(VEC)                                                         \
   hipLaunchKernelGGL((ck_readout_kernel<T, MODE, VEC>),                      \
@@ -2599,7 +2639,7 @@ static int ck_launch_scalar(CK_ARGS) {
   ck_plan(MODE, T_, S_, H, G, D, 16, &cap, &passes);
   const bool lstm = MODE == CK_MLSTM;
   float* raw = scratch;
-  float* ga = raw + (lstm ? (size_t)T_ * H * (DV + 1) : 0);
+  float* ga = raw + (lstm ? (size_t)T_ * H * ck_pitch(DV) : 0);
   float* gw = ga + (lstm ? (size_t)T_ * H : 0);
   float* ge = gw + (lstm ? (size_t)T_ * H : 0);
   float* gitems = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
@@ -2608,7 +2648,8 @@ static int ck_launch_scalar(CK_ARGS) {
   const int parts = ck_parts(MODE, T_, S_, H, DV, 16);
   float* part = hitems + (((size_t)cap * H * CkHead::TOTAL + 3) & ~(size_t)3);
   if (lstm)
-    hipLaunchKernelGGL((ck_gates_kernel<T>), dim3(S_ * H), dim3(64), 0,
+    hipLaunchKernelGGL((ck_gates_kernel<T>), dim3(S_ * H),
+                       dim3(64 * ck_gate_waves(T_, S_, H)), 0,
                        stream, ga, gw, ge, (const T*)in.a, in.lda,
                        (const T*)in.dec, in.lddec, in.p0, in.p1, (float*)aux,
                        (const int*)seq_rows, H, D, c0f);
@@ -2622,7 +2663,7 @@ static int ck_launch_scalar(CK_ARGS) {
 #define CK_SWEEP(PART, RUNS)                                                 \
   hipLaunchKernelGGL((ck_sweep_scalar_kernel<T, MODE, DP, PART>),            \
                      dim3(S_ * H * ncb * (RUNS)), dim3(256), 0, stream,      \
-                     lstm ? raw : (float*)out, lstm ? H * (DV + 1) : ldo,    \
+                     lstm ? raw : (float*)out, lstm ? H * ck_pitch(DV) : ldo,    \
                      gitems, hitems, cap, in, (const float*)p2,              \
                      (float*)state, (float*)aux, (const int*)seq_rows, S_,   \
                      H, G, D, DV, p * cap, part, parts)
@@ -2644,7 +2685,7 @@ static int ck_launch_wide(CK_ARGS) {
   ck_plan(MODE, T_, S_, H, G, D, CK_WIDE, &cap, &passes);
   const bool lstm = MODE == CK_MLSTM;
   float* raw = scratch;
-  float* ga = raw + (lstm ? (size_t)T_ * H * (DV + 1) : 0);
+  float* ga = raw + (lstm ? (size_t)T_ * H * ck_pitch(DV) : 0);
   float* gw = ga + (lstm ? (size_t)T_ * H : 0);
   float* ge = gw + (lstm ? (size_t)T_ * H : 0);
   float* gitems = scratch + ((ck_rows_floats(MODE, T_, H, DV) + 3) & ~3l);
@@ -2653,7 +2694,8 @@ static int ck_launch_wide(CK_ARGS) {
   const int parts = ck_parts(MODE, T_, S_, H, DV, CK_WIDE);
   float* part = hitems + (size_t)cap * H * CkWideHead::TOTAL;
   if (lstm)
-    hipLaunchKernelGGL((ck_gates_kernel<mx_bf16>), dim3(S_ * H), dim3(64), 0,
+    hipLaunchKernelGGL((ck_gates_kernel<mx_bf16>), dim3(S_ * H),
+                       dim3(64 * ck_gate_waves(T_, S_, H)), 0,
                        stream, ga, gw, ge, (const mx_bf16*)in.a, in.lda,
                        (const mx_bf16*)in.dec, in.lddec, in.p0, in.p1,
                        (float*)aux, (const int*)seq_rows, H, D, c0f);
@@ -2664,7 +2706,7 @@ static int ck_launch_wide(CK_ARGS) {
                        dim3(256), 0, stream, (char*)gitems, hitems, in, ga,
                        gw, (const int*)seq_rows, S_, H, G, D, scale, p * cap);
     const CkWideCall call = {
-        lstm ? raw : (float*)out, lstm ? H * (DV + 1) : ldo,
+        lstm ? raw : (float*)out, lstm ? H * ck_pitch(DV) : ldo,
         (const char*)gitems, hitems, cap, in, (const float*)p2, (float*)state,
         (float*)aux, (const int*)seq_rows, S_, H, G, D, DV, p * cap, part,
         parts};

@@ -1318,3 +1318,27 @@ def test_talk_attention_portion_shares(D, DV, softcap, splits):
         sink_vals=sinks.cuda(), splits=splits)
     # fp32 up to the bf16 rounding of the result
     assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("lens,DV", [([64, 65], 32), ([63, 16], 30),
+                                     ([1024, 17], 33), ([1025, 40], 32),
+                                     ([2100, 1, 300], 64)])
+def test_matrix_lstm_turns_of_waves(lens, DV, dtype):
+    """The gates' running maximum over waves of 64 tokens, workgroups of 16 waves
+    and several turns of them; outputs from rows on 16-byte borders and off them."""
+    H, D = 3, 16
+    segs = _segs(lens, [5, 0, 9][:len(lens)])
+    x, state, aux, call = _recurrence("mlstm", H, D, DV, segs, dtype)
+    # long stretches in which the maximum only decays, and steps up within them
+    for k in ("a", "dec"):
+        x[k][::] = (x[k].float() * 4 - (6 if k == "a" else 0)).to(dtype)
+    rows = torch.tensor(segs, dtype=torch.int32)
+    sr, ar = state.clone(), aux.clone()
+    want = call({k: v.float() for k, v in x.items()}, sr, ar, rows)
+    sg, ag = state.cuda(), aux.cuda()
+    got = call(_to_gpu(x), sg, ag, rows.cuda())
+    # sums over chunks of 16 or 32 rows; bf16 outputs are rounded
+    assert _rel(got, want) < (4e-3 if dtype == torch.bfloat16 else 4e-6)
+    assert _rel(sg, sr) < 4e-6 and _rel(ag, ar) < 4e-6
+    assert _rel(ag[..., D], ar[..., D]) < 1e-6
