@@ -357,11 +357,13 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
 
 // Merge of `KS` (at most AF_KS) partial records of every (token, head): 256 threads
 // of four entries each. Shares without a key have a denominator of 0 and no sums.
+// counted: the first record's third entry is how many there are; of a single one the
+// result is already there.
 #define AF_KS 16
 template <typename T>
 __global__ __launch_bounds__(256) void attn_records_kernel(
     T* __restrict__ out, int ldout, const float* __restrict__ part, int H,
-    int DV, int KS) {
+    int DV, int KS, int counted) {
   const int vpr = DV / 4, idx = blockIdx.y * 256 + threadIdx.x;
   if (idx >= H * vpr) return;
   const int h = idx / vpr, d = (idx - h * vpr) * 4;
@@ -369,11 +371,16 @@ __global__ __launch_bounds__(256) void attn_records_kernel(
       part + ((size_t)blockIdx.x * KS * H + h) * (DV + AF_HEAD);
   const size_t step = (size_t)H * (DV + AF_HEAD);
   float2 ml[AF_KS];
+#pragma unroll
+  for (int s = 0; s < AF_KS; ++s)
+    ml[s] = s < KS ? *(const float2*)(rec + s * step)
+                   : make_float2(PS_NEG_INF, 0.f);
+  const int count = counted ? (int)rec[2] : KS;
+  if (counted && count == 1) return;
   float mh = PS_NEG_INF;
 #pragma unroll
   for (int s = 0; s < AF_KS; ++s) {
-    ml[s] = s < KS ? *(const float2*)(rec + s * step)
-                   : make_float2(PS_NEG_INF, 0.f);
+    if (s >= count) ml[s].y = 0.f;
     if (ml[s].y != 0.f) mh = fmaxf(mh, ml[s].x);
   }
   float l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
@@ -396,13 +403,13 @@ __global__ __launch_bounds__(256) void attn_records_kernel(
 
 // Merge pass over records [T, KS, H, DV + 4] (DV in steps of 4, KS up to 16).
 extern "C" void mx_attn_records(void* out, int ldout, const void* part, int T_,
-                                int H, int DV, int KS, int dtype,
-                                void* stream) {
+                                int H, int DV, int KS, int counted,
+                                int dtype, void* stream) {
   MX_DISPATCH_DTYPE(dtype, {
     hipLaunchKernelGGL((attn_records_kernel<T>),
                        dim3(T_, (H * (DV / 4) + 255) / 256), dim3(256), 0,
                        (hipStream_t)stream, (T*)out, ldout, (const float*)part,
-                       H, DV, KS);
+                       H, DV, KS, counted);
   })
 }
 
@@ -464,6 +471,6 @@ extern "C" int mx_attn_f32(void* out, int ldout, const void* q, int ldq,
     AF_GO(8, 2);
 #undef AF_GO
   if (rc == 0 && a.KS > 1)
-    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, MX_F32, stream);
+    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, 0, MX_F32, stream);
   return rc;
 }

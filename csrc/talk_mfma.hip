@@ -37,8 +37,9 @@
 // spill at widths of 128 and are no faster at 64 (284 us, 272 with eight); orders of
 // the four parts that differ between the two waves of a SIMD spill as well.
 // Few rows behind many keys are a chain of tiles (3.5 us each) on a few CUs: there
-// several workgroups share a block's keys, and mx_attn_records merges what they have (70
-// rows behind 2000 keys 276 us whole, 50 in 16 shares).
+// several workgroups share a block's keys, as many as have two tiles, and
+// mx_attn_records merges what they have (70 rows behind 2000 keys 276 us whole, 50 in
+// 16 shares; a portion with too few keys for shares 3 us more for that launch).
 #include "attn_common.h"
 #include "scan_common.h"
 
@@ -57,6 +58,7 @@ union TmPack {
 
 #define TM_H 32
 #define TM_KT 32
+#define TM_SHARE 2  // tiles of a share at least
 // How far scores, in powers of two, may be above those that set the reference that
 // weights are relative to. The reference is as much above them: no weight is above 1.
 #define TM_FAR 8.f
@@ -78,7 +80,7 @@ struct TmArgs {
   float softcap;
   const float* sink_vals;
   int KS;       // workgroups that share a block's keys
-  float* part;  // [T, KS, 32, DV + 4]: maximum, denominator, sums
+  float* part;  // [T, KS, 32, DV + 4]: maximum, denominator, shares, -, sums
 };
 
 // A bf16 entry that is an infinity or no number.
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
   // one of the two waves of a SIMD first, so that its softmax comes beside
   // products of the other (324 -> 320 us)
   if (ND == 4 && wave < 4) __builtin_amdgcn_s_setprio(1);
-  int rs = 0;
+  int rs = 0, my_eff = 1;  // shares of this lane's row
   while (rs < ntok) {
     // batch rows rs .. re - 1 continue one sequence
     int re = rs + 1;
@@ -253,12 +255,15 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
     };
     int kmin = low(s_pos[rs]), kmax = s_pos[re - 1];
     if constexpr (PART) {  // this share's tiles
+      // the workgroups that have a share of these tiles
       const int all = (kmax - kmin) / TM_KT + 1, ks = blockIdx.y;
-      const int t0 = all * ks / a.KS, t1 = all * (ks + 1) / a.KS;
-      if (t0 == t1) {
+      const int eff = max(1, min(a.KS, all / TM_SHARE));
+      if (mine) my_eff = eff;
+      if (ks >= eff) {
         rs = re;
         continue;
       }
+      const int t0 = all * ks / eff, t1 = all * (ks + 1) / eff;
       kmax = min(kmax, kmin + t1 * TM_KT - 1);
       kmin += t0 * TM_KT;
     }
@@ -540,7 +545,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
     if (PART && wave == 0) sAL[(4 * g + i) * 16 + n] = m[i];
   }
   __syncthreads();
-  if (n >= ntok) return;
+  if (n >= ntok || (PART && (int)blockIdx.y >= my_eff)) return;
   unsigned short* o = a.out + (size_t)(tok0 + n) * a.ldout +
                       (16 * hb + wave * 2) * DV + 4 * g;
   const bool vec = (a.ldout & 3) == 0 && ((size_t)a.out & 7) == 0;
@@ -556,13 +561,16 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
         const float mt = sAL[(wave * 2 + h) * 16 + n];
         rec[0] = lt != 0.f ? mt * 0.693147181f : PS_NEG_INF;
         rec[1] = lt;
+        rec[2] = (float)my_eff;
       }
-      if (lt == 0.f) continue;  // no key of this share: no sums
+      if (my_eff > 1) {
+        if (lt != 0.f)  // else no key of this share: no sums
 #pragma unroll
-      for (int c = 0; c < NV; ++c)
-        *(float4*)(rec + 4 + 16 * c + 4 * g) =
-            make_float4(acc[h][c][0], acc[h][c][1], acc[h][c][2], acc[h][c][3]);
-      continue;
+          for (int c = 0; c < NV; ++c)
+            *(float4*)(rec + 4 + 16 * c + 4 * g) = make_float4(
+                acc[h][c][0], acc[h][c][1], acc[h][c][2], acc[h][c][3]);
+        continue;
+      }
     }
     const float f = 1.0f / lt;
 #pragma unroll
@@ -608,8 +616,8 @@ static int tm_launch(const TmArgs& a, hipStream_t stream) {
 }
 
 extern "C" void mx_attn_records(void* out, int ldout, const void* part, int T_,
-                                int H, int DV, int KS, int dtype,
-                                void* stream);
+                                int H, int DV, int KS, int counted,
+                                int dtype, void* stream);
 
 // Returns 0 when launched, 1 when the shape is outside this kernel: 32 heads
 // over at most 8 KV heads (a wave's four heads share one), widths 64 or 128,
@@ -637,6 +645,6 @@ extern "C" int mx_talk_mfma(
   const int rc = D == 64 ? (DV == 64 ? tm_launch<2, 4>(a, s) : tm_launch<2, 8>(a, s))
                          : (DV == 64 ? tm_launch<4, 4>(a, s) : tm_launch<4, 8>(a, s));
   if (rc == 0 && a.KS > 1)
-    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, MX_BF16, stream);
+    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, 1, MX_BF16, stream);
   return rc;
 }

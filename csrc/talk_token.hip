@@ -644,8 +644,8 @@ __global__ __launch_bounds__(512, 2) void talk_rows_f32_kernel(TtArgs a) {
 }
 
 extern "C" void mx_attn_records(void* out, int ldout, const void* part, int T_,
-                                int H, int DV, int KS, int dtype,
-                                void* stream);
+                                int H, int DV, int KS, int counted,
+                                int dtype, void* stream);
 
 template <typename T, int D, int DV>
 static int tt_launch(const TtArgs& a, hipStream_t stream) {
@@ -698,7 +698,7 @@ extern "C" int mx_talk_token(
                     : tt_launch<T, 128, 128>(a, s);
   })
   if (rc == 0 && a.KS > 1)
-    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, dtype, stream);
+    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, 0, dtype, stream);
   return rc;
 }
 
@@ -744,6 +744,6 @@ extern "C" int mx_talk_rows_f32(
                          : (DV == 64 ? tt_launch_rows<128, 64>(a, s)
                                      : tt_launch_rows<128, 128>(a, s));
   if (rc == 0 && a.KS > 1)
-    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, MX_F32, stream);
+    mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, 0, MX_F32, stream);
   return rc;
 }

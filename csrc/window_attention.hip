@@ -70,8 +70,12 @@ PS_DEV float wa_score(const WaArgs& a, float st, float base, float top) {
 
 #define WA_KT 64
 
-// DK: 16-entry steps of a key (D <= 16 DK), VB: 32-column blocks of a value
-template <int DK, int VB, bool CAP>
+#define WA_HEAD 4   // leading entries of a partial record
+#define WA_SHARE 3  // tiles of a portion's share at least
+
+// DK: 16-entry steps of a key (D <= 16 DK), VB: 32-column blocks of a value, PART:
+// several workgroups (up to KS, neighbours) share a tile's keys
+template <int DK, int VB, bool CAP, bool PART>
 __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
   // values: the four rows of a transposed read lie 16 banks apart
   constexpr int PK = DK * 16 + 8, PV = VB * 32 + 32;
@@ -87,7 +91,8 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
   // rows that see the most keys first
   const int GH = a.G * a.hblocks;
   const int gh = blockIdx.x % GH;
-  const int tile = NT - 1 - blockIdx.x / GH;
+  const int ks = PART ? blockIdx.x / GH % a.KS : 0;
+  const int tile = NT - 1 - blockIdx.x / GH / (PART ? a.KS : 1);
   const int g = gh / a.hblocks, hb = gh % a.hblocks;
   const int tok0 = tile * TPT, ntok = min(TPT, a.T - tok0);
   for (int c = tid; c < ntok; c += 256) {
@@ -146,7 +151,7 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
     m = i < 64 ? start1 : i < 127 ? start1 & (~1ull << (i - 64)) : 0;
     return m ? __ffsll(m) + 63 : ntok;
   };
-  int rs = 0;
+  int rs = 0, my_eff = 1;
   while (rs < ntok) {
     // batch rows rs .. re - 1 continue one sequence
     const int re = next_start(rs);
@@ -158,7 +163,16 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
     // kept first keys behind the run's earliest window, then the windows
     const int k0 = min(a.keep, kmin);
     const int nt0 = (k0 + WA_KT - 1) / WA_KT;
-    const int nt = nt0 + (kmax - kmin) / WA_KT + 1;
+    const int all = nt0 + (kmax - kmin) / WA_KT + 1;
+    // the workgroups that have a share of these tiles, and this one's
+    const int eff = PART ? max(1, min(a.KS, all / WA_SHARE)) : 1;
+    if (PART && mine) my_eff = eff;
+    if (PART && ks >= eff) {
+      rs = re;
+      continue;
+    }
+    const int n0 = PART ? all * ks / eff : 0;
+    const int nt = PART ? all * (ks + 1) / eff : all;
     // rows of other runs see nothing of this one
     const int pos = mine ? my_pos : -1;
     const int ia = max(wave * 32 / HPB, rs);
@@ -194,11 +208,11 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
                                 min(idx % CV * 8, DV - 8));
       }
     };
-    put_row(0, table[key_of(0) / a.BS], 1);
+    put_row(n0, table[key_of(n0) / a.BS], 1 - (n0 & 1));
     __syncthreads();  // also: the previous run's tiles are fully read
-    fetch(1);
-    int page = table[key_of(min(1, nt - 1)) / a.BS];
-    for (int n = 0; n < nt; ++n) {
+    fetch(1 - (n0 & 1));
+    int page = table[key_of(min(n0 + 1, nt - 1)) / a.BS];
+    for (int n = n0; n < nt; ++n) {
       // tile n from registers to its buffer, which tile n - 2 has left; what
       // lies past the last tile repeats it
 #pragma unroll
@@ -306,10 +320,42 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
   }
 
   l += __shfl_xor(l, 32, 64);  // a lane summed its own keys
-  if (!valid) return;
+  if (!valid || (PART && ks >= my_eff)) return;
   float own = 1.f;
-  if (a.sink)
-    own = kv_sink(a.sink_vals != nullptr ? a.sink_vals[head] : 0.f, &m, &l);
+  if (a.sink && (!PART || ks == 0)) {  // the sink is share 0's
+    const float sink = a.sink_vals != nullptr ? a.sink_vals[head] : 0.f;
+    if (PART && m == KV_LOW) {  // none of its keys: the sink alone
+      m = fminf(fmaxf(sink * KV_LOG2E, KV_LOW), -KV_LOW);
+      l = 1.f;
+    } else {
+      own = kv_sink(sink, &m, &l);
+    }
+  }
+  if constexpr (PART) {
+    // partial record per (token, share, head): max (natural log units),
+    // denominator, shares, one unused, DV sums
+    float* rec = a.part + (((size_t)tok * a.KS + ks) * a.H + head) *
+                              (size_t)(DV + WA_HEAD);
+    if (hi == 0) {
+      rec[0] = l != 0.f ? m * 0.69314718f : PS_NEG_INF;
+      rec[1] = l;
+      rec[2] = (float)my_eff;
+    }
+    if (my_eff > 1) {
+      if (l == 0.f) return;  // no key of this share: no sums
+#pragma unroll
+      for (int c = 0; c < VB; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int col = 32 * c + 8 * q + 4 * hi;
+          if (col < DV)  // in steps of 8
+            *(float4*)(rec + WA_HEAD + col) =
+                make_float4(acc[c][4 * q] * own, acc[c][4 * q + 1] * own,
+                            acc[c][4 * q + 2] * own, acc[c][4 * q + 3] * own);
+        }
+      return;
+    }
+  }
   const float f = own / l;
   unsigned short* o = a.out + (size_t)tok * a.ldout + (size_t)head * DV;
   const bool vec = ((DV | a.ldout) & 3) == 0 && ((size_t)a.out & 7) == 0;
@@ -339,7 +385,6 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
 // single tokens
 // ---------------------------------------------------------------------------
 #define WA_TT 32    // keys per tile of a wave
-#define WA_HEAD 4   // leading entries of a partial record
 
 // DK: 32-entry steps of a key (D <= 32 DK), VB: 32-column blocks of a value
 template <int DK, int VB, bool CAP>
@@ -569,6 +614,8 @@ extern "C" {
 
 void mx_latent_combine(void* out, int ldout, const void* part, int T_, int H,
                        int DV, int KS, void* stream);
+void mx_attn_records(void* out, int ldout, const void* part, int T_, int H,
+                     int DV, int KS, int counted, int dtype, void* stream);
 
 // Returns 0 when launched, 1 when the shape is outside these kernels: widths of
 // whole 16-byte vectors up to 128, rows on 16-byte borders. token: single
@@ -609,12 +656,17 @@ int mx_window_attention(void* out, int ldout, const void* q, int ldq,
     // keys 1314 -> 344 (876), 32 of 20 behind 100 70 -> 40 (58); 32/8 heads, 64 of
     // 5 behind 1000 356 -> 185 (366), 64 rows behind 2000 87 -> 81 (226). Down to
     // 16 rows, half a wave's: 344 -> 177, but 81 -> 97; up to 512 workgroups: 2
-    // prompts of 2048, 8 heads of 40 60 -> 67.
+    // prompts of 2048, 8 heads of 40 60 -> 67. With shares of the keys whole ones fill
+    // the CUs (70 rows behind 2500 keys 28 us, 37 with fewer rows; four portions of
+    // 17 beside longer tables, which end up without shares, 20, 13 without them).
     a.tpt = 128 / a.hpb;
-    while (a.tpt > 1 && a.tpt * a.hpb > 32 &&
+    a.KS = splits > 1 && scratch != nullptr ? splits : 1;
+    if (a.KS > 16) return 1;
+    a.part = (float*)scratch;
+    while (a.KS == 1 && a.tpt > 1 && a.tpt * a.hpb > 32 &&
            (unsigned)((T_ + a.tpt / 2 - 1) / (a.tpt / 2)) * gh <= 256)
       a.tpt /= 2;
-    grid = dim3((unsigned)((T_ + a.tpt - 1) / a.tpt) * gh);
+    grid = dim3((unsigned)((T_ + a.tpt - 1) / a.tpt) * gh * a.KS);
   } else {
     a.KS = splits > 1 && scratch != nullptr ? splits : 1;
     if (a.KS > 16) return 1;
@@ -642,9 +694,12 @@ int mx_window_attention(void* out, int ldout, const void* q, int ldq,
     if (token)                                                               \
       hipLaunchKernelGGL((window_token_kernel<DK, VB, CAP>), grid,           \
                          dim3(256), 0, (hipStream_t)stream, a);              \
+    else if (a.KS > 1)                                                       \
+      hipLaunchKernelGGL((window_prompt_kernel<2 * DK, VB, CAP, true>),      \
+                         grid, dim3(256), 0, (hipStream_t)stream, a);        \
     else                                                                     \
-      hipLaunchKernelGGL((window_prompt_kernel<2 * DK, VB, CAP>), grid,      \
-                         dim3(256), 0, (hipStream_t)stream, a);              \
+      hipLaunchKernelGGL((window_prompt_kernel<2 * DK, VB, CAP, false>),     \
+                         grid, dim3(256), 0, (hipStream_t)stream, a);        \
   } while (0)
 #define WA_CAP(DK, VB)     \
   do {                     \
@@ -663,8 +718,12 @@ int mx_window_attention(void* out, int ldout, const void* q, int ldq,
     WA_CAP(4, 4);
 #undef WA_CAP
 #undef WA_GO
-  if (token && a.KS > 1)
-    mx_latent_combine(out, ldout, scratch, T_, H, DV, a.KS, stream);
+  if (a.KS > 1) {
+    if (token)
+      mx_latent_combine(out, ldout, scratch, T_, H, DV, a.KS, stream);
+    else
+      mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, 1, MX_BF16, stream);
+  }
   return 0;
 }
 

@@ -882,6 +882,21 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
                 keys = min(keys, window + keep_first)
             shares = splits if splits > 0 else max(
                 1, min(16, 128 // groups, keys // 1024))
+        else:
+            # Several workgroups for a portion's keys where CUs are left, with
+            # three tiles of 64 each at least, of which the kernel counts those
+            # that are (us, 32/8 heads of 128, 128 (token, head) rows a workgroup
+            # in 1 / 2 / 4 / 8 shares: 70 tokens behind 2500 keys 93 / 53 / 35 /
+            # 28; 250 behind 2500 93 / 56 / 41 / 40; 559 behind 2500 93 / 74 / 71
+            # / 78; 1419 behind 2000 120 / 118 / 127 / 156)
+            rep = H // G
+            tokens = 128 // rep if rep < 128 else 1
+            groups = (T + tokens - 1) // tokens * G * ((rep + 127) // 128)
+            keys = block_tables.shape[1] * BS
+            if window > 0:
+                keys = min(keys, window + keep_first)
+            shares = splits if splits > 0 else max(
+                1, min(16, 512 // groups, keys // 192))
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
                             device=q.device) if shares > 1 else None)
         rc = _mx().mx_window_attention(

@@ -1342,3 +1342,33 @@ def test_matrix_lstm_turns_of_waves(lens, DV, dtype):
     assert _rel(got, want) < (4e-3 if dtype == torch.bfloat16 else 4e-6)
     assert _rel(sg, sr) < 4e-6 and _rel(ag, ar) < 4e-6
     assert _rel(ag[..., D], ar[..., D]) < 1e-6
+
+
+@pytest.mark.parametrize("splits", [1, 2, 5, 16])
+@pytest.mark.parametrize("H,G,D,DV,window,keep,softcap", [
+    (32, 8, 128, 128, 700, 70, 0.0), (6, 2, 40, 72, 0, 0, 9.0)])
+def test_window_attention_portion_shares(H, G, D, DV, window, keep, softcap,
+                                         splits):
+    """Portions whose keys several workgroups share: runs of some with shares and
+    of one without in a workgroup's rows, a share of kept keys, shares without a
+    key that a row sees, a sink that counts once also where share 0 has none."""
+    g = torch.Generator().manual_seed(31)
+    bs, L = 16, 1100
+    kc, vc, tables = _paged(L, G, D, DV, bs, torch.bfloat16, g, 2)
+    ts, tp = [], []
+    for s, a, b in ((0, 940, 985), (1, 0, 7), (1, 1090, 1100), (0, 31, 34)):
+        ts += [s] * (b - a)
+        tp += list(range(a, b))
+    T = len(ts)
+    q = torch.randn(T, H * D, generator=g).to(torch.bfloat16)
+    sinks = torch.randn(H, generator=g) * 2
+    ts, tp = (torch.tensor(x, dtype=torch.int32) for x in (ts, tp))
+    want = reference.talk_attention(
+        q.float().reshape(T, H, D), kc.float(), vc.float(), tables, ts, tp,
+        D ** -0.5, 0, window, True, None, keep, softcap, sinks)
+    got = ops.talk_attention(
+        *[x.cuda() for x in (q, kc, vc, tables, ts, tp)], D ** -0.5, H,
+        window=window, sink=True, softcap=softcap, variant=11,
+        keep_first=keep, sink_vals=sinks.cuda(), splits=splits)
+    # fp32 up to the bf16 rounding of the result
+    assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
