@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
     m = i < 64 ? start1 : i < 127 ? start1 & (~1ull << (i - 64)) : 0;
     return m ? __ffsll(m) + 63 : ntok;
   };
-  int rs = 0, my_eff = 1;
+  int rs = 0, my_eff = 1, my_ks = ks, from = 0;
   while (rs < ntok) {
     // batch rows rs .. re - 1 continue one sequence
     const int re = next_start(rs);
@@ -164,15 +164,24 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
     const int k0 = min(a.keep, kmin);
     const int nt0 = (k0 + WA_KT - 1) / WA_KT;
     const int all = nt0 + (kmax - kmin) / WA_KT + 1;
-    // the workgroups that have a share of these tiles, and this one's
+    // the workgroups that have a share of these tiles (from behind those of the run
+    // before on, so that short runs are not all the first one's), and this one's
     const int eff = PART ? max(1, min(a.KS, all / WA_SHARE)) : 1;
-    if (PART && mine) my_eff = eff;
-    if (PART && ks >= eff) {
-      rs = re;
-      continue;
+    const int share = PART ? (ks >= from ? ks - from : ks - from + a.KS) : 0;
+    if (PART) {
+      from += eff;
+      if (from >= a.KS) from -= a.KS;
+      if (mine) {
+        my_eff = eff;
+        my_ks = share;
+      }
+      if (share >= eff) {
+        rs = re;
+        continue;
+      }
     }
-    const int n0 = PART ? all * ks / eff : 0;
-    const int nt = PART ? all * (ks + 1) / eff : all;
+    const int n0 = PART ? all * share / eff : 0;
+    const int nt = PART ? all * (share + 1) / eff : all;
     // rows of other runs see nothing of this one
     const int pos = mine ? my_pos : -1;
     const int ia = max(wave * 32 / HPB, rs);
@@ -320,9 +329,9 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
   }
 
   l += __shfl_xor(l, 32, 64);  // a lane summed its own keys
-  if (!valid || (PART && ks >= my_eff)) return;
+  if (!valid || (PART && my_ks >= my_eff)) return;
   float own = 1.f;
-  if (a.sink && (!PART || ks == 0)) {  // the sink is share 0's
+  if (a.sink && (!PART || my_ks == 0)) {  // the sink is share 0's
     const float sink = a.sink_vals != nullptr ? a.sink_vals[head] : 0.f;
     if (PART && m == KV_LOW) {  // none of its keys: the sink alone
       m = fminf(fmaxf(sink * KV_LOG2E, KV_LOW), -KV_LOW);
@@ -334,7 +343,7 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
   if constexpr (PART) {
     // partial record per (token, share, head): max (natural log units),
     // denominator, shares, one unused, DV sums
-    float* rec = a.part + (((size_t)tok * a.KS + ks) * a.H + head) *
+    float* rec = a.part + (((size_t)tok * a.KS + my_ks) * a.H + head) *
                               (size_t)(DV + WA_HEAD);
     if (hi == 0) {
       rec[0] = l != 0.f ? m * 0.69314718f : PS_NEG_INF;
@@ -657,8 +666,10 @@ int mx_window_attention(void* out, int ldout, const void* q, int ldq,
     // 5 behind 1000 356 -> 185 (366), 64 rows behind 2000 87 -> 81 (226). Down to
     // 16 rows, half a wave's: 344 -> 177, but 81 -> 97; up to 512 workgroups: 2
     // prompts of 2048, 8 heads of 40 60 -> 67. With shares of the keys whole ones fill
-    // the CUs (70 rows behind 2500 keys 28 us, 37 with fewer rows; four portions of
-    // 17 beside longer tables, which end up without shares, 20, 13 without them).
+    // the CUs (70 rows behind 2500 keys 26 us, 37 with fewer rows). Portions that
+    // end up without shares, runs of a workgroup's rows over the workgroups that share
+    // them: four of 17 11.4 (20 with all of them the first one's, 11.8 without
+    // shares), eight of 30 14.0 (12.0 without shares and their merge).
     a.tpt = 128 / a.hpb;
     a.KS = splits > 1 && scratch != nullptr ? splits : 1;
     if (a.KS > 16) return 1;

@@ -229,6 +229,12 @@ class TalkAttention(nn.Module):
         # (tiled kernel); single tokens of different sequences share
         # nothing and take the split-key kernel, one workgroup per token.
         npt = min(getattr(meta, "num_prefill_tokens", T) or 0, T)
+        # where the longest of the portions ends (0: not known), once a step
+        end = shared.get("portions_end") if shared is not None else 0
+        if end is None:
+            host = getattr(meta, "seq_rows_host", None) or ()
+            end = shared["portions_end"] = max(
+                (p0 + n for r0, n, p0, *_ in host if r0 < npt), default=0)
         for a, b, variant in ((0, npt, 0), (npt, T, 3)):
             if b > a:
                 ops.talk_attention(
@@ -239,7 +245,8 @@ class TalkAttention(nn.Module):
                     keep_first=sp.keep_first, softcap=sp.softcap,
                     sink_vals=self.sink_vals, pool=pool,
                     key_scale=key_scale, slopes=self.slopes(proj.device),
-                    score_bound=self.score_bound)
+                    score_bound=self.score_bound,
+                    longest=0 if a else end)
         if sp.out_gate:
             ops.gated_act(proj[:, self.qkv_rows:], out, "sigmoid", out=out)
         return out

@@ -724,8 +724,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
                    splits: int = 0, keep_first: int = 0,
                    softcap: float = 0.0, sink_vals: torch.Tensor = None,
                    vdim: int = 0, pool=None, key_scale: torch.Tensor = None,
-                   slopes: torch.Tensor = None,
-                   score_bound: float = 0.0) -> torch.Tensor:
+                   slopes: torch.Tensor = None, score_bound: float = 0.0,
+                   longest: int = 0) -> torch.Tensor:
     """Paged attention of a ragged batch. q [T, H*D] (row-strided view
     allowed); token_seq/token_pos int32 [T] give each token's block-table
     row and position; talk: optional fp32 [H, H] score mix; chunk/window:
@@ -743,7 +743,9 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     scores (neither comes with a head mix, a cap or pooled blocks).
     score_bound > 0: the caller knows that no scaled score exceeds it in
     magnitude before the distance term; kernels may then pass over keys whose
-    weight is below 2^-40 of the largest one.
+    weight is below 2^-40 of the largest one. longest > 0: no row of the
+    batch is at or behind that position; without it the tables' width stands
+    for it where workgroups are planned (a wrong number costs time only).
     variant 0 picks the kernel for prompt portions (tiled thread-per-
     (head, query) where the shape fits), 3 for single tokens (split-key),
     both falling back to the plain one-workgroup-per-token kernel; 1 / 2 /
@@ -815,6 +817,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         assert talk.is_contiguous()
     if pool is not None:
         assert kp.is_contiguous() and vp.is_contiguous()
+    width = block_tables.shape[1] * BS
+    longest = min(longest, width) if longest > 0 else width
     # single tokens: when the batch is too small to fill the chip with one
     # workgroup per token, each token's keys are shared out over several
     # workgroups whose partial softmax records are merged afterwards
@@ -877,7 +881,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # 4 shares, 20 in 16; 2 x 30001 260 whole, 48 in 8 and in 12; 8
             # x 1024 16 whole, 20 in 2; 16 x 4001 41 whole, 46 in 2)
             groups = T * G * ((H // G + 15) // 16)
-            keys = block_tables.shape[1] * BS
+            keys = longest
             if window > 0:
                 keys = min(keys, window + keep_first)
             shares = splits if splits > 0 else max(
@@ -888,11 +892,13 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # that are (us, 32/8 heads of 128, 128 (token, head) rows a workgroup
             # in 1 / 2 / 4 / 8 shares: 70 tokens behind 2500 keys 93 / 53 / 35 /
             # 28; 250 behind 2500 93 / 56 / 41 / 40; 559 behind 2500 93 / 74 / 71
-            # / 78; 1419 behind 2000 120 / 118 / 127 / 156)
+            # / 78; 1419 behind 2000 120 / 118 / 127 / 156). Planned by the longest
+            # row: where that is one of other rows, shorter ones pay for the
+            # merge's launch (100 rows alone 10.8, beside tables of 4000 14.1).
             rep = H // G
             tokens = 128 // rep if rep < 128 else 1
             groups = (T + tokens - 1) // tokens * G * ((rep + 127) // 128)
-            keys = block_tables.shape[1] * BS
+            keys = longest
             if window > 0:
                 keys = min(keys, window + keep_first)
             shares = splits if splits > 0 else max(
@@ -916,7 +922,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             and talk is None and not extra and pool is None):
         token = variant in (3, 14)
         rep = H // G
-        keys = block_tables.shape[1] * BS
+        keys = longest
         if window > 0:
             keys = min(keys, window + keep_first)
         if chunk > 0:
@@ -954,7 +960,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     # a head mix over prompt portions in fp32
     if (variant in (0, 16) and talk is not None and not extra and pool is None
             and keep_first == 0 and q.dtype == torch.float32):
-        keys = block_tables.shape[1] * BS
+        keys = longest
         if window > 0:
             keys = min(keys, window)
         if chunk > 0:
@@ -984,7 +990,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     # a head mix over single tokens
     if (variant in (3, 15) and talk is not None and not extra and pool is None
             and keep_first == 0):
-        keys = block_tables.shape[1] * BS
+        keys = longest
         if window > 0:
             keys = min(keys, window)
         if chunk > 0:
@@ -1044,7 +1050,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # 32 CUs (us, heads of 128, in 1 / 2 / 4 / 8: 132 rows, one portion behind
         # 2882 keys 140 / 90 / 64 / 52, in 12 75; 400 behind 1500 259 / 150 / 93 /
         # 112; 1349 behind 1463 279 / 205; 1800 in three prompts 101 / 118)
-        keys = block_tables.shape[1] * BS
+        keys = longest
         if window > 0:
             keys = min(keys, window)
         if chunk > 0:
