@@ -183,6 +183,12 @@ def _rows_before_norm(rows: int, N: int, K: int) -> bool:
     19.9, 112 22.0 / 20.0; 144 24.0 / 25.5; 80 x 5120 x 4096 25.2 / 21.4, 112 26.1 /
     27.7, 149 x 5376 x 4096 28.4 / 27.1; 80 x 6144 x 4096 25.9 / 27.5, 144 30.8 /
     43.8, 176 1.02 times.
+    Of few rows of W, long ones: 65 x 3072 x 8192 24.0 / 40.7, 112 26.6 / 30.9, 128 27.6
+    / 46.2, 192 32.7 / 62.5 (decode steps of a 3b-sized stack of five layers 67 869 ->
+    795, 128 1020 -> 942, 192 1270 -> 1135), but 160 31.0 / 31.8; 67 x 2048 x 8192 20.2
+    / 23.5 (65 598 -> 585). A step gains some 2 us a product less than these
+    differences: 100 x 2048 x 8192 22.0 / 23.8, but steps 763 -> 769, 128 23.0 / 24.1
+    and 796 -> 820; 160 x 3072 x 8192 993 -> 1005.
     Fewer: few rows of W (17 x 2048 x 2048 10.1 / 13.7, 63 x 2048 x 4096 14.2 / 15.0, 48
     x 2560 x 2048 13.5 / 14.8; 25 x 2048 x 1024 9.0 / 8.4, 60 x 1024 x 1280 up to 1.2
     times, 48 x 2560 x 2560 14.5 / 12.7), of more 64 x 4096 x 4096 17.6 / 18.6 and 32 x
@@ -197,6 +203,10 @@ def _rows_before_norm(rows: int, N: int, K: int) -> bool:
                 (rows >= 32 or (K % 2048 == 0 and
                                 (K >= 14336 or not 3072 < N < 4608))))
     if rows > 64:
+        if K >= 6144 and 2944 <= N < 3584:
+            return rows <= 128 or rows == 192
+        if K >= 7168 and 2048 <= N <= 2112:
+            return rows <= 72
         if not 3584 <= N <= 6144 or K < 4096:
             return False
         if whole or K >= 8192:
@@ -222,7 +232,16 @@ def _rows_before_rope(rows: int, N: int, K: int) -> bool:
     5120 35.6 / 36.6, 192 x 10240 x 3584 37.9 / 42.0, 144 x 8192 x 8192 47.4 / 50.4;
     past the lines 96 x 4608 x 3584 23.6 / 23.4, 144 x 4608 x 4096 27.3 / 25.5, 135 x
     5376 x 4096 28.7 / 26.4, 128 x 8192 x 4096 32.5 / 30.0, 144 34.9 / 29.2, 128 x 10240
-    x 3584 32.1 / 31.5."""
+    x 3584 32.1 / 31.5.
+    17 to 48 rows (decode steps of six layers 560 -> 546 and 643 -> 627), rows of W of
+    2048 entries, where ranges of K fill the CUs with
+    whole steps (up to 2048 rows of W, or a multiple of 1024): 17 x 2048 x 2048 10.3 /
+    14.2, 17 x 3072 x 2048 12.8 / 15.2, 32 13.7 / 15.3, 48 14.7 / 15.4, 48 x 5120 x 2048
+    15.5 / 16.1; past the lines 57 x 4096 x 2048 15.6 / 15.5, 45 x 2304 x 2048 17.2 /
+    14.8, 47 x 3008 x 2048 16.6 / 15.2, 32 x 1536 x 1536 12.2 / 10.1, 32 x 3072 x 2560
+    14.3 / 13.0."""
+    if 17 <= rows <= 48 and K == 2048:
+        return 1536 <= N <= 2048 or (N <= 5120 and N % 1024 == 0)
     if not 128 <= rows <= 192 or not 4608 <= N <= 10240 or K < 3584:
         return False
     if rows % 32 == 0:

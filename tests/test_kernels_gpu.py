@@ -1387,6 +1387,34 @@ def test_parts_dispatch(behind, M, N, K, own):
     assert gemm_policy.parts(x[:, :-64], w[:, :-64], behind) is None
 
 
+@pytest.mark.parametrize("behind,M,N,K,own", [
+    ("norm", 65, 2944, 6144, True), ("norm", 128, 3520, 6144, True),
+    ("norm", 192, 3072, 6144, True), ("norm", 129, 3072, 8192, False),
+    ("norm", 193, 3072, 8192, False), ("norm", 65, 3072, 6080, False),
+    ("norm", 65, 2880, 8192, False), ("norm", 72, 2048, 7168, True),
+    ("norm", 72, 2112, 8192, True), ("norm", 73, 2048, 8192, False),
+    ("norm", 72, 1984, 8192, False), ("norm", 72, 2048, 7104, False),
+    ("rope", 17, 1536, 2048, True), ("rope", 48, 2048, 2048, True),
+    ("rope", 48, 5120, 2048, True), ("rope", 49, 3072, 2048, False),
+    ("rope", 16, 3072, 2048, False), ("rope", 17, 2112, 2048, False),
+    ("rope", 17, 1472, 2048, False), ("rope", 17, 6144, 2048, False),
+    ("rope", 17, 3072, 2112, False)])
+def test_parts_dispatch_narrow(behind, M, N, K, own):
+    """As above for few rows of W, with what the partial sums add up to."""
+    from production_stack_amd.ops import gemm_policy
+
+    gemm_policy.reset()
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(N, K, generator=g, device="cuda").to(torch.bfloat16)
+    got = gemm_policy.parts(x, w, behind)
+    assert (got is not None) == own
+    if own:
+        want = x.double() @ w.double().t()
+        # fp32 sums of K terms
+        assert (got.double().sum(0) - want).norm() <= 1e-5 * want.norm()
+
+
 @pytest.mark.parametrize("M,N,K,own", [
     (17, 28160, 2048, True), (64, 32768, 2048, True), (65, 28672, 2048, False),
     (17, 28096, 2048, False), (17, 32832, 2048, False),
