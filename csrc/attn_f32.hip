@@ -29,6 +29,11 @@
 // 7430 -> 84; 80 rows behind 334 keys 1360 -> 21; 1000 rows of 64 in 3 prompts 562 ->
 // 37; 1000 rows 122, half the fp32 matrix rate; one token behind 947 keys 345 -> 19;
 // 64 behind 1500 157, 5.1 TB/s.
+// Errors against 64 bits are those of the vector kernels or less (40 tokens of up to 900
+// keys 2.3e-7 and 2.1e-7, 128 of up to 300 2.1e-7 and 2.0e-7, 1000 rows behind 3000
+// 1.1e-6 and 4.9e-7): sums are short chains that are added up, scores by 16 entries,
+// outputs by tiles (40 tokens with outputs in one chain over all keys and scores by 32
+// 3.3e-7 and 78.7 us, 79.8 so).
 #include "attn_common.h"
 
 struct AfArgs {
@@ -61,7 +66,8 @@ PS_DEV bool af_odd(float x) { return !(fabsf(x) < INFINITY); }
 template <int NT, int NV, int NC, bool CAP>
 __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
   constexpr int COLS = 16 * NC, PA = NV * 64 + 4;
-  constexpr int NS = NC * NT > 8 ? 2 : 4;  // sums of a score; more would spill
+  constexpr int NS = NC * NT > 8 ? 2 : NT;  // sums of a score; more would spill
+  constexpr bool APART = NC == 1;
   extern __shared__ __align__(16) float sA[];  // [4][COLS][PA]: the merge
   __shared__ float s_m[4][COLS], s_l[4][COLS];
   __shared__ int s_seq[COLS], s_pos[COLS];
@@ -204,9 +210,14 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               const int j = j0 + i;
-              float x = st[c][0][i] + st[c][1][i];
-              if constexpr (NS == 4) x += st[c][2][i] + st[c][3][i];
-              x *= a.scale;
+              float y[NS];
+#pragma unroll
+              for (int s = 0; s < NS; ++s) y[s] = st[c][s][i];
+#pragma unroll
+              for (int w = NS / 2; w > 0; w /= 2)
+#pragma unroll
+                for (int s = 0; s < w; ++s) y[s] += y[s + w];
+              float x = y[0] * a.scale;
               if constexpr (CAP) x = a.cap * tanhf(x / a.cap);
               const bool vis = mine && j <= min(end, my_pos[c]) &&
                                (j >= my_lo[c] || j < a.keep);
@@ -228,9 +239,9 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               p[i] = expf(p[i] - m[c]);
-              l[c] += p[i];
               st[c][0][i] = p[i];
             }
+            l[c] += (p[0] + p[1]) + (p[2] + p[3]);
           }
           if (careful) {
 #pragma unroll 1
@@ -268,6 +279,9 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
                 for (int e = 0; e < 4; ++e)
                   if (af_odd((&vf[i][h].x)[e])) (&vf[i][h].x)[e] = 0.f;
           }
+          // a tile's products on their own where registers allow: added one by
+          // one to the sums of all tiles before, roundings grow with their number
+          kv_f32x4 sum[NC][NV][4];
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -275,9 +289,21 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
 #pragma unroll
               for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int c = 0; c < NC; ++c)
-                  acc[c][h][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                      (&vf[i][h].x)[e], st[c][0][i], acc[c][h][e], 0, 0, 0);
+                for (int c = 0; c < NC; ++c) {
+                  kv_f32x4& to = APART ? sum[c][h][e] : acc[c][h][e];
+                  const kv_f32x4 from =
+                      APART && i == 0 ? kv_f32x4{0.f, 0.f, 0.f, 0.f} : to;
+                  to = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                      (&vf[i][h].x)[e], st[c][0][i], from, 0, 0, 0);
+                }
+          if constexpr (APART) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+              for (int h = 0; h < NV; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[c][h][e] += sum[c][h][e];
+          }
         }
       }
       rs = re;

@@ -59,9 +59,13 @@ struct TtArgs {
 
 PS_DEV bool tt_odd(float x) { return !(fabsf(x) < INFINITY); }
 
-// How far a score may be above the one that set the reference that weights are
-// relative to, before it moves; the reference is as much above it, so that no weight
-// is above 1. Moving it is a product per sum.
+// How far a score of bf16 rows may be above the one that set the reference that weights
+// are relative to, before it moves; the reference is as much above it, so that no weight
+// is above 1. Moving it is a product per sum. fp32 rows take the maximum itself: the
+// distance of the largest scores to a reference above them is rounded (single tokens,
+// errors against 64 bits 5.2e-7 so and 3.6e-7, the vector kernel's 4.6e-7; four sums of a
+// score and two of a mix for two and one among it; 142 -> 148 us for 64 of up to 2250
+// keys, portions 64 -> 67).
 #define TT_FAR 8.f
 
 // What a lane has of a tile, in 16-byte pieces of P entries: KF of key n for a KV head,
@@ -209,20 +213,23 @@ __global__ __launch_bounds__(512, 2) void talk_token_kernel(TtArgs a) {
     kv_f32x4 sc[2], x;
 #pragma unroll
     for (int s = 0; s < KB; ++s) {
-      // sums of every other piece: shorter chains of roundings
-      kv_f32x4 st[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      // sums of every other piece (fourth one): shorter chains of roundings
+      constexpr int NS = BF ? 2 : 4;
+      kv_f32x4 st[NS];
+#pragma unroll
+      for (int f = 0; f < NS; ++f) st[f] = kv_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int f = 0; f < KF; ++f) {
         if constexpr (BF) {
-          st[f & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          st[f % NS] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               __builtin_bit_cast(tt_bf16x8, qf[f]),
-              __builtin_bit_cast(tt_bf16x8, kb[s][f]), st[f & 1], 0, 0, 0);
+              __builtin_bit_cast(tt_bf16x8, kb[s][f]), st[f % NS], 0, 0, 0);
         } else {
           const float4 q = *(const float4*)(sq + 4 * f * P);
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            st[f & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                (&q.x)[e], __uint_as_float((&kb[s][f].x)[e]), st[f & 1], 0, 0,
+            st[f % NS] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                (&q.x)[e], __uint_as_float((&kb[s][f].x)[e]), st[f % NS], 0, 0,
                 0);
         }
       }
@@ -230,7 +237,11 @@ __global__ __launch_bounds__(512, 2) void talk_token_kernel(TtArgs a) {
       fetch_k(s, next);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        sc[0][i] = s == 0 || g == KB * sp + s ? st[0][i] + st[1][i] : sc[0][i];
+        sc[0][i] = s == 0 || g == KB * sp + s
+                       ? (BF ? st[0][i] + st[1][i]
+                             : (st[0][i] + st[1][i]) +
+                                   (st[NS - 2][i] + st[NS - 1][i]))
+                       : sc[0][i];
     }
     if (SP == 1 || g / KB == sp) s_sc[turn][grp][hf][lane] = sc[0];
     __syncthreads();
@@ -239,12 +250,13 @@ __global__ __launch_bounds__(512, 2) void talk_token_kernel(TtArgs a) {
     turn ^= 1;
     // mixed scores: keys 4 g + i of head 16 hf + n
     x = kv_f32x4{0.f, 0.f, 0.f, 0.f};
+    kv_f32x4 y = x;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        x = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[h][i], tb[h][i], x, 0, 0,
-                                                 0);
+    for (int i = 0; i < 4; ++i) {
+      x = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[0][i], tb[0][i], x, 0, 0, 0);
+      y = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[1][i], tb[1][i], y, 0, 0, 0);
+    }
+    x += y;
     const int left = pos - lo - t * 16 - 4 * g;  // keys 4 g + i up to this i
     float mx = PS_NEG_INF;
 #pragma unroll
@@ -257,7 +269,7 @@ __global__ __launch_bounds__(512, 2) void talk_token_kernel(TtArgs a) {
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     if (__any(mx > m)) {
-      const float mn = mx > m ? mx + TT_FAR : m;
+      const float mn = mx > m ? (BF ? mx + TT_FAR : mx) : m;
       const float al = expf(m - mn);
       m = mn;
       l *= al;
@@ -534,7 +546,7 @@ __global__ __launch_bounds__(512, 2) void talk_rows_f32_kernel(TtArgs a) {
           mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
           mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
           if (__any(mx > m[q])) {
-            const float mn = mx > m[q] ? mx + TT_FAR : m[q];
+            const float mn = fmaxf(mx, m[q]);
             const float al = expf(m[q] - mn);
             m[q] = mn;
             l[q] *= al;
