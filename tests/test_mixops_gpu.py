@@ -1372,3 +1372,26 @@ def test_window_attention_portion_shares(H, G, D, DV, window, keep, softcap,
         keep_first=keep, sink_vals=sinks.cuda(), splits=splits)
     # fp32 up to the bf16 rounding of the result
     assert _rel(got.float().cpu().reshape(T, H, DV), want) < 3e-3
+
+
+@pytest.mark.parametrize("talk", [False, True])
+@pytest.mark.parametrize("longest", [0, 1, 130, 2000])
+def test_attention_longest_hint(talk, longest):
+    """Where the longest portion ends only plans the workgroups: unknown, too
+    small, as it is, beyond the tables."""
+    g = torch.Generator().manual_seed(33)
+    H, G, D, bs, L = 32, 8, 64, 16, 1500
+    kc, vc, tables = _paged(L, G, D, D, bs, torch.bfloat16, g, 2)
+    ts = torch.tensor([0] * 40 + [1] * 17, dtype=torch.int32)
+    tp = torch.cat([torch.arange(90, 130), torch.arange(17)]).int()
+    T = len(ts)
+    q = torch.randn(T, H * D, generator=g).to(torch.bfloat16)
+    mix = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g) if talk else None
+    want = reference.talk_attention(
+        q.float().reshape(T, H, D), kc.float(), vc.float(), tables, ts, tp,
+        D ** -0.5, 0, 0, True, mix)
+    got = ops.talk_attention(
+        *[x.cuda() for x in (q, kc, vc, tables, ts, tp)], D ** -0.5, H,
+        sink=True, talk=mix.cuda() if talk else None, longest=longest)
+    # fp32 up to the bf16 rounding of the result
+    assert _rel(got.float().cpu().reshape(T, H, D), want) < 3e-3
