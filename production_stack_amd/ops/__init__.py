@@ -817,7 +817,13 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         assert talk.is_contiguous()
     if pool is not None:
         assert kp.is_contiguous() and vp.is_contiguous()
+    # Keys of the longest portion: where nobody says, the tables' width, but beside
+    # more tables than portions usually are (a decode batch's) only the rows here. Too
+    # many shares cost a launch for their merge (window attention, 100 rows of 1
+    # sequence and 40 tokens of up to 3000 keys 85.6 -> 89.7 us in all).
     width = block_tables.shape[1] * BS
+    portion = (min(longest, width) if longest > 0 else
+               width if block_tables.shape[0] <= 4 else min(T, width))
     longest = min(longest, width) if longest > 0 else width
     # single tokens: when the batch is too small to fill the chip with one
     # workgroup per token, each token's keys are shared out over several
@@ -892,17 +898,24 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # that are (us, 32/8 heads of 128, 128 (token, head) rows a workgroup
             # in 1 / 2 / 4 / 8 shares: 70 tokens behind 2500 keys 93 / 53 / 35 /
             # 28; 250 behind 2500 93 / 56 / 41 / 40; 559 behind 2500 93 / 74 / 71
-            # / 78; 1419 behind 2000 120 / 118 / 127 / 156). Planned by the longest
-            # row: where that is one of other rows, shorter ones pay for the
-            # merge's launch (100 rows alone 10.8, beside tables of 4000 14.1).
+            # / 78; 1419 behind 2000 120 / 118 / 127 / 156). A tile takes 2.2 us at
+            # widths of 128, records their write and read and their merge 3 us: as
+            # many shares as make the least of both, none where that is not a fifth
+            # less (200 rows behind 200 20.6 us whole, 22.0 in 2).
             rep = H // G
             tokens = 128 // rep if rep < 128 else 1
             groups = (T + tokens - 1) // tokens * G * ((rep + 127) // 128)
-            keys = longest
+            keys = portion
             if window > 0:
                 keys = min(keys, window + keep_first)
-            shares = splits if splits > 0 else max(
-                1, min(16, 512 // groups, keys // 192))
+            shares = splits if splits > 0 else min(16, 512 // groups, keys // 192)
+            if splits <= 0 and shares > 1:
+                walk = keys / 64 * 2.2 * (D + DV) / 256
+                record = T * H * (DV + 4) * 1.6e-6
+                shares = min(shares, int((walk / record) ** 0.5))
+                if shares < 2 or walk / shares + record * shares + 3 > 0.8 * walk:
+                    shares = 1
+            shares = max(1, shares)
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
                             device=q.device) if shares > 1 else None)
         rc = _mx().mx_window_attention(
@@ -1049,15 +1062,18 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # each at least: a block of rows' two workgroups are one XCD's, which has
         # 32 CUs (us, heads of 128, in 1 / 2 / 4 / 8: 132 rows, one portion behind
         # 2882 keys 140 / 90 / 64 / 52, in 12 75; 400 behind 1500 259 / 150 / 93 /
-        # 112; 1349 behind 1463 279 / 205; 1800 in three prompts 101 / 118)
-        keys = longest
+        # 112; 1349 behind 1463 279 / 205; 1800 in three prompts 101 / 118). Two
+        # rounds of the CUs only where few rows see most keys (1200 rows 169 / 109, in
+        # three prompts 69 / 82).
+        keys = portion
         if window > 0:
             keys = min(keys, window)
         if chunk > 0:
             keys = min(keys, chunk)
         blocks = (T + 127) // 128           # of an XCD
         shares = asked if asked > 0 else max(1, min(
-            16 // blocks if blocks < 8 else 2 if blocks < 12 else 1,
+            16 // blocks if blocks <= 8 else
+            2 if blocks < 12 and 5 * keys >= 4 * T else 1,
             keys // 64))
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
                             device=q.device) if shares > 1 else None)
