@@ -825,6 +825,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     portion = (min(longest, width) if longest > 0 else
                width if block_tables.shape[0] <= 4 else min(T, width))
     longest = min(longest, width) if longest > 0 else width
+    rows = max(T, 1)  # what workgroups are planned for: kernels return at no rows
     # single tokens: when the batch is too small to fill the chip with one
     # workgroup per token, each token's keys are shared out over several
     # workgroups whose partial softmax records are merged afterwards
@@ -833,7 +834,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             and not extra and v_cache.data_ptr() == k_cache.data_ptr() and talk is None
             and chunk == 0 and keep_first == 0 and softcap == 0.0):
         shares = splits if splits > 0 else max(
-            1, min(16 if T <= 4 else 8, 256 // (T * ((H + 31) // 32))))
+            1, min(16 if T <= 4 else 8, 256 // (rows * ((H + 31) // 32))))
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
                             device=q.device) if shares > 1 else None)
         rc = _mx().mx_latent_decode(
@@ -856,7 +857,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         if token:
             # enough workgroups to fill the chip, a share being at least one
             # tile of rows per wave
-            groups = T * G * ((H // G + 15) // 16)
+            groups = rows * G * ((H // G + 15) // 16)
             shares = splits if splits > 0 else max(
                 1, min(16, 1024 // groups,
                        (window + 127) // 128 if window > 0 else 16))
@@ -886,7 +887,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # start (32/8 heads of 128: 1 token x 4001 keys 39 us whole, 19 in
             # 4 shares, 20 in 16; 2 x 30001 260 whole, 48 in 8 and in 12; 8
             # x 1024 16 whole, 20 in 2; 16 x 4001 41 whole, 46 in 2)
-            groups = T * G * ((H // G + 15) // 16)
+            groups = rows * G * ((H // G + 15) // 16)
             keys = longest
             if window > 0:
                 keys = min(keys, window + keep_first)
@@ -904,14 +905,14 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # less (200 rows behind 200 20.6 us whole, 22.0 in 2).
             rep = H // G
             tokens = 128 // rep if rep < 128 else 1
-            groups = (T + tokens - 1) // tokens * G * ((rep + 127) // 128)
+            groups = (rows + tokens - 1) // tokens * G * ((rep + 127) // 128)
             keys = portion
             if window > 0:
                 keys = min(keys, window + keep_first)
             shares = splits if splits > 0 else min(16, 512 // groups, keys // 192)
             if splits <= 0 and shares > 1:
                 walk = keys / 64 * 2.2 * (D + DV) / 256
-                record = T * H * (DV + 4) * 1.6e-6
+                record = rows * H * (DV + 4) * 1.6e-6
                 shares = min(shares, int((walk / record) ** 0.5))
                 if shares < 2 or walk / shares + record * shares + 3 > 0.8 * walk:
                     shares = 1
@@ -943,16 +944,16 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # 32 columns a wave where those fill the chip twice, else 16 (32/8 heads,
         # us, 16 / 32: 1000 rows of 128 alone 125 / 122, behind 3000 keys 258 /
         # 234; 400 rows 26.7 / 28.1; 1000 of 64 37.4 / 43.3)
-        rows = 16
+        cols = 16
         if not token and rep <= 32 and max(D, DV) > 64 and (
                 (T + 32 // rep - 1) // (32 // rep) * G >= 512):
-            rows = 32
+            cols = 32
         # Several workgroups for a tile's keys where CUs are left: records cost 3
         # us and 4 bytes a share and entry (1 token x 947 keys 46 us whole, 18.6
         # in 8 shares; 64 x 1500 162, 157 in 3, 193 in 12; 8 x 300 19.0, 14.5 in
         # 4; portions: 80 rows behind 334 keys 20.9, 23.9 in 2)
-        tpt = 1 if token else max(1, rows // rep)
-        groups = (T + tpt - 1) // tpt * G
+        tpt = 1 if token else max(1, cols // rep)
+        groups = (rows + tpt - 1) // tpt * G
         shares = splits if splits > 0 else max(1, min(
             16, (512 if token else 256) // groups,
             keys // (128 if token else 256)))
@@ -963,7 +964,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             _p(v_cache), _p(block_tables), block_tables.shape[1],
             _p(token_seq), _p(token_pos), T, H, G, D, DV, BS, _f(scale),
             int(chunk), int(window), int(bool(sink)), int(keep_first),
-            _f(softcap), _p(sink_vals), int(VR), int(token), int(rows),
+            _f(softcap), _p(sink_vals), int(VR), int(token), int(cols),
             int(shares), _p(part), _stream())
         if rc == 0:
             return out
@@ -983,7 +984,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # rows behind 817 keys in 1 / 6 / 12 shares 277 / 71 / 81; 254, of which 85
         # behind 1800, in 1 / 4 / 8 528 / 159 / 111; 1000 in 1 / 2 / 4 286 / 188 /
         # 208; 70 in 1 / 4 33 / 25), a tile of keys each at least
-        groups = (T + 3) // 4
+        groups = (rows + 3) // 4
         shares = splits if splits > 0 else max(1, min(
             16, (256 if groups <= 48 else 512) // groups, keys // 16))
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
@@ -1011,7 +1012,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # one workgroup a CU (bf16 64 tokens of up to 2250 keys in 1 / 2 / 4 / 8
         # shares 215 / 120 / 78 / 86 us), 48 keys each at least
         shares = splits if splits > 0 else max(
-            1, min(16, 256 // T, keys // 48))
+            1, min(16, 256 // rows, keys // 48))
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
                             device=q.device) if shares > 1 else None)
         rc = _mx().mx_talk_token(
@@ -1030,7 +1031,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if variant not in (3, 4, 5, 6):
         splits = 1
     elif splits <= 0:
-        splits = (max(1, min(8, 512 // T))
+        splits = (max(1, min(8, 512 // rows))
                   if T < 256 and variant not in (5, 6) else 1)
     if splits > 1:
         scratch = torch.empty((T, splits, H, DV + 2),
@@ -1070,7 +1071,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             keys = min(keys, window)
         if chunk > 0:
             keys = min(keys, chunk)
-        blocks = (T + 127) // 128           # of an XCD
+        blocks = (rows + 127) // 128         # of an XCD
         shares = asked if asked > 0 else max(1, min(
             16 // blocks if blocks <= 8 else
             2 if blocks < 12 and 5 * keys >= 4 * T else 1,

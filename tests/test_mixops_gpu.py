@@ -1395,3 +1395,19 @@ def test_attention_longest_hint(talk, longest):
         sink=True, talk=mix.cuda() if talk else None, longest=longest)
     # fp32 up to the bf16 rounding of the result
     assert _rel(got.float().cpu().reshape(T, H, D), want) < 3e-3
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("talk", [False, True])
+@pytest.mark.parametrize("variant", [0, 3])
+def test_attention_no_rows(dtype, talk, variant):
+    """An empty batch has an empty result, whatever kernel would take it."""
+    H, G, D, bs = 32, 8, 64, 16
+    kc = torch.zeros(4, G, bs, D, dtype=dtype, device="cuda")
+    none = torch.empty(0, dtype=torch.int32, device="cuda")
+    mix = torch.eye(H, device="cuda") if talk else None
+    out = ops.talk_attention(
+        torch.empty(0, H * D, dtype=dtype, device="cuda"), kc, kc.clone(),
+        torch.zeros(2, 4, dtype=torch.int32, device="cuda"), none, none,
+        D ** -0.5, H, sink=True, talk=mix, variant=variant)
+    assert out.shape == (0, H * D) and out.dtype == dtype
