@@ -50,7 +50,7 @@ struct AfArgs {
   float scale, cap;  // cap 0: none
   int chunk, window, keep, sink;
   const float* sink_vals;  // per head (nullptr: score 0)
-  int hide;                // scores that are no number count as hidden
+  int hide;                // scores that are no number hide their keys
   int tpt;                 // tokens per workgroup
   int KS;
   float* part;  // [T, KS, H, DV + AF_HEAD]
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
   kv_f32x4 acc[NC][NV][4];
   // The walk; again, `careful`, where values that are not finite were met: they
   // stay out of the products, in which a hidden key's weight of zero would carry
-  // them to columns that do not see it, and join those that do.
+  // them to columns that do not see it, and join those that do with their weights.
   bool careful = false;
 #pragma unroll 1
   for (;;) {
@@ -203,6 +203,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
           // scores: lane (g, n) has keys 4 g + i of column n
           const int j0 = first(t) + 4 * g;
           const int end = t < nt0 ? k0 - 1 : kmax;
+          bool seen[NC][4];
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             const bool mine = my_i[c] >= rs && my_i[c] < re;
@@ -221,7 +222,8 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
               if constexpr (CAP) x = a.cap * tanhf(x / a.cap);
               const bool vis = mine && j <= min(end, my_pos[c]) &&
                                (j >= my_lo[c] || j < a.keep);
-              p[i] = vis && !(a.hide && x != x) ? x : -INFINITY;
+              seen[c][i] = vis && (x > PS_NEG_INF || !a.hide);
+              p[i] = seen[c][i] ? x : -INFINITY;
               mx = fmaxf(mx, p[i]);
             }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -246,16 +248,18 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
           if (careful) {
 #pragma unroll 1
             for (int k = 0; k < AF_KT; ++k) {
-              const int j = first(t) + k;
               const float* vp = a.vc + (int64_t)__shfl(here, k, 64) * a.vr;
               int d0 = 16 * g;  // not known ahead: addresses are made here
               asm volatile("" : "+v"(d0));
-              bool vis[NC];
+              float w[NC];  // weights of key k, below 0 where it is hidden
 #pragma unroll
-              for (int c = 0; c < NC; ++c)
-                vis[c] = my_i[c] >= rs && my_i[c] < re &&
-                         j <= min(end, my_pos[c]) &&
-                         (j >= my_lo[c] || j < a.keep);
+              for (int c = 0; c < NC; ++c) {
+                float own = -1.f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                  if ((k & 3) == i && seen[c][i]) own = st[c][0][i];
+                w[c] = __shfl(own, k / 4 * 16 + n, 64);
+              }
 #pragma unroll
               for (int h = 0; h < NV; ++h)
 #pragma unroll
@@ -266,8 +270,8 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
                   for (int e = 0; e < 4; ++e)
 #pragma unroll
                     for (int c = 0; c < NC; ++c)
-                      if (vis[c] && af_odd((&x.x)[e]))
-                        acc[c][h][e][i] += (&x.x)[e];
+                      if (!(w[c] < 0.f) && af_odd((&x.x)[e]))
+                        acc[c][h][e][i] += w[c] * (&x.x)[e];
                   __builtin_amdgcn_sched_barrier(0);
                 }
             }

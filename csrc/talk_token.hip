@@ -379,7 +379,7 @@ __global__ __launch_bounds__(512, 2) void talk_token_kernel(TtArgs a) {
 // behind 334 1800 -> 39; of 64 2460 -> 47, 2550 -> 121, 1010 -> 27.
 // Hidden keys of a row have weights of zero, which values that are not finite would
 // carry into its sums; where sums are not finite the walk goes again with those kept
-// out of the products and added to the rows that see them.
+// out of the products and added, weighted, to the rows that see them.
 template <int D, int DV>
 __global__ __launch_bounds__(512, 2) void talk_rows_f32_kernel(TtArgs a) {
   constexpr int KF = D / 16, P = 4;
@@ -518,6 +518,7 @@ __global__ __launch_bounds__(512, 2) void talk_rows_f32_kernel(TtArgs a) {
         __syncthreads();
         const int j0 = kmin + t * 16 + 4 * g;
         float x[TW][4];
+        bool seen[TW][4];
 #pragma unroll
         for (int q = 0; q < TW; ++q) {
           const int r = r0 + q;
@@ -539,8 +540,9 @@ __global__ __launch_bounds__(512, 2) void talk_rows_f32_kernel(TtArgs a) {
           for (int i = 0; i < 4; ++i) {
             float v = y[i];
             if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
-            // no number counts as hidden
-            x[q][i] = j0 + i >= my_lo[q] && j0 + i <= hi && v == v ? v : -INFINITY;
+            // a score that is no number hides its key
+            seen[q][i] = j0 + i >= my_lo[q] && j0 + i <= hi && v > PS_NEG_INF;
+            x[q][i] = seen[q][i] ? v : -INFINITY;
             mx = fmaxf(mx, x[q][i]);
           }
           mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -568,16 +570,21 @@ __global__ __launch_bounds__(512, 2) void talk_rows_f32_kernel(TtArgs a) {
         if (careful) {
 #pragma unroll
           for (int q = 0; q < TW; ++q) {
-            const int r = r0 + q;
-            const int hi = r >= rs && r < re ? my_pos[q] : -1;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i) {
+              // weights of the four heads, below 0 where the key is hidden
+              const float own = seen[q][i] ? x[q][i] : -1.f;
+              float w[4];
+#pragma unroll
+              for (int u = 0; u < 4; ++u) w[u] = tt_quad(own, u);
 #pragma unroll
               for (int e = 0; e < NE; ++e) {
                 const float v = (&vb[i][e / P].x)[e % P];
-                if (tt_odd(v) && j0 + i >= my_lo[q] && j0 + i <= hi)
-                  acc[q][e] += v;
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                  if (tt_odd(v) && !(w[u] < 0.f)) acc[q][e][u] += w[u] * v;
               }
+            }
           }
 #pragma unroll
           for (int i = 0; i < 4; ++i)

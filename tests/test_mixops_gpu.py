@@ -1411,3 +1411,46 @@ def test_attention_no_rows(dtype, talk, variant):
         torch.zeros(2, 4, dtype=torch.int32, device="cuda"), none, none,
         D ** -0.5, H, sink=True, talk=mix, variant=variant)
     assert out.shape == (0, H * D) and out.dtype == dtype
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("case", ["key", "key and value", "far", "query",
+                                  "infinite key"])
+@pytest.mark.parametrize("talk,variant,general", [
+    (False, 13, 2), (False, 14, 4), (True, 16, 2), (True, 15, 4)])
+def test_attention_fp32_scores_no_number(talk, variant, general, case, splits):
+    """Scores that are no number, and values that are none behind a weight of
+    zero, do what they do in the vector kernels: they hide their key in portions,
+    whatever its value is, and reach the single tokens that see it."""
+    g = torch.Generator().manual_seed(21)
+    H, G, D, bs, L = 32, 8, 64, 16, 150
+    kc, vc, tables = _paged(L, G, D, D, bs, torch.float32, g, 2)
+    tp = torch.tensor([*range(40), *range(100, 150)], dtype=torch.int32)
+    ts = torch.tensor([0] * 40 + [1] * 50, dtype=torch.int32)
+    q = torch.randn(len(tp), H * D, generator=g)
+    mix = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)
+    nan, inf = float("nan"), float("inf")
+    page, row = tables[1, 7], 9         # position 121 of sequence 1
+    if case in ("key", "key and value"):
+        kc[page, :, row, 3] = nan
+    if case == "key and value":
+        vc[page, :, row] = nan
+    if case == "far":                   # exp of some -1000
+        q, kc, mix = q.abs(), kc.abs(), torch.eye(H)
+        kc[page, :, row] = -300.0
+        vc[page, :, row, 5] = inf
+    if case == "query":
+        q[60, :D] = nan
+    if case == "infinite key":
+        q, mix = q.abs(), mix.abs()
+        kc[page, :, row, 3] = -inf
+        vc[page, :, row] = nan
+    args = [x.cuda() for x in (q, kc, vc, tables, ts, tp)]
+    want, got = (ops.talk_attention(
+        *args, D ** -0.5, H, sink=True, talk=mix.cuda() if talk else None,
+        variant=v, splits=s) for v, s in ((general, 1), (variant, splits)))
+    assert torch.equal(torch.isnan(want), torch.isnan(got))
+    fin = torch.isfinite(want)
+    assert torch.equal(fin, torch.isfinite(got))
+    # fp32 sums of up to 150 and 128 terms on both sides
+    assert _rel(got[fin], want[fin]) < 4e-6
