@@ -35,6 +35,18 @@ from production_stack_amd.ops import gemm_policy
 DELTA_DECAY_SCALE = math.exp(-0.5)
 
 
+def _portions_end(meta, npt: int, shared: Optional[dict]) -> int:
+    """Where the longest of a step's prompt portions, its first npt rows, ends (0:
+    not known). Looked up once a step."""
+    end = shared.get("portions_end") if shared is not None else None
+    if end is None:
+        host = getattr(meta, "seq_rows_host", None) or ()
+        end = max((p0 + n for r0, n, p0, *_ in host if r0 < npt), default=0)
+        if shared is not None:
+            shared["portions_end"] = end
+    return end
+
+
 class TalkAttention(nn.Module):
     """Grouped-query softmax attention over the paged KV cache with the
     MixerSpec's options: score mixing across heads, aligned-chunk /
@@ -229,12 +241,7 @@ class TalkAttention(nn.Module):
         # (tiled kernel); single tokens of different sequences share
         # nothing and take the split-key kernel, one workgroup per token.
         npt = min(getattr(meta, "num_prefill_tokens", T) or 0, T)
-        # where the longest of the portions ends (0: not known), once a step
-        end = shared.get("portions_end") if shared is not None else 0
-        if end is None:
-            host = getattr(meta, "seq_rows_host", None) or ()
-            end = shared["portions_end"] = max(
-                (p0 + n for r0, n, p0, *_ in host if r0 < npt), default=0)
+        end = _portions_end(meta, npt, shared)
         for a, b, variant in ((0, npt, 0), (npt, T, 3)):
             if b > a:
                 ops.talk_attention(
@@ -246,7 +253,7 @@ class TalkAttention(nn.Module):
                     sink_vals=self.sink_vals, pool=pool,
                     key_scale=key_scale, slopes=self.slopes(proj.device),
                     score_bound=self.score_bound,
-                    longest=0 if a else end)
+                    longest=end if variant == 0 else 0)
         if sp.out_gate:
             ops.gated_act(proj[:, self.qkv_rows:], out, "sigmoid", out=out)
         return out
@@ -529,7 +536,9 @@ class LatentAttention(nn.Module):
                     meta.token_seq[a:b], meta.positions[a:b], self.scale, H,
                     window=sp.window, sink=sp.sink, out=o_lat[a - n:b - n],
                     variant=variant, softcap=sp.softcap,
-                    sink_vals=self.sink_vals, vdim=L)
+                    sink_vals=self.sink_vals, vdim=L,
+                    longest=(_portions_end(meta, npt, shared)
+                             if variant == 0 else 0))
         # expand the attended latents per head: [H, T, L] x [H, L, DV]
         ops.merge_heads(
             torch.bmm(o_lat.view(m, H, L).transpose(0, 1), self.uv),
@@ -575,8 +584,8 @@ class GeneralDelta(nn.Module):
         return ("state", self.H, self.D, self.D)
 
     def forward_from_proj(self, proj: torch.Tensor, meta, cache,
-                          out: Optional[torch.Tensor] = None
-                          ) -> torch.Tensor:
+                          out: Optional[torch.Tensor] = None,
+                          shared: Optional[dict] = None) -> torch.Tensor:
         HD = self.H * self.D
         r = proj[:, 0:HD]
         k = proj[:, HD:2 * HD]

@@ -164,8 +164,10 @@ class NanuraxLayer(nn.Module):
                 [self.mixer.out_weight.data, self.mlp.down.data],
                 dim=1).contiguous()
 
-    def forward(self, h: torch.Tensor, meta, cache) -> List[torch.Tensor]:
-        """h: normed input [T, width]. Returns the deltas that join the
+    def forward(self, h: torch.Tensor, meta, cache,
+                shared: Optional[dict] = None) -> List[torch.Tensor]:
+        """h: normed input [T, width]; shared: a dict of the step, in which its
+        layers find what one of them found out. Returns the deltas that join the
         residual stream (summed in fp32 by the next fused add+norm)."""
         if self.w_in is None:
             self.fuse()
@@ -178,10 +180,10 @@ class NanuraxLayer(nn.Module):
             cat = torch.empty((h.shape[0], mo + ff), dtype=h.dtype,
                               device=h.device)
             self.mixer.forward_from_proj(mproj, meta, cache,
-                                         out=cat[:, :mo])
+                                         out=cat[:, :mo], shared=shared)
             self.mlp.inner(fproj, out=cat[:, mo:])
             return [gemm_policy.linear(cat, self.w_out)]
-        mix = self.mixer.forward_from_proj(mproj, meta, cache)
+        mix = self.mixer.forward_from_proj(mproj, meta, cache, shared=shared)
         deltas = [gemm_policy.linear(mix, self.mixer.out_weight)]
         if self.mlp is not None:
             # routed feed-forward: fp32 sum of experts (+ shared), rounded
@@ -352,13 +354,14 @@ class NanuraxForCausalLM(nn.Module):
         cfg = self.cfg
         x = ops.embed_scale(token_ids, self.embed, cfg.embedding_scale)
         deltas: List[torch.Tensor] = []
+        shared: dict = {}
         hook = self.residual_hook
         for i, (layer, cache) in enumerate(zip(self.layers, caches)):
             h = ops.add_rms_norm32(x, deltas, layer.norm, cfg.rms_norm_eps,
                                    self.dtype)
             if hook is not None and i > 0:
                 hook(i - 1, x)
-            deltas = layer(h, meta, cache)
+            deltas = layer(h, meta, cache, shared)
         h = ops.add_rms_norm32(x, deltas, self.final_norm,
                                cfg.rms_norm_eps, self.dtype)
         if hook is not None:

@@ -392,3 +392,30 @@ def test_trace_run_command(ckpt, tmp_path):
                           .reshape(2, -1).copy())
     assert rel_err(g0, torch.stack([wa[0], wa[32], wb[6]])) < 2e-4
     assert rel_err(g2, torch.stack([wc[20], wa[39]])) < 2e-4
+
+
+def test_attention_is_told_where_portions_end(ckpt, monkeypatch):
+    """Every attention layer's portions know where the longest of a step's ends,
+    whichever comes first; its single tokens do not."""
+    from production_stack_amd import ops
+
+    path, _, _ = ckpt
+    eng = make_engine(path, "float32", "cpu")
+    calls = []
+    attend = ops.talk_attention
+
+    def record(*args, **kw):
+        calls.append((args[0].shape[0], kw["variant"], kw["longest"]))
+        return attend(*args, **kw)
+
+    monkeypatch.setattr(ops, "talk_attention", record)
+    steps = [[("a", 30, []), ("b", 9, [])],     # 0..29, 0..8
+             [("b", 5, []), ("a", 17, [16])],   # 9..13, 30..46
+             [("a", 1, [0]), ("b", 3, [])],     # 47; 14..16
+             [("b", 1, [0])]]
+    want = [[(39, 0, 30)], [(22, 0, 47)], [(3, 0, 17), (1, 3, 0)],
+            [(1, 3, 0)]]
+    for parts, expected in zip(steps, want):
+        calls.clear()
+        eng.replay_step([(r, tokens(n, 7), w) for r, n, w in parts])
+        assert calls == expected * 2            # two attention layers

@@ -644,3 +644,25 @@ def test_decode_graph_replays_match_eager(ckpt, dtype):
         assert g_tok == e_tok
         want = [oracle_greedy(cfg, W, p, n) for p, n in zip(prompts, lens)]
         assert [g_tok[f"r{i}"] for i in range(3)] == want
+
+
+def test_attention_is_told_where_portions_end(ckpt, monkeypatch):
+    """Short portions behind many keys, which latent layers attend to in the latent
+    space, know where the longest ends; single tokens do not."""
+    from production_stack_amd import ops
+
+    path, _, _ = ckpt
+    eng = make_engine(path, "float32", "cpu")
+    calls = []
+    attend = ops.talk_attention
+
+    def record(*args, **kw):
+        if kw.get("vdim"):
+            calls.append((args[0].shape[0], kw["variant"], kw["longest"]))
+        return attend(*args, **kw)
+
+    monkeypatch.setattr(ops, "talk_attention", record)
+    eng.replay_step([("a", tokens(120, 3), []), ("b", tokens(90, 4), [])])
+    assert not calls                        # unfolded
+    eng.replay_step([("a", tokens(2, 5), []), ("b", tokens(1, 6), [0])])
+    assert calls == [(2, 0, 122), (1, 3, 0)] * 4    # four latent layers
