@@ -746,6 +746,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     weight is below 2^-40 of the largest one. longest > 0: no row of the
     batch is at or behind that position; without it the tables' width stands
     for it where workgroups are planned (a wrong number costs time only).
+    splits > 0: workgroups that share a row's keys, where the kernel can (16 at
+    most in those that merge records), instead of what is planned.
     variant 0 picks the kernel for prompt portions (tiled thread-per-
     (head, query) where the shape fits), 3 for single tokens (split-key),
     both falling back to the plain one-workgroup-per-token kernel; 1 / 2 /
@@ -826,6 +828,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
                width if block_tables.shape[0] <= 4 else min(T, width))
     longest = min(longest, width) if longest > 0 else width
     rows = max(T, 1)  # what workgroups are planned for: kernels return at no rows
+    most = min(splits, 16)  # shares that records are merged of
     # single tokens: when the batch is too small to fill the chip with one
     # workgroup per token, each token's keys are shared out over several
     # workgroups whose partial softmax records are merged afterwards
@@ -909,8 +912,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             keys = portion
             if window > 0:
                 keys = min(keys, window + keep_first)
-            shares = splits if splits > 0 else min(16, 512 // groups, keys // 192)
-            if splits <= 0 and shares > 1:
+            shares = most if most > 0 else min(16, 512 // groups, keys // 192)
+            if most <= 0 and shares > 1:
                 walk = keys / 64 * 2.2 * (D + DV) / 256
                 record = rows * H * (DV + 4) * 1.6e-6
                 shares = min(shares, int((walk / record) ** 0.5))
@@ -954,7 +957,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # 4; portions: 80 rows behind 334 keys 20.9, 23.9 in 2)
         tpt = 1 if token else max(1, cols // rep)
         groups = (rows + tpt - 1) // tpt * G
-        shares = splits if splits > 0 else max(1, min(
+        shares = most if most > 0 else max(1, min(
             16, (512 if token else 256) // groups,
             keys // (128 if token else 256)))
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
@@ -985,7 +988,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # behind 1800, in 1 / 4 / 8 528 / 159 / 111; 1000 in 1 / 2 / 4 286 / 188 /
         # 208; 70 in 1 / 4 33 / 25), a tile of keys each at least
         groups = (rows + 3) // 4
-        shares = splits if splits > 0 else max(1, min(
+        shares = most if most > 0 else max(1, min(
             16, (256 if groups <= 48 else 512) // groups, keys // 16))
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
                             device=q.device) if shares > 1 else None)
@@ -1011,7 +1014,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             keys = min(keys, chunk)
         # one workgroup a CU (bf16 64 tokens of up to 2250 keys in 1 / 2 / 4 / 8
         # shares 215 / 120 / 78 / 86 us), 48 keys each at least
-        shares = splits if splits > 0 else max(
+        shares = most if most > 0 else max(
             1, min(16, 256 // rows, keys // 48))
         part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
                             device=q.device) if shares > 1 else None)
@@ -1027,7 +1030,6 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if variant == 15:
         raise RuntimeError(
             "talk_attention: shape or dtype outside the head-mix token kernel")
-    asked = splits
     if variant not in (3, 4, 5, 6):
         splits = 1
     elif splits <= 0:
@@ -1072,7 +1074,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         if chunk > 0:
             keys = min(keys, chunk)
         blocks = (rows + 127) // 128         # of an XCD
-        shares = asked if asked > 0 else max(1, min(
+        shares = most if most > 0 else max(1, min(
             16 // blocks if blocks <= 8 else
             2 if blocks < 12 and 5 * keys >= 4 * T else 1,
             keys // 64))

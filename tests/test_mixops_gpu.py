@@ -1454,3 +1454,25 @@ def test_attention_fp32_scores_no_number(talk, variant, general, case, splits):
     assert torch.equal(fin, torch.isfinite(got))
     # fp32 sums of up to 150 and 128 terms on both sides
     assert _rel(got[fin], want[fin]) < 4e-6
+
+
+@pytest.mark.parametrize("talk,variant,dtype", [
+    (False, 0, torch.bfloat16), (False, 11, torch.bfloat16),
+    (True, 0, torch.bfloat16), (True, 10, torch.bfloat16),
+    (False, 13, torch.float32), (False, 14, torch.float32),
+    (True, 15, torch.float32), (True, 16, torch.float32)])
+def test_attention_more_splits_than_records(talk, variant, dtype):
+    """More shares than records are merged of are as many as that."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    H, G, D, bs, T = 32, 8, 64, 16, 9
+    kc, vc = (torch.randn(40, G, bs, D, generator=g, device="cuda").to(dtype)
+              for _ in range(2))
+    tables = torch.randperm(40, generator=g, device="cuda").int()[None]
+    q = torch.randn(T, H * D, generator=g, device="cuda").to(dtype)
+    tp = torch.arange(T, dtype=torch.int32, device="cuda") + 610
+    ts = torch.zeros_like(tp)
+    mix = torch.eye(H, device="cuda") if talk else None
+    a, b = (ops.talk_attention(q, kc, vc, tables, ts, tp, D ** -0.5, H,
+                               talk=mix, variant=variant, splits=s)
+            for s in (16, 40))
+    assert torch.equal(a, b)
