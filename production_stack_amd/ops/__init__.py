@@ -829,6 +829,20 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     longest = min(longest, width) if longest > 0 else width
     rows = max(T, 1)  # what workgroups are planned for: kernels return at no rows
     most = min(splits, 16)  # shares that records are merged of
+
+    def records(shares: int):
+        # none for rows off 16-byte borders, which the kernels refuse
+        size = q.element_size()
+        if shares <= 1 or (q.stride(0) * size | VR * size | q.data_ptr()
+                           | k_cache.data_ptr() | v_cache.data_ptr()) % 16:
+            return None
+        return torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
+                           device=q.device)
+
+    # shapes that the kernels with a head mix take
+    mixes = (talk is not None and not extra and pool is None
+             and keep_first == 0 and H == 32 and H // G % 4 == 0
+             and D in (64, 128) and DV in (64, 128))
     # single tokens: when the batch is too small to fill the chip with one
     # workgroup per token, each token's keys are shared out over several
     # workgroups whose partial softmax records are merged afterwards
@@ -880,8 +894,10 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     # keys and values of their own, prompt portions or single tokens (also a
     # few rows: 64 rows of 32/8 heads behind 2048 keys 85 us against 257, 8 x 16
     # rows alone 16 against 16)
+    rep = H // G
     if (variant in (0, 3, 11, 12) and q.dtype == torch.bfloat16
-            and talk is None and chunk == 0 and not extra and pool is None):
+            and talk is None and chunk == 0 and not extra and pool is None
+            and max(D, DV) <= 128 and D % 8 == 0 and DV % 8 == 0):
         token = variant in (3, 12)
         shares = 1
         if token:
@@ -906,7 +922,6 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # widths of 128, records their write and read and their merge 3 us: as
             # many shares as make the least of both, none where that is not a fifth
             # less (200 rows behind 200 20.6 us whole, 22.0 in 2).
-            rep = H // G
             tokens = 128 // rep if rep < 128 else 1
             groups = (rows + tokens - 1) // tokens * G * ((rep + 127) // 128)
             keys = portion
@@ -920,8 +935,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
                 if shares < 2 or walk / shares + record * shares + 3 > 0.8 * walk:
                     shares = 1
             shares = max(1, shares)
-        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
-                            device=q.device) if shares > 1 else None)
+        part = records(shares)
         rc = _mx().mx_window_attention(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
@@ -936,9 +950,9 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             "talk_attention: shape or dtype outside the window kernels")
     # fp32 keys and values of their own, prompt portions or single tokens
     if (variant in (0, 3, 13, 14) and q.dtype == torch.float32
-            and talk is None and not extra and pool is None):
+            and talk is None and not extra and pool is None and rep <= 16
+            and max(D, DV) <= 128 and D % 16 == 0 and DV % 4 == 0):
         token = variant in (3, 14)
-        rep = H // G
         keys = longest
         if window > 0:
             keys = min(keys, window + keep_first)
@@ -948,20 +962,19 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # us, 16 / 32: 1000 rows of 128 alone 125 / 122, behind 3000 keys 258 /
         # 234; 400 rows 26.7 / 28.1; 1000 of 64 37.4 / 43.3)
         cols = 16
-        if not token and rep <= 32 and max(D, DV) > 64 and (
+        if not token and max(D, DV) > 64 and (
                 (T + 32 // rep - 1) // (32 // rep) * G >= 512):
             cols = 32
         # Several workgroups for a tile's keys where CUs are left: records cost 3
         # us and 4 bytes a share and entry (1 token x 947 keys 46 us whole, 18.6
         # in 8 shares; 64 x 1500 162, 157 in 3, 193 in 12; 8 x 300 19.0, 14.5 in
         # 4; portions: 80 rows behind 334 keys 20.9, 23.9 in 2)
-        tpt = 1 if token else max(1, cols // rep)
+        tpt = 1 if token else cols // rep
         groups = (rows + tpt - 1) // tpt * G
         shares = most if most > 0 else max(1, min(
             16, (512 if token else 256) // groups,
             keys // (128 if token else 256)))
-        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
-                            device=q.device) if shares > 1 else None)
+        part = records(shares)
         rc = _mx().mx_attn_f32(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
@@ -975,8 +988,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         raise RuntimeError(
             "talk_attention: shape or dtype outside the fp32 kernel")
     # a head mix over prompt portions in fp32
-    if (variant in (0, 16) and talk is not None and not extra and pool is None
-            and keep_first == 0 and q.dtype == torch.float32):
+    if variant in (0, 16) and mixes and q.dtype == torch.float32:
         keys = longest
         if window > 0:
             keys = min(keys, window)
@@ -990,8 +1002,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         groups = (rows + 3) // 4
         shares = most if most > 0 else max(1, min(
             16, (256 if groups <= 48 else 512) // groups, keys // 16))
-        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
-                            device=q.device) if shares > 1 else None)
+        part = records(shares)
         rc = _mx().mx_talk_rows_f32(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
@@ -1005,8 +1016,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         raise RuntimeError(
             "talk_attention: shape or dtype outside the fp32 head-mix kernel")
     # a head mix over single tokens
-    if (variant in (3, 15) and talk is not None and not extra and pool is None
-            and keep_first == 0):
+    if variant in (3, 15) and mixes:
         keys = longest
         if window > 0:
             keys = min(keys, window)
@@ -1016,8 +1026,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # shares 215 / 120 / 78 / 86 us), 48 keys each at least
         shares = most if most > 0 else max(
             1, min(16, 256 // rows, keys // 48))
-        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
-                            device=q.device) if shares > 1 else None)
+        part = records(shares)
         rc = _mx().mx_talk_token(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
@@ -1059,8 +1068,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         raise RuntimeError(
             "talk_attention: shape or dtype outside the matrix-core kernel")
     # a head mix over prompt portions on the matrix cores
-    if (variant in (0, 10) and q.dtype == torch.bfloat16 and talk is not None
-            and keep_first == 0 and pool is None):
+    if variant in (0, 10) and mixes and q.dtype == torch.bfloat16:
         # Several workgroups for the keys of 16 rows where CUs are left, 64 keys
         # each at least: a block of rows' two workgroups are one XCD's, which has
         # 32 CUs (us, heads of 128, in 1 / 2 / 4 / 8: 132 rows, one portion behind
@@ -1078,8 +1086,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             16 // blocks if blocks <= 8 else
             2 if blocks < 12 and 5 * keys >= 4 * T else 1,
             keys // 64))
-        part = (torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
-                            device=q.device) if shares > 1 else None)
+        part = records(shares)
         rc = _mx().mx_talk_mfma(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],

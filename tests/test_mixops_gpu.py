@@ -1476,3 +1476,36 @@ def test_attention_more_splits_than_records(talk, variant, dtype):
                                talk=mix, variant=variant, splits=s)
             for s in (16, 40))
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,D,DV,talk,pitch", [
+    (64, 1, 576, 512, False, 0),        # queries in a latent space
+    (64, 1, 64, 64, False, 4),          # rows off 16-byte borders
+    (24, 1, 128, 128, True, 0)])        # a mix over other than 32 heads
+def test_attention_records_where_kernels_take_them(H, G, D, DV, talk, pitch,
+                                                   dtype):
+    """No memory for the records of a kernel that does not take the shape."""
+    bs, T, blocks = 16, 20, 512
+    kc = torch.zeros(blocks, G, bs, D, dtype=dtype, device="cuda")
+    vc = kc if D == 576 else torch.zeros(blocks, G, bs, DV, dtype=dtype,
+                                         device="cuda")
+    tables = torch.arange(blocks, dtype=torch.int32, device="cuda")[None]
+    q = torch.zeros(T, H * D + pitch // (2 if dtype == torch.float32 else 1),
+                    dtype=dtype, device="cuda")[:, :H * D]
+    tp = torch.arange(T, dtype=torch.int32, device="cuda") + 100
+    out = torch.empty(T, H * DV, dtype=dtype, device="cuda")
+    mix = torch.eye(H, device="cuda") if talk else None
+
+    def run():
+        ops.talk_attention(q, kc, vc, tables, torch.zeros_like(tp), tp, 0.1, H,
+                           talk=mix, vdim=DV, out=out)
+
+    run()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    run()
+    # the zeros above and what the fall-back asks for are small
+    assert torch.cuda.max_memory_allocated() - before < 1 << 16
