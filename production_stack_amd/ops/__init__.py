@@ -745,7 +745,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     magnitude before the distance term; kernels may then pass over keys whose
     weight is below 2^-40 of the largest one. longest > 0: no row of the
     batch is at or behind that position; without it the tables' width stands
-    for it where workgroups are planned (a wrong number costs time only).
+    for it where workgroups are planned (a wrong number costs time only, and
+    short portions in wide tables pay for a merge without it).
     splits > 0: workgroups that share a row's keys, where the kernel can (16 at
     most in those that merge records), instead of what is planned.
     variant 0 picks the kernel for prompt portions (tiled thread-per-
@@ -819,13 +820,13 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         assert talk.is_contiguous()
     if pool is not None:
         assert kp.is_contiguous() and vp.is_contiguous()
-    # Keys of the longest portion: where nobody says, the tables' width, but beside
-    # more tables than portions usually are (a decode batch's) only the rows here. Too
-    # many shares cost a launch for their merge (window attention, 100 rows of 1
-    # sequence and 40 tokens of up to 3000 keys 85.6 -> 89.7 us in all).
+    # Keys that shares are planned for: where nobody says, the tables' width, however
+    # many tables. Planned in vain they cost the launch of a merge (us, beside 44
+    # sequences of 3000 keys, planned for the width / told: window attention, 100
+    # rows 14.1 / 11.0, 300 22.4 / 18.9; head mix, 100 rows 31.6 / 26.3); a chain that
+    # is not shared costs more (70 rows behind 2500 keys 31 in shares, 108 whole, head
+    # mix 54 and 339; 500 behind 2000 54 and 107).
     width = block_tables.shape[1] * BS
-    portion = (min(longest, width) if longest > 0 else
-               width if block_tables.shape[0] <= 4 else min(T, width))
     longest = min(longest, width) if longest > 0 else width
     rows = max(T, 1)  # what workgroups are planned for: kernels return at no rows
     most = min(splits, 16)  # shares that records are merged of
@@ -924,7 +925,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # less (200 rows behind 200 20.6 us whole, 22.0 in 2).
             tokens = 128 // rep if rep < 128 else 1
             groups = (rows + tokens - 1) // tokens * G * ((rep + 127) // 128)
-            keys = portion
+            keys = longest
             if window > 0:
                 keys = min(keys, window + keep_first)
             shares = most if most > 0 else min(16, 512 // groups, keys // 192)
@@ -1076,7 +1077,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # 112; 1349 behind 1463 279 / 205; 1800 in three prompts 101 / 118). Two
         # rounds of the CUs only where few rows see most keys (1200 rows 169 / 109, in
         # three prompts 69 / 82).
-        keys = portion
+        keys = longest
         if window > 0:
             keys = min(keys, window)
         if chunk > 0:

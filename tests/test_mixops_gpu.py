@@ -1509,3 +1509,50 @@ def test_attention_records_where_kernels_take_them(H, G, D, DV, talk, pitch,
     run()
     # the zeros above and what the fall-back asks for are small
     assert torch.cuda.max_memory_allocated() - before < 1 << 16
+
+
+class _Launches:
+    """The library, with the arguments of the calls that were made."""
+
+    def __init__(self, lib):
+        self.lib, self.made = lib, []
+
+    def __getattr__(self, name):
+        fn = getattr(self.lib, name)
+
+        def call(*args):
+            self.made.append((name, args))
+            return fn(*args)
+
+        return call
+
+    def shares(self):
+        return self.made[-1][1][-3]       # ahead of the records and the stream
+
+
+@pytest.mark.parametrize("talk,dtype", [
+    (False, torch.bfloat16), (True, torch.bfloat16),
+    (False, torch.float32), (True, torch.float32)])
+def test_attention_plan_is_of_the_keys(talk, dtype, monkeypatch):
+    """A portion's shares do not depend on how many tables the call has; a hint
+    takes the place of the tables' width."""
+    H, G, D, bs, T = 32, 8, 64, 16, 20
+    lib = _Launches(ops._mx())
+    monkeypatch.setattr(ops, "_mx", lambda: lib)
+    kc, vc = (torch.zeros(160, G, bs, D, dtype=dtype, device="cuda")
+              for _ in range(2))
+    q = torch.zeros(T, H * D, dtype=dtype, device="cuda")
+    tp = torch.arange(T, dtype=torch.int32, device="cuda") + 2400
+    mix = torch.eye(H, device="cuda") if talk else None
+
+    def shares(tables, longest=0):
+        ops.talk_attention(
+            q, kc, vc, torch.arange(160, dtype=torch.int32,
+                                    device="cuda").repeat(tables, 1),
+            torch.zeros_like(tp), tp, D ** -0.5, H, talk=mix, longest=longest)
+        return lib.shares()
+
+    assert shares(1) > 2
+    assert shares(1) == shares(4) == shares(5) == shares(100)
+    assert shares(1, 2420) == shares(100, 2420) > 2
+    assert shares(5, 100) < shares(5)
