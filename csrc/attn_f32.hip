@@ -387,8 +387,9 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
 
 // Merge of `KS` (at most AF_KS) partial records of every (token, head): 256 threads
 // of four entries each. Shares without a key have a denominator of 0 and no sums.
-// counted: the first record's third entry is how many there are; of a single one the
-// result is already there.
+// counted: the first record's third entry is how many there are, of a single one the
+// result is already there, and maxima are powers of two (as natural logarithms, ones
+// around 100 were rounded by 1e-5 of a share's weight).
 #define AF_KS 16
 template <typename T>
 __global__ __launch_bounds__(256) void attn_records_kernel(
@@ -418,7 +419,8 @@ __global__ __launch_bounds__(256) void attn_records_kernel(
   for (int s = 0; s < AF_KS; ++s) {
     if (ml[s].y == 0.f) continue;
     const float4 v = *(const float4*)(rec + s * step + AF_HEAD + d);
-    const float f = expf(ml[s].x - mh);
+    const float d = ml[s].x - mh;
+    const float f = counted ? __builtin_amdgcn_exp2f(d) : expf(d);
     l += ml[s].y * f;
     o[0] += v.x * f;
     o[1] += v.y * f;

@@ -80,7 +80,8 @@ struct TmArgs {
   float softcap;
   const float* sink_vals;
   int KS;       // workgroups that share a block's keys
-  float* part;  // [T, KS, 32, DV + 4]: maximum, denominator, shares, -, sums
+  float* part;  // [T, KS, 32, DV + 4]: maximum (a power of two), denominator,
+                // shares, -, sums
 };
 
 // A bf16 entry that is an infinity or no number.
@@ -559,7 +560,7 @@ __global__ __launch_bounds__(512) void talk_mfma_kernel(TmArgs a) {
                              16 * hb + wave * 2 + h) * (DV + 4);
       if (g == 0) {
         const float mt = sAL[(wave * 2 + h) * 16 + n];
-        rec[0] = lt != 0.f ? mt * 0.693147181f : PS_NEG_INF;
+        rec[0] = lt != 0.f ? mt : PS_NEG_INF;
         rec[1] = lt;
         rec[2] = (float)my_eff;
       }

@@ -341,12 +341,12 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(WaArgs a) {
     }
   }
   if constexpr (PART) {
-    // partial record per (token, share, head): max (natural log units),
+    // partial record per (token, share, head): max (in powers of two),
     // denominator, shares, one unused, DV sums
     float* rec = a.part + (((size_t)tok * a.KS + my_ks) * a.H + head) *
                               (size_t)(DV + WA_HEAD);
     if (hi == 0) {
-      rec[0] = l != 0.f ? m * 0.69314718f : PS_NEG_INF;
+      rec[0] = l != 0.f ? m : PS_NEG_INF;
       rec[1] = l;
       rec[2] = (float)my_eff;
     }

@@ -1556,3 +1556,26 @@ def test_attention_plan_is_of_the_keys(talk, dtype, monkeypatch):
     assert shares(1) == shares(4) == shares(5) == shares(100)
     assert shares(1, 2420) == shares(100, 2420) > 2
     assert shares(5, 100) < shares(5)
+
+
+@pytest.mark.parametrize("talk", [False, True])
+def test_attention_shares_of_far_scores(talk):
+    """Scores around 65536 powers of two: shares of the keys meet as one walk adds
+    them up. The scale makes no roundings of its own (it is half a power of two)."""
+    g = torch.Generator().manual_seed(41)
+    H, G, D, bs, L, T = 32, 8, 64, 16, 1024, 40
+    kc, vc, tables = _paged(L, G, D, D, bs, torch.bfloat16, g, 1)
+    q = torch.randn(T, H, D, generator=g)
+    q[..., :32] = 64.0
+    kc[..., :32] = 64.0
+    kc[..., 32:] *= 0.25
+    tp = torch.arange(L - T, L, dtype=torch.int32)
+    args = [x.cuda() for x in (q.reshape(T, H * D).to(torch.bfloat16), kc, vc,
+                               tables, torch.zeros_like(tp), tp)]
+    mix = torch.eye(H, device="cuda") if talk else None
+    one, more = (ops.talk_attention(
+        *args, 0.5 * math.log(2), H, talk=mix, variant=10 if talk else 11,
+        splits=s) for s in (1, 5))
+    # the same weights but for roundings of 2^-24: at most one result in a hundred
+    # goes to the next bf16 number, 2^-8 of it away
+    assert _rel(more.float(), one.float()) < 0.1 * 2 ** -8
