@@ -185,7 +185,10 @@ def _rows_before_norm(rows: int, N: int, K: int) -> bool:
     43.8, 176 1.02 times.
     Of few rows of W, long ones: 65 x 3072 x 8192 24.0 / 40.7, 112 26.6 / 30.9, 128 27.6
     / 46.2, 192 32.7 / 62.5 (decode steps of a 3b-sized stack of five layers 67 869 ->
-    795, 128 1020 -> 942, 192 1270 -> 1135), but 160 31.0 / 31.8; 67 x 2048 x 8192 20.2
+    795, 128 1020 -> 942, 192 1270 -> 1135), 161 30.7 / 35.8, 176 31.6 / 37.5, 191 32.6 /
+    37.8 (N 2944 to 3520, K 6144 to 10112: 161 to 191 rows 0.68 to 0.95 times), but 160
+    31.0 / 31.8 and 129 x 3072 x 6144 26.7 / 26.2 (steps of 161, 176 and 191 rows 920 ->
+    905, 1016 -> 1006, 988 -> 977); 67 x 2048 x 8192 20.2
     / 23.5 (65 598 -> 585). A step gains some 2 us a product less than these
     differences: 100 x 2048 x 8192 22.0 / 23.8, but steps 763 -> 769, 128 23.0 / 24.1
     and 796 -> 820; 160 x 3072 x 8192 993 -> 1005.
@@ -204,7 +207,7 @@ def _rows_before_norm(rows: int, N: int, K: int) -> bool:
                                 (K >= 14336 or not 3072 < N < 4608))))
     if rows > 64:
         if K >= 6144 and 2944 <= N < 3584:
-            return rows <= 128 or rows == 192
+            return rows <= 128 or rows > 160
         if K >= 7168 and 2048 <= N <= 2112:
             return rows <= 72
         if not 3584 <= N <= 6144 or K < 4096:
@@ -238,8 +241,9 @@ def _rows_before_rope(rows: int, N: int, K: int) -> bool:
     whole steps (up to 2048 rows of W, or a multiple of 1024): 17 x 2048 x 2048 10.3 /
     14.2, 17 x 3072 x 2048 12.8 / 15.2, 32 13.7 / 15.3, 48 14.7 / 15.4, 48 x 5120 x 2048
     15.5 / 16.1; past the lines 57 x 4096 x 2048 15.6 / 15.5, 45 x 2304 x 2048 17.2 /
-    14.8, 47 x 3008 x 2048 16.6 / 15.2, 32 x 1536 x 1536 12.2 / 10.1, 32 x 3072 x 2560
-    14.3 / 13.0."""
+    14.8, 47 x 3008 x 2048 16.6 / 15.2, 32 x 1536 x 1536 12.2 / 10.1, 32 x 3072 x 2304
+    13.8 / 12.7, 32 x 3072 x 2560 14.3 / 13.0; 48 x 3584 x 2048 14.7 / 15.0 and 48 x 6144 x
+    2048 16.6 / 16.6 are not worth a line."""
     if 17 <= rows <= 48 and K == 2048:
         return 1536 <= N <= 2048 or (N <= 5120 and N % 1024 == 0)
     if not 128 <= rows <= 192 or not 4608 <= N <= 10240 or K < 3584:

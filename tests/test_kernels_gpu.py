@@ -1415,6 +1415,18 @@ def test_parts_dispatch_narrow(behind, M, N, K, own):
         assert (got.double().sum(0) - want).norm() <= 1e-5 * want.norm()
 
 
+@pytest.mark.parametrize("M,own", [(128, True), (129, False), (160, False),
+                                   (161, True), (176, True), (191, True),
+                                   (192, True), (193, False)])
+@pytest.mark.parametrize("N,K", [(2944, 6144), (3072, 8192), (3520, 10176)])
+def test_parts_dispatch_narrow_ranges(M, N, K, own):
+    """Few long rows of W: ranges of rows, no single counts. (The library keeps 129
+    to 160 rows of fewer than 10240 entries.)"""
+    from production_stack_amd.ops import gemm_policy
+
+    assert gemm_policy._rows_before_norm(M, N, K) == own
+
+
 @pytest.mark.parametrize("M,N,K,own", [
     (17, 28160, 2048, True), (64, 32768, 2048, True), (65, 28672, 2048, False),
     (17, 28096, 2048, False), (17, 32832, 2048, False),
