@@ -464,7 +464,7 @@ static int af_launch(const AfArgs& a, hipStream_t stream) {
 // a KV head, key widths in steps of 16 and value widths in steps of 4 up to 128,
 // rows on 16-byte borders. token: single tokens (every batch row on its own), else
 // prompt portions. scratch fp32 [T, splits, H, DV + 4] when splits > 1; rows:
-// columns of a workgroup, 16 or 32 (single tokens: 16).
+// columns of a workgroup, 16 or 32 (single tokens and widths up to 64: 16).
 extern "C" int mx_attn_f32(void* out, int ldout, const void* q, int ldq,
                            const void* kc, const void* vc,
                            const void* block_tables, int max_blocks,
@@ -481,7 +481,7 @@ extern "C" int mx_attn_f32(void* out, int ldout, const void* q, int ldq,
       D > 128 || DV < 4 || DV % 4 || DV > 128 || ldq % 4 || vrow % 4 ||
       vrow < DV || (((size_t)q | (size_t)kc | (size_t)vc) & 15))
     return 1;
-  const bool wide = rows == 32 && !token;
+  const bool wide = rows == 32 && !token && (D > 64 || DV > 64);
   AfArgs a = {(float*)out, ldout, (const float*)q, ldq, (const float*)kc,
               (const float*)vc, vrow, (const int*)block_tables, max_blocks,
               (const int*)token_seq, (const int*)token_pos, T_, H, G, D, DV,
@@ -492,15 +492,15 @@ extern "C" int mx_attn_f32(void* out, int ldout, const void* q, int ldq,
               splits > 1 && scratch != nullptr ? splits : 1, (float*)scratch};
   hipStream_t s = (hipStream_t)stream;
   int rc;
-#define AF_GO(NT, NV)                                                   \
-  rc = softcap > 0.f ? (wide ? af_launch<NT, NV, 2, true>(a, s)         \
-                             : af_launch<NT, NV, 1, true>(a, s))        \
-                     : (wide ? af_launch<NT, NV, 2, false>(a, s)        \
-                             : af_launch<NT, NV, 1, false>(a, s))
+#define AF_GO(NT, NV, NC)                                    \
+  rc = softcap > 0.f ? af_launch<NT, NV, NC, true>(a, s) \
+                     : af_launch<NT, NV, NC, false>(a, s)
   if (D <= 64 && DV <= 64)
-    AF_GO(4, 1);
+    AF_GO(4, 1, 1);
+  else if (wide)
+    AF_GO(8, 2, 2);
   else
-    AF_GO(8, 2);
+    AF_GO(8, 2, 1);
 #undef AF_GO
   if (rc == 0 && a.KS > 1)
     mx_attn_records(out, ldout, scratch, T_, H, DV, a.KS, 0, MX_F32, stream);

@@ -27,6 +27,25 @@ def test_native_library_loaded():
     assert native.load() is not None
 
 
+class _Launches:
+    """The library, with the arguments of the calls that were made."""
+
+    def __init__(self, lib):
+        self.lib, self.made = lib, []
+
+    def __getattr__(self, name):
+        fn = getattr(self.lib, name)
+
+        def call(*args):
+            self.made.append((name, args))
+            return fn(*args)
+
+        return call
+
+    def shares(self):
+        return self.made[-1][1][-3]       # ahead of the records and the stream
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_embed_scale(dtype):
     g = torch.Generator().manual_seed(0)
@@ -1177,20 +1196,43 @@ def test_attention_fp32(H, G, D, DV, chunk, window, keep, softcap, variant,
     assert _rel(got[fin], want[fin]) < 3e-6
 
 
-def test_attention_fp32_wide():
-    """32 columns a wave, which prompts of some length take."""
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("kw", [dict(window=100, keep_first=5),
+                                dict(softcap=20.0), dict(chunk=70)])
+def test_attention_fp32_wide(kw, splits, monkeypatch):
+    """32 columns a wave, which 512 workgroups' rows and more take: rows of several
+    sequences in a workgroup's eight, a last one of three, values that are no
+    numbers and scores that are none."""
+    lib = _Launches(ops._mx())
+    monkeypatch.setattr(ops, "_mx", lambda: lib)
     g = torch.Generator(device="cuda").manual_seed(3)
-    H, G, D, bs, T = 32, 8, 128, 16, 271
-    kc, vc = (torch.randn(20, G, bs, D, generator=g, device="cuda")
+    H, G, D, bs, T = 32, 8, 128, 16, 523
+    kc, vc = (torch.randn(75, G, bs, D, generator=g, device="cuda")
               for _ in range(2))
-    tables = torch.randperm(20, generator=g, device="cuda").int()[None]
+    tables = torch.randperm(75, generator=g, device="cuda").int().view(3, 25)
     q = torch.randn(T, H * D, generator=g, device="cuda")
-    tp = torch.arange(T, dtype=torch.int32, device="cuda") + 20
-    ts = torch.zeros_like(tp)
-    for kw in (dict(window=100, keep_first=5), dict(softcap=20.0)):
-        want, got = (ops.talk_attention(q, kc, vc, tables, ts, tp, D ** -0.5,
-                                        H, variant=v, **kw) for v in (2, 13))
-        assert _rel(got, want) < 3e-6
+    ts, tp = [], []
+    for s, a, b in ((0, 20, 291), (1, 0, 3), (2, 120, 366), (1, 3, 6)):
+        ts += [s] * (b - a)
+        tp += range(a, b)
+    ts, tp = (torch.tensor(x, dtype=torch.int32, device="cuda")
+              for x in (ts, tp))
+    assert len(tp) == T
+    for odd in (False, True):
+        if odd:
+            vc[tables[0, 200 // bs], 3, 200 % bs, 1] = float("nan")
+            vc[tables[2, 300 // bs], 5, 300 % bs, 2] = float("inf")
+            kc[tables[2, 310 // bs], 1, 310 % bs, 7] = float("nan")
+        want, got = (ops.talk_attention(
+            q, kc, vc, tables, ts, tp, D ** -0.5, H, sink=True, variant=v,
+            splits=n, **kw) for v, n in ((2, 1), (13, splits)))
+        name, args = lib.made[-1]
+        assert name == "mx_attn_f32" and args[-4:-2] == (32, splits)
+        fin = torch.isfinite(want)
+        assert fin.all() != odd and torch.equal(fin, torch.isfinite(got))
+        assert torch.equal(torch.isnan(want), torch.isnan(got))
+        # sums of up to 366 and 128 roundings of 2^-24 on both sides
+        assert _rel(got[fin], want[fin]) < 3e-6
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -1509,25 +1551,6 @@ def test_attention_records_where_kernels_take_them(H, G, D, DV, talk, pitch,
     run()
     # the zeros above and what the fall-back asks for are small
     assert torch.cuda.max_memory_allocated() - before < 1 << 16
-
-
-class _Launches:
-    """The library, with the arguments of the calls that were made."""
-
-    def __init__(self, lib):
-        self.lib, self.made = lib, []
-
-    def __getattr__(self, name):
-        fn = getattr(self.lib, name)
-
-        def call(*args):
-            self.made.append((name, args))
-            return fn(*args)
-
-        return call
-
-    def shares(self):
-        return self.made[-1][1][-3]       # ahead of the records and the stream
 
 
 @pytest.mark.parametrize("talk,dtype", [
