@@ -35,16 +35,18 @@ from production_stack_amd.ops import gemm_policy
 DELTA_DECAY_SCALE = math.exp(-0.5)
 
 
-def _portions_end(meta, npt: int, shared: Optional[dict]) -> int:
-    """Where the longest of a step's prompt portions, its first npt rows, ends (0:
-    not known). Looked up once a step."""
-    end = shared.get("portions_end") if shared is not None else None
-    if end is None:
+def _portions(meta, npt: int, shared: Optional[dict]) -> dict:
+    """What attention plans a step's prompt portions, its first npt rows, with:
+    where the longest ends and how many there are (0: not known). Looked up once a
+    step."""
+    found = shared.get("portions") if shared is not None else None
+    if found is None:
         host = getattr(meta, "seq_rows_host", None) or ()
-        end = max((p0 + n for r0, n, p0, *_ in host if r0 < npt), default=0)
+        ends = [p0 + n for r0, n, p0, *_ in host if r0 < npt]
+        found = dict(longest=max(ends, default=0), portions=len(ends))
         if shared is not None:
-            shared["portions_end"] = end
-    return end
+            shared["portions"] = found
+    return found
 
 
 class TalkAttention(nn.Module):
@@ -241,7 +243,7 @@ class TalkAttention(nn.Module):
         # (tiled kernel); single tokens of different sequences share
         # nothing and take the split-key kernel, one workgroup per token.
         npt = min(getattr(meta, "num_prefill_tokens", T) or 0, T)
-        end = _portions_end(meta, npt, shared)
+        planned = _portions(meta, npt, shared)
         for a, b, variant in ((0, npt, 0), (npt, T, 3)):
             if b > a:
                 ops.talk_attention(
@@ -253,7 +255,7 @@ class TalkAttention(nn.Module):
                     sink_vals=self.sink_vals, pool=pool,
                     key_scale=key_scale, slopes=self.slopes(proj.device),
                     score_bound=self.score_bound,
-                    longest=end if variant == 0 else 0)
+                    **(planned if variant == 0 else {}))
         if sp.out_gate:
             ops.gated_act(proj[:, self.qkv_rows:], out, "sigmoid", out=out)
         return out
@@ -537,8 +539,7 @@ class LatentAttention(nn.Module):
                     window=sp.window, sink=sp.sink, out=o_lat[a - n:b - n],
                     variant=variant, softcap=sp.softcap,
                     sink_vals=self.sink_vals, vdim=L,
-                    longest=(_portions_end(meta, npt, shared)
-                             if variant == 0 else 0))
+                    **(_portions(meta, npt, shared) if variant == 0 else {}))
         # expand the attended latents per head: [H, T, L] x [H, L, DV]
         ops.merge_heads(
             torch.bmm(o_lat.view(m, H, L).transpose(0, 1), self.uv),

@@ -715,6 +715,49 @@ def kv_append(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
         _mx_dtype(k.dtype), _stream())
 
 
+def _window_shares(rows: int, H: int, G: int, D: int, DV: int, keys: int,
+                   runs: int) -> int:
+    """Workgroups that share the keys of a tile of prompt rows in window attention:
+    several where CUs are left, with three tiles of 64 keys each at least, of which
+    the kernel counts those that are (us, 32/8 heads of 128, 128 (token, head) rows a
+    workgroup in 1 / 2 / 4 / 8 shares: 70 tokens behind 2500 keys 93 / 53 / 35 / 28;
+    250 behind 2500 93 / 56 / 41 / 40; 559 behind 2500 93 / 74 / 71 / 78; 1419 behind
+    2000 120 / 118 / 127 / 156).
+
+    A workgroup takes the sequences (`runs` in all) in its rows one after the other:
+    2.5 us a tile of keys at widths of 128 and 1.5 tiles for the start of each. Whole,
+    it has fewer rows where those leave CUs idle (window_attention.hip), so fewer
+    sequences. Records' write and read and their merge take 3 us and more: as many
+    shares as make the least of all, none where that is not a fifth less (200 rows
+    behind 200 20.6 us whole, 22.0 in 2). Sequences of 2 rows behind 600 keys, 16 of
+    them 110 us whole, 182 in 3 shares, 40 in 16; 64 of them 111, 183 in 3, 50 in 16;
+    16 of 9 rows behind 4000 327 whole, 119 in 11 and 123 in 12; 200 of 9 behind 1000
+    286 whole, which they stay."""
+    rep = H // G
+    heads = min(rep, 128)
+    groups = G * ((rep + 127) // 128)   # workgroups of a tile of rows
+    tile = whole = 128 // heads
+    room = 512 // (-(-rows // tile) * groups)
+    if room < 2:
+        return 1
+    while (whole > 1 and whole * heads > 32
+           and -(-rows // (whole // 2)) * groups <= 256):
+        whole //= 2
+    step = 2.5 * (D + DV) / 256
+    tiles = keys / 64
+    per = rows / runs                   # rows of a sequence
+    met = (tile + per - 1) / per        # sequences of a workgroup's rows
+    record = rows * H * (DV + 4) * 1.6e-6
+    most = int(min(16, room, tiles / 3 * met,
+                   (met * tiles * step / record) ** 0.5))
+    if most < 2:
+        return 1
+    split = min(most, max(1, int(tiles / 3)))
+    shared = met * (tiles + 1.5 * split) / most * step + record * most + 3
+    alone = (whole + per - 1) / per * (tiles + 1.5) * step
+    return most if shared < 0.8 * alone else 1
+
+
 def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
                    v_cache: torch.Tensor, block_tables: torch.Tensor,
                    token_seq: torch.Tensor, token_pos: torch.Tensor,
@@ -725,7 +768,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
                    softcap: float = 0.0, sink_vals: torch.Tensor = None,
                    vdim: int = 0, pool=None, key_scale: torch.Tensor = None,
                    slopes: torch.Tensor = None, score_bound: float = 0.0,
-                   longest: int = 0) -> torch.Tensor:
+                   longest: int = 0, portions: int = 0) -> torch.Tensor:
     """Paged attention of a ragged batch. q [T, H*D] (row-strided view
     allowed); token_seq/token_pos int32 [T] give each token's block-table
     row and position; talk: optional fp32 [H, H] score mix; chunk/window:
@@ -746,7 +789,9 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     weight is below 2^-40 of the largest one. longest > 0: no row of the
     batch is at or behind that position; without it the tables' width stands
     for it where workgroups are planned (a wrong number costs time only, and
-    short portions in wide tables pay for a merge without it).
+    short portions in wide tables pay for a merge without it). portions > 0: how
+    many sequences' rows the batch holds, likewise (without it as many as there
+    are tables, or rows).
     splits > 0: workgroups that share a row's keys, where the kernel can (16 at
     most in those that merge records), instead of what is planned.
     variant 0 picks the kernel for prompt portions (tiled thread-per-
@@ -823,11 +868,12 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     # Keys that shares are planned for: where nobody says, the tables' width, however
     # many tables. Planned in vain they cost the launch of a merge (us, beside 44
     # sequences of 3000 keys, planned for the width / told: window attention, 100
-    # rows 14.1 / 11.0, 300 22.4 / 18.9; head mix, 100 rows 31.6 / 26.3); a chain that
+    # rows 15.7 / 10.9, 300 22.2 / 18.9; head mix, 100 rows 31.6 / 26.3); a chain that
     # is not shared costs more (70 rows behind 2500 keys 31 in shares, 108 whole, head
     # mix 54 and 339; 500 behind 2000 54 and 107).
     width = block_tables.shape[1] * BS
     longest = min(longest, width) if longest > 0 else width
+    portions = min(portions or block_tables.shape[0], T) or 1
     rows = max(T, 1)  # what workgroups are planned for: kernels return at no rows
     most = min(splits, 16)  # shares that records are merged of
 
@@ -914,28 +960,11 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             shares = splits if splits > 0 else max(
                 1, min(16, 128 // groups, keys // 1024))
         else:
-            # Several workgroups for a portion's keys where CUs are left, with
-            # three tiles of 64 each at least, of which the kernel counts those
-            # that are (us, 32/8 heads of 128, 128 (token, head) rows a workgroup
-            # in 1 / 2 / 4 / 8 shares: 70 tokens behind 2500 keys 93 / 53 / 35 /
-            # 28; 250 behind 2500 93 / 56 / 41 / 40; 559 behind 2500 93 / 74 / 71
-            # / 78; 1419 behind 2000 120 / 118 / 127 / 156). A tile takes 2.2 us at
-            # widths of 128, records their write and read and their merge 3 us: as
-            # many shares as make the least of both, none where that is not a fifth
-            # less (200 rows behind 200 20.6 us whole, 22.0 in 2).
-            tokens = 128 // rep if rep < 128 else 1
-            groups = (rows + tokens - 1) // tokens * G * ((rep + 127) // 128)
             keys = longest
             if window > 0:
                 keys = min(keys, window + keep_first)
-            shares = most if most > 0 else min(16, 512 // groups, keys // 192)
-            if most <= 0 and shares > 1:
-                walk = keys / 64 * 2.2 * (D + DV) / 256
-                record = rows * H * (DV + 4) * 1.6e-6
-                shares = min(shares, int((walk / record) ** 0.5))
-                if shares < 2 or walk / shares + record * shares + 3 > 0.8 * walk:
-                    shares = 1
-            shares = max(1, shares)
+            shares = most if most > 0 else _window_shares(
+                rows, H, G, D, DV, keys, portions)
         part = records(shares)
         rc = _mx().mx_window_attention(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),

@@ -1558,7 +1558,8 @@ def test_attention_records_where_kernels_take_them(H, G, D, DV, talk, pitch,
     (False, torch.float32), (True, torch.float32)])
 def test_attention_plan_is_of_the_keys(talk, dtype, monkeypatch):
     """A portion's shares do not depend on how many tables the call has; a hint
-    takes the place of the tables' width."""
+    takes the place of the tables' width. Of sequences that nobody counts, as many
+    as tables or rows are planned for."""
     H, G, D, bs, T = 32, 8, 64, 16, 20
     lib = _Launches(ops._mx())
     monkeypatch.setattr(ops, "_mx", lambda: lib)
@@ -1568,17 +1569,20 @@ def test_attention_plan_is_of_the_keys(talk, dtype, monkeypatch):
     tp = torch.arange(T, dtype=torch.int32, device="cuda") + 2400
     mix = torch.eye(H, device="cuda") if talk else None
 
-    def shares(tables, longest=0):
+    def shares(tables, longest=0, portions=1):
         ops.talk_attention(
             q, kc, vc, torch.arange(160, dtype=torch.int32,
                                     device="cuda").repeat(tables, 1),
-            torch.zeros_like(tp), tp, D ** -0.5, H, talk=mix, longest=longest)
+            torch.zeros_like(tp), tp, D ** -0.5, H, talk=mix, longest=longest,
+            portions=portions)
         return lib.shares()
 
     assert shares(1) > 2
     assert shares(1) == shares(4) == shares(5) == shares(100)
     assert shares(1, 2420) == shares(100, 2420) > 2
     assert shares(5, 100) < shares(5)
+    assert shares(5, 300, 0) == shares(5, 300, 5)
+    assert shares(100, 300, 0) == shares(100, 300, 20)
 
 
 @pytest.mark.parametrize("talk", [False, True])

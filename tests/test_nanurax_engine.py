@@ -396,7 +396,7 @@ def test_trace_run_command(ckpt, tmp_path):
 
 def test_attention_is_told_where_portions_end(ckpt, monkeypatch):
     """Every attention layer's portions know where the longest of a step's ends,
-    whichever comes first; its single tokens do not."""
+    whichever comes first, and how many they are; its single tokens do not."""
     from production_stack_amd import ops
 
     path, _, _ = ckpt
@@ -405,7 +405,8 @@ def test_attention_is_told_where_portions_end(ckpt, monkeypatch):
     attend = ops.talk_attention
 
     def record(*args, **kw):
-        calls.append((args[0].shape[0], kw["variant"], kw["longest"]))
+        calls.append((args[0].shape[0], kw["variant"],
+                      kw.get("longest"), kw.get("portions")))
         return attend(*args, **kw)
 
     monkeypatch.setattr(ops, "talk_attention", record)
@@ -413,8 +414,8 @@ def test_attention_is_told_where_portions_end(ckpt, monkeypatch):
              [("b", 5, []), ("a", 17, [16])],   # 9..13, 30..46
              [("a", 1, [0]), ("b", 3, [])],     # 47; 14..16
              [("b", 1, [0])]]
-    want = [[(39, 0, 30)], [(22, 0, 47)], [(3, 0, 17), (1, 3, 0)],
-            [(1, 3, 0)]]
+    want = [[(39, 0, 30, 2)], [(22, 0, 47, 2)],
+            [(3, 0, 17, 1), (1, 3, None, None)], [(1, 3, None, None)]]
     for parts, expected in zip(steps, want):
         calls.clear()
         eng.replay_step([(r, tokens(n, 7), w) for r, n, w in parts])

@@ -7,6 +7,7 @@ GPU kernel tests compare against a trustworthy baseline.
 import pytest
 import torch
 
+from production_stack_amd import ops
 from production_stack_amd.ops import reference
 
 
@@ -164,3 +165,27 @@ def test_gemm_policy_lines(rule, shape, own):
     from production_stack_amd.ops import gemm_policy
 
     assert getattr(gemm_policy, "_" + rule)(*shape) == own
+
+
+def test_window_attention_plan():
+    """Shares of portions' keys: of a sequence's rows alone behind many keys, of many
+    short sequences behind some, none where nothing is gained; never more than
+    records are merged of or than two rounds of the CUs."""
+    def plan(rows, keys, runs, H=32, G=8, D=128):
+        return ops._window_shares(rows, H, G, D, D, keys, runs)
+
+    assert plan(70, 2570, 1) >= 8 and plan(250, 2750, 1) in (4, 8)
+    assert plan(100, 100, 1) == plan(300, 300, 1) == plan(200, 400, 1) == 1
+    # as many keys of one sequence are less than those of each of many
+    assert plan(32, 602, 16) > plan(32, 602, 1) > 1
+    assert plan(128, 302, 64) > plan(128, 302, 1) == 1
+    assert plan(1419, 3419, 1) == plan(4000, 4000, 2) == 1
+    for H, G, D in ((32, 8, 128), (40, 1, 64), (300, 2, 8), (1, 1, 128)):
+        for rows in (1, 2, 31, 32, 33, 500, 5000):
+            for keys in (0, 1, 63, 200, 5000, 100000):
+                for runs in {1, 2, rows // 2 or 1, rows}:
+                    n = plan(rows, keys, min(runs, rows), H, G, D)
+                    heads = min(H // G, 128)
+                    groups = (-(-rows // (128 // heads)) * G
+                              * -(-(H // G) // 128))
+                    assert n == 1 or 1 < n <= min(16, 512 // groups)

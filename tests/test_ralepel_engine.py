@@ -648,7 +648,8 @@ def test_decode_graph_replays_match_eager(ckpt, dtype):
 
 def test_attention_is_told_where_portions_end(ckpt, monkeypatch):
     """Short portions behind many keys, which latent layers attend to in the latent
-    space, know where the longest ends; single tokens do not."""
+    space, know where the longest ends and how many they are; single tokens do
+    not."""
     from production_stack_amd import ops
 
     path, _, _ = ckpt
@@ -658,11 +659,13 @@ def test_attention_is_told_where_portions_end(ckpt, monkeypatch):
 
     def record(*args, **kw):
         if kw.get("vdim"):
-            calls.append((args[0].shape[0], kw["variant"], kw["longest"]))
+            calls.append((args[0].shape[0], kw["variant"],
+                      kw.get("longest"), kw.get("portions")))
         return attend(*args, **kw)
 
     monkeypatch.setattr(ops, "talk_attention", record)
     eng.replay_step([("a", tokens(120, 3), []), ("b", tokens(90, 4), [])])
     assert not calls                        # unfolded
     eng.replay_step([("a", tokens(2, 5), []), ("b", tokens(1, 6), [0])])
-    assert calls == [(2, 0, 122), (1, 3, 0)] * 4    # four latent layers
+    # four latent layers
+    assert calls == [(2, 0, 122, 1), (1, 3, None, None)] * 4
