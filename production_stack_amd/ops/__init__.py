@@ -746,15 +746,17 @@ def _window_shares(rows: int, H: int, G: int, D: int, DV: int, keys: int,
     step = 2.5 * (D + DV) / 256
     tiles = keys / 64
     per = rows / runs                   # rows of a sequence
-    met = (tile + per - 1) / per        # sequences of a workgroup's rows
+    full = max(1.0, tile / per)         # sequences that fill a workgroup's rows
     record = rows * H * (DV + 4) * 1.6e-6
-    most = int(min(16, room, tiles / 3 * met,
-                   (met * tiles * step / record) ** 0.5))
+    most = int(min(16, room, tiles / 3 * full,
+                   (full * tiles * step / record) ** 0.5))
     if most < 2:
         return 1
     split = min(most, max(1, int(tiles / 3)))
+    # sequences that reach into a workgroup's rows
+    met, few = (tile + per - 1) / per, (whole + per - 1) / per
     shared = met * (tiles + 1.5 * split) / most * step + record * most + 3
-    alone = (whole + per - 1) / per * (tiles + 1.5) * step
+    alone = few * (tiles + 1.5) * step
     return most if shared < 0.8 * alone else 1
 
 

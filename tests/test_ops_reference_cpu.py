@@ -174,7 +174,7 @@ def test_window_attention_plan():
     def plan(rows, keys, runs, H=32, G=8, D=128):
         return ops._window_shares(rows, H, G, D, D, keys, runs)
 
-    assert plan(70, 2570, 1) >= 8 and plan(250, 2750, 1) in (4, 8)
+    assert plan(70, 2570, 1) >= 8 and 4 <= plan(250, 2750, 1) <= 8
     assert plan(100, 100, 1) == plan(300, 300, 1) == plan(200, 400, 1) == 1
     # as many keys of one sequence are less than those of each of many
     assert plan(32, 602, 16) > plan(32, 602, 1) > 1
