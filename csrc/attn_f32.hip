@@ -27,13 +27,16 @@
 // quarter of the columns). 32/8 heads of 128, us, by the vector kernels of
 // talk_attention.hip -> by this one: 254 rows in 3 portions, one behind 2264 keys, cap
 // 7430 -> 84; 80 rows behind 334 keys 1360 -> 21; 1000 rows of 64 in 3 prompts 562 ->
-// 37; 1000 rows 122, half the fp32 matrix rate; one token behind 947 keys 345 -> 19;
-// 64 behind 1500 157, 5.1 TB/s.
+// 35; 1000 rows 119, with a cap 132, half the fp32 matrix rate; one token behind 947
+// keys 345 -> 19; 64 behind 1500 139, 5.7 TB/s.
 // Errors against 64 bits are those of the vector kernels or less (40 tokens of up to 900
-// keys 2.3e-7 and 2.1e-7, 128 of up to 300 2.1e-7 and 2.0e-7, 1000 rows behind 3000
-// 1.1e-6 and 4.9e-7): sums are short chains that are added up, scores by 16 entries,
-// outputs by tiles (40 tokens with outputs in one chain over all keys and scores by 32
-// 3.3e-7 and 78.7 us, 79.8 so).
+// keys 2.3e-7 and 2.1e-7, 128 of up to 300 2.1e-7 and 2.0e-7): with 16 columns a wave
+// sums are short chains that are added up, scores by 16 entries, outputs by tiles (40
+// tokens with outputs in one chain over all keys and scores by 32 3.3e-7 and 78.7 us,
+// 79.8 so). With 32 there are no registers for that: scores by 64 entries, outputs in
+// one chain over a wave's keys (vector / 16 / 32 columns: 523 rows 2.7e-7 / 1.4e-7 /
+// 2.2e-7, 1000 behind 3000 keys 1.4e-6 / 2.4e-7 / 5.9e-7, 523 behind 6000 1.8e-6 /
+// 2.7e-7 / 7.6e-7).
 #include "attn_common.h"
 
 struct AfArgs {

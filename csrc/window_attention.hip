@@ -669,7 +669,8 @@ int mx_window_attention(void* out, int ldout, const void* q, int ldq,
     // the CUs (70 rows behind 2500 keys 26 us, 37 with fewer rows). Portions that
     // end up without shares, runs of a workgroup's rows over the workgroups that share
     // them: four of 17 11.4 (20 with all of them the first one's, 11.8 without
-    // shares), eight of 30 14.0 (12.0 without shares and their merge).
+    // shares), eight of 30 14.0 (12.0 without shares and their merge, as they are
+    // planned where the call says how long and how many they are).
     a.tpt = 128 / a.hpb;
     a.KS = splits > 1 && scratch != nullptr ? splits : 1;
     if (a.KS > 16) return 1;
