@@ -715,6 +715,20 @@ def kv_append(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
         _mx_dtype(k.dtype), _stream())
 
 
+def _records(shares: int, q: torch.Tensor, k_cache: torch.Tensor,
+             v_cache: torch.Tensor, H: int, DV: int):
+    """Memory for the records of shares; none for rows off 16-byte borders, which
+    the kernels refuse (looked at where it is more than some 2 MB)."""
+    T = q.shape[0]
+    if T * shares * H > 4096:
+        size = q.element_size()
+        if (q.stride(0) * size | v_cache.shape[3] * size | q.data_ptr()
+                | k_cache.data_ptr() | v_cache.data_ptr()) % 16:
+            return None
+    return torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
+                       device=q.device)
+
+
 def _window_shares(rows: int, H: int, G: int, D: int, DV: int, keys: int,
                    runs: int) -> int:
     """Workgroups that share the keys of a tile of prompt rows in window attention:
@@ -734,19 +748,22 @@ def _window_shares(rows: int, H: int, G: int, D: int, DV: int, keys: int,
     16 of 9 rows behind 4000 327 whole, 119 in 11 and 123 in 12; 200 of 9 behind 1000
     286 whole, which they stay."""
     rep = H // G
-    heads = min(rep, 128)
+    heads = rep if rep < 128 else 128
     groups = G * ((rep + 127) // 128)   # workgroups of a tile of rows
     tile = whole = 128 // heads
-    room = 512 // (-(-rows // tile) * groups)
-    if room < 2:
+    room = 512 // ((rows + tile - 1) // tile * groups)
+    full = runs * tile / rows           # sequences that fill a workgroup's rows
+    if full < 1:
+        full = 1
+    elif full > runs:
+        full = runs
+    if room < 2 or keys * full < 384:
         return 1
     while (whole > 1 and whole * heads > 32
-           and -(-rows // (whole // 2)) * groups <= 256):
+           and (rows + whole // 2 - 1) // (whole // 2) * groups <= 256):
         whole //= 2
     step = 2.5 * (D + DV) / 256
     tiles = keys / 64
-    per = rows / runs                   # rows of a sequence
-    full = max(1.0, tile / per)         # sequences that fill a workgroup's rows
     record = rows * H * (DV + 4) * 1.6e-6
     most = int(min(16, room, tiles / 3 * full,
                    (full * tiles * step / record) ** 0.5))
@@ -754,7 +771,8 @@ def _window_shares(rows: int, H: int, G: int, D: int, DV: int, keys: int,
         return 1
     split = min(most, max(1, int(tiles / 3)))
     # sequences that reach into a workgroup's rows
-    met, few = (tile + per - 1) / per, (whole + per - 1) / per
+    met = min(runs, 1 + (tile - 1) * runs / rows)
+    few = min(runs, 1 + (whole - 1) * runs / rows)
     shared = met * (tiles + 1.5 * split) / most * step + record * most + 3
     alone = few * (tiles + 1.5) * step
     return most if shared < 0.8 * alone else 1
@@ -792,8 +810,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     batch is at or behind that position; without it the tables' width stands
     for it where workgroups are planned (a wrong number costs time only, and
     short portions in wide tables pay for a merge without it). portions > 0: how
-    many sequences' rows the batch holds, likewise (without it as many as there
-    are tables, or rows).
+    many sequences' rows the batch holds, likewise.
     splits > 0: workgroups that share a row's keys, where the kernel can (16 at
     most in those that merge records), instead of what is planned.
     variant 0 picks the kernel for prompt portions (tiled thread-per-
@@ -875,23 +892,13 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     # mix 54 and 339; 500 behind 2000 54 and 107).
     width = block_tables.shape[1] * BS
     longest = min(longest, width) if longest > 0 else width
-    portions = min(portions or block_tables.shape[0], T) or 1
+    portions = min(portions, T)
     rows = max(T, 1)  # what workgroups are planned for: kernels return at no rows
     most = min(splits, 16)  # shares that records are merged of
-
-    def records(shares: int):
-        # none for rows off 16-byte borders, which the kernels refuse
-        size = q.element_size()
-        if shares <= 1 or (q.stride(0) * size | VR * size | q.data_ptr()
-                           | k_cache.data_ptr() | v_cache.data_ptr()) % 16:
-            return None
-        return torch.empty((T, shares, H, DV + 4), dtype=torch.float32,
-                           device=q.device)
-
     # shapes that the kernels with a head mix take
-    mixes = (talk is not None and not extra and pool is None
-             and keep_first == 0 and H == 32 and H // G % 4 == 0
-             and D in (64, 128) and DV in (64, 128))
+    mixes = (talk is not None and H == 32 and 8 % G == 0 and pool is None
+             and keep_first == 0 and (D == 64 or D == 128)
+             and (DV == 64 or DV == 128))
     # single tokens: when the batch is too small to fill the chip with one
     # workgroup per token, each token's keys are shared out over several
     # workgroups whose partial softmax records are merged afterwards
@@ -966,8 +973,15 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             if window > 0:
                 keys = min(keys, window + keep_first)
             shares = most if most > 0 else _window_shares(
-                rows, H, G, D, DV, keys, portions)
-        part = records(shares)
+                rows, H, G, D, DV, keys, portions or 1)
+            if shares > 1 and most <= 0 and not portions:
+                # of nobody knows how many sequences: as one alone has shares,
+                # enough for as many as there can be
+                shares = max(shares, _window_shares(
+                    rows, H, G, D, DV, keys,
+                    min(block_tables.shape[0], rows)))
+        part = (None if shares <= 1 else
+                _records(shares, q, k_cache, v_cache, H, DV))
         rc = _mx().mx_window_attention(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
@@ -1006,7 +1020,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         shares = most if most > 0 else max(1, min(
             16, (512 if token else 256) // groups,
             keys // (128 if token else 256)))
-        part = records(shares)
+        part = (None if shares <= 1 else
+                _records(shares, q, k_cache, v_cache, H, DV))
         rc = _mx().mx_attn_f32(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
@@ -1034,7 +1049,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         groups = (rows + 3) // 4
         shares = most if most > 0 else max(1, min(
             16, (256 if groups <= 48 else 512) // groups, keys // 16))
-        part = records(shares)
+        part = (None if shares <= 1 else
+                _records(shares, q, k_cache, v_cache, H, DV))
         rc = _mx().mx_talk_rows_f32(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
@@ -1058,7 +1074,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
         # shares 215 / 120 / 78 / 86 us), 48 keys each at least
         shares = most if most > 0 else max(
             1, min(16, 256 // rows, keys // 48))
-        part = records(shares)
+        part = (None if shares <= 1 else
+                _records(shares, q, k_cache, v_cache, H, DV))
         rc = _mx().mx_talk_token(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],
@@ -1118,7 +1135,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
             16 // blocks if blocks <= 8 else
             2 if blocks < 12 and 5 * keys >= 4 * T else 1,
             keys // 64))
-        part = records(shares)
+        part = (None if shares <= 1 else
+                _records(shares, q, k_cache, v_cache, H, DV))
         rc = _mx().mx_talk_mfma(
             _p(out), _rows(out, "out"), _p(q), _rows(q, "q"), _p(k_cache),
             _p(v_cache), _p(block_tables), block_tables.shape[1],

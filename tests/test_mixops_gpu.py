@@ -1558,8 +1558,8 @@ def test_attention_records_where_kernels_take_them(H, G, D, DV, talk, pitch,
     (False, torch.float32), (True, torch.float32)])
 def test_attention_plan_is_of_the_keys(talk, dtype, monkeypatch):
     """A portion's shares do not depend on how many tables the call has; a hint
-    takes the place of the tables' width. Of sequences that nobody counts, as many
-    as tables or rows are planned for."""
+    takes the place of the tables' width. Where nobody counts the sequences, one
+    alone has to gain by shares."""
     H, G, D, bs, T = 32, 8, 64, 16, 20
     lib = _Launches(ops._mx())
     monkeypatch.setattr(ops, "_mx", lambda: lib)
@@ -1581,8 +1581,8 @@ def test_attention_plan_is_of_the_keys(talk, dtype, monkeypatch):
     assert shares(1) == shares(4) == shares(5) == shares(100)
     assert shares(1, 2420) == shares(100, 2420) > 2
     assert shares(5, 100) < shares(5)
-    assert shares(5, 300, 0) == shares(5, 300, 5)
-    assert shares(100, 300, 0) == shares(100, 300, 20)
+    assert shares(5, 100, 0) == shares(100, 100, 0) == shares(1, 100)
+    assert shares(5, 0, 0) >= shares(5)
 
 
 @pytest.mark.parametrize("talk", [False, True])
