@@ -27,7 +27,7 @@
 // quarter of the columns). 32/8 heads of 128, us, by the vector kernels of
 // talk_attention.hip -> by this one: 254 rows in 3 portions, one behind 2264 keys, cap
 // 7430 -> 84; 80 rows behind 334 keys 1360 -> 21; 1000 rows of 64 in 3 prompts 562 ->
-// 35; 1000 rows 119, with a cap 132, half the fp32 matrix rate; one token behind 947
+// 35; 1000 rows 120, with a cap 130, half the fp32 matrix rate; one token behind 947
 // keys 345 -> 19; 64 behind 1500 139, 5.7 TB/s.
 // Errors against 64 bits are those of the vector kernels or less (40 tokens of up to 900
 // keys 2.3e-7 and 2.1e-7, 128 of up to 300 2.1e-7 and 2.0e-7): with 16 columns a wave
@@ -71,6 +71,10 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
   constexpr int COLS = 16 * NC, PA = NV * 64 + 4;
   constexpr int NS = NC * NT > 8 ? 2 : NT;  // sums of a score; more would spill
   constexpr bool APART = NC == 1;
+  // Which keys are hidden is kept for the careful walk as masks or, with a cap and 32
+  // columns, found again there: registers (masks / found again, 1000 rows of 128 with a
+  // cap 132.8 / 130.0 us, without one 120.0 / 122.2).
+  constexpr bool AGAIN = NC == 2 && CAP;
   extern __shared__ __align__(16) float sA[];  // [4][COLS][PA]: the merge
   __shared__ float s_m[4][COLS], s_l[4][COLS];
   __shared__ int s_seq[COLS], s_pos[COLS];
@@ -207,6 +211,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
           const int j0 = first(t) + 4 * g;
           const int end = t < nt0 ? k0 - 1 : kmax;
           bool seen[NC][4];
+          unsigned hid = 0;
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             const bool mine = my_i[c] >= rs && my_i[c] < re;
@@ -231,6 +236,11 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
             }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            if (AGAIN && careful) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (p[i] == -INFINITY) hid |= 1u << (4 * c + i);
+            }
             if (__any(mx > m[c])) {
               const float mn = fmaxf(m[c], mx);
               const float al = expf(m[c] - mn);
@@ -260,7 +270,9 @@ __global__ __launch_bounds__(256, 2) void attn_f32_kernel(AfArgs a) {
                 float own = -1.f;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                  if ((k & 3) == i && seen[c][i]) own = st[c][0][i];
+                  if ((k & 3) == i &&
+                      (AGAIN ? !(hid >> (4 * c + i) & 1) : seen[c][i]))
+                    own = st[c][0][i];
                 w[c] = __shfl(own, k / 4 * 16 + n, 64);
               }
 #pragma unroll
