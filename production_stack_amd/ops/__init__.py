@@ -747,6 +747,8 @@ def _window_shares(rows: int, H: int, G: int, D: int, DV: int, keys: int,
     them 110 us whole, 182 in 3 shares, 40 in 16; 64 of them 111, 183 in 3, 50 in 16;
     16 of 9 rows behind 4000 327 whole, 119 in 11 and 123 in 12; 200 of 9 behind 1000
     286 whole, which they stay."""
+    if keys < 384 and runs == 1:        # two shares of three tiles
+        return 1
     rep = H // G
     heads = rep if rep < 128 else 128
     groups = G * ((rep + 127) // 128)   # workgroups of a tile of rows
@@ -892,9 +894,8 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     # mix 54 and 339; 500 behind 2000 54 and 107).
     width = block_tables.shape[1] * BS
     longest = min(longest, width) if longest > 0 else width
-    portions = min(portions, T)
-    rows = max(T, 1)  # what workgroups are planned for: kernels return at no rows
-    most = min(splits, 16)  # shares that records are merged of
+    rows = T or 1     # what workgroups are planned for: kernels return at no rows
+    most = splits if splits < 16 else 16    # shares that records are merged of
     # shapes that the kernels with a head mix take
     mixes = (talk is not None and H == 32 and 8 % G == 0 and pool is None
              and keep_first == 0 and (D == 64 or D == 128)
@@ -953,7 +954,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     rep = H // G
     if (variant in (0, 3, 11, 12) and q.dtype == torch.bfloat16
             and talk is None and chunk == 0 and not extra and pool is None
-            and max(D, DV) <= 128 and D % 8 == 0 and DV % 8 == 0):
+            and D <= 128 and DV <= 128 and (D | DV) % 8 == 0):
         token = variant in (3, 12)
         shares = 1
         if token:
@@ -997,7 +998,7 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor,
     # fp32 keys and values of their own, prompt portions or single tokens
     if (variant in (0, 3, 13, 14) and q.dtype == torch.float32
             and talk is None and not extra and pool is None and rep <= 16
-            and max(D, DV) <= 128 and D % 16 == 0 and DV % 4 == 0):
+            and D <= 128 and DV <= 128 and D % 16 == 0 and DV % 4 == 0):
         token = variant in (3, 14)
         keys = longest
         if window > 0:
